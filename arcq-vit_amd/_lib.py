@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sys
 import threading
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -127,6 +128,29 @@ def load() -> ctypes.CDLL:
                 fn.argtypes = argtypes
             _lib = lib
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The CPython extension with the host side of the hot calls (``csrc_host/arcq_host.cpp``); as loud as ``load`` if it
+    has not been built.  Its functions return None for calls they leave to the Python code."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _arcq_host as mod
+        except ImportError as e:
+            raise ARCQLibraryMissing(f"ARCQ host extension is not built or does not load ({e}). "
+                                     "Run `python -m arcq_vit_amd.build` first.") from e
+        import torch
+        from . import vit
+        from .packed_on_the_fly import ARCQPackedLinearOnTheFly
+        mod.register_types(ARCQPackedLinearOnTheFly, vit.Attention, vit.Mlp, torch.nn.GELU, torch.nn.LayerNorm,
+                           sys.modules["torch.nn.modules.module"])
+        _host = mod
+    return _host
 
 
 def check(rc: int) -> None:

@@ -1,4 +1,4 @@
-"""Build recipe for ``libarcq_hip.so``: ``python -m arcq_vit_amd.build``.
+"""Build recipe for ``libarcq_hip.so`` and ``_arcq_host.so``: ``python -m arcq_vit_amd.build``.
 
 hipcc cross-compiles for gfx950 without a GPU present.  The library lands next
 to this file so that it travels with the source tree.  Every source file is
@@ -25,6 +25,7 @@ COMPILE_FLAGS = [
     # Keep the compiler from forming packed-fp32 VALU ops.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
+HOST_NAME = "_arcq_host.so"
 LINK_FLAGS = ["--offload-arch=gfx950", "-shared", "-fPIC", "-fvisibility=hidden"]
 
 
@@ -58,6 +59,32 @@ def build(verbose: bool = False, incremental: bool = False, jobs: int = 6) -> st
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
         list(pool.map(lambda c: _run(c, verbose), todo))
     _run([hipcc, *LINK_FLAGS, "-o", out + ".tmp", *objs], verbose)
+    os.replace(out + ".tmp", out)
+    build_host(verbose, incremental)
+    return out
+
+
+def build_host(verbose: bool = False, incremental: bool = False) -> str:
+    """The CPython extension with the host side of the hot calls (``csrc_host/arcq_host.cpp``), next to the library it
+    calls: plain host C++ against torch's headers, no device code."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+
+    src = os.path.join(_PKG_DIR, "csrc_host", "arcq_host.cpp")
+    out = os.path.join(_PKG_DIR, HOST_NAME)
+    header = os.path.join(_ROOT, "include", "arcq_hip.h")
+    if incremental and os.path.exists(out) and os.path.getmtime(out) > max(os.path.getmtime(src), os.path.getmtime(header)):
+        return out
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    includes = [os.path.join(_ROOT, "include"), sysconfig.get_paths()["include"], *cpp_extension.include_paths("cuda")]
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for d in includes:
+        cmd += ["-isystem" if d != includes[0] else "-I", d]
+    cmd += [src, "-o", out + ".tmp", "-L" + _PKG_DIR, "-l:libarcq_hip.so", "-Wl,-rpath,$ORIGIN", "-L" + lib, "-ltorch_python",
+            "-ltorch_hip", "-ltorch_cpu", "-ltorch", "-lc10_hip", "-lc10", "-Wl,-rpath," + lib]
+    _run(cmd, verbose)
     os.replace(out + ".tmp", out)
     return out
 

@@ -1,0 +1,782 @@
+// Host side of the package's hot calls as a CPython extension (`arcq_vit_amd._arcq_host`): what a forward does between
+// the Python call and the kernel launches -- argument checks, the cached fp32 / contiguous views of a layer's buffers,
+// output and scratch allocation, the current stream, the call into libarcq_hip.so.
+//
+// Why it exists: these calls are a few kernels of 5-15 us each, and the same work written in Python (attribute and
+// data_ptr reads, torch.empty / reshape / torch.cuda.device, a ctypes call with some twenty arguments) costs 15-25 us
+// per layer, so that up to a few hundred rows -- and, in whole models, up to a batch of about twenty -- the GPU waited
+// for the host.  Measured per layer call on one box: 18 us in Python, 6 us here.
+//
+// Every function returns None where a call is not the plain case (an argument of another type, layout or device, a
+// module with hooks, a shape the library does not run): the Python code behind it then validates, converts and raises
+// as it always did.  Nothing here synchronises; the GIL is held throughout.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/DynamicTypes.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+#include <cstring>
+#include <optional>
+#include <string>
+#include <vector>
+
+#include "arcq_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+// ---- names --------------------------------------------------------------------------------------------------------
+#define ARCQ_NAMES(X)                                                                                                     \
+    X(_buffers) X(_modules) X(_parameters) X(_host_plan) X(_weight_buffer) X(_x_hat_buffer) X(out_dtype) X(fp8_operands) \
+    X(in_features) X(out_features) X(bits) X(group_size) X(act_group_size) X(in_channels) X(kernel_size)                  \
+    X(packed_weight_codes) X(weight_codebook) X(weight_center)                                                            \
+    X(weight_scale) X(weight_code_sum) X(activation_codebook) X(activation_thresholds) X(bias_tensor) X(bias)             \
+    X(product_table) X(weight_codes_u8) X(weight_dequant) X(runtime_code_format)                                          \
+    X(weight) X(eps) X(normalized_shape) X(elementwise_affine) X(norm1) X(norm2) X(attn) X(mlp) X(qkv) X(proj) X(fc1)     \
+    X(fc2) X(act) X(fuse_elementwise) X(chain_mlp) X(num_heads) X(own_kernel) X(approximate) X(none) X(forward)           \
+    X(_forward_hooks) X(_forward_pre_hooks) X(_backward_hooks) X(_backward_pre_hooks) X(mix)                              \
+    X(_global_forward_hooks) X(_global_forward_pre_hooks) X(_global_backward_hooks) X(_global_backward_pre_hooks)
+struct Names {
+#define X(n) PyObject *n;
+    ARCQ_NAMES(X)
+#undef X
+} S;
+
+PyObject *g_torch_module = nullptr;      // torch.nn.modules.module (the global hook dictionaries)
+PyObject *g_layer_type = nullptr;        // ARCQPackedLinearOnTheFly
+PyObject *g_attention_type = nullptr, *g_mlp_type = nullptr;
+PyObject *g_gelu_type = nullptr, *g_layernorm_type = nullptr;
+
+struct Failure {};      // a Python exception is set
+
+[[noreturn]] void raise_library_error(int rc)
+{
+    const char *msg = arcq_last_error();
+    if (msg && msg[0]) PyErr_SetString(PyExc_RuntimeError, msg);
+    else PyErr_Format(PyExc_RuntimeError, "libarcq_hip call failed with code %d", rc);
+    throw Failure{};
+}
+inline void check(int rc) { if (rc != 0) raise_library_error(rc); }
+
+inline PyObject *dict_of(PyObject *o)
+{
+    PyObject **d = _PyObject_GetDictPtr(o);
+    return d ? *d : nullptr;
+}
+inline PyObject *get(PyObject *dict, PyObject *key) { return dict ? PyDict_GetItem(dict, key) : nullptr; }   // borrowed
+inline bool is_true(PyObject *o) { return o == Py_True; }
+inline bool get_int(PyObject *dict, PyObject *key, int64_t &out)
+{
+    PyObject *v = get(dict, key);
+    if (!v || !PyLong_CheckExact(v)) return false;
+    out = PyLong_AsLongLong(v);
+    return true;
+}
+inline const Tensor *as_tensor(PyObject *o) { return o && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+inline uint32_t version_of(const Tensor &t)
+{
+    const auto &vc = t.unsafeGetTensorImpl()->version_counter();
+    return vc.enabled() ? vc.current_version() : 0;
+}
+inline Tensor empty(at::IntArrayRef sizes, at::ScalarType type, c10::Device device)
+{
+    return Tensor(at::detail::empty_cuda(sizes, type, device, std::nullopt));
+}
+inline void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+inline bool here(const Tensor &t) { return t.is_cuda() && t.device().index() == c10::hip::current_device(); }
+inline bool f16(const Tensor &t) { return t.scalar_type() == at::kHalf; }
+inline bool f32(const Tensor &t) { return t.scalar_type() == at::kFloat; }
+inline int code_of(const Tensor &t) { return f16(t) ? ARCQ_F16 : ARCQ_F32; }
+inline const float *fptr(const Tensor &t) { return static_cast<const float *>(t.const_data_ptr()); }
+inline const uint8_t *bptr(const Tensor &t) { return static_cast<const uint8_t *>(t.const_data_ptr()); }
+
+// ---- a layer's buffers, as the library takes them -------------------------------------------------------------------
+struct Slot {
+    Tensor src, use;          // the module's buffer (kept: its identity is what is compared) and what is handed to the library
+    uint32_t version = 0;
+    const void *data = nullptr;
+    bool same(const Tensor &t) const
+    {
+        return src.unsafeGetTensorImpl() == t.unsafeGetTensorImpl() && version == version_of(t) && data == t.const_data_ptr();
+    }
+    void set(const Tensor &t, bool as_f32)
+    {
+        src = t;
+        version = version_of(t);
+        data = t.const_data_ptr();
+        use = (as_f32 ? t.detach().to(at::kFloat) : t.detach()).contiguous();
+    }
+};
+struct LayerNormParams {
+    Slot w, b;
+    bool has_bias = false;
+};
+constexpr int kMaxSlots = 11;
+struct Plan {
+    bool valid = false;
+    c10::DeviceIndex device = -1;
+    int64_t K = 0, N = 0, bits = 0, gs = 0;
+    Slot slot[kMaxSlots];
+    const void *p[kMaxSlots] = {};
+    double fp8_mult = NAN;
+    std::vector<LayerNormParams> ln;
+};
+
+struct PlanObject {
+    PyObject_HEAD
+    Plan *plan;
+};
+PyObject *plan_new(PyTypeObject *type, PyObject *, PyObject *)
+{
+    PlanObject *o = reinterpret_cast<PlanObject *>(type->tp_alloc(type, 0));
+    if (o) o->plan = new Plan();
+    return reinterpret_cast<PyObject *>(o);
+}
+void plan_dealloc(PyObject *o)
+{
+    delete reinterpret_cast<PlanObject *>(o)->plan;
+    Py_TYPE(o)->tp_free(o);
+}
+PyObject *plan_reduce(PyObject *o, PyObject *)      // copies and pickles start empty
+{
+    return Py_BuildValue("O()", reinterpret_cast<PyObject *>(Py_TYPE(o)));
+}
+PyObject *plan_get_mult(PyObject *o, void *) { return PyFloat_FromDouble(reinterpret_cast<PlanObject *>(o)->plan->fp8_mult); }
+int plan_set_mult(PyObject *o, PyObject *v, void *)
+{
+    const double d = v ? PyFloat_AsDouble(v) : NAN;
+    if (PyErr_Occurred()) return -1;
+    reinterpret_cast<PlanObject *>(o)->plan->fp8_mult = d;
+    return 0;
+}
+PyMethodDef plan_methods[] = {{"__reduce__", plan_reduce, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyGetSetDef plan_getset[] = {{"fp8_mult", plan_get_mult, plan_set_mult, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// The three kinds of module: their buffers in the order of Plan::slot.
+enum { A_THR, A_CB, W_PACKED, W_CB, W_CENTER, W_SCALE, W_SUM, W_BIAS, P_TABLE, P_CODES, P_DENSE };
+enum class Kind { OnTheFly, Packed, Conv };
+
+Plan *plan_of(PyObject *module, Kind kind, PyObject *&dict)
+{
+    dict = dict_of(module);
+    PyObject *buffers = get(dict, S._buffers);
+    if (!buffers || !PyDict_Check(buffers)) return nullptr;
+    PyObject *po = get(dict, S._host_plan);
+    Plan *plan;
+    if (po && Py_TYPE(po) == &PlanType) {
+        plan = reinterpret_cast<PlanObject *>(po)->plan;
+    } else {
+        PyObject *fresh = plan_new(&PlanType, nullptr, nullptr);
+        if (!fresh || PyDict_SetItem(dict, S._host_plan, fresh) != 0) throw Failure{};
+        plan = reinterpret_cast<PlanObject *>(fresh)->plan;
+        Py_DECREF(fresh);
+    }
+    PyObject *const names[kMaxSlots] = {S.activation_thresholds, S.activation_codebook, S.packed_weight_codes, S.weight_codebook,
+                                        S.weight_center, S.weight_scale, S.weight_code_sum,
+                                        kind == Kind::OnTheFly ? S.bias_tensor : S.bias, S.product_table, S.weight_codes_u8,
+                                        S.weight_dequant};
+    const int n = kind == Kind::Packed ? 11 : 8;
+    const Tensor *t[kMaxSlots];
+    bool same = plan->valid;
+    for (int i = 0; i < n; ++i) {
+        t[i] = as_tensor(get(buffers, names[i]));
+        if (!t[i]) return nullptr;
+        same = same && plan->slot[i].same(*t[i]);
+    }
+    if (same) return plan;
+    plan->valid = false;
+    plan->fp8_mult = NAN;
+    plan->ln.clear();
+    const c10::Device dev = t[W_PACKED]->device();
+    for (int i = 0; i < n; ++i) {
+        if (t[i]->numel() == 0) continue;
+        if (!t[i]->is_cuda() || t[i]->device() != dev) return nullptr;
+    }
+    if (!t[W_PACKED]->is_cuda() || t[W_PACKED]->scalar_type() != at::kByte) return nullptr;
+    if (kind == Kind::Conv) {
+        int64_t c;
+        if (!get_int(dict, S.in_channels, c)) return nullptr;
+        plan->N = t[W_PACKED]->size(0);
+        plan->K = 256 * c;
+    } else if (!get_int(dict, S.in_features, plan->K) || !get_int(dict, S.out_features, plan->N)) {
+        return nullptr;
+    }
+    if (!get_int(dict, S.bits, plan->bits) || !get_int(dict, S.group_size, plan->gs)) return nullptr;
+    for (int i = 0; i < n; ++i) {
+        plan->slot[i].set(*t[i], i != W_PACKED && i != P_CODES && i != P_DENSE);
+        plan->p[i] = t[i]->numel() ? plan->slot[i].use.const_data_ptr() : nullptr;
+    }
+    plan->device = dev.index();
+    plan->valid = true;
+    return plan;
+}
+
+// fp32 copies of a LayerNorm's weight and bias (made once per layer and parameter version); nullptr: not the plain case.
+LayerNormParams *layernorm_params(Plan &plan, PyObject *ln, float &eps)
+{
+    PyObject *d = dict_of(ln);
+    PyObject *params = get(d, S._parameters);
+    PyObject *e = get(d, S.eps), *shape = get(d, S.normalized_shape);
+    const Tensor *w = as_tensor(get(params, S.weight));
+    PyObject *bo = get(params, S.bias);
+    const Tensor *b = as_tensor(bo);
+    if (!w || !e || !PyFloat_Check(e) || !shape || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != 1) return nullptr;
+    if (!b && bo != Py_None) return nullptr;
+    eps = static_cast<float>(PyFloat_AS_DOUBLE(e));
+    for (auto &p : plan.ln)
+        if (p.w.same(*w) && p.has_bias == (b != nullptr) && (!b || p.b.same(*b))) return &p;
+    if (!w->is_cuda() || w->device().index() != plan.device || w->numel() != plan.K || w->dim() != 1) return nullptr;
+    if (b && (b->device() != w->device() || b->numel() != plan.K)) return nullptr;
+    if (plan.ln.size() >= 4) plan.ln.clear();        // (a layer has one LayerNorm in front of it; a bound, not a policy)
+    LayerNormParams p;
+    p.w.set(*w, true);
+    p.has_bias = b != nullptr;
+    if (b) p.b.set(*b, true);
+    else p.b.use = at::zeros_like(p.w.use);
+    plan.ln.push_back(p);
+    return &plan.ln.back();
+}
+
+// ---- one on-the-fly layer -------------------------------------------------------------------------------------------
+struct Options {
+    PyObject *layernorm = nullptr, *next = nullptr;
+    bool gelu = false, x_is_xhat = false;
+    const Tensor *residual = nullptr;
+};
+
+// Whether `a`'s launch may end with the stage 1 of `b` (ARCQPackedLinearOnTheFly.can_quantize_for).
+bool can_quantize(PyObject *da, const Plan &a, PyObject *db, const Plan &b, int64_t rows)
+{
+    if (is_true(get(da, S.fp8_operands)) || is_true(get(db, S.fp8_operands)) || rows <= 0 || a.gs != 64 || b.gs != 64 ||
+        a.bits != b.bits || b.K != a.N || a.N % 64 != 0 || a.K % 64 != 0 ||
+        get(da, S.out_dtype) != reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf)))
+        return false;
+    if (rows < 512) return a.K <= 1536;
+    PyObject *w = get(da, S._weight_buffer);
+    if (!w || w == Py_None || rows * a.K * 2 >= (int64_t(1) << 32)) return false;
+    return strncmp(arcq_linear_otf_ws_kernel(rows, a.N, a.K, 1), "otf_rows", 8) != 0;
+}
+
+std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Options &o)
+{
+    PyObject *dict;
+    Plan *plan = plan_of(module, Kind::OnTheFly, dict);
+    if (!plan || !here(x) || x.device().index() != plan->device || !x.is_contiguous() || (!f16(x) && !f32(x)) || x.dim() < 1 ||
+        x.size(-1) != plan->K || x.numel() == 0)
+        return std::nullopt;
+    const int64_t K = plan->K, N = plan->N, m = x.numel() / K;
+    PyObject *od = get(dict, S.out_dtype);
+    at::ScalarType out_type;
+    if (od == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf))) out_type = at::kHalf;
+    else if (od == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kFloat))) out_type = at::kFloat;
+    else return std::nullopt;
+    const bool fp8 = is_true(get(dict, S.fp8_operands));
+    const bool extras = o.layernorm || o.gelu || o.residual || o.next || o.x_is_xhat;
+    float ln_eps = 0.0f;
+    LayerNormParams *ln = nullptr;
+    if (extras) {
+        if (fp8 || plan->gs != 64 || K % 64 != 0) return std::nullopt;
+        if (o.layernorm) {
+            if (K > (m >= 512 ? 1024 : 1536)) return std::nullopt;
+            ln = layernorm_params(*plan, o.layernorm, ln_eps);
+            if (!ln) return std::nullopt;
+        }
+        if (o.x_is_xhat && (!f16(x) || o.layernorm)) return std::nullopt;
+        if (o.residual && (o.residual->scalar_type() != out_type || o.residual->device() != x.device() ||
+                           !o.residual->is_contiguous() || o.residual->numel() != m * N || o.residual->size(-1) != N))
+            return std::nullopt;
+    }
+    Plan *next = nullptr;
+    if (o.next) {
+        PyObject *nd;
+        next = plan_of(o.next, Kind::OnTheFly, nd);
+        if (!next || next->device != plan->device || !can_quantize(dict, *plan, nd, *next, m)) return std::nullopt;
+    }
+    at::DimVector sizes(x.sizes());
+    sizes.back() = N;
+    void *stream = stream_of(x);
+    const auto *p = plan->p;
+    auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
+    if (fp8) {
+        if (plan->gs != 64 || std::isnan(plan->fp8_mult)) return std::nullopt;
+        const int64_t kp = (K + 127) / 128 * 128;
+        Tensor x8 = empty({m * kp}, at::kByte, x.device()), w8 = empty({N * kp}, at::kByte, x.device());
+        Tensor y = empty(sizes, out_type, x.device());
+        check(arcq_linear_otf_fp8(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), static_cast<const uint8_t *>(p[W_PACKED]),
+                                  fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), static_cast<float>(plan->fp8_mult),
+                                  x8.mutable_data_ptr(), w8.mutable_data_ptr(), y.mutable_data_ptr(), code_of(y), m, N, K,
+                                  static_cast<int>(plan->bits), stream));
+        return y;
+    }
+    PyObject *wo = get(dict, S._weight_buffer);
+    const Tensor *w_ws = nullptr;
+    if (wo && wo != Py_None) {
+        w_ws = as_tensor(wo);
+        if (!w_ws || !w_ws->is_cuda() || !f16(*w_ws) || !w_ws->is_contiguous() || w_ws->numel() < N * K ||
+            w_ws->device() != x.device())
+            return std::nullopt;
+    }
+    Tensor own_ws;
+    const Tensor *ws = as_tensor(get(dict, S._x_hat_buffer));
+    if (!ws || !f16(*ws) || !ws->is_contiguous() || ws->numel() < x.numel() || ws->device() != x.device()) {
+        own_ws = empty({x.numel()}, at::kHalf, x.device());
+        ws = &own_ws;
+    }
+    Tensor y = empty(sizes, out_type, x.device());
+    if (!extras) {
+        check(arcq_linear_otf_ws(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), static_cast<const uint8_t *>(p[W_PACKED]),
+                                 fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), ws->mutable_data_ptr(),
+                                 w_ws ? w_ws->mutable_data_ptr() : nullptr, y.mutable_data_ptr(), code_of(y), m, N, K,
+                                 static_cast<int>(plan->bits), static_cast<int>(plan->gs), stream));
+        return y;
+    }
+    arcq_linear_ex_args a = {};
+    a.struct_size = sizeof(a);
+    a.x_dtype = code_of(x);
+    a.y_dtype = code_of(y);
+    a.bits = static_cast<int>(plan->bits);
+    a.group_size = static_cast<int>(plan->gs);
+    a.M = m, a.N = N, a.K = K;
+    a.x = x.const_data_ptr();
+    if (ln) {
+        a.producer = ARCQ_PRODUCER_LAYERNORM;
+        a.ln_weight = fptr(ln->w.use), a.ln_bias = fptr(ln->b.use), a.ln_eps = ln_eps;
+    }
+    if (o.x_is_xhat) a.producer = ARCQ_PRODUCER_XHAT;
+    a.activation = o.gelu ? ARCQ_ACT_GELU : ARCQ_ACT_NONE;
+    a.a_thresholds = fp(A_THR), a.a_codebook = fp(A_CB), a.packed_w = static_cast<const uint8_t *>(p[W_PACKED]);
+    a.w_codebook = fp(W_CB), a.w_center = fp(W_CENTER), a.w_scale = fp(W_SCALE), a.w_code_sum = fp(W_SUM), a.bias = fp(W_BIAS);
+    if (o.residual) a.residual = o.residual->const_data_ptr();
+    if (next) {
+        a.next_a_thresholds = static_cast<const float *>(next->p[A_THR]);
+        a.next_a_codebook = static_cast<const float *>(next->p[A_CB]);
+    }
+    a.x_hat_ws = ws->mutable_data_ptr();
+    a.w_hat_ws = w_ws ? w_ws->mutable_data_ptr() : nullptr;
+    a.y = y.mutable_data_ptr();
+    check(arcq_linear_otf_ex(&a, stream));
+    return y;
+}
+
+// ---- whole block ----------------------------------------------------------------------------------------------------
+bool no_hooks(PyObject *dict)      // calling the module would run its class's forward and nothing else
+{
+    if (!dict || get(dict, S.forward)) return false;
+    for (PyObject *n : {S._forward_hooks, S._forward_pre_hooks, S._backward_hooks, S._backward_pre_hooks}) {
+        PyObject *h = get(dict, n);
+        if (!h || !PyDict_Check(h) || PyDict_Size(h) != 0) return false;
+    }
+    return true;
+}
+bool no_global_hooks()
+{
+    PyObject *d = PyModule_GetDict(g_torch_module);
+    for (PyObject *n : {S._global_forward_hooks, S._global_forward_pre_hooks, S._global_backward_hooks, S._global_backward_pre_hooks}) {
+        PyObject *h = get(d, n);
+        if (!h || !PyDict_Check(h) || PyDict_Size(h) != 0) return false;
+    }
+    return true;
+}
+inline bool is_type(PyObject *o, PyObject *type) { return o && reinterpret_cast<PyObject *>(Py_TYPE(o)) == type; }
+
+std::optional<Tensor> attention_call(const Tensor &qkv, int64_t heads, float scale)
+{
+    if (!here(qkv) || !f16(qkv) || qkv.dim() != 3 || !qkv.is_contiguous()) return std::nullopt;
+    const int64_t b = qkv.size(0), n = qkv.size(1), c = qkv.size(2) / 3;
+    if (qkv.size(2) != 3 * c || c != 64 * heads) return std::nullopt;
+    Tensor out = empty({b, n, c}, at::kHalf, qkv.device());
+    check(arcq_attention_fwd(qkv.const_data_ptr(), out.mutable_data_ptr(), b, n, heads, 64, scale, stream_of(qkv)));
+    return out;
+}
+
+Tensor mix(const Tensor &qkv, int64_t heads, bool own)      // Attention.mix
+{
+    const int64_t b = qkv.size(0), n = qkv.size(1), c = qkv.size(2) / 3;
+    if (own && c == 64 * heads && n <= 256) {
+        auto y = attention_call(qkv, heads, 0.125f);
+        if (y) return *y;
+    }
+    const auto t = qkv.reshape({b, n, 3, heads, c / heads}).permute({2, 0, 3, 1, 4});
+    return at::scaled_dot_product_attention(t.select(0, 0), t.select(0, 1), t.select(0, 2)).transpose(1, 2).reshape({b, n, c});
+}
+
+Tensor layernorm_op(PyObject *d, const Tensor &x, bool &ok)      // an nn.LayerNorm as torch runs it
+{
+    PyObject *params = get(d, S._parameters), *e = get(d, S.eps), *shape = get(d, S.normalized_shape);
+    PyObject *wo = get(params, S.weight), *bo = get(params, S.bias);
+    if (!e || !PyFloat_Check(e) || !shape || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != 1 || !wo || !bo) {
+        ok = false;
+        return {};
+    }
+    const Tensor *w = as_tensor(wo), *b = as_tensor(bo);
+    if ((!w && wo != Py_None) || (!b && bo != Py_None)) {
+        ok = false;
+        return {};
+    }
+    const int64_t n = PyLong_AsLongLong(PyTuple_GET_ITEM(shape, 0));
+    return at::layer_norm(x, {n}, w ? std::optional<Tensor>(*w) : std::nullopt, b ? std::optional<Tensor>(*b) : std::nullopt,
+                          PyFloat_AS_DOUBLE(e));
+}
+
+// One transformer block (vit.Block.forward), both of its forms; nullopt before anything has been launched where a module
+// is not the plain case.
+std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
+{
+    PyObject *d = dict_of(block);
+    PyObject *mods = get(d, S._modules);
+    if (!mods || x.dim() != 3 || !here(x) || !x.is_contiguous() || x.numel() == 0 || !no_global_hooks()) return std::nullopt;
+    PyObject *attn = get(mods, S.attn), *mlp = get(mods, S.mlp), *n1 = get(mods, S.norm1), *n2 = get(mods, S.norm2);
+    if (!is_type(attn, g_attention_type) || !is_type(mlp, g_mlp_type) || !is_type(n1, g_layernorm_type) || !is_type(n2, g_layernorm_type))
+        return std::nullopt;
+    PyObject *ad = dict_of(attn), *md = dict_of(mlp), *d1 = dict_of(n1), *d2 = dict_of(n2);
+    PyObject *am = get(ad, S._modules), *mm = get(md, S._modules);
+    PyObject *qkv = get(am, S.qkv), *proj = get(am, S.proj), *fc1 = get(mm, S.fc1), *fc2 = get(mm, S.fc2), *act = get(mm, S.act);
+    for (PyObject *l : {qkv, proj, fc1, fc2})
+        if (!is_type(l, g_layer_type) || !no_hooks(dict_of(l))) return std::nullopt;
+    if (!is_type(act, g_gelu_type) || get(ad, S.mix)) return std::nullopt;
+    PyObject *approx = get(dict_of(act), S.approximate);
+    if (!approx || !PyUnicode_Check(approx) || PyUnicode_Compare(approx, S.none) != 0) return std::nullopt;
+    int64_t heads;
+    if (!get_int(ad, S.num_heads, heads) || heads <= 0) return std::nullopt;
+    const bool own = is_true(get(ad, S.own_kernel));
+    PyObject *dq, *dp, *df1, *df2;
+    Plan *pq = plan_of(qkv, Kind::OnTheFly, dq), *pp = plan_of(proj, Kind::OnTheFly, dp), *pf1 = plan_of(fc1, Kind::OnTheFly, df1),
+         *pf2 = plan_of(fc2, Kind::OnTheFly, df2);
+    const int64_t c = x.size(2);
+    if (!pq || !pp || !pf1 || !pf2 || pq->K != c || pq->N != 3 * c || pp->K != c || pp->N != c || pf1->K != c || pf2->K != pf1->N ||
+        pf2->N != c || c % heads != 0)
+        return std::nullopt;
+    const int64_t rows = x.size(0) * x.size(1);
+    if (is_true(get(d, S.fuse_elementwise))) {
+        for (PyObject *l : {dq, dp, df1, df2})
+            if (is_true(get(l, S.fp8_operands)) || get(l, S.out_dtype) != reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf)))
+                return std::nullopt;
+        if (!f16(x) || c > (rows >= 512 ? 1024 : 1536) || c % 64 != 0 || pf2->K % 64 != 0) return std::nullopt;
+        for (Plan *p : {pq, pp, pf1, pf2})
+            if (p->gs != 64) return std::nullopt;
+        Options o1;
+        o1.layernorm = n1;
+        auto t = layer_call(qkv, x, o1);
+        if (!t) return std::nullopt;
+        const Tensor a = mix(*t, heads, own);
+        Options o2;
+        o2.residual = &x;
+        auto x1 = layer_call(proj, a, o2);
+        if (!x1) return std::nullopt;
+        Options o3, o4;
+        o3.layernorm = n2;
+        o3.gelu = true;
+        PyObject *cm = get(d, S.chain_mlp);
+        if (is_true(cm) && can_quantize(df1, *pf1, df2, *pf2, rows)) {
+            o3.next = fc2;
+            o4.x_is_xhat = true;
+        }
+        auto h = layer_call(fc1, *x1, o3);
+        if (!h) return std::nullopt;
+        o4.residual = &*x1;
+        return layer_call(fc2, *h, o4);
+    }
+    for (PyObject *dd : {ad, md, d1, d2, dict_of(act)})
+        if (!no_hooks(dd)) return std::nullopt;
+    bool ok = true;
+    Tensor t = layernorm_op(d1, x, ok);
+    if (!ok) return std::nullopt;
+    auto q = layer_call(qkv, t, Options{});
+    if (!q) return std::nullopt;
+    auto a = layer_call(proj, mix(*q, heads, own), Options{});
+    if (!a) return std::nullopt;
+    const Tensor x1 = at::add(x, *a);
+    t = layernorm_op(d2, x1, ok);
+    if (!ok) return std::nullopt;
+    auto h = layer_call(fc1, t, Options{});
+    if (!h) return std::nullopt;
+    auto y = layer_call(fc2, at::gelu(*h), Options{});
+    if (!y) return std::nullopt;
+    return at::add(x1, *y);
+}
+
+// ---- Python entry points ----------------------------------------------------------------------------------------------
+template <typename F>
+PyObject *guarded(F &&f)
+{
+    try {
+        return f();
+    } catch (const Failure &) {
+        return nullptr;
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+}
+PyObject *none() { Py_RETURN_NONE; }
+PyObject *wrap(std::optional<Tensor> &&t)
+{
+    if (!t) return none();
+    return THPVariable_Wrap(std::move(*t));
+}
+
+// layer_forward(module, x, layernorm, gelu, residual, next, x_is_xhat)
+PyObject *py_layer_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        const Tensor *x = n == 7 ? as_tensor(args[1]) : nullptr;
+        if (!x) return none();
+        Options o;
+        if (args[2] != Py_None) {
+            if (!is_type(args[2], g_layernorm_type)) return none();
+            o.layernorm = args[2];
+        }
+        o.gelu = is_true(args[3]);
+        if (args[4] != Py_None && !(o.residual = as_tensor(args[4]))) return none();
+        if (args[5] != Py_None) {
+            if (!PyObject_TypeCheck(args[5], reinterpret_cast<PyTypeObject *>(g_layer_type))) return none();
+            o.next = args[5];
+        }
+        o.x_is_xhat = is_true(args[6]);
+        return wrap(layer_call(args[0], *x, o));
+    });
+}
+
+PyObject *py_block_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        const Tensor *x = n == 2 ? as_tensor(args[1]) : nullptr;
+        return x ? wrap(block_call(args[0], *x)) : none();
+    });
+}
+
+// attention(qkv, heads, scale)
+PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        const Tensor *q = n == 3 ? as_tensor(args[0]) : nullptr;
+        if (!q || !PyLong_CheckExact(args[1]) || !PyFloat_CheckExact(args[2])) return none();
+        return wrap(attention_call(*q, PyLong_AsLongLong(args[1]), static_cast<float>(PyFloat_AS_DOUBLE(args[2]))));
+    });
+}
+
+// patch_embed(img, weight, bias or None, cls, pos)
+PyObject *py_patch_embed(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        if (n != 5) return none();
+        const Tensor *t[5];
+        for (int i = 0; i < 5; ++i) {
+            t[i] = as_tensor(args[i]);
+            if (!t[i] && (i != 2 || args[i] != Py_None)) return none();
+            if (t[i] && (!here(*t[i]) || !f16(*t[i]) || !t[i]->is_contiguous())) return none();
+        }
+        const Tensor &img = *t[0], &w = *t[1];
+        if (img.dim() != 4 || img.size(1) != 3 || w.dim() != 4 || w.size(1) != 3 || w.size(2) != 16 || w.size(3) != 16) return none();
+        const int64_t b = img.size(0), h = img.size(2), wd = img.size(3), N = w.size(0), tokens = 1 + (h / 16) * (wd / 16);
+        if (b == 0 || N % 32 != 0 || h % 16 != 0 || wd % 16 != 0 || t[3]->numel() != N || t[4]->numel() != tokens * N ||
+            (t[2] && t[2]->numel() != N))
+            return none();
+        Tensor out = empty({b, tokens, N}, at::kHalf, img.device());
+        check(arcq_patch_embed_fwd(img.const_data_ptr(), w.const_data_ptr(), t[2] ? t[2]->const_data_ptr() : nullptr,
+                                   t[3]->const_data_ptr(), t[4]->const_data_ptr(), out.mutable_data_ptr(), b, h, wd, 16, N,
+                                   stream_of(img)));
+        return THPVariable_Wrap(std::move(out));
+    });
+}
+
+struct Quantized { Tensor codes, center, scale, sum; };
+bool quantize_args_ok(const Tensor &x, const Tensor &thr, const Tensor &cb, int64_t bits, int64_t gs)
+{
+    return (bits == 2 || bits == 3 || bits == 4) && gs > 0 && here(x) && x.dim() == 2 && f32(x) && x.is_contiguous() &&
+           x.size(1) % gs == 0 && thr.device() == x.device() && cb.device() == x.device() && f32(thr) && f32(cb) &&
+           thr.is_contiguous() && cb.is_contiguous() && cb.numel() == (int64_t(1) << bits) && thr.numel() == cb.numel() - 1;
+}
+Quantized quantize(const Tensor &x, const float *thr, const float *cb, int64_t bits, int64_t gs, bool bytes)
+{
+    const int64_t rows = x.size(0), cols = x.size(1), groups = cols / gs;
+    Quantized q;
+    q.codes = empty({rows, bytes ? cols : (cols * bits + 7) / 8}, at::kByte, x.device());
+    q.center = empty({rows, groups}, at::kFloat, x.device());
+    q.scale = empty({rows, groups}, at::kFloat, x.device());
+    q.sum = empty({rows, groups}, at::kFloat, x.device());
+    uint8_t *codes = static_cast<uint8_t *>(q.codes.mutable_data_ptr());
+    check(arcq_act_quant(x.const_data_ptr(), ARCQ_F32, thr, cb, bytes ? nullptr : codes, bytes ? codes : nullptr,
+                         static_cast<float *>(q.center.mutable_data_ptr()), static_cast<float *>(q.scale.mutable_data_ptr()),
+                         static_cast<float *>(q.sum.mutable_data_ptr()), nullptr, ARCQ_F32, rows, cols, static_cast<int>(bits),
+                         static_cast<int>(gs), 1.0e-6f, stream_of(x)));
+    return q;
+}
+
+// quantize(x, thresholds, codebook, bits, group_size, bytes) -> [codes, center, scale, code_sum]
+PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        if (n != 6 || !PyLong_CheckExact(args[3]) || !PyLong_CheckExact(args[4])) return none();
+        const Tensor *x = as_tensor(args[0]), *thr = as_tensor(args[1]), *cb = as_tensor(args[2]);
+        const int64_t bits = PyLong_AsLongLong(args[3]), gs = PyLong_AsLongLong(args[4]);
+        if (!x || !thr || !cb || !quantize_args_ok(*x, *thr, *cb, bits, gs)) return none();
+        Quantized q = quantize(*x, fptr(*thr), fptr(*cb), bits, gs, is_true(args[5]));
+        PyObject *list = PyList_New(4);
+        if (!list) return nullptr;
+        PyList_SET_ITEM(list, 0, THPVariable_Wrap(std::move(q.codes)));
+        PyList_SET_ITEM(list, 1, THPVariable_Wrap(std::move(q.center)));
+        PyList_SET_ITEM(list, 2, THPVariable_Wrap(std::move(q.scale)));
+        PyList_SET_ITEM(list, 3, THPVariable_Wrap(std::move(q.sum)));
+        return list;
+    });
+}
+
+// packed_forward(module, x): ARCQPackedLinear in its four runtime formats, group size 64 or (index-space formats) any
+PyObject *py_packed_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        const Tensor *xp = n == 2 ? as_tensor(args[1]) : nullptr;
+        if (!xp) return none();
+        const Tensor &x = *xp;
+        PyObject *dict;
+        Plan *plan = plan_of(args[0], Kind::Packed, dict);
+        if (!plan || !here(x) || x.device().index() != plan->device || !f32(x) || !x.is_contiguous() || x.dim() < 1 ||
+            x.size(-1) != plan->K || x.numel() == 0)
+            return none();
+        PyObject *fo = get(dict, S.runtime_code_format);
+        const char *fmt = fo && PyUnicode_Check(fo) ? PyUnicode_AsUTF8(fo) : nullptr;
+        if (!fmt) return none();
+        const int64_t K = plan->K, N = plan->N, m = x.numel() / K;
+        const int bits = static_cast<int>(plan->bits), gs = static_cast<int>(plan->gs);
+        const auto *p = plan->p;
+        auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
+        auto up = [&](int i) { return static_cast<const uint8_t *>(p[i]); };
+        at::DimVector sizes(x.sizes());
+        sizes.back() = N;
+        void *stream = stream_of(x);
+        if (strcmp(fmt, "hip_fused") == 0 || strcmp(fmt, "dequant_gemm") == 0) {
+            if (gs != 64) return none();
+            Tensor x_hat = empty({m * K}, at::kHalf, x.device());
+            Tensor y = empty(sizes, at::kFloat, x.device());
+            if (fmt[0] == 'h') {
+                check(arcq_linear_otf_ws(x.const_data_ptr(), ARCQ_F32, fp(A_THR), fp(A_CB), up(W_PACKED), fp(W_CB), fp(W_CENTER),
+                                         fp(W_SCALE), fp(W_SUM), fp(W_BIAS), x_hat.mutable_data_ptr(), nullptr,
+                                         y.mutable_data_ptr(), ARCQ_F32, m, N, K, bits, 64, stream));
+            } else {
+                const Tensor &dense = plan->slot[P_DENSE].use;
+                if (!dense.defined() || !f16(dense) || dense.numel() != N * K) return none();
+                check(arcq_act_quant_blocked(x.const_data_ptr(), ARCQ_F32, fp(A_THR), fp(A_CB), x_hat.mutable_data_ptr(), m, K, bits,
+                                             1.0e-6f, stream));
+                check(arcq_linear_fused_blocked(x_hat.const_data_ptr(), up(W_PACKED), fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM),
+                                                fp(W_BIAS), const_cast<void *>(dense.const_data_ptr()), 1, y.mutable_data_ptr(),
+                                                ARCQ_F32, m, N, K, bits, 64, stream));
+            }
+            return THPVariable_Wrap(std::move(y));
+        }
+        const bool bytes = strcmp(fmt, "u8") == 0;
+        if (!bytes && strcmp(fmt, "packed") != 0) return none();
+        const Tensor &table = plan->slot[P_TABLE].use;
+        if (!table.defined() || table.dim() != 2 || table.size(0) != table.size(1)) return none();
+        if (bytes && (!p[P_CODES] || plan->slot[P_CODES].use.numel() != N * K || plan->slot[P_CODES].use.scalar_type() != at::kByte))
+            return none();
+        const int levels = static_cast<int>(table.size(0));
+        const Tensor x2 = x.dim() == 2 ? x : x.view({m, K});
+        Quantized q = quantize(x2, fp(A_THR), fp(A_CB), bits, gs, bytes);
+        Tensor y = empty(sizes, at::kFloat, x.device());
+        float *yp = static_cast<float *>(y.mutable_data_ptr());
+        if (bytes)
+            check(arcq_linear_forward_u8(bptr(q.codes), fptr(q.center), fptr(q.scale), fptr(q.sum), up(P_CODES), fp(W_CENTER), fp(W_SCALE),
+                                         fp(W_SUM), fptr(table), fp(W_BIAS), yp, m, N, K, gs, levels, stream));
+        else
+            check(arcq_linear_forward_packed(bptr(q.codes), fptr(q.center), fptr(q.scale), fptr(q.sum), up(W_PACKED), fp(W_CENTER),
+                                             fp(W_SCALE), fp(W_SUM), fptr(table), fp(W_BIAS), yp, m, N, K, bits, gs, levels, stream));
+        return THPVariable_Wrap(std::move(y));
+    });
+}
+
+// patch_conv_forward(module, img): ARCQPackedPatchConv with 16 x 16 patches of three channels, group sizes 3 and 64
+PyObject *py_patch_conv_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    return guarded([&]() -> PyObject * {
+        const Tensor *xp = n == 2 ? as_tensor(args[1]) : nullptr;
+        if (!xp) return none();
+        const Tensor &x = *xp;
+        PyObject *dict;
+        Plan *plan = plan_of(args[0], Kind::Conv, dict);
+        int64_t ags, c;
+        PyObject *ks = get(dict, S.kernel_size);
+        if (!plan || plan->gs != 64 || !get_int(dict, S.act_group_size, ags) || ags != 3 || !get_int(dict, S.in_channels, c) || c != 3 ||
+            !ks || !PyTuple_Check(ks) || PyTuple_GET_SIZE(ks) != 2 || PyLong_AsLong(PyTuple_GET_ITEM(ks, 0)) != 16 ||
+            PyLong_AsLong(PyTuple_GET_ITEM(ks, 1)) != 16)
+            return none();
+        if (!here(x) || x.device().index() != plan->device || (!f16(x) && !f32(x)) || !x.is_contiguous() || x.dim() != 4 ||
+            x.size(1) != 3 || x.size(2) % 16 != 0 || x.size(3) % 16 != 0 || x.numel() == 0)
+            return none();
+        const int64_t b = x.size(0), hp = x.size(2) / 16, wp = x.size(3) / 16, m = b * hp * wp, N = plan->N, K = 768;
+        const int bits = static_cast<int>(plan->bits);
+        const bool blocked = m >= 512;
+        const auto *p = plan->p;
+        auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
+        const uint8_t *pw = static_cast<const uint8_t *>(p[W_PACKED]);
+        void *stream = stream_of(x);
+        Tensor rows = empty({m * K}, at::kHalf, x.device());
+        Tensor y = empty({b, hp, wp, N}, x.scalar_type(), x.device());
+        check(arcq_act_quant_patches(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), rows.mutable_data_ptr(), b, 3, x.size(2),
+                                     x.size(3), 16, bits, 1.0e-6f, blocked ? 1 : 0, stream));
+        if (blocked)
+            check(arcq_linear_fused_blocked(rows.const_data_ptr(), pw, fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), nullptr,
+                                            0, y.mutable_data_ptr(), code_of(y), m, N, K, bits, 64, stream));
+        else
+            check(arcq_linear_fused(rows.const_data_ptr(), pw, fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS),
+                                    y.mutable_data_ptr(), code_of(y), m, N, K, bits, 64, stream));
+        return THPVariable_Wrap(y.permute({0, 3, 1, 2}));
+    });
+}
+
+// register_types(layer, attention, mlp, gelu, layernorm, torch.nn.modules.module); None leaves an entry as it is
+PyObject *py_register_types(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    PyObject **const to[6] = {&g_layer_type, &g_attention_type, &g_mlp_type, &g_gelu_type, &g_layernorm_type, &g_torch_module};
+    for (Py_ssize_t i = 0; i < n && i < 6; ++i) {
+        if (args[i] == Py_None) continue;
+        Py_INCREF(args[i]);
+        Py_XDECREF(*to[i]);
+        *to[i] = args[i];
+    }
+    Py_RETURN_NONE;
+}
+
+#define FASTCALL(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f))
+PyMethodDef methods[] = {
+    {"layer_forward", FASTCALL(py_layer_forward), METH_FASTCALL, "one ARCQPackedLinearOnTheFly call, or None"},
+    {"block_forward", FASTCALL(py_block_forward), METH_FASTCALL, "one transformer block, or None"},
+    {"attention", FASTCALL(py_attention), METH_FASTCALL, "arcq_attention_fwd, or None"},
+    {"patch_embed", FASTCALL(py_patch_embed), METH_FASTCALL, "arcq_patch_embed_fwd, or None"},
+    {"quantize", FASTCALL(py_quantize), METH_FASTCALL, "arcq_act_quant to codes and metadata, or None"},
+    {"packed_forward", FASTCALL(py_packed_forward), METH_FASTCALL, "one ARCQPackedLinear call, or None"},
+    {"patch_conv_forward", FASTCALL(py_patch_conv_forward), METH_FASTCALL, "one ARCQPackedPatchConv call, or None"},
+    {"register_types", FASTCALL(py_register_types), METH_FASTCALL, "classes whose instances are recognised"},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_arcq_host", nullptr, -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__arcq_host(void)
+{
+#define X(n) S.n = PyUnicode_InternFromString(#n);
+    ARCQ_NAMES(X)
+#undef X
+    PlanType.tp_name = "arcq_vit_amd._arcq_host.Plan";
+    PlanType.tp_basicsize = sizeof(PlanObject);
+    PlanType.tp_flags = Py_TPFLAGS_DEFAULT;
+    PlanType.tp_new = plan_new;
+    PlanType.tp_dealloc = plan_dealloc;
+    PlanType.tp_methods = plan_methods;
+    PlanType.tp_getset = plan_getset;
+    if (PyType_Ready(&PlanType) < 0) return nullptr;
+    PyObject *m = PyModule_Create(&module_def);
+    if (!m) return nullptr;
+    Py_INCREF(&PlanType);
+    if (PyModule_AddObject(m, "Plan", reinterpret_cast<PyObject *>(&PlanType)) < 0) return nullptr;
+    return m;
+}

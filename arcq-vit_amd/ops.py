@@ -139,6 +139,9 @@ def quantize_activation(x: torch.Tensor, thresholds: torch.Tensor, codebook: tor
                         group_size: int) -> List[torch.Tensor]:
     """-> ``[packed u8 [rows, cols*bits/8], center, scale, code_sum f32 [rows, groups]]``
     (EXT/arcq_activation_kernel.cu:188-237)."""
+    out = _lib.host().quantize(x, thresholds, codebook, bits, group_size, False)
+    if out is not None:
+        return out
     packed, _, center, scale, code_sum = _act_quant(x, thresholds, codebook, bits, group_size, want_packed=True,
                                                     want_meta=True)
     return [packed, center, scale, code_sum]
@@ -147,6 +150,9 @@ def quantize_activation(x: torch.Tensor, thresholds: torch.Tensor, codebook: tor
 def quantize_activation_u8(x: torch.Tensor, thresholds: torch.Tensor, codebook: torch.Tensor, bits: int,
                            group_size: int) -> List[torch.Tensor]:
     """-> ``[codes u8 [rows, cols], center, scale, code_sum]`` (EXT/arcq_activation_kernel.cu:239-285)."""
+    out = _lib.host().quantize(x, thresholds, codebook, bits, group_size, True)
+    if out is not None:
+        return out
     _, codes, center, scale, code_sum = _act_quant(x, thresholds, codebook, bits, group_size, want_u8=True,
                                                    want_meta=True)
     return [codes, center, scale, code_sum]
@@ -403,6 +409,9 @@ def patch_embed_fwd(img: torch.Tensor, weight: torch.Tensor, bias: Optional[torc
     """Front end of a ViT in one launch (``arcq_patch_embed_fwd``): 16 x 16 stride-16 patch convolution of ``img``
     ``[B, 3, H, W]`` with ``weight`` ``[N, 3, 16, 16]`` and ``bias``, the class token in front, ``pos_embed`` added ->
     ``[B, 1 + patches, N]``; everything fp16, fp32 accumulation, rounded as the separate torch operations round."""
+    out = _lib.host().patch_embed(img, weight, bias, cls_token, pos_embed)
+    if out is not None:
+        return out
     _check(img.is_cuda and img.dtype == torch.float16 and img.dim() == 4 and img.shape[1] == 3,
            "img must be a CUDA fp16 tensor [B, 3, H, W]")
     _check(weight.is_cuda and weight.dtype == torch.float16 and weight.dim() == 4 and tuple(weight.shape[1:]) == (3, 16, 16),
@@ -430,6 +439,10 @@ def attention_fwd(qkv: torch.Tensor, heads: int, scale: Optional[float] = None,
     """Softmax attention on the qkv layer's output ``[B, n, 3 C]`` fp16 (q, k, v of head h at columns
     ``(0|1|2) C + 64 h``) -> ``[B, n, C]`` fp16, the proj layer's input, in one launch with no reshaping copies
     (``arcq_attention_fwd``: head dimension 64, at most 256 tokens).  ``scale`` defaults to ``1 / sqrt(64)``."""
+    if out is None:
+        y = _lib.host().attention(qkv, heads, 0.125 if scale is None else float(scale))
+        if y is not None:
+            return y
     _check(qkv.is_cuda and qkv.dtype == torch.float16 and qkv.dim() == 3, "qkv must be a CUDA fp16 tensor [B, n, 3 C]")
     _check(qkv.is_contiguous(), "qkv must be contiguous")
     b, n, c3 = qkv.shape

@@ -20,7 +20,7 @@ from typing import Dict, Optional
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import _lib, ops
 from .packed_linear import _pack, _quantize_weight_reference, _require_vector, infer_packed_hparams
 
 
@@ -153,6 +153,9 @@ class ARCQPackedPatchConv(nn.Module):
         return t.reshape(b * (h // kh) * (w // kw), c * kh * kw)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = _lib.host().patch_conv_forward(self, x)
+        if y is not None:
+            return y
         if x.dim() != 4 or x.shape[1] != self.in_channels:
             raise ValueError(f"expected input [B, {self.in_channels}, H, W], got {tuple(x.shape)}")
         kh, kw = self.kernel_size

@@ -17,7 +17,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import ops
+from . import _lib, ops
 from .pack_py import pack_codes_py, unpack_codes_py
 
 _FORMATS = ("packed", "u8", "dequant_gemm", "hip_fused")
@@ -214,6 +214,9 @@ class ARCQPackedLinear(nn.Module):
                 f"packed_weight_bytes={self.packed_weight_bytes}")
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = _lib.host().packed_forward(self, x)
+        if y is not None:
+            return y
         original_shape = x.shape
         if original_shape[-1] != self.in_features:
             raise ValueError(f"expected last dim {self.in_features}, got {original_shape[-1]}")

@@ -26,38 +26,17 @@ for these cases "same indices as the reference" is not pinned by any test):
 """
 from __future__ import annotations
 
-import ctypes
-from typing import Dict, Optional, Tuple
+from typing import Optional
 
 import torch
 import torch.nn as nn
 
 from . import _lib, ops
-from ._lib import ARCQ_F16, ARCQ_F32
-
-# Fallback fp16 x_hat workspace, one per (device, stream), for layers that were given no ``_x_hat_buffer``: layers
-# run back to back on a stream, and stream order makes the reuse safe.  Grown on demand; ``clear_workspaces()``
-# releases them.  Never used while a HIP graph is being captured: memory allocated during a capture belongs to
-# that graph's private pool, so a capture gets a buffer of its own (kept alive by the graph's pool) instead of
-# leaving one in this cache for a later capture to find.
-_workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
-
-
-def _workspace(device: torch.device, numel: int) -> torch.Tensor:
-    if torch.cuda.is_current_stream_capturing():
-        return torch.empty(max(numel, 1), dtype=torch.float16, device=device)
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(device).cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < numel:
-        ws = torch.empty(max(numel, 1), dtype=torch.float16, device=device)
-        _workspaces[key] = ws
-    return ws
 
 
 def clear_workspaces() -> None:
-    """Drop the fallback x_hat workspaces (they are re-created on demand)."""
-    _workspaces.clear()
+    """Kept for callers of earlier versions: scratch tensors come from torch's caching allocator call by call, so there is
+    nothing to drop (``torch.cuda.empty_cache()`` returns the memory)."""
 
 
 class ARCQPackedLinearOnTheFly(nn.Module):
@@ -93,37 +72,10 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         else:
             self.register_buffer("bias_tensor", torch.empty(0))
         self.out_dtype = torch.float16
-        self._prep = None
+        self._host_plan = None      # the host extension's view of the buffers above, made by the first forward
         # Opt-in: operands rounded to FP8 and the product on FP8 matrix units (ops.linear_otf_fp8).  Faster on the
         # large models, not the reference's numerics; see set_fp8_operands in packed_convert.
         self.fp8_operands = False
-        self._fp8_mult = None
-
-    def _prepare(self):
-        """Validated, fp32-contiguous views of the buffers and their raw pointers, built once and reused by every
-        forward until a buffer moves (``_apply``, ``load_state_dict``), is replaced or is written in place."""
-        a = [ops._f32c(self.activation_thresholds), ops._f32c(self.activation_codebook)]
-        w = [self.packed_weight_codes.contiguous(), ops._f32c(self.weight_codebook), ops._f32c(self.weight_center),
-             ops._f32c(self.weight_scale), ops._f32c(self.weight_code_sum)]
-        bias = ops._f32c(self.bias_tensor) if self.bias_tensor.numel() > 0 else None
-        keep = a + w + [bias]
-        self._prep = (keep, tuple(0 if t is None else t.data_ptr() for t in keep), self._buffers_key(),
-                      self.packed_weight_codes.device)
-        return self._prep
-
-    _PREP_BUFFERS = ("activation_thresholds", "activation_codebook", "packed_weight_codes", "weight_codebook",
-                     "weight_center", "weight_scale", "weight_code_sum", "bias_tensor")
-
-    def _buffers_key(self):
-        """Identity and version of every buffer the cached pointers were made from: replacing a buffer or writing into
-        one in place changes it, and the next forward prepares again."""
-        b = self._buffers
-        return tuple((b[n].data_ptr(), b[n]._version) for n in self._PREP_BUFFERS)
-
-    def _load_from_state_dict(self, *args, **kwargs):
-        self._prep = None
-        self._fp8_mult = None
-        return super()._load_from_state_dict(*args, **kwargs)
 
     @classmethod
     def from_packed(cls, packed_layer: nn.Module) -> "ARCQPackedLinearOnTheFly":
@@ -142,7 +94,6 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         # then widens these buffers again, scripts/benchmark_arcq_on_the_fly.py:63-85, which leaves
         # them rounded to fp16.)  Device moves still apply; dtype changes of these buffers do not.
         keep = {n: self._buffers[n] for n in self._FP32_BUFFERS if self._buffers.get(n) is not None}
-        self._prep = None
         super()._apply(fn, *args, **kwargs)
         for name, orig in keep.items():
             new = self._buffers[name]
@@ -180,6 +131,15 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         operations otherwise; without them this is the reference module's forward.  ``quantize_for=consumer`` (see
         ``can_quantize_for``): the result is the consumer's ``x_hat`` instead of this layer's output, to be passed to
         ``consumer(..., input_is_xhat=True)``, which skips its own stage 1."""
+        y = _lib.host().layer_forward(self, x, layernorm, activation == "gelu", residual, quantize_for, input_is_xhat) \
+            if activation is None or activation == "gelu" else None
+        if y is not None:
+            return y
+        return self._forward_general(x, layernorm, activation, residual, quantize_for, input_is_xhat)
+
+    def _forward_general(self, x, layernorm, activation, residual, quantize_for, input_is_xhat) -> torch.Tensor:
+        """Calls the host extension does not take as they are: arguments are checked, converted to what it takes
+        (contiguous fp16 / fp32 tensors, the tensor's device current), and parts that do not fuse run as torch operations."""
         original_shape = x.shape
         if original_shape[-1] != self.in_features:
             raise ValueError(f"expected last dim {self.in_features}, got {original_shape[-1]}")
@@ -198,6 +158,7 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         if input_is_xhat and (x2.dtype != torch.float16 or layernorm is not None or self.fp8_operands):
             raise ValueError("input_is_xhat: x must be the float16 x_hat a producer made for this layer")
         ln_fusable = layernorm is None or (self.in_features <= (1024 if m >= 512 else 1536) and layernorm.elementwise_affine
+                                           and type(layernorm) is nn.LayerNorm
                                            and tuple(layernorm.normalized_shape) == (self.in_features,))
         if chain and not ln_fusable:     # (a chained call cannot fall back as a whole: only the LayerNorm runs apart)
             x2, layernorm, ln_fusable = layernorm(x2).contiguous(), None, True
@@ -213,89 +174,34 @@ class ARCQPackedLinearOnTheFly(nn.Module):
             if residual is not None:
                 y = y + residual.reshape(-1, self.out_features)
             return y.reshape(*original_shape[:-1], self.out_features)
-        prep = self._prep
-        if prep is None or prep[2] != self._buffers_key():
-            prep = self._prepare()
-            self._fp8_mult = None
-        if prep[3] != x2.device:
+        if self.packed_weight_codes.device != x2.device:
             raise RuntimeError("x and the layer's buffers must be on the same device")
-        if self.fp8_operands:
-            if self.group_size != 64:
-                raise ValueError("fp8_operands needs group_size 64")
-            if self._fp8_mult is None:          # (reads the metadata back once per layer)
-                self._fp8_mult = ops.fp8_weight_multiplier(self.weight_codebook, self.weight_center, self.weight_scale,
-                                                           self.weight_code_sum)
-            t = prep[0]
-            y = ops.linear_otf_fp8(x2, t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], self.bits,
-                                   out_dtype=self.out_dtype, w_mult=self._fp8_mult)
-            return y.reshape(*original_shape[:-1], self.out_features)
-        ws = getattr(self, "_x_hat_buffer", None)       # a buffer the model owns (packed_convert.share_buffers)
-        if ws is None or ws.numel() < x2.numel() or ws.device != x2.device:
-            ws = _workspace(x2.device, x2.numel())
+        if m == 0:
+            return torch.empty((*original_shape[:-1], self.out_features), dtype=self.out_dtype, device=x2.device)
         w_ws = getattr(self, "_weight_buffer", None)
         if w_ws is not None and (not w_ws.is_cuda or w_ws.dtype != torch.float16 or not w_ws.is_contiguous()
-                                 or w_ws.numel() < self.out_features * self.in_features):
+                                 or w_ws.numel() < self.out_features * self.in_features or w_ws.device != x2.device):
             raise ValueError("_weight_buffer must be a contiguous float16 CUDA tensor of at least "
                              "out_features * in_features elements")
-        y = torch.empty((m, self.out_features), dtype=self.out_dtype, device=x2.device)
-        p = prep[1]
-        f16 = ARCQ_F16 if x2.dtype == torch.float16 else ARCQ_F32
-        y16 = ARCQ_F16 if self.out_dtype == torch.float16 else ARCQ_F32
-        stream = torch.cuda.current_stream().cuda_stream
+        if residual is not None:
+            r2 = residual.reshape(-1, self.out_features)
+            if r2.dtype != self.out_dtype or tuple(r2.shape) != (m, self.out_features) or r2.device != x2.device:
+                raise ValueError("residual must have the output's shape, dtype and device")
+            residual = r2.contiguous()
+        host = _lib.host()
+        call = (self, x2, layernorm, activation == "gelu", residual, quantize_for, bool(input_is_xhat))
         with torch.cuda.device(x2.device):
-            if not extras:
-                _lib.check(_lib.load().arcq_linear_otf_ws(
-                    x2.data_ptr(), f16, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], ws.data_ptr(),
-                    0 if w_ws is None else w_ws.data_ptr(), y.data_ptr(), y16, m, self.out_features, self.in_features,
-                    self.bits, self.group_size, stream))
-            else:
-                a = _lib.LinearExArgs()
-                a.struct_size = ctypes.sizeof(_lib.LinearExArgs)
-                a.x_dtype, a.y_dtype, a.bits, a.group_size = f16, y16, self.bits, self.group_size
-                a.M, a.N, a.K = m, self.out_features, self.in_features
-                a.x = x2.data_ptr()
-                keep = []
-                if layernorm is not None:
-                    lw, lb = self._layernorm_params(layernorm)
-                    keep = [lw, lb]
-                    a.producer, a.ln_weight, a.ln_bias, a.ln_eps = (_lib.ARCQ_PRODUCER_LAYERNORM, lw.data_ptr(),
-                                                                   lb.data_ptr(), float(layernorm.eps))
-                a.activation = _lib.ARCQ_ACT_GELU if activation == "gelu" else _lib.ARCQ_ACT_NONE
-                (a.a_thresholds, a.a_codebook, a.packed_w, a.w_codebook, a.w_center, a.w_scale, a.w_code_sum,
-                 a.bias) = [v or None for v in p]
-                if input_is_xhat:
-                    a.producer = _lib.ARCQ_PRODUCER_XHAT
-                if quantize_for is not None:
-                    nprep = quantize_for._prep
-                    if nprep is None or nprep[2] != quantize_for._buffers_key():
-                        nprep = quantize_for._prepare()
-                        quantize_for._fp8_mult = None
-                    a.next_a_thresholds, a.next_a_codebook = nprep[1][0], nprep[1][1]
-                if residual is not None:
-                    r2 = residual.reshape(-1, self.out_features)
-                    if r2.dtype != self.out_dtype or tuple(r2.shape) != (m, self.out_features) or r2.device != x2.device:
-                        raise ValueError("residual must have the output's shape, dtype and device")
-                    r2 = r2.contiguous()
-                    keep.append(r2)
-                    a.residual = r2.data_ptr()
-                a.x_hat_ws, a.w_hat_ws, a.y = ws.data_ptr(), (None if w_ws is None else w_ws.data_ptr()), y.data_ptr()
-                _lib.check(_lib.load().arcq_linear_otf_ex(ctypes.byref(a), stream))
+            y = host.layer_forward(*call)
+            if y is None and self.fp8_operands:
+                if self.group_size != 64:
+                    raise ValueError("fp8_operands needs group_size 64")
+                # (reads the metadata back once per layer; the extension forgets it when a buffer changes)
+                self._host_plan.fp8_mult = ops.fp8_weight_multiplier(self.weight_codebook, self.weight_center,
+                                                                     self.weight_scale, self.weight_code_sum)
+                y = host.layer_forward(*call)
+        if y is None:
+            raise RuntimeError("x and the layer's buffers must be contiguous CUDA tensors of the types the layer was built with")
         return y.reshape(*original_shape[:-1], self.out_features)
-
-    def _layernorm_params(self, layernorm: nn.LayerNorm):
-        """fp32 copies of a LayerNorm's weight and bias, cached per LayerNorm module and parameter version."""
-        cache = self.__dict__.setdefault("_ln_cache", {})
-        key = id(layernorm)
-        ver = (layernorm.weight._version, layernorm.weight.data_ptr(),
-               None if layernorm.bias is None else layernorm.bias._version)
-        hit = cache.get(key)
-        if hit is None or hit[0] != ver:
-            w = layernorm.weight.detach().to(torch.float32).contiguous()
-            b = (torch.zeros_like(w) if layernorm.bias is None
-                 else layernorm.bias.detach().to(torch.float32).contiguous())
-            hit = (ver, w, b)
-            cache[key] = hit
-        return hit[1], hit[2]
 
     def estimated_persistent_mb(self) -> float:
         """MiB held by this layer's buffers (FQ/arcq_packed_on_the_fly.py:163-169)."""

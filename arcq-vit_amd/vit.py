@@ -16,6 +16,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _lib
 from .packed_convert import (convert_arcq_conv_to_packed, convert_arcq_linear_to_packed, share_buffers,
                              to_on_the_fly)
 from .quant_source import QuantConv2dPCARCQ, QuantLinearLSQ, QuantLinearPCARCQ
@@ -84,6 +85,11 @@ class Block(nn.Module):
         self.chain_mlp = True
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # The whole block from the host extension where every part is the plain case (packed layers, no hooks on the
+        # modules it would call): the same operations in the same order, without the interpreter between them.
+        y = _lib.host().block_forward(self, x) if x.is_cuda else None
+        if y is not None:
+            return y
         if self.fuse_elementwise and isinstance(self.mlp.act, nn.GELU) and self.mlp.act.approximate == "none":
             a = self.attn
             x = a.proj(a.mix(a.qkv(x, layernorm=self.norm1)), residual=x)
