@@ -37,6 +37,27 @@ class LinearExArgs(ctypes.Structure):
                 ("next_a_thresholds", ctypes.c_void_p), ("next_a_codebook", ctypes.c_void_p)]
 
 
+class PrepareWeights(ctypes.Structure):
+    """``arcq_prepare_weights`` of include/arcq_hip.h."""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("packed", "codebook", "center", "scale", "code_sum", "w_hat")] + [
+        ("N", ctypes.c_int64), ("K", ctypes.c_int64), ("row_major", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+
+
+class PrepareArgs(ctypes.Structure):
+    """``arcq_prepare_args``."""
+    _fields_ = [("x_dtype", ctypes.c_int32), ("bits", ctypes.c_int32), ("ln_eps", ctypes.c_float), ("reserved", ctypes.c_int32),
+                ("rows", ctypes.c_int64), ("K", ctypes.c_int64)] + [
+        (n, ctypes.c_void_p) for n in ("x", "ln_weight", "ln_bias", "thresholds", "codebook", "x_hat")] + [
+        ("weights", PrepareWeights * 2)]
+
+
+class LinearPreparedArgs(ctypes.Structure):
+    """``arcq_linear_prepared_args``."""
+    _fields_ = [(n, ctypes.c_int32) for n in ("y_dtype", "activation", "next_bits", "w_row_major")] + [
+        (n, ctypes.c_int64) for n in ("M", "N", "K")] + [
+        (n, ctypes.c_void_p) for n in ("x_hat", "w_hat", "bias", "residual", "next_thresholds", "next_codebook", "y")]
+
+
 ARCQ_PRODUCER_NONE, ARCQ_PRODUCER_LAYERNORM, ARCQ_PRODUCER_XHAT = 0, 1, 2
 ARCQ_ACT_NONE, ARCQ_ACT_GELU = 0, 1
 
@@ -61,6 +82,9 @@ _SIGNATURES = {
                                _c_ptr, _c_int, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_ptr],
     "arcq_linear_otf_ex": [ctypes.POINTER(LinearExArgs), _c_ptr],
     "arcq_xhat_layout": [_c_i64],
+    "arcq_prepared_row_major": [_c_i64, _c_i64, _c_i64],
+    "arcq_prepare": [ctypes.POINTER(PrepareArgs), _c_ptr],
+    "arcq_linear_prepared": [ctypes.POINTER(LinearPreparedArgs), _c_ptr],
     "arcq_act_quant_blocked_ln": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_f32, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_int,
                                   _c_f32, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr],
     "arcq_act_quant_blocked": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_int, _c_f32, _c_ptr],
@@ -78,6 +102,7 @@ _SIGNATURES = {
     "arcq_act_quant_patches": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_f32,
                                _c_int, _c_ptr],
     "arcq_patch_embed_fwd": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr],
+    "arcq_attention_quant_fwd": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, _c_ptr],
     "arcq_attention_fwd": [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, _c_ptr],
     "arcq_linear_forward_packed": [_c_ptr] * 11 + [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_ptr],
     "arcq_linear_forward_u8": [_c_ptr] * 11 + [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_ptr],

@@ -356,13 +356,13 @@ __device__ __forceinline__ void next_quant_setup(const float *__restrict__ thr, 
 }
 
 // One staged chunk (32 rows x 64 fp16 values, the rows `pitch` bytes apart) -> x_hat of the consuming layer.
-// `gelu`: the exact GELU of the staged (rounded) values first, rounded to fp16 again.  dst_block = base of the chunk's
-// 32-row block in the consumer's block layout, `rows` = rows of that block (32, or fewer for a last block),
-// piece0 = index of the chunk's first 16-byte piece (column / 8).  The whole wave calls it.
+// `gelu`: the exact GELU of the staged (rounded) values first, rounded to fp16 again.  dst = the chunk's first 16-byte
+// piece of this lane's row (lane / 2) in the consumer's block layout, whose pieces are `rows` rows apart; `live` = whether
+// the row is stored.  The whole wave calls it.
 template <int BITS>
-__device__ __forceinline__ void next_quant_chunk(const unsigned char *lds, int nwaves,
-                                                 const unsigned char *stage, int pitch, int lane, bool gelu, float eps,
-                                                 __half *dst_block, int rows, int piece0)
+__device__ __forceinline__ void next_quant_rows(const unsigned char *lds, int nwaves,
+                                                const unsigned char *stage, int pitch, int lane, bool gelu, float eps,
+                                                __half *dst, int rows, bool live)
 {
     typedef uint32_t u32x4_nq __attribute__((ext_vector_type(4)));
     constexpr int L = 1 << BITS;
@@ -404,9 +404,19 @@ __device__ __forceinline__ void next_quant_chunk(const unsigned char *lds, int n
             const __half2 h = __floats2half2_rn(fma_f32(s, v[j] - code_mean, mu), fma_f32(s, v[j + 1] - code_mean, mu));
             o[d] = *reinterpret_cast<const uint32_t *>(&h);
         }
-        if (r < rows)
-            store_writethrough16(dst_block + (static_cast<int64_t>(piece0 + hf * 4 + i) * rows + r) * 8, o[0], o[1], o[2], o[3]);
+        if (live) store_writethrough16(dst + static_cast<int64_t>(hf * 4 + i) * rows * 8, o[0], o[1], o[2], o[3]);
     }
+}
+
+// The same for a chunk whose 32 rows are one block of the consumer's layout: dst_block = base of that block, `rows` = its
+// rows (32, or fewer for a last block), piece0 = index of the chunk's first 16-byte piece (column / 8).
+template <int BITS>
+__device__ __forceinline__ void next_quant_chunk(const unsigned char *lds, int nwaves,
+                                                 const unsigned char *stage, int pitch, int lane, bool gelu, float eps,
+                                                 __half *dst_block, int rows, int piece0)
+{
+    const int r = lane >> 1;
+    next_quant_rows<BITS>(lds, nwaves, stage, pitch, lane, gelu, eps, dst_block + (static_cast<int64_t>(piece0) * rows + r) * 8, rows, r < rows);
 }
 
 }  // namespace arcq

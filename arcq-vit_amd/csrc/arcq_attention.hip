@@ -18,7 +18,7 @@
 // rounded to fp16, ARE the second operand of O^T = V^T P^T for the keys {16 s + 4 h + c, 16 s + 8 + 4 h + c}; the
 // matching eight values of V^T are two 8-byte LDS reads.  fp32 scores, softmax and accumulation; P rounded to fp16;
 // normalisation by the row sum at the end.  Beyond 128 keys the keys go in two chunks with a running maximum and sum.
-#include "arcq_common.h"
+#include "arcq_act_quant_core.h"
 
 namespace arcq {
 namespace {
@@ -32,9 +32,15 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 constexpr int kHeadDim = 64;
 constexpr int kKPitch = kHeadDim * 2 + 16;          // bytes per key row of K in LDS
 
-template <int NKB>      // 32-key blocks (= 32-query tiles = waves): ceil(n / 32)
+// NKB = 32-key blocks (= 32-query tiles = waves): ceil(n / 32).
+// NQ = 0, or the bits of the proj layer's activation quantizer: `out` then receives that layer's x_hat (stage 1 of the
+// rounded output; a head's 64 dims are one quantization group) in the 32-row block layout of the [B n, C] tensor instead of
+// the output.  A wave's 32 x 64 outputs go through its own 32 rows of K in LDS (all waves are done with it) into the
+// lane-pair routine of the GEMM epilogues.
+template <int NKB, int NQ>
 __global__ void __launch_bounds__(64 * NKB) __attribute__((amdgpu_waves_per_eu(4)))     // two workgroups of up to 8 waves on a CU
-attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n, int H, float scale)
+attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n, int H, float scale,
+                 const float *__restrict__ nq_thr, const float *__restrict__ nq_cb, int total_rows)
 {
     constexpr int kKeys = 32 * NKB;
     // bytes per dim row of V^T in LDS: the row stride in dwords is 2 mod 4, which spreads both the transposing writes
@@ -44,6 +50,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
     constexpr int NCH = (NKB + CH - 1) / CH;
     __shared__ __attribute__((aligned(16))) unsigned char ks[kKeys * kKPitch];
     __shared__ __attribute__((aligned(16))) unsigned char vt[kHeadDim * kVPitch];
+    __shared__ __attribute__((aligned(16))) unsigned char nq_lds[NQ ? next_quant_lds_bytes(NQ ? NQ : 2) : 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lh = lane >> 5;
     const int h = blockIdx.x, b = blockIdx.y;
@@ -66,6 +73,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
             vreg[i][j] = key < n ? *reinterpret_cast<const u32x4_t *>(src + C) : zero4;
         }
     }
+    if constexpr (NQ != 0) next_quant_setup<NQ>(nq_thr, nq_cb, nq_lds, tid, 64 * NKB);       // while K and V are on their way
     // ---- this wave's queries: lane (q, half) holds Q[q][16 kk + 8 half ... + 7] for kk = 0..3 ----
     const int q = wave * 32 + lr;
     u32x4_t qf[4];
@@ -173,6 +181,31 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
         }
     }
     l += __shfl_xor(l, 32);
+    if constexpr (NQ != 0) {
+        __syncthreads();                                     // everyone is done with K
+        unsigned char *stage = ks + wave * 32 * kKPitch;
+        const float inv = 1.0f / l;
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const __half2 a = __floats2half2_rn(oacc[jb][4 * t] * inv, oacc[jb][4 * t + 1] * inv);
+                const __half2 c = __floats2half2_rn(oacc[jb][4 * t + 2] * inv, oacc[jb][4 * t + 3] * inv);
+                u32x2_t pk;
+                pk[0] = *reinterpret_cast<const uint32_t *>(&a);
+                pk[1] = *reinterpret_cast<const uint32_t *>(&c);
+                *reinterpret_cast<u32x2_t *>(stage + lr * kKPitch + (jb * 32 + 8 * t + 4 * lh) * 2) = pk;
+            }
+        __builtin_amdgcn_wave_barrier();
+        // This lane's row of the chunk (rows past the image's last query: zero scores of zero queries, not stored).
+        const int qr = wave * 32 + (lane >> 1);
+        const int64_t row = row0 + qr;
+        const int blk = static_cast<int>(row >> 5);
+        const int nrows = min(32, total_rows - blk * 32);
+        next_quant_rows<NQ>(nq_lds, NKB, stage, kKPitch, lane, false, 1.0e-6f,
+                            out + static_cast<int64_t>(blk) * 32 * C + (static_cast<int64_t>(h) * 8 * nrows + (row & 31)) * 8, nrows, qr < n);
+        return;
+    }
     // ---- normalise, round, store: each lane 4 runs of 4 consecutive dims per 32-dim block ----
     if (q < n) {
         const float inv = 1.0f / l;
@@ -191,11 +224,48 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
     }
 }
 
-template <int NKB>
-void launch_attention(const void *qkv, void *out, int B, int n, int H, float scale, hipStream_t stream)
+template <int NKB, int NQ>
+void launch_attention(const void *qkv, void *out, int B, int n, int H, float scale, const float *thr, const float *cb, hipStream_t stream)
 {
-    hipLaunchKernelGGL((attention_kernel<NKB>), dim3(H, B), dim3(64 * NKB), 0, stream, static_cast<const __half *>(qkv),
-                       static_cast<__half *>(out), n, H, scale);
+    hipLaunchKernelGGL((attention_kernel<NKB, NQ>), dim3(H, B), dim3(64 * NKB), 0, stream, static_cast<const __half *>(qkv),
+                       static_cast<__half *>(out), n, H, scale, thr, cb, B * n);
+}
+
+template <int NQ>
+void launch_attention_n(const void *qkv, void *out, int B, int n, int H, float scale, const float *thr, const float *cb, hipStream_t st)
+{
+    switch ((n + 31) / 32) {
+    case 1: launch_attention<1, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 2: launch_attention<2, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 3: launch_attention<3, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 4: launch_attention<4, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 5: launch_attention<5, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 6: launch_attention<6, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 7: launch_attention<7, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    default: launch_attention<8, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    }
+}
+
+int attention_checked(const char *fn, const void *qkv, void *out, int64_t B, int64_t n, int64_t H, int64_t head_dim, float scale,
+                      int nq_bits, const float *thr, const float *cb, void *stream)
+{
+    if (B < 0 || n < 0 || H < 0) return fail(ARCQ_ERR_SHAPE, "%s: negative size", fn);
+    if (!(scale > 0.0f)) return fail(ARCQ_ERR_UNSUPPORTED, "%s: scale must be positive", fn);
+    if (head_dim != kHeadDim) return fail(ARCQ_ERR_UNSUPPORTED, "%s: head_dim must be 64 (got %lld)", fn, static_cast<long long>(head_dim));
+    if (n > 256) return fail(ARCQ_ERR_UNSUPPORTED, "%s: at most 256 tokens (got %lld)", fn, static_cast<long long>(n));
+    if (B * n * H == 0) return ARCQ_OK;
+    if (!qkv || !out || (nq_bits && (!thr || !cb))) return fail(ARCQ_ERR_NULL, "%s: NULL tensor pointer", fn);
+    if (!aligned(qkv, 16) || !aligned(out, nq_bits ? 16 : 8))
+        return fail(ARCQ_ERR_ALIGN, "%s: qkv must be 16-byte, out %d-byte aligned", fn, nq_bits ? 16 : 8);
+    if (B > 65535 || H > (1 << 20) || B * n * 3 * H * head_dim >= (int64_t(1) << 40))
+        return fail(ARCQ_ERR_SHAPE, "%s: tensor too large", fn);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int b = static_cast<int>(B), nn = static_cast<int>(n), hh = static_cast<int>(H);
+    if (nq_bits == 0) launch_attention_n<0>(qkv, out, b, nn, hh, scale, thr, cb, st);
+    else if (nq_bits == 4) launch_attention_n<4>(qkv, out, b, nn, hh, scale, thr, cb, st);
+    else if (nq_bits == 3) launch_attention_n<3>(qkv, out, b, nn, hh, scale, thr, cb, st);
+    else launch_attention_n<2>(qkv, out, b, nn, hh, scale, thr, cb, st);
+    return launch_status(fn);
 }
 
 }  // namespace
@@ -206,26 +276,13 @@ using namespace arcq;
 ARCQ_API int arcq_attention_fwd(const void *qkv, void *out, int64_t B, int64_t n, int64_t H, int64_t head_dim, float scale,
                                 void *stream)
 {
-    if (B < 0 || n < 0 || H < 0) return fail(ARCQ_ERR_SHAPE, "arcq_attention_fwd: negative size");
-    if (!(scale > 0.0f)) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_attention_fwd: scale must be positive");
-    if (head_dim != kHeadDim) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_attention_fwd: head_dim must be 64 (got %lld)", static_cast<long long>(head_dim));
-    if (n > 256) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_attention_fwd: at most 256 tokens (got %lld)", static_cast<long long>(n));
-    if (B * n * H == 0) return ARCQ_OK;
-    if (!qkv || !out) return fail(ARCQ_ERR_NULL, "arcq_attention_fwd: NULL tensor pointer");
-    if (!aligned(qkv, 16) || !aligned(out, 8)) return fail(ARCQ_ERR_ALIGN, "arcq_attention_fwd: qkv must be 16-byte, out 8-byte aligned");
-    if (B > 65535 || H > (1 << 20) || B * n * 3 * H * head_dim >= (int64_t(1) << 40))
-        return fail(ARCQ_ERR_SHAPE, "arcq_attention_fwd: tensor too large");
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const int b = static_cast<int>(B), nn = static_cast<int>(n), hh = static_cast<int>(H);
-    switch ((nn + 31) / 32) {
-    case 1: launch_attention<1>(qkv, out, b, nn, hh, scale, st); break;
-    case 2: launch_attention<2>(qkv, out, b, nn, hh, scale, st); break;
-    case 3: launch_attention<3>(qkv, out, b, nn, hh, scale, st); break;
-    case 4: launch_attention<4>(qkv, out, b, nn, hh, scale, st); break;
-    case 5: launch_attention<5>(qkv, out, b, nn, hh, scale, st); break;
-    case 6: launch_attention<6>(qkv, out, b, nn, hh, scale, st); break;
-    case 7: launch_attention<7>(qkv, out, b, nn, hh, scale, st); break;
-    default: launch_attention<8>(qkv, out, b, nn, hh, scale, st); break;
-    }
-    return launch_status("arcq_attention_fwd");
+    return attention_checked("arcq_attention_fwd", qkv, out, B, n, H, head_dim, scale, 0, nullptr, nullptr, stream);
+}
+
+ARCQ_API int arcq_attention_quant_fwd(const void *qkv, const float *thresholds, const float *codebook, int bits, void *x_hat,
+                                      int64_t B, int64_t n, int64_t H, int64_t head_dim, float scale, void *stream)
+{
+    if (!bits_ok(bits)) return fail(ARCQ_ERR_BITS, "arcq_attention_quant_fwd: bits must be 2, 3, or 4");
+    if (B * n >= (int64_t(1) << 26)) return fail(ARCQ_ERR_SHAPE, "arcq_attention_quant_fwd: tensor too large");
+    return attention_checked("arcq_attention_quant_fwd", qkv, x_hat, B, n, H, head_dim, scale, bits, thresholds, codebook, stream);
 }

@@ -58,6 +58,10 @@ int linear_fused_blocked(const void *x_hat_blocked, const uint8_t *packed_w, con
 // GPU); what the weight-stationary kernels size their row ranges by (one workgroup per compute unit).
 int device_cus();
 
+// Prepared operands (arcq_prepare): g.x_hat in the 32-row block layout, w_hat in the 32-column block layout; N a multiple
+// of 32, K of 64.
+void launch_gemm_tile(const GemmArgs &g, const void *w_hat, hipStream_t stream);
+
 // Small-M kernel (64 x 64 tiles, K split across the waves of a workgroup); requires K >= 64.
 void launch_gemm_splitk(const GemmArgs &g, hipStream_t stream);
 // arcq_linear_fused with GELU / a residual ([M,N] of y's type) on the rounded outputs; with either set it needs the

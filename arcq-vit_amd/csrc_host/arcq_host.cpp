@@ -21,6 +21,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
+#include <algorithm>
 #include <cstring>
 #include <optional>
 #include <string>
@@ -266,6 +267,69 @@ bool can_quantize(PyObject *da, const Plan &a, PyObject *db, const Plan &b, int6
     return strncmp(arcq_linear_otf_ws_kernel(rows, a.N, a.K, 1), "otf_rows", 8) != 0;
 }
 
+// ---- prepared operands: stage 1 and the weights in one launch, then the product -----------------------------------------
+struct Weights {                 // w_hat of one layer inside a scratch tensor
+    void *ptr;
+    bool row_major;
+};
+// Fields of arcq_prepare_args for a layer's own tensors.
+void set_weights(arcq_prepare_weights &w, const Plan &p, const Weights &out)
+{
+    w.packed = static_cast<const uint8_t *>(p.p[W_PACKED]);
+    w.codebook = static_cast<const float *>(p.p[W_CB]), w.center = static_cast<const float *>(p.p[W_CENTER]);
+    w.scale = static_cast<const float *>(p.p[W_SCALE]), w.code_sum = static_cast<const float *>(p.p[W_SUM]);
+    w.w_hat = out.ptr, w.N = p.N, w.K = p.K, w.row_major = out.row_major ? 1 : 0;
+}
+void run_prepare(const Tensor &x, int64_t rows, const Plan &first, const LayerNormParams *ln, float ln_eps, void *x_hat, const Weights &w_first,
+                 const Plan *second, const Weights *w_second, void *stream)
+{
+    arcq_prepare_args a = {};
+    a.x_dtype = code_of(x);
+    a.bits = static_cast<int32_t>(first.bits);
+    a.rows = rows, a.K = first.K;
+    a.x = x.const_data_ptr();
+    if (ln) a.ln_weight = fptr(ln->w.use), a.ln_bias = fptr(ln->b.use), a.ln_eps = ln_eps;
+    a.thresholds = static_cast<const float *>(first.p[A_THR]), a.codebook = static_cast<const float *>(first.p[A_CB]);
+    a.x_hat = x_hat;
+    set_weights(a.weights[0], first, w_first);
+    if (second) set_weights(a.weights[1], *second, *w_second);
+    check(arcq_prepare(&a, stream));
+}
+void run_product(const Plan &p, int64_t rows, const void *x_hat, const Weights &w, const Tensor *residual, bool gelu, const Plan *next,
+                 void *y, int y_dtype, void *stream)
+{
+    arcq_linear_prepared_args a = {};
+    a.y_dtype = y_dtype;
+    a.activation = gelu ? ARCQ_ACT_GELU : ARCQ_ACT_NONE;
+    a.w_row_major = w.row_major ? 1 : 0;
+    a.M = rows, a.N = p.N, a.K = p.K;
+    a.x_hat = x_hat, a.w_hat = w.ptr;
+    a.bias = static_cast<const float *>(p.p[W_BIAS]);
+    if (residual) a.residual = residual->const_data_ptr();
+    if (next) {
+        a.next_thresholds = static_cast<const float *>(next->p[A_THR]), a.next_codebook = static_cast<const float *>(next->p[A_CB]);
+        a.next_bits = static_cast<int32_t>(next->bits);
+    }
+    a.y = y;
+    check(arcq_linear_prepared(&a, stream));
+}
+bool can_prepare(const Plan &p, int64_t rows)
+{
+    return p.gs == 64 && p.K % 64 == 0 && p.N % 32 == 0 && rows * p.K < (int64_t(1) << 31) && p.N * p.K < (int64_t(1) << 31) &&
+           rows < (int64_t(1) << 26);
+}
+// Whether one layer call runs as prepare + product.  Below 512 rows from K = 768 on (up to 512 inputs the one-launch kernel
+// is 1 us faster: 7.7 against 9.6 us at 197 x 384 x 384; 12.9 against 11.1 at 2 304 x 768, 43 against 16.5 with a LayerNorm
+// at 3 072 x 1 024); above wherever the tile kernels run the product and no one-launch kernel would (1 000 rows: 384 -> 1 152
+// 13.1 -> 12.0 us, 1 024 -> 3 072 32 -> 19, 4 096 -> 1 024 51 -> 32).
+bool prepare_pays(const Plan &p, int64_t rows, bool f16_input, bool has_ws, bool layernorm)
+{
+    if (!can_prepare(p, rows) || (layernorm && p.K > 2048)) return false;
+    if (rows < 512) return p.K >= 768;
+    if (arcq_prepared_row_major(rows, p.N, p.K)) return false;
+    return !(f16_input && has_ws && strncmp(arcq_linear_otf_ws_kernel(rows, p.N, p.K, 1), "otf_rows", 8) == 0);
+}
+
 std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Options &o)
 {
     PyObject *dict;
@@ -286,7 +350,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
     if (extras) {
         if (fp8 || plan->gs != 64 || K % 64 != 0) return std::nullopt;
         if (o.layernorm) {
-            if (K > (m >= 512 ? 1024 : 1536)) return std::nullopt;
+            if (K > 1024 && (K > 1536 || m >= 512)) return std::nullopt;
             ln = layernorm_params(*plan, o.layernorm, ln_eps);
             if (!ln) return std::nullopt;
         }
@@ -324,6 +388,18 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
         if (!w_ws || !w_ws->is_cuda() || !f16(*w_ws) || !w_ws->is_contiguous() || w_ws->numel() < N * K ||
             w_ws->device() != x.device())
             return std::nullopt;
+    }
+    if (!next && !o.x_is_xhat && prepare_pays(*plan, m, f16(x), w_ws != nullptr, ln != nullptr)) {
+        // (x_hat and w_hat in one scratch tensor; w_hat first: 512-byte runs stay aligned)
+        const bool lent = w_ws != nullptr;
+        Tensor scratch = empty({(lent ? 0 : N * K) + m * K}, at::kHalf, x.device());
+        char *base = static_cast<char *>(scratch.mutable_data_ptr());
+        const Weights w{lent ? w_ws->mutable_data_ptr() : base, false};
+        void *x_hat = lent ? base : base + N * K * 2;
+        Tensor y = empty(sizes, out_type, x.device());
+        run_prepare(x, m, *plan, ln, ln_eps, x_hat, w, nullptr, nullptr, stream);
+        run_product(*plan, m, x_hat, w, o.residual, o.gelu, nullptr, y.mutable_data_ptr(), code_of(y), stream);
+        return y;
     }
     Tensor own_ws;
     const Tensor *ws = as_tensor(get(dict, S._x_hat_buffer));
@@ -427,6 +503,43 @@ Tensor layernorm_op(PyObject *d, const Tensor &x, bool &ok)      // an nn.LayerN
                           PyFloat_AS_DOUBLE(e));
 }
 
+// The fused block on prepared operands, seven launches: [LayerNorm + stage 1, weights of qkv and proj] -> qkv -> attention
+// ending with proj's stage 1 -> proj + skip -> [LayerNorm + stage 1, weights of fc1 and fc2] -> fc1 + GELU + fc2's stage 1
+// -> fc2 + skip.  All intermediate tensors come from the caching allocator, w_hat of two layers at a time included.
+std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t heads, bool own, Plan &pq, Plan &pp, Plan &pf1, Plan &pf2,
+                                     PyObject *n1, PyObject *n2, bool chain)
+{
+    const int64_t b = x.size(0), n = x.size(1), C = x.size(2);
+    if (!own || !chain || n > 256 || C != 64 * heads || C > 2048 || pf1.N % 64 != 0) return std::nullopt;
+    for (const Plan *p : {&pq, &pp, &pf1, &pf2})
+        if (!can_prepare(*p, rows) || p->bits != pq.bits) return std::nullopt;
+    // Not where the one-launch layer kernels are at their best (one 64-row tile on most compute units, short rows): DeiT-S at
+    // 12 608 rows 1 625 us a forward against 1 939, DeiT-B 3 969 against 4 373; at 9 456 rows 4 % either way, below and above
+    // that range the seven launches win (6 304 rows: 1 353 -> 1 262 us; 25 216 rows: 3 341 -> 3 286).
+    if (rows > 9000 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) return std::nullopt;
+    float e1, e2;
+    LayerNormParams *l1 = layernorm_params(pq, n1, e1), *l2 = layernorm_params(pf1, n2, e2);
+    if (!l1 || !l2) return std::nullopt;
+    void *stream = stream_of(x);
+    auto layout = [&](const Plan &p) { return arcq_prepared_row_major(rows, p.N, p.K) != 0; };
+    const int64_t wq = pq.N * pq.K, wp = pp.N * pp.K, w1 = pf1.N * pf1.K, w2 = pf2.N * pf2.K;
+    Tensor w = empty({std::max(wq + wp, w1 + w2)}, at::kHalf, x.device());
+    char *wb = static_cast<char *>(w.mutable_data_ptr());
+    Tensor xh = empty({rows * C}, at::kHalf, x.device());
+    Tensor wide = empty({rows * std::max(pq.N, pf1.N)}, at::kHalf, x.device());       // qkv's output, then fc1's quantized output
+    Tensor x1 = empty(x.sizes(), at::kHalf, x.device()), y = empty(x.sizes(), at::kHalf, x.device());
+    const Weights hq{wb, layout(pq)}, hp{wb + wq * 2, layout(pp)}, h1{wb, layout(pf1)}, h2{wb + w1 * 2, layout(pf2)};
+    run_prepare(x, rows, pq, l1, e1, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
+    run_product(pq, rows, xh.const_data_ptr(), hq, nullptr, false, nullptr, wide.mutable_data_ptr(), ARCQ_F16, stream);
+    check(arcq_attention_quant_fwd(wide.const_data_ptr(), static_cast<const float *>(pp.p[A_THR]), static_cast<const float *>(pp.p[A_CB]),
+                                   static_cast<int>(pp.bits), xh.mutable_data_ptr(), b, n, heads, 64, 0.125f, stream));
+    run_product(pp, rows, xh.const_data_ptr(), hp, &x, false, nullptr, x1.mutable_data_ptr(), ARCQ_F16, stream);
+    run_prepare(x1, rows, pf1, l2, e2, xh.mutable_data_ptr(), h1, &pf2, &h2, stream);
+    run_product(pf1, rows, xh.const_data_ptr(), h1, nullptr, true, &pf2, wide.mutable_data_ptr(), ARCQ_F16, stream);
+    run_product(pf2, rows, wide.const_data_ptr(), h2, &x1, false, nullptr, y.mutable_data_ptr(), ARCQ_F16, stream);
+    return y;
+}
+
 // One transformer block (vit.Block.forward), both of its forms; nullopt before anything has been launched where a module
 // is not the plain case.
 std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
@@ -463,6 +576,8 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
         if (!f16(x) || c > (rows >= 512 ? 1024 : 1536) || c % 64 != 0 || pf2->K % 64 != 0) return std::nullopt;
         for (Plan *p : {pq, pp, pf1, pf2})
             if (p->gs != 64) return std::nullopt;
+        auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, is_true(get(d, S.chain_mlp)));
+        if (whole) return whole;
         Options o1;
         o1.layernorm = n1;
         auto t = layer_call(qkv, x, o1);

@@ -269,6 +269,47 @@ int arcq_act_quant_blocked_ln(const void *x, int x_dtype, const float *ln_weight
                               const uint8_t *packed_w, const float *w_codebook, const float *w_center,
                               const float *w_scale, const float *w_code_sum, void *w_hat, int64_t N, void *stream);
 
+/* ---- the layer in two launches on prepared operands ---------------------------------------------------------
+ * arcq_prepare: x_hat of one tensor (optionally LayerNorm over its rows first, K <= 2048) in the 32-row block layout
+ * (arcq_act_quant_blocked), and w_hat of up to two layers (any K; the same bits) as fp16 in the 32-column block layout
+ * [N/32][K/8][32 columns][8 values], in one launch.  rows = 0: weights only; weights[i].packed = NULL: no such job.
+ * arcq_linear_prepared: y = x_hat * w_hat^T + bias on them, N a multiple of 32, with the options of arcq_linear_otf_ex
+ * (next_*: y receives the consuming layer's x_hat, always in the block layout here).  Below 512 rows the products of
+ * the groups g = w, w + 8, ... are summed apart for w = 0 .. 7 and added in that order, from 512 rows on k ascends:
+ * the orders of the other entry points, i.e. the same bits as theirs. */
+typedef struct arcq_prepare_weights {
+    const uint8_t *packed;                                   /* 16-byte aligned */
+    const float *codebook, *center, *scale, *code_sum;
+    void *w_hat;
+    int64_t N, K;
+    int32_t row_major, reserved;                             /* row_major != 0: w_hat as [N][K] instead of column blocks */
+} arcq_prepare_weights;
+typedef struct arcq_prepare_args {
+    int32_t x_dtype, bits;
+    float ln_eps;
+    int32_t reserved;
+    int64_t rows, K;
+    const void *x;
+    const float *ln_weight, *ln_bias;                        /* NULL: no LayerNorm; 16-byte aligned */
+    const float *thresholds, *codebook;
+    void *x_hat;
+    arcq_prepare_weights weights[2];
+} arcq_prepare_args;
+int arcq_prepare(const arcq_prepare_args *args, void *stream);
+typedef struct arcq_linear_prepared_args {
+    int32_t y_dtype, activation, next_bits, w_row_major;
+    int64_t M, N, K;
+    const void *x_hat, *w_hat;
+    const float *bias;
+    const void *residual;                                    /* [M,N] of y's type, or NULL */
+    const float *next_thresholds, *next_codebook;
+    void *y;
+} arcq_linear_prepared_args;
+int arcq_linear_prepared(const arcq_linear_prepared_args *args, void *stream);
+/* Layout of w_hat that arcq_linear_prepared runs fastest on for these sizes: 0 = column blocks (any M), 1 = row-major
+ * (M >= 512: the weight-stationary kernels, which want many row blocks). */
+int arcq_prepared_row_major(int64_t M, int64_t N, int64_t K);
+
 /* arcq_linear_otf_ws for callers that cannot allocate device memory or lend workspaces (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The two
  * scratch buffers come from a static device array of ARCQ_STATIC_SCRATCH_BYTES inside the library, of which every GPU
@@ -335,6 +376,11 @@ int arcq_linear_otf_fp8(const void *x, int x_dtype, const float *a_thresholds, c
  * head_dim must be 64, n <= 256 and scale > 0 (ARCQ_ERR_UNSUPPORTED otherwise); qkv 16-byte, out 8-byte aligned. */
 int arcq_attention_fwd(const void *qkv, void *out, int64_t B, int64_t n, int64_t H, int64_t head_dim, float scale,
                        void *stream);
+
+/* The same with the proj layer's stage 1 as the last step (a head is one group of 64): x_hat [B*n, H*64] fp16 in the 32-row
+ * block layout, the bits of arcq_act_quant_blocked on arcq_attention_fwd's output; thresholds / codebook are the proj layer's. */
+int arcq_attention_quant_fwd(const void *qkv, const float *thresholds, const float *codebook, int bits, void *x_hat,
+                             int64_t B, int64_t n, int64_t H, int64_t head_dim, float scale, void *stream);
 
 /* ---- stage 1 of a quantized patch-embedding convolution ---------------------
  * QuantConv2dPCARCQ (FQ/quant_backends.py:329-384; the activation quantizer groups min(64, in_channels) = 3 channels
