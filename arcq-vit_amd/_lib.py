@@ -58,6 +58,14 @@ class LinearPreparedArgs(ctypes.Structure):
         (n, ctypes.c_void_p) for n in ("x_hat", "w_hat", "bias", "residual", "next_thresholds", "next_codebook", "y")]
 
 
+class LinearIndexArgs(ctypes.Structure):
+    """``arcq_linear_index_args``."""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("x_codes", "x_center", "x_scale", "x_code_sum", "w_codes", "w_center", "w_scale",
+                                               "w_code_sum", "product_table", "a_codebook", "w_codebook", "bias", "y")] + [
+        (n, ctypes.c_int64) for n in ("rows", "out_features", "in_features")] + [
+        (n, ctypes.c_int32) for n in ("bits", "group_size", "levels", "reserved")]
+
+
 ARCQ_PRODUCER_NONE, ARCQ_PRODUCER_LAYERNORM, ARCQ_PRODUCER_XHAT = 0, 1, 2
 ARCQ_ACT_NONE, ARCQ_ACT_GELU = 0, 1
 
@@ -104,6 +112,7 @@ _SIGNATURES = {
     "arcq_patch_embed_fwd": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr],
     "arcq_attention_quant_fwd": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, _c_ptr],
     "arcq_attention_fwd": [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, _c_ptr],
+    "arcq_linear_index": [ctypes.POINTER(LinearIndexArgs), _c_ptr],
     "arcq_linear_forward_packed": [_c_ptr] * 11 + [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_ptr],
     "arcq_linear_forward_u8": [_c_ptr] * 11 + [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_ptr],
 }

@@ -282,6 +282,301 @@ linear_index_tile_kernel(const uint8_t *__restrict__ xq, const float *__restrict
     }
 }
 
+// ---- group size 64, the codebooks at hand -------------------------------------------------------------------------------
+// What bounds the tiled kernel above is its table gather: two operands' address arithmetic and a conflicting 4-byte LDS
+// read per product (random entries of a 256-entry table).  The product table of a layer is P[a][b] = RN32(cb_a[a] * cb_w[b]),
+// so with the two codebooks at hand an entry is one multiplication of two decoded values.  Every workgroup checks that on
+// the table it was given (levels^2 comparisons); where it does not hold the same loops run with the gather.
+//
+// A wave owns a tile of 8 R rows x 8 C outputs, a lane R x C of them (rows ly + 8 i, outputs lx + 8 k), and decodes the two
+// operands of a group into its own LDS region, half a group (32 j) at a time: [j / 4][row or output][4], so that one 16-byte
+// read brings four j of a row: 3 bytes of LDS reads per product at R = 2, C = 4.  What bounds it now is the
+// vector pipe: multiply, (fp64: convert,) add per product, 71 of the 111 us of 1576 x 384 -> 1536; the decoding is the rest.
+//
+// The sum over j of one group does not depend on the other groups, so the waves of a workgroup share ONE tile and take the
+// groups g = wave, wave + S, ...; only the terms they yield are added in the order of the groups, by all threads together,
+// once per round of S groups.  That makes small launches S times shorter and leaves every addition where the reference has
+// it: serial over j in fp64 for the packed format, the 32-lane tree for the byte format (eight j of one residue class mod
+// 8 at a time, the classes in the order 0 4 2 6 1 5 3 7, which is the tree depth first), terms in ascending g.
+// Measured, whole calls, this kernel against the tiled one: 1576 x 384 -> 1536 (4 bits) 111 against 186 us, 12608 rows 744
+// against 1172; 1576 x 768 -> 768 108 / 207; byte codes 394 x 768 -> 768 35 / 86, 12608 x 384 -> 1536 546 / 1177.
+constexpr int kIdxMinWaves = 3, kIdxMaxWaves = 4;
+constexpr int kIdxRegion = 32 * 33 * 8;            // bytes per wave: operands of half a group, then its terms (33-double pitch)
+
+template <int BITS, int R, int C>
+__global__ void __launch_bounds__(256, R == 1 ? 4 : 3)
+linear_index_wide_kernel(const uint8_t *__restrict__ xq, const float *__restrict__ xc, const float *__restrict__ xs,
+                         const float *__restrict__ xcs, const uint8_t *__restrict__ wq,
+                         const float *__restrict__ wc, const float *__restrict__ ws, const float *__restrict__ wcs,
+                         const float *__restrict__ table, const float *__restrict__ a_cb, const float *__restrict__ w_cb,
+                         const float *__restrict__ bias, float *__restrict__ y, int rows, int out_f, int G, int levels)
+{
+#pragma clang fp contract(off)
+    constexpr bool kPacked = BITS != 0;
+    constexpr int kLevels = kPacked ? 1 << BITS : 16;
+    constexpr int TR = 8 * R, TC = 8 * C;
+    constexpr int kRowBytes = kPacked ? 8 * BITS : 64;
+    constexpr int kPieceBytes = kRowBytes / 8;                        // eight codes
+    constexpr int kPieceDwords = kPacked ? 1 : 2;
+    constexpr int kXJobs = TR * 8 / 64, kWJobs = TC * 8 / 64;          // pieces per lane and group
+    constexpr int kPitch = TC + 1;                                     // terms per row of the tile
+    using acc_t = typename std::conditional<kPacked, double, float>::type;
+    static_assert((TR + TC) * 32 * 4 <= kIdxRegion && TR * kPitch * static_cast<int>(sizeof(acc_t)) <= kIdxRegion, "LDS region");
+    __shared__ float s_table[kLevels * kLevels], s_acb[kLevels], s_wcb[kLevels];
+    extern __shared__ __attribute__((aligned(16))) unsigned char idx_smem[];     // [S waves][kIdxRegion]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nthreads = blockDim.x, S = nthreads >> 6;
+    const int lx = lane & 7, ly = lane >> 3;
+    const int r0 = blockIdx.y * TR, o0 = blockIdx.x * TC;
+    unsigned char *region = idx_smem + wave * kIdxRegion;
+    float *s_x = reinterpret_cast<float *>(region), *s_w = s_x + TR * 32;
+
+    // Pieces: job i of a lane is row lane % T, piece (lane / T) + i * (64 / T) of the group (T = TR or TC; rows past the end
+    // repeat the last one and are not stored).
+    const uint8_t *x_src = xq + static_cast<int64_t>(min(r0 + lane % TR, rows - 1)) * G * kRowBytes + (lane / TR) * kPieceBytes;
+    const uint8_t *w_src = wq + static_cast<int64_t>(min(o0 + lane % TC, out_f - 1)) * G * kRowBytes + (lane / TC) * kPieceBytes;
+    uint32_t xn[kXJobs][kPieceDwords], wn[kWJobs][kPieceDwords];
+    auto load_piece = [](const uint8_t *p, uint32_t (&d)[kPieceDwords]) __attribute__((always_inline)) {
+        if constexpr (kPacked) {
+            d[0] = load_codes8<BITS>(p);
+        } else {
+            const uint2 v = *reinterpret_cast<const uint2 *>(p);
+            d[0] = v.x;
+            d[1] = v.y;
+        }
+    };
+    auto fetch = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kXJobs; ++i) load_piece(x_src + static_cast<int64_t>(g) * kRowBytes + i * (64 / TR) * kPieceBytes, xn[i]);
+#pragma unroll
+        for (int i = 0; i < kWJobs; ++i) load_piece(w_src + static_cast<int64_t>(g) * kRowBytes + i * (64 / TC) * kPieceBytes, wn[i]);
+    };
+    if (wave < G) fetch(wave);
+    int same = 1;
+    for (int i = tid; i < levels * levels; i += nthreads) {
+        const float t = table[i];
+        s_table[i] = t;
+        same &= static_cast<int>(__float_as_uint(t) == __float_as_uint(a_cb[i / levels] * w_cb[i % levels]));
+    }
+    if (tid < levels) s_acb[tid] = a_cb[tid], s_wcb[tid] = w_cb[tid];
+    const bool outer = __syncthreads_and(same) != 0;
+    // With its address seen by an asm statement the region is memory the statements in the loops below may touch, so its
+    // reads stay where they are written.  (The compiler otherwise moves all reads of a group to its top: 500 registers.)
+    asm volatile("" ::"v"(region) : "memory");
+
+    // The outputs this thread sums: TR * TC of them over the workgroup, consecutive in a row.
+    constexpr int kSums = (TR * TC + 64 * kIdxMinWaves - 1) / (64 * kIdxMinWaves);
+    acc_t acc[kSums];
+#pragma unroll
+    for (int i = 0; i < kSums; ++i) {
+        const int p = i * nthreads + tid, o = o0 + p % TC;
+        acc[i] = (bias && p < TR * TC && o < out_f) ? static_cast<acc_t>(bias[o]) : static_cast<acc_t>(0);
+    }
+
+    auto body = [&](auto outer_c) __attribute__((always_inline)) {
+        constexpr bool OUTER = decltype(outer_c)::value;
+        // An operand's decoded value: its codebook entry, or (gather) its share of the byte offset of the table entry.
+        auto x_value = [&](uint32_t c) __attribute__((always_inline)) { return OUTER ? s_acb[c] : __uint_as_float(c * static_cast<uint32_t>(levels) * 4u); };
+        auto w_value = [&](uint32_t c) __attribute__((always_inline)) { return OUTER ? s_wcb[c] : __uint_as_float(c * 4u); };
+        auto product = [&](float xv, float wv) __attribute__((always_inline)) {
+            if constexpr (OUTER) return xv * wv;
+            else return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(s_table) + (__float_as_uint(xv) + __float_as_uint(wv)));
+        };
+        // Half `h` of a group into LDS.  Packed: j = 32 h ... + 31, slot jq = (j % 32) / 4.  Bytes: the classes j % 8 = h' + {0, 4,
+        // 2, 6} with h' = h, class number n (0..3) and piece p at slot 2 n + p / 4.
+        auto put = [&](float *dst, int T, auto jobs_c, const uint32_t (*codes)[kPieceDwords], int h, auto value) __attribute__((always_inline)) {
+            constexpr int JOBS = decltype(jobs_c)::value;
+            const int row = lane % T, p0 = lane / T;
+#pragma unroll
+            for (int i = 0; i < JOBS; ++i) {
+                const int p = p0 + i * (64 / T);
+                if constexpr (kPacked) {
+                    if ((p >> 2) == h) {
+                        float v[8];
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) v[q] = value((codes[i][0] >> (BITS * q)) & ((1u << BITS) - 1u));
+                        float *d = dst + ((p & 3) * 2 * T + row) * 4;
+                        *reinterpret_cast<float4 *>(d) = make_float4(v[0], v[1], v[2], v[3]);
+                        *reinterpret_cast<float4 *>(d + T * 4) = make_float4(v[4], v[5], v[6], v[7]);
+                    }
+                } else {
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) {
+                        const uint32_t d = (n & 1) ? codes[i][kPieceDwords - 1] : codes[i][0];      // bytes 4.. / 0..3
+                        const uint32_t c = (d >> (8 * (h + (n & 2)))) & 255u;
+                        dst[((2 * n + (p >> 2)) * T + row) * 4 + (p & 3)] = value(c);
+                    }
+                }
+            }
+        };
+        const int rounds = (G + S - 1) / S;
+        for (int round = 0; round < rounds; ++round) {
+            const int g = round * S + wave;
+            if (g < G) {
+                uint32_t xk[kXJobs][kPieceDwords], wk[kWJobs][kPieceDwords];
+#pragma unroll
+                for (int i = 0; i < kXJobs; ++i)
+#pragma unroll
+                    for (int d = 0; d < kPieceDwords; ++d) xk[i][d] = xn[i][d];
+#pragma unroll
+                for (int i = 0; i < kWJobs; ++i)
+#pragma unroll
+                    for (int d = 0; d < kPieceDwords; ++d) wk[i][d] = wn[i][d];
+                if (g + S < G) fetch(g + S);
+                acc_t cross[R][C];
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int c = 0; c < C; ++c) cross[r][c] = 0;
+#pragma unroll 1
+                for (int h = 0; h < 2; ++h) {
+                    put(s_x, TR, std::integral_constant<int, kXJobs>{}, xk, h, x_value);
+                    put(s_w, TC, std::integral_constant<int, kWJobs>{}, wk, h, w_value);
+                    asm volatile("" ::: "memory");          // (wave-private LDS: operations execute in order)
+                    if constexpr (kPacked) {
+#pragma unroll 1
+                        for (int jq = 0; jq < 8; ++jq) {
+                            float4 xv[R], wv[C];
+#pragma unroll
+                            for (int r = 0; r < R; ++r) xv[r] = *reinterpret_cast<const float4 *>(s_x + (jq * TR + ly + 8 * r) * 4);
+#pragma unroll
+                            for (int c = 0; c < C; ++c) wv[c] = *reinterpret_cast<const float4 *>(s_w + (jq * TC + lx + 8 * c) * 4);
+                            const float *xf = reinterpret_cast<const float *>(xv), *wf = reinterpret_cast<const float *>(wv);
+#pragma unroll
+                            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                                for (int r = 0; r < R; ++r)
+#pragma unroll
+                                    for (int c = 0; c < C; ++c) cross[r][c] += static_cast<double>(product(xf[4 * r + q], wf[4 * c + q]));
+                        }
+                    } else {
+                        float n3a[R][C];                     // the sum of this half's first two classes (offset 4)
+#pragma unroll 1
+                        for (int pair = 0; pair < 2; ++pair) {
+                            float n2a[R][C];
+#pragma unroll
+                            for (int e = 0; e < 2; ++e) {
+                                const int n = 2 * pair + e;
+                                float4 xv[R][2];
+#pragma unroll
+                                for (int r = 0; r < R; ++r)
+#pragma unroll
+                                    for (int k = 0; k < 2; ++k) xv[r][k] = *reinterpret_cast<const float4 *>(s_x + ((2 * n + k) * TR + ly + 8 * r) * 4);
+#pragma unroll
+                                for (int c = 0; c < C; ++c) {
+                                    float4 wv[2];
+#pragma unroll
+                                    for (int k = 0; k < 2; ++k) wv[k] = *reinterpret_cast<const float4 *>(s_w + ((2 * n + k) * TC + lx + 8 * c) * 4);
+                                    const float w0[4] = {wv[0].x, wv[0].y, wv[0].z, wv[0].w}, w1[4] = {wv[1].x, wv[1].y, wv[1].z, wv[1].w};
+#pragma unroll
+                                    for (int r = 0; r < R; ++r) {
+                                        const float x0[4] = {xv[r][0].x, xv[r][0].y, xv[r][0].z, xv[r][0].w}, x1[4] = {xv[r][1].x, xv[r][1].y, xv[r][1].z, xv[r][1].w};
+                                        float leaf[4];       // lanes c, c + 8, c + 16, c + 24 of the class
+#pragma unroll
+                                        for (int q = 0; q < 4; ++q) leaf[q] = product(x0[q], w0[q]) + product(x1[q], w1[q]);
+                                        const float n2 = (leaf[0] + leaf[2]) + (leaf[1] + leaf[3]);     // offsets 16, 8
+                                        if (e == 0) n2a[r][c] = n2;
+                                        else n2a[r][c] += n2;                                             // offset 4
+                                    }
+                                }
+                                asm volatile("" ::: "memory");
+                            }
+#pragma unroll
+                            for (int r = 0; r < R; ++r)
+#pragma unroll
+                                for (int c = 0; c < C; ++c) {
+                                    if (pair == 0) {
+                                        n3a[r][c] = n2a[r][c];
+                                    } else {
+                                        const float n4 = n3a[r][c] + n2a[r][c];                           // offset 2
+                                        cross[r][c] = h == 0 ? n4 : cross[r][c] + n4;                     // offset 1
+                                    }
+                                }
+                        }
+                    }
+                    asm volatile("" ::: "memory");
+                }
+                // ---- the group's closed form (EXT/arcq_linear_kernel.cu:65-74 / :187-197), into the wave's LDS region ----
+                acc_t *term = reinterpret_cast<acc_t *>(region);
+                float wcv[C], wsv[C], wmv[C];
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    const int64_t wm = static_cast<int64_t>(min(o0 + lx + 8 * c, out_f - 1)) * G + g;
+                    wcv[c] = wc[wm], wsv[c] = ws[wm], wmv[c] = wcs[wm];
+                }
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int64_t xm = static_cast<int64_t>(min(r0 + ly + 8 * r, rows - 1)) * G + g;
+                    const float xcv = xc[xm], xsv = xs[xm], xcsv = xcs[xm];
+#pragma unroll
+                    for (int c = 0; c < C; ++c) {
+                        acc_t v;
+                        if constexpr (kPacked) {
+                            const double mu_term = 64.0 * static_cast<double>(xcv) * static_cast<double>(wcv[c]);
+                            const double residual_term = static_cast<double>(xsv) * static_cast<double>(wsv[c]) *
+                                (cross[r][c] - (static_cast<double>(xcsv) * static_cast<double>(wmv[c])) / 64.0);
+                            v = mu_term + residual_term;
+                        } else {
+                            const float mu_term = 64.0f * xcv * wcv[c];
+                            const float residual_term = xsv * wsv[c] * (cross[r][c] - (xcsv * wmv[c]) / 64.0f);
+                            v = mu_term + residual_term;
+                        }
+                        term[(ly + 8 * r) * kPitch + lx + 8 * c] = v;
+                    }
+                }
+            }
+            __syncthreads();
+            const int live = min(S, G - round * S);
+#pragma unroll
+            for (int i = 0; i < kSums; ++i) {
+                const int p = i * nthreads + tid;
+                if (p < TR * TC) {
+                    const unsigned char *src = idx_smem + ((p / TC) * kPitch + p % TC) * static_cast<int>(sizeof(acc_t));
+                    for (int w = 0; w < live; ++w) acc[i] += *reinterpret_cast<const acc_t *>(src + w * kIdxRegion);
+                }
+            }
+            __syncthreads();
+        }
+    };
+    if (outer) body(std::true_type{});
+    else body(std::false_type{});
+#pragma unroll
+    for (int i = 0; i < kSums; ++i) {
+        const int p = i * nthreads + tid;
+        const int r = r0 + p / TC, o = o0 + p % TC;
+        if (p < TR * TC && r < rows && o < out_f) y[static_cast<int64_t>(r) * out_f + o] = static_cast<float>(acc[i]);
+    }
+}
+
+struct IndexArgs {
+    const uint8_t *xq;
+    const float *xc, *xs, *xcs;
+    const uint8_t *wq;
+    const float *wc, *ws, *wcs, *table, *a_cb, *w_cb, *bias;
+    float *y;
+    int rows, out_f, G, levels;
+};
+template <int BITS, int R, int C>
+void launch_index_wide(const IndexArgs &a, hipStream_t stream)
+{
+    // Waves per workgroup: the count that leaves the fewest of them without a group in the last round, the larger one of
+    // equals (384 -> 1536, six groups, 12608 rows: three waves 744, four waves 832 us).
+    int S = kIdxMaxWaves;
+    for (int s = kIdxMaxWaves - 1; s >= kIdxMinWaves; --s)
+        if ((a.G + s - 1) / s * s < (a.G + S - 1) / S * S) S = s;
+    hipLaunchKernelGGL((linear_index_wide_kernel<BITS, R, C>), dim3((a.out_f + 8 * C - 1) / (8 * C), (a.rows + 8 * R - 1) / (8 * R)), dim3(64 * S),
+                       S * kIdxRegion, stream, a.xq, a.xc, a.xs, a.xcs, a.wq, a.wc, a.ws, a.wcs, a.table, a.a_cb, a.w_cb, a.bias, a.y, a.rows,
+                       a.out_f, a.G, a.levels);
+}
+// Four outputs and two rows per lane; one row where that leaves at most 1024 workgroups (four per CU), whose duration is
+// one wave's (197 x 768 -> 768, 600 of them: 30.6 against 34.2 us; 394 x 768 -> 768: 42.4 against 42.9, byte codes 40.6
+// against 34.5).  Four rows spill nothing but leave two waves per SIMD: 1576 x 384 -> 1536 131 us against 121.
+template <int BITS>
+void launch_index(const IndexArgs &a, hipStream_t stream)
+{
+    if (static_cast<int64_t>((a.rows + 7) / 8) * ((a.out_f + 31) / 32) <= 1024) launch_index_wide<BITS, 1, 4>(a, stream);
+    else launch_index_wide<BITS, 2, 4>(a, stream);
+}
+
 // Launches of at most this many 16 x 64 tiles give every thread one output instead of four.
 constexpr int kSmallTiles = 512;
 static size_t tile_table_bytes(int levels) { return static_cast<size_t>(levels) * levels * sizeof(float); }
@@ -386,4 +681,33 @@ ARCQ_API int arcq_linear_forward_u8(const uint8_t *x_codes, const float *x_cente
                        static_cast<hipStream_t>(stream), x_codes, x_center, x_scale, x_code_sum, w_codes, w_center,
                        w_scale, w_code_sum, product_table, bias, y, rows, out_features, in_features, group_size, levels);
     return launch_status("arcq_linear_forward_u8");
+}
+
+ARCQ_API int arcq_linear_index(const arcq_linear_index_args *a, void *stream)
+{
+    if (!a) return fail(ARCQ_ERR_NULL, "arcq_linear_index: args must not be NULL");
+    if (a->bits != 0 && !bits_ok(a->bits)) return fail(ARCQ_ERR_BITS, "arcq_linear_index: bits must be 2, 3, or 4 (or 0 for byte codes)");
+    const bool wide = a->group_size == 64 && a->in_features > 0 && a->in_features % 64 == 0 && a->levels >= 1 && a->a_codebook && a->w_codebook &&
+                      (a->bits ? a->levels == (1 << a->bits) : a->levels <= 16) && a->rows > 0 && a->out_features > 0 &&
+                      a->rows < (1 << 19) && a->out_features < (1 << 28) && a->x_codes && a->x_center && a->x_scale && a->x_code_sum &&
+                      a->w_codes && a->w_center && a->w_scale && a->w_code_sum && a->product_table && a->y && aligned(a->x_codes, 8) &&
+                      aligned(a->w_codes, 8);
+    if (!wide) {           // anything else, and what is wrong: the entry points that take no codebooks
+        if (a->bits)
+            return arcq_linear_forward_packed(a->x_codes, a->x_center, a->x_scale, a->x_code_sum, a->w_codes, a->w_center, a->w_scale,
+                                              a->w_code_sum, a->product_table, a->bias, a->y, a->rows, a->out_features, a->in_features,
+                                              a->bits, a->group_size, a->levels, stream);
+        return arcq_linear_forward_u8(a->x_codes, a->x_center, a->x_scale, a->x_code_sum, a->w_codes, a->w_center, a->w_scale, a->w_code_sum,
+                                      a->product_table, a->bias, a->y, a->rows, a->out_features, a->in_features, a->group_size, a->levels,
+                                      stream);
+    }
+    const IndexArgs g{a->x_codes, a->x_center, a->x_scale, a->x_code_sum, a->w_codes, a->w_center, a->w_scale, a->w_code_sum, a->product_table,
+                      a->a_codebook, a->w_codebook, a->bias, a->y, static_cast<int>(a->rows), static_cast<int>(a->out_features),
+                      static_cast<int>(a->in_features / 64), a->levels};
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (a->bits == 4) launch_index<4>(g, st);
+    else if (a->bits == 3) launch_index<3>(g, st);
+    else if (a->bits == 2) launch_index<2>(g, st);
+    else launch_index<0>(g, st);
+    return launch_status("arcq_linear_index");
 }

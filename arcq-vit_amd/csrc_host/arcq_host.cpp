@@ -792,19 +792,21 @@ PyObject *py_packed_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
         if (!bytes && strcmp(fmt, "packed") != 0) return none();
         const Tensor &table = plan->slot[P_TABLE].use;
         if (!table.defined() || table.dim() != 2 || table.size(0) != table.size(1)) return none();
+        if (plan->slot[A_CB].use.numel() != table.size(0) || plan->slot[W_CB].use.numel() != table.size(0)) return none();
         if (bytes && (!p[P_CODES] || plan->slot[P_CODES].use.numel() != N * K || plan->slot[P_CODES].use.scalar_type() != at::kByte))
             return none();
         const int levels = static_cast<int>(table.size(0));
         const Tensor x2 = x.dim() == 2 ? x : x.view({m, K});
         Quantized q = quantize(x2, fp(A_THR), fp(A_CB), bits, gs, bytes);
         Tensor y = empty(sizes, at::kFloat, x.device());
-        float *yp = static_cast<float *>(y.mutable_data_ptr());
-        if (bytes)
-            check(arcq_linear_forward_u8(bptr(q.codes), fptr(q.center), fptr(q.scale), fptr(q.sum), up(P_CODES), fp(W_CENTER), fp(W_SCALE),
-                                         fp(W_SUM), fptr(table), fp(W_BIAS), yp, m, N, K, gs, levels, stream));
-        else
-            check(arcq_linear_forward_packed(bptr(q.codes), fptr(q.center), fptr(q.scale), fptr(q.sum), up(W_PACKED), fp(W_CENTER),
-                                             fp(W_SCALE), fp(W_SUM), fptr(table), fp(W_BIAS), yp, m, N, K, bits, gs, levels, stream));
+        arcq_linear_index_args a = {};
+        a.x_codes = bptr(q.codes), a.x_center = fptr(q.center), a.x_scale = fptr(q.scale), a.x_code_sum = fptr(q.sum);
+        a.w_codes = up(bytes ? P_CODES : W_PACKED), a.w_center = fp(W_CENTER), a.w_scale = fp(W_SCALE), a.w_code_sum = fp(W_SUM);
+        a.product_table = fptr(table), a.a_codebook = fp(A_CB), a.w_codebook = fp(W_CB), a.bias = fp(W_BIAS);
+        a.y = static_cast<float *>(y.mutable_data_ptr());
+        a.rows = m, a.out_features = N, a.in_features = K;
+        a.bits = bytes ? 0 : bits, a.group_size = gs, a.levels = levels;
+        check(arcq_linear_index(&a, stream));
         return THPVariable_Wrap(std::move(y));
     });
 }

@@ -446,6 +446,21 @@ int arcq_linear_forward_u8(const uint8_t *x_codes, const float *x_center, const 
                            int64_t rows, int64_t out_features, int64_t in_features,
                            int group_size, int levels, void *stream);
 
+/* Either of the two (bits = 0: byte codes) with the codebooks the product table was made from: where
+ * product_table[a][b] == a_codebook[a] * w_codebook[b] (rounded to fp32; the kernel checks) an entry is computed instead of
+ * gathered.  Same results bit for bit; group size 64 (others, and calls without codebooks, go to the entry points above). */
+typedef struct arcq_linear_index_args {
+    const uint8_t *x_codes;
+    const float *x_center, *x_scale, *x_code_sum;
+    const uint8_t *w_codes;
+    const float *w_center, *w_scale, *w_code_sum;
+    const float *product_table, *a_codebook, *w_codebook, *bias;
+    float *y;
+    int64_t rows, out_features, in_features;
+    int32_t bits, group_size, levels, reserved;
+} arcq_linear_index_args;
+int arcq_linear_index(const arcq_linear_index_args *args, void *stream);
+
 #ifdef __cplusplus
 }
 #endif
