@@ -40,12 +40,12 @@ class LinearExArgs(ctypes.Structure):
 class PrepareWeights(ctypes.Structure):
     """``arcq_prepare_weights`` of include/arcq_hip.h."""
     _fields_ = [(n, ctypes.c_void_p) for n in ("packed", "codebook", "center", "scale", "code_sum", "w_hat")] + [
-        ("N", ctypes.c_int64), ("K", ctypes.c_int64), ("row_major", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+        ("N", ctypes.c_int64), ("K", ctypes.c_int64), ("row_major", ctypes.c_int32), ("w_mult", ctypes.c_float)]
 
 
 class PrepareArgs(ctypes.Structure):
     """``arcq_prepare_args``."""
-    _fields_ = [("x_dtype", ctypes.c_int32), ("bits", ctypes.c_int32), ("ln_eps", ctypes.c_float), ("reserved", ctypes.c_int32),
+    _fields_ = [("x_dtype", ctypes.c_int32), ("bits", ctypes.c_int32), ("ln_eps", ctypes.c_float), ("fp8", ctypes.c_int32),
                 ("rows", ctypes.c_int64), ("K", ctypes.c_int64)] + [
         (n, ctypes.c_void_p) for n in ("x", "ln_weight", "ln_bias", "thresholds", "codebook", "x_hat")] + [
         ("weights", PrepareWeights * 2)]
@@ -55,7 +55,8 @@ class LinearPreparedArgs(ctypes.Structure):
     """``arcq_linear_prepared_args``."""
     _fields_ = [(n, ctypes.c_int32) for n in ("y_dtype", "activation", "next_bits", "w_row_major")] + [
         (n, ctypes.c_int64) for n in ("M", "N", "K")] + [
-        (n, ctypes.c_void_p) for n in ("x_hat", "w_hat", "bias", "residual", "next_thresholds", "next_codebook", "y")]
+        (n, ctypes.c_void_p) for n in ("x_hat", "w_hat", "bias", "residual", "next_thresholds", "next_codebook", "y")] + [
+        ("fp8", ctypes.c_int32), ("w_mult", ctypes.c_float)]
 
 
 class LinearIndexArgs(ctypes.Structure):
@@ -91,6 +92,7 @@ _SIGNATURES = {
     "arcq_linear_otf_ex": [ctypes.POINTER(LinearExArgs), _c_ptr],
     "arcq_xhat_layout": [_c_i64],
     "arcq_prepared_row_major": [_c_i64, _c_i64, _c_i64],
+    "arcq_prepared_row_major_fp8": [_c_i64, _c_i64, _c_i64],
     "arcq_prepare": [ctypes.POINTER(PrepareArgs), _c_ptr],
     "arcq_linear_prepared": [ctypes.POINTER(LinearPreparedArgs), _c_ptr],
     "arcq_act_quant_blocked_ln": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_f32, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_int,
@@ -111,6 +113,7 @@ _SIGNATURES = {
                                _c_int, _c_ptr],
     "arcq_patch_embed_fwd": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr],
     "arcq_attention_quant_fwd": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, _c_ptr],
+    "arcq_attention_quant_fp8_fwd": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, _c_ptr],
     "arcq_attention_fwd": [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, _c_ptr],
     "arcq_linear_index": [ctypes.POINTER(LinearIndexArgs), _c_ptr],
     "arcq_linear_forward_packed": [_c_ptr] * 11 + [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_ptr],
@@ -179,10 +182,10 @@ def host():
             raise ARCQLibraryMissing(f"ARCQ host extension is not built or does not load ({e}). "
                                      "Run `python -m arcq_vit_amd.build` first.") from e
         import torch
-        from . import vit
+        from . import ops, vit
         from .packed_on_the_fly import ARCQPackedLinearOnTheFly
         mod.register_types(ARCQPackedLinearOnTheFly, vit.Attention, vit.Mlp, torch.nn.GELU, torch.nn.LayerNorm,
-                           sys.modules["torch.nn.modules.module"])
+                           sys.modules["torch.nn.modules.module"], ops.fp8_weight_multiplier)
         _host = mod
     return _host
 

@@ -7,6 +7,37 @@
 
 namespace arcq {
 
+// ---- FP8 operands (OCP E4M3) ---------------------------------------------------------------------------------------
+constexpr float kFp8Max = 448.0f;
+
+// Eight floats -> eight FP8 (E4M3, round to nearest even, finite values saturating at +-448, NaN kept) in two dwords.
+__device__ __forceinline__ void to_fp8x8(const float (&v)[8], uint32_t &lo, uint32_t &hi)
+{
+    float c[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) c[i] = v[i] != v[i] ? v[i] : fminf(fmaxf(v[i], -kFp8Max), kFp8Max);      // (NaN stays NaN)
+    int a = 0, b = 0;
+    a = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], a, false);
+    a = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], a, true);
+    b = __builtin_amdgcn_cvt_pk_fp8_f32(c[4], c[5], b, false);
+    b = __builtin_amdgcn_cvt_pk_fp8_f32(c[6], c[7], b, true);
+    lo = static_cast<uint32_t>(a);
+    hi = static_cast<uint32_t>(b);
+}
+
+// Sixteen reconstructed values s (v[j0 + e] - code_mean) + mu as one 16-byte piece.
+template <int N>
+__device__ __forceinline__ void xhat_fp8x16(const float (&v)[N], int j0, float s, float code_mean, float mu, uint32_t (&o)[4])
+{
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        float t[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] = fma_f32(s, v[j0 + 8 * p + e] - code_mean, mu);
+        to_fp8x8(t, o[2 * p], o[2 * p + 1]);
+    }
+}
+
 constexpr int kMaxBuckets = 512;   // table entries 0 .. nb (nb <= 512); entry nb is reached by t == 8 only
 
 // Bucket geometry: t in [-8, 8] maps to floor(f), f = t * scale + 8 * scale rounded to a multiple of 1/8; nb = 16 * scale
@@ -358,11 +389,12 @@ __device__ __forceinline__ void next_quant_setup(const float *__restrict__ thr, 
 // One staged chunk (32 rows x 64 fp16 values, the rows `pitch` bytes apart) -> x_hat of the consuming layer.
 // `gelu`: the exact GELU of the staged (rounded) values first, rounded to fp16 again.  dst = the chunk's first 16-byte
 // piece of this lane's row (lane / 2) in the consumer's block layout, whose pieces are `rows` rows apart; `live` = whether
-// the row is stored.  The whole wave calls it.
-template <int BITS>
+// the row is stored.  F8: the consumer's operands are FP8 (16 values a piece); `pad`: the chunk is the last of a row whose
+// length is an odd number of groups, and the row's padding to 128 values is written too.  The whole wave calls it.
+template <int BITS, bool F8 = false>
 __device__ __forceinline__ void next_quant_rows(const unsigned char *lds, int nwaves,
                                                 const unsigned char *stage, int pitch, int lane, bool gelu, float eps,
-                                                __half *dst, int rows, bool live)
+                                                void *dst, int rows, bool live, bool pad = false)
 {
     typedef uint32_t u32x4_nq __attribute__((ext_vector_type(4)));
     constexpr int L = 1 << BITS;
@@ -395,28 +427,40 @@ __device__ __forceinline__ void next_quant_rows(const unsigned char *lds, int nw
     group_stats32x2(v, eps, mu, var, s);
     group_codes32x2_lds<BITS>(v, mu, var, s, th_lds, bq, table, lut, ok, lane, sum);
     const float code_mean = sum * 0.015625f;
+    char *out = static_cast<char *>(dst);
+    if constexpr (F8) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        uint32_t o[4];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            const int j = 8 * i + 2 * d;
-            const __half2 h = __floats2half2_rn(fma_f32(s, v[j] - code_mean, mu), fma_f32(s, v[j + 1] - code_mean, mu));
-            o[d] = *reinterpret_cast<const uint32_t *>(&h);
+        for (int i = 0; i < 2; ++i) {
+            uint32_t o[4];
+            xhat_fp8x16(v, 16 * i, s, code_mean, mu, o);
+            if (live) store_writethrough16(out + static_cast<int64_t>(hf * 2 + i) * rows * 16, o[0], o[1], o[2], o[3]);
+            if (live && pad) store_writethrough16(out + static_cast<int64_t>(4 + hf * 2 + i) * rows * 16, 0, 0, 0, 0);
         }
-        if (live) store_writethrough16(dst + static_cast<int64_t>(hf * 4 + i) * rows * 8, o[0], o[1], o[2], o[3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t o[4];
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const int j = 8 * i + 2 * d;
+                const __half2 h = __floats2half2_rn(fma_f32(s, v[j] - code_mean, mu), fma_f32(s, v[j + 1] - code_mean, mu));
+                o[d] = *reinterpret_cast<const uint32_t *>(&h);
+            }
+            if (live) store_writethrough16(out + static_cast<int64_t>(hf * 4 + i) * rows * 16, o[0], o[1], o[2], o[3]);
+        }
     }
 }
 
-// The same for a chunk whose 32 rows are one block of the consumer's layout: dst_block = base of that block, `rows` = its
-// rows (32, or fewer for a last block), piece0 = index of the chunk's first 16-byte piece (column / 8).
-template <int BITS>
-__device__ __forceinline__ void next_quant_chunk(const unsigned char *lds, int nwaves,
-                                                 const unsigned char *stage, int pitch, int lane, bool gelu, float eps,
-                                                 __half *dst_block, int rows, int piece0)
+// The same for a chunk whose 32 rows are block `blk` of the consumer's operand at x_hat (N values a row, M rows): c0 = the
+// chunk's first column.
+template <int BITS, bool F8>
+__device__ __forceinline__ void next_quant_block(const unsigned char *lds, int nwaves, const unsigned char *stage, int pitch,
+                                                 int lane, bool gelu, float eps, void *x_hat, int blk, int M, int N, int c0)
 {
-    const int r = lane >> 1;
-    next_quant_rows<BITS>(lds, nwaves, stage, pitch, lane, gelu, eps, dst_block + (static_cast<int64_t>(piece0) * rows + r) * 8, rows, r < rows);
+    const int r = lane >> 1, rows = min(32, M - blk * 32);
+    const int row_bytes = F8 ? (N + 127) / 128 * 128 : N * 2;
+    char *dst = static_cast<char *>(x_hat) + static_cast<int64_t>(blk) * 32 * row_bytes + (static_cast<int64_t>(F8 ? c0 / 16 : c0 / 8) * rows + r) * 16;
+    next_quant_rows<BITS, F8>(lds, nwaves, stage, pitch, lane, gelu, eps, dst, rows, r < rows, F8 && c0 + 64 == N && (N & 64) != 0);
 }
 
 }  // namespace arcq

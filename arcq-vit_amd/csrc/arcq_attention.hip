@@ -37,7 +37,8 @@ constexpr int kKPitch = kHeadDim * 2 + 16;          // bytes per key row of K in
 // rounded output; a head's 64 dims are one quantization group) in the 32-row block layout of the [B n, C] tensor instead of
 // the output.  A wave's 32 x 64 outputs go through its own 32 rows of K in LDS (all waves are done with it) into the
 // lane-pair routine of the GEMM epilogues.
-template <int NKB, int NQ>
+// F8: that operand as FP8 (rows padded to 128 values).
+template <int NKB, int NQ, bool F8>
 __global__ void __launch_bounds__(64 * NKB) __attribute__((amdgpu_waves_per_eu(4)))     // two workgroups of up to 8 waves on a CU
 attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n, int H, float scale,
                  const float *__restrict__ nq_thr, const float *__restrict__ nq_cb, int total_rows)
@@ -202,8 +203,9 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
         const int64_t row = row0 + qr;
         const int blk = static_cast<int>(row >> 5);
         const int nrows = min(32, total_rows - blk * 32);
-        next_quant_rows<NQ>(nq_lds, NKB, stage, kKPitch, lane, false, 1.0e-6f,
-                            out + static_cast<int64_t>(blk) * 32 * C + (static_cast<int64_t>(h) * 8 * nrows + (row & 31)) * 8, nrows, qr < n);
+        const int row_bytes = F8 ? (C + 127) / 128 * 128 : C * 2;
+        char *dst = reinterpret_cast<char *>(out) + static_cast<int64_t>(blk) * 32 * row_bytes + (static_cast<int64_t>(h) * (F8 ? 4 : 8) * nrows + (row & 31)) * 16;
+        next_quant_rows<NQ, F8>(nq_lds, NKB, stage, kKPitch, lane, false, 1.0e-6f, dst, nrows, qr < n, F8 && h == H - 1 && (H & 1) != 0);
         return;
     }
     // ---- normalise, round, store: each lane 4 runs of 4 consecutive dims per 32-dim block ----
@@ -224,30 +226,30 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
     }
 }
 
-template <int NKB, int NQ>
+template <int NKB, int NQ, bool F8>
 void launch_attention(const void *qkv, void *out, int B, int n, int H, float scale, const float *thr, const float *cb, hipStream_t stream)
 {
-    hipLaunchKernelGGL((attention_kernel<NKB, NQ>), dim3(H, B), dim3(64 * NKB), 0, stream, static_cast<const __half *>(qkv),
+    hipLaunchKernelGGL((attention_kernel<NKB, NQ, F8>), dim3(H, B), dim3(64 * NKB), 0, stream, static_cast<const __half *>(qkv),
                        static_cast<__half *>(out), n, H, scale, thr, cb, B * n);
 }
 
-template <int NQ>
+template <int NQ, bool F8 = false>
 void launch_attention_n(const void *qkv, void *out, int B, int n, int H, float scale, const float *thr, const float *cb, hipStream_t st)
 {
     switch ((n + 31) / 32) {
-    case 1: launch_attention<1, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
-    case 2: launch_attention<2, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
-    case 3: launch_attention<3, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
-    case 4: launch_attention<4, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
-    case 5: launch_attention<5, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
-    case 6: launch_attention<6, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
-    case 7: launch_attention<7, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
-    default: launch_attention<8, NQ>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 1: launch_attention<1, NQ, F8>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 2: launch_attention<2, NQ, F8>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 3: launch_attention<3, NQ, F8>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 4: launch_attention<4, NQ, F8>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 5: launch_attention<5, NQ, F8>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 6: launch_attention<6, NQ, F8>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    case 7: launch_attention<7, NQ, F8>(qkv, out, B, n, H, scale, thr, cb, st); break;
+    default: launch_attention<8, NQ, F8>(qkv, out, B, n, H, scale, thr, cb, st); break;
     }
 }
 
 int attention_checked(const char *fn, const void *qkv, void *out, int64_t B, int64_t n, int64_t H, int64_t head_dim, float scale,
-                      int nq_bits, const float *thr, const float *cb, void *stream)
+                      int nq_bits, const float *thr, const float *cb, void *stream, bool fp8 = false)
 {
     if (B < 0 || n < 0 || H < 0) return fail(ARCQ_ERR_SHAPE, "%s: negative size", fn);
     if (!(scale > 0.0f)) return fail(ARCQ_ERR_UNSUPPORTED, "%s: scale must be positive", fn);
@@ -261,7 +263,11 @@ int attention_checked(const char *fn, const void *qkv, void *out, int64_t B, int
         return fail(ARCQ_ERR_SHAPE, "%s: tensor too large", fn);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int b = static_cast<int>(B), nn = static_cast<int>(n), hh = static_cast<int>(H);
-    if (nq_bits == 0) launch_attention_n<0>(qkv, out, b, nn, hh, scale, thr, cb, st);
+    if (fp8) {
+        if (nq_bits == 4) launch_attention_n<4, true>(qkv, out, b, nn, hh, scale, thr, cb, st);
+        else if (nq_bits == 3) launch_attention_n<3, true>(qkv, out, b, nn, hh, scale, thr, cb, st);
+        else launch_attention_n<2, true>(qkv, out, b, nn, hh, scale, thr, cb, st);
+    } else if (nq_bits == 0) launch_attention_n<0>(qkv, out, b, nn, hh, scale, thr, cb, st);
     else if (nq_bits == 4) launch_attention_n<4>(qkv, out, b, nn, hh, scale, thr, cb, st);
     else if (nq_bits == 3) launch_attention_n<3>(qkv, out, b, nn, hh, scale, thr, cb, st);
     else launch_attention_n<2>(qkv, out, b, nn, hh, scale, thr, cb, st);
@@ -285,4 +291,12 @@ ARCQ_API int arcq_attention_quant_fwd(const void *qkv, const float *thresholds, 
     if (!bits_ok(bits)) return fail(ARCQ_ERR_BITS, "arcq_attention_quant_fwd: bits must be 2, 3, or 4");
     if (B * n >= (int64_t(1) << 26)) return fail(ARCQ_ERR_SHAPE, "arcq_attention_quant_fwd: tensor too large");
     return attention_checked("arcq_attention_quant_fwd", qkv, x_hat, B, n, H, head_dim, scale, bits, thresholds, codebook, stream);
+}
+
+ARCQ_API int arcq_attention_quant_fp8_fwd(const void *qkv, const float *thresholds, const float *codebook, int bits, void *x8,
+                                          int64_t B, int64_t n, int64_t H, int64_t head_dim, float scale, void *stream)
+{
+    if (!bits_ok(bits)) return fail(ARCQ_ERR_BITS, "arcq_attention_quant_fp8_fwd: bits must be 2, 3, or 4");
+    if (B * n >= (int64_t(1) << 26)) return fail(ARCQ_ERR_SHAPE, "arcq_attention_quant_fp8_fwd: tensor too large");
+    return attention_checked("arcq_attention_quant_fp8_fwd", qkv, x8, B, n, H, head_dim, scale, bits, thresholds, codebook, stream, true);
 }

@@ -19,23 +19,7 @@
 namespace arcq {
 namespace {
 
-constexpr float kFp8Max = 448.0f;
 constexpr int kFp8Waves = 4;
-
-// Eight floats -> eight FP8 (E4M3, round to nearest even, finite values saturating at +-448, NaN kept) in two dwords.
-__device__ __forceinline__ void to_fp8x8(const float (&v)[8], uint32_t &lo, uint32_t &hi)
-{
-    float c[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) c[i] = v[i] != v[i] ? v[i] : fminf(fmaxf(v[i], -kFp8Max), kFp8Max);      // (NaN stays NaN)
-    int a = 0, b = 0;
-    a = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], a, false);
-    a = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], a, true);
-    b = __builtin_amdgcn_cvt_pk_fp8_f32(c[4], c[5], b, false);
-    b = __builtin_amdgcn_cvt_pk_fp8_f32(c[6], c[7], b, true);
-    lo = static_cast<uint32_t>(a);
-    hi = static_cast<uint32_t>(b);
-}
 
 // Stage 2 with FP8 output: one thread per eight weights (one piece of codes), value = w_mult * w_hat.  Rows of w8 are
 // `ldw` bytes apart (ldw >= K, a multiple of 8); the bytes from K to ldw are written as zeros (FP8 0.0).  Thread t of

@@ -24,7 +24,13 @@ struct GemmArgs {
     // receives stage 1 of the layer that consumes this one's output (its thresholds / codebook, `bits` levels) in
     // that layer's 32-row block layout.  No residual in this mode.
     const float *next_thr = nullptr, *next_cb = nullptr;
+    // FP8 operands (launch_gemm_tile, launch_gemm_fp8; x_hat and w_hat then hold K rounded up to 128 values a row, and the
+    // quantized output is FP8 too): products are multiplied by fp8_inv, a power of two, before the bias.
+    bool fp8 = false;
+    float fp8_inv = 1.0f;
 };
+// 4 KB units (32 rows x 128 bytes) of a row block of an operand.
+inline int operand_units(int K, bool fp8) { return fp8 ? (K + 127) / 128 : K / 64; }
 
 // Large-M kernel (256-column x up-to-256-row workgroup tiles); requires K >= 64.
 void launch_gemm_stream(const GemmArgs &g, hipStream_t stream);
@@ -61,6 +67,8 @@ int device_cus();
 // Prepared operands (arcq_prepare): g.x_hat in the 32-row block layout, w_hat in the 32-column block layout; N a multiple
 // of 32, K of 64.
 void launch_gemm_tile(const GemmArgs &g, const void *w_hat, hipStream_t stream);
+// FP8 operands, w_hat row-major [N][K rounded up to 128].
+void launch_gemm_fp8(const GemmArgs &g, const void *w_hat, hipStream_t stream);
 
 // Small-M kernel (64 x 64 tiles, K split across the waves of a workgroup); requires K >= 64.
 void launch_gemm_splitk(const GemmArgs &g, hipStream_t stream);

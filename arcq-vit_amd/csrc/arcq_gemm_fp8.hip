@@ -16,6 +16,7 @@
 // order in fp32, whatever the pass structure.
 #include "arcq_common.h"
 #include "arcq_gemm.h"
+#include "arcq_act_quant_core.h"
 
 #include <stdlib.h>
 #include <type_traits>
@@ -51,11 +52,14 @@ template <int V> __device__ __forceinline__ void wait_vmcnt()
     asm volatile("" ::: "memory");
 }
 
-template <typename TOUT, int WAVES, int SG, bool DB>
+// NQ = 0, or the bits of the consuming layer's quantizer (y then receives its FP8 operand; fp16 outputs, N a multiple of 64).
+template <typename TOUT, int WAVES, int SG, bool DB, int NQ>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_fp8_kernel(const uint8_t *__restrict__ xb, const float *__restrict__ bias, TOUT *__restrict__ y, int M, int N, int K,
-                int row_ranges, int blocks_per_range, const uint8_t *__restrict__ w_hat, float inv_mult)
+                int row_ranges, int blocks_per_range, const uint8_t *__restrict__ w_hat, float inv_mult,
+                const TOUT *__restrict__ residual, int gelu, const float *__restrict__ nx_thr, const float *__restrict__ nx_cb)
 {
+    static_assert(NQ == 0 || sizeof(TOUT) == 2, "the next layer's stage 1 works on fp16 outputs");
     constexpr int kWaves = WAVES;
     constexpr int kSliceGroups = SG;
     constexpr int kPieces = Fp8Cfg<WAVES, SG, DB>::kPieces;
@@ -96,6 +100,8 @@ gemm_fp8_kernel(const uint8_t *__restrict__ xb, const float *__restrict__ bias, 
     unsigned char *stage = smem + kAllSlabs + wave * kStageTile;
 
     if (tid < kSlabN) s_bias[tid] = (bias && n_base + tid < N) ? bias[n_base + tid] : 0.0f;
+    unsigned char *nq_lds = smem + Fp8Cfg<WAVES, SG, DB>::kSmem;
+    if constexpr (NQ != 0) next_quant_setup<NQ>(nx_thr, nx_cb, nq_lds, tid, 64 * WAVES);      // (the first slab fill's barriers publish it)
     // Direct global -> LDS loads: the slab is filled as one flat run of 16-byte pieces (piece p = row * kPieces +
     // column; the hardware writes lane l's piece at the wave-uniform LDS base + 16 l), 64 pieces per instruction
     // whatever the row length; padding pieces and the columns past a short last slice are skipped.  The caller
@@ -289,6 +295,13 @@ gemm_fp8_kernel(const uint8_t *__restrict__ xb, const float *__restrict__ bias, 
                     }
                 }
                 __builtin_amdgcn_wave_barrier();
+                if constexpr (NQ != 0) {
+                    const int c0 = n_base + jb * 32 + ch * kChunkCols;          // the chunk is one group of the consumer's rows
+                    if (c0 < N)
+                        next_quant_block<NQ, true>(nq_lds, kWaves, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
+                    __builtin_amdgcn_wave_barrier();
+                    continue;
+                }
                 const int col = n_base + jb * 32 + ch * kChunkCols + (lane & 7) * kVec;
                 const int row0 = pblk * 32 + (lane >> 3);
                 TOUT *dst0 = y + static_cast<int64_t>(row0) * N + col;
@@ -296,6 +309,13 @@ gemm_fp8_kernel(const uint8_t *__restrict__ xb, const float *__restrict__ bias, 
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     v[i] = *reinterpret_cast<const u32x4_t *>(stage + (i * 8 + (lane >> 3)) * kStageRow + (lane & 7) * 16);
+                if (residual || gelu) {          // wave-uniform
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (row0 + i * 8 < M && col < N)
+                            post_ops16<TOUT>(v[i], residual ? residual + static_cast<int64_t>(row0 + i * 8) * N + col : nullptr,
+                                             gelu != 0, (N % kVec) == 0 ? kVec : N - col);
+                }
                 if (whole) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
@@ -467,28 +487,41 @@ gemm_fp8_kernel(const uint8_t *__restrict__ xb, const float *__restrict__ bias, 
     }
 }
 
-template <typename TOUT, int WAVES, int SG, bool DB>
-void launch_fp8_t(const void *x8, const void *w8, const float *bias, float inv_mult, void *y, int M, int N, int K,
-                  hipStream_t stream)
+template <typename TOUT, int NQ>
+void launch_fp8_t(const GemmArgs &g, const void *w8, hipStream_t stream)
 {
-    auto kernel = gemm_fp8_kernel<TOUT, WAVES, SG, DB>;
-    constexpr int kSmem = Fp8Cfg<WAVES, SG, DB>::kSmem;
-    allow_dynamic_lds<gemm_fp8_kernel<TOUT, WAVES, SG, DB>>(kSmem);
+    constexpr int kSmem = Fp8Cfg<8, 3, true>::kSmem + (NQ ? next_quant_lds_bytes(NQ) : 0);
+    allow_dynamic_lds<gemm_fp8_kernel<TOUT, 8, 3, true, NQ>>(kSmem);
     // Row ranges: one workgroup per compute unit (tiles = slabs x ranges ~ the number of compute units).
-    const int n_slabs = (N + kSlabN - 1) / kSlabN;
-    const int total_blocks = (M + 31) / 32;
+    const int n_slabs = (g.N + kSlabN - 1) / kSlabN;
+    const int total_blocks = (g.M + 31) / 32;
     int ranges = device_cus() / n_slabs;
     if (ranges < 1) ranges = 1;
     if (ranges > total_blocks) ranges = total_blocks;
     const int blocks_per_range = (total_blocks + ranges - 1) / ranges;
     ranges = (total_blocks + blocks_per_range - 1) / blocks_per_range;
     const int tiles = n_slabs * ranges;
-    hipLaunchKernelGGL(kernel, dim3(8 * ((tiles + 7) / 8)), dim3(64 * WAVES), kSmem, stream,
-                       static_cast<const uint8_t *>(x8), bias, static_cast<TOUT *>(y), M, N, K, ranges, blocks_per_range,
-                       static_cast<const uint8_t *>(w8), inv_mult);
+    hipLaunchKernelGGL((gemm_fp8_kernel<TOUT, 8, 3, true, NQ>), dim3(8 * ((tiles + 7) / 8)), dim3(64 * 8), kSmem, stream,
+                       static_cast<const uint8_t *>(g.x_hat), g.bias, static_cast<TOUT *>(g.y), g.M, g.N, 128 * operand_units(g.K, true),
+                       ranges, blocks_per_range, static_cast<const uint8_t *>(w8), g.fp8_inv, static_cast<const TOUT *>(g.residual),
+                       g.gelu ? 1 : 0, g.next_thr, g.next_cb);
 }
 
 }  // namespace
+
+void launch_gemm_fp8(const GemmArgs &g, const void *w_hat, hipStream_t stream)
+{
+    if (g.next_thr) {
+        if (g.bits == 4) launch_fp8_t<__half, 4>(g, w_hat, stream);
+        else if (g.bits == 3) launch_fp8_t<__half, 3>(g, w_hat, stream);
+        else launch_fp8_t<__half, 2>(g, w_hat, stream);
+    } else if (g.y_f16) {
+        launch_fp8_t<__half, 0>(g, w_hat, stream);
+    } else {
+        launch_fp8_t<float, 0>(g, w_hat, stream);
+    }
+}
+
 }  // namespace arcq
 
 using namespace arcq;
@@ -509,11 +542,10 @@ ARCQ_API int arcq_linear_fp8_blocked(const void *x8_blocked, const void *w8, con
         return fail(ARCQ_ERR_SHAPE, "arcq_linear_fp8_blocked: M, N or K too large");
     if (!aligned(x8_blocked, 16) || !aligned(w8, 16) || !aligned(y, 16))
         return fail(ARCQ_ERR_ALIGN, "arcq_linear_fp8_blocked: x8_blocked, w8 and y must be 16-byte aligned");
-    const float inv = 1.0f / w_mult;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (y_dtype == ARCQ_F16)
-        launch_fp8_t<__half, 8, 3, true>(x8_blocked, w8, bias, inv, y, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), st);
-    else
-        launch_fp8_t<float, 8, 3, true>(x8_blocked, w8, bias, inv, y, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), st);
+    GemmArgs g{x8_blocked, nullptr, nullptr, nullptr, nullptr, nullptr, bias, y, y_dtype == ARCQ_F16, static_cast<int>(M),
+               static_cast<int>(N), static_cast<int>(K), 4};
+    g.fp8 = true;
+    g.fp8_inv = 1.0f / w_mult;
+    launch_gemm_fp8(g, w8, static_cast<hipStream_t>(stream));
     return launch_status("arcq_linear_fp8_blocked");
 }

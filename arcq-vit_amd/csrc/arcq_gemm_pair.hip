@@ -55,7 +55,7 @@ template <int V> __device__ __forceinline__ void wait_vmcnt()
 
 // NQ = 0, or the bits (2 / 3 / 4) of the activation quantizer of the layer that consumes this one's output: y then
 // receives that layer's x_hat (stage 1 of the rounded, optionally GELU'd output) in the block layout instead of the
-// output itself (arcq_act_quant_core.h, next_quant_chunk); fp16 output and N a multiple of 64 only.
+// output itself (arcq_act_quant_core.h, next_quant_block); fp16 output and N a multiple of 64 only.
 template <typename TOUT, int WAVES, int SG, bool DB, int NQ>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, TOUT *__restrict__ y, int M, int N, int K,
@@ -285,9 +285,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
                 if constexpr (NQ != 0) {
                     const int c0 = n_base + jb * 32 + ch * kChunkCols;          // the chunk is one group of the consumer's rows
                     if (c0 < N)
-                        next_quant_chunk<NQ>(nq_lds, kWaves, stage, kStageRow, lane, gelu != 0, 1.0e-6f,
-                                             reinterpret_cast<__half *>(y) + static_cast<int64_t>(pblk) * 32 * N,
-                                             min(32, M - pblk * 32), c0 / 8);
+                        next_quant_block<NQ, false>(nq_lds, kWaves, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
                     __builtin_amdgcn_wave_barrier();
                     continue;
                 }

@@ -75,7 +75,7 @@ __device__ __forceinline__ uint32_t code_at(const uint32_t (&w)[BITS], int q)
 // where the registers allow it: the LDS round trip under load is longer than one k-step of four MFMAs).
 // NQ = 0, or the bits (2 / 3 / 4) of the activation quantizer of the layer that consumes this one's output: y then
 // receives that layer's x_hat in the block layout instead of the output itself (arcq_act_quant_core.h,
-// next_quant_chunk); fp16 output, N a multiple of 64, copied weights and eight waves only.
+// next_quant_block); fp16 output, N a multiple of 64, copied weights and eight waves only.
 template <int BITS, typename TOUT, bool PRE, int WAVES, int AHEAD, int NQ = 0>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_slab8_kernel(const __half *__restrict__ xb, const uint8_t *__restrict__ pw, const float *__restrict__ cb,
@@ -393,9 +393,7 @@ gemm_slab8_kernel(const __half *__restrict__ xb, const uint8_t *__restrict__ pw,
                 if constexpr (NQ != 0) {
                     const int c0 = n_base + jb * 32 + ch * kChunkCols;          // the chunk is one group of the consumer's rows
                     if (c0 < N)
-                        next_quant_chunk<NQ>(nq_lds, kWaves, stage, kStageRow, lane, gelu != 0, 1.0e-6f,
-                                             reinterpret_cast<__half *>(y) + static_cast<int64_t>(pblk) * 32 * N,
-                                             min(32, M - pblk * 32), c0 / 8);
+                        next_quant_block<NQ, false>(nq_lds, kWaves, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
                     __builtin_amdgcn_wave_barrier();
                     continue;
                 }

@@ -20,31 +20,48 @@
 #include "arcq_act_quant_core.h"
 #include "arcq_gemm.h"
 
+#include <type_traits>
+
 namespace arcq {
 namespace {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef int i32x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kStages = 4;
-constexpr int kGroupBytes = 4096;           // 32 rows x 64 values
+constexpr int kGroupBytes = 4096;           // 32 rows x 64 values (FP8: 128 values)
 
 template <int V> __device__ __forceinline__ void wait_vm()
 {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(V) : "memory");
 }
 
-// Outputs of an accumulator register block -> fp16 / fp32 in an LDS tile (rows `pitch` bytes apart), bias added.
-template <typename TOUT>
-__device__ __forceinline__ void stage_block(const float16_t &acc, const float *s_bias, unsigned char *tile, int pitch, int lr, int lh)
+// FP8 operands: one MFMA of 64 k-values from two 16-byte pieces of each operand.
+__device__ __forceinline__ float16_t mfma_fp8(const u32x4_t (&w)[2], const u32x4_t (&x)[2], const float16_t &acc)
+{
+    i32x8_t wf, xf;
+    __builtin_memcpy(&wf, &w, 32);
+    __builtin_memcpy(&xf, &x, 32);
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf, xf, acc, 0, 0, 0, 0, 0, 0);
+}
+
+// Outputs of an accumulator register block -> fp16 / fp32 in an LDS tile (rows `pitch` bytes apart), bias added (F8: after the
+// multiplication by `inv`, a power of two, which is exact).
+template <typename TOUT, bool F8>
+__device__ __forceinline__ void stage_block(const float16_t &acc, const float *s_bias, unsigned char *tile, int pitch, int lr, int lh,
+                                            float inv)
 {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const float4 b = *reinterpret_cast<const float4 *>(s_bias + 8 * q + 4 * lh);
-        const float o0 = acc[4 * q] + b.x, o1 = acc[4 * q + 1] + b.y, o2 = acc[4 * q + 2] + b.z, o3 = acc[4 * q + 3] + b.w;
+        float a[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = F8 ? acc[4 * q + e] * inv : acc[4 * q + e];
+        const float o0 = a[0] + b.x, o1 = a[1] + b.y, o2 = a[2] + b.z, o3 = a[3] + b.w;
         unsigned char *dst = tile + lr * pitch + (8 * q + 4 * lh) * static_cast<int>(sizeof(TOUT));
         if constexpr (sizeof(TOUT) == 2) {
             const __half2 lo = __floats2half2_rn(o0, o1), hi = __floats2half2_rn(o2, o3);
@@ -62,11 +79,11 @@ __device__ __forceinline__ void stage_block(const float16_t &acc, const float *s
 }
 
 // WM x WN waves per workgroup; NQ = 0 or the bits of the consuming layer's quantizer (y then receives its x_hat).
-template <int TM, int TN, int WM, int WN, typename TOUT, int NQ>
+template <int TM, int TN, int WM, int WN, typename TOUT, int NQ, bool F8>
 __global__ void __launch_bounds__(64 * WM * WN)
-gemm_tile_kernel(const __half *__restrict__ xb, const __half *__restrict__ wb, const float *__restrict__ bias,
-                 TOUT *__restrict__ y, int M, int N, int K, int m_tiles, int n_tiles, int m_fastest,
-                 const TOUT *__restrict__ residual, int gelu, const float *__restrict__ nx_thr, const float *__restrict__ nx_cb)
+gemm_tile_kernel(const unsigned char *__restrict__ xb, const unsigned char *__restrict__ wb, const float *__restrict__ bias,
+                 TOUT *__restrict__ y, int M, int N, int G, int m_tiles, int n_tiles, int m_fastest,
+                 const TOUT *__restrict__ residual, int gelu, const float *__restrict__ nx_thr, const float *__restrict__ nx_cb, float inv)
 {
     constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
     constexpr int RBT = TM / 32, CBT = TN / 32;                  // 32-row / 32-column blocks of the tile
@@ -91,7 +108,6 @@ gemm_tile_kernel(const __half *__restrict__ xb, const __half *__restrict__ wb, c
     const int mt = m_fastest ? tile_no % m_tiles : tile_no / n_tiles;
     const int nt = m_fastest ? tile_no / m_tiles : tile_no % n_tiles;
     const int m0 = mt * TM, n0 = nt * TN;
-    const int G = K / 64;
     const int row_blocks = (M + 31) / 32, col_blocks = N / 32;
 
     // This wave's loads: load q moves the quarter q % 4 of block q / 4 of the stage.  LDS always holds 32 rows per piece
@@ -106,12 +122,12 @@ gemm_tile_kernel(const __half *__restrict__ xb, const __half *__restrict__ wb, c
         if (b < RBT) {
             const int blk = min(m0 / 32 + b, row_blocks - 1);
             const int r = min(32, M - blk * 32);
-            src[j] = reinterpret_cast<const char *>(xb) + static_cast<int64_t>(blk) * K * 64;
+            src[j] = reinterpret_cast<const char *>(xb) + static_cast<int64_t>(blk) * G * kGroupBytes;
             voff[j] = static_cast<uint32_t>(((piece >> 5) * r + min(piece & 31, r - 1)) * 16);
             gstep[j] = static_cast<uint32_t>(r * 128);
         } else {
             const int blk = min(n0 / 32 + (b - RBT), col_blocks - 1);
-            src[j] = reinterpret_cast<const char *>(wb) + static_cast<int64_t>(blk) * K * 64;
+            src[j] = reinterpret_cast<const char *>(wb) + static_cast<int64_t>(blk) * G * kGroupBytes;
             voff[j] = static_cast<uint32_t>(piece * 16);
             gstep[j] = kGroupBytes;
         }
@@ -142,8 +158,9 @@ gemm_tile_kernel(const __half *__restrict__ xb, const __half *__restrict__ wb, c
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
     const int wm = wave / WN, wn = wave - wm * WN;
-    const unsigned char *a_lane = smem + wm * RB * kGroupBytes + lh * 2048 + lr * 16;
-    const unsigned char *b_lane = smem + (RBT + wn * CB) * kGroupBytes + lh * 2048 + lr * 16;
+    constexpr int kHalf = F8 ? 1024 : 2048;      // FP8: lane half h covers k = 64 step + 32 h ... + 31, two pieces
+    const unsigned char *a_lane = smem + wm * RB * kGroupBytes + lh * kHalf + lr * 16;
+    const unsigned char *b_lane = smem + (RBT + wn * CB) * kGroupBytes + lh * kHalf + lr * 16;
     for (int g = 0; g < G; ++g) {
         // Group g has landed for this wave; after the barrier for all of them, and everyone is done with group g - 1.
         const int ahead = G - 1 - g;
@@ -153,6 +170,23 @@ gemm_tile_kernel(const __half *__restrict__ xb, const __half *__restrict__ wb, c
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (g + kStages - 1 < G) issue((g + kStages - 1) % kStages);
         const int off = (g % kStages) * kStageBytes;
+        if constexpr (F8) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                u32x4_t af[RB][2], bf[CB][2];
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+#pragma unroll
+                    for (int i = 0; i < RB; ++i) af[i][p] = *reinterpret_cast<const u32x4_t *>(a_lane + off + i * kGroupBytes + s * 2048 + p * 512);
+#pragma unroll
+                    for (int j = 0; j < CB; ++j) bf[j][p] = *reinterpret_cast<const u32x4_t *>(b_lane + off + j * kGroupBytes + s * 2048 + p * 512);
+                }
+#pragma unroll
+                for (int i = 0; i < RB; ++i)
+#pragma unroll
+                    for (int j = 0; j < CB; ++j) acc[i][j] = mfma_fp8(bf[j], af[i], acc[i][j]);
+            }
+        } else
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
             half8_t af[RB], bf[CB];
@@ -174,8 +208,8 @@ gemm_tile_kernel(const __half *__restrict__ xb, const __half *__restrict__ wb, c
     for (int i = 0; i < RB; ++i)
 #pragma unroll
         for (int j = 0; j < CB; ++j)
-            stage_block<TOUT>(acc[i][j], s_bias + (wn * CB + j) * 32, smem + (wm * RB + i) * 32 * kOutPitch + (wn * CB + j) * 32 * static_cast<int>(sizeof(TOUT)),
-                              kOutPitch, lr, lh);
+            stage_block<TOUT, F8>(acc[i][j], s_bias + (wn * CB + j) * 32, smem + (wm * RB + i) * 32 * kOutPitch + (wn * CB + j) * 32 * static_cast<int>(sizeof(TOUT)),
+                                  kOutPitch, lr, lh, inv);
     __syncthreads();
     if constexpr (NQ != 0) {
         static_assert(TN % 64 == 0 && sizeof(TOUT) == 2, "whole groups of fp16 outputs");
@@ -184,8 +218,8 @@ gemm_tile_kernel(const __half *__restrict__ xb, const __half *__restrict__ wb, c
             const int rb = job % RBT, gc = job / RBT;
             const int blk = m0 / 32 + rb, c0 = n0 + gc * 64;
             if (blk < row_blocks && c0 < N)
-                next_quant_chunk<NQ>(nq_lds, kWaves, smem + rb * 32 * kOutPitch + gc * 128, kOutPitch, lane, gelu != 0, 1.0e-6f,
-                                     reinterpret_cast<__half *>(y) + static_cast<int64_t>(blk) * 32 * N, min(32, M - blk * 32), c0 / 8);
+                next_quant_block<NQ, F8>(nq_lds, kWaves, smem + rb * 32 * kOutPitch + gc * 128, kOutPitch, lane, gelu != 0, 1.0e-6f, y, blk, M,
+                                         N, c0);
         }
     } else {
         constexpr int kVec = 16 / static_cast<int>(sizeof(TOUT));
@@ -206,24 +240,25 @@ gemm_tile_kernel(const __half *__restrict__ xb, const __half *__restrict__ wb, c
     }
 }
 
-template <int TM, int TN, int WM, int WN, typename TOUT, int NQ>
+template <int TM, int TN, int WM, int WN, typename TOUT, int NQ, bool F8>
 void launch_tile(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 {
     constexpr int kSmem = kStages * (TM / 32 + TN / 32) * kGroupBytes + TN * 4 + (NQ ? next_quant_lds_bytes(NQ) : 0);
-    allow_dynamic_lds<gemm_tile_kernel<TM, TN, WM, WN, TOUT, NQ>>(kSmem);
+    allow_dynamic_lds<gemm_tile_kernel<TM, TN, WM, WN, TOUT, NQ, F8>>(kSmem);
     const int mt = (g.M + TM - 1) / TM, nt = (g.N + TN - 1) / TN;
     const int m_fastest = g.M < g.N ? 1 : 0;
-    hipLaunchKernelGGL((gemm_tile_kernel<TM, TN, WM, WN, TOUT, NQ>), dim3(8 * ((mt * nt + 7) / 8)), dim3(64 * WM * WN), kSmem, stream,
-                       static_cast<const __half *>(g.x_hat), static_cast<const __half *>(w_hat), g.bias, static_cast<TOUT *>(g.y), g.M, g.N,
-                       g.K, mt, nt, m_fastest, static_cast<const TOUT *>(g.residual), g.gelu ? 1 : 0, g.next_thr, g.next_cb);
+    hipLaunchKernelGGL((gemm_tile_kernel<TM, TN, WM, WN, TOUT, NQ, F8>), dim3(8 * ((mt * nt + 7) / 8)), dim3(64 * WM * WN), kSmem, stream,
+                       static_cast<const unsigned char *>(g.x_hat), static_cast<const unsigned char *>(w_hat), g.bias,
+                       static_cast<TOUT *>(g.y), g.M, g.N, operand_units(g.K, F8), mt, nt, m_fastest, static_cast<const TOUT *>(g.residual),
+                       g.gelu ? 1 : 0, g.next_thr, g.next_cb, g.fp8_inv);
 }
 
 // ---- fewer than 512 rows ------------------------------------------------------------------------------------------
-template <typename TOUT, int RB, int CB, int NQ>
+template <typename TOUT, int RB, int CB, int NQ, bool F8>
 __global__ void __launch_bounds__(512)
-gemm_tile_split_kernel(const __half *__restrict__ xb, const __half *__restrict__ wb, const float *__restrict__ bias,
-                       TOUT *__restrict__ y, int M, int N, int K, const TOUT *__restrict__ residual, int gelu,
-                       const float *__restrict__ nx_thr, const float *__restrict__ nx_cb)
+gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char *__restrict__ wb, const float *__restrict__ bias,
+                       TOUT *__restrict__ y, int M, int N, int G, const TOUT *__restrict__ residual, int gelu,
+                       const float *__restrict__ nx_thr, const float *__restrict__ nx_cb, float inv)
 {
     constexpr int NW = 8;
     constexpr int RT = 32 * RB, CT = 32 * CB;
@@ -232,7 +267,6 @@ gemm_tile_split_kernel(const __half *__restrict__ xb, const __half *__restrict__
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lh = lane >> 5;
     const int m0 = blockIdx.y * RT, n0 = blockIdx.x * CT;
-    const int G = K / 64;
     const int row_blocks = (M + 31) / 32, col_blocks = N / 32;
     const char *a_src[RB], *b_src[CB];
     int a_step[RB];                      // bytes between k-steps
@@ -241,21 +275,23 @@ gemm_tile_split_kernel(const __half *__restrict__ xb, const __half *__restrict__
         const int blk = min(m0 / 32 + i, row_blocks - 1);
         const int r = min(32, M - blk * 32);
         a_step[i] = r * 16;
-        a_src[i] = reinterpret_cast<const char *>(xb) + static_cast<int64_t>(blk) * K * 64 + lh * 4 * a_step[i] + min(lr, r - 1) * 16;
+        a_src[i] = reinterpret_cast<const char *>(xb) + static_cast<int64_t>(blk) * G * kGroupBytes + lh * (F8 ? 2 : 4) * a_step[i] +
+                   min(lr, r - 1) * 16;
     }
 #pragma unroll
     for (int j = 0; j < CB; ++j) {
         const int blk = min(n0 / 32 + j, col_blocks - 1);
-        b_src[j] = reinterpret_cast<const char *>(wb) + static_cast<int64_t>(blk) * K * 64 + lh * 2048 + lr * 16;
+        b_src[j] = reinterpret_cast<const char *>(wb) + static_cast<int64_t>(blk) * G * kGroupBytes + lh * (F8 ? 1024 : 2048) + lr * 16;
     }
     struct Ops { u32x4_t a[RB][4], b[CB][4]; };
     auto fetch = [&](int g, Ops &o) __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
+            const int p = F8 ? (kk >> 1) * 4 + (kk & 1) : kk;        // FP8: two pieces per k-step of 64
 #pragma unroll
-            for (int i = 0; i < RB; ++i) o.a[i][kk] = *reinterpret_cast<const u32x4_t *>(a_src[i] + (g * 8 + kk) * a_step[i]);
+            for (int i = 0; i < RB; ++i) o.a[i][kk] = *reinterpret_cast<const u32x4_t *>(a_src[i] + (g * 8 + p) * a_step[i]);
 #pragma unroll
-            for (int j = 0; j < CB; ++j) o.b[j][kk] = *reinterpret_cast<const u32x4_t *>(b_src[j] + g * kGroupBytes + kk * 512);
+            for (int j = 0; j < CB; ++j) o.b[j][kk] = *reinterpret_cast<const u32x4_t *>(b_src[j] + g * kGroupBytes + p * 512);
         }
     };
     Ops o0, o1;
@@ -273,6 +309,17 @@ gemm_tile_split_kernel(const __half *__restrict__ xb, const __half *__restrict__
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
     auto compute = [&](const Ops &o) __attribute__((always_inline)) {
+        if constexpr (F8) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int i = 0; i < RB; ++i)
+#pragma unroll
+                    for (int j = 0; j < CB; ++j) {
+                        const u32x4_t w2[2] = {o.b[j][2 * s], o.b[j][2 * s + 1]}, x2[2] = {o.a[i][2 * s], o.a[i][2 * s + 1]};
+                        acc[i][j] = mfma_fp8(w2, x2, acc[i][j]);
+                    }
+        } else
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
             half8_t af[RB], bf[CB];
@@ -343,7 +390,7 @@ gemm_tile_split_kernel(const __half *__restrict__ xb, const __half *__restrict__
     }
     TOUT out[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) out[e] = from_float<TOUT>(sum[e] + bv[e]);
+    for (int e = 0; e < E; ++e) out[e] = from_float<TOUT>((F8 ? sum[e] * inv : sum[e]) + bv[e]);
     if constexpr (NQ != 0) {
         // The rounded (GELU'd) outputs as an fp16 tile over the partial sums of wave 0 .. (everyone has read them), then
         // stage 1 of the consumer on its 32-row chunks of 64 columns.
@@ -359,8 +406,7 @@ gemm_tile_split_kernel(const __half *__restrict__ xb, const __half *__restrict__
         if (wave < RB) {
             const int blk = m0 / 32 + wave;
             if (blk < row_blocks && n0 < N)
-                next_quant_chunk<NQ>(nq_lds, NW, smem + wave * 32 * kStageRow, kStageRow, lane, false, 1.0e-6f,
-                                     reinterpret_cast<__half *>(y) + static_cast<int64_t>(blk) * 32 * N, min(32, M - blk * 32), n0 / 8);
+                next_quant_block<NQ, F8>(nq_lds, NW, smem + wave * 32 * kStageRow, kStageRow, lane, false, 1.0e-6f, y, blk, M, N, n0);
         }
     } else if (live) {
         if (residual || gelu) {
@@ -372,18 +418,19 @@ gemm_tile_split_kernel(const __half *__restrict__ xb, const __half *__restrict__
     }
 }
 
-template <typename TOUT, int RB, int CB, int NQ>
+template <typename TOUT, int RB, int CB, int NQ, bool F8>
 void launch_split(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 {
     constexpr int kSmem = 8 * 32 * RB * (32 * CB * 4 + 16) + (NQ ? next_quant_lds_bytes(NQ) : 0);
-    allow_dynamic_lds<gemm_tile_split_kernel<TOUT, RB, CB, NQ>>(kSmem);
+    allow_dynamic_lds<gemm_tile_split_kernel<TOUT, RB, CB, NQ, F8>>(kSmem);
     const dim3 grid((g.N + 32 * CB - 1) / (32 * CB), (g.M + 32 * RB - 1) / (32 * RB));
-    hipLaunchKernelGGL((gemm_tile_split_kernel<TOUT, RB, CB, NQ>), grid, dim3(512), kSmem, stream, static_cast<const __half *>(g.x_hat),
-                       static_cast<const __half *>(w_hat), g.bias, static_cast<TOUT *>(g.y), g.M, g.N, g.K,
-                       static_cast<const TOUT *>(g.residual), g.gelu ? 1 : 0, g.next_thr, g.next_cb);
+    hipLaunchKernelGGL((gemm_tile_split_kernel<TOUT, RB, CB, NQ, F8>), grid, dim3(512), kSmem, stream,
+                       static_cast<const unsigned char *>(g.x_hat), static_cast<const unsigned char *>(w_hat), g.bias,
+                       static_cast<TOUT *>(g.y), g.M, g.N, operand_units(g.K, F8), static_cast<const TOUT *>(g.residual), g.gelu ? 1 : 0,
+                       g.next_thr, g.next_cb, g.fp8_inv);
 }
 
-template <typename TOUT, int NQ>
+template <typename TOUT, int NQ, bool F8>
 void pick(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 {
     const int cus = device_cus();
@@ -391,31 +438,37 @@ void pick(const GemmArgs &g, const void *w_hat, hipStream_t stream)
         const int64_t t11 = static_cast<int64_t>((g.M + 31) / 32) * (g.N / 32);
         const int64_t t12 = static_cast<int64_t>((g.M + 31) / 32) * ((g.N + 63) / 64);
         if constexpr (NQ == 0) {
-            if (t11 <= 2 * cus) return launch_split<TOUT, 1, 1, 0>(g, w_hat, stream);
+            if (t11 <= 2 * cus) return launch_split<TOUT, 1, 1, 0, F8>(g, w_hat, stream);
         }
-        if (t12 <= 2 * cus) return launch_split<TOUT, 1, 2, NQ>(g, w_hat, stream);
-        return launch_split<TOUT, 2, 2, NQ>(g, w_hat, stream);
+        if (t12 <= 2 * cus) return launch_split<TOUT, 1, 2, NQ, F8>(g, w_hat, stream);
+        return launch_split<TOUT, 2, 2, NQ, F8>(g, w_hat, stream);
     }
     // 64 x 64 tiles (two workgroups on a CU) while they fit the chip at once, 128 x 128 beyond: measured crossovers between
     // 480 and 600 tiles at K = 384, 768 and 1 024 (384 -> 1 536 at 1 576 rows, 600 tiles: 7.9 against 6.9 us; 1 024 -> 3 072 at
     // 591 rows, 480 tiles: 9.2 against 11.5).  64 x 128 was never the fastest (one workgroup per CU for its LDS).
     const int64_t t64 = static_cast<int64_t>((g.M + 63) / 64) * ((g.N + 63) / 64);
-    if (t64 <= 2 * cus) return launch_tile<64, 64, 2, 2, TOUT, NQ>(g, w_hat, stream);
-    return launch_tile<128, 128, 2, 4, TOUT, NQ>(g, w_hat, stream);
+    if (t64 <= 2 * cus) return launch_tile<64, 64, 2, 2, TOUT, NQ, F8>(g, w_hat, stream);
+    return launch_tile<128, 128, 2, 4, TOUT, NQ, F8>(g, w_hat, stream);
 }
 
 }  // namespace
 
 void launch_gemm_tile(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 {
-    if (g.next_thr) {
-        if (g.bits == 4) pick<__half, 4>(g, w_hat, stream);
-        else if (g.bits == 3) pick<__half, 3>(g, w_hat, stream);
-        else pick<__half, 2>(g, w_hat, stream);
-        return;
-    }
-    if (g.y_f16) pick<__half, 0>(g, w_hat, stream);
-    else pick<float, 0>(g, w_hat, stream);
+    auto run = [&](auto f8c) {
+        constexpr bool F8 = decltype(f8c)::value;
+        if (g.next_thr) {
+            if (g.bits == 4) pick<__half, 4, F8>(g, w_hat, stream);
+            else if (g.bits == 3) pick<__half, 3, F8>(g, w_hat, stream);
+            else pick<__half, 2, F8>(g, w_hat, stream);
+        } else if (g.y_f16) {
+            pick<__half, 0, F8>(g, w_hat, stream);
+        } else {
+            pick<float, 0, F8>(g, w_hat, stream);
+        }
+    };
+    if (g.fp8) run(std::true_type{});
+    else run(std::false_type{});
 }
 
 }  // namespace arcq
@@ -424,6 +477,12 @@ using namespace arcq;
 
 // Column blocks and the tile kernels up to the size where the weight-stationary kernels have the row blocks they want:
 // 8 per workgroup for the two-blocks-per-wave kernel (gemm_pair_pays), or 6 000 rows for the eight-wave one.
+ARCQ_API int arcq_prepared_row_major_fp8(int64_t M, int64_t N, int64_t K)
+{
+    (void)K;
+    return N % 32 != 0 || M >= 6000 ? 1 : 0;
+}
+
 ARCQ_API int arcq_prepared_row_major(int64_t M, int64_t N, int64_t K)
 {
     if (M < 512) return 0;
@@ -458,6 +517,14 @@ ARCQ_API int arcq_linear_prepared(const arcq_linear_prepared_args *a, void *stre
     g.gelu = a->activation == ARCQ_ACT_GELU;
     g.next_thr = a->next_thresholds;
     g.next_cb = a->next_codebook;
+    g.fp8 = a->fp8 != 0;
+    if (g.fp8) {
+        if (!(a->w_mult > 0.0f)) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_linear_prepared: w_mult must be positive");
+        g.fp8_inv = 1.0f / a->w_mult;
+        if (a->w_row_major) launch_gemm_fp8(g, a->w_hat, static_cast<hipStream_t>(stream));
+        else launch_gemm_tile(g, a->w_hat, static_cast<hipStream_t>(stream));
+        return launch_status("arcq_linear_prepared");
+    }
     if (a->w_row_major) {
         if (a->M < 512) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_linear_prepared: row-major weights need 512 rows or more");
         launch_gemm_slab8(g, a->w_hat, static_cast<hipStream_t>(stream));

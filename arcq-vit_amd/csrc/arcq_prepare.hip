@@ -13,6 +13,7 @@
 //     and four 16-byte stores per group and lane, every store of the wave two 512-byte runs of the weight block layout.
 //     All index arithmetic is 32-bit.  (weight_dequant8_kernel owns 8 weights per thread: the 64-bit division and the
 //     three metadata loads per 8 weights made it 10 us for 4096 x 1024; here 4.)
+// FP8 operands (F8): the same work with pieces of 16 values and rows padded with zeros to 128 values.
 // Arithmetic: arcq_act_quant_core.h and the stage-2 expression, unchanged -- bit-identical to the stand-alone kernels.
 #include "arcq_act_quant_core.h"
 #include "arcq_gemm.h"
@@ -29,8 +30,9 @@ constexpr int kPrepThreads = 64 * kPrepWaves;
 struct PrepWeights {
     const uint8_t *packed;
     const float *cb, *center, *scale, *code_sum;
-    __half *out;             // [N/32][K/8][32][8], or [N][K] if row_major
+    void *out;               // [N/32][K/8][32][8] fp16, or [N][K] if row_major; FP8: [N/32][Kp/16][32][16] or [N][Kp]
     int N, G;                // G = K / 64
+    float mult;              // FP8: power of two in front of the rounding
     int row_major;
     unsigned blocks;         // workgroups (0: no such job)
 };
@@ -59,8 +61,20 @@ __device__ __forceinline__ uint32_t prep_code_at(const uint32_t (&w)[BITS], int 
     return v & ((1u << BITS) - 1u);
 }
 
+// Sixteen reconstructed weights times `mult` as one FP8 piece.
+__device__ __forceinline__ void weights_fp8x16(const float (&v)[32], int j0, float mg, float s, float c, float mult, uint32_t (&o)[4])
+{
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        float t[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] = fma_f32(v[j0 + 8 * p + e] - mg, s, c) * mult;
+        to_fp8x8(t, o[2 * p], o[2 * p + 1]);
+    }
+}
+
 // One wave: columns 32 nb ... + 31 of groups 4 gq ... + 3 of a layer's weights.  `lut`: the codebook per lane.
-template <int BITS>
+template <int BITS, bool F8>
 __device__ __forceinline__ void prep_weights(const PrepWeights &w, unsigned block, float *lut)
 {
     constexpr int L = 1 << BITS;
@@ -89,7 +103,10 @@ __device__ __forceinline__ void prep_weights(const PrepWeights &w, unsigned bloc
     }
     __syncthreads();
     const char *lut_lane = reinterpret_cast<const char *>(lut) + lane * 4;
-    __half *dst = w.out + static_cast<int64_t>(nb) * (w.G * 2048) + (g0 * 8 + half * 4) * 256 + (lane & 31) * 8;
+    const int row_groups = F8 ? (w.G + 1) / 2 * 2 : w.G;
+    constexpr int kPieces = F8 ? 4 : 8;            // 16-byte pieces of a group
+    char *dst = static_cast<char *>(w.out) + static_cast<int64_t>(nb) * (row_groups * kPieces * 512) + (g0 * kPieces + half * (kPieces / 2)) * 512 +
+                (lane & 31) * 16;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         if (i >= ng) break;
@@ -98,30 +115,43 @@ __device__ __forceinline__ void prep_weights(const PrepWeights &w, unsigned bloc
 #pragma unroll
         for (int e = 0; e < 32; ++e) v[e] = *reinterpret_cast<const float *>(lut_lane + (prep_code_at<BITS>(codes[i], e) << 8));
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p = 0; p < kPieces / 2; ++p) {
             uint32_t o[4];
+            if constexpr (F8) {
+                weights_fp8x16(v, 16 * p, mg, s[i], c[i], w.mult, o);
+            } else {
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const __half2 h = __floats2half2_rn(fma_f32(v[p * 8 + 2 * d] - mg, s[i], c[i]), fma_f32(v[p * 8 + 2 * d + 1] - mg, s[i], c[i]));
-                o[d] = *reinterpret_cast<const uint32_t *>(&h);
+                for (int d = 0; d < 4; ++d) {
+                    const __half2 h = __floats2half2_rn(fma_f32(v[p * 8 + 2 * d] - mg, s[i], c[i]), fma_f32(v[p * 8 + 2 * d + 1] - mg, s[i], c[i]));
+                    o[d] = *reinterpret_cast<const uint32_t *>(&h);
+                }
             }
-            store_writethrough16(dst + (i * 8 + p) * 256, o[0], o[1], o[2], o[3]);
+            store_writethrough16(dst + (i * kPieces + p) * 512, o[0], o[1], o[2], o[3]);
         }
+    }
+    if (F8 && mine && g0 + ng == w.G && row_groups > w.G) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) store_writethrough16(dst + (ng * kPieces + p) * 512, 0, 0, 0, 0);
     }
 }
 
-// Row-major output: eight weights per thread, consecutive threads consecutive 16-byte pieces of a row.
-template <int BITS>
+// Row-major output: a 16-byte piece per thread, consecutive threads consecutive pieces of a row.
+template <int BITS, bool F8>
 __device__ __forceinline__ void prep_weights_rows(const PrepWeights &w, unsigned block, float *lut)
 {
     constexpr int L = 1 << BITS;
     const int lane = threadIdx.x & 63;
-    const uint32_t per_row = static_cast<uint32_t>(w.G) * 8;
+    constexpr uint32_t kPieces = F8 ? 4 : 8;       // of a group
+    const uint32_t live = static_cast<uint32_t>(w.G) * kPieces;
+    const uint32_t per_row = F8 ? (live + 7) / 8 * 8 : live;
     const uint32_t idx = block * kPrepThreads + threadIdx.x;
     const bool mine = idx < static_cast<uint32_t>(w.N) * per_row;
-    const uint32_t n = mine ? idx / per_row : 0, k8 = mine ? idx - n * per_row : 0;
-    const uint32_t codes = load_codes8<BITS>(w.packed + static_cast<int64_t>(n * per_row + k8) * BITS);
-    const int64_t mi = static_cast<int64_t>(n) * w.G + (k8 >> 3);
+    const uint32_t n = mine ? idx / per_row : 0, at = mine ? idx - n * per_row : 0;
+    const bool padding = at >= live;
+    const uint32_t k = padding ? 0 : at;
+    const uint8_t *src = w.packed + static_cast<int64_t>(n * live + k) * ((F8 ? 2 : 1) * BITS);
+    const uint32_t codes = load_codes8<BITS>(src), more = F8 ? load_codes8<BITS>(src + BITS) : 0;
+    const int64_t mi = static_cast<int64_t>(n) * w.G + k / kPieces;
     const float c = w.center[mi], s = w.scale[mi], m = w.code_sum[mi] * 0.015625f;
     if (threadIdx.x < 64) {
 #pragma unroll
@@ -129,7 +159,17 @@ __device__ __forceinline__ void prep_weights_rows(const PrepWeights &w, unsigned
     }
     __syncthreads();
     if (!mine) return;
-    uint32_t o[4];
+    uint32_t o[4] = {0, 0, 0, 0};
+    if constexpr (F8) {
+        if (!padding) {
+            float v[32];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) v[e] = lut[(((e < 8 ? codes : more) >> (BITS * (e & 7))) & (L - 1)) * 64 + lane];
+            weights_fp8x16(v, 0, m, s, c, w.mult, o);
+        }
+        store_writethrough16(static_cast<char *>(w.out) + static_cast<int64_t>(idx) * 16, o[0], o[1], o[2], o[3]);
+        return;
+    }
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
         float v[2];
@@ -138,16 +178,16 @@ __device__ __forceinline__ void prep_weights_rows(const PrepWeights &w, unsigned
         const __half2 h = __floats2half2_rn(v[0], v[1]);
         o[d] = *reinterpret_cast<const uint32_t *>(&h);
     }
-    store_writethrough16(w.out + static_cast<int64_t>(idx) * 8, o[0], o[1], o[2], o[3]);
+    store_writethrough16(static_cast<char *>(w.out) + static_cast<int64_t>(idx) * 16, o[0], o[1], o[2], o[3]);
 }
 
 // LN = true: LayerNorm over the rows first; GC = all G groups of a row (2 GC lanes per row).
 // LN = false: a wave takes R rows x GC groups; consecutive waves take consecutive group chunks.
 // rows_per_wave = R; chunks = group chunks per row (1 with a LayerNorm).
-template <typename TIN, int BITS, bool LN>
+template <typename TIN, int BITS, bool LN, bool F8>
 __global__ void __launch_bounds__(kPrepThreads)
 prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta, float ln_eps,
-               const float *__restrict__ thr, const float *__restrict__ cb, __half *__restrict__ x_hat, float eps, int rows,
+               const float *__restrict__ thr, const float *__restrict__ cb, char *__restrict__ x_hat, float eps, int rows,
                int G, int GC, int R, int chunks, int tiles, PrepWeights w0, PrepWeights w1)
 {
     constexpr int L = 1 << BITS;
@@ -161,8 +201,8 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const
         const bool second = blockIdx.x >= w0.blocks;
         const PrepWeights &w = second ? w1 : w0;
         const unsigned block = blockIdx.x - (second ? w0.blocks : 0);
-        if (w.row_major) prep_weights_rows<BITS>(w, block, lut);
-        else prep_weights<BITS>(w, block, lut);
+        if (w.row_major) prep_weights_rows<BITS, F8>(w, block, lut);
+        else prep_weights<BITS, F8>(w, block, lut);
         return;
     }
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -210,6 +250,9 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const
 #pragma unroll
     for (int w = 0; w < kPrepWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
     const float fk = static_cast<float>(K);
+    constexpr int kPieces = F8 ? 4 : 8;                     // 16-byte pieces of a group of x_hat
+    const int row_groups = F8 ? (G + 1) / 2 * 2 : G;        // with the padding
+    const int row_bytes = row_groups * kPieces * 16;
 
     const int trips = (tiles + (LN ? 1 : kPrepWaves) * wgs - 1) / ((LN ? 1 : kPrepWaves) * wgs);      // the same for every wave
     for (int trip = 0, t = first; trip < trips; ++trip, t += step) {
@@ -283,36 +326,40 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const
         group_stats32x2(xv, eps, mu, var, s);
         group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
         const float code_mean = sum_codes * 0.015625f;
-        uint4 o[4];
+        uint4 o[kPieces / 2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < kPieces / 2; ++i) {
             uint32_t w[4];
+            if constexpr (F8) {
+                xhat_fp8x16(xv, 16 * i, s, code_mean, mu, w);
+            } else {
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const int j = 8 * i + 2 * d;
-                const __half2 h = __floats2half2_rn(fma_f32(s, xv[j] - code_mean, mu), fma_f32(s, xv[j + 1] - code_mean, mu));
-                w[d] = *reinterpret_cast<const uint32_t *>(&h);
+                for (int d = 0; d < 4; ++d) {
+                    const int j = 8 * i + 2 * d;
+                    const __half2 h = __floats2half2_rn(fma_f32(s, xv[j] - code_mean, mu), fma_f32(s, xv[j + 1] - code_mean, mu));
+                    w[d] = *reinterpret_cast<const uint32_t *>(&h);
+                }
             }
             o[i] = make_uint4(w[0], w[1], w[2], w[3]);
         }
-        // ---- out: piece (k8, row) at LDS slot k8 * rows_in_tile + row, then 16 bytes per lane, rows fastest ----
+        // ---- out: piece (k, row) at LDS slot k * rows_in_tile + row, then 16 bytes per lane, rows fastest ----
         if constexpr (LN) {
             const int RW = kPrepWaves * R;
             if (lane_used) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    *reinterpret_cast<uint4 *>(tile + ((pl * 4 + i) * RW + wave * R + rl) * 16) = o[i];
+                for (int i = 0; i < kPieces / 2; ++i)
+                    *reinterpret_cast<uint4 *>(tile + ((pl * (kPieces / 2) + i) * RW + wave * R + rl) * 16) = o[i];
             }
             __syncthreads();
             const int r0 = t * RW;
-            const int pieces = GC * 8 * RW;
+            const int live = GC * kPieces * RW, pieces = row_groups * kPieces * RW;
             for (int p = tid; p < pieces; p += kPrepThreads) {
-                const int k8 = p / RW, r = p - k8 * RW;
+                const int k = p / RW, r = p - k * RW;
                 const int rr = r0 + r;
                 if (rr < rows) {
-                    const uint4 v = *reinterpret_cast<const uint4 *>(tile + p * 16);
+                    const uint4 v = !F8 || p < live ? *reinterpret_cast<const uint4 *>(tile + p * 16) : make_uint4(0, 0, 0, 0);
                     const int blk = rr >> 5, nrows = min(32, rows - blk * 32);
-                    store_writethrough16(x_hat + static_cast<int64_t>(blk) * 32 * K + (k8 * nrows + (rr & 31)) * 8, v.x, v.y, v.z, v.w);
+                    store_writethrough16(x_hat + static_cast<int64_t>(blk) * 32 * row_bytes + (k * nrows + (rr & 31)) * 16, v.x, v.y, v.z, v.w);
                 }
             }
             __syncthreads();
@@ -320,21 +367,23 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const
             unsigned char *mine = tile + wave * 4096;
             if (lane_used) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4 *>(mine + ((pl * 4 + i) * R + rl) * 16) = o[i];
+                for (int i = 0; i < kPieces / 2; ++i) *reinterpret_cast<uint4 *>(mine + ((pl * (kPieces / 2) + i) * R + rl) * 16) = o[i];
             }
             __builtin_amdgcn_wave_barrier();
-            // R is a power of two and R * GC = 32 here: 256 pieces, four per lane
+            // R is a power of two and R * GC = 32 here: 256 pieces, four per lane (FP8: two)
             const int rt0 = my_row - rl;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < kPieces / 2; ++i) {
                 const int p = i * 64 + lane;
-                const int k8 = p / R, r = p - k8 * R;
+                const int k = p / R, r = p - k * R;
                 const int rr = rt0 + r;
-                if (rr < rows && t < tiles && my_g0 * 8 + k8 < G * 8) {
+                if (rr < rows && t < tiles && my_g0 * kPieces + k < G * kPieces) {
                     const uint4 v = *reinterpret_cast<const uint4 *>(mine + p * 16);
                     const int blk = rr >> 5, nrows = min(32, rows - blk * 32);
-                    store_writethrough16(x_hat + static_cast<int64_t>(blk) * 32 * K + ((my_g0 * 8 + k8) * nrows + (rr & 31)) * 8, v.x, v.y,
-                                         v.z, v.w);
+                    char *dst = x_hat + static_cast<int64_t>(blk) * 32 * row_bytes + ((my_g0 * kPieces + k) * nrows + (rr & 31)) * 16;
+                    store_writethrough16(dst, v.x, v.y, v.z, v.w);
+                    // (an odd number of groups: GC = 1, and the last group's tile writes the padding group too)
+                    if (F8 && row_groups > G && my_g0 == G - 1) store_writethrough16(dst + kPieces * nrows * 16, 0, 0, 0, 0);
                 }
             }
             __builtin_amdgcn_wave_barrier();
@@ -343,7 +392,7 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const
     }
 }
 
-template <typename TIN>
+template <typename TIN, bool F8>
 void launch_prepare_t(const arcq_prepare_args &a, const PrepWeights &w0, const PrepWeights &w1, hipStream_t stream)
 {
     const int G = static_cast<int>(a.K / 64), rows = static_cast<int>(a.rows);
@@ -374,9 +423,9 @@ void launch_prepare_t(const arcq_prepare_args &a, const PrepWeights &w0, const P
     if (grid == 0) return;
 #define ARCQ_LAUNCH_PREP(B, LNV)                                                                                              \
     do {                                                                                                                       \
-        hipLaunchKernelGGL((prepare_kernel<TIN, B, LNV>), dim3(grid), dim3(kPrepThreads), smem, stream,                        \
+        hipLaunchKernelGGL((prepare_kernel<TIN, B, LNV, F8>), dim3(grid), dim3(kPrepThreads), smem, stream,                    \
                            static_cast<const TIN *>(a.x), a.ln_weight, a.ln_bias, a.ln_eps, a.thresholds, a.codebook,          \
-                           static_cast<__half *>(a.x_hat), 1.0e-6f, rows, G, GC, R, chunks, tiles, w0, w1);                    \
+                           static_cast<char *>(a.x_hat), 1.0e-6f, rows, G, GC, R, chunks, tiles, w0, w1);                      \
     } while (0)
     if (a.bits == 4) { if (ln) ARCQ_LAUNCH_PREP(4, true); else ARCQ_LAUNCH_PREP(4, false); }
     else if (a.bits == 3) { if (ln) ARCQ_LAUNCH_PREP(3, true); else ARCQ_LAUNCH_PREP(3, false); }
@@ -405,10 +454,12 @@ ARCQ_API int arcq_prepare(const arcq_prepare_args *a, void *stream)
         if (!w.codebook || !w.center || !w.scale || !w.code_sum || !w.w_hat) return fail(ARCQ_ERR_NULL, "arcq_prepare: NULL weight tensor pointer");
         if (!aligned(w.w_hat, 16) || !aligned(w.packed, 16)) return fail(ARCQ_ERR_ALIGN, "arcq_prepare: w_hat and packed must be 16-byte aligned");
         const int G = static_cast<int>(w.K / 64);
-        // workgroups: waves of 32 columns x 4 groups, or threads of 8 weights
-        const unsigned items = w.row_major ? static_cast<unsigned>((w.N * G * 8 + 63) / 64) : static_cast<unsigned>(w.N / 32) * ((G + 3) / 4);
-        pw[i] = PrepWeights{w.packed, w.codebook, w.center, w.scale, w.code_sum, static_cast<__half *>(w.w_hat),
-                            static_cast<int>(w.N), G, w.row_major != 0, (items + kPrepWaves - 1) / kPrepWaves};
+        // workgroups: waves of 32 columns x 4 groups, or threads of a piece
+        if (a->fp8 && !(w.w_mult > 0.0f)) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_prepare: w_mult must be positive");
+        const int row_pieces = a->fp8 ? (G + 1) / 2 * 8 : G * 8;
+        const unsigned items = w.row_major ? static_cast<unsigned>((w.N * row_pieces + 63) / 64) : static_cast<unsigned>(w.N / 32) * ((G + 3) / 4);
+        pw[i] = PrepWeights{w.packed, w.codebook, w.center, w.scale, w.code_sum, w.w_hat, static_cast<int>(w.N), G, w.w_mult,
+                            w.row_major != 0, (items + kPrepWaves - 1) / kPrepWaves};
     }
     if (a->rows > 0) {
         if (a->K % 64 != 0 || a->K == 0) return fail(ARCQ_ERR_GROUP, "arcq_prepare: in_features must be a positive multiple of 64");
@@ -422,7 +473,14 @@ ARCQ_API int arcq_prepare(const arcq_prepare_args *a, void *stream)
             return fail(ARCQ_ERR_ALIGN, "arcq_prepare: x, x_hat, ln_weight and ln_bias must be 16-byte aligned");
     }
     if (a->rows == 0 && !pw[0].blocks && !pw[1].blocks) return ARCQ_OK;
-    if (a->x_dtype == ARCQ_F32) launch_prepare_t<float>(*a, pw[0], pw[1], static_cast<hipStream_t>(stream));
-    else launch_prepare_t<__half>(*a, pw[0], pw[1], static_cast<hipStream_t>(stream));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (a->fp8) {
+        if (a->x_dtype == ARCQ_F32) launch_prepare_t<float, true>(*a, pw[0], pw[1], st);
+        else launch_prepare_t<__half, true>(*a, pw[0], pw[1], st);
+    } else if (a->x_dtype == ARCQ_F32) {
+        launch_prepare_t<float, false>(*a, pw[0], pw[1], st);
+    } else {
+        launch_prepare_t<__half, false>(*a, pw[0], pw[1], st);
+    }
     return launch_status("arcq_prepare");
 }

@@ -54,6 +54,7 @@ PyObject *g_torch_module = nullptr;      // torch.nn.modules.module (the global 
 PyObject *g_layer_type = nullptr;        // ARCQPackedLinearOnTheFly
 PyObject *g_attention_type = nullptr, *g_mlp_type = nullptr;
 PyObject *g_gelu_type = nullptr, *g_layernorm_type = nullptr;
+PyObject *g_fp8_multiplier = nullptr;    // ops.fp8_weight_multiplier
 
 struct Failure {};      // a Python exception is set
 
@@ -271,7 +272,9 @@ bool can_quantize(PyObject *da, const Plan &a, PyObject *db, const Plan &b, int6
 struct Weights {                 // w_hat of one layer inside a scratch tensor
     void *ptr;
     bool row_major;
+    bool fp8 = false;            // FP8 operands: rows of Kp = K rounded up to 128 bytes
 };
+int64_t operand_row_bytes(int64_t K, bool fp8) { return fp8 ? (K + 127) / 128 * 128 : 2 * K; }
 // Fields of arcq_prepare_args for a layer's own tensors.
 void set_weights(arcq_prepare_weights &w, const Plan &p, const Weights &out)
 {
@@ -279,6 +282,7 @@ void set_weights(arcq_prepare_weights &w, const Plan &p, const Weights &out)
     w.codebook = static_cast<const float *>(p.p[W_CB]), w.center = static_cast<const float *>(p.p[W_CENTER]);
     w.scale = static_cast<const float *>(p.p[W_SCALE]), w.code_sum = static_cast<const float *>(p.p[W_SUM]);
     w.w_hat = out.ptr, w.N = p.N, w.K = p.K, w.row_major = out.row_major ? 1 : 0;
+    w.w_mult = static_cast<float>(p.fp8_mult);
 }
 void run_prepare(const Tensor &x, int64_t rows, const Plan &first, const LayerNormParams *ln, float ln_eps, void *x_hat, const Weights &w_first,
                  const Plan *second, const Weights *w_second, void *stream)
@@ -286,6 +290,7 @@ void run_prepare(const Tensor &x, int64_t rows, const Plan &first, const LayerNo
     arcq_prepare_args a = {};
     a.x_dtype = code_of(x);
     a.bits = static_cast<int32_t>(first.bits);
+    a.fp8 = w_first.fp8 ? 1 : 0;
     a.rows = rows, a.K = first.K;
     a.x = x.const_data_ptr();
     if (ln) a.ln_weight = fptr(ln->w.use), a.ln_bias = fptr(ln->b.use), a.ln_eps = ln_eps;
@@ -311,6 +316,7 @@ void run_product(const Plan &p, int64_t rows, const void *x_hat, const Weights &
         a.next_bits = static_cast<int32_t>(next->bits);
     }
     a.y = y;
+    a.fp8 = w.fp8 ? 1 : 0, a.w_mult = static_cast<float>(p.fp8_mult);
     check(arcq_linear_prepared(&a, stream));
 }
 bool can_prepare(const Plan &p, int64_t rows)
@@ -507,7 +513,7 @@ Tensor layernorm_op(PyObject *d, const Tensor &x, bool &ok)      // an nn.LayerN
 // ending with proj's stage 1 -> proj + skip -> [LayerNorm + stage 1, weights of fc1 and fc2] -> fc1 + GELU + fc2's stage 1
 // -> fc2 + skip.  All intermediate tensors come from the caching allocator, w_hat of two layers at a time included.
 std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t heads, bool own, Plan &pq, Plan &pp, Plan &pf1, Plan &pf2,
-                                     PyObject *n1, PyObject *n2, bool chain)
+                                     PyObject *n1, PyObject *n2, bool chain, bool fp8)
 {
     const int64_t b = x.size(0), n = x.size(1), C = x.size(2);
     if (!own || !chain || n > 256 || C != 64 * heads || C > 2048 || pf1.N % 64 != 0) return std::nullopt;
@@ -516,28 +522,47 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
     // Not where the one-launch layer kernels are at their best (one 64-row tile on most compute units, short rows): DeiT-S at
     // 12 608 rows 1 625 us a forward against 1 939, DeiT-B 3 969 against 4 373; at 9 456 rows 4 % either way, below and above
     // that range the seven launches win (6 304 rows: 1 353 -> 1 262 us; 25 216 rows: 3 341 -> 3 286).
-    if (rows > 9000 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) return std::nullopt;
+    if (!fp8 && rows > 9000 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) return std::nullopt;
     float e1, e2;
     LayerNormParams *l1 = layernorm_params(pq, n1, e1), *l2 = layernorm_params(pf1, n2, e2);
     if (!l1 || !l2) return std::nullopt;
     void *stream = stream_of(x);
-    auto layout = [&](const Plan &p) { return arcq_prepared_row_major(rows, p.N, p.K) != 0; };
-    const int64_t wq = pq.N * pq.K, wp = pp.N * pp.K, w1 = pf1.N * pf1.K, w2 = pf2.N * pf2.K;
-    Tensor w = empty({std::max(wq + wp, w1 + w2)}, at::kHalf, x.device());
+    auto layout = [&](const Plan &p) {
+        return (fp8 ? arcq_prepared_row_major_fp8(rows, p.N, p.K) : arcq_prepared_row_major(rows, p.N, p.K)) != 0;
+    };
+    auto weight_bytes = [&](const Plan &p) { return p.N * operand_row_bytes(p.K, fp8); };
+    const int64_t wq = weight_bytes(pq), wp = weight_bytes(pp), w1 = weight_bytes(pf1), w2 = weight_bytes(pf2);
+    Tensor w = empty({std::max(wq + wp, w1 + w2)}, at::kByte, x.device());
     char *wb = static_cast<char *>(w.mutable_data_ptr());
-    Tensor xh = empty({rows * C}, at::kHalf, x.device());
-    Tensor wide = empty({rows * std::max(pq.N, pf1.N)}, at::kHalf, x.device());       // qkv's output, then fc1's quantized output
+    Tensor xh = empty({rows * operand_row_bytes(C, fp8)}, at::kByte, x.device());
+    // qkv's output, then fc1's quantized output
+    Tensor wide = empty({rows * std::max(2 * pq.N, operand_row_bytes(pf2.K, fp8))}, at::kByte, x.device());
     Tensor x1 = empty(x.sizes(), at::kHalf, x.device()), y = empty(x.sizes(), at::kHalf, x.device());
-    const Weights hq{wb, layout(pq)}, hp{wb + wq * 2, layout(pp)}, h1{wb, layout(pf1)}, h2{wb + w1 * 2, layout(pf2)};
+    const Weights hq{wb, layout(pq), fp8}, hp{wb + wq, layout(pp), fp8}, h1{wb, layout(pf1), fp8}, h2{wb + w1, layout(pf2), fp8};
     run_prepare(x, rows, pq, l1, e1, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
     run_product(pq, rows, xh.const_data_ptr(), hq, nullptr, false, nullptr, wide.mutable_data_ptr(), ARCQ_F16, stream);
-    check(arcq_attention_quant_fwd(wide.const_data_ptr(), static_cast<const float *>(pp.p[A_THR]), static_cast<const float *>(pp.p[A_CB]),
-                                   static_cast<int>(pp.bits), xh.mutable_data_ptr(), b, n, heads, 64, 0.125f, stream));
+    check((fp8 ? arcq_attention_quant_fp8_fwd : arcq_attention_quant_fwd)(wide.const_data_ptr(), static_cast<const float *>(pp.p[A_THR]),
+        static_cast<const float *>(pp.p[A_CB]), static_cast<int>(pp.bits), xh.mutable_data_ptr(), b, n, heads, 64, 0.125f, stream));
     run_product(pp, rows, xh.const_data_ptr(), hp, &x, false, nullptr, x1.mutable_data_ptr(), ARCQ_F16, stream);
     run_prepare(x1, rows, pf1, l2, e2, xh.mutable_data_ptr(), h1, &pf2, &h2, stream);
     run_product(pf1, rows, xh.const_data_ptr(), h1, nullptr, true, &pf2, wide.mutable_data_ptr(), ARCQ_F16, stream);
     run_product(pf2, rows, wide.const_data_ptr(), h2, &x1, false, nullptr, y.mutable_data_ptr(), ARCQ_F16, stream);
     return y;
+}
+
+// The power of two inside a layer's FP8 weights (reads the metadata back to the host: once per layer and set of buffers).
+void find_fp8_multiplier(Plan &p)
+{
+    if (!std::isnan(p.fp8_mult)) return;
+    PyObject *args[4];
+    const int slots[4] = {W_CB, W_CENTER, W_SCALE, W_SUM};
+    for (int i = 0; i < 4; ++i) args[i] = THPVariable_Wrap(p.slot[slots[i]].use);
+    PyObject *r = PyObject_CallFunctionObjArgs(g_fp8_multiplier, args[0], args[1], args[2], args[3], nullptr);
+    for (PyObject *a : args) Py_DECREF(a);
+    if (!r) throw Failure{};
+    p.fp8_mult = PyFloat_AsDouble(r);
+    Py_DECREF(r);
+    if (PyErr_Occurred()) throw Failure{};
 }
 
 // One transformer block (vit.Block.forward), both of its forms; nullopt before anything has been launched where a module
@@ -570,14 +595,17 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
         return std::nullopt;
     const int64_t rows = x.size(0) * x.size(1);
     if (is_true(get(d, S.fuse_elementwise))) {
+        const bool fp8 = is_true(get(dq, S.fp8_operands));
         for (PyObject *l : {dq, dp, df1, df2})
-            if (is_true(get(l, S.fp8_operands)) || get(l, S.out_dtype) != reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf)))
+            if (is_true(get(l, S.fp8_operands)) != fp8 || get(l, S.out_dtype) != reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf)))
                 return std::nullopt;
         if (!f16(x) || c > (rows >= 512 ? 1024 : 1536) || c % 64 != 0 || pf2->K % 64 != 0) return std::nullopt;
         for (Plan *p : {pq, pp, pf1, pf2})
             if (p->gs != 64) return std::nullopt;
-        auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, is_true(get(d, S.chain_mlp)));
-        if (whole) return whole;
+        if (fp8)
+            for (Plan *p : {pq, pp, pf1, pf2}) find_fp8_multiplier(*p);
+        auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, is_true(get(d, S.chain_mlp)), fp8);
+        if (whole || fp8) return whole;
         Options o1;
         o1.layernorm = n1;
         auto t = layer_call(qkv, x, o1);
@@ -850,11 +878,12 @@ PyObject *py_patch_conv_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
     });
 }
 
-// register_types(layer, attention, mlp, gelu, layernorm, torch.nn.modules.module); None leaves an entry as it is
+// register_types(layer, attention, mlp, gelu, layernorm, torch.nn.modules.module, fp8_weight_multiplier); None leaves an entry as it is
 PyObject *py_register_types(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
-    PyObject **const to[6] = {&g_layer_type, &g_attention_type, &g_mlp_type, &g_gelu_type, &g_layernorm_type, &g_torch_module};
-    for (Py_ssize_t i = 0; i < n && i < 6; ++i) {
+    PyObject **const to[7] = {&g_layer_type, &g_attention_type, &g_mlp_type, &g_gelu_type, &g_layernorm_type, &g_torch_module,
+                              &g_fp8_multiplier};
+    for (Py_ssize_t i = 0; i < n && i < 7; ++i) {
         if (args[i] == Py_None) continue;
         Py_INCREF(args[i]);
         Py_XDECREF(*to[i]);

@@ -276,18 +276,22 @@ int arcq_act_quant_blocked_ln(const void *x, int x_dtype, const float *ln_weight
  * arcq_linear_prepared: y = x_hat * w_hat^T + bias on them, N a multiple of 32, with the options of arcq_linear_otf_ex
  * (next_*: y receives the consuming layer's x_hat, always in the block layout here).  Below 512 rows the products of
  * the groups g = w, w + 8, ... are summed apart for w = 0 .. 7 and added in that order, from 512 rows on k ascends:
- * the orders of the other entry points, i.e. the same bits as theirs. */
+ * the orders of the other entry points, i.e. the same bits as theirs.
+ * fp8 != 0 (opt-in, see arcq_act_quant_fp8): rows of both operands are padded with zeros to Kp = K rounded up to 128
+ * values; x_hat is [rows/32][Kp/16][32 rows][16 values] bytes, w_hat [N/32][Kp/16][32 columns][16 values] or [N][Kp]
+ * (any M), and next_* makes the consumer's operand of that kind. */
 typedef struct arcq_prepare_weights {
     const uint8_t *packed;                                   /* 16-byte aligned */
     const float *codebook, *center, *scale, *code_sum;
     void *w_hat;
     int64_t N, K;
-    int32_t row_major, reserved;                             /* row_major != 0: w_hat as [N][K] instead of column blocks */
+    int32_t row_major;                                       /* != 0: w_hat as [N][K] instead of column blocks */
+    float w_mult;                                            /* fp8: as arcq_weight_dequant_fp8 */
 } arcq_prepare_weights;
 typedef struct arcq_prepare_args {
     int32_t x_dtype, bits;
     float ln_eps;
-    int32_t reserved;
+    int32_t fp8;                                             /* != 0: x_hat and w_hat as FP8 operands (see below) */
     int64_t rows, K;
     const void *x;
     const float *ln_weight, *ln_bias;                        /* NULL: no LayerNorm; 16-byte aligned */
@@ -304,11 +308,14 @@ typedef struct arcq_linear_prepared_args {
     const void *residual;                                    /* [M,N] of y's type, or NULL */
     const float *next_thresholds, *next_codebook;
     void *y;
+    int32_t fp8;                                             /* != 0: the operands (and the quantized output) are FP8 */
+    float w_mult;                                            /* fp8: the factor inside w_hat */
 } arcq_linear_prepared_args;
 int arcq_linear_prepared(const arcq_linear_prepared_args *args, void *stream);
 /* Layout of w_hat that arcq_linear_prepared runs fastest on for these sizes: 0 = column blocks (any M), 1 = row-major
  * (M >= 512: the weight-stationary kernels, which want many row blocks). */
 int arcq_prepared_row_major(int64_t M, int64_t N, int64_t K);
+int arcq_prepared_row_major_fp8(int64_t M, int64_t N, int64_t K);       /* the same for FP8 operands */
 
 /* arcq_linear_otf_ws for callers that cannot allocate device memory or lend workspaces (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The two
@@ -381,6 +388,9 @@ int arcq_attention_fwd(const void *qkv, void *out, int64_t B, int64_t n, int64_t
  * block layout, the bits of arcq_act_quant_blocked on arcq_attention_fwd's output; thresholds / codebook are the proj layer's. */
 int arcq_attention_quant_fwd(const void *qkv, const float *thresholds, const float *codebook, int bits, void *x_hat,
                              int64_t B, int64_t n, int64_t H, int64_t head_dim, float scale, void *stream);
+/* The same with that operand as FP8 (arcq_prepare, fp8). */
+int arcq_attention_quant_fp8_fwd(const void *qkv, const float *thresholds, const float *codebook, int bits, void *x8,
+                                 int64_t B, int64_t n, int64_t H, int64_t head_dim, float scale, void *stream);
 
 /* ---- stage 1 of a quantized patch-embedding convolution ---------------------
  * QuantConv2dPCARCQ (FQ/quant_backends.py:329-384; the activation quantizer groups min(64, in_channels) = 3 channels
