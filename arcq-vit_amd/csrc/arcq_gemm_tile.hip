@@ -254,11 +254,11 @@ void launch_tile(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 }
 
 // ---- fewer than 512 rows ------------------------------------------------------------------------------------------
-template <typename TOUT, int RB, int CB, int NQ, bool F8>
+template <typename TOUT, int RB, int CB, int NQ>
 __global__ void __launch_bounds__(512)
 gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char *__restrict__ wb, const float *__restrict__ bias,
                        TOUT *__restrict__ y, int M, int N, int G, const TOUT *__restrict__ residual, int gelu,
-                       const float *__restrict__ nx_thr, const float *__restrict__ nx_cb, float inv)
+                       const float *__restrict__ nx_thr, const float *__restrict__ nx_cb)
 {
     constexpr int NW = 8;
     constexpr int RT = 32 * RB, CT = 32 * CB;
@@ -275,23 +275,21 @@ gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char
         const int blk = min(m0 / 32 + i, row_blocks - 1);
         const int r = min(32, M - blk * 32);
         a_step[i] = r * 16;
-        a_src[i] = reinterpret_cast<const char *>(xb) + static_cast<int64_t>(blk) * G * kGroupBytes + lh * (F8 ? 2 : 4) * a_step[i] +
-                   min(lr, r - 1) * 16;
+        a_src[i] = reinterpret_cast<const char *>(xb) + static_cast<int64_t>(blk) * G * kGroupBytes + lh * 4 * a_step[i] + min(lr, r - 1) * 16;
     }
 #pragma unroll
     for (int j = 0; j < CB; ++j) {
         const int blk = min(n0 / 32 + j, col_blocks - 1);
-        b_src[j] = reinterpret_cast<const char *>(wb) + static_cast<int64_t>(blk) * G * kGroupBytes + lh * (F8 ? 1024 : 2048) + lr * 16;
+        b_src[j] = reinterpret_cast<const char *>(wb) + static_cast<int64_t>(blk) * G * kGroupBytes + lh * 2048 + lr * 16;
     }
     struct Ops { u32x4_t a[RB][4], b[CB][4]; };
     auto fetch = [&](int g, Ops &o) __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
-            const int p = F8 ? (kk >> 1) * 4 + (kk & 1) : kk;        // FP8: two pieces per k-step of 64
 #pragma unroll
-            for (int i = 0; i < RB; ++i) o.a[i][kk] = *reinterpret_cast<const u32x4_t *>(a_src[i] + (g * 8 + p) * a_step[i]);
+            for (int i = 0; i < RB; ++i) o.a[i][kk] = *reinterpret_cast<const u32x4_t *>(a_src[i] + (g * 8 + kk) * a_step[i]);
 #pragma unroll
-            for (int j = 0; j < CB; ++j) o.b[j][kk] = *reinterpret_cast<const u32x4_t *>(b_src[j] + g * kGroupBytes + p * 512);
+            for (int j = 0; j < CB; ++j) o.b[j][kk] = *reinterpret_cast<const u32x4_t *>(b_src[j] + g * kGroupBytes + kk * 512);
         }
     };
     Ops o0, o1;
@@ -309,17 +307,6 @@ gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
     auto compute = [&](const Ops &o) __attribute__((always_inline)) {
-        if constexpr (F8) {
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-#pragma unroll
-                for (int i = 0; i < RB; ++i)
-#pragma unroll
-                    for (int j = 0; j < CB; ++j) {
-                        const u32x4_t w2[2] = {o.b[j][2 * s], o.b[j][2 * s + 1]}, x2[2] = {o.a[i][2 * s], o.a[i][2 * s + 1]};
-                        acc[i][j] = mfma_fp8(w2, x2, acc[i][j]);
-                    }
-        } else
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
             half8_t af[RB], bf[CB];
@@ -390,7 +377,7 @@ gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char
     }
     TOUT out[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) out[e] = from_float<TOUT>((F8 ? sum[e] * inv : sum[e]) + bv[e]);
+    for (int e = 0; e < E; ++e) out[e] = from_float<TOUT>(sum[e] + bv[e]);
     if constexpr (NQ != 0) {
         // The rounded (GELU'd) outputs as an fp16 tile over the partial sums of wave 0 .. (everyone has read them), then
         // stage 1 of the consumer on its 32-row chunks of 64 columns.
@@ -406,7 +393,7 @@ gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char
         if (wave < RB) {
             const int blk = m0 / 32 + wave;
             if (blk < row_blocks && n0 < N)
-                next_quant_block<NQ, F8>(nq_lds, NW, smem + wave * 32 * kStageRow, kStageRow, lane, false, 1.0e-6f, y, blk, M, N, n0);
+                next_quant_block<NQ, false>(nq_lds, NW, smem + wave * 32 * kStageRow, kStageRow, lane, false, 1.0e-6f, y, blk, M, N, n0);
         }
     } else if (live) {
         if (residual || gelu) {
@@ -418,30 +405,30 @@ gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char
     }
 }
 
-template <typename TOUT, int RB, int CB, int NQ, bool F8>
+template <typename TOUT, int RB, int CB, int NQ>
 void launch_split(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 {
     constexpr int kSmem = 8 * 32 * RB * (32 * CB * 4 + 16) + (NQ ? next_quant_lds_bytes(NQ) : 0);
-    allow_dynamic_lds<gemm_tile_split_kernel<TOUT, RB, CB, NQ, F8>>(kSmem);
+    allow_dynamic_lds<gemm_tile_split_kernel<TOUT, RB, CB, NQ>>(kSmem);
     const dim3 grid((g.N + 32 * CB - 1) / (32 * CB), (g.M + 32 * RB - 1) / (32 * RB));
-    hipLaunchKernelGGL((gemm_tile_split_kernel<TOUT, RB, CB, NQ, F8>), grid, dim3(512), kSmem, stream,
+    hipLaunchKernelGGL((gemm_tile_split_kernel<TOUT, RB, CB, NQ>), grid, dim3(512), kSmem, stream,
                        static_cast<const unsigned char *>(g.x_hat), static_cast<const unsigned char *>(w_hat), g.bias,
-                       static_cast<TOUT *>(g.y), g.M, g.N, operand_units(g.K, F8), static_cast<const TOUT *>(g.residual), g.gelu ? 1 : 0,
-                       g.next_thr, g.next_cb, g.fp8_inv);
+                       static_cast<TOUT *>(g.y), g.M, g.N, g.K / 64, static_cast<const TOUT *>(g.residual), g.gelu ? 1 : 0, g.next_thr,
+                       g.next_cb);
 }
 
 template <typename TOUT, int NQ, bool F8>
 void pick(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 {
     const int cus = device_cus();
-    if (g.M < 512) {
+    if (!F8 && g.M < 512) {      // (FP8: one order of k at every M, the order of the other FP8 kernel)
         const int64_t t11 = static_cast<int64_t>((g.M + 31) / 32) * (g.N / 32);
         const int64_t t12 = static_cast<int64_t>((g.M + 31) / 32) * ((g.N + 63) / 64);
         if constexpr (NQ == 0) {
-            if (t11 <= 2 * cus) return launch_split<TOUT, 1, 1, 0, F8>(g, w_hat, stream);
+            if (t11 <= 2 * cus) return launch_split<TOUT, 1, 1, 0>(g, w_hat, stream);
         }
-        if (t12 <= 2 * cus) return launch_split<TOUT, 1, 2, NQ, F8>(g, w_hat, stream);
-        return launch_split<TOUT, 2, 2, NQ, F8>(g, w_hat, stream);
+        if (t12 <= 2 * cus) return launch_split<TOUT, 1, 2, NQ>(g, w_hat, stream);
+        return launch_split<TOUT, 2, 2, NQ>(g, w_hat, stream);
     }
     // 64 x 64 tiles (two workgroups on a CU) while they fit the chip at once, 128 x 128 beyond: measured crossovers between
     // 480 and 600 tiles at K = 384, 768 and 1 024 (384 -> 1 536 at 1 576 rows, 600 tiles: 7.9 against 6.9 us; 1 024 -> 3 072 at

@@ -181,6 +181,7 @@ __device__ __forceinline__ void prep_weights_rows(const PrepWeights &w, unsigned
     store_writethrough16(static_cast<char *>(w.out) + static_cast<int64_t>(idx) * 16, o[0], o[1], o[2], o[3]);
 }
 
+// F8 (LN = false only): FP8 operands.
 // LN = true: LayerNorm over the rows first; GC = all G groups of a row (2 GC lanes per row).
 // LN = false: a wave takes R rows x GC groups; consecutive waves take consecutive group chunks.
 // rows_per_wave = R; chunks = group chunks per row (1 with a LayerNorm).
@@ -352,12 +353,12 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const
             }
             __syncthreads();
             const int r0 = t * RW;
-            const int live = GC * kPieces * RW, pieces = row_groups * kPieces * RW;
+            const int pieces = GC * kPieces * RW;
             for (int p = tid; p < pieces; p += kPrepThreads) {
                 const int k = p / RW, r = p - k * RW;
                 const int rr = r0 + r;
                 if (rr < rows) {
-                    const uint4 v = !F8 || p < live ? *reinterpret_cast<const uint4 *>(tile + p * 16) : make_uint4(0, 0, 0, 0);
+                    const uint4 v = *reinterpret_cast<const uint4 *>(tile + p * 16);
                     const int blk = rr >> 5, nrows = min(32, rows - blk * 32);
                     store_writethrough16(x_hat + static_cast<int64_t>(blk) * 32 * row_bytes + (k * nrows + (rr & 31)) * 16, v.x, v.y, v.z, v.w);
                 }
@@ -427,9 +428,17 @@ void launch_prepare_t(const arcq_prepare_args &a, const PrepWeights &w0, const P
                            static_cast<const TIN *>(a.x), a.ln_weight, a.ln_bias, a.ln_eps, a.thresholds, a.codebook,          \
                            static_cast<char *>(a.x_hat), 1.0e-6f, rows, G, GC, R, chunks, tiles, w0, w1);                      \
     } while (0)
-    if (a.bits == 4) { if (ln) ARCQ_LAUNCH_PREP(4, true); else ARCQ_LAUNCH_PREP(4, false); }
-    else if (a.bits == 3) { if (ln) ARCQ_LAUNCH_PREP(3, true); else ARCQ_LAUNCH_PREP(3, false); }
-    else { if (ln) ARCQ_LAUNCH_PREP(2, true); else ARCQ_LAUNCH_PREP(2, false); }
+    if constexpr (!F8) {
+        if (ln) {
+            if (a.bits == 4) ARCQ_LAUNCH_PREP(4, true);
+            else if (a.bits == 3) ARCQ_LAUNCH_PREP(3, true);
+            else ARCQ_LAUNCH_PREP(2, true);
+            return;
+        }
+    }
+    if (a.bits == 4) ARCQ_LAUNCH_PREP(4, false);
+    else if (a.bits == 3) ARCQ_LAUNCH_PREP(3, false);
+    else ARCQ_LAUNCH_PREP(2, false);
 #undef ARCQ_LAUNCH_PREP
 }
 
@@ -467,8 +476,8 @@ ARCQ_API int arcq_prepare(const arcq_prepare_args *a, void *stream)
         if (!a->x || !a->thresholds || !a->codebook || !a->x_hat) return fail(ARCQ_ERR_NULL, "arcq_prepare: NULL tensor pointer");
         if (a->x == a->x_hat) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_prepare: x_hat must not alias x");
         if (a->rows >= (int64_t(1) << 26) || a->rows * a->K >= (int64_t(1) << 31)) return fail(ARCQ_ERR_SHAPE, "arcq_prepare: tensor too large");
-        if (a->ln_weight && (!a->ln_bias || a->K > 2048))
-            return fail(ARCQ_ERR_UNSUPPORTED, "arcq_prepare: the LayerNorm needs weight and bias and in_features <= 2048");
+        if (a->ln_weight && (!a->ln_bias || a->K > 2048 || a->fp8))
+            return fail(ARCQ_ERR_UNSUPPORTED, "arcq_prepare: the LayerNorm needs weight and bias, in_features <= 2048 and fp16 operands");
         if (!aligned(a->x, 16) || !aligned(a->x_hat, 16) || !aligned(a->ln_weight, 16) || !aligned(a->ln_bias, 16))
             return fail(ARCQ_ERR_ALIGN, "arcq_prepare: x, x_hat, ln_weight and ln_bias must be 16-byte aligned");
     }

@@ -296,7 +296,7 @@ void run_prepare(const Tensor &x, int64_t rows, const Plan &first, const LayerNo
     if (ln) a.ln_weight = fptr(ln->w.use), a.ln_bias = fptr(ln->b.use), a.ln_eps = ln_eps;
     a.thresholds = static_cast<const float *>(first.p[A_THR]), a.codebook = static_cast<const float *>(first.p[A_CB]);
     a.x_hat = x_hat;
-    set_weights(a.weights[0], first, w_first);
+    if (w_first.ptr) set_weights(a.weights[0], first, w_first);
     if (second) set_weights(a.weights[1], *second, *w_second);
     check(arcq_prepare(&a, stream));
 }
@@ -509,23 +509,38 @@ Tensor layernorm_op(PyObject *d, const Tensor &x, bool &ok)      // an nn.LayerN
                           PyFloat_AS_DOUBLE(e));
 }
 
-// The fused block on prepared operands, seven launches: [LayerNorm + stage 1, weights of qkv and proj] -> qkv -> attention
-// ending with proj's stage 1 -> proj + skip -> [LayerNorm + stage 1, weights of fc1 and fc2] -> fc1 + GELU + fc2's stage 1
-// -> fc2 + skip.  All intermediate tensors come from the caching allocator, w_hat of two layers at a time included.
+// A block on prepared operands: [LayerNorm + stage 1, weights of qkv and proj] -> qkv -> attention ending with proj's stage 1
+// -> proj + skip -> [LayerNorm + stage 1, weights of fc1 and fc2] -> fc1 + GELU + fc2's stage 1 -> fc2 + skip: seven launches.
+// All intermediate tensors come from the caching allocator, w_hat of two layers at a time included.
+//   fused == false: the LayerNorms are torch's (own launches); everything else that is folded into the products (skips, GELU,
+//                   fc2's stage 1) gives the bits of the separate kernels anyway
+//   fp8:            FP8 operands.  LayerNorms as torch runs them: that is what the layers do one by one, and a network of
+//                   quantizers does not forgive another order of summation (one changed bit is 10 % of the logits 12 blocks on)
+//   attention that the library's kernel does not run (or is not to): torch's, then stage 1 of proj as a launch of its own
 std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t heads, bool own, Plan &pq, Plan &pp, Plan &pf1, Plan &pf2,
-                                     PyObject *n1, PyObject *n2, bool chain, bool fp8)
+                                     PyObject *n1, PyObject *n2, bool fused, bool fp8)
 {
     const int64_t b = x.size(0), n = x.size(1), C = x.size(2);
-    if (!own || !chain || n > 256 || C != 64 * heads || C > 2048 || pf1.N % 64 != 0) return std::nullopt;
+    const bool fuse_ln = fused && !fp8;
+    const bool own_attention = own && n <= 256 && C == 64 * heads;
+    if ((fuse_ln && C > 2048) || pf1.N % 64 != 0) return std::nullopt;
     for (const Plan *p : {&pq, &pp, &pf1, &pf2})
         if (!can_prepare(*p, rows) || p->bits != pq.bits) return std::nullopt;
     // Not where the one-launch layer kernels are at their best (one 64-row tile on most compute units, short rows): DeiT-S at
     // 12 608 rows 1 625 us a forward against 1 939, DeiT-B 3 969 against 4 373; at 9 456 rows 4 % either way, below and above
     // that range the seven launches win (6 304 rows: 1 353 -> 1 262 us; 25 216 rows: 3 341 -> 3 286).
-    if (!fp8 && rows > 9000 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) return std::nullopt;
-    float e1, e2;
-    LayerNormParams *l1 = layernorm_params(pq, n1, e1), *l2 = layernorm_params(pf1, n2, e2);
-    if (!l1 || !l2) return std::nullopt;
+    if (fuse_ln && rows > 9000 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) return std::nullopt;
+    float e1 = 0, e2 = 0;
+    LayerNormParams *l1 = nullptr, *l2 = nullptr;
+    Tensor t = x;
+    if (fuse_ln) {
+        l1 = layernorm_params(pq, n1, e1), l2 = layernorm_params(pf1, n2, e2);
+        if (!l1 || !l2) return std::nullopt;
+    } else {
+        bool ok = true;
+        t = layernorm_op(dict_of(n1), x, ok);
+        if (!ok) return std::nullopt;
+    }
     void *stream = stream_of(x);
     auto layout = [&](const Plan &p) {
         return (fp8 ? arcq_prepared_row_major_fp8(rows, p.N, p.K) : arcq_prepared_row_major(rows, p.N, p.K)) != 0;
@@ -535,16 +550,24 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
     Tensor w = empty({std::max(wq + wp, w1 + w2)}, at::kByte, x.device());
     char *wb = static_cast<char *>(w.mutable_data_ptr());
     Tensor xh = empty({rows * operand_row_bytes(C, fp8)}, at::kByte, x.device());
-    // qkv's output, then fc1's quantized output
-    Tensor wide = empty({rows * std::max(2 * pq.N, operand_row_bytes(pf2.K, fp8))}, at::kByte, x.device());
+    Tensor wide = empty({rows * operand_row_bytes(pf2.K, fp8)}, at::kByte, x.device());       // fc1's quantized output
+    Tensor qkv = empty({b, n, pq.N}, at::kHalf, x.device());
     Tensor x1 = empty(x.sizes(), at::kHalf, x.device()), y = empty(x.sizes(), at::kHalf, x.device());
     const Weights hq{wb, layout(pq), fp8}, hp{wb + wq, layout(pp), fp8}, h1{wb, layout(pf1), fp8}, h2{wb + w1, layout(pf2), fp8};
-    run_prepare(x, rows, pq, l1, e1, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
-    run_product(pq, rows, xh.const_data_ptr(), hq, nullptr, false, nullptr, wide.mutable_data_ptr(), ARCQ_F16, stream);
-    check((fp8 ? arcq_attention_quant_fp8_fwd : arcq_attention_quant_fwd)(wide.const_data_ptr(), static_cast<const float *>(pp.p[A_THR]),
-        static_cast<const float *>(pp.p[A_CB]), static_cast<int>(pp.bits), xh.mutable_data_ptr(), b, n, heads, 64, 0.125f, stream));
+    run_prepare(t, rows, pq, l1, e1, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
+    run_product(pq, rows, xh.const_data_ptr(), hq, nullptr, false, nullptr, qkv.mutable_data_ptr(), ARCQ_F16, stream);
+    if (own_attention) {
+        check((fp8 ? arcq_attention_quant_fp8_fwd : arcq_attention_quant_fwd)(qkv.const_data_ptr(), static_cast<const float *>(pp.p[A_THR]),
+            static_cast<const float *>(pp.p[A_CB]), static_cast<int>(pp.bits), xh.mutable_data_ptr(), b, n, heads, 64, 0.125f, stream));
+    } else {
+        const Tensor a = mix(qkv, heads, false).contiguous();
+        run_prepare(a, rows, pp, nullptr, 0, xh.mutable_data_ptr(), Weights{nullptr, false, fp8}, nullptr, nullptr, stream);
+    }
     run_product(pp, rows, xh.const_data_ptr(), hp, &x, false, nullptr, x1.mutable_data_ptr(), ARCQ_F16, stream);
-    run_prepare(x1, rows, pf1, l2, e2, xh.mutable_data_ptr(), h1, &pf2, &h2, stream);
+    bool ok = true;
+    t = fuse_ln ? x1 : layernorm_op(dict_of(n2), x1, ok);
+    if (!ok) return std::nullopt;
+    run_prepare(t, rows, pf1, l2, e2, xh.mutable_data_ptr(), h1, &pf2, &h2, stream);
     run_product(pf1, rows, xh.const_data_ptr(), h1, nullptr, true, &pf2, wide.mutable_data_ptr(), ARCQ_F16, stream);
     run_product(pf2, rows, wide.const_data_ptr(), h2, &x1, false, nullptr, y.mutable_data_ptr(), ARCQ_F16, stream);
     return y;
@@ -604,8 +627,12 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
             if (p->gs != 64) return std::nullopt;
         if (fp8)
             for (Plan *p : {pq, pp, pf1, pf2}) find_fp8_multiplier(*p);
-        auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, is_true(get(d, S.chain_mlp)), fp8);
-        if (whole || fp8) return whole;
+        const bool chain = is_true(get(d, S.chain_mlp));
+        if (chain && (fp8 || (own && x.size(1) <= 256 && c == 64 * heads))) {
+            auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, true, fp8);
+            if (whole) return whole;
+        }
+        if (fp8) return std::nullopt;
         Options o1;
         o1.layernorm = n1;
         auto t = layer_call(qkv, x, o1);
@@ -630,6 +657,13 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
     }
     for (PyObject *dd : {ad, md, d1, d2, dict_of(act)})
         if (!no_hooks(dd)) return std::nullopt;
+    bool plain = f16(x) && c % 64 == 0 && pf2->K % 64 == 0;
+    for (PyObject *l : {dq, dp, df1, df2})
+        plain = plain && !is_true(get(l, S.fp8_operands)) && get(l, S.out_dtype) == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf));
+    if (plain) {
+        auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, false, false);
+        if (whole) return whole;
+    }
     bool ok = true;
     Tensor t = layernorm_op(d1, x, ok);
     if (!ok) return std::nullopt;

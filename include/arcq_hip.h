@@ -279,7 +279,7 @@ int arcq_act_quant_blocked_ln(const void *x, int x_dtype, const float *ln_weight
  * the orders of the other entry points, i.e. the same bits as theirs.
  * fp8 != 0 (opt-in, see arcq_act_quant_fp8): rows of both operands are padded with zeros to Kp = K rounded up to 128
  * values; x_hat is [rows/32][Kp/16][32 rows][16 values] bytes, w_hat [N/32][Kp/16][32 columns][16 values] or [N][Kp]
- * (any M), and next_* makes the consumer's operand of that kind. */
+ * (any M), and next_* makes the consumer's operand of that kind.  No LayerNorm then, and k ascends at every M. */
 typedef struct arcq_prepare_weights {
     const uint8_t *packed;                                   /* 16-byte aligned */
     const float *codebook, *center, *scale, *code_sum;
