@@ -358,157 +358,15 @@ act_quant_small_kernel(const TIN *__restrict__ x, const float *__restrict__ thr,
     }
 }
 
-// Block-layout stage 1 with two lanes per group.  A wave tile is 32 rows x ONE group; lane l owns row l / 2 and the
-// half l % 2 of the group (arcq_act_quant_core.h: two-phase serial sums, same bits as one lane per group).  Halving
-// the tile doubles the number of work items, which is what the K = 384 layers of DeiT-S need: 1 182 whole tiles on
-// 1 024 SIMDs leave 158 SIMDs with two tiles (2 x 1 470 instructions), 2 364 half tiles at most three (3 x 740).
-// Data moves through a wave-private LDS tile (rows of the tile = rows of the tensor, odd dword pitch): coalesced
-// 16-byte loads in, every piece column out as one 512-byte run of the block layout.
-template <typename TIN, int BITS, bool BUILDER>
-__global__ void __launch_bounds__(64 * (kWaves + (BUILDER ? 1 : 0)))
-act_quant_blocked2_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const float *__restrict__ cb,
-                          __half *__restrict__ x_hat, float eps, int groups_per_row, int64_t rows, WeightJob wj)
-{
-    constexpr int L = 1 << BITS;
-    constexpr int kInPitch = Tile<TIN>::stride, kOutPitch = Tile<__half>::stride;     // dwords per tile row
-    constexpr int kPieces = 64 / Tile<TIN>::vec;           // 16-byte pieces per row of the tile (8 fp16 / 16 fp32)
-    constexpr int kRowsPerInstr = 64 / kPieces;            // 8 / 4
-    constexpr int kIters = 32 / kRowsPerInstr;             // 4 / 8
-    __shared__ uint32_t tiles[kWaves][32 * kInPitch];
-    __shared__ float lut[L * 64];
-    __shared__ Bucket table[kMaxBuckets + 1];
-    __shared__ int slow_slots[kWaves];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    if (blockIdx.x < wj.blocks) {          // workgroup-uniform: this workgroup rebuilds weights and is done
-        if (!BUILDER || wave < kWaves)     // (256 threads per weight block; the fifth wave has nothing to do, and the
-            weight_dequant8_block<__half, BITS, 64 * kWaves>(blockIdx.x, lut, wj.packed, wj.cb, wj.center, wj.scale,
-                                                             wj.code_sum, wj.out, wj.N, wj.K, 64);
-        else                               //  routine's barrier is counted per workgroup: it joins it)
-            __syncthreads();
-        return;
-    }
-    // BUILDER: the workgroup has a fifth wave that owns no tile; it builds the lookup tables while the four tile waves
-    // load their first tile and take its statistics, meets them at the one barrier of the kernel, and is done.  That
-    // takes the table construction (a third of a half tile's instruction chain) off every tile wave's path.  Without
-    // it the four tile waves build the tables together between the two halves of their first tile.
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(thr, cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
-    if (BUILDER && wave == kWaves) {
-        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, lane, 64);
-        __syncthreads();
-        return;
-    }
-    const int64_t wg = blockIdx.x - wj.blocks;
-    const int64_t act_blocks = gridDim.x - wj.blocks;
-    const int64_t ntiles = ((rows + 31) / 32) * groups_per_row;
-    const int64_t row_elems = static_cast<int64_t>(groups_per_row) * 64;
-    uint32_t *tile = tiles[wave];
-
-    uint4 raw[kIters];
-    auto fetch = [&](int64_t t) {          // tile t = (row block t / G, group t % G); zero-fills past the end
-        const int64_t rb = t / groups_per_row;
-        const int g = static_cast<int>(t - rb * groups_per_row);
-        const int64_t r0 = rb * 32 + lane / kPieces;
-        const TIN *p = x + r0 * row_elems + g * 64 + (lane % kPieces) * Tile<TIN>::vec;
-#pragma unroll
-        for (int i = 0; i < kIters; ++i)         // rows past the tensor's end (a ragged last block) read as zeros
-            raw[i] = (t < ntiles && r0 + i * kRowsPerInstr < rows) ? *reinterpret_cast<const uint4 *>(p + i * kRowsPerInstr * row_elems)
-                                                                   : make_uint4(0, 0, 0, 0);
-    };
-    fetch(wg * kWaves + wave);
-    bool table_ok = false, tables_built = false;
-    const int row = lane >> 1, half = lane & 1;
-    if constexpr (!BUILDER) {
-        // Without a builder wave the four tile waves build the tables first, while their first tile is on its way:
-        // nothing else is live in registers yet (building them between the halves of the first tile, with the tile's
-        // 32 values held, took 169 VGPRs: two waves per SIMD instead of three).
-        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, 64 * kWaves);
-        __syncthreads();
-        table_ok = true;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
-        tables_built = true;
-    }
-
-    for (int64_t tile0 = wg * kWaves; tile0 < ntiles; tile0 += act_blocks * kWaves) {
-        const int64_t t = tile0 + wave;
-        {
-            uint32_t *dst = tile + (lane / kPieces) * kInPitch + (lane % kPieces) * 4;
-#pragma unroll
-            for (int i = 0; i < kIters; ++i) {
-                uint32_t *d = dst + i * kRowsPerInstr * kInPitch;
-                d[0] = raw[i].x; d[1] = raw[i].y; d[2] = raw[i].z; d[3] = raw[i].w;
-            }
-        }
-        __builtin_amdgcn_wave_barrier();      // the tile is private to the wave and LDS operations execute in order
-        float xv[32];
-        {
-            const uint32_t *src = tile + row * kInPitch + half * (32 * static_cast<int>(sizeof(TIN)) / 4);
-            if constexpr (sizeof(TIN) == 4) {
-#pragma unroll
-                for (int j = 0; j < 32; ++j) xv[j] = __uint_as_float(src[j]);
-            } else {
-#pragma unroll
-                for (int p = 0; p < 16; ++p) {
-                    const uint32_t w = src[p];
-                    xv[2 * p] = __half2float(__ushort_as_half(static_cast<unsigned short>(w & 0xffffu)));
-                    xv[2 * p + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(w >> 16)));
-                }
-            }
-        }
-        fetch(t + act_blocks * kWaves);       // the wave's next tile (nothing past the end) loads under this one's arithmetic
-        float mu, var, s, sum_codes;
-        group_stats32x2(xv, eps, mu, var, s);
-        if (BUILDER && !tables_built) {       // once per workgroup: the builder wave's tables are ready
-            __syncthreads();
-            table_ok = (slow_slots[0] == 0);
-            tables_built = true;
-        }
-        group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
-        const float code_mean = sum_codes * 0.015625f;
-        {
-            // Every lane has read its inputs (program order within the wave), so rows may be rewritten, with the
-            // output pitch.
-            uint32_t *dst = tile + row * kOutPitch + half * 16;
-#pragma unroll
-            for (int p = 0; p < 16; ++p) {
-                const __half2 h = __floats2half2_rn(fma_f32(s, xv[2 * p] - code_mean, mu), fma_f32(s, xv[2 * p + 1] - code_mean, mu));
-                dst[p] = *reinterpret_cast<const uint32_t *>(&h);
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (t < ntiles) {
-            const int64_t rb = t / groups_per_row;
-            const int g = static_cast<int>(t - rb * groups_per_row);
-            const int r = lane & 31;
-            const int nrows = static_cast<int>(rows - rb * 32 < 32 ? rows - rb * 32 : 32);     // < 32 in a ragged last block,
-            __half *base = x_hat + rb * (row_elems * 32) + (static_cast<int64_t>(g) * 8 * nrows + r) * 8;   // stored compactly
-            if (r < nrows) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {  // instruction j: piece columns 2j and 2j + 1, nrows x 16 bytes each
-                    const int kp = j * 2 + (lane >> 5);
-                    const uint32_t *src = tile + r * kOutPitch + kp * 4;
-                    store_writethrough16(base + kp * (nrows * 8), src[0], src[1], src[2], src[3]);
-                }
-            }
-        }
-        __builtin_amdgcn_wave_barrier();      // the tile is refilled in the next iteration
-    }
-}
-
 // LayerNorm fused in front of the block-layout stage 1.  A workgroup owns one 32-row block and all G = K / 64 groups of
-// it, one wave per group (wave tile = 32 rows x one group, two lanes per group, as act_quant_blocked2_kernel), so the
+// it, one wave per group (wave tile = 32 rows x one group, two lanes per group, as prepare_kernel), so the
 // row statistics LayerNorm needs are a sum over the workgroup: every lane folds its 32 values serially, the 2 G
 // partial sums of a row meet in LDS and every lane of the row adds them up in the same fixed order.
 //   mean = (sum of the partial sums, group by group, lower half first) / K
 //   var  = (the same sum over (x - mean)^2) / K
 //   y    = ((x - mean) * (1 / sqrt(var + ln_eps))) * gamma + beta        three roundings, no fma
 // y is rounded to the input's type (what a stand-alone LayerNorm kernel would have stored) and then quantized and
-// reconstructed exactly as act_quant_blocked2_kernel does.  MAXW = most waves (groups) per workgroup.
+// reconstructed exactly as prepare_kernel does.  MAXW = most waves (groups) per workgroup.
 template <typename TIN, int BITS, int MAXW>
 __global__ void __launch_bounds__(64 * MAXW)
 act_quant_rows_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta,
@@ -766,92 +624,9 @@ static int launch(const void *x, const float *thr, const float *cb, uint8_t *pac
     return launch_status("arcq_act_quant");
 }
 
-template <typename TIN>
-static int launch_blocked(const void *x, const float *thr, const float *cb, void *x_hat, int64_t rows, int64_t cols,
-                          int bits, float eps, hipStream_t stream, const WeightJob &wj)
-{
-    const int groups_per_row = static_cast<int>(cols / 64);
-    const int64_t ntiles = ((rows + 31) / 32) * groups_per_row;
-    const int64_t want = (ntiles + kWaves - 1) / kWaves;
-    // Up to 2 048 tiles (512 workgroups, two per CU) the launch is latency-bound: every wave takes one tile and a fifth
-    // wave per workgroup builds the lookup tables meanwhile (M = 6 304, K = 384: 6.7 us against 7.6 without it).  Beyond
-    // that the grid is what the chip holds at once (1 024 workgroups of four waves, four waves per SIMD), the tables are
-    // built once per workgroup before its first tile, and each wave walks its tiles with the next one's loads in flight
-    // (one workgroup per four tiles, tables rebuilt every time: K = 1 536 at M = 12 608 27-30 us instead of 18-19,
-    // ViT-L's K = 4 096 input 230-258 instead of 171-178).
-    const bool builder = ntiles <= 2048;
-    const int64_t cap = 1024;
-    const unsigned blocks = static_cast<unsigned>(want < cap ? want : cap) + wj.blocks;
-#define ARCQ_LAUNCH_BLOCKED(B)                                                                                            \
-    do {                                                                                                                  \
-        if (builder)                                                                                                      \
-            hipLaunchKernelGGL((act_quant_blocked2_kernel<TIN, B, true>), dim3(blocks), dim3(64 * (kWaves + 1)), 0, stream, \
-                               static_cast<const TIN *>(x), thr, cb, static_cast<__half *>(x_hat), eps, groups_per_row, rows, wj); \
-        else                                                                                                              \
-            hipLaunchKernelGGL((act_quant_blocked2_kernel<TIN, B, false>), dim3(blocks), dim3(64 * kWaves), 0, stream,   \
-                               static_cast<const TIN *>(x), thr, cb, static_cast<__half *>(x_hat), eps, groups_per_row, rows, wj); \
-    } while (0)
-    if (bits == 4) ARCQ_LAUNCH_BLOCKED(4);
-    else if (bits == 3) ARCQ_LAUNCH_BLOCKED(3);
-    else ARCQ_LAUNCH_BLOCKED(2);
-#undef ARCQ_LAUNCH_BLOCKED
-    return launch_status("arcq_act_quant_blocked");
-}
-
 }  // namespace arcq
 
 using namespace arcq;
-
-static int act_quant_blocked_checked(const void *x, int x_dtype, const float *thresholds, const float *codebook,
-                                     void *x_hat_blocked, int64_t rows, int64_t cols, int bits, float eps, void *stream,
-                                     const WeightJob &wj)
-{
-    if (!bits_ok(bits)) return fail(ARCQ_ERR_BITS, "arcq_act_quant_blocked: bits must be 2, 3, or 4");
-    if (rows < 0 || cols < 0) return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_blocked: bad sizes");
-    if (cols % 64 != 0) return fail(ARCQ_ERR_GROUP, "arcq_act_quant_blocked: in_features must be divisible by 64");
-    if (x_dtype != ARCQ_F32 && x_dtype != ARCQ_F16)
-        return fail(ARCQ_ERR_DTYPE, "arcq_act_quant_blocked: x must be float32 or float16");
-    if (rows * cols == 0 && wj.blocks == 0) return ARCQ_OK;
-    if (!x || !thresholds || !codebook || !x_hat_blocked)
-        return fail(ARCQ_ERR_NULL, "arcq_act_quant_blocked: x, thresholds, codebook and x_hat_blocked must not be NULL");
-    if (x_hat_blocked == x) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_act_quant_blocked: x_hat_blocked must not alias x");
-    if (rows * cols * 2 >= (int64_t(1) << 32)) return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_blocked: tensor too large");
-    if (!aligned(x, 16) || !aligned(x_hat_blocked, 16))
-        return fail(ARCQ_ERR_ALIGN, "arcq_act_quant_blocked: x and x_hat_blocked must be 16-byte aligned");
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (x_dtype == ARCQ_F32)
-        return launch_blocked<float>(x, thresholds, codebook, x_hat_blocked, rows, cols, bits, eps, st, wj);
-    return launch_blocked<__half>(x, thresholds, codebook, x_hat_blocked, rows, cols, bits, eps, st, wj);
-}
-
-ARCQ_API int arcq_act_quant_blocked(const void *x, int x_dtype, const float *thresholds, const float *codebook,
-                                    void *x_hat_blocked, int64_t rows, int64_t cols, int bits, float eps, void *stream)
-{
-    return act_quant_blocked_checked(x, x_dtype, thresholds, codebook, x_hat_blocked, rows, cols, bits, eps, stream,
-                                     WeightJob{});
-}
-
-// Stage 1 into the block layout and, in the same launch, w_hat[N, cols] (fp16, group size 64) from the layer's packed
-// weights: the two inputs of the copying GEMM variant.
-ARCQ_API int arcq_act_quant_blocked_with_weights(const void *x, int x_dtype, const float *thresholds,
-                                                 const float *codebook, void *x_hat_blocked, int64_t rows, int64_t cols,
-                                                 int bits, float eps, const uint8_t *packed_w, const float *w_codebook,
-                                                 const float *w_center, const float *w_scale, const float *w_code_sum,
-                                                 void *w_hat, int64_t N, void *stream)
-{
-    if (N < 0) return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_blocked_with_weights: bad sizes");
-    if (N == 0 || cols <= 0 || cols % 64 != 0)      // no weights to rebuild (or sizes the plain entry point reports)
-        return arcq_act_quant_blocked(x, x_dtype, thresholds, codebook, x_hat_blocked, rows, cols, bits, eps, stream);
-    if (!packed_w || !w_codebook || !w_center || !w_scale || !w_code_sum || !w_hat)
-        return fail(ARCQ_ERR_NULL, "arcq_act_quant_blocked_with_weights: NULL weight tensor pointer");
-    if (!aligned(w_hat, 16) || !aligned(packed_w, 4))
-        return fail(ARCQ_ERR_ALIGN, "arcq_act_quant_blocked_with_weights: w_hat must be 16-byte, packed_w 4-byte aligned");
-    if (N * (cols / 8) >= (int64_t(1) << 38))
-        return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_blocked_with_weights: weight tensor too large");
-    WeightJob wj{packed_w, w_codebook, w_center, w_scale, w_code_sum, static_cast<__half *>(w_hat), N, cols,
-                 static_cast<unsigned>((N * (cols / 8) + 255) / 256)};
-    return act_quant_blocked_checked(x, x_dtype, thresholds, codebook, x_hat_blocked, rows, cols, bits, eps, stream, wj);
-}
 
 template <typename TIN>
 static int launch_rows_ln(const void *x, const float *gamma, const float *beta, float ln_eps, const float *thr, const float *cb,

@@ -20,6 +20,7 @@
 #include "arcq_act_quant_core.h"
 #include "arcq_gemm.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace arcq {
@@ -462,21 +463,18 @@ void launch_gemm_tile(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 
 using namespace arcq;
 
-// Column blocks and the tile kernels up to the size where the weight-stationary kernels have the row blocks they want:
-// 8 per workgroup for the two-blocks-per-wave kernel (gemm_pair_pays), or 6 000 rows for the eight-wave one.
-ARCQ_API int arcq_prepared_row_major_fp8(int64_t M, int64_t N, int64_t K)
-{
-    (void)K;
-    return N % 32 != 0 || M >= 6000 ? 1 : 0;
-}
-
+// Column blocks and the tile kernels up to the size where a workgroup of the weight-stationary kernels has five row blocks
+// (one workgroup per compute unit).  Measured at M = 591 .. 25 216 on all layers of the tiny, small, base and large models,
+// fp16 and FP8: the tile kernels win or tie at every shape with four or fewer (3 152 x 768 x 3 072: 31 against 35 us) and
+// lose at every one with five or more (1 576 x 3 072 x 768 with fc2's stage 1: 30 against 25; 6 304 x 768 x 3 072: 55 / 43).
 ARCQ_API int arcq_prepared_row_major(int64_t M, int64_t N, int64_t K)
 {
-    if (M < 512) return 0;
+    (void)K;
     if (N % 32 != 0) return 1;
-    GemmArgs g{};
-    g.M = static_cast<int>(M), g.N = static_cast<int>(N), g.K = static_cast<int>(K);
-    return gemm_pair_pays(g) || M >= 6000 ? 1 : 0;
+    if (M < 512) return 0;
+    const int64_t slabs = (N + 127) / 128, blocks = (M + 31) / 32;
+    const int64_t ranges = std::min<int64_t>(std::max<int64_t>(device_cus() / slabs, 1), blocks);
+    return (blocks + ranges - 1) / ranges >= 5 ? 1 : 0;
 }
 
 ARCQ_API int arcq_linear_prepared(const arcq_linear_prepared_args *a, void *stream)

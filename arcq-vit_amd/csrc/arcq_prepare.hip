@@ -3,10 +3,10 @@
 //
 // Latency-bound up to a few thousand rows (it is one dependent chain: load -> LayerNorm sums -> group sums -> codes ->
 // store, beside another: codes -> lookups -> store), vector-ALU-bound beyond.  What the split of the work does about it:
-//   * A wave owns whole rows when there is a LayerNorm (two lanes per group, 2 G lanes per row, as many rows as fit 64
-//     lanes), so the row sums stay inside the wave: no workgroup barrier, and the number of workgroups is rows / 8 (G =
-//     16) instead of rows / 32.  (act_quant_rows_ln_kernel owns 32 rows per workgroup and meets at five barriers: 18 us
-//     at 591 x 1024 where this takes 7.)  Without one a wave owns 8 or more rows x up to four groups.
+//   * prepare_ln_kernel: a wave owns whole rows, so no row sum needs a workgroup barrier and the number of workgroups is
+//     rows / 8 (G = 16) instead of rows / 32.  (act_quant_rows_ln_kernel owns 32 rows per workgroup and meets at five
+//     barriers: 18 us at 591 x 1024.)
+//   * prepare_kernel: no LayerNorm, tiles of 32 rows x one group.
 //   * x_hat goes to the block layout through LDS in runs of at least 8 rows x 16 bytes, i.e. whole 128-byte lines
 //     wherever the tensor's rows allow it.
 //   * Weights: a wave owns 32 output columns x four groups, lane = (column, half group): 32 codes, one set of metadata
@@ -17,6 +17,8 @@
 // Arithmetic: arcq_act_quant_core.h and the stage-2 expression, unchanged -- bit-identical to the stand-alone kernels.
 #include "arcq_act_quant_core.h"
 #include "arcq_gemm.h"
+
+#include <algorithm>
 
 namespace arcq {
 namespace {
@@ -181,15 +183,173 @@ __device__ __forceinline__ void prep_weights_rows(const PrepWeights &w, unsigned
     store_writethrough16(static_cast<char *>(w.out) + static_cast<int64_t>(idx) * 16, o[0], o[1], o[2], o[3]);
 }
 
-// F8 (LN = false only): FP8 operands.
-// LN = true: LayerNorm over the rows first; GC = all G groups of a row (2 GC lanes per row).
-// LN = false: a wave takes R rows x GC groups; consecutive waves take consecutive group chunks.
-// rows_per_wave = R; chunks = group chunks per row (1 with a LayerNorm).
-template <typename TIN, int BITS, bool LN, bool F8>
-__global__ void __launch_bounds__(kPrepThreads)
-prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta, float ln_eps,
-               const float *__restrict__ thr, const float *__restrict__ cb, char *__restrict__ x_hat, float eps, int rows,
-               int G, int GC, int R, int chunks, int tiles, PrepWeights w0, PrepWeights w1)
+// Weight workgroups come first: they are the longer chain where the rows are few.
+template <int BITS, bool F8>
+__device__ __forceinline__ bool prep_weight_workgroup(const PrepWeights &w0, const PrepWeights &w1, float *lut)
+{
+    if (blockIdx.x >= w0.blocks + w1.blocks) return false;
+    if (threadIdx.x >= kPrepThreads) {          // a table builder has nothing to do here; the job's one barrier counts it
+        __syncthreads();
+        return true;
+    }
+    const bool second = blockIdx.x >= w0.blocks;
+    const PrepWeights &w = second ? w1 : w0;
+    const unsigned block = blockIdx.x - (second ? w0.blocks : 0);
+    if (w.row_major) prep_weights_rows<BITS, F8>(w, block, lut);
+    else prep_weights<BITS, F8>(w, block, lut);
+    return true;
+}
+
+template <typename TIN> struct PrepTile;           // a 32-row x 64-value tile in LDS: odd dword pitch, values per 16 bytes
+template <> struct PrepTile<float> { static constexpr int pitch = 65, vec = 4; };
+template <> struct PrepTile<__half> { static constexpr int pitch = 33, vec = 8; };
+
+// Stage 1 without a LayerNorm: memory-bound from a few thousand rows on (12 608 x 768 fp16: 10.8 us, 8 at the copy rate).  A
+// wave tile is 32 rows x ONE group; lane l owns row l / 2 and the half l % 2 of the group (arcq_act_quant_core.h).  Data moves
+// through a wave-private LDS tile (rows of the tile = rows of the tensor): coalesced 16-byte loads in, every piece column out as
+// one 512-byte run of the block layout.  (Lanes that load their 64 contiguous bytes themselves, four partial lines per
+// instruction: 16.0 us.)
+// BUILDER: a fifth wave that owns no tile builds the lookup tables while the four tile waves load their first tile and take
+// its statistics.  Without it the four build the tables together before their first tile.
+template <typename TIN, int BITS, bool F8, bool BUILDER>
+__global__ void __launch_bounds__(64 * (kPrepWaves + (BUILDER ? 1 : 0)))
+prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const float *__restrict__ cb, char *__restrict__ x_hat, float eps,
+               int rows, int G, PrepWeights w0, PrepWeights w1)
+{
+    constexpr int L = 1 << BITS;
+    constexpr int kInPitch = PrepTile<TIN>::pitch;
+    constexpr int kLoads = 64 / PrepTile<TIN>::vec;        // 16-byte loads per row of the tile (8 fp16 / 16 fp32)
+    constexpr int kRowsPerInstr = 64 / kLoads;             // 8 / 4
+    constexpr int kIters = 32 / kRowsPerInstr;             // 4 / 8
+    constexpr int kPieces = F8 ? 4 : 8;                    // 16-byte pieces of a group of x_hat
+    constexpr int kOutDwords = kPieces * 4, kOutPitch = kOutDwords + 1;
+    __shared__ uint32_t tiles[kPrepWaves][32 * kInPitch];
+    __shared__ float lut[L * 64];
+    __shared__ Bucket table[kMaxBuckets + 1];
+    __shared__ int slow_slots[kPrepWaves];
+    if (prep_weight_workgroup<BITS, F8>(w0, w1, lut)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float th[L - 1], cbv[L];
+    load_quant_params<BITS>(thr, cb, th, cbv);
+    const BucketScale bq = pick_bucket_scale<BITS>(th);
+    if (BUILDER && wave == kPrepWaves) {
+        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, lane, 64);
+        __syncthreads();
+        return;
+    }
+    const int wg = blockIdx.x - (w0.blocks + w1.blocks), wgs = gridDim.x - (w0.blocks + w1.blocks);
+    const int tiles_total = ((rows + 31) / 32) * G;
+    const int64_t K = static_cast<int64_t>(G) * 64;
+    const int row_groups = F8 ? (G + 1) / 2 * 2 : G;       // with the padding
+    const int64_t block_bytes = static_cast<int64_t>(row_groups) * kPieces * 16 * 32;
+    uint32_t *tile = tiles[wave];
+
+    uint4 raw[kIters];
+    auto fetch = [&](int t) {                              // tile t = (row block t / G, group t % G); zeros past the end
+        const int rb = t / G, g = t - rb * G;
+        const int r0 = rb * 32 + lane / kLoads;
+        const TIN *p = x + r0 * K + g * 64 + (lane % kLoads) * PrepTile<TIN>::vec;
+#pragma unroll
+        for (int i = 0; i < kIters; ++i)
+            raw[i] = t < tiles_total && r0 + i * kRowsPerInstr < rows ? *reinterpret_cast<const uint4 *>(p + i * kRowsPerInstr * K)
+                                                                      : make_uint4(0, 0, 0, 0);
+    };
+    fetch(wg * kPrepWaves + wave);
+    bool table_ok = false, tables_built = false;
+    const int row = lane >> 1, half = lane & 1;
+    if constexpr (!BUILDER) {
+        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, kPrepThreads);
+        __syncthreads();
+        table_ok = true;
+#pragma unroll
+        for (int w = 0; w < kPrepWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
+        tables_built = true;
+    }
+    for (int tile0 = wg * kPrepWaves; tile0 < tiles_total; tile0 += wgs * kPrepWaves) {
+        const int t = tile0 + wave;
+        {
+            uint32_t *dst = tile + (lane / kLoads) * kInPitch + (lane % kLoads) * 4;
+#pragma unroll
+            for (int i = 0; i < kIters; ++i) {
+                uint32_t *d = dst + i * kRowsPerInstr * kInPitch;
+                d[0] = raw[i].x; d[1] = raw[i].y; d[2] = raw[i].z; d[3] = raw[i].w;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();                   // the tile is private to the wave and LDS operations execute in order
+        float xv[32];
+        {
+            const uint32_t *src = tile + row * kInPitch + half * (32 * static_cast<int>(sizeof(TIN)) / 4);
+            if constexpr (sizeof(TIN) == 4) {
+#pragma unroll
+                for (int j = 0; j < 32; ++j) xv[j] = __uint_as_float(src[j]);
+            } else {
+#pragma unroll
+                for (int p = 0; p < 16; ++p) {
+                    const uint32_t w = src[p];
+                    xv[2 * p] = __half2float(__ushort_as_half(static_cast<unsigned short>(w & 0xffffu)));
+                    xv[2 * p + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(w >> 16)));
+                }
+            }
+        }
+        fetch(t + wgs * kPrepWaves);                       // the wave's next tile loads under this one's arithmetic
+        float mu, var, s, sum_codes;
+        group_stats32x2(xv, eps, mu, var, s);
+        if (BUILDER && !tables_built) {                    // once per workgroup: the builder wave's tables are ready
+            __syncthreads();
+            table_ok = (slow_slots[0] == 0);
+            tables_built = true;
+        }
+        group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
+        const float code_mean = sum_codes * 0.015625f;
+        {
+            uint32_t *dst = tile + row * kOutPitch + half * (kOutDwords / 2);
+            if constexpr (F8) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    uint32_t o[4];
+                    xhat_fp8x16(xv, 16 * i, s, code_mean, mu, o);
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) dst[4 * i + d] = o[d];
+                }
+            } else {
+#pragma unroll
+                for (int p = 0; p < 16; ++p) {
+                    const __half2 h = __floats2half2_rn(fma_f32(s, xv[2 * p] - code_mean, mu), fma_f32(s, xv[2 * p + 1] - code_mean, mu));
+                    dst[p] = *reinterpret_cast<const uint32_t *>(&h);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (t < tiles_total) {
+            const int rb = t / G, g = t - rb * G;
+            const int r = lane & 31;
+            const int nrows = min(32, rows - rb * 32);     // < 32 in a ragged last block, which is stored compactly
+            char *base = x_hat + rb * block_bytes + (g * kPieces * nrows + r) * 16;
+            if (r < nrows) {
+#pragma unroll
+                for (int j = 0; j < kPieces / 2; ++j) {    // instruction j: piece columns 2j and 2j + 1, nrows x 16 bytes each
+                    const int kp = j * 2 + (lane >> 5);
+                    const uint32_t *src = tile + r * kOutPitch + kp * 4;
+                    store_writethrough16(base + kp * (nrows * 16), src[0], src[1], src[2], src[3]);
+                    if (F8 && row_groups > G && g == G - 1) store_writethrough16(base + (kPieces + kp) * (nrows * 16), 0, 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();                   // the tile is refilled in the next iteration
+    }
+}
+
+// LayerNorm over the rows first.  Wave w of a workgroup's tile takes rows R w ... R w + R - 1, 2 G lanes per row, so that the
+// row sums stay inside the wave.  Vector-ALU-bound from a few thousand rows on, one dependent chain below.  The partial sums of
+// a row go through wave-private LDS padded with zeros to a multiple of eight (x + 0 leaves the sum as it is), so that all reads
+// of a sum are in flight together, and gamma and beta lie in LDS (pitch 36 per 32 values: conflict-free 16-byte reads).  With
+// one read per loop trip and gamma / beta from L2: see the figures at the launch.
+constexpr int kGammaPitch = 36;
+template <typename TIN, int BITS>
+__global__ void __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(4)))
+prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta, float ln_eps,
+                  const float *__restrict__ thr, const float *__restrict__ cb, char *__restrict__ x_hat, float eps, int rows,
+                  int G, int R, int tiles, PrepWeights w0, PrepWeights w1)
 {
     constexpr int L = 1 << BITS;
     constexpr int kIn = 32 * static_cast<int>(sizeof(TIN)) / 16;       // 16-byte loads per lane (32 values)
@@ -197,51 +357,36 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const
     __shared__ float lut[L * 64];
     __shared__ Bucket table[kMaxBuckets + 1];
     __shared__ int slow_slots[kPrepWaves];
-    // The weight workgroups come first: they are the longer chain where the rows are few.
-    if (blockIdx.x < w0.blocks + w1.blocks) {
-        const bool second = blockIdx.x >= w0.blocks;
-        const PrepWeights &w = second ? w1 : w0;
-        const unsigned block = blockIdx.x - (second ? w0.blocks : 0);
-        if (w.row_major) prep_weights_rows<BITS, F8>(w, block, lut);
-        else prep_weights<BITS, F8>(w, block, lut);
-        return;
-    }
+    if (prep_weight_workgroup<BITS, false>(w0, w1, lut)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wg = blockIdx.x - (w0.blocks + w1.blocks), wgs = gridDim.x - (w0.blocks + w1.blocks);
-    const int P = 2 * GC;                                   // lanes per row
+    const int P = 2 * G;                                    // lanes per row
     const int rl = lane / P, pl = lane - rl * P;            // row of the wave, lane of the row
     const int K = G * 64;
     const bool lane_used = rl < R;
-    unsigned char *tile = prep_smem;                         // LN: the workgroup's; else wave-private
-    float *part = reinterpret_cast<float *>(prep_smem + (LN ? kPrepWaves * R * GC * 128 : kPrepWaves * 4096)) + wave * (64 + 16);
-    const int pstride = P;                                   // partial sums of a row
+    const int RW = kPrepWaves * R;                          // rows of a tile
+    const int chunks = (P + 7) / 8;                         // of eight partial sums
+    unsigned char *tile = prep_smem;                        // RW * G * 128 bytes
+    float *part = reinterpret_cast<float *>(prep_smem + RW * G * 128) + wave * (R * chunks * 8);
+    float *s_gamma = reinterpret_cast<float *>(prep_smem + RW * G * 128) + kPrepWaves * (R * chunks * 8);
+    float *s_beta = s_gamma + P * kGammaPitch;
 
-    // Tile t: rows t0 ... of chunk ch.  With a LayerNorm a tile is the workgroup's 4 R rows (wave w rows R w ...);
-    // without one it is a wave's R rows x GC groups, numbered chunk-fastest.
     uint4 raw[kIn];
-    int row, g0;
-    bool valid;
-    auto locate = [&](int t) {
-        if constexpr (LN) {
-            row = t * (kPrepWaves * R) + wave * R + rl;
-            g0 = 0;
-            valid = lane_used && t < tiles && row < rows;
-        } else {
-            const int rt = t / chunks;
-            row = rt * R + rl;
-            g0 = (t - rt * chunks) * GC;
-            valid = lane_used && t < tiles && row < rows && g0 + (pl >> 1) < G;
-        }
-    };
     auto fetch = [&](int t) {
-        locate(t);
-        const uint4 *p = reinterpret_cast<const uint4 *>(x + static_cast<int64_t>(valid ? row : 0) * K + (valid ? g0 * 64 + pl * 32 : 0));
+        const int row = t * RW + wave * R + rl;
+        const bool valid = lane_used && t < tiles && row < rows;
+        const uint4 *p = reinterpret_cast<const uint4 *>(x + static_cast<int64_t>(valid ? row : 0) * K + (valid ? pl * 32 : 0));
 #pragma unroll
         for (int i = 0; i < kIn; ++i) raw[i] = valid ? p[i] : make_uint4(0, 0, 0, 0);
     };
-    const int first = LN ? wg : wg * kPrepWaves + wave;
-    const int step = LN ? wgs : wgs * kPrepWaves;
-    fetch(first);
+    fetch(wg);
+    for (int i = tid; i < K / 4; i += kPrepThreads) {
+        const float4 gv = reinterpret_cast<const float4 *>(gamma)[i], bv = reinterpret_cast<const float4 *>(beta)[i];
+        const int at = (i >> 3) * kGammaPitch + (i & 7) * 4;
+        *reinterpret_cast<float4 *>(s_gamma + at) = gv;
+        *reinterpret_cast<float4 *>(s_beta + at) = bv;
+    }
+    for (int i = lane; i < R * chunks * 8; i += 64) part[i] = 0.0f;
     float th[L - 1], cbv[L];
     load_quant_params<BITS>(thr, cb, th, cbv);
     const BucketScale bq = pick_bucket_scale<BITS>(th);
@@ -251,12 +396,10 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const
 #pragma unroll
     for (int w = 0; w < kPrepWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
     const float fk = static_cast<float>(K);
-    constexpr int kPieces = F8 ? 4 : 8;                     // 16-byte pieces of a group of x_hat
-    const int row_groups = F8 ? (G + 1) / 2 * 2 : G;        // with the padding
-    const int row_bytes = row_groups * kPieces * 16;
+    float *my_part = part + (lane_used ? rl : 0) * (chunks * 8);
+    const float *my_gamma = s_gamma + (lane_used ? pl : 0) * kGammaPitch, *my_beta = s_beta + (lane_used ? pl : 0) * kGammaPitch;
 
-    const int trips = (tiles + (LN ? 1 : kPrepWaves) * wgs - 1) / ((LN ? 1 : kPrepWaves) * wgs);      // the same for every wave
-    for (int trip = 0, t = first; trip < trips; ++trip, t += step) {
+    for (int t = wg; t < tiles; t += wgs) {
         float xv[32];
         if constexpr (sizeof(TIN) == 2) {
 #pragma unroll
@@ -275,177 +418,162 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const
                 xv[4 * i + 2] = __uint_as_float(raw[i].z); xv[4 * i + 3] = __uint_as_float(raw[i].w);
             }
         }
-        const int my_row = row, my_g0 = g0;
-        const bool my_valid = valid;
-        if (trip + 1 < trips) fetch(t + step);            // the next tile loads under this one's arithmetic
-        if constexpr (LN) {
-            // Row sums: every lane folds its 32 values serially, the row's 2 G partial sums are added in a fixed order
-            // (group by group, lower half first) by every lane of the row.  The partial sums go through wave-private
-            // LDS, whose operations execute in order.
-            auto row_total = [&](float mine) {
-                if (lane_used) part[rl * pstride + pl] = mine;
-                __builtin_amdgcn_wave_barrier();
-                const float *src = part + (lane_used ? rl : 0) * pstride;
-                float acc = 0.0f;
-                for (int i = 0; i < P; i += 2) {
-                    const float2 v = *reinterpret_cast<const float2 *>(src + i);
-                    acc += v.x;
-                    acc += v.y;
-                }
-                __builtin_amdgcn_wave_barrier();
-                return acc;
-            };
-            float a = 0.0f;
+        if (t + wgs < tiles) fetch(t + wgs);                // the next tile loads under this one's arithmetic
+        // Row sums: every lane folds its 32 values serially, the row's 2 G partial sums are added in order (group by group,
+        // lower half first) by every lane of the row.
+        auto row_total = [&](float mine) {
+            if (lane_used) my_part[pl] = mine;
+            __builtin_amdgcn_wave_barrier();
+            float acc = 0.0f;
+            for (int c0 = 0; c0 < chunks; c0 += 4) {        // (one trip up to K = 1 024)
+                float4 v[4][2];
 #pragma unroll
-            for (int j = 0; j < 32; ++j) a += xv[j];
-            const float mean = row_total(a) / fk;
-            float q = 0.0f;
+                for (int c = 0; c < 4; ++c)
+                    if (c0 + c < chunks) {
+                        v[c][0] = *reinterpret_cast<const float4 *>(my_part + (c0 + c) * 8);
+                        v[c][1] = *reinterpret_cast<const float4 *>(my_part + (c0 + c) * 8 + 4);
+                    }
 #pragma unroll
-            for (int j = 0; j < 32; ++j) {
-                xv[j] -= mean;
-                const float sq = xv[j] * xv[j];
-                q += sq;
+                for (int c = 0; c < 4; ++c)
+                    if (c0 + c < chunks) {
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            acc += v[c][h].x;
+                            acc += v[c][h].y;
+                            acc += v[c][h].z;
+                            acc += v[c][h].w;
+                        }
+                    }
             }
-            const float rstd = 1.0f / sqrtf(row_total(q) / fk + ln_eps);
-            const float4 *gp = reinterpret_cast<const float4 *>(gamma + (lane_used ? pl : 0) * 32);
-            const float4 *bp = reinterpret_cast<const float4 *>(beta + (lane_used ? pl : 0) * 32);
+            __builtin_amdgcn_wave_barrier();
+            return acc;
+        };
+        float a = 0.0f;
 #pragma unroll
-            for (int j4 = 0; j4 < 8; ++j4) {
-                const float4 gv = gp[j4], bv = bp[j4];
-                const float g4[4] = {gv.x, gv.y, gv.z, gv.w}, b4[4] = {bv.x, bv.y, bv.z, bv.w};
+        for (int j = 0; j < 32; ++j) a += xv[j];
+        const float mean = row_total(a) / fk;
+        float q = 0.0f;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float tv = xv[4 * j4 + e] * rstd;
-                    const float u = tv * g4[e];
-                    float yv = u + b4[e];
-                    if constexpr (sizeof(TIN) == 2) yv = __half2float(__float2half_rn(yv));     // what a LayerNorm kernel stores
-                    xv[4 * j4 + e] = yv;
-                }
+        for (int j = 0; j < 32; ++j) {
+            xv[j] -= mean;
+            const float sq = xv[j] * xv[j];
+            q += sq;
+        }
+        const float rstd = 1.0f / sqrtf(row_total(q) / fk + ln_eps);
+#pragma unroll
+        for (int j4 = 0; j4 < 8; ++j4) {
+            const float4 gv = *reinterpret_cast<const float4 *>(my_gamma + 4 * j4), bv = *reinterpret_cast<const float4 *>(my_beta + 4 * j4);
+            const float g4[4] = {gv.x, gv.y, gv.z, gv.w}, b4[4] = {bv.x, bv.y, bv.z, bv.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float tv = xv[4 * j4 + e] * rstd;
+                const float u = tv * g4[e];
+                float yv = u + b4[e];
+                if constexpr (sizeof(TIN) == 2) yv = __half2float(__float2half_rn(yv));     // what a LayerNorm kernel stores
+                xv[4 * j4 + e] = yv;
             }
         }
         float mu, var, s, sum_codes;
         group_stats32x2(xv, eps, mu, var, s);
         group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
         const float code_mean = sum_codes * 0.015625f;
-        uint4 o[kPieces / 2];
+        // ---- out: piece (k8, row) at LDS slot k8 * RW + row, then 16 bytes per lane, rows fastest ----
+        if (lane_used) {
 #pragma unroll
-        for (int i = 0; i < kPieces / 2; ++i) {
-            uint32_t w[4];
-            if constexpr (F8) {
-                xhat_fp8x16(xv, 16 * i, s, code_mean, mu, w);
-            } else {
+            for (int i = 0; i < 4; ++i) {
+                uint32_t w[4];
 #pragma unroll
                 for (int d = 0; d < 4; ++d) {
                     const int j = 8 * i + 2 * d;
                     const __half2 h = __floats2half2_rn(fma_f32(s, xv[j] - code_mean, mu), fma_f32(s, xv[j + 1] - code_mean, mu));
                     w[d] = *reinterpret_cast<const uint32_t *>(&h);
                 }
+                *reinterpret_cast<uint4 *>(tile + ((pl * 4 + i) * RW + wave * R + rl) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
             }
-            o[i] = make_uint4(w[0], w[1], w[2], w[3]);
         }
-        // ---- out: piece (k, row) at LDS slot k * rows_in_tile + row, then 16 bytes per lane, rows fastest ----
-        if constexpr (LN) {
-            const int RW = kPrepWaves * R;
-            if (lane_used) {
-#pragma unroll
-                for (int i = 0; i < kPieces / 2; ++i)
-                    *reinterpret_cast<uint4 *>(tile + ((pl * (kPieces / 2) + i) * RW + wave * R + rl) * 16) = o[i];
+        __syncthreads();
+        const int r0 = t * RW;
+        const int pieces = G * 8 * RW;
+        for (int p = tid; p < pieces; p += kPrepThreads) {
+            const int k8 = p / RW, r = p - k8 * RW;
+            const int rr = r0 + r;
+            if (rr < rows) {
+                const uint4 v = *reinterpret_cast<const uint4 *>(tile + p * 16);
+                const int blk = rr >> 5, nrows = min(32, rows - blk * 32);
+                store_writethrough16(x_hat + static_cast<int64_t>(blk) * 64 * K + (k8 * nrows + (rr & 31)) * 16, v.x, v.y, v.z, v.w);
             }
-            __syncthreads();
-            const int r0 = t * RW;
-            const int pieces = GC * kPieces * RW;
-            for (int p = tid; p < pieces; p += kPrepThreads) {
-                const int k = p / RW, r = p - k * RW;
-                const int rr = r0 + r;
-                if (rr < rows) {
-                    const uint4 v = *reinterpret_cast<const uint4 *>(tile + p * 16);
-                    const int blk = rr >> 5, nrows = min(32, rows - blk * 32);
-                    store_writethrough16(x_hat + static_cast<int64_t>(blk) * 32 * row_bytes + (k * nrows + (rr & 31)) * 16, v.x, v.y, v.z, v.w);
-                }
-            }
-            __syncthreads();
-        } else {
-            unsigned char *mine = tile + wave * 4096;
-            if (lane_used) {
-#pragma unroll
-                for (int i = 0; i < kPieces / 2; ++i) *reinterpret_cast<uint4 *>(mine + ((pl * (kPieces / 2) + i) * R + rl) * 16) = o[i];
-            }
-            __builtin_amdgcn_wave_barrier();
-            // R is a power of two and R * GC = 32 here: 256 pieces, four per lane (FP8: two)
-            const int rt0 = my_row - rl;
-#pragma unroll
-            for (int i = 0; i < kPieces / 2; ++i) {
-                const int p = i * 64 + lane;
-                const int k = p / R, r = p - k * R;
-                const int rr = rt0 + r;
-                if (rr < rows && t < tiles && my_g0 * kPieces + k < G * kPieces) {
-                    const uint4 v = *reinterpret_cast<const uint4 *>(mine + p * 16);
-                    const int blk = rr >> 5, nrows = min(32, rows - blk * 32);
-                    char *dst = x_hat + static_cast<int64_t>(blk) * 32 * row_bytes + ((my_g0 * kPieces + k) * nrows + (rr & 31)) * 16;
-                    store_writethrough16(dst, v.x, v.y, v.z, v.w);
-                    // (an odd number of groups: GC = 1, and the last group's tile writes the padding group too)
-                    if (F8 && row_groups > G && my_g0 == G - 1) store_writethrough16(dst + kPieces * nrows * 16, 0, 0, 0, 0);
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-            (void)my_valid;
         }
+        __syncthreads();
     }
 }
 
-template <typename TIN, bool F8>
-void launch_prepare_t(const arcq_prepare_args &a, const PrepWeights &w0, const PrepWeights &w1, hipStream_t stream)
+template <typename TIN, int BITS, bool F8>
+void launch_prepare_t(const arcq_prepare_args &a, float eps, const PrepWeights &w0, const PrepWeights &w1, hipStream_t stream)
 {
     const int G = static_cast<int>(a.K / 64), rows = static_cast<int>(a.rows);
-    const bool ln = a.ln_weight != nullptr;
-    int GC, R, chunks, tiles, wgs;
-    size_t smem;
-    if (ln) {
-        GC = G;
-        R = 64 / (2 * G);
-        chunks = 1;
-        tiles = (rows + kPrepWaves * R - 1) / (kPrepWaves * R);
-        wgs = tiles;
-        smem = static_cast<size_t>(kPrepWaves) * R * GC * 128;
-    } else {
-        GC = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
-        R = 32 / GC;
-        chunks = G / GC;
-        tiles = ((rows + R - 1) / R) * chunks;
-        wgs = (tiles + kPrepWaves - 1) / kPrepWaves;
-        smem = kPrepWaves * 4096;
-    }
-    smem += kPrepWaves * (64 + 16) * sizeof(float);
-    // Beyond four workgroups per CU the waves walk their tiles: the lookup tables are built once per workgroup.
-    const int cap = 4 * device_cus();
-    if (rows == 0) wgs = 0;
-    else if (wgs > cap) wgs = cap;
-    const unsigned grid = w0.blocks + w1.blocks + static_cast<unsigned>(wgs);
-    if (grid == 0) return;
-#define ARCQ_LAUNCH_PREP(B, LNV)                                                                                              \
-    do {                                                                                                                       \
-        hipLaunchKernelGGL((prepare_kernel<TIN, B, LNV, F8>), dim3(grid), dim3(kPrepThreads), smem, stream,                    \
-                           static_cast<const TIN *>(a.x), a.ln_weight, a.ln_bias, a.ln_eps, a.thresholds, a.codebook,          \
-                           static_cast<char *>(a.x_hat), 1.0e-6f, rows, G, GC, R, chunks, tiles, w0, w1);                      \
-    } while (0)
+    const unsigned weights = w0.blocks + w1.blocks;
+    const TIN *x = static_cast<const TIN *>(a.x);
+    char *x_hat = static_cast<char *>(a.x_hat);
     if constexpr (!F8) {
-        if (ln) {
-            if (a.bits == 4) ARCQ_LAUNCH_PREP(4, true);
-            else if (a.bits == 3) ARCQ_LAUNCH_PREP(3, true);
-            else ARCQ_LAUNCH_PREP(2, true);
+        if (a.ln_weight && rows > 0) {
+            const int R = 64 / (2 * G), tiles = (rows + kPrepWaves * R - 1) / (kPrepWaves * R);
+            const size_t smem = static_cast<size_t>(kPrepWaves) * R * G * 128 + kPrepWaves * (R * ((2 * G + 7) / 8) * 8) * 4 +
+                                static_cast<size_t>(2 * G) * kGammaPitch * 8;
+            // Beyond four workgroups per CU the waves walk their tiles: the lookup tables are built once per workgroup.
+            const int wgs = std::min(tiles, 4 * device_cus());
+            hipLaunchKernelGGL((prepare_ln_kernel<TIN, BITS>), dim3(weights + wgs), dim3(kPrepThreads), smem, stream, x, a.ln_weight,
+                               a.ln_bias, a.ln_eps, a.thresholds, a.codebook, x_hat, eps, rows, G, R, tiles, w0, w1);
             return;
         }
     }
-    if (a.bits == 4) ARCQ_LAUNCH_PREP(4, false);
-    else if (a.bits == 3) ARCQ_LAUNCH_PREP(3, false);
-    else ARCQ_LAUNCH_PREP(2, false);
-#undef ARCQ_LAUNCH_PREP
+    // Up to 2 048 tiles (two workgroups per CU) the launch is latency-bound: every wave takes one tile and a fifth wave builds the
+    // tables meanwhile (6 304 x 384: 6.7 us against 7.6 without it).  Beyond that the grid is what the chip holds at once, the
+    // tables are built once per workgroup and the waves walk their tiles with the next one's loads in flight (12 608 x 1 536:
+    // 18-19 us; a workgroup per four tiles 27-30).
+    const int tiles = ((rows + 31) / 32) * G, wgs = std::min((tiles + kPrepWaves - 1) / kPrepWaves, 4 * device_cus());
+    if (weights + wgs == 0) return;
+    if (tiles <= 2048)
+        hipLaunchKernelGGL((prepare_kernel<TIN, BITS, F8, true>), dim3(weights + wgs), dim3(kPrepThreads + 64), 0, stream, x, a.thresholds,
+                           a.codebook, x_hat, eps, rows, G, w0, w1);
+    else
+        hipLaunchKernelGGL((prepare_kernel<TIN, BITS, F8, false>), dim3(weights + wgs), dim3(kPrepThreads), 0, stream, x, a.thresholds,
+                           a.codebook, x_hat, eps, rows, G, w0, w1);
+}
+
+template <typename TIN, bool F8>
+void launch_prepare_bits(const arcq_prepare_args &a, float eps, const PrepWeights &w0, const PrepWeights &w1, hipStream_t stream)
+{
+    if (a.bits == 4) launch_prepare_t<TIN, 4, F8>(a, eps, w0, w1, stream);
+    else if (a.bits == 3) launch_prepare_t<TIN, 3, F8>(a, eps, w0, w1, stream);
+    else launch_prepare_t<TIN, 2, F8>(a, eps, w0, w1, stream);
+}
+
+PrepWeights weight_job(const arcq_prepare_weights &w, bool fp8)
+{
+    const int G = static_cast<int>(w.K / 64);
+    const int row_pieces = fp8 ? (G + 1) / 2 * 8 : G * 8;
+    // workgroups: waves of 32 columns x 4 groups, or threads of a piece
+    const unsigned items = w.row_major ? static_cast<unsigned>((w.N * row_pieces + 63) / 64) : static_cast<unsigned>(w.N / 32) * ((G + 3) / 4);
+    return PrepWeights{w.packed, w.codebook, w.center, w.scale, w.code_sum, w.w_hat, static_cast<int>(w.N), G, w.w_mult,
+                       w.row_major != 0, (items + kPrepWaves - 1) / kPrepWaves};
 }
 
 }  // namespace
 }  // namespace arcq
 
 using namespace arcq;
+
+static void launch_prepare(const arcq_prepare_args &a, float eps, const PrepWeights &w0, const PrepWeights &w1, hipStream_t stream)
+{
+    if (a.fp8) {
+        if (a.x_dtype == ARCQ_F32) launch_prepare_bits<float, true>(a, eps, w0, w1, stream);
+        else launch_prepare_bits<__half, true>(a, eps, w0, w1, stream);
+    } else if (a.x_dtype == ARCQ_F32) {
+        launch_prepare_bits<float, false>(a, eps, w0, w1, stream);
+    } else {
+        launch_prepare_bits<__half, false>(a, eps, w0, w1, stream);
+    }
+}
 
 ARCQ_API int arcq_prepare(const arcq_prepare_args *a, void *stream)
 {
@@ -465,10 +593,7 @@ ARCQ_API int arcq_prepare(const arcq_prepare_args *a, void *stream)
         const int G = static_cast<int>(w.K / 64);
         // workgroups: waves of 32 columns x 4 groups, or threads of a piece
         if (a->fp8 && !(w.w_mult > 0.0f)) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_prepare: w_mult must be positive");
-        const int row_pieces = a->fp8 ? (G + 1) / 2 * 8 : G * 8;
-        const unsigned items = w.row_major ? static_cast<unsigned>((w.N * row_pieces + 63) / 64) : static_cast<unsigned>(w.N / 32) * ((G + 3) / 4);
-        pw[i] = PrepWeights{w.packed, w.codebook, w.center, w.scale, w.code_sum, w.w_hat, static_cast<int>(w.N), G, w.w_mult,
-                            w.row_major != 0, (items + kPrepWaves - 1) / kPrepWaves};
+        pw[i] = weight_job(w, a->fp8 != 0);
     }
     if (a->rows > 0) {
         if (a->K % 64 != 0 || a->K == 0) return fail(ARCQ_ERR_GROUP, "arcq_prepare: in_features must be a positive multiple of 64");
@@ -482,14 +607,55 @@ ARCQ_API int arcq_prepare(const arcq_prepare_args *a, void *stream)
             return fail(ARCQ_ERR_ALIGN, "arcq_prepare: x, x_hat, ln_weight and ln_bias must be 16-byte aligned");
     }
     if (a->rows == 0 && !pw[0].blocks && !pw[1].blocks) return ARCQ_OK;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (a->fp8) {
-        if (a->x_dtype == ARCQ_F32) launch_prepare_t<float, true>(*a, pw[0], pw[1], st);
-        else launch_prepare_t<__half, true>(*a, pw[0], pw[1], st);
-    } else if (a->x_dtype == ARCQ_F32) {
-        launch_prepare_t<float, false>(*a, pw[0], pw[1], st);
-    } else {
-        launch_prepare_t<__half, false>(*a, pw[0], pw[1], st);
-    }
+    launch_prepare(*a, 1.0e-6f, pw[0], pw[1], static_cast<hipStream_t>(stream));
     return launch_status("arcq_prepare");
+}
+
+static int act_quant_blocked(const void *x, int x_dtype, const float *thresholds, const float *codebook, void *x_hat_blocked,
+                             int64_t rows, int64_t cols, int bits, float eps, const PrepWeights &w, void *stream)
+{
+    if (!bits_ok(bits)) return fail(ARCQ_ERR_BITS, "arcq_act_quant_blocked: bits must be 2, 3, or 4");
+    if (rows < 0 || cols < 0) return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_blocked: bad sizes");
+    if (cols % 64 != 0) return fail(ARCQ_ERR_GROUP, "arcq_act_quant_blocked: in_features must be divisible by 64");
+    if (x_dtype != ARCQ_F32 && x_dtype != ARCQ_F16)
+        return fail(ARCQ_ERR_DTYPE, "arcq_act_quant_blocked: x must be float32 or float16");
+    if (rows * cols == 0 && w.blocks == 0) return ARCQ_OK;
+    if (!x || !thresholds || !codebook || !x_hat_blocked)
+        return fail(ARCQ_ERR_NULL, "arcq_act_quant_blocked: x, thresholds, codebook and x_hat_blocked must not be NULL");
+    if (x_hat_blocked == x) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_act_quant_blocked: x_hat_blocked must not alias x");
+    if (rows * cols * 2 >= (int64_t(1) << 32)) return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_blocked: tensor too large");
+    if (!aligned(x, 16) || !aligned(x_hat_blocked, 16))
+        return fail(ARCQ_ERR_ALIGN, "arcq_act_quant_blocked: x and x_hat_blocked must be 16-byte aligned");
+    arcq_prepare_args a = {};
+    a.x_dtype = x_dtype, a.bits = bits, a.rows = rows, a.K = cols;
+    a.x = x, a.thresholds = thresholds, a.codebook = codebook, a.x_hat = x_hat_blocked;
+    launch_prepare(a, eps, w, PrepWeights{}, static_cast<hipStream_t>(stream));
+    return launch_status("arcq_act_quant_blocked");
+}
+
+ARCQ_API int arcq_act_quant_blocked(const void *x, int x_dtype, const float *thresholds, const float *codebook,
+                                    void *x_hat_blocked, int64_t rows, int64_t cols, int bits, float eps, void *stream)
+{
+    return act_quant_blocked(x, x_dtype, thresholds, codebook, x_hat_blocked, rows, cols, bits, eps, PrepWeights{}, stream);
+}
+
+// Stage 1 into the block layout and, in the same launch, w_hat[N, cols] (fp16, group size 64) from the layer's packed
+// weights: the two inputs of the copying GEMM variant.
+ARCQ_API int arcq_act_quant_blocked_with_weights(const void *x, int x_dtype, const float *thresholds,
+                                                 const float *codebook, void *x_hat_blocked, int64_t rows, int64_t cols,
+                                                 int bits, float eps, const uint8_t *packed_w, const float *w_codebook,
+                                                 const float *w_center, const float *w_scale, const float *w_code_sum,
+                                                 void *w_hat, int64_t N, void *stream)
+{
+    if (N < 0) return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_blocked_with_weights: bad sizes");
+    if (N == 0 || cols <= 0 || cols % 64 != 0)      // no weights to rebuild (or sizes the plain entry point reports)
+        return arcq_act_quant_blocked(x, x_dtype, thresholds, codebook, x_hat_blocked, rows, cols, bits, eps, stream);
+    if (!packed_w || !w_codebook || !w_center || !w_scale || !w_code_sum || !w_hat)
+        return fail(ARCQ_ERR_NULL, "arcq_act_quant_blocked_with_weights: NULL weight tensor pointer");
+    if (!aligned(w_hat, 16) || !aligned(packed_w, 4))
+        return fail(ARCQ_ERR_ALIGN, "arcq_act_quant_blocked_with_weights: w_hat must be 16-byte, packed_w 4-byte aligned");
+    if (N * cols >= (int64_t(1) << 31))
+        return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_blocked_with_weights: weight tensor too large");
+    const arcq_prepare_weights w = {packed_w, w_codebook, w_center, w_scale, w_code_sum, w_hat, N, cols, 1, 1.0f};
+    return act_quant_blocked(x, x_dtype, thresholds, codebook, x_hat_blocked, rows, cols, bits, eps, weight_job(w, false), stream);
 }

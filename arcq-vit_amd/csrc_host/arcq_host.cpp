@@ -542,9 +542,7 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
         if (!ok) return std::nullopt;
     }
     void *stream = stream_of(x);
-    auto layout = [&](const Plan &p) {
-        return (fp8 ? arcq_prepared_row_major_fp8(rows, p.N, p.K) : arcq_prepared_row_major(rows, p.N, p.K)) != 0;
-    };
+    auto layout = [&](const Plan &p) { return arcq_prepared_row_major(rows, p.N, p.K) != 0; };
     auto weight_bytes = [&](const Plan &p) { return p.N * operand_row_bytes(p.K, fp8); };
     const int64_t wq = weight_bytes(pq), wp = weight_bytes(pp), w1 = weight_bytes(pf1), w2 = weight_bytes(pf2);
     Tensor w = empty({std::max(wq + wp, w1 + w2)}, at::kByte, x.device());

@@ -368,8 +368,8 @@ def run_config(model, bits, batch, steps, warmup, dev, use_graph=False):
         "act_gbs": act_bytes * steps / t_act / 1e9,
         "flops_per_step": flops, "gemm_bytes_per_step": gemm_bytes, "gemm_kernels": per_kernel,
         # stage-1 kernel of the first layer's shape (the large-M layers all take the same one)
-        "act_kernel": {"copy": "act_quant_blocked2_kernel (block layout, weight reconstruction carried along)",
-                       "blocked": "act_quant_blocked2_kernel (block layout)",
+        "act_kernel": {"copy": "prepare_kernel (block layout, weight reconstruction carried along)",
+                       "blocked": "prepare_kernel (block layout)",
                        "rowmajor": "act_quant_g64_kernel / act_quant_small_kernel (row-major)"}[
                            act_layers[0].mode(lib, m) if act_layers else "blocked"],
     }

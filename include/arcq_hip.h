@@ -313,9 +313,8 @@ typedef struct arcq_linear_prepared_args {
 } arcq_linear_prepared_args;
 int arcq_linear_prepared(const arcq_linear_prepared_args *args, void *stream);
 /* Layout of w_hat that arcq_linear_prepared runs fastest on for these sizes: 0 = column blocks (any M), 1 = row-major
- * (M >= 512: the weight-stationary kernels, which want many row blocks). */
+ * (the weight-stationary kernels, which want many row blocks; fp16 operands: M >= 512). */
 int arcq_prepared_row_major(int64_t M, int64_t N, int64_t K);
-int arcq_prepared_row_major_fp8(int64_t M, int64_t N, int64_t K);       /* the same for FP8 operands */
 
 /* arcq_linear_otf_ws for callers that cannot allocate device memory or lend workspaces (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The two
