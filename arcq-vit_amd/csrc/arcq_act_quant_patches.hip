@@ -10,7 +10,15 @@
 // equal, bit for bit, what that kernel writes for the NHWC pixels; what is new is the order of the work: one wave = 32
 // patches x one pixel row of theirs, a lane = eight neighbouring pixels, loads and stores of 16 contiguous bytes, no
 // NHWC copy of the image and no gather of the patch rows afterwards.
-#include "arcq_common.h"
+//
+// Bound by the vector ALUs.  With plain divisions (six of them a pixel, about ten instructions each) and the compare chain (45
+// instructions a value at four bits) a pixel took 230 instructions and 64 images 28 us, 19 MB in and 19 MB out (8 us at the copy
+// rate).  The quotients are therefore reciprocal products with two fused corrections and the codes bucket lookups, as in
+// arcq_act_quant_core.h (about 110 instructions); waves walk their items so that a workgroup builds its tables once.
+#include "arcq_prepare_core.h"
+#include "arcq_gemm.h"
+
+#include <algorithm>
 
 namespace arcq {
 namespace {
@@ -19,100 +27,197 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kP = 16, kC = 3, kKP = kC * kP * kP;      // patch side, channels, 768 values per patch row
 
-template <typename TIN, int BITS>
-__global__ void __launch_bounds__(256)
-act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ thr, const float *__restrict__ cb,
-                         __half *__restrict__ x_hat, int B, int H, int W, float eps, int blocked)
+// RN(d / s) from y = RN(1 / s): exact where neither the operands nor the residuals leave the normal range.
+__device__ __forceinline__ float quotient(float d, float s, float y)
+{
+    float q = d * y;
+    float e = __fmaf_rn(-s, q, d);
+    q = __fmaf_rn(e, y, q);
+    e = __fmaf_rn(-s, q, d);
+    return __fmaf_rn(e, y, q);
+}
+__device__ __forceinline__ bool in_range(float v) { return v == 0.0f || (fabsf(v) >= 0x1p-60f && fabsf(v) <= 0x1p60f); }
+
+// One pixel: its three channels quantized and reconstructed in place.  Returns whether every quotient was in range (FAST).
+template <int BITS, bool FAST>
+__device__ __forceinline__ bool quantize_pixel(float (&x)[kC], float eps, const float (&th)[(1 << BITS) - 1], const float (&cbv)[1 << BITS],
+                                               const BucketScale &bq, const Bucket *table, const char *lut_lane)
 {
     constexpr int L = 1 << BITS;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int lr = lane & 31, lh = lane >> 5;
-    const int pw = W / kP, np = (H / kP) * pw;
-    const int M = B * np;
-    const int64_t wv = static_cast<int64_t>(blockIdx.x) * 4 + (tid >> 6);      // wave = (block of 32 patches, pixel row i)
-    const int blk = static_cast<int>(wv >> 4), i = static_cast<int>(wv & 15);
-    const int m = blk * 32 + lr;
-    if (blk * 32 >= M) return;
-    float th[L - 1], cbv[L];
+    constexpr float third = 1.0f / 3.0f;
+    const float fgs = static_cast<float>(kC);
+    auto by3 = [&](float v) { return FAST ? quotient(v, fgs, third) : v / fgs; };
+    float sum = 0.0f;
 #pragma unroll
-    for (int q = 0; q < L - 1; ++q) th[q] = thr[q];
-#pragma unroll
-    for (int q = 0; q < L; ++q) cbv[q] = cb[q];
-    const int mc = min(m, M - 1);
-    const int b = mc / np, p = mc - b * np, py = p / pw, px = p - py * pw;
-    const TIN *src = img + (static_cast<int64_t>(b) * kC * H + py * kP + i) * W + px * kP + 8 * lh;
-    const int64_t plane = static_cast<int64_t>(H) * W;
-    float x[kC][8];
+    for (int c = 0; c < kC; ++c) sum += x[c];
+    const float mu = by3(sum);
+    float var = 0.0f;
 #pragma unroll
     for (int c = 0; c < kC; ++c) {
-        if constexpr (sizeof(TIN) == 2) {
-            const u32x4_t v = *reinterpret_cast<const u32x4_t *>(src + c * plane);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                x[c][2 * e] = __half2float(__ushort_as_half(static_cast<unsigned short>(v[e] & 0xffffu)));
-                x[c][2 * e + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(v[e] >> 16)));
-            }
-        } else {
-            const float4 v0 = *reinterpret_cast<const float4 *>(src + c * plane);
-            const float4 v1 = *reinterpret_cast<const float4 *>(src + c * plane + 4);
-            x[c][0] = v0.x, x[c][1] = v0.y, x[c][2] = v0.z, x[c][3] = v0.w;
-            x[c][4] = v1.x, x[c][5] = v1.y, x[c][6] = v1.z, x[c][7] = v1.w;
-        }
+        x[c] -= mu;
+        var += x[c] * x[c];
     }
-    const float fgs = static_cast<float>(kC);
-    __half out[kC][8];
+    const float s = sqrtf(by3(var) + eps);
+    float y = 0.0f, sum_codes = 0.0f;
+    if constexpr (FAST) y = 1.0f / s;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        float mu = 0.0f;
-#pragma unroll
-        for (int c = 0; c < kC; ++c) mu += x[c][e];
-        mu /= fgs;
-        float var = 0.0f;
-#pragma unroll
-        for (int c = 0; c < kC; ++c) {
-            const float d = x[c][e] - mu;
-            var += d * d;
-        }
-        const float s = sqrtf(var / fgs + eps);
-        float cv[kC], sum_codes = 0.0f;
-#pragma unroll
-        for (int c = 0; c < kC; ++c) {
-            const float t = (x[c][e] - mu) / s;
+    for (int c = 0; c < kC; ++c) {
+        float v;
+        if constexpr (FAST) {
+            const float t = quotient(x[c], s, y);
+            const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(table) + bucket_offset_of(t, bq));
+            const uint32_t code = static_cast<uint32_t>(bk.base) + ((t > bk.thr) ? 1u : 0u);
+            v = *reinterpret_cast<const float *>(lut_lane + (code << 8));
+        } else {
             // while (code < L - 1 && t > thr[code]) ++code, with the codebook value picked along the way
-            float v = cbv[0];
+            const float t = x[c] / s;
+            v = cbv[0];
             bool alive = true;
 #pragma unroll
             for (int q = 0; q < L - 1; ++q) {
                 alive = alive && (t > th[q]);
                 v = alive ? cbv[q + 1] : v;
             }
-            cv[c] = v;
-            sum_codes += v;
         }
-        const float code_mean = sum_codes / fgs;
-#pragma unroll
-        for (int c = 0; c < kC; ++c) out[c][e] = __float2half_rn(fma_f32(s, cv[c] - code_mean, mu));
+        x[c] = v;
+        sum_codes += v;
     }
-    if (m >= M) return;
-    // piece column of (c, i, half): k / 8 = c * 32 + 2 i + lh
-    const int rows = min(32, M - blk * 32);
+    const float code_mean = by3(sum_codes);
 #pragma unroll
-    for (int c = 0; c < kC; ++c) {
-        const int kp = c * 32 + 2 * i + lh;
-        __half *dst = blocked ? x_hat + static_cast<int64_t>(blk) * 32 * kKP + (static_cast<int64_t>(kp) * rows + lr) * 8
-                              : x_hat + static_cast<int64_t>(m) * kKP + kp * 8;
-        *reinterpret_cast<u32x4_t *>(dst) = *reinterpret_cast<const u32x4_t *>(out[c]);
+    for (int c = 0; c < kC; ++c) x[c] = fma_f32(s, x[c] - code_mean, mu);
+    // (the residuals d_c are 0 or at least 2^-90 once |mu| >= 2^-66 or all of them are 0)
+    return in_range(sum) && in_range(var) && in_range(sum_codes) && s >= 0x1p-60f && s <= 0x1p60f && !(fabsf(mu) < 0x1p-66f && var > 0.0f);
+}
+
+template <typename TIN, int BITS>
+__global__ void __launch_bounds__(kPrepThreads)
+act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ thr, const float *__restrict__ cb,
+                         __half *__restrict__ x_hat, int B, int H, int W, float eps, int blocked, int items, PrepWeights weights)
+{
+    constexpr int L = 1 << BITS;
+    constexpr int kIn = 8 * static_cast<int>(sizeof(TIN)) / 16;
+    __shared__ float lut[L * 64];
+    __shared__ Bucket table[kMaxBuckets + 1];
+    __shared__ int slow_slots[kPrepWaves];
+    if (prep_weight_workgroup<BITS, false>(weights, PrepWeights{}, lut)) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int lr = lane & 31, lh = lane >> 5;
+    const int pw = W / kP, np = (H / kP) * pw;
+    const int M = B * np;
+    const int64_t plane = static_cast<int64_t>(H) * W;
+    const int step = (gridDim.x - weights.blocks) * kPrepWaves;
+    int item = (blockIdx.x - weights.blocks) * kPrepWaves + (tid >> 6);      // (block of 32 patches, pixel row i)
+    uint4 raw[kC][kIn];
+    auto fetch = [&](int it) {
+        it = min(it, items - 1);
+        const int m = min((it >> 4) * 32 + lr, M - 1), i = it & 15;
+        const int b = m / np, p = m - b * np, py = p / pw, px = p - py * pw;
+        const TIN *src = img + (static_cast<int64_t>(b) * kC * H + py * kP + i) * W + px * kP + 8 * lh;
+#pragma unroll
+        for (int c = 0; c < kC; ++c)
+#pragma unroll
+            for (int j = 0; j < kIn; ++j) raw[c][j] = reinterpret_cast<const uint4 *>(src + c * plane)[j];
+    };
+    fetch(item);
+    float th[L - 1], cbv[L];
+    load_quant_params<BITS>(thr, cb, th, cbv);
+    const BucketScale bq = pick_bucket_scale<BITS>(th);
+    build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, kPrepThreads);
+    __syncthreads();
+    bool table_ok = true;
+#pragma unroll
+    for (int w = 0; w < kPrepWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
+    const char *lut_lane = reinterpret_cast<const char *>(lut) + lane * 4;
+
+    for (; item < items; item += step) {
+        float x[8][kC];
+        auto unpack = [&]() {
+#pragma unroll
+            for (int c = 0; c < kC; ++c)
+#pragma unroll
+                for (int j = 0; j < kIn; ++j) {
+                    const uint32_t w[4] = {raw[c][j].x, raw[c][j].y, raw[c][j].z, raw[c][j].w};
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        if constexpr (sizeof(TIN) == 2) {
+                            x[2 * d][c] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[d] & 0xffffu)));
+                            x[2 * d + 1][c] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[d] >> 16)));
+                        } else {
+                            x[4 * j + d][c] = __uint_as_float(w[d]);
+                        }
+                    }
+                }
+        };
+        unpack();
+        bool ok = table_ok;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ok = quantize_pixel<BITS, true>(x[e], eps, th, cbv, bq, table, lut_lane) && ok;
+        if (!__all(ok)) {
+            unpack();
+#pragma unroll
+            for (int e = 0; e < 8; ++e) quantize_pixel<BITS, false>(x[e], eps, th, cbv, bq, table, lut_lane);
+        }
+        const int blk = item >> 4, i = item & 15, m = blk * 32 + lr;
+        fetch(item + step);                                    // (the next item's pixels while this one's leave)
+        if (m < M) {
+            // piece column of (c, i, half): k / 8 = c * 32 + 2 i + lh
+            const int rows = min(32, M - blk * 32);
+#pragma unroll
+            for (int c = 0; c < kC; ++c) {
+                const int kp = c * 32 + 2 * i + lh;
+                __half *dst = blocked ? x_hat + static_cast<int64_t>(blk) * 32 * kKP + (static_cast<int64_t>(kp) * rows + lr) * 8
+                                      : x_hat + static_cast<int64_t>(m) * kKP + kp * 8;
+                uint32_t o[4];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    const __half2 h = __floats2half2_rn(x[2 * d][c], x[2 * d + 1][c]);
+                    o[d] = *reinterpret_cast<const uint32_t *>(&h);
+                }
+                store_writethrough16(dst, o[0], o[1], o[2], o[3]);
+            }
+        }
     }
 }
 
 template <typename TIN, int BITS>
 void launch_patches(const void *img, const float *thr, const float *cb, void *x_hat, int B, int H, int W, float eps, int blocked,
-                    hipStream_t stream)
+                    const PrepWeights &weights, hipStream_t stream)
 {
     const int64_t M = static_cast<int64_t>(B) * (H / kP) * (W / kP);
-    const int64_t waves = (M + 31) / 32 * 16;
-    hipLaunchKernelGGL((act_quant_patches_kernel<TIN, BITS>), dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0, stream,
-                       static_cast<const TIN *>(img), thr, cb, static_cast<__half *>(x_hat), B, H, W, eps, blocked);
+    const int items = static_cast<int>((M + 31) / 32 * 16);
+    const int wgs = std::min((items + kPrepWaves - 1) / kPrepWaves, 4 * device_cus());
+    hipLaunchKernelGGL((act_quant_patches_kernel<TIN, BITS>), dim3(weights.blocks + wgs), dim3(kPrepThreads), 0, stream,
+                       static_cast<const TIN *>(img), thr, cb, static_cast<__half *>(x_hat), B, H, W, eps, blocked, items, weights);
+}
+
+int patches_checked(const char *fn, const void *img, int img_dtype, const float *thresholds, const float *codebook, void *x_hat, int64_t B,
+                    int64_t C, int64_t H, int64_t W, int64_t patch, int bits, float eps, int blocked, const PrepWeights &weights,
+                    void *stream)
+{
+    if (!bits_ok(bits)) return fail(ARCQ_ERR_BITS, "%s: bits must be 2, 3, or 4", fn);
+    if (B < 0 || H < 0 || W < 0) return fail(ARCQ_ERR_SHAPE, "%s: negative size", fn);
+    if (C != kC || patch != kP)
+        return fail(ARCQ_ERR_UNSUPPORTED, "%s: three channels and 16 x 16 patches only (got C=%lld, patch=%lld)", fn,
+                    static_cast<long long>(C), static_cast<long long>(patch));
+    if (H % kP || W % kP) return fail(ARCQ_ERR_SHAPE, "%s: image sides must be multiples of 16", fn);
+    if (img_dtype != ARCQ_F32 && img_dtype != ARCQ_F16) return fail(ARCQ_ERR_DTYPE, "%s: img must be float32 or float16", fn);
+    if (B * H * W == 0) return ARCQ_OK;
+    if (!img || !thresholds || !codebook || !x_hat) return fail(ARCQ_ERR_NULL, "%s: NULL pointer", fn);
+    if (!aligned(img, 16) || !aligned(x_hat, 16)) return fail(ARCQ_ERR_ALIGN, "%s: img and x_hat must be 16-byte aligned", fn);
+    if (B > (1 << 20) || H > (1 << 14) || W > (1 << 14) || B * (H / kP) * (W / kP) >= (int64_t(1) << 26))
+        return fail(ARCQ_ERR_SHAPE, "%s: tensor too large", fn);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int b = static_cast<int>(B), h = static_cast<int>(H), w = static_cast<int>(W);
+#define ARCQ_GO(T) \
+    do { \
+        if (bits == 4) launch_patches<T, 4>(img, thresholds, codebook, x_hat, b, h, w, eps, blocked, weights, st); \
+        else if (bits == 3) launch_patches<T, 3>(img, thresholds, codebook, x_hat, b, h, w, eps, blocked, weights, st); \
+        else launch_patches<T, 2>(img, thresholds, codebook, x_hat, b, h, w, eps, blocked, weights, st); \
+    } while (0)
+    if (img_dtype == ARCQ_F16) ARCQ_GO(__half);
+    else ARCQ_GO(float);
+#undef ARCQ_GO
+    return launch_status(fn);
 }
 
 }  // namespace
@@ -124,28 +229,16 @@ ARCQ_API int arcq_act_quant_patches(const void *img, int img_dtype, const float 
                                     int64_t B, int64_t C, int64_t H, int64_t W, int64_t patch, int bits, float eps, int blocked,
                                     void *stream)
 {
-    if (!bits_ok(bits)) return fail(ARCQ_ERR_BITS, "arcq_act_quant_patches: bits must be 2, 3, or 4");
-    if (B < 0 || H < 0 || W < 0) return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_patches: negative size");
-    if (C != kC || patch != kP)
-        return fail(ARCQ_ERR_UNSUPPORTED, "arcq_act_quant_patches: three channels and 16 x 16 patches only (got C=%lld, patch=%lld)",
-                    static_cast<long long>(C), static_cast<long long>(patch));
-    if (H % kP || W % kP) return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_patches: image sides must be multiples of 16");
-    if (img_dtype != ARCQ_F32 && img_dtype != ARCQ_F16) return fail(ARCQ_ERR_DTYPE, "arcq_act_quant_patches: img must be float32 or float16");
-    if (B * H * W == 0) return ARCQ_OK;
-    if (!img || !thresholds || !codebook || !x_hat) return fail(ARCQ_ERR_NULL, "arcq_act_quant_patches: NULL pointer");
-    if (!aligned(img, 16) || !aligned(x_hat, 16)) return fail(ARCQ_ERR_ALIGN, "arcq_act_quant_patches: img and x_hat must be 16-byte aligned");
-    if (B > (1 << 20) || H > (1 << 14) || W > (1 << 14) || B * (H / kP) * (W / kP) >= (int64_t(1) << 26))
-        return fail(ARCQ_ERR_SHAPE, "arcq_act_quant_patches: tensor too large");
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const int b = static_cast<int>(B), h = static_cast<int>(H), w = static_cast<int>(W);
-#define ARCQ_GO(T) \
-    do { \
-        if (bits == 4) launch_patches<T, 4>(img, thresholds, codebook, x_hat, b, h, w, eps, blocked, st); \
-        else if (bits == 3) launch_patches<T, 3>(img, thresholds, codebook, x_hat, b, h, w, eps, blocked, st); \
-        else launch_patches<T, 2>(img, thresholds, codebook, x_hat, b, h, w, eps, blocked, st); \
-    } while (0)
-    if (img_dtype == ARCQ_F16) ARCQ_GO(__half);
-    else ARCQ_GO(float);
-#undef ARCQ_GO
-    return launch_status("arcq_act_quant_patches");
+    return patches_checked("arcq_act_quant_patches", img, img_dtype, thresholds, codebook, x_hat, B, C, H, W, patch, bits, eps, blocked,
+                           PrepWeights{}, stream);
+}
+
+ARCQ_API int arcq_prepare_patches(const void *img, int img_dtype, const float *thresholds, const float *codebook, void *x_hat, int64_t B,
+                                  int64_t C, int64_t H, int64_t W, int64_t patch, int bits, float eps, const arcq_prepare_weights *weights,
+                                  void *stream)
+{
+    PrepWeights w;
+    const int rc = weight_job_checked("arcq_prepare_patches", weights, false, w);
+    if (rc != ARCQ_OK) return rc;
+    return patches_checked("arcq_prepare_patches", img, img_dtype, thresholds, codebook, x_hat, B, C, H, W, patch, bits, eps, 1, w, stream);
 }

@@ -321,18 +321,17 @@ void run_product(const Plan &p, int64_t rows, const void *x_hat, const Weights &
 }
 bool can_prepare(const Plan &p, int64_t rows)
 {
-    return p.gs == 64 && p.K % 64 == 0 && p.N % 32 == 0 && rows * p.K < (int64_t(1) << 31) && p.N * p.K < (int64_t(1) << 31) &&
+    return p.gs == 64 && p.K % 64 == 0 && (p.N % 32 == 0 || rows >= 512) && rows * p.K < (int64_t(1) << 31) && p.N * p.K < (int64_t(1) << 31) &&
            rows < (int64_t(1) << 26);
 }
 // Whether one layer call runs as prepare + product.  Below 512 rows from K = 768 on (up to 512 inputs the one-launch kernel
 // is 1 us faster: 7.7 against 9.6 us at 197 x 384 x 384; 12.9 against 11.1 at 2 304 x 768, 43 against 16.5 with a LayerNorm
-// at 3 072 x 1 024); above wherever the tile kernels run the product and no one-launch kernel would (1 000 rows: 384 -> 1 152
-// 13.1 -> 12.0 us, 1 024 -> 3 072 32 -> 19, 4 096 -> 1 024 51 -> 32).
+// at 3 072 x 1 024); above wherever no one-launch kernel would run (1 000 rows: 384 -> 1 152 13.1 -> 12.0 us, 1 024 -> 3 072
+// 32 -> 19, 4 096 -> 1 024 51 -> 32).
 bool prepare_pays(const Plan &p, int64_t rows, bool f16_input, bool has_ws, bool layernorm)
 {
     if (!can_prepare(p, rows) || (layernorm && p.K > 2048)) return false;
     if (rows < 512) return p.K >= 768;
-    if (arcq_prepared_row_major(rows, p.N, p.K)) return false;
     return !(f16_input && has_ws && strncmp(arcq_linear_otf_ws_kernel(rows, p.N, p.K, 1), "otf_rows", 8) == 0);
 }
 
@@ -400,7 +399,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
         const bool lent = w_ws != nullptr;
         Tensor scratch = empty({(lent ? 0 : N * K) + m * K}, at::kHalf, x.device());
         char *base = static_cast<char *>(scratch.mutable_data_ptr());
-        const Weights w{lent ? w_ws->mutable_data_ptr() : base, false};
+        const Weights w{lent ? w_ws->mutable_data_ptr() : base, arcq_prepared_row_major(m, N, K) != 0};
         void *x_hat = lent ? base : base + N * K * 2;
         Tensor y = empty(sizes, out_type, x.device());
         run_prepare(x, m, *plan, ln, ln_eps, x_hat, w, nullptr, nullptr, stream);
@@ -626,7 +625,7 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
         if (fp8)
             for (Plan *p : {pq, pp, pf1, pf2}) find_fp8_multiplier(*p);
         const bool chain = is_true(get(d, S.chain_mlp));
-        if (chain && (fp8 || (own && x.size(1) <= 256 && c == 64 * heads))) {
+        if (chain) {
             auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, true, fp8);
             if (whole) return whole;
         }
@@ -831,8 +830,16 @@ PyObject *py_packed_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
         void *stream = stream_of(x);
         if (strcmp(fmt, "hip_fused") == 0 || strcmp(fmt, "dequant_gemm") == 0) {
             if (gs != 64) return none();
-            Tensor x_hat = empty({m * K}, at::kHalf, x.device());
             Tensor y = empty(sizes, at::kFloat, x.device());
+            if (fmt[0] == 'h' && prepare_pays(*plan, m, false, false, false)) {
+                Tensor scratch = empty({N * K + m * K}, at::kHalf, x.device());
+                char *base = static_cast<char *>(scratch.mutable_data_ptr());
+                const Weights w{base, arcq_prepared_row_major(m, N, K) != 0};
+                run_prepare(x, m, *plan, nullptr, 0, base + N * K * 2, w, nullptr, nullptr, stream);
+                run_product(*plan, m, base + N * K * 2, w, nullptr, false, nullptr, y.mutable_data_ptr(), ARCQ_F32, stream);
+                return THPVariable_Wrap(std::move(y));
+            }
+            Tensor x_hat = empty({m * K}, at::kHalf, x.device());
             if (fmt[0] == 'h') {
                 check(arcq_linear_otf_ws(x.const_data_ptr(), ARCQ_F32, fp(A_THR), fp(A_CB), up(W_PACKED), fp(W_CB), fp(W_CENTER),
                                          fp(W_SCALE), fp(W_SUM), fp(W_BIAS), x_hat.mutable_data_ptr(), nullptr,
@@ -891,21 +898,28 @@ PyObject *py_patch_conv_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
             return none();
         const int64_t b = x.size(0), hp = x.size(2) / 16, wp = x.size(3) / 16, m = b * hp * wp, N = plan->N, K = 768;
         const int bits = static_cast<int>(plan->bits);
-        const bool blocked = m >= 512;
         const auto *p = plan->p;
         auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
         const uint8_t *pw = static_cast<const uint8_t *>(p[W_PACKED]);
         void *stream = stream_of(x);
-        Tensor rows = empty({m * K}, at::kHalf, x.device());
         Tensor y = empty({b, hp, wp, N}, x.scalar_type(), x.device());
+        if (can_prepare(*plan, m)) {
+            Tensor scratch = empty({N * K + m * K}, at::kHalf, x.device());
+            char *base = static_cast<char *>(scratch.mutable_data_ptr());
+            const Weights w{base, arcq_prepared_row_major(m, N, K) != 0};
+            void *x_hat = base + N * K * 2;
+            arcq_prepare_weights pwt = {};
+            set_weights(pwt, *plan, w);
+            check(arcq_prepare_patches(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), x_hat, b, 3, x.size(2), x.size(3), 16, bits,
+                                       1.0e-6f, &pwt, stream));
+            run_product(*plan, m, x_hat, w, nullptr, false, nullptr, y.mutable_data_ptr(), code_of(y), stream);
+            return THPVariable_Wrap(y.permute({0, 3, 1, 2}));
+        }
+        Tensor rows = empty({m * K}, at::kHalf, x.device());
         check(arcq_act_quant_patches(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), rows.mutable_data_ptr(), b, 3, x.size(2),
-                                     x.size(3), 16, bits, 1.0e-6f, blocked ? 1 : 0, stream));
-        if (blocked)
-            check(arcq_linear_fused_blocked(rows.const_data_ptr(), pw, fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), nullptr,
-                                            0, y.mutable_data_ptr(), code_of(y), m, N, K, bits, 64, stream));
-        else
-            check(arcq_linear_fused(rows.const_data_ptr(), pw, fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS),
-                                    y.mutable_data_ptr(), code_of(y), m, N, K, bits, 64, stream));
+                                     x.size(3), 16, bits, 1.0e-6f, 0, stream));
+        check(arcq_linear_fused(rows.const_data_ptr(), pw, fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS),
+                                y.mutable_data_ptr(), code_of(y), m, N, K, bits, 64, stream));
         return THPVariable_Wrap(y.permute({0, 3, 1, 2}));
     });
 }

@@ -300,6 +300,10 @@ typedef struct arcq_prepare_args {
     arcq_prepare_weights weights[2];
 } arcq_prepare_args;
 int arcq_prepare(const arcq_prepare_args *args, void *stream);
+/* arcq_act_quant_patches into the block layout, with the weights of one layer in the same launch. */
+int arcq_prepare_patches(const void *img, int img_dtype, const float *thresholds, const float *codebook, void *x_hat,
+                         int64_t B, int64_t C, int64_t H, int64_t W, int64_t patch, int bits, float eps,
+                         const arcq_prepare_weights *weights, void *stream);
 typedef struct arcq_linear_prepared_args {
     int32_t y_dtype, activation, next_bits, w_row_major;
     int64_t M, N, K;
