@@ -36,10 +36,10 @@ __device__ __forceinline__ float quotient(float d, float s, float y)
     e = __fmaf_rn(-s, q, d);
     return __fmaf_rn(e, y, q);
 }
-__device__ __forceinline__ bool in_range(float v) { return v == 0.0f || (fabsf(v) >= 0x1p-60f && fabsf(v) <= 0x1p60f); }
+__device__ __forceinline__ bool in_range(float v) { return (v == 0.0f) | ((fabsf(v) >= 0x1p-60f) & (fabsf(v) <= 0x1p60f)); }
 
 // One pixel: its three channels quantized and reconstructed in place.  Returns whether every quotient was in range (FAST).
-template <int BITS, bool FAST>
+template <int BITS, bool FAST, bool HALF>
 __device__ __forceinline__ bool quantize_pixel(float (&x)[kC], float eps, const float (&th)[(1 << BITS) - 1], const float (&cbv)[1 << BITS],
                                                const BucketScale &bq, const Bucket *table, const char *lut_lane)
 {
@@ -85,8 +85,11 @@ __device__ __forceinline__ bool quantize_pixel(float (&x)[kC], float eps, const 
     const float code_mean = by3(sum_codes);
 #pragma unroll
     for (int c = 0; c < kC; ++c) x[c] = fma_f32(s, x[c] - code_mean, mu);
-    // (the residuals d_c are 0 or at least 2^-90 once |mu| >= 2^-66 or all of them are 0)
-    return in_range(sum) && in_range(var) && in_range(sum_codes) && s >= 0x1p-60f && s <= 0x1p60f && !(fabsf(mu) < 0x1p-66f && var > 0.0f);
+    // d_c is 0 or at least 2^-90 once |mu| >= 2^-66 or all of them are 0 -- and for fp16 inputs (HALF), multiples of 2^-24, always:
+    // their mean is 0 or at least 2^-26, and a mean of exactly 0 (one pixel in a thousand) leaves d_c = x_c.
+    // (No short circuits: a branch per pixel would keep the eight pixels of a lane from overlapping.)
+    const bool means_ok = HALF | !((fabsf(mu) < 0x1p-66f) & (var > 0.0f));
+    return in_range(sum) & in_range(var) & in_range(sum_codes) & (s >= 0x1p-60f) & (s <= 0x1p60f) & means_ok;
 }
 
 template <typename TIN, int BITS>
@@ -151,11 +154,11 @@ act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ 
         unpack();
         bool ok = table_ok;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ok = quantize_pixel<BITS, true>(x[e], eps, th, cbv, bq, table, lut_lane) && ok;
+        for (int e = 0; e < 8; ++e) ok = ok & quantize_pixel<BITS, true, sizeof(TIN) == 2>(x[e], eps, th, cbv, bq, table, lut_lane);
         if (!__all(ok)) {
             unpack();
 #pragma unroll
-            for (int e = 0; e < 8; ++e) quantize_pixel<BITS, false>(x[e], eps, th, cbv, bq, table, lut_lane);
+            for (int e = 0; e < 8; ++e) quantize_pixel<BITS, false, sizeof(TIN) == 2>(x[e], eps, th, cbv, bq, table, lut_lane);
         }
         const int blk = item >> 4, i = item & 15, m = blk * 32 + lr;
         fetch(item + step);                                    // (the next item's pixels while this one's leave)

@@ -7,6 +7,7 @@
 // serial CPU evaluation bit for bit; contraction is switched off for that reason.  Group size 64
 // runs the tiled kernels further down; the two kernels right below take any group size.
 #include "arcq_common.h"
+#include "arcq_gemm.h"
 
 #include <type_traits>
 
@@ -303,8 +304,8 @@ linear_index_tile_kernel(const uint8_t *__restrict__ xq, const float *__restrict
 constexpr int kIdxMinWaves = 3, kIdxMaxWaves = 4;
 constexpr int kIdxRegion = 32 * 33 * 8;            // bytes per wave: operands of half a group, then its terms (33-double pitch)
 
-template <int BITS, int R, int C>
-__global__ void __launch_bounds__(256, R == 1 ? 4 : 3)
+template <int BITS, int R, int C, int MAXW>
+__global__ void __launch_bounds__(64 * MAXW, MAXW > kIdxMaxWaves ? 1 : R == 1 ? 4 : 3)
 linear_index_wide_kernel(const uint8_t *__restrict__ xq, const float *__restrict__ xc, const float *__restrict__ xs,
                          const float *__restrict__ xcs, const uint8_t *__restrict__ wq,
                          const float *__restrict__ wc, const float *__restrict__ ws, const float *__restrict__ wcs,
@@ -555,15 +556,21 @@ struct IndexArgs {
     float *y;
     int rows, out_f, G, levels;
 };
-template <int BITS, int R, int C>
+template <int BITS, int R, int C, int MAXW>
 void launch_index_wide(const IndexArgs &a, hipStream_t stream)
 {
     // Waves per workgroup: the count that leaves the fewest of them without a group in the last round, the larger one of
-    // equals (384 -> 1536, six groups, 12608 rows: three waves 744, four waves 832 us).
-    int S = kIdxMaxWaves;
-    for (int s = kIdxMaxWaves - 1; s >= kIdxMinWaves; --s)
-        if ((a.G + s - 1) / s * s < (a.G + S - 1) / S * S) S = s;
-    hipLaunchKernelGGL((linear_index_wide_kernel<BITS, R, C>), dim3((a.out_f + 8 * C - 1) / (8 * C), (a.rows + 8 * R - 1) / (8 * R)), dim3(64 * S),
+    // equals (384 -> 1536, six groups, 12608 rows: three waves 744, four waves 832 us); of sixteen, the fewest for the fewest rounds.
+    int S = MAXW;
+    if constexpr (MAXW > kIdxMaxWaves) {
+        const int rounds = (a.G + MAXW - 1) / MAXW;
+        S = (a.G + rounds - 1) / rounds;
+        allow_dynamic_lds<linear_index_wide_kernel<BITS, R, C, MAXW>>(MAXW * kIdxRegion);
+    } else {
+        for (int s = kIdxMaxWaves - 1; s >= kIdxMinWaves; --s)
+            if ((a.G + s - 1) / s * s < (a.G + S - 1) / S * S) S = s;
+    }
+    hipLaunchKernelGGL((linear_index_wide_kernel<BITS, R, C, MAXW>), dim3((a.out_f + 8 * C - 1) / (8 * C), (a.rows + 8 * R - 1) / (8 * R)), dim3(64 * S),
                        S * kIdxRegion, stream, a.xq, a.xc, a.xs, a.xcs, a.wq, a.wc, a.ws, a.wcs, a.table, a.a_cb, a.w_cb, a.bias, a.y, a.rows,
                        a.out_f, a.G, a.levels);
 }
@@ -573,8 +580,11 @@ void launch_index_wide(const IndexArgs &a, hipStream_t stream)
 template <int BITS>
 void launch_index(const IndexArgs &a, hipStream_t stream)
 {
-    if (static_cast<int64_t>((a.rows + 7) / 8) * ((a.out_f + 31) / 32) <= 1024) launch_index_wide<BITS, 1, 4>(a, stream);
-    else launch_index_wide<BITS, 2, 4>(a, stream);
+    const int64_t small_tiles = static_cast<int64_t>((a.rows + 7) / 8) * ((a.out_f + 31) / 32);
+    // No more workgroups than compute units: up to sixteen waves each, i.e. as few rounds of groups as possible.
+    if (small_tiles <= device_cus() && a.G > kIdxMaxWaves) launch_index_wide<BITS, 1, 4, 16>(a, stream);
+    else if (small_tiles <= 1024) launch_index_wide<BITS, 1, 4, kIdxMaxWaves>(a, stream);
+    else launch_index_wide<BITS, 2, 4, kIdxMaxWaves>(a, stream);
 }
 
 // Launches of at most this many 16 x 64 tiles give every thread one output instead of four.

@@ -1,6 +1,6 @@
 // Weights of a layer reconstructed by extra workgroups in front of a stage-1 launch's grid.
 //
-// A wave owns 32 output columns x four groups, lane = (column, half group): 32 codes, one set of metadata
+// A wave owns 32 output columns x four groups (fewer in small layers), lane = (column, half group): 32 codes, one set of metadata
 // and four 16-byte stores per group and lane, every store of the wave two 512-byte runs of the weight block layout.
 // All index arithmetic is 32-bit.  (weight_dequant8_kernel owns 8 weights per thread: the 64-bit division and the
 // three metadata loads per 8 weights made it 10 us for 4096 x 1024; here 4.)
@@ -23,6 +23,7 @@ struct PrepWeights {
     int N, G;                // G = K / 64
     float mult;              // FP8: power of two in front of the rounding
     int row_major;
+    int wave_groups;         // column blocks: groups per wave (1, 2 or 4)
     unsigned blocks;         // workgroups (0: no such job)
 };
 
@@ -62,18 +63,18 @@ __device__ __forceinline__ void weights_fp8x16(const float (&v)[32], int j0, flo
     }
 }
 
-// One wave: columns 32 nb ... + 31 of groups 4 gq ... + 3 of a layer's weights.  `lut`: the codebook per lane.
+// One wave: columns 32 nb ... + 31 of `wave_groups` groups of a layer's weights.  `lut`: the codebook per lane.
 template <int BITS, bool F8>
 __device__ __forceinline__ void prep_weights(const PrepWeights &w, unsigned block, float *lut)
 {
     constexpr int L = 1 << BITS;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int quads = (w.G + 3) >> 2;
+    const int runs = (w.G + w.wave_groups - 1) / w.wave_groups;
     const int item = static_cast<int>(block) * kPrepWaves + wave;
-    const int nb = item / quads, g0 = (item - nb * quads) * 4;
+    const int nb = item / runs, g0 = (item - nb * runs) * w.wave_groups;
     const bool mine = nb * 32 < w.N;
     const int n = nb * 32 + (lane & 31), half = lane >> 5;
-    const int ng = mine ? min(4, w.G - g0) : 0;
+    const int ng = mine ? min(w.wave_groups, w.G - g0) : 0;
     uint32_t codes[4][BITS];
     float c[4], s[4], m[4];
     const uint8_t *src = w.packed + static_cast<int64_t>(n) * (w.G * 8 * BITS) + g0 * (8 * BITS) + half * (4 * BITS);
@@ -191,10 +192,14 @@ inline PrepWeights weight_job(const arcq_prepare_weights &w, bool fp8)
 {
     const int G = static_cast<int>(w.K / 64);
     const int row_pieces = fp8 ? (G + 1) / 2 * 8 : G * 8;
-    // workgroups: waves of 32 columns x 4 groups, or threads of a piece
-    const unsigned items = w.row_major ? static_cast<unsigned>((w.N * row_pieces + 63) / 64) : static_cast<unsigned>(w.N / 32) * ((G + 3) / 4);
+    // Groups per wave: four while that makes two waves for every SIMD; a smaller job is as long as one wave's chain, and a wave
+    // with one group is done a microsecond or two earlier.
+    const unsigned columns = static_cast<unsigned>(w.N / 32);
+    const int wg = columns * G >= 8192u ? 4 : columns * G >= 4096u ? 2 : 1;
+    // workgroups: waves of 32 columns x wg groups, or threads of a piece
+    const unsigned items = w.row_major ? static_cast<unsigned>((w.N * row_pieces + 63) / 64) : columns * ((G + wg - 1) / wg);
     return PrepWeights{w.packed, w.codebook, w.center, w.scale, w.code_sum, w.w_hat, static_cast<int>(w.N), G, w.w_mult,
-                       w.row_major != 0, (items + kPrepWaves - 1) / kPrepWaves};
+                       w.row_major != 0, wg, (items + kPrepWaves - 1) / kPrepWaves};
 }
 
 // The job of a caller's description (packed == NULL: none), checked.
