@@ -34,7 +34,8 @@
 // The arithmetic itself lives in arcq_act_quant_core.h (shared with the fused small-M layer kernel).
 #include "arcq_act_quant_core.h"
 #include "arcq_gemm.h"
-#include "arcq_weight_dequant_core.h"
+
+#include <algorithm>
 
 namespace arcq {
 
@@ -154,17 +155,6 @@ __device__ __forceinline__ void pack64(const uint32_t (&c)[64], uint32_t (&w)[2 
 }
 
 // CODES = false drops everything only the code outputs need (the on-the-fly layer asks for x_hat alone).
-// Weight reconstruction carried along by a block-layout stage-1 launch: the first `blocks` workgroups of the grid
-// rebuild out[N,K] (fp16) from packed codes instead of quantizing activations.  Both are inputs of the same GEMM and
-// independent of each other, so one launch does for two.  blocks == 0: nothing to carry.
-struct WeightJob {
-    const uint8_t *packed;
-    const float *cb, *center, *scale, *code_sum;
-    __half *out;
-    int64_t N, K;
-    unsigned blocks;
-};
-
 template <typename TIN, typename TOUT, int BITS, bool CODES>
 __global__ void __launch_bounds__(64 * kWaves)
 act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const float *__restrict__ cb,
@@ -275,6 +265,109 @@ act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
             store_tile<TOUT>(x_hat, elem0, elem_end, tile, lane);
         }
         __syncthreads();   // the tile is reloaded in the next iteration
+    }
+}
+
+// Codes and metadata, no x_hat (the encoding direction): memory-bound.  A wave tile is 32 consecutive groups, which are
+// contiguous in the row-major tensor; two lanes share a group (arcq_act_quant_core.h), the inputs are loaded coalesced and
+// change places in a wave-private LDS tile, and lane l's 32 codes lie at l times their size behind the tile's first: every
+// store of the wave is one contiguous run.  The waves walk their tiles with the next one's loads in flight.  (A lane per group,
+// act_quant_g64_kernel: 297 registers, one or two waves per SIMD; 12 608 x 1 536 fp32 at four bits 31.7 us against 19.1; 18.4 at the copy rate.)
+// BUILDER as in prepare_kernel: a fifth wave builds the lookup tables of a workgroup whose waves have one tile each.
+template <typename TIN, int BITS, bool BYTES, bool BUILDER>
+__global__ void __launch_bounds__(64 * (kWaves + (BUILDER ? 1 : 0)))
+act_quant_codes_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const float *__restrict__ cb,
+                       uint8_t *__restrict__ codes, float *__restrict__ center, float *__restrict__ scale, float *__restrict__ code_sum,
+                       int64_t total_groups, float eps)
+{
+    constexpr int L = 1 << BITS;
+    constexpr int kPitch = Tile<TIN>::stride, kVec = Tile<TIN>::vec;
+    constexpr int kLoads = 64 / kVec, kIters = 32 / kVec;              // 16-byte loads per group, per lane and tile
+    constexpr int kCodeBits = BYTES ? 8 : BITS;
+    __shared__ uint32_t tiles[kWaves][32 * kPitch];
+    __shared__ float lut[L * 64];
+    __shared__ Bucket table[kMaxBuckets + 1];
+    __shared__ int slow_slots[kWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float th[L - 1], cbv[L];
+    load_quant_params<BITS>(thr, cb, th, cbv);
+    const BucketScale bq = pick_bucket_scale<BITS>(th);
+    if (BUILDER && wave == kWaves) {
+        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, lane, 64);
+        __syncthreads();
+        return;
+    }
+    const int64_t ntiles = (total_groups + 31) / 32, step = static_cast<int64_t>(gridDim.x) * kWaves;
+    uint32_t *tile = tiles[wave];
+    uint4 raw[kIters];
+    auto fetch = [&](int64_t t) {                                      // zeros past the end
+        const int64_t g = t * 32 + lane / kLoads;
+        const TIN *p = x + t * 2048 + lane * kVec;
+#pragma unroll
+        for (int i = 0; i < kIters; ++i)
+            raw[i] = g + i * (64 / kLoads) < total_groups ? *reinterpret_cast<const uint4 *>(p + i * 64 * kVec) : make_uint4(0, 0, 0, 0);
+    };
+    int64_t t = static_cast<int64_t>(blockIdx.x) * kWaves + wave;
+    fetch(t);
+    bool table_ok = false, tables_built = false;
+    if constexpr (!BUILDER) {
+        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, 64 * kWaves);
+        __syncthreads();
+        table_ok = true;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
+        tables_built = true;
+    }
+    const int row = lane >> 1, half = lane & 1;
+    for (int64_t tile0 = static_cast<int64_t>(blockIdx.x) * kWaves; tile0 < ntiles; tile0 += step, t += step) {
+        {
+            uint32_t *dst = tile + (lane / kLoads) * kPitch + (lane % kLoads) * 4;
+#pragma unroll
+            for (int i = 0; i < kIters; ++i) {
+                uint32_t *d = dst + i * (64 / kLoads) * kPitch;
+                d[0] = raw[i].x; d[1] = raw[i].y; d[2] = raw[i].z; d[3] = raw[i].w;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();                               // wave-private: LDS operations execute in order
+        float xv[32];
+        {
+            const uint32_t *src = tile + row * kPitch + half * (32 * static_cast<int>(sizeof(TIN)) / 4);
+            if constexpr (sizeof(TIN) == 4) {
+#pragma unroll
+                for (int j = 0; j < 32; ++j) xv[j] = __uint_as_float(src[j]);
+            } else {
+#pragma unroll
+                for (int p = 0; p < 16; ++p) {
+                    const uint32_t w = src[p];
+                    xv[2 * p] = __half2float(__ushort_as_half(static_cast<unsigned short>(w & 0xffffu)));
+                    xv[2 * p + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(w >> 16)));
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        fetch(t + step);
+        float mu, var, s, sum_codes;
+        group_stats32x2(xv, eps, mu, var, s);
+        if (BUILDER && !tables_built) {
+            __syncthreads();
+            table_ok = slow_slots[0] == 0;
+            tables_built = true;
+        }
+        uint32_t w[kCodeBits];
+        group_codes32x2<BITS, kCodeBits>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes, w);
+        const int64_t g = t * 32 + row;
+        if (t < ntiles && g < total_groups) {
+            uint8_t *dst = codes + (t * 64 + lane) * (4 * kCodeBits);
+#pragma unroll
+            for (int d = 0; d + 4 <= kCodeBits; d += 4) *reinterpret_cast<uint4 *>(dst + 4 * d) = make_uint4(w[d], w[d + 1], w[d + 2], w[d + 3]);
+            if constexpr (kCodeBits == 3) *reinterpret_cast<uint3 *>(dst) = make_uint3(w[0], w[1], w[2]);
+            if constexpr (kCodeBits == 2) *reinterpret_cast<uint2 *>(dst) = make_uint2(w[0], w[1]);
+            if (half == 0) {
+                if (center) center[g] = mu;
+                if (scale) scale[g] = s;
+                if (code_sum) code_sum[g] = sum_codes;
+            }
+        }
     }
 }
 
@@ -445,6 +538,26 @@ static int launch(const void *x, const float *thr, const float *cb, uint8_t *pac
         else if (bits == 3) ARCQ_LAUNCH_SMALL(3);
         else ARCQ_LAUNCH_SMALL(2);
 #undef ARCQ_LAUNCH_SMALL
+    } else if (fast && !x_hat && (packed != nullptr) != (codes_u8 != nullptr)) {
+        // The grid is what the chip holds at once (fp32: three workgroups per CU, by their LDS and registers; a fourth that starts
+        // behind them costs 15 %); one tile per wave up to 2 048 tiles (a fifth wave per workgroup builds the tables then).
+        // fp32, four bits, codes and metadata: 12 608 x 1 536 31.7 -> 19.1 us, 50 432 x 1 024 71 -> 41, 394 x 768 7.5 -> 5.3.
+        const int64_t ntiles = (total_groups + 31) / 32, want = (ntiles + kWaves - 1) / kWaves;
+        const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(want, (sizeof(TIN) == 4 ? 3 : 4) * device_cus()));
+        uint8_t *codes = packed ? packed : codes_u8;
+#define ARCQ_LAUNCH_CODES(B, Y)                                                                                                        \
+    do {                                                                                                                               \
+        if (ntiles <= 2048)                                                                                                            \
+            hipLaunchKernelGGL((act_quant_codes_kernel<TIN, B, Y, true>), dim3(blocks), dim3(64 * (kWaves + 1)), 0, stream, xin, thr,   \
+                               cb, codes, center, scale, code_sum, total_groups, eps);                                                  \
+        else                                                                                                                           \
+            hipLaunchKernelGGL((act_quant_codes_kernel<TIN, B, Y, false>), dim3(blocks), dim3(64 * kWaves), 0, stream, xin, thr, cb,    \
+                               codes, center, scale, code_sum, total_groups, eps);                                                      \
+    } while (0)
+        if (bits == 4) { if (packed) ARCQ_LAUNCH_CODES(4, false); else ARCQ_LAUNCH_CODES(4, true); }
+        else if (bits == 3) { if (packed) ARCQ_LAUNCH_CODES(3, false); else ARCQ_LAUNCH_CODES(3, true); }
+        else { if (packed) ARCQ_LAUNCH_CODES(2, false); else ARCQ_LAUNCH_CODES(2, true); }
+#undef ARCQ_LAUNCH_CODES
     } else if (fast) {
         const int64_t ntiles = (total_groups + kTileGroups - 1) / kTileGroups;
         // Up to 3 workgroups fit a CU (LDS); more tiles than that are walked by the grid-stride loop.

@@ -258,14 +258,22 @@ __device__ __forceinline__ void group_stats32x2(float (&xv)[32], float eps, floa
 }
 
 // xv: residuals on entry, cb[code_j] on exit; sum_out = the serial sum of all 64 cb[code_j], in both lanes.  The
-// whole wave must call it (the fast/slow decision is wave-uniform).
-template <int BITS>
+// whole wave must call it (the fast/slow decision is wave-uniform).  CODE_BITS != 0: the 32 codes too, packed CODE_BITS apart
+// into `words`.
+template <int BITS, int CODE_BITS = 0>
 __device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float var, float s,
                                                 const float (&th)[(1 << BITS) - 1], const BucketScale &bq,
                                                 const Bucket *table, const float *lut, bool table_ok, int lane,
-                                                float &sum_out)
+                                                float &sum_out, uint32_t *words = nullptr)
 {
     constexpr int L = 1 << BITS;
+    auto put = [&](int j, uint32_t c) __attribute__((always_inline)) {
+        if constexpr (CODE_BITS != 0) {
+            const int bit = j * CODE_BITS, d = bit >> 5, sh = bit & 31;
+            words[d] = sh == 0 ? c : words[d] | (c << sh);
+            if (sh + CODE_BITS > 32) words[d + 1] = c >> (32 - sh);
+        }
+    };
     const bool lane_fast = (s >= 0x1p-60f) && (s <= 0x1p60f) && !(fabsf(mu) < 0x1p-66f && var > 0.0f);
     const bool fast = table_ok && __all(lane_fast);
     if (fast) {
@@ -283,6 +291,7 @@ __device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float
             const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(table) + bucket_offset_of(q, bq));
             const uint32_t c = static_cast<uint32_t>(bk.base) + ((q > bk.thr) ? 1u : 0u);
             xv[j] = *reinterpret_cast<const float *>(lut_lane + (c << 8));
+            put(j, c);
         }
     } else {
 #pragma unroll
@@ -296,6 +305,7 @@ __device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float
                 c += alive ? 1u : 0u;
             }
             xv[j] = lut[c * 64 + lane];
+            put(j, c);
         }
     }
     sum_out = pair_serial_sum(xv);

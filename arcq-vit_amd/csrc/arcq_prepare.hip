@@ -347,10 +347,11 @@ void launch_prepare_t(const arcq_prepare_args &a, float eps, const PrepWeights &
         }
     }
     // Up to 2 048 tiles (two workgroups per CU) the launch is latency-bound: every wave takes one tile and a fifth wave builds the
-    // tables meanwhile (6 304 x 384: 6.7 us against 7.6 without it).  Beyond that the grid is what the chip holds at once, the
+    // tables meanwhile (6 304 x 384: 6.7 us against 7.6 without it).  Beyond that the grid is what the chip holds at once (fp32: three
+    // workgroups per CU; 12 608 x 1 536 25.4 -> 21.7 us against four), the
     // tables are built once per workgroup and the waves walk their tiles with the next one's loads in flight (12 608 x 1 536:
     // 18-19 us; a workgroup per four tiles 27-30).
-    const int tiles = ((rows + 31) / 32) * G, wgs = std::min((tiles + kPrepWaves - 1) / kPrepWaves, 4 * device_cus());
+    const int tiles = ((rows + 31) / 32) * G, wgs = std::min((tiles + kPrepWaves - 1) / kPrepWaves, (sizeof(TIN) == 4 ? 3 : 4) * device_cus());
     if (weights + wgs == 0) return;
     if (tiles <= 2048)
         hipLaunchKernelGGL((prepare_kernel<TIN, BITS, F8, true>), dim3(weights + wgs), dim3(kPrepThreads + 64), 0, stream, x, a.thresholds,
