@@ -423,12 +423,17 @@ void pick(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 {
     const int cus = device_cus();
     if (!F8 && g.M < 512) {      // (FP8: one order of k at every M, the order of the other FP8 kernel)
-        const int64_t t11 = static_cast<int64_t>((g.M + 31) / 32) * (g.N / 32);
-        const int64_t t12 = static_cast<int64_t>((g.M + 31) / 32) * ((g.N + 63) / 64);
+        // The smallest tile whose launch is one round of workgroups (one per CU); where even 64 x 64 tiles take two, the small
+        // ones spread better.  Measured at 65 .. 511 rows on the layers of the small, base and large models: 1 024 -> 3 072 at 197
+        // rows 5.9 us with 64 x 64 against 7.1 with 32 x 64 (336 of them) and 6.0 with 32 x 32 (672), at 394 rows (336 / 624 /
+        // 1 248) 10.3 / 10.1 / 8.5; 4 096 -> 1 024 at 394 rows 9.9 with 32 x 64 against 11.8 with 32 x 32 (416).
+        const int64_t rt = (g.M + 31) / 32, t11 = rt * (g.N / 32), t12 = rt * ((g.N + 63) / 64);
+        const int64_t t22 = static_cast<int64_t>((g.M + 63) / 64) * ((g.N + 63) / 64);
         if constexpr (NQ == 0) {
-            if (t11 <= 2 * cus) return launch_split<TOUT, 1, 1, 0>(g, w_hat, stream);
+            if (t11 <= cus || (t12 > cus && t22 > cus)) return launch_split<TOUT, 1, 1, 0>(g, w_hat, stream);
         }
-        if (t12 <= 2 * cus) return launch_split<TOUT, 1, 2, NQ>(g, w_hat, stream);
+        // (with the consumer's stage 1: 768 -> 3 072 at 197 rows 8.9 us with 64 x 64 against 10.7, at 394 rows 16.4 / 14.4)
+        if (t12 <= cus || (t22 > cus && t12 <= 3 * cus)) return launch_split<TOUT, 1, 2, NQ>(g, w_hat, stream);
         return launch_split<TOUT, 2, 2, NQ>(g, w_hat, stream);
     }
     // 64 x 64 tiles (two workgroups on a CU) while they fit the chip at once, 128 x 128 beyond: measured crossovers between
