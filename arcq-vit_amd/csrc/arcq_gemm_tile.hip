@@ -98,7 +98,7 @@ gemm_tile_kernel(const unsigned char *__restrict__ xb, const unsigned char *__re
     float *s_bias = reinterpret_cast<float *>(smem + kStages * kStageBytes);      // [TN]
     unsigned char *nq_lds = reinterpret_cast<unsigned char *>(s_bias + TN);
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 31, lh = lane >> 5;
     // Tiles are dealt so that each XCD takes a contiguous run; along the run the operand that is cheaper to fetch once
     // per XCD is the one that repeats (m_fastest: few rows, every XCD reads all of x_hat and an eighth of the weights).
@@ -139,8 +139,7 @@ gemm_tile_kernel(const unsigned char *__restrict__ xb, const unsigned char *__re
 #pragma unroll
         for (int j = 0; j < LPW; ++j) {
             const uint32_t lds = lds0 + static_cast<uint32_t>(slot * kStageBytes + j * 1024);
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src[j] + voff[j]), "s"(__builtin_amdgcn_readfirstlane(lds))
-                         : "memory", "m0");
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff[j]), "s"(src[j]), "s"(lds) : "memory", "m0");
             src[j] += gstep[j];
         }
     };
