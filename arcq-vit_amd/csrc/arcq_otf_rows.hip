@@ -238,7 +238,7 @@ otf_rows_kernel(const RowsParams p)
             }
         }
         if (p.gamma) {
-            // LayerNorm over the row, arithmetic and summation order of act_quant_rows_ln_kernel: every lane folds its
+            // LayerNorm over the row, arithmetic and summation order of prepare_ln_kernel: every lane folds its
             // 32 values serially, the 2 G partial sums of a row meet in LDS and are added group by group, lower half
             // first; y = ((x - mean) * rstd) * gamma + beta, rounded to fp16 as a LayerNorm kernel would store it.
             const float fk = static_cast<float>(K);

@@ -176,7 +176,7 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
         os_convert_group<TIN, EL>(in, xv);
     };
     // LayerNorm of the rows of tile t, on xv in place: arithmetic and summation order of the stand-alone LayerNorm +
-    // stage-1 kernel (act_quant_rows_ln_kernel): every half group of 32 values is summed serially, a row's 2 G
+    // stage-1 kernel (prepare_ln_kernel): every half group of 32 values is summed serially, a row's 2 G
     // partial sums are added in order, mean = sum / K, var = the same sum over (x - mean)^2, / K,
     // y = ((x - mean) * (1 / sqrt(var + eps))) * weight + bias, rounded to x's type.  The partial sums of a wave's
     // rows meet in a wave-private piece of LDS (LDS operations of one wave execute in order: no barrier needed).
