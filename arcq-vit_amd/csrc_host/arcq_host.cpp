@@ -96,7 +96,14 @@ inline void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t
 inline bool here(const Tensor &t) { return t.is_cuda() && t.device().index() == c10::hip::current_device(); }
 inline bool f16(const Tensor &t) { return t.scalar_type() == at::kHalf; }
 inline bool f32(const Tensor &t) { return t.scalar_type() == at::kFloat; }
-inline int code_of(const Tensor &t) { return f16(t) ? ARCQ_F16 : ARCQ_F32; }
+// The library's code of a tensor's type.  It knows two: every tensor that an operation of torch's made (autocast chooses the
+// type of some) goes through as_operand first.
+inline int code_of(const Tensor &t)
+{
+    TORCH_CHECK(f16(t) || f32(t), "expected a float16 or float32 tensor, got ", t.scalar_type());
+    return f16(t) ? ARCQ_F16 : ARCQ_F32;
+}
+inline Tensor as_operand(const Tensor &t) { return (f16(t) || f32(t) ? t : t.to(at::kHalf)).contiguous(); }
 inline const float *fptr(const Tensor &t) { return static_cast<const float *>(t.const_data_ptr()); }
 inline const uint8_t *bptr(const Tensor &t) { return static_cast<const uint8_t *>(t.const_data_ptr()); }
 
@@ -557,7 +564,7 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
         check((fp8 ? arcq_attention_quant_fp8_fwd : arcq_attention_quant_fwd)(qkv.const_data_ptr(), static_cast<const float *>(pp.p[A_THR]),
             static_cast<const float *>(pp.p[A_CB]), static_cast<int>(pp.bits), xh.mutable_data_ptr(), b, n, heads, 64, 0.125f, stream));
     } else {
-        const Tensor a = mix(qkv, heads, false).contiguous();
+        const Tensor a = as_operand(mix(qkv, heads, false));          // (bf16 under autocast to that type)
         run_prepare(a, rows, pp, nullptr, 0, xh.mutable_data_ptr(), Weights{nullptr, false, fp8}, nullptr, nullptr, stream);
     }
     run_product(pp, rows, xh.const_data_ptr(), hp, &x, false, nullptr, x1.mutable_data_ptr(), ARCQ_F16, stream);
@@ -634,7 +641,7 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
         o1.layernorm = n1;
         auto t = layer_call(qkv, x, o1);
         if (!t) return std::nullopt;
-        const Tensor a = mix(*t, heads, own);
+        const Tensor a = as_operand(mix(*t, heads, own));
         Options o2;
         o2.residual = &x;
         auto x1 = layer_call(proj, a, o2);
@@ -664,14 +671,14 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
     bool ok = true;
     Tensor t = layernorm_op(d1, x, ok);
     if (!ok) return std::nullopt;
-    auto q = layer_call(qkv, t, Options{});
+    auto q = layer_call(qkv, as_operand(t), Options{});
     if (!q) return std::nullopt;
-    auto a = layer_call(proj, mix(*q, heads, own), Options{});
+    auto a = layer_call(proj, as_operand(mix(*q, heads, own)), Options{});
     if (!a) return std::nullopt;
     const Tensor x1 = at::add(x, *a);
     t = layernorm_op(d2, x1, ok);
     if (!ok) return std::nullopt;
-    auto h = layer_call(fc1, t, Options{});
+    auto h = layer_call(fc1, as_operand(t), Options{});
     if (!h) return std::nullopt;
     auto y = layer_call(fc2, at::gelu(*h), Options{});
     if (!y) return std::nullopt;

@@ -1,0 +1,62 @@
+"""What the host extension promises around its hot calls: the plain case only, and the interpreter's results where it takes
+over -- types that autocast chooses, flags of any type, copies of modules, grad mode, alignment, memory, threads."""
+import numpy as np
+import pytest
+import torch
+
+import arcq_vit_amd as A
+from arcq_vit_amd import synth
+from arcq_vit_amd.vit import build_packed_vit
+
+pytestmark = pytest.mark.gpu
+
+
+def _packed(k, n, fmt="packed", bits=4, seed=1):
+    src = A.QuantLinearPCARCQ(k, n, True, bits, bits, 64)
+    cb = synth.quantile_codebook(bits)
+    src.act_quant.set_codebook(cb)
+    src.weight_quant.set_codebook(cb)
+    with torch.no_grad():
+        src.linear.weight.copy_(synth.make_weight(n, k, seed))
+        src.linear.bias.copy_(synth.make_bias(n, seed))
+    return A.ARCQPackedLinear(src.eval(), fmt).cuda()
+
+
+def _on_the_fly(k, n, bits=4, seed=1):
+    return A.ARCQPackedLinearOnTheFly.from_packed(_packed(k, n, bits=bits, seed=seed))
+
+
+def _vit(**kw):
+    return build_packed_vit("deit_tiny", 4, num_classes=10, depth=1, **kw)
+
+
+def _tokens(*shape, dtype=torch.float16, seed=3):
+    rows = int(np.prod(shape[:-1]))
+    return synth.make_activation(rows, shape[-1], seed).reshape(shape).cuda().to(dtype)
+
+
+def _interpreted(block, x):
+    """The block as the interpreter runs it, layer by layer: a hook on one of its layers is enough for that."""
+    hook = block.attn.qkv.register_forward_hook(lambda *_: None)
+    try:
+        return block(x)
+    finally:
+        hook.remove()
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("half", [True, False])
+@pytest.mark.parametrize("batch,tokens", [(2, 197), (5, 197), (1, 300)])
+def test_block_under_bf16_autocast(cuda, batch, tokens, half, fused):
+    """torch's attention then hands proj a bf16 tensor, which proj takes rounded to fp16."""
+    block = _vit(half_chain=half, fuse_elementwise=fused).blocks[0]
+    x = _tokens(batch, tokens, 192, dtype=torch.float16 if half else torch.float32)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        try:
+            want = _interpreted(block, x)
+        except ValueError:                 # (a skip connection of another type than the layers' outputs does not fuse)
+            with pytest.raises(ValueError, match="residual"):
+                block(x)
+            return
+        got = block(x)
+    assert got.dtype == want.dtype and torch.equal(got, want)
