@@ -73,7 +73,17 @@ inline PyObject *dict_of(PyObject *o)
     return d ? *d : nullptr;
 }
 inline PyObject *get(PyObject *dict, PyObject *key) { return dict ? PyDict_GetItem(dict, key) : nullptr; }   // borrowed
-inline bool is_true(PyObject *o) { return o == Py_True; }
+// What `if o:` decides; an absent attribute is false.  (May run code of a class's own __bool__.)
+inline bool is_true(PyObject *o)
+{
+    if (o == Py_True) return true;
+    if (!o || o == Py_False || o == Py_None) return false;
+    Py_INCREF(o);
+    const int r = PyObject_IsTrue(o);
+    Py_DECREF(o);
+    if (r < 0) throw Failure{};
+    return r == 1;
+}
 inline bool get_int(PyObject *dict, PyObject *key, int64_t &out)
 {
     PyObject *v = get(dict, key);

@@ -60,3 +60,46 @@ def test_block_under_bf16_autocast(cuda, batch, tokens, half, fused):
             return
         got = block(x)
     assert got.dtype == want.dtype and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("yes,no", [(1, 0), (np.bool_(True), np.bool_(False)), ("yes", "")])
+def test_flags_of_any_type(cuda, yes, no):
+    """Flags decide by their truth, as `if flag:` does, wherever the extension reads them."""
+    fc1, fc2 = _on_the_fly(192, 768), _on_the_fly(768, 192)
+    x = _tokens(197, 192)
+    with torch.no_grad():
+        h = fc1(x, activation="gelu", quantize_for=fc2)
+        ready = fc2(h, input_is_xhat=True)
+        assert torch.equal(fc2(h, input_is_xhat=yes), ready)
+        assert not torch.equal(fc2(h, input_is_xhat=no), ready)
+        f16 = fc1(x)
+        fc1.fp8_operands = True
+        f8 = fc1(x)
+        fc1.fp8_operands = yes
+        assert torch.equal(fc1(x), f8) and not torch.equal(f16, f8)
+        fc1.fp8_operands = no
+        assert torch.equal(fc1(x), f16)
+
+
+def test_block_flags_of_any_type(cuda):
+    x = _tokens(3, 197, 192)
+    results = {}
+    for name, yes, no in (("bool", True, False), ("int", 1, 0)):
+        block = _vit().blocks[0]
+        with torch.no_grad():
+            for fuse, own, chain in ((yes, yes, yes), (yes, no, no), (no, yes, yes), (no, no, no)):
+                block.fuse_elementwise, block.attn.own_kernel, block.chain_mlp = fuse, own, chain
+                results.setdefault((bool(fuse), bool(own), bool(chain)), []).append(block(x))
+    assert all(torch.equal(a, b) for a, b in results.values())
+    assert not torch.equal(results[True, True, True][0], results[False, False, False][0])
+
+
+def test_a_flag_that_raises(cuda):
+    class Odd:
+        def __bool__(self):
+            raise KeyError("odd")
+
+    layer = _on_the_fly(192, 768)
+    layer.fp8_operands = Odd()
+    with pytest.raises(KeyError, match="odd"):
+        layer(_tokens(197, 192))
