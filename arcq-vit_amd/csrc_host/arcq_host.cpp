@@ -23,6 +23,7 @@
 #include <cmath>
 #include <algorithm>
 #include <cstring>
+#include <memory>
 #include <optional>
 #include <string>
 #include <vector>
@@ -140,7 +141,6 @@ struct LayerNormParams {
 };
 constexpr int kMaxSlots = 11;
 struct Plan {
-    bool valid = false;
     c10::DeviceIndex device = -1;
     int64_t K = 0, N = 0, bits = 0, gs = 0;
     Slot slot[kMaxSlots];
@@ -149,72 +149,61 @@ struct Plan {
     std::vector<LayerNormParams> ln;
 };
 
+// The plan of one module, kept in its __dict__.  `owner` is the module it was made for: copy.copy and DataParallel's replicas
+// copy the __dict__ and with it the reference, and a module that finds another one's plan makes its own.  (An address can be
+// compared here: a plan is used only by the living module at it, and every other holder replaces it before the first use.)
+// A plan is not changed by later calls on other buffers: those publish a new one, and a call in flight keeps the one it
+// began with -- Python code that runs in the middle of a call lets other threads call the same module.
 struct PlanObject {
     PyObject_HEAD
-    Plan *plan;
+    std::shared_ptr<Plan> plan;
+    const void *owner;
 };
 PyObject *plan_new(PyTypeObject *type, PyObject *, PyObject *)
 {
     PlanObject *o = reinterpret_cast<PlanObject *>(type->tp_alloc(type, 0));
-    if (o) o->plan = new Plan();
+    if (o) new (&o->plan) std::shared_ptr<Plan>();
     return reinterpret_cast<PyObject *>(o);
 }
 void plan_dealloc(PyObject *o)
 {
-    delete reinterpret_cast<PlanObject *>(o)->plan;
+    reinterpret_cast<PlanObject *>(o)->plan.~shared_ptr();
     Py_TYPE(o)->tp_free(o);
 }
 PyObject *plan_reduce(PyObject *o, PyObject *)      // copies and pickles start empty
 {
     return Py_BuildValue("O()", reinterpret_cast<PyObject *>(Py_TYPE(o)));
 }
-PyObject *plan_get_mult(PyObject *o, void *) { return PyFloat_FromDouble(reinterpret_cast<PlanObject *>(o)->plan->fp8_mult); }
-int plan_set_mult(PyObject *o, PyObject *v, void *)
-{
-    const double d = v ? PyFloat_AsDouble(v) : NAN;
-    if (PyErr_Occurred()) return -1;
-    reinterpret_cast<PlanObject *>(o)->plan->fp8_mult = d;
-    return 0;
-}
 PyMethodDef plan_methods[] = {{"__reduce__", plan_reduce, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
-PyGetSetDef plan_getset[] = {{"fp8_mult", plan_get_mult, plan_set_mult, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // The three kinds of module: their buffers in the order of Plan::slot.
 enum { A_THR, A_CB, W_PACKED, W_CB, W_CENTER, W_SCALE, W_SUM, W_BIAS, P_TABLE, P_CODES, P_DENSE };
 enum class Kind { OnTheFly, Packed, Conv };
 
-Plan *plan_of(PyObject *module, Kind kind, PyObject *&dict)
+std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, PyObject *&dict)
 {
     dict = dict_of(module);
     PyObject *buffers = get(dict, S._buffers);
     if (!buffers || !PyDict_Check(buffers)) return nullptr;
     PyObject *po = get(dict, S._host_plan);
-    Plan *plan;
-    if (po && Py_TYPE(po) == &PlanType) {
+    std::shared_ptr<Plan> plan;
+    if (po && Py_TYPE(po) == &PlanType && reinterpret_cast<PlanObject *>(po)->owner == module)
         plan = reinterpret_cast<PlanObject *>(po)->plan;
-    } else {
-        PyObject *fresh = plan_new(&PlanType, nullptr, nullptr);
-        if (!fresh || PyDict_SetItem(dict, S._host_plan, fresh) != 0) throw Failure{};
-        plan = reinterpret_cast<PlanObject *>(fresh)->plan;
-        Py_DECREF(fresh);
-    }
     PyObject *const names[kMaxSlots] = {S.activation_thresholds, S.activation_codebook, S.packed_weight_codes, S.weight_codebook,
                                         S.weight_center, S.weight_scale, S.weight_code_sum,
                                         kind == Kind::OnTheFly ? S.bias_tensor : S.bias, S.product_table, S.weight_codes_u8,
                                         S.weight_dequant};
     const int n = kind == Kind::Packed ? 11 : 8;
     const Tensor *t[kMaxSlots];
-    bool same = plan->valid;
+    bool same = plan != nullptr;
     for (int i = 0; i < n; ++i) {
         t[i] = as_tensor(get(buffers, names[i]));
         if (!t[i]) return nullptr;
         same = same && plan->slot[i].same(*t[i]);
     }
     if (same) return plan;
-    plan->valid = false;
-    plan->fp8_mult = NAN;
-    plan->ln.clear();
+    plan = std::make_shared<Plan>();
     const c10::Device dev = t[W_PACKED]->device();
     for (int i = 0; i < n; ++i) {
         if (t[i]->numel() == 0) continue;
@@ -235,12 +224,18 @@ Plan *plan_of(PyObject *module, Kind kind, PyObject *&dict)
         plan->p[i] = t[i]->numel() ? plan->slot[i].use.const_data_ptr() : nullptr;
     }
     plan->device = dev.index();
-    plan->valid = true;
+    PlanObject *fresh = reinterpret_cast<PlanObject *>(plan_new(&PlanType, nullptr, nullptr));
+    if (!fresh) throw Failure{};
+    fresh->plan = plan;
+    fresh->owner = module;
+    const int rc = PyDict_SetItem(dict, S._host_plan, reinterpret_cast<PyObject *>(fresh));
+    Py_DECREF(fresh);
+    if (rc != 0) throw Failure{};
     return plan;
 }
 
-// fp32 copies of a LayerNorm's weight and bias (made once per layer and parameter version); nullptr: not the plain case.
-LayerNormParams *layernorm_params(Plan &plan, PyObject *ln, float &eps)
+// fp32 copies of a LayerNorm's weight and bias (made once per layer and parameter version); nullopt: not the plain case.
+std::optional<LayerNormParams> layernorm_params(Plan &plan, PyObject *ln, float &eps)
 {
     PyObject *d = dict_of(ln);
     PyObject *params = get(d, S._parameters);
@@ -248,13 +243,13 @@ LayerNormParams *layernorm_params(Plan &plan, PyObject *ln, float &eps)
     const Tensor *w = as_tensor(get(params, S.weight));
     PyObject *bo = get(params, S.bias);
     const Tensor *b = as_tensor(bo);
-    if (!w || !e || !PyFloat_Check(e) || !shape || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != 1) return nullptr;
-    if (!b && bo != Py_None) return nullptr;
+    if (!w || !e || !PyFloat_Check(e) || !shape || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != 1) return std::nullopt;
+    if (!b && bo != Py_None) return std::nullopt;
     eps = static_cast<float>(PyFloat_AS_DOUBLE(e));
     for (auto &p : plan.ln)
-        if (p.w.same(*w) && p.has_bias == (b != nullptr) && (!b || p.b.same(*b))) return &p;
-    if (!w->is_cuda() || w->device().index() != plan.device || w->numel() != plan.K || w->dim() != 1) return nullptr;
-    if (b && (b->device() != w->device() || b->numel() != plan.K)) return nullptr;
+        if (p.w.same(*w) && p.has_bias == (b != nullptr) && (!b || p.b.same(*b))) return p;
+    if (!w->is_cuda() || w->device().index() != plan.device || w->numel() != plan.K || w->dim() != 1) return std::nullopt;
+    if (b && (b->device() != w->device() || b->numel() != plan.K)) return std::nullopt;
     if (plan.ln.size() >= 4) plan.ln.clear();        // (a layer has one LayerNorm in front of it; a bound, not a policy)
     LayerNormParams p;
     p.w.set(*w, true);
@@ -262,7 +257,7 @@ LayerNormParams *layernorm_params(Plan &plan, PyObject *ln, float &eps)
     if (b) p.b.set(*b, true);
     else p.b.use = at::zeros_like(p.w.use);
     plan.ln.push_back(p);
-    return &plan.ln.back();
+    return p;
 }
 
 // ---- one on-the-fly layer -------------------------------------------------------------------------------------------
@@ -352,10 +347,25 @@ bool prepare_pays(const Plan &p, int64_t rows, bool f16_input, bool has_ws, bool
     return !(f16_input && has_ws && strncmp(arcq_linear_otf_ws_kernel(rows, p.N, p.K, 1), "otf_rows", 8) == 0);
 }
 
+// The power of two inside a layer's FP8 weights (reads the metadata back to the host: once per layer and set of buffers).
+void find_fp8_multiplier(Plan &p)
+{
+    if (!std::isnan(p.fp8_mult)) return;
+    PyObject *args[4];
+    const int slots[4] = {W_CB, W_CENTER, W_SCALE, W_SUM};
+    for (int i = 0; i < 4; ++i) args[i] = THPVariable_Wrap(p.slot[slots[i]].use);
+    PyObject *r = PyObject_CallFunctionObjArgs(g_fp8_multiplier, args[0], args[1], args[2], args[3], nullptr);
+    for (PyObject *a : args) Py_DECREF(a);
+    if (!r) throw Failure{};
+    p.fp8_mult = PyFloat_AsDouble(r);
+    Py_DECREF(r);
+    if (PyErr_Occurred()) throw Failure{};
+}
+
 std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Options &o)
 {
     PyObject *dict;
-    Plan *plan = plan_of(module, Kind::OnTheFly, dict);
+    const auto plan = plan_of(module, Kind::OnTheFly, dict);
     if (!plan || !here(x) || x.device().index() != plan->device || !x.is_contiguous() || (!f16(x) && !f32(x)) || x.dim() < 1 ||
         x.size(-1) != plan->K || x.numel() == 0)
         return std::nullopt;
@@ -368,7 +378,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
     const bool fp8 = is_true(get(dict, S.fp8_operands));
     const bool extras = o.layernorm || o.gelu || o.residual || o.next || o.x_is_xhat;
     float ln_eps = 0.0f;
-    LayerNormParams *ln = nullptr;
+    std::optional<LayerNormParams> ln;
     if (extras) {
         if (fp8 || plan->gs != 64 || K % 64 != 0) return std::nullopt;
         if (o.layernorm) {
@@ -381,7 +391,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
                            !o.residual->is_contiguous() || o.residual->numel() != m * N || o.residual->size(-1) != N))
             return std::nullopt;
     }
-    Plan *next = nullptr;
+    std::shared_ptr<Plan> next;
     if (o.next) {
         PyObject *nd;
         next = plan_of(o.next, Kind::OnTheFly, nd);
@@ -393,7 +403,8 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
     const auto *p = plan->p;
     auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
     if (fp8) {
-        if (plan->gs != 64 || std::isnan(plan->fp8_mult)) return std::nullopt;
+        if (plan->gs != 64) return std::nullopt;
+        find_fp8_multiplier(*plan);
         const int64_t kp = (K + 127) / 128 * 128;
         Tensor x8 = empty({m * kp}, at::kByte, x.device()), w8 = empty({N * kp}, at::kByte, x.device());
         Tensor y = empty(sizes, out_type, x.device());
@@ -411,7 +422,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
             w_ws->device() != x.device())
             return std::nullopt;
     }
-    if (!next && !o.x_is_xhat && prepare_pays(*plan, m, f16(x), w_ws != nullptr, ln != nullptr)) {
+    if (!next && !o.x_is_xhat && prepare_pays(*plan, m, f16(x), w_ws != nullptr, ln.has_value())) {
         // (x_hat and w_hat in one scratch tensor; w_hat first: 512-byte runs stay aligned)
         const bool lent = w_ws != nullptr;
         Tensor scratch = empty({(lent ? 0 : N * K) + m * K}, at::kHalf, x.device());
@@ -419,7 +430,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
         const Weights w{lent ? w_ws->mutable_data_ptr() : base, arcq_prepared_row_major(m, N, K) != 0};
         void *x_hat = lent ? base : base + N * K * 2;
         Tensor y = empty(sizes, out_type, x.device());
-        run_prepare(x, m, *plan, ln, ln_eps, x_hat, w, nullptr, nullptr, stream);
+        run_prepare(x, m, *plan, ln ? &*ln : nullptr, ln_eps, x_hat, w, nullptr, nullptr, stream);
         run_product(*plan, m, x_hat, w, o.residual, o.gelu, nullptr, y.mutable_data_ptr(), code_of(y), stream);
         return y;
     }
@@ -547,7 +558,7 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
     // that range the seven launches win (6 304 rows: 1 353 -> 1 262 us; 25 216 rows: 3 341 -> 3 286).
     if (fuse_ln && rows > 9000 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) return std::nullopt;
     float e1 = 0, e2 = 0;
-    LayerNormParams *l1 = nullptr, *l2 = nullptr;
+    std::optional<LayerNormParams> l1, l2;
     Tensor t = x;
     if (fuse_ln) {
         l1 = layernorm_params(pq, n1, e1), l2 = layernorm_params(pf1, n2, e2);
@@ -568,7 +579,7 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
     Tensor qkv = empty({b, n, pq.N}, at::kHalf, x.device());
     Tensor x1 = empty(x.sizes(), at::kHalf, x.device()), y = empty(x.sizes(), at::kHalf, x.device());
     const Weights hq{wb, layout(pq), fp8}, hp{wb + wq, layout(pp), fp8}, h1{wb, layout(pf1), fp8}, h2{wb + w1, layout(pf2), fp8};
-    run_prepare(t, rows, pq, l1, e1, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
+    run_prepare(t, rows, pq, l1 ? &*l1 : nullptr, e1, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
     run_product(pq, rows, xh.const_data_ptr(), hq, nullptr, false, nullptr, qkv.mutable_data_ptr(), ARCQ_F16, stream);
     if (own_attention) {
         check((fp8 ? arcq_attention_quant_fp8_fwd : arcq_attention_quant_fwd)(qkv.const_data_ptr(), static_cast<const float *>(pp.p[A_THR]),
@@ -581,25 +592,10 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
     bool ok = true;
     t = fuse_ln ? x1 : layernorm_op(dict_of(n2), x1, ok);
     if (!ok) return std::nullopt;
-    run_prepare(t, rows, pf1, l2, e2, xh.mutable_data_ptr(), h1, &pf2, &h2, stream);
+    run_prepare(t, rows, pf1, l2 ? &*l2 : nullptr, e2, xh.mutable_data_ptr(), h1, &pf2, &h2, stream);
     run_product(pf1, rows, xh.const_data_ptr(), h1, nullptr, true, &pf2, wide.mutable_data_ptr(), ARCQ_F16, stream);
     run_product(pf2, rows, wide.const_data_ptr(), h2, &x1, false, nullptr, y.mutable_data_ptr(), ARCQ_F16, stream);
     return y;
-}
-
-// The power of two inside a layer's FP8 weights (reads the metadata back to the host: once per layer and set of buffers).
-void find_fp8_multiplier(Plan &p)
-{
-    if (!std::isnan(p.fp8_mult)) return;
-    PyObject *args[4];
-    const int slots[4] = {W_CB, W_CENTER, W_SCALE, W_SUM};
-    for (int i = 0; i < 4; ++i) args[i] = THPVariable_Wrap(p.slot[slots[i]].use);
-    PyObject *r = PyObject_CallFunctionObjArgs(g_fp8_multiplier, args[0], args[1], args[2], args[3], nullptr);
-    for (PyObject *a : args) Py_DECREF(a);
-    if (!r) throw Failure{};
-    p.fp8_mult = PyFloat_AsDouble(r);
-    Py_DECREF(r);
-    if (PyErr_Occurred()) throw Failure{};
 }
 
 // One transformer block (vit.Block.forward), both of its forms; nullopt before anything has been launched where a module
@@ -624,8 +620,8 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
     if (!get_int(ad, S.num_heads, heads) || heads <= 0) return std::nullopt;
     const bool own = is_true(get(ad, S.own_kernel));
     PyObject *dq, *dp, *df1, *df2;
-    Plan *pq = plan_of(qkv, Kind::OnTheFly, dq), *pp = plan_of(proj, Kind::OnTheFly, dp), *pf1 = plan_of(fc1, Kind::OnTheFly, df1),
-         *pf2 = plan_of(fc2, Kind::OnTheFly, df2);
+    const auto pq = plan_of(qkv, Kind::OnTheFly, dq), pp = plan_of(proj, Kind::OnTheFly, dp), pf1 = plan_of(fc1, Kind::OnTheFly, df1),
+               pf2 = plan_of(fc2, Kind::OnTheFly, df2);
     const int64_t c = x.size(2);
     if (!pq || !pp || !pf1 || !pf2 || pq->K != c || pq->N != 3 * c || pp->K != c || pp->N != c || pf1->K != c || pf2->K != pf1->N ||
         pf2->N != c || c % heads != 0)
@@ -637,10 +633,10 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
             if (is_true(get(l, S.fp8_operands)) != fp8 || get(l, S.out_dtype) != reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf)))
                 return std::nullopt;
         if (!f16(x) || c > (rows >= 512 ? 1024 : 1536) || c % 64 != 0 || pf2->K % 64 != 0) return std::nullopt;
-        for (Plan *p : {pq, pp, pf1, pf2})
+        for (Plan *p : {pq.get(), pp.get(), pf1.get(), pf2.get()})
             if (p->gs != 64) return std::nullopt;
         if (fp8)
-            for (Plan *p : {pq, pp, pf1, pf2}) find_fp8_multiplier(*p);
+            for (Plan *p : {pq.get(), pp.get(), pf1.get(), pf2.get()}) find_fp8_multiplier(*p);
         const bool chain = is_true(get(d, S.chain_mlp));
         if (chain) {
             auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, true, fp8);
@@ -830,7 +826,7 @@ PyObject *py_packed_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
         if (!xp) return none();
         const Tensor &x = *xp;
         PyObject *dict;
-        Plan *plan = plan_of(args[0], Kind::Packed, dict);
+        const auto plan = plan_of(args[0], Kind::Packed, dict);
         if (!plan || !here(x) || x.device().index() != plan->device || !f32(x) || !x.is_contiguous() || x.dim() < 1 ||
             x.size(-1) != plan->K || x.numel() == 0)
             return none();
@@ -903,7 +899,7 @@ PyObject *py_patch_conv_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
         if (!xp) return none();
         const Tensor &x = *xp;
         PyObject *dict;
-        Plan *plan = plan_of(args[0], Kind::Conv, dict);
+        const auto plan = plan_of(args[0], Kind::Conv, dict);
         int64_t ags, c;
         PyObject *ks = get(dict, S.kernel_size);
         if (!plan || plan->gs != 64 || !get_int(dict, S.act_group_size, ags) || ags != 3 || !get_int(dict, S.in_channels, c) || c != 3 ||
@@ -981,7 +977,6 @@ PyMODINIT_FUNC PyInit__arcq_host(void)
     PlanType.tp_new = plan_new;
     PlanType.tp_dealloc = plan_dealloc;
     PlanType.tp_methods = plan_methods;
-    PlanType.tp_getset = plan_getset;
     if (PyType_Ready(&PlanType) < 0) return nullptr;
     PyObject *m = PyModule_Create(&module_def);
     if (!m) return nullptr;

@@ -31,7 +31,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
-from . import _lib, ops
+from . import _lib
 
 
 def clear_workspaces() -> None:
@@ -188,17 +188,10 @@ class ARCQPackedLinearOnTheFly(nn.Module):
             if r2.dtype != self.out_dtype or tuple(r2.shape) != (m, self.out_features) or r2.device != x2.device:
                 raise ValueError("residual must have the output's shape, dtype and device")
             residual = r2.contiguous()
-        host = _lib.host()
-        call = (self, x2, layernorm, activation == "gelu", residual, quantize_for, bool(input_is_xhat))
+        if self.fp8_operands and self.group_size != 64:
+            raise ValueError("fp8_operands needs group_size 64")
         with torch.cuda.device(x2.device):
-            y = host.layer_forward(*call)
-            if y is None and self.fp8_operands:
-                if self.group_size != 64:
-                    raise ValueError("fp8_operands needs group_size 64")
-                # (reads the metadata back once per layer; the extension forgets it when a buffer changes)
-                self._host_plan.fp8_mult = ops.fp8_weight_multiplier(self.weight_codebook, self.weight_center,
-                                                                     self.weight_scale, self.weight_code_sum)
-                y = host.layer_forward(*call)
+            y = _lib.host().layer_forward(self, x2, layernorm, activation == "gelu", residual, quantize_for, input_is_xhat)
         if y is None:
             raise RuntimeError("x and the layer's buffers must be contiguous CUDA tensors of the types the layer was built with")
         return y.reshape(*original_shape[:-1], self.out_features)

@@ -103,3 +103,51 @@ def test_a_flag_that_raises(cuda):
     layer.fp8_operands = Odd()
     with pytest.raises(KeyError, match="odd"):
         layer(_tokens(197, 192))
+
+
+def test_copies_of_a_layer_have_plans_of_their_own(cuda):
+    """DataParallel's replicas and shallow copies carry the __dict__ of the layer they were made from."""
+    import copy
+    layer, x = _on_the_fly(192, 768), _tokens(197, 192)
+    with torch.no_grad():
+        want = layer(x)
+        replica = layer._replicate_for_data_parallel()
+        assert replica._host_plan is layer._host_plan                  # handed over by the copy, not to be used by it
+        replica._buffers["bias_tensor"] = layer.bias_tensor + 64.0
+        shifted = replica(x)
+        assert not torch.equal(shifted, want) and replica._host_plan is not layer._host_plan
+        plans = layer._host_plan, replica._host_plan
+        assert torch.equal(layer(x), want) and torch.equal(replica(x), shifted)
+        assert (layer._host_plan, replica._host_plan) == plans         # neither call disturbed the other's
+        for other in (copy.copy(layer), copy.deepcopy(layer)):
+            assert torch.equal(other(x), want) and other._host_plan is not layer._host_plan
+
+
+def test_replicas_on_threads_and_streams(cuda):
+    """A layer and its replica with other weights, called from two threads on streams of their own while their buffers are
+    replaced: with FP8 operands a call then stops to read the metadata back, and the other thread runs meanwhile."""
+    import threading
+    layer, x = _on_the_fly(192, 768), _tokens(600, 192)
+    layer.fp8_operands = True
+    replica = layer._replicate_for_data_parallel()
+    replica._buffers["weight_scale"] = layer.weight_scale * 64.0
+    replica._buffers["weight_center"] = layer.weight_center * 64.0
+    with torch.no_grad():
+        want = [m(x).clone() for m in (layer, replica)]
+    assert not torch.equal(*want)
+    torch.cuda.synchronize()
+    failures = []
+
+    def work(module, expected):
+        with torch.cuda.stream(torch.cuda.Stream()), torch.no_grad():
+            for _ in range(20):
+                module._buffers["weight_scale"] = module.weight_scale.clone()
+                if not torch.equal(module(x), expected):
+                    failures.append(module)
+
+    threads = [threading.Thread(target=work, args=a) for a in zip((layer, replica), want)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures
