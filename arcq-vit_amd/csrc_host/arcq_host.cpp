@@ -119,25 +119,53 @@ inline const float *fptr(const Tensor &t) { return static_cast<const float *>(t.
 inline const uint8_t *bptr(const Tensor &t) { return static_cast<const uint8_t *>(t.const_data_ptr()); }
 
 // ---- a layer's buffers, as the library takes them -------------------------------------------------------------------
+// One buffer as it was last seen: compared at every call, and converted only where the library does not take it as it lies.
+// The memory stays the module's to give back: the storage is held weakly, which is enough for its address to name it.
 struct Slot {
-    Tensor src, use;          // the module's buffer (kept: its identity is what is compared) and what is handed to the library
+    std::optional<c10::weak_intrusive_ptr<c10::StorageImpl>> storage;
+    Tensor copy;              // fp32 / contiguous, where the tensor is not
     uint32_t version = 0;
     const void *data = nullptr;
+    at::ScalarType type = at::kByte;
+    at::DimVector sizes, strides;
     bool same(const Tensor &t) const
     {
-        return src.unsafeGetTensorImpl() == t.unsafeGetTensorImpl() && version == version_of(t) && data == t.const_data_ptr();
+        return storage && storage->_unsafe_get_target() == t.unsafeGetTensorImpl()->unsafe_storage().unsafeGetStorageImpl() &&
+               version == version_of(t) && data == t.const_data_ptr() && type == t.scalar_type() && t.sizes().equals(sizes) &&
+               t.strides().equals(strides);
     }
     void set(const Tensor &t, bool as_f32)
     {
-        src = t;
+        storage.emplace(t.storage().getWeakStorageImpl());
         version = version_of(t);
         data = t.const_data_ptr();
-        use = (as_f32 ? t.detach().to(at::kFloat) : t.detach()).contiguous();
+        type = t.scalar_type();
+        sizes = t.sizes();
+        strides = t.strides();
+        const Tensor use = (as_f32 ? t.detach().to(at::kFloat) : t.detach()).contiguous();
+        if (use.const_data_ptr() != data) copy = use;
+    }
+    const void *ptr() const { return copy.defined() ? copy.const_data_ptr() : data; }
+    int64_t numel() const { return c10::multiply_integers(sizes); }
+};
+// References to Python objects for the length of a call (the GIL is held where it is made and where it ends).
+struct Refs {
+    std::vector<PyObject *> held;
+    Refs() { held.reserve(40); }
+    Refs(const Refs &) = delete;
+    ~Refs() { for (PyObject *o : held) Py_DECREF(o); }
+    void add(PyObject *o)
+    {
+        Py_INCREF(o);
+        held.push_back(o);
     }
 };
 struct LayerNormParams {
     Slot w, b;
-    bool has_bias = false;
+    Tensor no_bias;           // zeros, for a LayerNorm without one
+    bool has_bias() const { return !no_bias.defined(); }
+    const float *weight() const { return static_cast<const float *>(w.ptr()); }
+    const float *bias() const { return has_bias() ? static_cast<const float *>(b.ptr()) : fptr(no_bias); }
 };
 constexpr int kMaxSlots = 11;
 struct Plan {
@@ -170,9 +198,9 @@ void plan_dealloc(PyObject *o)
     reinterpret_cast<PlanObject *>(o)->plan.~shared_ptr();
     Py_TYPE(o)->tp_free(o);
 }
-PyObject *plan_reduce(PyObject *o, PyObject *)      // copies and pickles start empty
+PyObject *plan_reduce(PyObject *, PyObject *)       // copies and pickles hold None in its place
 {
-    return Py_BuildValue("O()", reinterpret_cast<PyObject *>(Py_TYPE(o)));
+    return Py_BuildValue("O()", reinterpret_cast<PyObject *>(Py_TYPE(Py_None)));
 }
 PyMethodDef plan_methods[] = {{"__reduce__", plan_reduce, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
@@ -181,7 +209,8 @@ PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 enum { A_THR, A_CB, W_PACKED, W_CB, W_CENTER, W_SCALE, W_SUM, W_BIAS, P_TABLE, P_CODES, P_DENSE };
 enum class Kind { OnTheFly, Packed, Conv };
 
-std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, PyObject *&dict)
+// `refs` takes the module and its buffers for the length of the call: the plan itself does not keep them.
+std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, Refs &refs, PyObject *&dict)
 {
     dict = dict_of(module);
     PyObject *buffers = get(dict, S._buffers);
@@ -197,9 +226,12 @@ std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, PyObject *&dict)
     const int n = kind == Kind::Packed ? 11 : 8;
     const Tensor *t[kMaxSlots];
     bool same = plan != nullptr;
+    refs.add(module);
     for (int i = 0; i < n; ++i) {
-        t[i] = as_tensor(get(buffers, names[i]));
+        PyObject *o = get(buffers, names[i]);
+        t[i] = as_tensor(o);
         if (!t[i]) return nullptr;
+        refs.add(o);
         same = same && plan->slot[i].same(*t[i]);
     }
     if (same) return plan;
@@ -221,7 +253,7 @@ std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, PyObject *&dict)
     if (!get_int(dict, S.bits, plan->bits) || !get_int(dict, S.group_size, plan->gs)) return nullptr;
     for (int i = 0; i < n; ++i) {
         plan->slot[i].set(*t[i], i != W_PACKED && i != P_CODES && i != P_DENSE);
-        plan->p[i] = t[i]->numel() ? plan->slot[i].use.const_data_ptr() : nullptr;
+        plan->p[i] = t[i]->numel() ? plan->slot[i].ptr() : nullptr;
     }
     plan->device = dev.index();
     PlanObject *fresh = reinterpret_cast<PlanObject *>(plan_new(&PlanType, nullptr, nullptr));
@@ -235,7 +267,7 @@ std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, PyObject *&dict)
 }
 
 // fp32 copies of a LayerNorm's weight and bias (made once per layer and parameter version); nullopt: not the plain case.
-std::optional<LayerNormParams> layernorm_params(Plan &plan, PyObject *ln, float &eps)
+std::optional<LayerNormParams> layernorm_params(Plan &plan, PyObject *ln, Refs &refs, float &eps)
 {
     PyObject *d = dict_of(ln);
     PyObject *params = get(d, S._parameters);
@@ -245,17 +277,18 @@ std::optional<LayerNormParams> layernorm_params(Plan &plan, PyObject *ln, float 
     const Tensor *b = as_tensor(bo);
     if (!w || !e || !PyFloat_Check(e) || !shape || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != 1) return std::nullopt;
     if (!b && bo != Py_None) return std::nullopt;
+    refs.add(get(params, S.weight));
+    refs.add(bo);
     eps = static_cast<float>(PyFloat_AS_DOUBLE(e));
     for (auto &p : plan.ln)
-        if (p.w.same(*w) && p.has_bias == (b != nullptr) && (!b || p.b.same(*b))) return p;
+        if (p.w.same(*w) && p.has_bias() == (b != nullptr) && (!b || p.b.same(*b))) return p;
     if (!w->is_cuda() || w->device().index() != plan.device || w->numel() != plan.K || w->dim() != 1) return std::nullopt;
     if (b && (b->device() != w->device() || b->numel() != plan.K)) return std::nullopt;
     if (plan.ln.size() >= 4) plan.ln.clear();        // (a layer has one LayerNorm in front of it; a bound, not a policy)
     LayerNormParams p;
     p.w.set(*w, true);
-    p.has_bias = b != nullptr;
     if (b) p.b.set(*b, true);
-    else p.b.use = at::zeros_like(p.w.use);
+    else p.no_bias = at::zeros({plan.K}, w->options().dtype(at::kFloat).requires_grad(false));
     plan.ln.push_back(p);
     return p;
 }
@@ -305,7 +338,7 @@ void run_prepare(const Tensor &x, int64_t rows, const Plan &first, const LayerNo
     a.fp8 = w_first.fp8 ? 1 : 0;
     a.rows = rows, a.K = first.K;
     a.x = x.const_data_ptr();
-    if (ln) a.ln_weight = fptr(ln->w.use), a.ln_bias = fptr(ln->b.use), a.ln_eps = ln_eps;
+    if (ln) a.ln_weight = ln->weight(), a.ln_bias = ln->bias(), a.ln_eps = ln_eps;
     a.thresholds = static_cast<const float *>(first.p[A_THR]), a.codebook = static_cast<const float *>(first.p[A_CB]);
     a.x_hat = x_hat;
     if (w_first.ptr) set_weights(a.weights[0], first, w_first);
@@ -348,14 +381,12 @@ bool prepare_pays(const Plan &p, int64_t rows, bool f16_input, bool has_ws, bool
 }
 
 // The power of two inside a layer's FP8 weights (reads the metadata back to the host: once per layer and set of buffers).
-void find_fp8_multiplier(Plan &p)
+void find_fp8_multiplier(Plan &p, PyObject *dict)
 {
     if (!std::isnan(p.fp8_mult)) return;
-    PyObject *args[4];
-    const int slots[4] = {W_CB, W_CENTER, W_SCALE, W_SUM};
-    for (int i = 0; i < 4; ++i) args[i] = THPVariable_Wrap(p.slot[slots[i]].use);
-    PyObject *r = PyObject_CallFunctionObjArgs(g_fp8_multiplier, args[0], args[1], args[2], args[3], nullptr);
-    for (PyObject *a : args) Py_DECREF(a);
+    PyObject *b = get(dict, S._buffers);
+    PyObject *r = PyObject_CallFunctionObjArgs(g_fp8_multiplier, get(b, S.weight_codebook), get(b, S.weight_center), get(b, S.weight_scale),
+                                               get(b, S.weight_code_sum), nullptr);
     if (!r) throw Failure{};
     p.fp8_mult = PyFloat_AsDouble(r);
     Py_DECREF(r);
@@ -364,8 +395,9 @@ void find_fp8_multiplier(Plan &p)
 
 std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Options &o)
 {
+    Refs refs;
     PyObject *dict;
-    const auto plan = plan_of(module, Kind::OnTheFly, dict);
+    const auto plan = plan_of(module, Kind::OnTheFly, refs, dict);
     if (!plan || !here(x) || x.device().index() != plan->device || !x.is_contiguous() || (!f16(x) && !f32(x)) || x.dim() < 1 ||
         x.size(-1) != plan->K || x.numel() == 0)
         return std::nullopt;
@@ -383,7 +415,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
         if (fp8 || plan->gs != 64 || K % 64 != 0) return std::nullopt;
         if (o.layernorm) {
             if (K > 1024 && (K > 1536 || m >= 512)) return std::nullopt;
-            ln = layernorm_params(*plan, o.layernorm, ln_eps);
+            ln = layernorm_params(*plan, o.layernorm, refs, ln_eps);
             if (!ln) return std::nullopt;
         }
         if (o.x_is_xhat && (!f16(x) || o.layernorm)) return std::nullopt;
@@ -394,7 +426,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
     std::shared_ptr<Plan> next;
     if (o.next) {
         PyObject *nd;
-        next = plan_of(o.next, Kind::OnTheFly, nd);
+        next = plan_of(o.next, Kind::OnTheFly, refs, nd);
         if (!next || next->device != plan->device || !can_quantize(dict, *plan, nd, *next, m)) return std::nullopt;
     }
     at::DimVector sizes(x.sizes());
@@ -404,7 +436,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
     auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
     if (fp8) {
         if (plan->gs != 64) return std::nullopt;
-        find_fp8_multiplier(*plan);
+        find_fp8_multiplier(*plan, dict);
         const int64_t kp = (K + 127) / 128 * 128;
         Tensor x8 = empty({m * kp}, at::kByte, x.device()), w8 = empty({N * kp}, at::kByte, x.device());
         Tensor y = empty(sizes, out_type, x.device());
@@ -458,7 +490,7 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
     a.x = x.const_data_ptr();
     if (ln) {
         a.producer = ARCQ_PRODUCER_LAYERNORM;
-        a.ln_weight = fptr(ln->w.use), a.ln_bias = fptr(ln->b.use), a.ln_eps = ln_eps;
+        a.ln_weight = ln->weight(), a.ln_bias = ln->bias(), a.ln_eps = ln_eps;
     }
     if (o.x_is_xhat) a.producer = ARCQ_PRODUCER_XHAT;
     a.activation = o.gelu ? ARCQ_ACT_GELU : ARCQ_ACT_NONE;
@@ -545,7 +577,7 @@ Tensor layernorm_op(PyObject *d, const Tensor &x, bool &ok)      // an nn.LayerN
 //                   quantizers does not forgive another order of summation (one changed bit is 10 % of the logits 12 blocks on)
 //   attention that the library's kernel does not run (or is not to): torch's, then stage 1 of proj as a launch of its own
 std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t heads, bool own, Plan &pq, Plan &pp, Plan &pf1, Plan &pf2,
-                                     PyObject *n1, PyObject *n2, bool fused, bool fp8)
+                                     PyObject *n1, PyObject *n2, Refs &refs, bool fused, bool fp8)
 {
     const int64_t b = x.size(0), n = x.size(1), C = x.size(2);
     const bool fuse_ln = fused && !fp8;
@@ -561,7 +593,7 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
     std::optional<LayerNormParams> l1, l2;
     Tensor t = x;
     if (fuse_ln) {
-        l1 = layernorm_params(pq, n1, e1), l2 = layernorm_params(pf1, n2, e2);
+        l1 = layernorm_params(pq, n1, refs, e1), l2 = layernorm_params(pf1, n2, refs, e2);
         if (!l1 || !l2) return std::nullopt;
     } else {
         bool ok = true;
@@ -619,9 +651,10 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
     int64_t heads;
     if (!get_int(ad, S.num_heads, heads) || heads <= 0) return std::nullopt;
     const bool own = is_true(get(ad, S.own_kernel));
+    Refs refs;
     PyObject *dq, *dp, *df1, *df2;
-    const auto pq = plan_of(qkv, Kind::OnTheFly, dq), pp = plan_of(proj, Kind::OnTheFly, dp), pf1 = plan_of(fc1, Kind::OnTheFly, df1),
-               pf2 = plan_of(fc2, Kind::OnTheFly, df2);
+    const auto pq = plan_of(qkv, Kind::OnTheFly, refs, dq), pp = plan_of(proj, Kind::OnTheFly, refs, dp),
+               pf1 = plan_of(fc1, Kind::OnTheFly, refs, df1), pf2 = plan_of(fc2, Kind::OnTheFly, refs, df2);
     const int64_t c = x.size(2);
     if (!pq || !pp || !pf1 || !pf2 || pq->K != c || pq->N != 3 * c || pp->K != c || pp->N != c || pf1->K != c || pf2->K != pf1->N ||
         pf2->N != c || c % heads != 0)
@@ -636,10 +669,10 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
         for (Plan *p : {pq.get(), pp.get(), pf1.get(), pf2.get()})
             if (p->gs != 64) return std::nullopt;
         if (fp8)
-            for (Plan *p : {pq.get(), pp.get(), pf1.get(), pf2.get()}) find_fp8_multiplier(*p);
+            for (auto [p, l] : {std::pair(pq.get(), dq), {pp.get(), dp}, {pf1.get(), df1}, {pf2.get(), df2}}) find_fp8_multiplier(*p, l);
         const bool chain = is_true(get(d, S.chain_mlp));
         if (chain) {
-            auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, true, fp8);
+            auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, refs, true, fp8);
             if (whole) return whole;
         }
         if (fp8) return std::nullopt;
@@ -671,7 +704,7 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
     for (PyObject *l : {dq, dp, df1, df2})
         plain = plain && !is_true(get(l, S.fp8_operands)) && get(l, S.out_dtype) == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf));
     if (plain) {
-        auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, false, false);
+        auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, refs, false, false);
         if (whole) return whole;
     }
     bool ok = true;
@@ -825,8 +858,9 @@ PyObject *py_packed_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
         const Tensor *xp = n == 2 ? as_tensor(args[1]) : nullptr;
         if (!xp) return none();
         const Tensor &x = *xp;
+        Refs refs;
         PyObject *dict;
-        const auto plan = plan_of(args[0], Kind::Packed, dict);
+        const auto plan = plan_of(args[0], Kind::Packed, refs, dict);
         if (!plan || !here(x) || x.device().index() != plan->device || !f32(x) || !x.is_contiguous() || x.dim() < 1 ||
             x.size(-1) != plan->K || x.numel() == 0)
             return none();
@@ -858,31 +892,30 @@ PyObject *py_packed_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
                                          fp(W_SCALE), fp(W_SUM), fp(W_BIAS), x_hat.mutable_data_ptr(), nullptr,
                                          y.mutable_data_ptr(), ARCQ_F32, m, N, K, bits, 64, stream));
             } else {
-                const Tensor &dense = plan->slot[P_DENSE].use;
-                if (!dense.defined() || !f16(dense) || dense.numel() != N * K) return none();
+                const Slot &dense = plan->slot[P_DENSE];
+                if (dense.type != at::kHalf || dense.numel() != N * K) return none();
                 check(arcq_act_quant_blocked(x.const_data_ptr(), ARCQ_F32, fp(A_THR), fp(A_CB), x_hat.mutable_data_ptr(), m, K, bits,
                                              1.0e-6f, stream));
                 check(arcq_linear_fused_blocked(x_hat.const_data_ptr(), up(W_PACKED), fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM),
-                                                fp(W_BIAS), const_cast<void *>(dense.const_data_ptr()), 1, y.mutable_data_ptr(),
+                                                fp(W_BIAS), const_cast<void *>(dense.ptr()), 1, y.mutable_data_ptr(),
                                                 ARCQ_F32, m, N, K, bits, 64, stream));
             }
             return THPVariable_Wrap(std::move(y));
         }
         const bool bytes = strcmp(fmt, "u8") == 0;
         if (!bytes && strcmp(fmt, "packed") != 0) return none();
-        const Tensor &table = plan->slot[P_TABLE].use;
-        if (!table.defined() || table.dim() != 2 || table.size(0) != table.size(1)) return none();
-        if (plan->slot[A_CB].use.numel() != table.size(0) || plan->slot[W_CB].use.numel() != table.size(0)) return none();
-        if (bytes && (!p[P_CODES] || plan->slot[P_CODES].use.numel() != N * K || plan->slot[P_CODES].use.scalar_type() != at::kByte))
-            return none();
-        const int levels = static_cast<int>(table.size(0));
+        const Slot &table = plan->slot[P_TABLE];
+        if (table.sizes.size() != 2 || table.sizes[0] != table.sizes[1]) return none();
+        if (plan->slot[A_CB].numel() != table.sizes[0] || plan->slot[W_CB].numel() != table.sizes[0]) return none();
+        if (bytes && (!p[P_CODES] || plan->slot[P_CODES].numel() != N * K || plan->slot[P_CODES].type != at::kByte)) return none();
+        const int levels = static_cast<int>(table.sizes[0]);
         const Tensor x2 = x.dim() == 2 ? x : x.view({m, K});
         Quantized q = quantize(x2, fp(A_THR), fp(A_CB), bits, gs, bytes);
         Tensor y = empty(sizes, at::kFloat, x.device());
         arcq_linear_index_args a = {};
         a.x_codes = bptr(q.codes), a.x_center = fptr(q.center), a.x_scale = fptr(q.scale), a.x_code_sum = fptr(q.sum);
         a.w_codes = up(bytes ? P_CODES : W_PACKED), a.w_center = fp(W_CENTER), a.w_scale = fp(W_SCALE), a.w_code_sum = fp(W_SUM);
-        a.product_table = fptr(table), a.a_codebook = fp(A_CB), a.w_codebook = fp(W_CB), a.bias = fp(W_BIAS);
+        a.product_table = fp(P_TABLE), a.a_codebook = fp(A_CB), a.w_codebook = fp(W_CB), a.bias = fp(W_BIAS);
         a.y = static_cast<float *>(y.mutable_data_ptr());
         a.rows = m, a.out_features = N, a.in_features = K;
         a.bits = bytes ? 0 : bits, a.group_size = gs, a.levels = levels;
@@ -898,8 +931,9 @@ PyObject *py_patch_conv_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
         const Tensor *xp = n == 2 ? as_tensor(args[1]) : nullptr;
         if (!xp) return none();
         const Tensor &x = *xp;
+        Refs refs;
         PyObject *dict;
-        const auto plan = plan_of(args[0], Kind::Conv, dict);
+        const auto plan = plan_of(args[0], Kind::Conv, refs, dict);
         int64_t ags, c;
         PyObject *ks = get(dict, S.kernel_size);
         if (!plan || plan->gs != 64 || !get_int(dict, S.act_group_size, ags) || ags != 3 || !get_int(dict, S.in_channels, c) || c != 3 ||

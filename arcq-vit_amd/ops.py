@@ -553,6 +553,7 @@ def fp8_weight_multiplier(w_codebook: torch.Tensor, w_center: torch.Tensor, w_sc
     """Power of two that moves a layer's reconstructed weights into FP8's normal range: the largest one that keeps a
     bound on ``|w_hat|`` (``|center| + |scale| (max |cb| + |code_sum| / 64)`` over all groups) at or below half the
     largest FP8 value.  Reads the metadata back to the host: compute it once per layer."""
+    w_codebook, w_center, w_scale, w_code_sum = (t.detach().float() for t in (w_codebook, w_center, w_scale, w_code_sum))
     cb = float(w_codebook.abs().max())
     bound = float((w_center.abs() + w_scale.abs() * (cb + w_code_sum.abs() / 64.0)).max())
     if not bound > 0.0:

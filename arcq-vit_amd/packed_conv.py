@@ -130,6 +130,7 @@ class ARCQPackedPatchConv(nn.Module):
     def _apply(self, fn, *args, **kwargs):
         # model.half() must not narrow the fp32 metadata; device moves still apply.
         keep = {n: self._buffers[n] for n in self._FP32_BUFFERS if self._buffers.get(n) is not None}
+        self._host_plan = None          # the host extension's view of the buffers, and the copies it holds where they were
         super()._apply(fn, *args, **kwargs)
         for name, orig in keep.items():
             new = self._buffers[name]

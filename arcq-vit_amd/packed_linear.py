@@ -207,6 +207,10 @@ class ARCQPackedLinear(nn.Module):
         return self
 
     # -- nn.Module API --------------------------------------------------------------------
+    def _apply(self, fn, *args, **kwargs):
+        self._host_plan = None      # the host extension's view of the buffers, and the copies it holds where they were
+        return super()._apply(fn, *args, **kwargs)
+
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, "
                 f"bits={self.bits}, group_size={self.group_size}, "

@@ -94,12 +94,17 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         # then widens these buffers again, scripts/benchmark_arcq_on_the_fly.py:63-85, which leaves
         # them rounded to fp16.)  Device moves still apply; dtype changes of these buffers do not.
         keep = {n: self._buffers[n] for n in self._FP32_BUFFERS if self._buffers.get(n) is not None}
+        self._host_plan = None          # and with it the copies it holds where they were
         super()._apply(fn, *args, **kwargs)
         for name, orig in keep.items():
             new = self._buffers[name]
             if new.dtype != orig.dtype:
                 self._buffers[name] = orig.to(device=new.device)
         return self
+
+    def _load_from_state_dict(self, *args, **kwargs):
+        self._host_plan = None
+        return super()._load_from_state_dict(*args, **kwargs)
 
     def can_quantize_for(self, consumer: nn.Module, rows: int) -> bool:
         """Whether ``forward(..., quantize_for=consumer)`` is available: this layer's launch then ends with the

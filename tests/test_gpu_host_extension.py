@@ -151,3 +151,73 @@ def test_replicas_on_threads_and_streams(cuda):
     for t in threads:
         t.join()
     assert not failures
+
+
+@pytest.mark.parametrize("kind", ["packed", "dequant_gemm", "on_the_fly", "conv"])
+def test_a_module_that_moves_away_leaves_no_memory_behind(cuda, kind):
+    """Neither the buffers nor the fp32 copies of those that are not fp32 outlive `.cpu()` in the extension's plan."""
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    if kind == "conv":
+        src = A.QuantConv2dPCARCQ(3, 4096, 16, 16, 0, True, 4, 4, 64)
+        for q in (src.act_quant, src.weight_quant):
+            q.set_codebook(synth.quantile_codebook(4))
+        module, x = A.ARCQPackedPatchConv(src).cuda(), synth.make_images(1, 1).cuda()
+    else:
+        module = _on_the_fly(4096, 4096) if kind == "on_the_fly" else _packed(4096, 4096, kind)
+        x = _tokens(600, 4096, dtype=torch.float32)
+    module.weight_scale = module.weight_scale.half()                       # needs an fp32 copy
+    with torch.no_grad():
+        module(x)
+    assert module._host_plan is not None
+    module.cpu()
+    del x
+    assert torch.cuda.memory_allocated() - before < 1 << 16
+
+
+def test_a_replaced_buffer_is_not_kept(cuda):
+    layer, x = _packed(4096, 4096, "dequant_gemm"), _tokens(600, 4096, dtype=torch.float32)
+    with torch.no_grad():
+        want = layer(x)
+        before = torch.cuda.memory_allocated()
+        layer.weight_dequant = layer.weight_dequant.clone()
+        assert torch.cuda.memory_allocated() - before < 1 << 16
+        assert torch.equal(layer(x), want)
+
+
+def test_views_of_a_buffer_are_other_buffers(cuda):
+    """The same memory under other sizes or strides: the copies made from it are made again."""
+    layer, x = _on_the_fly(192, 192), _tokens(197, 192)
+    with torch.no_grad():
+        square = torch.rand(192, 192, device=cuda) * 0.02
+        layer.weight_scale = square[:, :3]
+        a = layer(x)
+        layer.weight_scale = square.t()[:, :3]
+        b = layer(x)
+        layer.weight_scale = square[:, :3].contiguous()
+        assert torch.equal(layer(x), a)
+        layer.weight_scale = square.t()[:, :3].contiguous()
+        assert torch.equal(layer(x), b) and not torch.equal(a, b)
+
+
+def test_parameters_may_be_swapped(cuda):
+    """`torch.__future__.set_swap_module_params_on_conversion` refuses tensors that something else refers to."""
+    block, x = _vit(fuse_elementwise=True).blocks[0], _tokens(2, 197, 192)
+    with torch.no_grad():
+        want = block(x)
+    torch.__future__.set_swap_module_params_on_conversion(True)
+    try:
+        block.cpu().cuda()
+    finally:
+        torch.__future__.set_swap_module_params_on_conversion(False)
+    with torch.no_grad():
+        assert torch.equal(block(x), want)
+
+
+def test_modules_with_a_plan_pickle_without_it(cuda, tmp_path):
+    layer, x = _on_the_fly(192, 768), _tokens(197, 192)
+    with torch.no_grad():
+        want = layer(x)
+        torch.save(layer, tmp_path / "layer.pt")
+        again = torch.load(tmp_path / "layer.pt", weights_only=False)
+        assert again._host_plan is None and torch.equal(again(x), want)
