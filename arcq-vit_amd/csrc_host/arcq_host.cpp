@@ -94,11 +94,9 @@ inline bool get_int(PyObject *dict, PyObject *key, int64_t &out)
 }
 inline const Tensor *as_tensor(PyObject *o) { return o && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
 
-inline uint32_t version_of(const Tensor &t)
-{
-    const auto &vc = t.unsafeGetTensorImpl()->version_counter();
-    return vc.enabled() ? vc.current_version() : 0;
-}
+// Inference tensors have no version: a change in place leaves no trace on them, and nothing derived from one is kept.
+inline bool has_version(const Tensor &t) { return t.unsafeGetTensorImpl()->version_counter().enabled(); }
+inline uint32_t version_of(const Tensor &t) { return has_version(t) ? t.unsafeGetTensorImpl()->version_counter().current_version() : 0; }
 inline Tensor empty(at::IntArrayRef sizes, at::ScalarType type, c10::Device device)
 {
     return Tensor(at::detail::empty_cuda(sizes, type, device, std::nullopt));
@@ -124,6 +122,7 @@ inline const uint8_t *bptr(const Tensor &t) { return static_cast<const uint8_t *
 struct Slot {
     std::optional<c10::weak_intrusive_ptr<c10::StorageImpl>> storage;
     Tensor copy;              // fp32 / contiguous, where the tensor is not
+    bool tracked = true;      // changes in place show in its version
     uint32_t version = 0;
     const void *data = nullptr;
     at::ScalarType type = at::kByte;
@@ -132,11 +131,12 @@ struct Slot {
     {
         return storage && storage->_unsafe_get_target() == t.unsafeGetTensorImpl()->unsafe_storage().unsafeGetStorageImpl() &&
                version == version_of(t) && data == t.const_data_ptr() && type == t.scalar_type() && t.sizes().equals(sizes) &&
-               t.strides().equals(strides);
+               t.strides().equals(strides) && tracked == has_version(t) && (tracked || !copy.defined());
     }
     void set(const Tensor &t, bool as_f32)
     {
         storage.emplace(t.storage().getWeakStorageImpl());
+        tracked = has_version(t);
         version = version_of(t);
         data = t.const_data_ptr();
         type = t.scalar_type();
@@ -383,7 +383,8 @@ bool prepare_pays(const Plan &p, int64_t rows, bool f16_input, bool has_ws, bool
 // The power of two inside a layer's FP8 weights (reads the metadata back to the host: once per layer and set of buffers).
 void find_fp8_multiplier(Plan &p, PyObject *dict)
 {
-    if (!std::isnan(p.fp8_mult)) return;
+    const bool tracked = p.slot[W_CB].tracked && p.slot[W_CENTER].tracked && p.slot[W_SCALE].tracked && p.slot[W_SUM].tracked;
+    if (tracked && !std::isnan(p.fp8_mult)) return;
     PyObject *b = get(dict, S._buffers);
     PyObject *r = PyObject_CallFunctionObjArgs(g_fp8_multiplier, get(b, S.weight_codebook), get(b, S.weight_center), get(b, S.weight_scale),
                                                get(b, S.weight_code_sum), nullptr);

@@ -221,3 +221,33 @@ def test_modules_with_a_plan_pickle_without_it(cuda, tmp_path):
         torch.save(layer, tmp_path / "layer.pt")
         again = torch.load(tmp_path / "layer.pt", weights_only=False)
         assert again._host_plan is None and torch.equal(again(x), want)
+
+
+def test_inference_tensors_changed_in_place(cuda):
+    """Tensors made under inference_mode carry no version: what a layer derives from its own and from a LayerNorm's (fp32
+    copies, the FP8 multiplier) follows a change in place all the same."""
+    x, xl = _tokens(197, 192), _tokens(600, 192)
+    with torch.inference_mode():
+        layer, norm = _on_the_fly(192, 768), torch.nn.LayerNorm(192).cuda().half()
+        layer.weight_scale = layer.weight_scale.half()
+        assert layer.weight_scale.is_inference() and norm.weight.is_inference()
+
+        def results():
+            layer.fp8_operands = True
+            f8 = layer(xl)
+            layer.fp8_operands = False
+            return layer(x), layer(x, layernorm=norm), f8
+
+        before = results()
+        layer.weight_scale.mul_(1024)
+        layer.weight_center.mul_(1024)
+        norm.weight.mul_(2)
+        norm.bias.add_(0.5)
+        after = results()
+        layer, weight, bias = _on_the_fly(192, 768), norm.weight, norm.bias
+        layer.weight_scale = layer.weight_scale.half() * 1024
+        layer.weight_center = layer.weight_center * 1024
+        norm = torch.nn.LayerNorm(192).cuda().half()
+        norm.load_state_dict({"weight": weight, "bias": bias})
+        assert all(torch.equal(a, b) for a, b in zip(after, results()))
+        assert not any(torch.equal(a, b) for a, b in zip(after, before))
