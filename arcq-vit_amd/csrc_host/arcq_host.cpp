@@ -37,7 +37,7 @@ using at::Tensor;
 // ---- names --------------------------------------------------------------------------------------------------------
 #define ARCQ_NAMES(X)                                                                                                     \
     X(_buffers) X(_modules) X(_parameters) X(_host_plan) X(_weight_buffer) X(_x_hat_buffer) X(out_dtype) X(fp8_operands) \
-    X(in_features) X(out_features) X(bits) X(group_size) X(act_group_size) X(in_channels) X(kernel_size)                  \
+    X(in_features) X(out_features) X(bits) X(group_size) X(act_group_size) X(in_channels) X(out_channels) X(kernel_size)                  \
     X(packed_weight_codes) X(weight_codebook) X(weight_center)                                                            \
     X(weight_scale) X(weight_code_sum) X(activation_codebook) X(activation_thresholds) X(bias_tensor) X(bias)             \
     X(product_table) X(weight_codes_u8) X(weight_dequant) X(runtime_code_format)                                          \
@@ -209,6 +209,19 @@ PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 enum { A_THR, A_CB, W_PACKED, W_CB, W_CENTER, W_SCALE, W_SUM, W_BIAS, P_TABLE, P_CODES, P_DENSE };
 enum class Kind { OnTheFly, Packed, Conv };
 
+// Whether the buffers hold what the kernels will read for the layer's sizes: a buffer may have been replaced since the module
+// checked them.  `indexed`: the index-space formats, whose quantizer takes no other length of a codebook.
+bool shapes_ok(const Plan &p, const Tensor *const *t, bool indexed)
+{
+    if (p.bits < 2 || p.bits > 4 || p.gs <= 0 || p.K <= 0 || p.N <= 0 || p.K % p.gs != 0) return false;
+    const int64_t levels = int64_t(1) << p.bits, meta = p.N * (p.K / p.gs);
+    if (t[W_PACKED]->dim() != 2 || t[W_PACKED]->size(0) != p.N || t[W_PACKED]->size(1) != (p.K * p.bits + 7) / 8) return false;
+    if (t[A_CB]->numel() < levels || t[W_CB]->numel() < levels || t[A_THR]->numel() < levels - 1) return false;
+    if (indexed && (t[A_CB]->numel() != levels || t[A_THR]->numel() != levels - 1)) return false;
+    for (int i : {W_CENTER, W_SCALE, W_SUM})
+        if (t[i]->numel() < meta) return false;
+    return t[W_BIAS]->numel() == 0 || t[W_BIAS]->numel() >= p.N;
+}
 // `refs` takes the module and its buffers for the length of the call: the plan itself does not keep them.
 std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, Refs &refs, PyObject *&dict)
 {
@@ -243,14 +256,14 @@ std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, Refs &refs, PyObject 
     }
     if (!t[W_PACKED]->is_cuda() || t[W_PACKED]->scalar_type() != at::kByte) return nullptr;
     if (kind == Kind::Conv) {
-        int64_t c;
-        if (!get_int(dict, S.in_channels, c)) return nullptr;
-        plan->N = t[W_PACKED]->size(0);
+        int64_t c;                       // (the call below serves 16 x 16 patches only)
+        if (!get_int(dict, S.in_channels, c) || !get_int(dict, S.out_channels, plan->N)) return nullptr;
         plan->K = 256 * c;
     } else if (!get_int(dict, S.in_features, plan->K) || !get_int(dict, S.out_features, plan->N)) {
         return nullptr;
     }
     if (!get_int(dict, S.bits, plan->bits) || !get_int(dict, S.group_size, plan->gs)) return nullptr;
+    if (!shapes_ok(*plan, t, kind == Kind::Packed)) return nullptr;
     for (int i = 0; i < n; ++i) {
         plan->slot[i].set(*t[i], i != W_PACKED && i != P_CODES && i != P_DENSE);
         plan->p[i] = t[i]->numel() ? plan->slot[i].ptr() : nullptr;

@@ -51,6 +51,22 @@ def _f32c(t: torch.Tensor) -> torch.Tensor:
     return t.to(torch.float32).contiguous()
 
 
+def _check_weights(n: int, k: int, group_size: int, center: torch.Tensor, scale: torch.Tensor, code_sum: torch.Tensor,
+                   bias: Optional[torch.Tensor]) -> None:
+    """The per-group metadata and the bias hold at least what the kernels read for ``[n, k]`` weights."""
+    need = n * (k // max(int(group_size), 1))
+    for name, t in (("w_center", center), ("w_scale", scale), ("w_code_sum", code_sum)):
+        _check(t.numel() >= need, f"{name} has {t.numel()} entries, {need} needed for [out_features, groups]")
+    _check(bias is None or bias.numel() == 0 or bias.numel() >= n, "bias must have out_features entries")
+
+
+def _check_codebooks(bits: int, w_codebook: Optional[torch.Tensor], a_thresholds: Optional[torch.Tensor] = None,
+                     a_codebook: Optional[torch.Tensor] = None) -> None:
+    for name, t, need in (("w_codebook", w_codebook, 1 << bits), ("a_thresholds", a_thresholds, (1 << bits) - 1),
+                          ("a_codebook", a_codebook, 1 << bits)):
+        _check(t is None or t.numel() >= need, f"{name} must have {need} entries for {bits}-bit codes")
+
+
 # ---------------------------------------------------------------------------------------------
 # bit packing -- EXT/arcq_pack_kernel.cu:94-158
 # ---------------------------------------------------------------------------------------------
@@ -215,6 +231,8 @@ def unpack_weight_hip(packed: torch.Tensor, codebook: torch.Tensor, center: torc
     groups = center.shape[1]
     in_f = groups * int(group_size)
     _check(packed.shape[1] == (in_f * bits + 7) // 8, "packed row length does not match in_features*bits/8")
+    _check_weights(out_f, in_f, group_size, center, scale, code_sum, None)
+    _check_codebooks(bits, codebook)
     packed = packed.contiguous()
     codebook, center, scale, code_sum = _f32c(codebook), _f32c(center), _f32c(scale), _f32c(code_sum)
     if out is None:
@@ -253,6 +271,8 @@ def linear_fused(x_hat: torch.Tensor, packed_w: torch.Tensor, w_codebook: torch.
     m, k = x_hat.shape
     n = packed_w.shape[0]
     _check(packed_w.shape[1] == (k * bits + 7) // 8, "packed_w row length does not match K*bits/8")
+    _check_weights(n, k, group_size, w_center, w_scale, w_code_sum, bias)
+    _check_codebooks(bits, w_codebook)
     y = torch.empty((m, n), dtype=out_dtype, device=x_hat.device)
     b = None if bias is None or bias.numel() == 0 else _f32c(bias)
     w = [packed_w.contiguous(), _f32c(w_codebook), _f32c(w_center), _f32c(w_scale), _f32c(w_code_sum)]
@@ -288,6 +308,8 @@ def linear_otf(x: torch.Tensor, a_thresholds: torch.Tensor, a_codebook: torch.Te
     m, k = x.shape
     n = packed_w.shape[0]
     _check(packed_w.shape[1] == (k * bits + 7) // 8, "packed_w row length does not match K*bits/8")
+    _check_weights(n, k, group_size, w_center, w_scale, w_code_sum, bias)
+    _check_codebooks(bits, w_codebook, a_thresholds, a_codebook)
     if x_hat_ws is None:
         x_hat_ws = torch.empty((m, k), dtype=torch.float16, device=x.device)
     else:
@@ -324,6 +346,7 @@ def quantize_activation_blocked(x: torch.Tensor, thresholds: torch.Tensor, codeb
     x = x.contiguous()
     m, k = x.shape
     _check(k % 64 == 0, "the block layout needs K divisible by 64")
+    _check_codebooks(bits, None, thresholds, codebook)
     if out is None:      # whole blocks: [M/32, K/8, 32, 8]; a ragged last block is stored compactly behind them: flat
         shape = (m // 32, k // 8, 32, 8) if m % 32 == 0 else (m * k,)
         out = torch.empty(shape, dtype=torch.float16, device=x.device)
@@ -341,6 +364,8 @@ def quantize_activation_blocked(x: torch.Tensor, thresholds: torch.Tensor, codeb
             _check(packed_w.is_cuda and packed_w.dtype == torch.uint8 and packed_w.dim() == 2
                    and packed_w.shape[1] == (k * bits + 7) // 8, "packed_w must be uint8 [N, K*bits/8]")
             _check(w_hat is not None, "weights need a w_hat buffer")
+            _check_weights(n, k, 64, *weights[2:], None)
+            _check_codebooks(bits, weights[1])
             _check_w_ws(w_hat, n, k)
             meta = [_f32c(t) for t in weights[1:]]
             _lib.check(_lib.load().arcq_act_quant_blocked_with_weights(
@@ -360,6 +385,7 @@ def quantize_activation_blocked_ln(x: torch.Tensor, ln_weight: torch.Tensor, ln_
     x = x.contiguous()
     m, k = x.shape
     _check(k % 64 == 0 and 64 <= k <= 1024, "the fused LayerNorm needs K divisible by 64 and at most 1024")
+    _check_codebooks(bits, None, thresholds, codebook)
     if out is None:
         shape = (m // 32, k // 8, 32, 8) if m % 32 == 0 else (m * k,)
         out = torch.empty(shape, dtype=torch.float16, device=x.device)
@@ -373,7 +399,11 @@ def quantize_activation_blocked_ln(x: torch.Tensor, ln_weight: torch.Tensor, ln_
     if weights is not None:
         packed_w = weights[0].contiguous()
         n = packed_w.shape[0]
+        _check(packed_w.is_cuda and packed_w.dtype == torch.uint8 and packed_w.dim() == 2
+               and packed_w.shape[1] == (k * bits + 7) // 8, "packed_w must be uint8 [N, K*bits/8]")
         _check(w_hat is not None, "weights need a w_hat buffer")
+        _check_weights(n, k, 64, *weights[2:], None)
+        _check_codebooks(bits, weights[1])
         _check_w_ws(w_hat, n, k)
         keep = [packed_w] + [_f32c(t) for t in weights[1:]]
         wp = [_ptr(t) for t in keep] + [_ptr(w_hat), n]
@@ -394,6 +424,7 @@ def quantize_patches(img: torch.Tensor, thresholds: torch.Tensor, codebook: torc
     _check_bits(bits)
     b, _, h, w = img.shape
     _check(h % 16 == 0 and w % 16 == 0, "image sides must be multiples of 16")
+    _check_codebooks(bits, None, thresholds, codebook)
     img = img.contiguous()
     m = b * (h // 16) * (w // 16)
     out = torch.empty(m * 768 if blocked else (m, 768), dtype=torch.float16, device=img.device)
@@ -486,6 +517,8 @@ def linear_otf_ex(x: torch.Tensor, a_thresholds: torch.Tensor, a_codebook: torch
     m, k = x.shape
     n = packed_w.shape[0]
     _check(packed_w.shape[1] == (k * bits + 7) // 8, "packed_w row length does not match K*bits/8")
+    _check_weights(n, k, group_size, w_center, w_scale, w_code_sum, bias)
+    _check_codebooks(bits, w_codebook, a_thresholds, a_codebook)
     if x_hat_ws is None:
         x_hat_ws = torch.empty(m * k, dtype=torch.float16, device=x.device)
     y = torch.empty((m, n), dtype=out_dtype, device=x.device)
@@ -534,6 +567,7 @@ def quantize_activation_fp8(x: torch.Tensor, thresholds: torch.Tensor, codebook:
     group size 64.  Codes, ``mu`` and ``s`` are those of ``quantize_activation``."""
     _check(x.is_cuda and x.dim() == 2, "x must be a CUDA tensor of shape [M, K]")
     _check_bits(bits)
+    _check_codebooks(bits, None, thresholds, codebook)
     x = x.contiguous()
     m, k = x.shape
     if out is None:
@@ -570,6 +604,8 @@ def unpack_weight_fp8(packed: torch.Tensor, codebook: torch.Tensor, center: torc
     n = packed.shape[0]
     k = center.shape[1] * 64
     _check(packed.shape[1] == (k * bits + 7) // 8, "packed row length does not match in_features*bits/8")
+    _check_weights(n, k, 64, center, scale, code_sum, None)
+    _check_codebooks(bits, codebook)
     if out is None:
         out = torch.empty((n, k), dtype=torch.float8_e4m3fn, device=packed.device)
     else:
@@ -606,6 +642,8 @@ def linear_otf_fp8(x: torch.Tensor, a_thresholds: torch.Tensor, a_codebook: torc
     n = packed_w.shape[0]
     _check(k % 64 == 0 and k > 0, "in_features must be a positive multiple of the group size 64")
     _check(packed_w.shape[1] == (k * bits + 7) // 8, "packed_w row length does not match K*bits/8")
+    _check_weights(n, k, 64, w_center, w_scale, w_code_sum, bias)
+    _check_codebooks(bits, w_codebook, a_thresholds, a_codebook)
     if w_mult is None:
         w_mult = fp8_weight_multiplier(w_codebook, w_center, w_scale, w_code_sum)
     kp = fp8_padded_k(k)
@@ -666,6 +704,8 @@ def linear_fused_blocked(x_hat_blocked: torch.Tensor, m: int, k: int, packed_w: 
     _check_bits(bits)
     n = packed_w.shape[0]
     _check(packed_w.shape[1] == (k * bits + 7) // 8, "packed_w row length does not match K*bits/8")
+    _check_weights(n, k, 64, w_center, w_scale, w_code_sum, bias)
+    _check_codebooks(bits, w_codebook)
     y = torch.empty((m, n), dtype=out_dtype, device=x_hat_blocked.device)
     b = None if bias is None or bias.numel() == 0 else _f32c(bias)
     w = [packed_w.contiguous(), _f32c(w_codebook), _f32c(w_center), _f32c(w_scale), _f32c(w_code_sum)]
@@ -680,6 +720,14 @@ def linear_fused_blocked(x_hat_blocked: torch.Tensor, m: int, k: int, packed_w: 
 # ---------------------------------------------------------------------------------------------
 # index-space linears -- EXT/arcq_linear_kernel.cu:206-353
 # ---------------------------------------------------------------------------------------------
+def _check_index(rows: int, out_features: int, in_features: int, group_size: int, x_center, x_scale, x_code_sum, w_center,
+                 w_scale, w_code_sum, product_table, bias) -> None:
+    _check_weights(out_features, in_features, group_size, w_center, w_scale, w_code_sum, bias)
+    need = rows * (in_features // int(group_size))
+    _check(all(t.numel() >= need for t in (x_center, x_scale, x_code_sum)), "x_center, x_scale and x_code_sum must be [rows, groups]")
+    _check(product_table.dim() == 2 and product_table.shape[0] == product_table.shape[1], "product_table must be square")
+
+
 def arcq_linear_forward(packed_x: torch.Tensor, x_center: torch.Tensor, x_scale: torch.Tensor,
                         x_code_sum: torch.Tensor, packed_w: torch.Tensor, w_center: torch.Tensor,
                         w_scale: torch.Tensor, w_code_sum: torch.Tensor, product_table: torch.Tensor,
@@ -697,6 +745,8 @@ def arcq_linear_forward(packed_x: torch.Tensor, x_center: torch.Tensor, x_scale:
     _check(packed_x.dim() == 2 and packed_x.shape[1] == pc, "packed_x row length does not match in_features*bits/8")
     _check(packed_w.dim() == 2 and packed_w.shape == (int(out_features), pc),
            "packed_w shape does not match [out_features, in_features*bits/8]")
+    _check_index(packed_x.shape[0], int(out_features), int(in_features), group_size, x_center, x_scale, x_code_sum, w_center, w_scale,
+                 w_code_sum, product_table, bias)
     rows = packed_x.shape[0]
     levels = product_table.shape[0]
     y = torch.empty((rows, int(out_features)), dtype=torch.float32, device=packed_x.device)
@@ -729,6 +779,8 @@ def arcq_linear_forward_u8(x_codes: torch.Tensor, x_center: torch.Tensor, x_scal
     _check(product_table.dtype == torch.float32, "product_table must be float32")
     rows, in_features = x_codes.shape
     out_features = w_codes.shape[0]
+    _check_index(rows, out_features, in_features, group_size, x_center, x_scale, x_code_sum, w_center, w_scale, w_code_sum,
+                 product_table, bias)
     levels = product_table.shape[0]
     y = torch.empty((rows, out_features), dtype=torch.float32, device=x_codes.device)
     b = None

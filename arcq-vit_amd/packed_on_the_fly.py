@@ -198,7 +198,8 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         with torch.cuda.device(x2.device):
             y = _lib.host().layer_forward(self, x2, layernorm, activation == "gelu", residual, quantize_for, input_is_xhat)
         if y is None:
-            raise RuntimeError("x and the layer's buffers must be contiguous CUDA tensors of the types the layer was built with")
+            raise RuntimeError("x and the layer's buffers must be contiguous CUDA tensors of the types and shapes the layer was "
+                               "built with")
         return y.reshape(*original_shape[:-1], self.out_features)
 
     def estimated_persistent_mb(self) -> float:

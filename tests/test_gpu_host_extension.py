@@ -251,3 +251,36 @@ def test_inference_tensors_changed_in_place(cuda):
         norm.load_state_dict({"weight": weight, "bias": bias})
         assert all(torch.equal(a, b) for a, b in zip(after, results()))
         assert not any(torch.equal(a, b) for a, b in zip(after, before))
+
+
+def _cut(t):
+    return t[:-1].contiguous()
+
+
+@pytest.mark.parametrize("fmt", ["packed", "u8", "dequant_gemm", "hip_fused", "on_the_fly", "conv"])
+def test_buffers_replaced_by_smaller_ones_are_refused(cuda, fmt):
+    """The kernels read what the layer's sizes say; a buffer that holds less is refused before anything is launched."""
+    if fmt == "conv":
+        src = A.QuantConv2dPCARCQ(3, 64, 16, 16, 0, True, 4, 4, 64)
+        for q in (src.act_quant, src.weight_quant):
+            q.set_codebook(synth.quantile_codebook(4))
+        layer, inputs = A.ARCQPackedPatchConv(src).cuda(), [synth.make_images(b, 1).cuda() for b in (1, 4)]
+    else:
+        layer = _on_the_fly(768, 256) if fmt == "on_the_fly" else _packed(768, 256, fmt)
+        inputs = [_tokens(m, 768, dtype=torch.float32) for m in (7, 600)]
+    index = fmt in ("packed", "u8")
+    names = ["packed_weight_codes" if fmt != "u8" else "weight_codes_u8", "weight_center", "weight_scale", "weight_code_sum",
+             "activation_codebook", "activation_thresholds", "bias_tensor" if fmt == "on_the_fly" else "bias",
+             "product_table" if index else "weight_codebook"] + (["weight_dequant"] if fmt == "dequant_gemm" else [])
+    for x in inputs:
+        with torch.no_grad():
+            want = layer(x)
+            for name in names:
+                good = layer._buffers[name]
+                bad = [_cut(good)] + ([good[:, :-1].contiguous()] if good.dim() == 2 else [])
+                for b in bad:
+                    layer._buffers[name] = b
+                    with pytest.raises(RuntimeError):
+                        layer(x)
+                layer._buffers[name] = good
+                assert torch.equal(layer(x), want)
