@@ -113,6 +113,8 @@ inline int code_of(const Tensor &t)
     return f16(t) ? ARCQ_F16 : ARCQ_F32;
 }
 inline Tensor as_operand(const Tensor &t) { return (f16(t) || f32(t) ? t : t.to(at::kHalf)).contiguous(); }
+inline bool aligned16(const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+inline bool aligned16(const Tensor &t) { return aligned16(t.const_data_ptr()); }
 inline const float *fptr(const Tensor &t) { return static_cast<const float *>(t.const_data_ptr()); }
 inline const uint8_t *bptr(const Tensor &t) { return static_cast<const uint8_t *>(t.const_data_ptr()); }
 
@@ -133,7 +135,7 @@ struct Slot {
                version == version_of(t) && data == t.const_data_ptr() && type == t.scalar_type() && t.sizes().equals(sizes) &&
                t.strides().equals(strides) && tracked == has_version(t) && (tracked || !copy.defined());
     }
-    void set(const Tensor &t, bool as_f32)
+    void set(const Tensor &t, bool as_f32, bool align = false)
     {
         storage.emplace(t.storage().getWeakStorageImpl());
         tracked = has_version(t);
@@ -144,6 +146,7 @@ struct Slot {
         strides = t.strides();
         const Tensor use = (as_f32 ? t.detach().to(at::kFloat) : t.detach()).contiguous();
         if (use.const_data_ptr() != data) copy = use;
+        else if (align && !aligned16(data)) copy = use.clone();
     }
     const void *ptr() const { return copy.defined() ? copy.const_data_ptr() : data; }
     int64_t numel() const { return c10::multiply_integers(sizes); }
@@ -299,8 +302,8 @@ std::optional<LayerNormParams> layernorm_params(Plan &plan, PyObject *ln, Refs &
     if (b && (b->device() != w->device() || b->numel() != plan.K)) return std::nullopt;
     if (plan.ln.size() >= 4) plan.ln.clear();        // (a layer has one LayerNorm in front of it; a bound, not a policy)
     LayerNormParams p;
-    p.w.set(*w, true);
-    if (b) p.b.set(*b, true);
+    p.w.set(*w, true, true);
+    if (b) p.b.set(*b, true, true);
     else p.no_bias = at::zeros({plan.K}, w->options().dtype(at::kFloat).requires_grad(false));
     plan.ln.push_back(p);
     return p;
@@ -377,20 +380,21 @@ void run_product(const Plan &p, int64_t rows, const void *x_hat, const Weights &
     a.fp8 = w.fp8 ? 1 : 0, a.w_mult = static_cast<float>(p.fp8_mult);
     check(arcq_linear_prepared(&a, stream));
 }
+// (packed codes that are not 16-byte aligned are left to the kernels and entry points that take them, or say why not)
 bool can_prepare(const Plan &p, int64_t rows)
 {
-    return p.gs == 64 && p.K % 64 == 0 && (p.N % 32 == 0 || rows >= 512) && rows * p.K < (int64_t(1) << 31) && p.N * p.K < (int64_t(1) << 31) &&
+    return aligned16(p.p[W_PACKED]) && p.gs == 64 && p.K % 64 == 0 && (p.N % 32 == 0 || rows >= 512) && rows * p.K < (int64_t(1) << 31) && p.N * p.K < (int64_t(1) << 31) &&
            rows < (int64_t(1) << 26);
 }
 // Whether one layer call runs as prepare + product.  Below 512 rows from K = 768 on (up to 512 inputs the one-launch kernel
 // is 1 us faster: 7.7 against 9.6 us at 197 x 384 x 384; 12.9 against 11.1 at 2 304 x 768, 43 against 16.5 with a LayerNorm
 // at 3 072 x 1 024); above wherever no one-launch kernel would run (1 000 rows: 384 -> 1 152 13.1 -> 12.0 us, 1 024 -> 3 072
 // 32 -> 19, 4 096 -> 1 024 51 -> 32).
-bool prepare_pays(const Plan &p, int64_t rows, bool f16_input, bool has_ws, bool layernorm)
+bool prepare_pays(const Plan &p, const Tensor &x, int64_t rows, bool has_ws, bool layernorm)
 {
-    if (!can_prepare(p, rows) || (layernorm && p.K > 2048)) return false;
+    if (!can_prepare(p, rows) || !aligned16(x) || (layernorm && p.K > 2048)) return false;
     if (rows < 512) return p.K >= 768;
-    return !(f16_input && has_ws && strncmp(arcq_linear_otf_ws_kernel(rows, p.N, p.K, 1), "otf_rows", 8) == 0);
+    return !(f16(x) && has_ws && strncmp(arcq_linear_otf_ws_kernel(rows, p.N, p.K, 1), "otf_rows", 8) == 0);
 }
 
 // The power of two inside a layer's FP8 weights (reads the metadata back to the host: once per layer and set of buffers).
@@ -468,9 +472,9 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
             w_ws->device() != x.device())
             return std::nullopt;
     }
-    if (!next && !o.x_is_xhat && prepare_pays(*plan, m, f16(x), w_ws != nullptr, ln.has_value())) {
+    if (!next && !o.x_is_xhat && prepare_pays(*plan, x, m, w_ws != nullptr, ln.has_value())) {
         // (x_hat and w_hat in one scratch tensor; w_hat first: 512-byte runs stay aligned)
-        const bool lent = w_ws != nullptr;
+        const bool lent = w_ws != nullptr && aligned16(*w_ws);
         Tensor scratch = empty({(lent ? 0 : N * K) + m * K}, at::kHalf, x.device());
         char *base = static_cast<char *>(scratch.mutable_data_ptr());
         const Weights w{lent ? w_ws->mutable_data_ptr() : base, arcq_prepared_row_major(m, N, K) != 0};
@@ -596,7 +600,7 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
     const int64_t b = x.size(0), n = x.size(1), C = x.size(2);
     const bool fuse_ln = fused && !fp8;
     const bool own_attention = own && n <= 256 && C == 64 * heads;
-    if ((fuse_ln && C > 2048) || pf1.N % 64 != 0) return std::nullopt;
+    if ((fuse_ln && C > 2048) || pf1.N % 64 != 0 || !aligned16(x)) return std::nullopt;      // (x is also proj's residual)
     for (const Plan *p : {&pq, &pp, &pf1, &pf2})
         if (!can_prepare(*p, rows) || p->bits != pq.bits) return std::nullopt;
     // Not where the one-launch layer kernels are at their best (one 64-row tile on most compute units, short rows): DeiT-S at
@@ -891,8 +895,9 @@ PyObject *py_packed_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
         void *stream = stream_of(x);
         if (strcmp(fmt, "hip_fused") == 0 || strcmp(fmt, "dequant_gemm") == 0) {
             if (gs != 64) return none();
+            if (fmt[0] == 'h' && !aligned16(x)) return none();      // (the general path's stage 1 takes any alignment)
             Tensor y = empty(sizes, at::kFloat, x.device());
-            if (fmt[0] == 'h' && prepare_pays(*plan, m, false, false, false)) {
+            if (fmt[0] == 'h' && prepare_pays(*plan, x, m, false, false)) {
                 Tensor scratch = empty({N * K + m * K}, at::kHalf, x.device());
                 char *base = static_cast<char *>(scratch.mutable_data_ptr());
                 const Weights w{base, arcq_prepared_row_major(m, N, K) != 0};

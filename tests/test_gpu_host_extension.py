@@ -284,3 +284,59 @@ def test_buffers_replaced_by_smaller_ones_are_refused(cuda, fmt):
                         layer(x)
                 layer._buffers[name] = good
                 assert torch.equal(layer(x), want)
+
+
+def _misaligned(t, by=1):
+    """The same values, contiguous, `by` elements off a 16-byte boundary."""
+    flat = torch.empty(t.numel() + 16, dtype=t.dtype, device=t.device)[by:by + t.numel()]
+    return flat.copy_(t.reshape(-1)).view(t.shape)
+
+
+@pytest.mark.parametrize("m,k,n", [(197, 768, 768), (197, 192, 768), (100, 1536, 384), (511, 1024, 4096)])
+def test_layer_on_input_off_the_16_byte_boundary(cuda, m, k, n):
+    layer = _on_the_fly(k, n)
+    for dtype in (torch.float16, torch.float32):
+        x = _tokens(m, k, dtype=dtype)
+        with torch.no_grad():
+            assert torch.equal(layer(_misaligned(x)), layer(x))
+
+
+@pytest.mark.parametrize("m", [1, 197, 1000, 5000])
+def test_hip_fused_on_input_off_the_16_byte_boundary(cuda, m):
+    layer, x = _packed(768, 768, "hip_fused"), _tokens(m, 768, dtype=torch.float32)
+    with torch.no_grad():
+        assert torch.equal(layer(_misaligned(x)), layer(x))
+
+
+@pytest.mark.parametrize("batch", [1, 8, 40])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_block_on_input_off_the_16_byte_boundary(cuda, batch, fp8):
+    from arcq_vit_amd.packed_convert import set_fp8_operands
+    vit = _vit(fuse_elementwise=fp8, own_attention=fp8)
+    if fp8:
+        set_fp8_operands(vit)
+    x = _misaligned(_tokens(batch, 197, 192))
+    with torch.no_grad():
+        assert torch.equal(vit.blocks(x), _interpreted(vit.blocks[0], x))
+
+
+@pytest.mark.parametrize("batch", [8, 40])
+def test_block_on_packed_codes_at_a_4_byte_boundary(cuda, batch):
+    """The one-launch layer kernels take them (from 512 rows on, with the weight buffer lent); so does the block."""
+    vit = _vit(shared_buffers=True, max_rows=batch * 197)
+    block, x = vit.blocks[0], _tokens(batch, 197, 192)
+    with torch.no_grad():
+        for layer in (block.attn.qkv, block.mlp.fc1):
+            layer.packed_weight_codes = _misaligned(layer.packed_weight_codes, 4)
+        assert torch.equal(block(x), _interpreted(block, x))
+
+
+def test_weight_buffer_and_layernorm_off_the_16_byte_boundary(cuda):
+    layer, x = _on_the_fly(768, 768), _tokens(197, 768)
+    norm = torch.nn.LayerNorm(768).cuda()
+    with torch.no_grad():
+        norm.weight.uniform_(0.5, 1.5)
+        want, with_norm = layer(x), layer(x, layernorm=norm)
+        layer._weight_buffer = torch.zeros(768 * 768 + 1, dtype=torch.float16, device=cuda)[1:]
+        norm.weight = torch.nn.Parameter(_misaligned(norm.weight))
+        assert torch.equal(layer(x), want) and torch.equal(layer(x, layernorm=norm), with_norm)
