@@ -14,6 +14,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <c10/core/GradMode.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
@@ -721,6 +722,9 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
     bool plain = f16(x) && c % 64 == 0 && pf2->K % 64 == 0;
     for (PyObject *l : {dq, dp, df1, df2})
         plain = plain && !is_true(get(l, S.fp8_operands)) && get(l, S.out_dtype) == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf));
+    // The skip connections of a default block carry gradients and tangents, torch's additions below record them.  (The packed layers
+    // pass none, and a fused block never did.)
+    plain = plain && !(c10::GradMode::is_enabled() && x.requires_grad()) && !x._fw_grad(0).defined();
     if (plain) {
         auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, refs, false, false);
         if (whole) return whole;

@@ -340,3 +340,23 @@ def test_weight_buffer_and_layernorm_off_the_16_byte_boundary(cuda):
         layer._weight_buffer = torch.zeros(768 * 768 + 1, dtype=torch.float16, device=cuda)[1:]
         norm.weight = torch.nn.Parameter(_misaligned(norm.weight))
         assert torch.equal(layer(x), want) and torch.equal(layer(x, layernorm=norm), with_norm)
+
+
+def test_gradients_pass_the_skip_connections(cuda):
+    """d block(x) / dx of a default block is the identity (the packed layers pass no gradient), so that what stands in front of
+    the blocks is trained; the same for tangents."""
+    import torch.autograd.forward_ad as fw
+    vit = _vit()
+    x = _tokens(2, 197, 192).requires_grad_()
+    y = vit.blocks(x)
+    weight = torch.rand_like(x)
+    (y * weight).sum().backward()
+    assert torch.equal(x.grad, weight)
+    with torch.no_grad():
+        assert torch.equal(vit.blocks(x), y) and not vit.blocks(x).requires_grad
+    images = synth.make_images(2, 1).cuda().half()
+    vit(images).sum().backward()
+    assert all(p.grad is not None for p in (vit.cls_token, vit.pos_embed, vit.patch_embed.proj.weight))
+    with torch.no_grad(), fw.dual_level():
+        dual = fw.unpack_dual(vit.blocks(fw.make_dual(x.detach(), weight)))
+        assert torch.equal(dual.tangent, weight) and torch.equal(dual.primal, y)
