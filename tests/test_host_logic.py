@@ -523,3 +523,23 @@ def test_linear_ex_args_mirror_the_header():
                                                      "int64_t": ctypes.c_int64, "float": ctypes.c_float}[base]
             want.append((name.lstrip("*"), ctype))
     assert [(n, t) for n, t in _lib.LinearExArgs._fields_] == want
+
+
+def test_blocks_trace_symbolically():
+    """torch.fx traces a default block, whole models too, with the packed layers as leaves: nothing branches on the traced
+    tensor."""
+    import torch.fx
+    from arcq_vit_amd.vit import VisionTransformer, build_packed_vit
+
+    class Tracer(torch.fx.Tracer):
+        def is_leaf_module(self, m, name):
+            return isinstance(m, A.ARCQPackedLinearOnTheFly) or super().is_leaf_module(m, name)
+
+    torch.manual_seed(0)
+    plain = VisionTransformer(64, 2, 1, 128, num_classes=4, img=32).eval()
+    x = torch.randn(2, 3, 32, 32)
+    with torch.no_grad():
+        assert torch.equal(torch.fx.symbolic_trace(plain)(x), plain(x))
+    packed = build_packed_vit("deit_tiny", 4, depth=1, num_classes=4, device="cpu")
+    leaves = [n.target for n in Tracer().trace(packed.blocks[0]).nodes if n.op == "call_module"]
+    assert leaves == ["norm1", "attn.qkv", "attn.proj", "norm2", "mlp.fc1", "mlp.act", "mlp.fc2"]
