@@ -19,6 +19,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/DynamicTypes.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
@@ -754,8 +755,8 @@ PyObject *guarded(F &&f)
         return f();
     } catch (const Failure &) {
         return nullptr;
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+    } catch (const std::exception &) {
+        torch::translate_exception_to_python(std::current_exception());       // OutOfMemoryError and its like keep their types
         return nullptr;
     }
 }

@@ -360,3 +360,19 @@ def test_gradients_pass_the_skip_connections(cuda):
     with torch.no_grad(), fw.dual_level():
         dual = fw.unpack_dual(vit.blocks(fw.make_dual(x.detach(), weight)))
         assert torch.equal(dual.tangent, weight) and torch.equal(dual.primal, y)
+
+
+@pytest.mark.parametrize("kind", ["on_the_fly", "hip_fused", "packed"])
+def test_out_of_memory_keeps_its_type(cuda, kind):
+    """A caller that halves its batch on torch.OutOfMemoryError sees that type from the extension's allocations too."""
+    layer = _on_the_fly(64, 1 << 14) if kind == "on_the_fly" else _packed(64, 1 << 14, kind)
+    x = _tokens(1 << 15, 64, dtype=torch.float32)                         # the output: 1 or 2 GiB
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (512 << 20)) / total)
+    try:
+        with torch.no_grad(), pytest.raises(torch.OutOfMemoryError):
+            layer(x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
