@@ -9,7 +9,9 @@
 //
 // Every function returns None where a call is not the plain case (an argument of another type, layout or device, a
 // module with hooks, a shape the library does not run): the Python code behind it then validates, converts and raises
-// as it always did.  Nothing here synchronises; the GIL is held throughout.
+// as it always did.  Nothing here synchronises (but for the one FP8 multiplier of a layer).  What a call needs of its modules
+// is read first, under the GIL; allocations, torch operations and launches follow without it, so that threads on streams
+// of their own run side by side.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -27,6 +29,7 @@
 #include <cstring>
 #include <memory>
 #include <optional>
+#include <stdexcept>
 #include <string>
 #include <vector>
 
@@ -61,21 +64,27 @@ PyObject *g_fp8_multiplier = nullptr;    // ops.fp8_weight_multiplier
 
 struct Failure {};      // a Python exception is set
 
-[[noreturn]] void raise_library_error(int rc)
+// The part of a call that touches no Python object.
+struct NoGil {
+    PyThreadState *state = PyEval_SaveThread();
+    NoGil() = default;
+    NoGil(const NoGil &) = delete;
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+inline void check(int rc)
 {
+    if (rc == 0) return;
     const char *msg = arcq_last_error();
-    if (msg && msg[0]) PyErr_SetString(PyExc_RuntimeError, msg);
-    else PyErr_Format(PyExc_RuntimeError, "libarcq_hip call failed with code %d", rc);
-    throw Failure{};
+    throw std::runtime_error(msg && msg[0] ? std::string(msg) : "libarcq_hip call failed with code " + std::to_string(rc));
 }
-inline void check(int rc) { if (rc != 0) raise_library_error(rc); }
 
 inline PyObject *dict_of(PyObject *o)
 {
     PyObject **d = _PyObject_GetDictPtr(o);
     return d ? *d : nullptr;
 }
-inline PyObject *get(PyObject *dict, PyObject *key) { return dict ? PyDict_GetItem(dict, key) : nullptr; }   // borrowed
+inline PyObject *get(PyObject *dict, PyObject *key) { return dict ? PyDict_GetItemWithError(dict, key) : nullptr; }   // borrowed (str keys: no errors)
 // What `if o:` decides; an absent attribute is false.  (May run code of a class's own __bool__.)
 inline bool is_true(PyObject *o)
 {
@@ -155,8 +164,8 @@ struct Slot {
 };
 // References to Python objects for the length of a call (the GIL is held where it is made and where it ends).
 struct Refs {
-    std::vector<PyObject *> held;
-    Refs() { held.reserve(40); }
+    c10::SmallVector<PyObject *, 64> held;      // (a block: four layers, two LayerNorms, nine modules)
+    Refs() = default;
     Refs(const Refs &) = delete;
     ~Refs() { for (PyObject *o : held) Py_DECREF(o); }
     void add(PyObject *o)
@@ -284,8 +293,14 @@ std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, Refs &refs, PyObject 
     return plan;
 }
 
-// fp32 copies of a LayerNorm's weight and bias (made once per layer and parameter version); nullopt: not the plain case.
-std::optional<LayerNormParams> layernorm_params(Plan &plan, PyObject *ln, Refs &refs, float &eps)
+// A LayerNorm in front of a layer's stage 1, as the library takes it; `weight_copy` and `bias_copy` keep what is not the module's.
+struct FusedLayerNorm {
+    const float *weight, *bias;
+    float eps;
+    Tensor weight_copy, bias_copy;
+};
+// fp32 copies of its weight and bias are made once per layer and parameter version.  False: not the plain case.
+bool read_fused_layernorm(Plan &plan, PyObject *ln, Refs &refs, FusedLayerNorm &out)
 {
     PyObject *d = dict_of(ln);
     PyObject *params = get(d, S._parameters);
@@ -293,41 +308,95 @@ std::optional<LayerNormParams> layernorm_params(Plan &plan, PyObject *ln, Refs &
     const Tensor *w = as_tensor(get(params, S.weight));
     PyObject *bo = get(params, S.bias);
     const Tensor *b = as_tensor(bo);
-    if (!w || !e || !PyFloat_Check(e) || !shape || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != 1) return std::nullopt;
-    if (!b && bo != Py_None) return std::nullopt;
+    if (!w || !e || !PyFloat_Check(e) || !shape || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != 1) return false;
+    if (!b && bo != Py_None) return false;
     refs.add(get(params, S.weight));
     refs.add(bo);
-    eps = static_cast<float>(PyFloat_AS_DOUBLE(e));
-    for (auto &p : plan.ln)
-        if (p.w.same(*w) && p.has_bias() == (b != nullptr) && (!b || p.b.same(*b))) return p;
-    if (!w->is_cuda() || w->device().index() != plan.device || w->numel() != plan.K || w->dim() != 1) return std::nullopt;
-    if (b && (b->device() != w->device() || b->numel() != plan.K)) return std::nullopt;
-    if (plan.ln.size() >= 4) plan.ln.clear();        // (a layer has one LayerNorm in front of it; a bound, not a policy)
-    LayerNormParams p;
-    p.w.set(*w, true, true);
-    if (b) p.b.set(*b, true, true);
-    else p.no_bias = at::zeros({plan.K}, w->options().dtype(at::kFloat).requires_grad(false));
-    plan.ln.push_back(p);
-    return p;
+    out.eps = static_cast<float>(PyFloat_AS_DOUBLE(e));
+    const LayerNormParams *found = nullptr;
+    for (const auto &p : plan.ln)
+        if (p.w.same(*w) && p.has_bias() == (b != nullptr) && (!b || p.b.same(*b))) found = &p;
+    if (!found) {
+        if (!w->is_cuda() || w->device().index() != plan.device || w->numel() != plan.K || w->dim() != 1) return false;
+        if (b && (b->device() != w->device() || b->numel() != plan.K)) return false;
+        LayerNormParams p;
+        p.w.set(*w, true, true);
+        if (b) p.b.set(*b, true, true);
+        else p.no_bias = at::zeros({plan.K}, w->options().dtype(at::kFloat).requires_grad(false));
+        if (plan.ln.size() >= 4) plan.ln.clear();        // (a layer has one LayerNorm in front of it; a bound, not a policy)
+        plan.ln.push_back(std::move(p));
+        found = &plan.ln.back();
+    }
+    out.weight = found->weight(), out.weight_copy = found->w.copy;
+    out.bias = found->bias(), out.bias_copy = found->has_bias() ? found->b.copy : found->no_bias;
+    return true;
 }
 
 // ---- one on-the-fly layer -------------------------------------------------------------------------------------------
+struct Layer {                   // what a call needs of an ARCQPackedLinearOnTheFly
+    std::shared_ptr<Plan> plan;
+    std::optional<at::ScalarType> out;      // none: a type the library does not write
+    bool fp8 = false;
+    float fp8_mult = 1.0f;
+    bool lends = false;                     // has a _weight_buffer ...
+    Tensor weight_buffer, x_hat_buffer;     // ... undefined if it is no tensor
+};
+
+// The power of two inside a layer's FP8 weights (reads the metadata back to the host: once per layer and set of buffers).
+float fp8_multiplier(Plan &p, PyObject *dict)
+{
+    const bool tracked = p.slot[W_CB].tracked && p.slot[W_CENTER].tracked && p.slot[W_SCALE].tracked && p.slot[W_SUM].tracked;
+    if (tracked && !std::isnan(p.fp8_mult)) return static_cast<float>(p.fp8_mult);
+    PyObject *b = get(dict, S._buffers);
+    PyObject *r = PyObject_CallFunctionObjArgs(g_fp8_multiplier, get(b, S.weight_codebook), get(b, S.weight_center), get(b, S.weight_scale),
+                                               get(b, S.weight_code_sum), nullptr);
+    if (!r) throw Failure{};
+    const double mult = PyFloat_AsDouble(r);
+    Py_DECREF(r);
+    if (PyErr_Occurred()) throw Failure{};
+    p.fp8_mult = mult;
+    return static_cast<float>(mult);
+}
+
+bool read_layer(PyObject *module, Refs &refs, Layer &l)
+{
+    PyObject *dict;
+    l.plan = plan_of(module, Kind::OnTheFly, refs, dict);
+    if (!l.plan) return false;
+    PyObject *od = get(dict, S.out_dtype);
+    if (od == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf))) l.out = at::kHalf;
+    else if (od == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kFloat))) l.out = at::kFloat;
+    PyObject *wo = get(dict, S._weight_buffer);
+    l.lends = wo && wo != Py_None;
+    if (const Tensor *t = as_tensor(wo)) l.weight_buffer = *t;
+    if (const Tensor *t = as_tensor(get(dict, S._x_hat_buffer))) l.x_hat_buffer = *t;
+    l.fp8 = is_true(get(dict, S.fp8_operands));
+    if (l.fp8 && l.plan->gs == 64) l.fp8_mult = fp8_multiplier(*l.plan, dict);
+    return true;
+}
+// A buffer lent for scratch of `numel` fp16 values on the device of x.
+bool lent(const Tensor &buffer, int64_t numel, const Tensor &x)
+{
+    return buffer.defined() && buffer.is_cuda() && f16(buffer) && buffer.is_contiguous() && buffer.numel() >= numel &&
+           buffer.device() == x.device();
+}
+
 struct Options {
-    PyObject *layernorm = nullptr, *next = nullptr;
+    const FusedLayerNorm *layernorm = nullptr;
+    const Layer *next = nullptr;
     bool gelu = false, x_is_xhat = false;
     const Tensor *residual = nullptr;
 };
 
 // Whether `a`'s launch may end with the stage 1 of `b` (ARCQPackedLinearOnTheFly.can_quantize_for).
-bool can_quantize(PyObject *da, const Plan &a, PyObject *db, const Plan &b, int64_t rows)
+bool can_quantize(const Layer &la, const Layer &lb, int64_t rows)
 {
-    if (is_true(get(da, S.fp8_operands)) || is_true(get(db, S.fp8_operands)) || rows <= 0 || a.gs != 64 || b.gs != 64 ||
-        a.bits != b.bits || b.K != a.N || a.N % 64 != 0 || a.K % 64 != 0 ||
-        get(da, S.out_dtype) != reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf)))
+    const Plan &a = *la.plan, &b = *lb.plan;
+    if (la.fp8 || lb.fp8 || rows <= 0 || a.gs != 64 || b.gs != 64 || a.bits != b.bits || b.K != a.N || a.N % 64 != 0 || a.K % 64 != 0 ||
+        la.out != at::kHalf)
         return false;
     if (rows < 512) return a.K <= 1536;
-    PyObject *w = get(da, S._weight_buffer);
-    if (!w || w == Py_None || rows * a.K * 2 >= (int64_t(1) << 32)) return false;
+    if (!la.lends || rows * a.K * 2 >= (int64_t(1) << 32)) return false;
     return strncmp(arcq_linear_otf_ws_kernel(rows, a.N, a.K, 1), "otf_rows", 8) != 0;
 }
 
@@ -335,7 +404,8 @@ bool can_quantize(PyObject *da, const Plan &a, PyObject *db, const Plan &b, int6
 struct Weights {                 // w_hat of one layer inside a scratch tensor
     void *ptr;
     bool row_major;
-    bool fp8 = false;            // FP8 operands: rows of Kp = K rounded up to 128 bytes
+    bool fp8 = false;            // FP8 operands: rows of Kp = K rounded up to 128 bytes, times `mult`
+    float mult = 1.0f;
 };
 int64_t operand_row_bytes(int64_t K, bool fp8) { return fp8 ? (K + 127) / 128 * 128 : 2 * K; }
 // Fields of arcq_prepare_args for a layer's own tensors.
@@ -345,9 +415,9 @@ void set_weights(arcq_prepare_weights &w, const Plan &p, const Weights &out)
     w.codebook = static_cast<const float *>(p.p[W_CB]), w.center = static_cast<const float *>(p.p[W_CENTER]);
     w.scale = static_cast<const float *>(p.p[W_SCALE]), w.code_sum = static_cast<const float *>(p.p[W_SUM]);
     w.w_hat = out.ptr, w.N = p.N, w.K = p.K, w.row_major = out.row_major ? 1 : 0;
-    w.w_mult = static_cast<float>(p.fp8_mult);
+    w.w_mult = out.mult;
 }
-void run_prepare(const Tensor &x, int64_t rows, const Plan &first, const LayerNormParams *ln, float ln_eps, void *x_hat, const Weights &w_first,
+void run_prepare(const Tensor &x, int64_t rows, const Plan &first, const FusedLayerNorm *ln, void *x_hat, const Weights &w_first,
                  const Plan *second, const Weights *w_second, void *stream)
 {
     arcq_prepare_args a = {};
@@ -356,7 +426,7 @@ void run_prepare(const Tensor &x, int64_t rows, const Plan &first, const LayerNo
     a.fp8 = w_first.fp8 ? 1 : 0;
     a.rows = rows, a.K = first.K;
     a.x = x.const_data_ptr();
-    if (ln) a.ln_weight = ln->weight(), a.ln_bias = ln->bias(), a.ln_eps = ln_eps;
+    if (ln) a.ln_weight = ln->weight, a.ln_bias = ln->bias, a.ln_eps = ln->eps;
     a.thresholds = static_cast<const float *>(first.p[A_THR]), a.codebook = static_cast<const float *>(first.p[A_CB]);
     a.x_hat = x_hat;
     if (w_first.ptr) set_weights(a.weights[0], first, w_first);
@@ -379,7 +449,7 @@ void run_product(const Plan &p, int64_t rows, const void *x_hat, const Weights &
         a.next_bits = static_cast<int32_t>(next->bits);
     }
     a.y = y;
-    a.fp8 = w.fp8 ? 1 : 0, a.w_mult = static_cast<float>(p.fp8_mult);
+    a.fp8 = w.fp8 ? 1 : 0, a.w_mult = w.mult;
     check(arcq_linear_prepared(&a, stream));
 }
 // (packed codes that are not 16-byte aligned are left to the kernels and entry points that take them, or say why not)
@@ -399,103 +469,64 @@ bool prepare_pays(const Plan &p, const Tensor &x, int64_t rows, bool has_ws, boo
     return !(f16(x) && has_ws && strncmp(arcq_linear_otf_ws_kernel(rows, p.N, p.K, 1), "otf_rows", 8) == 0);
 }
 
-// The power of two inside a layer's FP8 weights (reads the metadata back to the host: once per layer and set of buffers).
-void find_fp8_multiplier(Plan &p, PyObject *dict)
+bool takes(const Layer &l, const Tensor &x)
 {
-    const bool tracked = p.slot[W_CB].tracked && p.slot[W_CENTER].tracked && p.slot[W_SCALE].tracked && p.slot[W_SUM].tracked;
-    if (tracked && !std::isnan(p.fp8_mult)) return;
-    PyObject *b = get(dict, S._buffers);
-    PyObject *r = PyObject_CallFunctionObjArgs(g_fp8_multiplier, get(b, S.weight_codebook), get(b, S.weight_center), get(b, S.weight_scale),
-                                               get(b, S.weight_code_sum), nullptr);
-    if (!r) throw Failure{};
-    p.fp8_mult = PyFloat_AsDouble(r);
-    Py_DECREF(r);
-    if (PyErr_Occurred()) throw Failure{};
+    return here(x) && x.device().index() == l.plan->device && x.is_contiguous() && (f16(x) || f32(x)) && x.dim() >= 1 &&
+           x.size(-1) == l.plan->K && x.numel() != 0;
 }
 
-std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Options &o)
+// One layer's launches; nullopt before the first where the call is not the plain case.  No Python object is touched.
+std::optional<Tensor> run_layer(const Layer &l, const Tensor &x, const Options &o)
 {
-    Refs refs;
-    PyObject *dict;
-    const auto plan = plan_of(module, Kind::OnTheFly, refs, dict);
-    if (!plan || !here(x) || x.device().index() != plan->device || !x.is_contiguous() || (!f16(x) && !f32(x)) || x.dim() < 1 ||
-        x.size(-1) != plan->K || x.numel() == 0)
-        return std::nullopt;
+    if (!takes(l, x) || !l.out) return std::nullopt;
+    const Plan *plan = l.plan.get();
     const int64_t K = plan->K, N = plan->N, m = x.numel() / K;
-    PyObject *od = get(dict, S.out_dtype);
-    at::ScalarType out_type;
-    if (od == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf))) out_type = at::kHalf;
-    else if (od == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kFloat))) out_type = at::kFloat;
-    else return std::nullopt;
-    const bool fp8 = is_true(get(dict, S.fp8_operands));
+    const at::ScalarType out_type = *l.out;
     const bool extras = o.layernorm || o.gelu || o.residual || o.next || o.x_is_xhat;
-    float ln_eps = 0.0f;
-    std::optional<LayerNormParams> ln;
     if (extras) {
-        if (fp8 || plan->gs != 64 || K % 64 != 0) return std::nullopt;
-        if (o.layernorm) {
-            if (K > 1024 && (K > 1536 || m >= 512)) return std::nullopt;
-            ln = layernorm_params(*plan, o.layernorm, refs, ln_eps);
-            if (!ln) return std::nullopt;
-        }
+        if (l.fp8 || plan->gs != 64 || K % 64 != 0) return std::nullopt;
+        if (o.layernorm && K > 1024 && (K > 1536 || m >= 512)) return std::nullopt;
         if (o.x_is_xhat && (!f16(x) || o.layernorm)) return std::nullopt;
         if (o.residual && (o.residual->scalar_type() != out_type || o.residual->device() != x.device() ||
                            !o.residual->is_contiguous() || o.residual->numel() != m * N || o.residual->size(-1) != N))
             return std::nullopt;
     }
-    std::shared_ptr<Plan> next;
-    if (o.next) {
-        PyObject *nd;
-        next = plan_of(o.next, Kind::OnTheFly, refs, nd);
-        if (!next || next->device != plan->device || !can_quantize(dict, *plan, nd, *next, m)) return std::nullopt;
-    }
+    if (o.next && (o.next->plan->device != plan->device || !can_quantize(l, *o.next, m))) return std::nullopt;
     at::DimVector sizes(x.sizes());
     sizes.back() = N;
     void *stream = stream_of(x);
     const auto *p = plan->p;
     auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
-    if (fp8) {
+    if (l.fp8) {
         if (plan->gs != 64) return std::nullopt;
-        find_fp8_multiplier(*plan, dict);
         const int64_t kp = (K + 127) / 128 * 128;
         Tensor x8 = empty({m * kp}, at::kByte, x.device()), w8 = empty({N * kp}, at::kByte, x.device());
         Tensor y = empty(sizes, out_type, x.device());
         check(arcq_linear_otf_fp8(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), static_cast<const uint8_t *>(p[W_PACKED]),
-                                  fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), static_cast<float>(plan->fp8_mult),
+                                  fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), l.fp8_mult,
                                   x8.mutable_data_ptr(), w8.mutable_data_ptr(), y.mutable_data_ptr(), code_of(y), m, N, K,
                                   static_cast<int>(plan->bits), stream));
         return y;
     }
-    PyObject *wo = get(dict, S._weight_buffer);
-    const Tensor *w_ws = nullptr;
-    if (wo && wo != Py_None) {
-        w_ws = as_tensor(wo);
-        if (!w_ws || !w_ws->is_cuda() || !f16(*w_ws) || !w_ws->is_contiguous() || w_ws->numel() < N * K ||
-            w_ws->device() != x.device())
-            return std::nullopt;
-    }
-    if (!next && !o.x_is_xhat && prepare_pays(*plan, x, m, w_ws != nullptr, ln.has_value())) {
+    if (l.lends && !lent(l.weight_buffer, N * K, x)) return std::nullopt;
+    const Tensor *w_ws = l.lends ? &l.weight_buffer : nullptr;
+    if (!o.next && !o.x_is_xhat && prepare_pays(*plan, x, m, w_ws != nullptr, o.layernorm != nullptr)) {
         // (x_hat and w_hat in one scratch tensor; w_hat first: 512-byte runs stay aligned)
-        const bool lent = w_ws != nullptr && aligned16(*w_ws);
-        Tensor scratch = empty({(lent ? 0 : N * K) + m * K}, at::kHalf, x.device());
+        const bool use_ws = w_ws != nullptr && aligned16(*w_ws);
+        Tensor scratch = empty({(use_ws ? 0 : N * K) + m * K}, at::kHalf, x.device());
         char *base = static_cast<char *>(scratch.mutable_data_ptr());
-        const Weights w{lent ? w_ws->mutable_data_ptr() : base, arcq_prepared_row_major(m, N, K) != 0};
-        void *x_hat = lent ? base : base + N * K * 2;
+        const Weights w{use_ws ? w_ws->mutable_data_ptr() : base, arcq_prepared_row_major(m, N, K) != 0};
+        void *x_hat = use_ws ? base : base + N * K * 2;
         Tensor y = empty(sizes, out_type, x.device());
-        run_prepare(x, m, *plan, ln ? &*ln : nullptr, ln_eps, x_hat, w, nullptr, nullptr, stream);
+        run_prepare(x, m, *plan, o.layernorm, x_hat, w, nullptr, nullptr, stream);
         run_product(*plan, m, x_hat, w, o.residual, o.gelu, nullptr, y.mutable_data_ptr(), code_of(y), stream);
         return y;
     }
-    Tensor own_ws;
-    const Tensor *ws = as_tensor(get(dict, S._x_hat_buffer));
-    if (!ws || !f16(*ws) || !ws->is_contiguous() || ws->numel() < x.numel() || ws->device() != x.device()) {
-        own_ws = empty({x.numel()}, at::kHalf, x.device());
-        ws = &own_ws;
-    }
+    const Tensor ws = lent(l.x_hat_buffer, x.numel(), x) ? l.x_hat_buffer : empty({x.numel()}, at::kHalf, x.device());
     Tensor y = empty(sizes, out_type, x.device());
     if (!extras) {
         check(arcq_linear_otf_ws(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), static_cast<const uint8_t *>(p[W_PACKED]),
-                                 fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), ws->mutable_data_ptr(),
+                                 fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), ws.mutable_data_ptr(),
                                  w_ws ? w_ws->mutable_data_ptr() : nullptr, y.mutable_data_ptr(), code_of(y), m, N, K,
                                  static_cast<int>(plan->bits), static_cast<int>(plan->gs), stream));
         return y;
@@ -508,20 +539,20 @@ std::optional<Tensor> layer_call(PyObject *module, const Tensor &x, const Option
     a.group_size = static_cast<int>(plan->gs);
     a.M = m, a.N = N, a.K = K;
     a.x = x.const_data_ptr();
-    if (ln) {
+    if (o.layernorm) {
         a.producer = ARCQ_PRODUCER_LAYERNORM;
-        a.ln_weight = ln->weight(), a.ln_bias = ln->bias(), a.ln_eps = ln_eps;
+        a.ln_weight = o.layernorm->weight, a.ln_bias = o.layernorm->bias, a.ln_eps = o.layernorm->eps;
     }
     if (o.x_is_xhat) a.producer = ARCQ_PRODUCER_XHAT;
     a.activation = o.gelu ? ARCQ_ACT_GELU : ARCQ_ACT_NONE;
     a.a_thresholds = fp(A_THR), a.a_codebook = fp(A_CB), a.packed_w = static_cast<const uint8_t *>(p[W_PACKED]);
     a.w_codebook = fp(W_CB), a.w_center = fp(W_CENTER), a.w_scale = fp(W_SCALE), a.w_code_sum = fp(W_SUM), a.bias = fp(W_BIAS);
     if (o.residual) a.residual = o.residual->const_data_ptr();
-    if (next) {
-        a.next_a_thresholds = static_cast<const float *>(next->p[A_THR]);
-        a.next_a_codebook = static_cast<const float *>(next->p[A_CB]);
+    if (o.next) {
+        a.next_a_thresholds = static_cast<const float *>(o.next->plan->p[A_THR]);
+        a.next_a_codebook = static_cast<const float *>(o.next->plan->p[A_CB]);
     }
-    a.x_hat_ws = ws->mutable_data_ptr();
+    a.x_hat_ws = ws.mutable_data_ptr();
     a.w_hat_ws = w_ws ? w_ws->mutable_data_ptr() : nullptr;
     a.y = y.mutable_data_ptr();
     check(arcq_linear_otf_ex(&a, stream));
@@ -570,22 +601,24 @@ Tensor mix(const Tensor &qkv, int64_t heads, bool own)      // Attention.mix
     return at::scaled_dot_product_attention(t.select(0, 0), t.select(0, 1), t.select(0, 2)).transpose(1, 2).reshape({b, n, c});
 }
 
-Tensor layernorm_op(PyObject *d, const Tensor &x, bool &ok)      // an nn.LayerNorm as torch runs it
+struct LayerNorm {               // an nn.LayerNorm as torch runs it
+    std::optional<Tensor> weight, bias;
+    int64_t n = 0;
+    double eps = 0;
+    Tensor operator()(const Tensor &x) const { return at::layer_norm(x, {n}, weight, bias, eps); }
+};
+bool read_layernorm(PyObject *d, LayerNorm &out)
 {
     PyObject *params = get(d, S._parameters), *e = get(d, S.eps), *shape = get(d, S.normalized_shape);
     PyObject *wo = get(params, S.weight), *bo = get(params, S.bias);
-    if (!e || !PyFloat_Check(e) || !shape || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != 1 || !wo || !bo) {
-        ok = false;
-        return {};
-    }
+    if (!e || !PyFloat_Check(e) || !shape || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != 1 || !wo || !bo) return false;
     const Tensor *w = as_tensor(wo), *b = as_tensor(bo);
-    if ((!w && wo != Py_None) || (!b && bo != Py_None)) {
-        ok = false;
-        return {};
-    }
-    const int64_t n = PyLong_AsLongLong(PyTuple_GET_ITEM(shape, 0));
-    return at::layer_norm(x, {n}, w ? std::optional<Tensor>(*w) : std::nullopt, b ? std::optional<Tensor>(*b) : std::nullopt,
-                          PyFloat_AS_DOUBLE(e));
+    if ((!w && wo != Py_None) || (!b && bo != Py_None)) return false;
+    if (w) out.weight = *w;
+    if (b) out.bias = *b;
+    out.n = PyLong_AsLongLong(PyTuple_GET_ITEM(shape, 0));
+    out.eps = PyFloat_AS_DOUBLE(e);
+    return true;
 }
 
 // A block on prepared operands: [LayerNorm + stage 1, weights of qkv and proj] -> qkv -> attention ending with proj's stage 1
@@ -596,12 +629,20 @@ Tensor layernorm_op(PyObject *d, const Tensor &x, bool &ok)      // an nn.LayerN
 //   fp8:            FP8 operands.  LayerNorms as torch runs them: that is what the layers do one by one, and a network of
 //                   quantizers does not forgive another order of summation (one changed bit is 10 % of the logits 12 blocks on)
 //   attention that the library's kernel does not run (or is not to): torch's, then stage 1 of proj as a launch of its own
-std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t heads, bool own, Plan &pq, Plan &pp, Plan &pf1, Plan &pf2,
-                                     PyObject *n1, PyObject *n2, Refs &refs, bool fused, bool fp8)
+struct BlockParts {
+    int64_t heads;
+    bool own;                    // attention on the library's kernel where it serves the shape
+    bool fused, fp8;
+    Layer qkv, proj, fc1, fc2;
+    LayerNorm norm1, norm2;                  // as torch runs them: not fused, or FP8 operands
+    FusedLayerNorm fused1, fused2;           // inside qkv's and fc1's launches
+};
+std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64_t rows)
 {
+    const Plan &pq = *k.qkv.plan, &pp = *k.proj.plan, &pf1 = *k.fc1.plan, &pf2 = *k.fc2.plan;
     const int64_t b = x.size(0), n = x.size(1), C = x.size(2);
-    const bool fuse_ln = fused && !fp8;
-    const bool own_attention = own && n <= 256 && C == 64 * heads;
+    const bool fp8 = k.fp8, fuse_ln = k.fused && !fp8;
+    const bool own_attention = k.own && n <= 256 && C == 64 * k.heads;
     if ((fuse_ln && C > 2048) || pf1.N % 64 != 0 || !aligned16(x)) return std::nullopt;      // (x is also proj's residual)
     for (const Plan *p : {&pq, &pp, &pf1, &pf2})
         if (!can_prepare(*p, rows) || p->bits != pq.bits) return std::nullopt;
@@ -609,17 +650,7 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
     // 12 608 rows 1 625 us a forward against 1 939, DeiT-B 3 969 against 4 373; at 9 456 rows 4 % either way, below and above
     // that range the seven launches win (6 304 rows: 1 353 -> 1 262 us; 25 216 rows: 3 341 -> 3 286).
     if (fuse_ln && rows > 9000 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) return std::nullopt;
-    float e1 = 0, e2 = 0;
-    std::optional<LayerNormParams> l1, l2;
-    Tensor t = x;
-    if (fuse_ln) {
-        l1 = layernorm_params(pq, n1, refs, e1), l2 = layernorm_params(pf1, n2, refs, e2);
-        if (!l1 || !l2) return std::nullopt;
-    } else {
-        bool ok = true;
-        t = layernorm_op(dict_of(n1), x, ok);
-        if (!ok) return std::nullopt;
-    }
+    Tensor t = fuse_ln ? x : k.norm1(x);
     void *stream = stream_of(x);
     auto layout = [&](const Plan &p) { return arcq_prepared_row_major(rows, p.N, p.K) != 0; };
     auto weight_bytes = [&](const Plan &p) { return p.N * operand_row_bytes(p.K, fp8); };
@@ -630,28 +661,78 @@ std::optional<Tensor> block_prepared(const Tensor &x, int64_t rows, int64_t head
     Tensor wide = empty({rows * operand_row_bytes(pf2.K, fp8)}, at::kByte, x.device());       // fc1's quantized output
     Tensor qkv = empty({b, n, pq.N}, at::kHalf, x.device());
     Tensor x1 = empty(x.sizes(), at::kHalf, x.device()), y = empty(x.sizes(), at::kHalf, x.device());
-    const Weights hq{wb, layout(pq), fp8}, hp{wb + wq, layout(pp), fp8}, h1{wb, layout(pf1), fp8}, h2{wb + w1, layout(pf2), fp8};
-    run_prepare(t, rows, pq, l1 ? &*l1 : nullptr, e1, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
+    const Weights hq{wb, layout(pq), fp8, k.qkv.fp8_mult}, hp{wb + wq, layout(pp), fp8, k.proj.fp8_mult},
+                  h1{wb, layout(pf1), fp8, k.fc1.fp8_mult}, h2{wb + w1, layout(pf2), fp8, k.fc2.fp8_mult};
+    run_prepare(t, rows, pq, fuse_ln ? &k.fused1 : nullptr, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
     run_product(pq, rows, xh.const_data_ptr(), hq, nullptr, false, nullptr, qkv.mutable_data_ptr(), ARCQ_F16, stream);
     if (own_attention) {
         check((fp8 ? arcq_attention_quant_fp8_fwd : arcq_attention_quant_fwd)(qkv.const_data_ptr(), static_cast<const float *>(pp.p[A_THR]),
-            static_cast<const float *>(pp.p[A_CB]), static_cast<int>(pp.bits), xh.mutable_data_ptr(), b, n, heads, 64, 0.125f, stream));
+            static_cast<const float *>(pp.p[A_CB]), static_cast<int>(pp.bits), xh.mutable_data_ptr(), b, n, k.heads, 64, 0.125f, stream));
     } else {
-        const Tensor a = as_operand(mix(qkv, heads, false));          // (bf16 under autocast to that type)
-        run_prepare(a, rows, pp, nullptr, 0, xh.mutable_data_ptr(), Weights{nullptr, false, fp8}, nullptr, nullptr, stream);
+        const Tensor a = as_operand(mix(qkv, k.heads, false));        // (bf16 under autocast to that type)
+        run_prepare(a, rows, pp, nullptr, xh.mutable_data_ptr(), Weights{nullptr, false, fp8}, nullptr, nullptr, stream);
     }
     run_product(pp, rows, xh.const_data_ptr(), hp, &x, false, nullptr, x1.mutable_data_ptr(), ARCQ_F16, stream);
-    bool ok = true;
-    t = fuse_ln ? x1 : layernorm_op(dict_of(n2), x1, ok);
-    if (!ok) return std::nullopt;
-    run_prepare(t, rows, pf1, l2 ? &*l2 : nullptr, e2, xh.mutable_data_ptr(), h1, &pf2, &h2, stream);
+    t = fuse_ln ? x1 : k.norm2(x1);
+    run_prepare(t, rows, pf1, fuse_ln ? &k.fused2 : nullptr, xh.mutable_data_ptr(), h1, &pf2, &h2, stream);
     run_product(pf1, rows, xh.const_data_ptr(), h1, nullptr, true, &pf2, wide.mutable_data_ptr(), ARCQ_F16, stream);
     run_product(pf2, rows, wide.const_data_ptr(), h2, &x1, false, nullptr, y.mutable_data_ptr(), ARCQ_F16, stream);
     return y;
 }
 
-// One transformer block (vit.Block.forward), both of its forms; nullopt before anything has been launched where a module
-// is not the plain case.
+// One transformer block (vit.Block.forward), both of its forms.  No Python object is touched.
+std::optional<Tensor> run_block(const BlockParts &k, const Tensor &x, bool chain)
+{
+    const int64_t rows = x.size(0) * x.size(1);
+    if (k.fused) {
+        if (chain) {
+            auto whole = block_prepared(k, x, rows);
+            if (whole) return whole;
+        }
+        if (k.fp8) return std::nullopt;
+        Options o1;
+        o1.layernorm = &k.fused1;
+        auto t = run_layer(k.qkv, x, o1);
+        if (!t) return std::nullopt;
+        const Tensor a = as_operand(mix(*t, k.heads, k.own));
+        Options o2;
+        o2.residual = &x;
+        auto x1 = run_layer(k.proj, a, o2);
+        if (!x1) return std::nullopt;
+        Options o3, o4;
+        o3.layernorm = &k.fused2;
+        o3.gelu = true;
+        if (chain && can_quantize(k.fc1, k.fc2, rows)) {
+            o3.next = &k.fc2;
+            o4.x_is_xhat = true;
+        }
+        auto h = run_layer(k.fc1, *x1, o3);
+        if (!h) return std::nullopt;
+        o4.residual = &*x1;
+        return run_layer(k.fc2, *h, o4);
+    }
+    bool plain = f16(x) && x.size(2) % 64 == 0 && k.fc2.plan->K % 64 == 0;
+    for (const Layer *l : {&k.qkv, &k.proj, &k.fc1, &k.fc2}) plain = plain && !l->fp8 && l->out == at::kHalf;
+    // The skip connections of a default block carry gradients and tangents, torch's additions below record them.  (The packed layers
+    // pass none, and a fused block never did.)
+    plain = plain && !(c10::GradMode::is_enabled() && x.requires_grad()) && !x._fw_grad(0).defined();
+    if (plain) {
+        auto whole = block_prepared(k, x, rows);
+        if (whole) return whole;
+    }
+    auto q = run_layer(k.qkv, as_operand(k.norm1(x)), Options{});
+    if (!q) return std::nullopt;
+    auto a = run_layer(k.proj, as_operand(mix(*q, k.heads, k.own)), Options{});
+    if (!a) return std::nullopt;
+    const Tensor x1 = at::add(x, *a);
+    auto h = run_layer(k.fc1, as_operand(k.norm2(x1)), Options{});
+    if (!h) return std::nullopt;
+    auto y = run_layer(k.fc2, at::gelu(*h), Options{});
+    if (!y) return std::nullopt;
+    return at::add(x1, *y);
+}
+
+// nullopt before anything has been launched where a module is not the plain case
 std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
 {
     PyObject *d = dict_of(block);
@@ -668,83 +749,36 @@ std::optional<Tensor> block_call(PyObject *block, const Tensor &x)
     if (!is_type(act, g_gelu_type) || get(ad, S.mix)) return std::nullopt;
     PyObject *approx = get(dict_of(act), S.approximate);
     if (!approx || !PyUnicode_Check(approx) || PyUnicode_Compare(approx, S.none) != 0) return std::nullopt;
-    int64_t heads;
-    if (!get_int(ad, S.num_heads, heads) || heads <= 0) return std::nullopt;
-    const bool own = is_true(get(ad, S.own_kernel));
-    Refs refs;
-    PyObject *dq, *dp, *df1, *df2;
-    const auto pq = plan_of(qkv, Kind::OnTheFly, refs, dq), pp = plan_of(proj, Kind::OnTheFly, refs, dp),
-               pf1 = plan_of(fc1, Kind::OnTheFly, refs, df1), pf2 = plan_of(fc2, Kind::OnTheFly, refs, df2);
-    const int64_t c = x.size(2);
-    if (!pq || !pp || !pf1 || !pf2 || pq->K != c || pq->N != 3 * c || pp->K != c || pp->N != c || pf1->K != c || pf2->K != pf1->N ||
-        pf2->N != c || c % heads != 0)
+    Refs refs;                   // (reading flags and FP8 metadata may run Python code)
+    for (PyObject *o : {attn, mlp, n1, n2, qkv, proj, fc1, fc2, act}) refs.add(o);
+    BlockParts k;
+    if (!get_int(ad, S.num_heads, k.heads) || k.heads <= 0) return std::nullopt;
+    k.own = is_true(get(ad, S.own_kernel));
+    k.fused = is_true(get(d, S.fuse_elementwise));
+    const bool chain = k.fused && is_true(get(d, S.chain_mlp));
+    if (!k.fused)
+        for (PyObject *dd : {ad, md, d1, d2, dict_of(act)})
+            if (!no_hooks(dd)) return std::nullopt;
+    if (!read_layer(qkv, refs, k.qkv) || !read_layer(proj, refs, k.proj) || !read_layer(fc1, refs, k.fc1) || !read_layer(fc2, refs, k.fc2))
         return std::nullopt;
-    const int64_t rows = x.size(0) * x.size(1);
-    if (is_true(get(d, S.fuse_elementwise))) {
-        const bool fp8 = is_true(get(dq, S.fp8_operands));
-        for (PyObject *l : {dq, dp, df1, df2})
-            if (is_true(get(l, S.fp8_operands)) != fp8 || get(l, S.out_dtype) != reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf)))
-                return std::nullopt;
-        if (!f16(x) || c > (rows >= 512 ? 1024 : 1536) || c % 64 != 0 || pf2->K % 64 != 0) return std::nullopt;
-        for (Plan *p : {pq.get(), pp.get(), pf1.get(), pf2.get()})
-            if (p->gs != 64) return std::nullopt;
-        if (fp8)
-            for (auto [p, l] : {std::pair(pq.get(), dq), {pp.get(), dp}, {pf1.get(), df1}, {pf2.get(), df2}}) find_fp8_multiplier(*p, l);
-        const bool chain = is_true(get(d, S.chain_mlp));
-        if (chain) {
-            auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, refs, true, fp8);
-            if (whole) return whole;
-        }
-        if (fp8) return std::nullopt;
-        Options o1;
-        o1.layernorm = n1;
-        auto t = layer_call(qkv, x, o1);
-        if (!t) return std::nullopt;
-        const Tensor a = as_operand(mix(*t, heads, own));
-        Options o2;
-        o2.residual = &x;
-        auto x1 = layer_call(proj, a, o2);
-        if (!x1) return std::nullopt;
-        Options o3, o4;
-        o3.layernorm = n2;
-        o3.gelu = true;
-        PyObject *cm = get(d, S.chain_mlp);
-        if (is_true(cm) && can_quantize(df1, *pf1, df2, *pf2, rows)) {
-            o3.next = fc2;
-            o4.x_is_xhat = true;
-        }
-        auto h = layer_call(fc1, *x1, o3);
-        if (!h) return std::nullopt;
-        o4.residual = &*x1;
-        return layer_call(fc2, *h, o4);
+    const Plan &pq = *k.qkv.plan, &pp = *k.proj.plan, &pf1 = *k.fc1.plan, &pf2 = *k.fc2.plan;
+    const int64_t c = x.size(2), rows = x.size(0) * x.size(1);
+    if (pq.K != c || pq.N != 3 * c || pp.K != c || pp.N != c || pf1.K != c || pf2.K != pf1.N || pf2.N != c || c % k.heads != 0)
+        return std::nullopt;
+    k.fp8 = k.fused && k.qkv.fp8;
+    if (k.fused) {
+        for (const Layer *l : {&k.qkv, &k.proj, &k.fc1, &k.fc2})
+            if (l->fp8 != k.fp8 || l->out != at::kHalf || l->plan->gs != 64) return std::nullopt;
+        if (!f16(x) || c > (rows >= 512 ? 1024 : 1536) || c % 64 != 0 || pf2.K % 64 != 0) return std::nullopt;
     }
-    for (PyObject *dd : {ad, md, d1, d2, dict_of(act)})
-        if (!no_hooks(dd)) return std::nullopt;
-    bool plain = f16(x) && c % 64 == 0 && pf2->K % 64 == 0;
-    for (PyObject *l : {dq, dp, df1, df2})
-        plain = plain && !is_true(get(l, S.fp8_operands)) && get(l, S.out_dtype) == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf));
-    // The skip connections of a default block carry gradients and tangents, torch's additions below record them.  (The packed layers
-    // pass none, and a fused block never did.)
-    plain = plain && !(c10::GradMode::is_enabled() && x.requires_grad()) && !x._fw_grad(0).defined();
-    if (plain) {
-        auto whole = block_prepared(x, rows, heads, own, *pq, *pp, *pf1, *pf2, n1, n2, refs, false, false);
-        if (whole) return whole;
+    if (k.fused && !k.fp8) {
+        if (!read_fused_layernorm(*k.qkv.plan, n1, refs, k.fused1) || !read_fused_layernorm(*k.fc1.plan, n2, refs, k.fused2))
+            return std::nullopt;
+    } else if (!read_layernorm(d1, k.norm1) || !read_layernorm(d2, k.norm2)) {
+        return std::nullopt;
     }
-    bool ok = true;
-    Tensor t = layernorm_op(d1, x, ok);
-    if (!ok) return std::nullopt;
-    auto q = layer_call(qkv, as_operand(t), Options{});
-    if (!q) return std::nullopt;
-    auto a = layer_call(proj, as_operand(mix(*q, heads, own)), Options{});
-    if (!a) return std::nullopt;
-    const Tensor x1 = at::add(x, *a);
-    t = layernorm_op(d2, x1, ok);
-    if (!ok) return std::nullopt;
-    auto h = layer_call(fc1, as_operand(t), Options{});
-    if (!h) return std::nullopt;
-    auto y = layer_call(fc2, at::gelu(*h), Options{});
-    if (!y) return std::nullopt;
-    return at::add(x1, *y);
+    NoGil released;
+    return run_block(k, x, chain);
 }
 
 // ---- Python entry points ----------------------------------------------------------------------------------------------
@@ -773,19 +807,28 @@ PyObject *py_layer_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
     return guarded([&]() -> PyObject * {
         const Tensor *x = n == 7 ? as_tensor(args[1]) : nullptr;
         if (!x) return none();
+        Refs refs;
+        Layer layer, next;
+        FusedLayerNorm ln;
         Options o;
-        if (args[2] != Py_None) {
-            if (!is_type(args[2], g_layernorm_type)) return none();
-            o.layernorm = args[2];
-        }
         o.gelu = is_true(args[3]);
-        if (args[4] != Py_None && !(o.residual = as_tensor(args[4]))) return none();
-        if (args[5] != Py_None) {
-            if (!PyObject_TypeCheck(args[5], reinterpret_cast<PyTypeObject *>(g_layer_type))) return none();
-            o.next = args[5];
-        }
         o.x_is_xhat = is_true(args[6]);
-        return wrap(layer_call(args[0], *x, o));
+        if (args[4] != Py_None && !(o.residual = as_tensor(args[4]))) return none();
+        if (!read_layer(args[0], refs, layer) || !takes(layer, *x)) return none();
+        if (args[2] != Py_None) {
+            if (!is_type(args[2], g_layernorm_type) || !read_fused_layernorm(*layer.plan, args[2], refs, ln)) return none();
+            o.layernorm = &ln;
+        }
+        if (args[5] != Py_None) {
+            if (!PyObject_TypeCheck(args[5], reinterpret_cast<PyTypeObject *>(g_layer_type)) || !read_layer(args[5], refs, next)) return none();
+            o.next = &next;
+        }
+        std::optional<Tensor> y;
+        {
+            NoGil released;
+            y = run_layer(layer, *x, o);
+        }
+        return wrap(std::move(y));
     });
 }
 
@@ -803,7 +846,14 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n)
     return guarded([&]() -> PyObject * {
         const Tensor *q = n == 3 ? as_tensor(args[0]) : nullptr;
         if (!q || !PyLong_CheckExact(args[1]) || !PyFloat_CheckExact(args[2])) return none();
-        return wrap(attention_call(*q, PyLong_AsLongLong(args[1]), static_cast<float>(PyFloat_AS_DOUBLE(args[2]))));
+        const int64_t heads = PyLong_AsLongLong(args[1]);
+        const float scale = static_cast<float>(PyFloat_AS_DOUBLE(args[2]));
+        std::optional<Tensor> y;
+        {
+            NoGil released;
+            y = attention_call(*q, heads, scale);
+        }
+        return wrap(std::move(y));
     });
 }
 
@@ -824,10 +874,14 @@ PyObject *py_patch_embed(PyObject *, PyObject *const *args, Py_ssize_t n)
         if (b == 0 || N % 32 != 0 || h % 16 != 0 || wd % 16 != 0 || t[3]->numel() != N || t[4]->numel() != tokens * N ||
             (t[2] && t[2]->numel() != N))
             return none();
-        Tensor out = empty({b, tokens, N}, at::kHalf, img.device());
-        check(arcq_patch_embed_fwd(img.const_data_ptr(), w.const_data_ptr(), t[2] ? t[2]->const_data_ptr() : nullptr,
-                                   t[3]->const_data_ptr(), t[4]->const_data_ptr(), out.mutable_data_ptr(), b, h, wd, 16, N,
-                                   stream_of(img)));
+        Tensor out;
+        {
+            NoGil released;
+            out = empty({b, tokens, N}, at::kHalf, img.device());
+            check(arcq_patch_embed_fwd(img.const_data_ptr(), w.const_data_ptr(), t[2] ? t[2]->const_data_ptr() : nullptr,
+                                       t[3]->const_data_ptr(), t[4]->const_data_ptr(), out.mutable_data_ptr(), b, h, wd, 16, N,
+                                       stream_of(img)));
+        }
         return THPVariable_Wrap(std::move(out));
     });
 }
@@ -863,7 +917,12 @@ PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t n)
         const Tensor *x = as_tensor(args[0]), *thr = as_tensor(args[1]), *cb = as_tensor(args[2]);
         const int64_t bits = PyLong_AsLongLong(args[3]), gs = PyLong_AsLongLong(args[4]);
         if (!x || !thr || !cb || !quantize_args_ok(*x, *thr, *cb, bits, gs)) return none();
-        Quantized q = quantize(*x, fptr(*thr), fptr(*cb), bits, gs, is_true(args[5]));
+        const bool bytes = is_true(args[5]);
+        Quantized q;
+        {
+            NoGil released;
+            q = quantize(*x, fptr(*thr), fptr(*cb), bits, gs, bytes);
+        }
         PyObject *list = PyList_New(4);
         if (!list) return nullptr;
         PyList_SET_ITEM(list, 0, THPVariable_Wrap(std::move(q.codes)));
@@ -874,78 +933,118 @@ PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t n)
     });
 }
 
+enum class Format { Fused, DequantGemm, Packed, Bytes };
+// ARCQPackedLinear's launches in one of its runtime formats; nullopt before the first where the call is not the plain case.
+std::optional<Tensor> run_packed(const Plan &plan, Format fmt, const Tensor &x)
+{
+    const int64_t K = plan.K, N = plan.N, m = x.numel() / K;
+    const int bits = static_cast<int>(plan.bits), gs = static_cast<int>(plan.gs);
+    const auto *p = plan.p;
+    auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
+    auto up = [&](int i) { return static_cast<const uint8_t *>(p[i]); };
+    at::DimVector sizes(x.sizes());
+    sizes.back() = N;
+    void *stream = stream_of(x);
+    if (fmt == Format::Fused) {
+        if (gs != 64 || !aligned16(x)) return std::nullopt;             // (the general path's stage 1 takes any alignment)
+        Tensor y = empty(sizes, at::kFloat, x.device());
+        if (prepare_pays(plan, x, m, false, false)) {
+            Tensor scratch = empty({N * K + m * K}, at::kHalf, x.device());
+            char *base = static_cast<char *>(scratch.mutable_data_ptr());
+            const Weights w{base, arcq_prepared_row_major(m, N, K) != 0};
+            run_prepare(x, m, plan, nullptr, base + N * K * 2, w, nullptr, nullptr, stream);
+            run_product(plan, m, base + N * K * 2, w, nullptr, false, nullptr, y.mutable_data_ptr(), ARCQ_F32, stream);
+            return y;
+        }
+        Tensor x_hat = empty({m * K}, at::kHalf, x.device());
+        check(arcq_linear_otf_ws(x.const_data_ptr(), ARCQ_F32, fp(A_THR), fp(A_CB), up(W_PACKED), fp(W_CB), fp(W_CENTER), fp(W_SCALE),
+                                 fp(W_SUM), fp(W_BIAS), x_hat.mutable_data_ptr(), nullptr, y.mutable_data_ptr(), ARCQ_F32, m, N, K, bits,
+                                 64, stream));
+        return y;
+    }
+    if (fmt == Format::DequantGemm) {
+        const Slot &dense = plan.slot[P_DENSE];
+        if (gs != 64 || dense.type != at::kHalf || dense.numel() != N * K) return std::nullopt;
+        Tensor x_hat = empty({m * K}, at::kHalf, x.device()), y = empty(sizes, at::kFloat, x.device());
+        check(arcq_act_quant_blocked(x.const_data_ptr(), ARCQ_F32, fp(A_THR), fp(A_CB), x_hat.mutable_data_ptr(), m, K, bits, 1.0e-6f, stream));
+        check(arcq_linear_fused_blocked(x_hat.const_data_ptr(), up(W_PACKED), fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS),
+                                        const_cast<void *>(dense.ptr()), 1, y.mutable_data_ptr(), ARCQ_F32, m, N, K, bits, 64, stream));
+        return y;
+    }
+    const bool bytes = fmt == Format::Bytes;
+    const Slot &table = plan.slot[P_TABLE];
+    if (table.sizes.size() != 2 || table.sizes[0] != table.sizes[1]) return std::nullopt;
+    if (plan.slot[A_CB].numel() != table.sizes[0] || plan.slot[W_CB].numel() != table.sizes[0]) return std::nullopt;
+    if (bytes && (!p[P_CODES] || plan.slot[P_CODES].numel() != N * K || plan.slot[P_CODES].type != at::kByte)) return std::nullopt;
+    const Tensor x2 = x.dim() == 2 ? x : x.view({m, K});
+    Quantized q = quantize(x2, fp(A_THR), fp(A_CB), bits, gs, bytes);
+    Tensor y = empty(sizes, at::kFloat, x.device());
+    arcq_linear_index_args a = {};
+    a.x_codes = bptr(q.codes), a.x_center = fptr(q.center), a.x_scale = fptr(q.scale), a.x_code_sum = fptr(q.sum);
+    a.w_codes = up(bytes ? P_CODES : W_PACKED), a.w_center = fp(W_CENTER), a.w_scale = fp(W_SCALE), a.w_code_sum = fp(W_SUM);
+    a.product_table = fp(P_TABLE), a.a_codebook = fp(A_CB), a.w_codebook = fp(W_CB), a.bias = fp(W_BIAS);
+    a.y = static_cast<float *>(y.mutable_data_ptr());
+    a.rows = m, a.out_features = N, a.in_features = K;
+    a.bits = bytes ? 0 : bits, a.group_size = gs, a.levels = static_cast<int>(table.sizes[0]);
+    check(arcq_linear_index(&a, stream));
+    return y;
+}
+
 // packed_forward(module, x): ARCQPackedLinear in its four runtime formats, group size 64 or (index-space formats) any
 PyObject *py_packed_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     return guarded([&]() -> PyObject * {
-        const Tensor *xp = n == 2 ? as_tensor(args[1]) : nullptr;
-        if (!xp) return none();
-        const Tensor &x = *xp;
+        const Tensor *x = n == 2 ? as_tensor(args[1]) : nullptr;
+        if (!x) return none();
         Refs refs;
         PyObject *dict;
         const auto plan = plan_of(args[0], Kind::Packed, refs, dict);
-        if (!plan || !here(x) || x.device().index() != plan->device || !f32(x) || !x.is_contiguous() || x.dim() < 1 ||
-            x.size(-1) != plan->K || x.numel() == 0)
+        if (!plan || !here(*x) || x->device().index() != plan->device || !f32(*x) || !x->is_contiguous() || x->dim() < 1 ||
+            x->size(-1) != plan->K || x->numel() == 0)
             return none();
         PyObject *fo = get(dict, S.runtime_code_format);
-        const char *fmt = fo && PyUnicode_Check(fo) ? PyUnicode_AsUTF8(fo) : nullptr;
-        if (!fmt) return none();
-        const int64_t K = plan->K, N = plan->N, m = x.numel() / K;
-        const int bits = static_cast<int>(plan->bits), gs = static_cast<int>(plan->gs);
-        const auto *p = plan->p;
-        auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
-        auto up = [&](int i) { return static_cast<const uint8_t *>(p[i]); };
-        at::DimVector sizes(x.sizes());
-        sizes.back() = N;
-        void *stream = stream_of(x);
-        if (strcmp(fmt, "hip_fused") == 0 || strcmp(fmt, "dequant_gemm") == 0) {
-            if (gs != 64) return none();
-            if (fmt[0] == 'h' && !aligned16(x)) return none();      // (the general path's stage 1 takes any alignment)
-            Tensor y = empty(sizes, at::kFloat, x.device());
-            if (fmt[0] == 'h' && prepare_pays(*plan, x, m, false, false)) {
-                Tensor scratch = empty({N * K + m * K}, at::kHalf, x.device());
-                char *base = static_cast<char *>(scratch.mutable_data_ptr());
-                const Weights w{base, arcq_prepared_row_major(m, N, K) != 0};
-                run_prepare(x, m, *plan, nullptr, 0, base + N * K * 2, w, nullptr, nullptr, stream);
-                run_product(*plan, m, base + N * K * 2, w, nullptr, false, nullptr, y.mutable_data_ptr(), ARCQ_F32, stream);
-                return THPVariable_Wrap(std::move(y));
-            }
-            Tensor x_hat = empty({m * K}, at::kHalf, x.device());
-            if (fmt[0] == 'h') {
-                check(arcq_linear_otf_ws(x.const_data_ptr(), ARCQ_F32, fp(A_THR), fp(A_CB), up(W_PACKED), fp(W_CB), fp(W_CENTER),
-                                         fp(W_SCALE), fp(W_SUM), fp(W_BIAS), x_hat.mutable_data_ptr(), nullptr,
-                                         y.mutable_data_ptr(), ARCQ_F32, m, N, K, bits, 64, stream));
-            } else {
-                const Slot &dense = plan->slot[P_DENSE];
-                if (dense.type != at::kHalf || dense.numel() != N * K) return none();
-                check(arcq_act_quant_blocked(x.const_data_ptr(), ARCQ_F32, fp(A_THR), fp(A_CB), x_hat.mutable_data_ptr(), m, K, bits,
-                                             1.0e-6f, stream));
-                check(arcq_linear_fused_blocked(x_hat.const_data_ptr(), up(W_PACKED), fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM),
-                                                fp(W_BIAS), const_cast<void *>(dense.ptr()), 1, y.mutable_data_ptr(),
-                                                ARCQ_F32, m, N, K, bits, 64, stream));
-            }
-            return THPVariable_Wrap(std::move(y));
+        const char *name = fo && PyUnicode_Check(fo) ? PyUnicode_AsUTF8(fo) : nullptr;
+        if (!name) return none();
+        Format fmt;
+        if (strcmp(name, "hip_fused") == 0) fmt = Format::Fused;
+        else if (strcmp(name, "dequant_gemm") == 0) fmt = Format::DequantGemm;
+        else if (strcmp(name, "packed") == 0) fmt = Format::Packed;
+        else if (strcmp(name, "u8") == 0) fmt = Format::Bytes;
+        else return none();
+        std::optional<Tensor> y;
+        {
+            NoGil released;
+            y = run_packed(*plan, fmt, *x);
         }
-        const bool bytes = strcmp(fmt, "u8") == 0;
-        if (!bytes && strcmp(fmt, "packed") != 0) return none();
-        const Slot &table = plan->slot[P_TABLE];
-        if (table.sizes.size() != 2 || table.sizes[0] != table.sizes[1]) return none();
-        if (plan->slot[A_CB].numel() != table.sizes[0] || plan->slot[W_CB].numel() != table.sizes[0]) return none();
-        if (bytes && (!p[P_CODES] || plan->slot[P_CODES].numel() != N * K || plan->slot[P_CODES].type != at::kByte)) return none();
-        const int levels = static_cast<int>(table.sizes[0]);
-        const Tensor x2 = x.dim() == 2 ? x : x.view({m, K});
-        Quantized q = quantize(x2, fp(A_THR), fp(A_CB), bits, gs, bytes);
-        Tensor y = empty(sizes, at::kFloat, x.device());
-        arcq_linear_index_args a = {};
-        a.x_codes = bptr(q.codes), a.x_center = fptr(q.center), a.x_scale = fptr(q.scale), a.x_code_sum = fptr(q.sum);
-        a.w_codes = up(bytes ? P_CODES : W_PACKED), a.w_center = fp(W_CENTER), a.w_scale = fp(W_SCALE), a.w_code_sum = fp(W_SUM);
-        a.product_table = fp(P_TABLE), a.a_codebook = fp(A_CB), a.w_codebook = fp(W_CB), a.bias = fp(W_BIAS);
-        a.y = static_cast<float *>(y.mutable_data_ptr());
-        a.rows = m, a.out_features = N, a.in_features = K;
-        a.bits = bytes ? 0 : bits, a.group_size = gs, a.levels = levels;
-        check(arcq_linear_index(&a, stream));
-        return THPVariable_Wrap(std::move(y));
+        return wrap(std::move(y));
     });
+}
+
+Tensor run_patches(const Plan &plan, const Tensor &x)
+{
+    const int64_t b = x.size(0), hp = x.size(2) / 16, wp = x.size(3) / 16, m = b * hp * wp, N = plan.N, K = 768;
+    const int bits = static_cast<int>(plan.bits);
+    auto fp = [&](int i) { return static_cast<const float *>(plan.p[i]); };
+    void *stream = stream_of(x);
+    Tensor y = empty({b, hp, wp, N}, x.scalar_type(), x.device());
+    if (can_prepare(plan, m)) {
+        Tensor scratch = empty({N * K + m * K}, at::kHalf, x.device());
+        char *base = static_cast<char *>(scratch.mutable_data_ptr());
+        const Weights w{base, arcq_prepared_row_major(m, N, K) != 0};
+        void *x_hat = base + N * K * 2;
+        arcq_prepare_weights pwt = {};
+        set_weights(pwt, plan, w);
+        check(arcq_prepare_patches(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), x_hat, b, 3, x.size(2), x.size(3), 16, bits, 1.0e-6f,
+                                   &pwt, stream));
+        run_product(plan, m, x_hat, w, nullptr, false, nullptr, y.mutable_data_ptr(), code_of(y), stream);
+        return y.permute({0, 3, 1, 2});
+    }
+    Tensor rows = empty({m * K}, at::kHalf, x.device());
+    check(arcq_act_quant_patches(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), rows.mutable_data_ptr(), b, 3, x.size(2), x.size(3), 16,
+                                 bits, 1.0e-6f, 0, stream));
+    check(arcq_linear_fused(rows.const_data_ptr(), static_cast<const uint8_t *>(plan.p[W_PACKED]), fp(W_CB), fp(W_CENTER), fp(W_SCALE),
+                            fp(W_SUM), fp(W_BIAS), y.mutable_data_ptr(), code_of(y), m, N, K, bits, 64, stream));
+    return y.permute({0, 3, 1, 2});
 }
 
 // patch_conv_forward(module, img): ARCQPackedPatchConv with 16 x 16 patches of three channels, group sizes 3 and 64
@@ -967,31 +1066,12 @@ PyObject *py_patch_conv_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
         if (!here(x) || x.device().index() != plan->device || (!f16(x) && !f32(x)) || !x.is_contiguous() || x.dim() != 4 ||
             x.size(1) != 3 || x.size(2) % 16 != 0 || x.size(3) % 16 != 0 || x.numel() == 0)
             return none();
-        const int64_t b = x.size(0), hp = x.size(2) / 16, wp = x.size(3) / 16, m = b * hp * wp, N = plan->N, K = 768;
-        const int bits = static_cast<int>(plan->bits);
-        const auto *p = plan->p;
-        auto fp = [&](int i) { return static_cast<const float *>(p[i]); };
-        const uint8_t *pw = static_cast<const uint8_t *>(p[W_PACKED]);
-        void *stream = stream_of(x);
-        Tensor y = empty({b, hp, wp, N}, x.scalar_type(), x.device());
-        if (can_prepare(*plan, m)) {
-            Tensor scratch = empty({N * K + m * K}, at::kHalf, x.device());
-            char *base = static_cast<char *>(scratch.mutable_data_ptr());
-            const Weights w{base, arcq_prepared_row_major(m, N, K) != 0};
-            void *x_hat = base + N * K * 2;
-            arcq_prepare_weights pwt = {};
-            set_weights(pwt, *plan, w);
-            check(arcq_prepare_patches(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), x_hat, b, 3, x.size(2), x.size(3), 16, bits,
-                                       1.0e-6f, &pwt, stream));
-            run_product(*plan, m, x_hat, w, nullptr, false, nullptr, y.mutable_data_ptr(), code_of(y), stream);
-            return THPVariable_Wrap(y.permute({0, 3, 1, 2}));
+        Tensor y;
+        {
+            NoGil released;
+            y = run_patches(*plan, x);
         }
-        Tensor rows = empty({m * K}, at::kHalf, x.device());
-        check(arcq_act_quant_patches(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), rows.mutable_data_ptr(), b, 3, x.size(2),
-                                     x.size(3), 16, bits, 1.0e-6f, 0, stream));
-        check(arcq_linear_fused(rows.const_data_ptr(), pw, fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS),
-                                y.mutable_data_ptr(), code_of(y), m, N, K, bits, 64, stream));
-        return THPVariable_Wrap(y.permute({0, 3, 1, 2}));
+        return THPVariable_Wrap(std::move(y));
     });
 }
 

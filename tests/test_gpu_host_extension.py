@@ -376,3 +376,81 @@ def test_out_of_memory_keeps_its_type(cuda, kind):
             layer(x)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+@pytest.mark.parametrize("kind", ["layer", "block", "packed", "quantize"])
+def test_other_threads_run_during_a_call(cuda, kind):
+    """A call that has to wait (here for memory: the allocator's cached segments are too small, and giving them back waits for
+    the GPU) does not hold the interpreter's lock meanwhile."""
+    import threading
+    import time
+    x = _tokens(1 << 18, 64, dtype=torch.float32)
+    if kind == "quantize":
+        cb = synth.quantile_codebook(4)
+        thr, cb = synth.midpoint_thresholds(cb).cuda(), cb.cuda()
+        wide = torch.randn(1 << 18, 1024, device=cuda)
+        call = lambda: A.quantize_activation_u8(wide, thr, cb, 4, 64)      # codes of 256 MiB
+        small = lambda: A.quantize_activation_u8(wide[:64], thr, cb, 4, 64)
+    elif kind == "block":
+        block, tokens = _vit().blocks[0], _tokens(1500, 197, 192)          # over 1 GiB of scratch
+        call, small = lambda: block(tokens), lambda: block(tokens[:1])
+    else:
+        layer = _on_the_fly(64, 1024) if kind == "layer" else _packed(64, 1024, kind)
+        call, small = lambda: layer(x), lambda: layer(x[:64])              # outputs of 512 MiB / 1 GiB
+    total = torch.cuda.get_device_properties(0).total_memory
+    longest, stop = [0.0], threading.Event()
+
+    def tick():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(0.001)
+            now = time.perf_counter()
+            longest[0], last = max(longest[0], now - last), now
+
+    with torch.no_grad():
+        small()
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        used = torch.cuda.memory_reserved()
+        segments = [torch.empty(100 << 20, dtype=torch.uint8, device=cuda) for _ in range(20)]
+        torch.cuda.set_per_process_memory_fraction((used + (2100 << 20)) / total)
+        del segments
+        ticker = threading.Thread(target=tick)
+        ticker.start()
+        try:
+            torch.cuda._sleep(500_000_000)                                 # GPU busy for some tenths of a second
+            start = time.perf_counter()
+            call()
+            took = time.perf_counter() - start
+        finally:
+            stop.set()
+            ticker.join()
+            torch.cuda.synchronize()
+            torch.cuda.set_per_process_memory_fraction(1.0)
+    if took < 0.05:
+        pytest.skip("the call did not have to wait")
+    assert longest[0] < took / 2, (took, longest[0])
+
+
+def test_one_layer_from_several_threads(cuda):
+    """Threads on streams of their own call one model; each gets its own input's result."""
+    import threading
+    vit = _vit(own_attention=True, fuse_elementwise=True)
+    inputs = [_tokens(3, 197, 192, seed=s) for s in range(4)]
+    with torch.no_grad():
+        want = [vit.blocks(x).clone() for x in inputs]
+    torch.cuda.synchronize()
+    failures = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()), torch.no_grad():
+            for _ in range(30):
+                if not torch.equal(vit.blocks(inputs[i]), want[i]):
+                    failures.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(inputs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures
