@@ -9,6 +9,7 @@ import ctypes
 import os
 import sys
 import threading
+import warnings
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libarcq_hip.so")
@@ -171,17 +172,30 @@ def load() -> ctypes.CDLL:
 _host = None
 
 
+class _NoHost:
+    """In the place of the host extension where that does not load: every call is left to the Python code behind it."""
+
+    def _leave(*args):
+        return None
+
+    layer_forward = block_forward = attention = patch_embed = quantize = packed_forward = patch_conv_forward = _leave
+
+
 def host():
-    """The CPython extension with the host side of the hot calls (``csrc_host/arcq_host.cpp``); as loud as ``load`` if it
-    has not been built.  Its functions return None for calls they leave to the Python code."""
+    """The CPython extension with the host side of the hot calls (``csrc_host/arcq_host.cpp``).  Its functions return None for
+    calls they leave to the Python code.  It is built against one torch; where it does not load, the same kernels are called
+    through ctypes (slower in host time and, for whole blocks, in launches), which is said once.  Without the library itself
+    this raises, as ``load`` does."""
     global _host
     if _host is None:
         load()
         try:
             from . import _arcq_host as mod
         except ImportError as e:
-            raise ARCQLibraryMissing(f"ARCQ host extension is not built or does not load ({e}). "
-                                     "Run `python -m arcq_vit_amd.build` first.") from e
+            warnings.warn(f"ARCQ host extension is not built or does not load ({e}); the kernels are called through ctypes, which "
+                          "is slower. Run `python -m arcq_vit_amd.build` to build it.", RuntimeWarning, stacklevel=3)
+            _host = _NoHost
+            return _host
         import torch
         from . import ops, vit
         from .packed_on_the_fly import ARCQPackedLinearOnTheFly
@@ -189,6 +203,13 @@ def host():
                            sys.modules["torch.nn.modules.module"], ops.fp8_weight_multiplier)
         _host = mod
     return _host
+
+
+def host_for_block():
+    """``host()`` for a module that need not hold a packed layer: it runs without the library too."""
+    if _host is None and not os.path.exists(LIB_PATH):
+        return _NoHost
+    return host()
 
 
 def check(rc: int) -> None:

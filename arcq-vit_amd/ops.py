@@ -53,17 +53,21 @@ def _f32c(t: torch.Tensor) -> torch.Tensor:
 
 def _check_weights(n: int, k: int, group_size: int, center: torch.Tensor, scale: torch.Tensor, code_sum: torch.Tensor,
                    bias: Optional[torch.Tensor]) -> None:
-    """The per-group metadata and the bias hold at least what the kernels read for ``[n, k]`` weights."""
+    """The per-group metadata and the bias are on a GPU and hold at least what the kernels read for ``[n, k]`` weights."""
     need = n * (k // max(int(group_size), 1))
     for name, t in (("w_center", center), ("w_scale", scale), ("w_code_sum", code_sum)):
+        _check(t.is_cuda, f"{name} must be CUDA tensor")
         _check(t.numel() >= need, f"{name} has {t.numel()} entries, {need} needed for [out_features, groups]")
-    _check(bias is None or bias.numel() == 0 or bias.numel() >= n, "bias must have out_features entries")
+    if bias is not None and bias.numel() > 0:
+        _check(bias.is_cuda, "bias must be CUDA tensor")
+        _check(bias.numel() >= n, "bias must have out_features entries")
 
 
 def _check_codebooks(bits: int, w_codebook: Optional[torch.Tensor], a_thresholds: Optional[torch.Tensor] = None,
                      a_codebook: Optional[torch.Tensor] = None) -> None:
     for name, t, need in (("w_codebook", w_codebook, 1 << bits), ("a_thresholds", a_thresholds, (1 << bits) - 1),
                           ("a_codebook", a_codebook, 1 << bits)):
+        _check(t is None or t.is_cuda, f"{name} must be CUDA tensor")
         _check(t is None or t.numel() >= need, f"{name} must have {need} entries for {bits}-bit codes")
 
 
@@ -724,7 +728,9 @@ def _check_index(rows: int, out_features: int, in_features: int, group_size: int
                  w_scale, w_code_sum, product_table, bias) -> None:
     _check_weights(out_features, in_features, group_size, w_center, w_scale, w_code_sum, bias)
     need = rows * (in_features // int(group_size))
-    _check(all(t.numel() >= need for t in (x_center, x_scale, x_code_sum)), "x_center, x_scale and x_code_sum must be [rows, groups]")
+    _check(all(t.is_cuda and t.numel() >= need for t in (x_center, x_scale, x_code_sum)),
+           "x_center, x_scale and x_code_sum must be CUDA tensors [rows, groups]")
+    _check(product_table.is_cuda, "product_table must be CUDA tensor")
     _check(product_table.dim() == 2 and product_table.shape[0] == product_table.shape[1], "product_table must be square")
 
 

@@ -31,7 +31,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
-from . import _lib
+from . import _lib, ops
 
 
 def clear_workspaces() -> None:
@@ -73,6 +73,7 @@ class ARCQPackedLinearOnTheFly(nn.Module):
             self.register_buffer("bias_tensor", torch.empty(0))
         self.out_dtype = torch.float16
         self._host_plan = None      # the host extension's view of the buffers above, made by the first forward
+        self._fp8_mult = None       # what _fp8_multiplier keeps (without the extension)
         # Opt-in: operands rounded to FP8 and the product on FP8 matrix units (ops.linear_otf_fp8).  Faster on the
         # large models, not the reference's numerics; see set_fp8_operands in packed_convert.
         self.fp8_operands = False
@@ -94,7 +95,7 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         # then widens these buffers again, scripts/benchmark_arcq_on_the_fly.py:63-85, which leaves
         # them rounded to fp16.)  Device moves still apply; dtype changes of these buffers do not.
         keep = {n: self._buffers[n] for n in self._FP32_BUFFERS if self._buffers.get(n) is not None}
-        self._host_plan = None          # and with it the copies it holds where they were
+        self._host_plan = self._fp8_mult = None         # and with them what they hold where the layer was
         super()._apply(fn, *args, **kwargs)
         for name, orig in keep.items():
             new = self._buffers[name]
@@ -103,7 +104,7 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         return self
 
     def _load_from_state_dict(self, *args, **kwargs):
-        self._host_plan = None
+        self._host_plan = self._fp8_mult = None
         return super()._load_from_state_dict(*args, **kwargs)
 
     def can_quantize_for(self, consumer: nn.Module, rows: int) -> bool:
@@ -198,9 +199,46 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         with torch.cuda.device(x2.device):
             y = _lib.host().layer_forward(self, x2, layernorm, activation == "gelu", residual, quantize_for, input_is_xhat)
         if y is None:
-            raise RuntimeError("x and the layer's buffers must be contiguous CUDA tensors of the types and shapes the layer was "
-                               "built with")
+            y = self._forward_ops(x2, layernorm, activation, residual, quantize_for, input_is_xhat)
         return y.reshape(*original_shape[:-1], self.out_features)
+
+    def _forward_ops(self, x2, layernorm, activation, residual, quantize_for, input_is_xhat) -> torch.Tensor:
+        """The same layer through the operators: without the host extension, and for what it does not take (which the operators
+        refuse, saying why)."""
+        if tuple(self.packed_weight_codes.shape) != (self.out_features, (self.in_features * self.bits + 7) // 8):
+            raise RuntimeError(f"packed_weight_codes has shape {tuple(self.packed_weight_codes.shape)}, which is not the layer's")
+        if any(b.numel() > 0 and b.device != x2.device for b in self._buffers.values()):
+            raise RuntimeError("x and the layer's buffers must be on the same device")
+        args = (x2, self.activation_thresholds, self.activation_codebook, self.packed_weight_codes, self.weight_codebook,
+                self.weight_center, self.weight_scale, self.weight_code_sum, self.bias_tensor, self.bits)
+        if self.fp8_operands:
+            return ops.linear_otf_fp8(*args, out_dtype=self.out_dtype, w_mult=self._fp8_multiplier())
+        xh_ws, w_ws = getattr(self, "_x_hat_buffer", None), getattr(self, "_weight_buffer", None)
+        if (xh_ws is not None and (xh_ws.dtype != torch.float16 or not xh_ws.is_contiguous() or xh_ws.numel() < x2.numel()
+                                   or xh_ws.device != x2.device)):
+            xh_ws = None
+        common = dict(out_dtype=self.out_dtype, x_hat_ws=xh_ws, w_hat_ws=w_ws)
+        if layernorm is None and activation is None and residual is None and quantize_for is None and not input_is_xhat:
+            return ops.linear_otf(*args, self.group_size, scratch=True, **common)
+        ln = None
+        if layernorm is not None:
+            bias = torch.zeros_like(layernorm.weight) if layernorm.bias is None else layernorm.bias
+            ln = (layernorm.weight.detach(), bias.detach(), layernorm.eps)
+        following = None if quantize_for is None else (quantize_for.activation_thresholds, quantize_for.activation_codebook)
+        return ops.linear_otf_ex(*args, self.group_size, layernorm=ln, gelu=activation == "gelu", residual=residual,
+                                 next_quant=following, x_is_xhat=bool(input_is_xhat), **common)
+
+    def _fp8_multiplier(self) -> float:
+        """``ops.fp8_weight_multiplier`` of the layer, read back once per set of buffers (they are held, so that their addresses
+        name them); at every call where they are inference tensors, whose changes in place leave no trace."""
+        meta = (self.weight_codebook, self.weight_center, self.weight_scale, self.weight_code_sum)
+        if any(t.is_inference() for t in meta):
+            return ops.fp8_weight_multiplier(*meta)
+        key = tuple((t.data_ptr(), t._version) for t in meta)
+        kept = self.__dict__.get("_fp8_mult")
+        if kept is None or kept[0] != key:
+            kept = self._fp8_mult = (key, ops.fp8_weight_multiplier(*meta), tuple(t.detach() for t in meta))
+        return kept[1]
 
     def estimated_persistent_mb(self) -> float:
         """MiB held by this layer's buffers (FQ/arcq_packed_on_the_fly.py:163-169)."""

@@ -27,6 +27,7 @@ def cuda():
         pytest.skip("no GPU")
     from arcq_vit_amd import _lib
     _lib.load()  # raises if the HIP library is not built: GPU tests must not pass without it
+    assert _lib.host() is not _lib._NoHost, "the host extension does not load"
     return torch.device("cuda:0")
 
 

@@ -258,8 +258,9 @@ def _cut(t):
 
 
 @pytest.mark.parametrize("fmt", ["packed", "u8", "dequant_gemm", "hip_fused", "on_the_fly", "conv"])
-def test_buffers_replaced_by_smaller_ones_are_refused(cuda, fmt):
-    """The kernels read what the layer's sizes say; a buffer that holds less is refused before anything is launched."""
+def test_buffers_replaced_by_unfit_ones_are_refused(cuda, fmt):
+    """The kernels read what the layer's sizes say; a buffer that holds less, or lies in host memory, is refused before anything
+    is launched."""
     if fmt == "conv":
         src = A.QuantConv2dPCARCQ(3, 64, 16, 16, 0, True, 4, 4, 64)
         for q in (src.act_quant, src.weight_quant):
@@ -277,7 +278,7 @@ def test_buffers_replaced_by_smaller_ones_are_refused(cuda, fmt):
             want = layer(x)
             for name in names:
                 good = layer._buffers[name]
-                bad = [_cut(good)] + ([good[:, :-1].contiguous()] if good.dim() == 2 else [])
+                bad = [_cut(good), good.cpu()] + ([good[:, :-1].contiguous()] if good.dim() == 2 else [])
                 for b in bad:
                     layer._buffers[name] = b
                     with pytest.raises(RuntimeError):
@@ -454,3 +455,53 @@ def test_one_layer_from_several_threads(cuda):
     for t in threads:
         t.join()
     assert not failures
+
+
+def _without_extension(monkeypatch):
+    from arcq_vit_amd import _lib
+    monkeypatch.setattr(_lib, "_host", _lib._NoHost)
+
+
+@pytest.mark.parametrize("m,k,n,bits", [(1, 64, 64, 2), (197, 192, 768, 4), (197, 768, 3072, 3), (394, 1024, 1024, 4), (1000, 384, 1152, 4),
+                                        (600, 1536, 200, 3)])
+def test_layers_without_the_extension(cuda, monkeypatch, m, k, n, bits):
+    """The same kernels through ctypes: the bits of the extension's calls, for every form of a layer's call."""
+    layer, norm = _on_the_fly(k, n, bits), torch.nn.LayerNorm(k).cuda().half()
+    following = _on_the_fly(n, 64, bits) if n % 64 == 0 else None
+    layer._weight_buffer = torch.zeros(n * k, dtype=torch.float16, device=cuda)
+    x, skip = _tokens(m, k), _tokens(m, n, seed=4)
+
+    def results():
+        out = [layer(x), layer(x.float()), layer(x, activation="gelu"), layer(x, residual=skip), layer(x, layernorm=norm),
+               layer(x, layernorm=norm, activation="gelu", residual=skip)]
+        if following is not None and layer.can_quantize_for(following, m):
+            out.append(following(layer(x, layernorm=norm, activation="gelu", quantize_for=following), input_is_xhat=True))
+        layer.fp8_operands = True
+        out += [layer(x), layer(x, residual=skip)]
+        layer.fp8_operands = False
+        return out
+
+    with torch.no_grad():
+        want = results()
+        _without_extension(monkeypatch)
+        got = results()
+    assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("batch", [1, 5, 40])
+def test_blocks_without_the_extension(cuda, monkeypatch, batch, fused):
+    block, x = _vit(fuse_elementwise=fused, own_attention=fused).blocks[0], _tokens(batch, 197, 192)
+    with torch.no_grad():
+        want = block(x)
+        _without_extension(monkeypatch)
+        assert torch.equal(block(x), want)
+
+
+@pytest.mark.parametrize("fmt", ["packed", "u8", "dequant_gemm", "hip_fused"])
+def test_formats_without_the_extension(cuda, monkeypatch, fmt):
+    layer, xs = _packed(768, 256, fmt), [_tokens(m, 768, dtype=torch.float32) for m in (7, 600)]
+    with torch.no_grad():
+        want = [layer(x) for x in xs]
+        _without_extension(monkeypatch)
+        assert all(torch.equal(layer(x), y) for x, y in zip(xs, want))

@@ -543,3 +543,25 @@ def test_blocks_trace_symbolically():
     packed = build_packed_vit("deit_tiny", 4, depth=1, num_classes=4, device="cpu")
     leaves = [n.target for n in Tracer().trace(packed.blocks[0]).nodes if n.op == "call_module"]
     assert leaves == ["norm1", "attn.qkv", "attn.proj", "norm2", "mlp.fc1", "mlp.act", "mlp.fc2"]
+
+
+def test_a_host_extension_that_does_not_load_is_said_and_done_without(monkeypatch):
+    """Built against another torch, or not built: the Python code behind it takes every call; without the library itself the
+    packed layers still refuse to run."""
+    import sys
+    from arcq_vit_amd import _lib, vit
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setitem(sys.modules, "arcq_vit_amd._arcq_host", None)       # importing it raises ImportError
+    monkeypatch.delattr(sys.modules["arcq_vit_amd"], "_arcq_host", raising=False)
+    with pytest.warns(RuntimeWarning, match="host extension is not built or does not load"):
+        host = _lib.host()
+    assert host.block_forward(None, None) is None and host.layer_forward(1, 2, 3, 4, 5, 6, 7) is None
+    assert _lib.host() is host
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", "/nonexistent/libarcq_hip.so")
+    with pytest.raises(_lib.ARCQLibraryMissing):
+        _lib.host()
+    assert _lib.host_for_block().block_forward(None, None) is None           # a floating-point block needs neither
+    with pytest.raises(_lib.ARCQLibraryMissing):
+        A.ARCQPackedLinear(_source())(torch.zeros(2, 128))
