@@ -623,7 +623,6 @@ bool read_layernorm(PyObject *d, LayerNorm &out)
 
 // A block on prepared operands: [LayerNorm + stage 1, weights of qkv and proj] -> qkv -> attention ending with proj's stage 1
 // -> proj + skip -> [LayerNorm + stage 1, weights of fc1 and fc2] -> fc1 + GELU + fc2's stage 1 -> fc2 + skip: seven launches.
-// All intermediate tensors come from the caching allocator, w_hat of two layers at a time included.
 //   fused == false: the LayerNorms are torch's (own launches); everything else that is folded into the products (skips, GELU,
 //                   fc2's stage 1) gives the bits of the separate kernels anyway
 //   fp8:            FP8 operands.  LayerNorms as torch runs them: that is what the layers do one by one, and a network of
@@ -655,14 +654,19 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
     auto layout = [&](const Plan &p) { return arcq_prepared_row_major(rows, p.N, p.K) != 0; };
     auto weight_bytes = [&](const Plan &p) { return p.N * operand_row_bytes(p.K, fp8); };
     const int64_t wq = weight_bytes(pq), wp = weight_bytes(pp), w1 = weight_bytes(pf1), w2 = weight_bytes(pf2);
-    Tensor w = empty({std::max(wq + wp, w1 + w2)}, at::kByte, x.device());
-    char *wb = static_cast<char *>(w.mutable_data_ptr());
-    Tensor xh = empty({rows * operand_row_bytes(C, fp8)}, at::kByte, x.device());
-    Tensor wide = empty({rows * operand_row_bytes(pf2.K, fp8)}, at::kByte, x.device());       // fc1's quantized output
+    // Scratch from the layers' lent buffers where they have room, else from the allocator.  Two weights are in use at a time, and
+    // fc1 reads its x_hat while it writes fc2's: of a pair that shares a buffer one lies elsewhere (fc1's x_hat where qkv was).
+    auto scratch = [&](const Tensor &buffer, int64_t bytes) {
+        return lent(buffer, (bytes + 1) / 2, x) && aligned16(buffer) ? buffer : empty({bytes}, at::kByte, x.device());
+    };
+    auto at_byte = [](const Tensor &t, int64_t i) { return static_cast<char *>(t.mutable_data_ptr()) + i; };
+    const Tensor w_attn = scratch(k.qkv.weight_buffer, wq + wp), xh = scratch(k.qkv.x_hat_buffer, rows * operand_row_bytes(C, fp8));
+    const Tensor wide = scratch(k.fc2.x_hat_buffer, rows * operand_row_bytes(pf2.K, fp8));         // fc1's quantized output
+    const Tensor w_fc1 = scratch(k.fc1.weight_buffer, w1), w_fc2 = empty({w2}, at::kByte, x.device());
     Tensor qkv = empty({b, n, pq.N}, at::kHalf, x.device());
     Tensor x1 = empty(x.sizes(), at::kHalf, x.device()), y = empty(x.sizes(), at::kHalf, x.device());
-    const Weights hq{wb, layout(pq), fp8, k.qkv.fp8_mult}, hp{wb + wq, layout(pp), fp8, k.proj.fp8_mult},
-                  h1{wb, layout(pf1), fp8, k.fc1.fp8_mult}, h2{wb + w1, layout(pf2), fp8, k.fc2.fp8_mult};
+    const Weights hq{at_byte(w_attn, 0), layout(pq), fp8, k.qkv.fp8_mult}, hp{at_byte(w_attn, wq), layout(pp), fp8, k.proj.fp8_mult},
+                  h1{at_byte(w_fc1, 0), layout(pf1), fp8, k.fc1.fp8_mult}, h2{at_byte(w_fc2, 0), layout(pf2), fp8, k.fc2.fp8_mult};
     run_prepare(t, rows, pq, fuse_ln ? &k.fused1 : nullptr, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
     run_product(pq, rows, xh.const_data_ptr(), hq, nullptr, false, nullptr, qkv.mutable_data_ptr(), ARCQ_F16, stream);
     if (own_attention) {
@@ -674,8 +678,8 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
     }
     run_product(pp, rows, xh.const_data_ptr(), hp, &x, false, nullptr, x1.mutable_data_ptr(), ARCQ_F16, stream);
     t = fuse_ln ? x1 : k.norm2(x1);
-    run_prepare(t, rows, pf1, fuse_ln ? &k.fused2 : nullptr, xh.mutable_data_ptr(), h1, &pf2, &h2, stream);
-    run_product(pf1, rows, xh.const_data_ptr(), h1, nullptr, true, &pf2, wide.mutable_data_ptr(), ARCQ_F16, stream);
+    run_prepare(t, rows, pf1, fuse_ln ? &k.fused2 : nullptr, qkv.mutable_data_ptr(), h1, &pf2, &h2, stream);
+    run_product(pf1, rows, qkv.const_data_ptr(), h1, nullptr, true, &pf2, wide.mutable_data_ptr(), ARCQ_F16, stream);
     run_product(pf2, rows, wide.const_data_ptr(), h2, &x1, false, nullptr, y.mutable_data_ptr(), ARCQ_F16, stream);
     return y;
 }

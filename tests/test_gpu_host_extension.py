@@ -505,3 +505,36 @@ def test_formats_without_the_extension(cuda, monkeypatch, fmt):
         want = [layer(x) for x in xs]
         _without_extension(monkeypatch)
         assert all(torch.equal(layer(x), y) for x, y in zip(xs, want))
+
+
+@pytest.mark.parametrize("fused,fp8", [(False, False), (True, False), (True, True)])
+def test_blocks_use_the_lent_buffers(cuda, fused, fp8):
+    """With `share_buffers` a forward's peak holds no second copy of what was lent; the results are those without."""
+    from arcq_vit_amd.packed_convert import set_fp8_operands, share_buffers
+    vit, x = _vit(fuse_elementwise=fused, own_attention=True), _tokens(32, 197, 192)
+    if fp8:
+        set_fp8_operands(vit)
+    rows = 32 * 197
+
+    def peak():
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        y = vit.blocks(x)
+        torch.cuda.synchronize()
+        return y, torch.cuda.max_memory_allocated() - before
+
+    with torch.no_grad():
+        vit.blocks(x)
+        want, alone = peak()
+        share_buffers(vit, rows)
+        got, lent = peak()
+        assert torch.equal(got, want)
+        unit = rows * 192 * (1 if fp8 else 2)                             # x_hat of 192 values: one unit, fc2's: four
+        assert lent <= alone - 5 * unit + (1 << 20), (alone / unit, lent / unit)
+        share_buffers(vit, rows - 1)                                      # too small for fc2's x_hat: allocated again
+        assert torch.equal(vit.blocks(x), want)
+        for other in (torch.zeros(10, device=cuda), None):                # no fp16 buffer; none
+            for layer in (vit.blocks[0].attn.qkv, vit.blocks[0].mlp.fc2):
+                layer._x_hat_buffer = other
+            assert torch.equal(vit.blocks(x), want)
