@@ -645,10 +645,18 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
     if ((fuse_ln && C > 2048) || pf1.N % 64 != 0 || !aligned16(x)) return std::nullopt;      // (x is also proj's residual)
     for (const Plan *p : {&pq, &pp, &pf1, &pf2})
         if (!can_prepare(*p, rows) || p->bits != pq.bits) return std::nullopt;
-    // Not where the one-launch layer kernels are at their best (one 64-row tile on most compute units, short rows): DeiT-S at
-    // 12 608 rows 1 625 us a forward against 1 939, DeiT-B 3 969 against 4 373; at 9 456 rows 4 % either way, below and above
-    // that range the seven launches win (6 304 rows: 1 353 -> 1 262 us; 25 216 rows: 3 341 -> 3 286).
-    if (fuse_ln && rows > 9000 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) return std::nullopt;
+    // Not where the one-launch layer kernels are at their best (one 64-row tile on most compute units, short rows).  With the
+    // LayerNorms inside: DeiT-S at 12 608 rows 1 625 us a forward against 1 939, DeiT-B 3 969 against 4 373; at 9 456 rows 4 %
+    // either way, below and above that range the seven launches win (6 304 rows: 1 353 -> 1 262 us; 25 216 rows: 3 341 -> 3 286).
+    // With torch's LayerNorms and GELU those kernels run only on lent weight buffers, and win later and only beside torch's
+    // attention: 10 638 rows DeiT-S 2 311 us against 2 264 here, DeiT-B 4 498 / 4 406, 11 032 rows 2 318 / 2 439 and 4 607 / 4 879,
+    // 12 608 rows 2 399 / 2 564 and 4 892 / 5 147; without lent buffers (two launches a layer) 2 667 / 2 590 and 5 207 / 5 178, with
+    // the library's attention, which takes proj's stage 1 along, 2 285 / 2 263 and 4 740 / 4 679, with more than one tile on a
+    // compute unit (DeiT-Tiny, 17 730 rows) 2 287 / 2 201.
+    if (!fp8 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) {
+        const bool lends = k.qkv.lends && k.proj.lends && k.fc1.lends && k.fc2.lends;
+        if (fuse_ln ? rows > 9000 : lends && !own_attention && rows > 10800 && rows <= 16384) return std::nullopt;
+    }
     Tensor t = fuse_ln ? x : k.norm1(x);
     void *stream = stream_of(x);
     auto layout = [&](const Plan &p) { return arcq_prepared_row_major(rows, p.N, p.K) != 0; };
