@@ -18,6 +18,7 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/GradMode.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/DynamicTypes.h>
@@ -162,6 +163,9 @@ struct Slot {
     const void *ptr() const { return copy.defined() ? copy.const_data_ptr() : data; }
     int64_t numel() const { return c10::multiply_integers(sizes); }
 };
+// Copies made while the stream is captured belong to the graph: nothing has run that fills them, and their memory is the graph's.
+// Such a call uses them and keeps nothing.
+inline bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 // References to Python objects for the length of a call (the GIL is held where it is made and where it ends).
 struct Refs {
     c10::SmallVector<PyObject *, 64> held;      // (a block: four layers, two LayerNorms, nine modules)
@@ -283,6 +287,7 @@ std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, Refs &refs, PyObject 
         plan->p[i] = t[i]->numel() ? plan->slot[i].ptr() : nullptr;
     }
     plan->device = dev.index();
+    if (std::any_of(plan->slot, plan->slot + n, [](const Slot &s) { return s.copy.defined(); }) && capturing()) return plan;
     PlanObject *fresh = reinterpret_cast<PlanObject *>(plan_new(&PlanType, nullptr, nullptr));
     if (!fresh) throw Failure{};
     fresh->plan = plan;
@@ -313,19 +318,22 @@ bool read_fused_layernorm(Plan &plan, PyObject *ln, Refs &refs, FusedLayerNorm &
     refs.add(get(params, S.weight));
     refs.add(bo);
     out.eps = static_cast<float>(PyFloat_AS_DOUBLE(e));
+    LayerNormParams p;
     const LayerNormParams *found = nullptr;
-    for (const auto &p : plan.ln)
-        if (p.w.same(*w) && p.has_bias() == (b != nullptr) && (!b || p.b.same(*b))) found = &p;
+    for (const auto &q : plan.ln)
+        if (q.w.same(*w) && q.has_bias() == (b != nullptr) && (!b || q.b.same(*b))) found = &q;
     if (!found) {
         if (!w->is_cuda() || w->device().index() != plan.device || w->numel() != plan.K || w->dim() != 1) return false;
         if (b && (b->device() != w->device() || b->numel() != plan.K)) return false;
-        LayerNormParams p;
         p.w.set(*w, true, true);
         if (b) p.b.set(*b, true, true);
         else p.no_bias = at::zeros({plan.K}, w->options().dtype(at::kFloat).requires_grad(false));
-        if (plan.ln.size() >= 4) plan.ln.clear();        // (a layer has one LayerNorm in front of it; a bound, not a policy)
-        plan.ln.push_back(std::move(p));
-        found = &plan.ln.back();
+        found = &p;
+        if (!(p.w.copy.defined() || p.b.copy.defined() || p.no_bias.defined()) || !capturing()) {
+            if (plan.ln.size() >= 4) plan.ln.clear();        // (a layer has one LayerNorm in front of it; a bound, not a policy)
+            plan.ln.push_back(std::move(p));
+            found = &plan.ln.back();
+        }
     }
     out.weight = found->weight(), out.weight_copy = found->w.copy;
     out.bias = found->bias(), out.bias_copy = found->has_bias() ? found->b.copy : found->no_bias;

@@ -560,3 +560,28 @@ def test_default_blocks_choose_the_faster_launches(cuda, batch, buffers, own, la
         one_by_one = "CUDAFunctor_add" in _kernels(lambda: block(x))      # torch's skip connections
         assert one_by_one == layers
         assert torch.equal(block(x), _interpreted(block, x))
+
+
+def test_copies_made_during_capture_stay_in_the_graph(cuda):
+    """A first call under capture records the conversion of its metadata and LayerNorm parameters; an eager call in front of the
+    first replay makes its own."""
+    x, norm = _tokens(197, 192), torch.nn.LayerNorm(192).cuda().half()
+    with torch.no_grad():
+        norm.weight.uniform_(0.5, 1.5)
+        scale = _on_the_fly(192, 768).weight_scale.half()
+        layers = [_on_the_fly(192, 768) for _ in range(2)]
+        for layer in layers:
+            layer.weight_scale = scale
+        want = layers[0](x, layernorm=norm)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = layers[1](x, layernorm=norm)
+        assert torch.equal(layers[1](x, layernorm=norm), want)
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            assert torch.equal(layers[1](x, layernorm=norm), want) and torch.equal(y, want)
+        del graph, y
+        torch.cuda.empty_cache()
+        assert torch.equal(layers[1](x, layernorm=norm), want)
