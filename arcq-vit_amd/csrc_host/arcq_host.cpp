@@ -166,6 +166,17 @@ struct Slot {
 // Copies made while the stream is captured belong to the graph: nothing has run that fills them, and their memory is the graph's.
 // Such a call uses them and keeps nothing.
 inline bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+// The stream that fills a set of copies, until they are known to be filled: the first call from another stream waits for it.
+// (A capture begins with a synchronised device, and may not wait.)
+struct FilledOn {
+    std::optional<c10::hip::HIPStream> stream;
+    void settle()
+    {
+        if (!stream || *stream == c10::hip::getCurrentHIPStream(stream->device_index()) || capturing()) return;
+        stream->synchronize();
+        stream.reset();
+    }
+};
 // References to Python objects for the length of a call (the GIL is held where it is made and where it ends).
 struct Refs {
     c10::SmallVector<PyObject *, 64> held;      // (a block: four layers, two LayerNorms, nine modules)
@@ -181,6 +192,8 @@ struct Refs {
 struct LayerNormParams {
     Slot w, b;
     Tensor no_bias;           // zeros, for a LayerNorm without one
+    FilledOn filled;
+    bool copied() const { return w.copy.defined() || b.copy.defined() || no_bias.defined(); }
     bool has_bias() const { return !no_bias.defined(); }
     const float *weight() const { return static_cast<const float *>(w.ptr()); }
     const float *bias() const { return has_bias() ? static_cast<const float *>(b.ptr()) : fptr(no_bias); }
@@ -191,6 +204,7 @@ struct Plan {
     int64_t K = 0, N = 0, bits = 0, gs = 0;
     Slot slot[kMaxSlots];
     const void *p[kMaxSlots] = {};
+    FilledOn filled;
     double fp8_mult = NAN;
     std::vector<LayerNormParams> ln;
 };
@@ -265,7 +279,10 @@ std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, Refs &refs, PyObject 
         refs.add(o);
         same = same && plan->slot[i].same(*t[i]);
     }
-    if (same) return plan;
+    if (same) {
+        plan->filled.settle();
+        return plan;
+    }
     plan = std::make_shared<Plan>();
     const c10::Device dev = t[W_PACKED]->device();
     for (int i = 0; i < n; ++i) {
@@ -287,7 +304,10 @@ std::shared_ptr<Plan> plan_of(PyObject *module, Kind kind, Refs &refs, PyObject 
         plan->p[i] = t[i]->numel() ? plan->slot[i].ptr() : nullptr;
     }
     plan->device = dev.index();
-    if (std::any_of(plan->slot, plan->slot + n, [](const Slot &s) { return s.copy.defined(); }) && capturing()) return plan;
+    if (std::any_of(plan->slot, plan->slot + n, [](const Slot &s) { return s.copy.defined(); })) {
+        if (capturing()) return plan;
+        plan->filled.stream = c10::hip::getCurrentHIPStream(plan->device);
+    }
     PlanObject *fresh = reinterpret_cast<PlanObject *>(plan_new(&PlanType, nullptr, nullptr));
     if (!fresh) throw Failure{};
     fresh->plan = plan;
@@ -319,8 +339,8 @@ bool read_fused_layernorm(Plan &plan, PyObject *ln, Refs &refs, FusedLayerNorm &
     refs.add(bo);
     out.eps = static_cast<float>(PyFloat_AS_DOUBLE(e));
     LayerNormParams p;
-    const LayerNormParams *found = nullptr;
-    for (const auto &q : plan.ln)
+    LayerNormParams *found = nullptr;
+    for (auto &q : plan.ln)
         if (q.w.same(*w) && q.has_bias() == (b != nullptr) && (!b || q.b.same(*b))) found = &q;
     if (!found) {
         if (!w->is_cuda() || w->device().index() != plan.device || w->numel() != plan.K || w->dim() != 1) return false;
@@ -329,12 +349,14 @@ bool read_fused_layernorm(Plan &plan, PyObject *ln, Refs &refs, FusedLayerNorm &
         if (b) p.b.set(*b, true, true);
         else p.no_bias = at::zeros({plan.K}, w->options().dtype(at::kFloat).requires_grad(false));
         found = &p;
-        if (!(p.w.copy.defined() || p.b.copy.defined() || p.no_bias.defined()) || !capturing()) {
+        if (!p.copied() || !capturing()) {
+            if (p.copied()) p.filled.stream = c10::hip::getCurrentHIPStream(plan.device);
             if (plan.ln.size() >= 4) plan.ln.clear();        // (a layer has one LayerNorm in front of it; a bound, not a policy)
             plan.ln.push_back(std::move(p));
             found = &plan.ln.back();
         }
     }
+    found->filled.settle();
     out.weight = found->weight(), out.weight_copy = found->w.copy;
     out.bias = found->bias(), out.bias_copy = found->has_bias() ? found->b.copy : found->no_bias;
     return true;
@@ -347,7 +369,7 @@ struct Layer {                   // what a call needs of an ARCQPackedLinearOnTh
     bool fp8 = false;
     float fp8_mult = 1.0f;
     bool lends = false;                     // has a _weight_buffer ...
-    Tensor weight_buffer, x_hat_buffer;     // ... undefined if it is no tensor
+    const Tensor *weight_buffer = nullptr, *x_hat_buffer = nullptr;       // ... that may be no tensor
 };
 
 // The power of two inside a layer's FP8 weights (reads the metadata back to the host: once per layer and set of buffers).
@@ -376,17 +398,18 @@ bool read_layer(PyObject *module, Refs &refs, Layer &l)
     else if (od == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kFloat))) l.out = at::kFloat;
     PyObject *wo = get(dict, S._weight_buffer);
     l.lends = wo && wo != Py_None;
-    if (const Tensor *t = as_tensor(wo)) l.weight_buffer = *t;
-    if (const Tensor *t = as_tensor(get(dict, S._x_hat_buffer))) l.x_hat_buffer = *t;
+    PyObject *xo = get(dict, S._x_hat_buffer);
+    if ((l.weight_buffer = as_tensor(wo))) refs.add(wo);
+    if ((l.x_hat_buffer = as_tensor(xo))) refs.add(xo);
     l.fp8 = is_true(get(dict, S.fp8_operands));
     if (l.fp8 && l.plan->gs == 64) l.fp8_mult = fp8_multiplier(*l.plan, dict);
     return true;
 }
 // A buffer lent for scratch of `numel` fp16 values on the device of x.
-bool lent(const Tensor &buffer, int64_t numel, const Tensor &x)
+bool lent(const Tensor *buffer, int64_t numel, const Tensor &x)
 {
-    return buffer.defined() && buffer.is_cuda() && f16(buffer) && buffer.is_contiguous() && buffer.numel() >= numel &&
-           buffer.device() == x.device();
+    return buffer && buffer->is_cuda() && f16(*buffer) && buffer->is_contiguous() && buffer->numel() >= numel &&
+           buffer->device() == x.device();
 }
 
 struct Options {
@@ -517,7 +540,7 @@ std::optional<Tensor> run_layer(const Layer &l, const Tensor &x, const Options &
         return y;
     }
     if (l.lends && !lent(l.weight_buffer, N * K, x)) return std::nullopt;
-    const Tensor *w_ws = l.lends ? &l.weight_buffer : nullptr;
+    const Tensor *w_ws = l.lends ? l.weight_buffer : nullptr;
     if (!o.next && !o.x_is_xhat && prepare_pays(*plan, x, m, w_ws != nullptr, o.layernorm != nullptr)) {
         // (x_hat and w_hat in one scratch tensor; w_hat first: 512-byte runs stay aligned)
         const bool use_ws = w_ws != nullptr && aligned16(*w_ws);
@@ -530,11 +553,16 @@ std::optional<Tensor> run_layer(const Layer &l, const Tensor &x, const Options &
         run_product(*plan, m, x_hat, w, o.residual, o.gelu, nullptr, y.mutable_data_ptr(), code_of(y), stream);
         return y;
     }
-    const Tensor ws = lent(l.x_hat_buffer, x.numel(), x) ? l.x_hat_buffer : empty({x.numel()}, at::kHalf, x.device());
+    Tensor own_ws;
+    const Tensor *ws = l.x_hat_buffer;
+    if (!lent(ws, x.numel(), x)) {
+        own_ws = empty({x.numel()}, at::kHalf, x.device());
+        ws = &own_ws;
+    }
     Tensor y = empty(sizes, out_type, x.device());
     if (!extras) {
         check(arcq_linear_otf_ws(x.const_data_ptr(), code_of(x), fp(A_THR), fp(A_CB), static_cast<const uint8_t *>(p[W_PACKED]),
-                                 fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), ws.mutable_data_ptr(),
+                                 fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM), fp(W_BIAS), ws->mutable_data_ptr(),
                                  w_ws ? w_ws->mutable_data_ptr() : nullptr, y.mutable_data_ptr(), code_of(y), m, N, K,
                                  static_cast<int>(plan->bits), static_cast<int>(plan->gs), stream));
         return y;
@@ -560,7 +588,7 @@ std::optional<Tensor> run_layer(const Layer &l, const Tensor &x, const Options &
         a.next_a_thresholds = static_cast<const float *>(o.next->plan->p[A_THR]);
         a.next_a_codebook = static_cast<const float *>(o.next->plan->p[A_CB]);
     }
-    a.x_hat_ws = ws.mutable_data_ptr();
+    a.x_hat_ws = ws->mutable_data_ptr();
     a.w_hat_ws = w_ws ? w_ws->mutable_data_ptr() : nullptr;
     a.y = y.mutable_data_ptr();
     check(arcq_linear_otf_ex(&a, stream));
@@ -672,8 +700,8 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
     const int64_t wq = weight_bytes(pq), wp = weight_bytes(pp), w1 = weight_bytes(pf1), w2 = weight_bytes(pf2);
     // Scratch from the layers' lent buffers where they have room, else from the allocator.  Two weights are in use at a time, and
     // fc1 reads its x_hat while it writes fc2's: of a pair that shares a buffer one lies elsewhere (fc1's x_hat where qkv was).
-    auto scratch = [&](const Tensor &buffer, int64_t bytes) {
-        return lent(buffer, (bytes + 1) / 2, x) && aligned16(buffer) ? buffer : empty({bytes}, at::kByte, x.device());
+    auto scratch = [&](const Tensor *buffer, int64_t bytes) {
+        return lent(buffer, (bytes + 1) / 2, x) && aligned16(*buffer) ? *buffer : empty({bytes}, at::kByte, x.device());
     };
     auto at_byte = [](const Tensor &t, int64_t i) { return static_cast<char *>(t.mutable_data_ptr()) + i; };
     const Tensor w_attn = scratch(k.qkv.weight_buffer, wq + wp), xh = scratch(k.qkv.x_hat_buffer, rows * operand_row_bytes(C, fp8));

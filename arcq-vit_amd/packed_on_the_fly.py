@@ -137,7 +137,8 @@ class ARCQPackedLinearOnTheFly(nn.Module):
         operations otherwise; without them this is the reference module's forward.  ``quantize_for=consumer`` (see
         ``can_quantize_for``): the result is the consumer's ``x_hat`` instead of this layer's output, to be passed to
         ``consumer(..., input_is_xhat=True)``, which skips its own stage 1."""
-        y = _lib.host().layer_forward(self, x, layernorm, activation == "gelu", residual, quantize_for, input_is_xhat) \
+        host = _lib._host or _lib.host()
+        y = host.layer_forward(self, x, layernorm, activation == "gelu", residual, quantize_for, input_is_xhat) \
             if activation is None or activation == "gelu" else None
         if y is not None:
             return y

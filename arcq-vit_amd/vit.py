@@ -88,9 +88,10 @@ class Block(nn.Module):
         # The whole block from the host extension where every part is the plain case (packed layers, no hooks on the
         # modules it would call): the same operations in the same order, without the interpreter between them.  (A tracer's
         # stand-in for x is no tensor and takes the code below.)
-        y = _lib.host_for_block().block_forward(self, x) if isinstance(x, torch.Tensor) and x.is_cuda else None
-        if y is not None:
-            return y
+        if isinstance(x, torch.Tensor) and x.is_cuda:
+            y = (_lib._host or _lib.host_for_block()).block_forward(self, x)
+            if y is not None:
+                return y
         if self.fuse_elementwise and isinstance(self.mlp.act, nn.GELU) and self.mlp.act.approximate == "none":
             a = self.attn
             x = a.proj(a.mix(a.qkv(x, layernorm=self.norm1)), residual=x)

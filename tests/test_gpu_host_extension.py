@@ -585,3 +585,24 @@ def test_copies_made_during_capture_stay_in_the_graph(cuda):
         del graph, y
         torch.cuda.empty_cache()
         assert torch.equal(layers[1](x, layernorm=norm), want)
+
+
+def test_copies_are_ready_for_every_stream(cuda):
+    """The stream of the first call makes the fp32 copies; a call on another stream that comes before they are made waits."""
+    x = _tokens(197, 192)
+    with torch.no_grad():
+        norm, scale = torch.nn.LayerNorm(192).cuda().half(), _on_the_fly(192, 768).weight_scale.half()
+        norm.weight.uniform_(0.5, 1.5)
+        layers = [_on_the_fly(192, 768) for _ in range(2)]
+        for layer in layers:
+            layer.weight_scale = scale
+        want = layers[0](x, layernorm=norm)
+        first, second = torch.cuda.Stream(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(first):
+            torch.cuda._sleep(200_000_000)
+            a = layers[1](x, layernorm=norm)
+        with torch.cuda.stream(second):
+            b = layers[1](x, layernorm=norm)
+        torch.cuda.synchronize()
+        assert torch.equal(a, want) and torch.equal(b, want)
