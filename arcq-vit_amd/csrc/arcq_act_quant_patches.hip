@@ -38,6 +38,11 @@ __device__ __forceinline__ float quotient(float d, float s, float y)
 }
 __device__ __forceinline__ bool in_range(float v) { return (v == 0.0f) | ((fabsf(v) >= 0x1p-60f) & (fabsf(v) <= 0x1p60f)); }
 
+// The fast form looks every quotient up before it is known to be in range (what it finds otherwise is not used): the payload of an
+// fp32 NaN may name any of the offsets that bucket_offset_of can give (that of an fp16 one, widened, has no bits there), and a table
+// with two thresholds in one bucket one code more than there are.  Both tables have an entry for it.
+template <typename TIN> constexpr int kTableEntries = sizeof(TIN) == 4 ? 0x1ff8 / static_cast<int>(sizeof(Bucket)) + 1 : kMaxBuckets + 1;
+
 // One pixel: its three channels quantized and reconstructed in place.  Returns whether every quotient was in range (FAST).
 template <int BITS, bool FAST, bool HALF>
 __device__ __forceinline__ bool quantize_pixel(float (&x)[kC], float eps, const float (&th)[(1 << BITS) - 1], const float (&cbv)[1 << BITS],
@@ -99,8 +104,8 @@ act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ 
 {
     constexpr int L = 1 << BITS;
     constexpr int kIn = 8 * static_cast<int>(sizeof(TIN)) / 16;
-    __shared__ float lut[L * 64];
-    __shared__ Bucket table[kMaxBuckets + 1];
+    __shared__ float lut[(L + 1) * 64];
+    __shared__ Bucket table[kTableEntries<TIN>];
     __shared__ int slow_slots[kPrepWaves];
     if (prep_weight_workgroup<BITS, false>(weights, PrepWeights{}, lut)) return;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -126,6 +131,8 @@ act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ 
     load_quant_params<BITS>(thr, cb, th, cbv);
     const BucketScale bq = pick_bucket_scale<BITS>(th);
     build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, kPrepThreads);
+    if constexpr (sizeof(TIN) == 4)
+        for (int b = bq.nb + 1 + tid; b < kTableEntries<TIN>; b += kPrepThreads) table[b] = Bucket{__int_as_float(0x7f800000), 0};
     __syncthreads();
     bool table_ok = true;
 #pragma unroll
