@@ -24,11 +24,12 @@ template <typename TIN> struct PrepTile;           // a 32-row x 64-value tile i
 template <> struct PrepTile<float> { static constexpr int pitch = 65, vec = 4; };
 template <> struct PrepTile<__half> { static constexpr int pitch = 33, vec = 8; };
 
-// Stage 1 without a LayerNorm: memory-bound from a few thousand rows on (12 608 x 768 fp16: 10.8 us, 8 at the copy rate).  A
-// wave tile is 32 rows x ONE group; lane l owns row l / 2 and the half l % 2 of the group (arcq_act_quant_core.h).  Data moves
-// through a wave-private LDS tile (rows of the tile = rows of the tensor): coalesced 16-byte loads in, every piece column out as
-// one 512-byte run of the block layout.  (Lanes that load their 64 contiguous bytes themselves, four partial lines per
-// instruction: 16.0 us.)
+// Stage 1 without a LayerNorm.  From a few thousand rows on fp16 input is bound by the vector ALUs (12 608 x 1 536: 17.0 us, they
+// issue during 95 % of it, 78 MB = 4.6 TB/s; 12 608 x 768: 10.8 us, 8 at the rate of a copy), fp32 input by memory (12 608 x
+// 1 536: 22.7 us, 116 MB = 5.1 TB/s).  A wave tile is 32 rows x ONE group; lane l owns row l / 2 and the half l % 2 of the group
+// (arcq_act_quant_core.h).  Data moves through a wave-private LDS tile (rows of the tile = rows of the tensor): coalesced 16-byte
+// loads in, every piece column out as one 512-byte run of the block layout.  (Lanes that load their 64 contiguous bytes
+// themselves, four partial lines per instruction: 16.0 us.)
 // BUILDER: a fifth wave that owns no tile builds the lookup tables while the four tile waves load their first tile and take
 // its statistics.  Without it the four build the tables together before their first tile.
 template <typename TIN, int BITS, bool F8, bool BUILDER>

@@ -3,16 +3,16 @@ benchmarks), constructor and buffers as FQ/arcq_packed_on_the_fly.py:93-135.
 
 Reference forward (:137-161): fp16 copy of x -> Triton quantize+reconstruct in place -> Triton
 unpack of the whole weight into an fp16 buffer in HBM -> cuBLAS ``F.linear``.  Here the layer is one
-or two HIP launches (``arcq_linear_otf_ws`` / ``arcq_linear_otf_ex``): stage 1 writes x_hat (fp16)
-into a workspace or keeps it in LDS, and the fused unpack + fp16 MFMA GEMM follows.  Where the
-dense weight lives depends on ``_weight_buffer`` (the flat fp16 scratch the reference's benchmark
-shares between all layers, scripts/benchmark_arcq_on_the_fly.py:182-191, read at :148-158):
-  * not set: the GEMM kernel rebuilds the weight tile by tile in LDS; the dense weight never exists
-    in HBM;
-  * set (what ``packed_convert.share_buffers`` and ``bench.py`` do): from 512 rows on the fp16
-    weight is reconstructed into it inside the layer's first (or only) launch and the GEMM reads it
-    from there, i.e. it does pass through memory (L2-resident, a few MB) -- the reference's
-    unpack-then-GEMM order without a launch of its own; below 512 rows it is not used.
+or two HIP launches: ``arcq_linear_otf_ws`` / ``arcq_linear_otf_ex``, or ``arcq_prepare`` (stage 1 and the
+weights in one launch) and ``arcq_linear_prepared`` (the product), whichever is faster for the sizes
+(the rule and its figures: ``prepare_pays`` in csrc_host/arcq_host.cpp).  x_hat (fp16) lies in a workspace or
+in LDS, and so do the dense fp16 weights:
+  * below 512 rows and 768 inputs they are rebuilt tile by tile in LDS and never exist in memory;
+  * else they are reconstructed in the layer's first (or only) launch and pass through memory (L2-resident, a
+    few MB) -- the reference's unpack-then-GEMM order without a launch of its own -- in ``_weight_buffer`` where
+    that is set (the flat fp16 scratch the reference's benchmark shares between all layers,
+    scripts/benchmark_arcq_on_the_fly.py:182-191, read at :148-158; ``packed_convert.share_buffers`` sets it),
+    otherwise in scratch of the call's own.  The one-launch kernels from 512 rows on run only with it.
 The result is bit-identical either way.
 
 Differences from the reference module that a caller can observe (all on the side of more accuracy;

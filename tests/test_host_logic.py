@@ -468,7 +468,7 @@ def test_bench_host_side_contract():
     finally:
         sys.path.pop(0)
     for (model, bits, batch), kernels in {("deit_small", 4, 64): ("otf_rows_kernel", "otf_rows_phased_kernel"),
-                                          ("deit_base", 4, 64): ("gemm_pair_kernel",),
+                                          ("deit_base", 4, 64): ("otf_rows_kernel", "otf_rows_phased_kernel"),
                                           ("vit_large", 3, 256): ("gemm_pair_kernel",)}.items():
         for kernel in kernels:
             traffic = bench.profiled_traffic(model, bits, batch, kernel)
