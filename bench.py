@@ -17,7 +17,7 @@ the one with the largest share of its time; for DeiT-S that is a whole-layer ker
 stage 1 and the weight reconstruction: algorithmic flops (2*M*N*K) of its launches divided by their time alone,
 measured here with HIP events on the launch stream in a graph of only these launches; ``roofline.layer`` is the
 whole step against the same peaks; ``roofline.weights_rebuilt_inside_gemm`` the variant that dequantizes inside
-the GEMM.  ``other_configs`` times the other BASELINE configurations (DeiT-B W4A4 batch 64, ViT-L W3A3 batch
+the GEMM.  ``other_configs`` times the other benchmark configurations (DeiT-B W4A4 batch 64, ViT-L W3A3 batch
 256) briefly in the same run, each with its own whole-step roofline.  ``cpu_baseline`` times the oracle's
 restatement of the reference's fake-quant CPU path (quantize + reconstruct activation and weight, fp32 matmul)
 on a bounded sample on this host.
@@ -99,7 +99,7 @@ def parse_args():
     ap.add_argument("--no-bs1", action="store_true")
     ap.add_argument("--no-model", action="store_true", help="skip the model_forward block (whole ViT forward)")
     ap.add_argument("--no-other-configs", action="store_true",
-                    help="skip the short runs of the other BASELINE configurations (default run only)")
+                    help="skip the short runs of the other benchmark configurations (default run only)")
     ap.add_argument("--fp8", action="store_true",
                     help="also time the same step with FP8 operands (ops.linear_otf_fp8: not the reference's numerics; "
                          "reported in a block of its own, never as `value`)")
@@ -733,7 +733,7 @@ def main():
         out["bs1"]["cold_cache"] = cold_cache_bs1(args.model, args.bits, max(args.steps, 50), max(args.warmup, 10), dev)
         out["bs1"]["chained"] = chained_step(args.model, args.bits, 1, max(args.steps, 50), max(args.warmup, 10), dev)
     if not args.no_other_configs and (args.model, args.bits, args.batch) == ("deit_small", 4, 64):
-        # the other BASELINE configurations, a short timed run each (their own whole-step roofline; same kernels as
+        # the other benchmark configurations, a short timed run each (their own whole-step roofline; same kernels as
         # `bench.py --model ... --bits ... --batch ...` times at length)
         out["other_configs"] = {}
         for name, (mo, bi, ba, st) in {"deit_small_w3a3_bs64": ("deit_small", 3, 64, 20), "deit_base_w4a4_bs64": ("deit_base", 4, 64, 10),
