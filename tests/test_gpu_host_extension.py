@@ -1,8 +1,11 @@
 """What the host extension promises around its hot calls: the plain case only, and the interpreter's results where it takes
 over -- types that autocast chooses, flags of any type, copies of modules, grad mode, alignment, memory, threads."""
+import collections
+
 import numpy as np
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import arcq_vit_amd as A
 from arcq_vit_amd import synth
@@ -44,6 +47,18 @@ def _interpreted(block, x):
         hook.remove()
 
 
+class _CountOps(TorchDispatchMode):
+    """Counts torch's operations, those of C++ code included (each of them comes back to Python for it)."""
+
+    def __init__(self):
+        super().__init__()
+        self.seen = collections.Counter()
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen[str(func)] += 1
+        return func(*args, **(kwargs or {}))
+
+
 @pytest.mark.parametrize("fused", [False, True])
 @pytest.mark.parametrize("half", [True, False])
 @pytest.mark.parametrize("batch,tokens", [(2, 197), (5, 197), (1, 300)])
@@ -59,7 +74,11 @@ def test_block_under_bf16_autocast(cuda, batch, tokens, half, fused):
                 block(x)
             return
         got = block(x)
+        with _CountOps() as ops:
+            assert torch.equal(block(x), got)
     assert got.dtype == want.dtype and torch.equal(got, want)
+    attentions = sum(n for name, n in ops.seen.items() if "scaled_dot_product" in name)
+    assert attentions == 1 and ops.seen["aten.native_layer_norm.default"] == (0 if fused else 2), ops.seen
 
 
 @pytest.mark.parametrize("yes,no", [(1, 0), (np.bool_(True), np.bool_(False)), ("yes", "")])
@@ -532,6 +551,13 @@ def test_blocks_use_the_lent_buffers(cuda, fused, fp8):
         assert torch.equal(got, want)
         unit = rows * 192 * (1 if fp8 else 2)                             # x_hat of 192 values: one unit, fc2's: four
         assert lent <= alone - 5 * unit + (1 << 20), (alone / unit, lent / unit)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = vit.blocks(x)
+        for _ in range(3):                                                # replays with eager work in the same buffers between
+            y.zero_()
+            graph.replay()
+            assert torch.equal(y, want) and torch.equal(vit.blocks(x), want)
         share_buffers(vit, rows - 1)                                      # too small for fc2's x_hat: allocated again
         assert torch.equal(vit.blocks(x), want)
         for other in (torch.zeros(10, device=cuda), None):                # no fp16 buffer; none
