@@ -9,9 +9,10 @@
 //
 // Every function returns None where a call is not the plain case (an argument of another type, layout or device, a
 // module with hooks, a shape the library does not run): the Python code behind it then validates, converts and raises
-// as it always did.  Nothing here synchronises (but for the one FP8 multiplier of a layer).  What a call needs of its modules
-// is read first, under the GIL; allocations, torch operations and launches follow without it, so that threads on streams
-// of their own run side by side.
+// as it always did.  Nothing here synchronises, but for what is done once per layer: its FP8 multiplier is read back, and the
+// first call from a second stream waits for the copies that the first one makes.  What a call needs of its modules is read
+// first, under the GIL; allocations, torch operations and launches follow without it, so that threads on streams of their
+// own run side by side.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -85,7 +86,8 @@ inline PyObject *dict_of(PyObject *o)
     PyObject **d = _PyObject_GetDictPtr(o);
     return d ? *d : nullptr;
 }
-inline PyObject *get(PyObject *dict, PyObject *key) { return dict ? PyDict_GetItemWithError(dict, key) : nullptr; }   // borrowed (str keys: no errors)
+// A borrowed reference.  (The keys are interned strings, whose lookup cannot fail.)
+inline PyObject *get(PyObject *dict, PyObject *key) { return dict ? PyDict_GetItemWithError(dict, key) : nullptr; }
 // What `if o:` decides; an absent attribute is false.  (May run code of a class's own __bool__.)
 inline bool is_true(PyObject *o)
 {
@@ -486,8 +488,8 @@ void run_product(const Plan &p, int64_t rows, const void *x_hat, const Weights &
 // (packed codes that are not 16-byte aligned are left to the kernels and entry points that take them, or say why not)
 bool can_prepare(const Plan &p, int64_t rows)
 {
-    return aligned16(p.p[W_PACKED]) && p.gs == 64 && p.K % 64 == 0 && (p.N % 32 == 0 || rows >= 512) && rows * p.K < (int64_t(1) << 31) && p.N * p.K < (int64_t(1) << 31) &&
-           rows < (int64_t(1) << 26);
+    return aligned16(p.p[W_PACKED]) && p.gs == 64 && p.K % 64 == 0 && (p.N % 32 == 0 || rows >= 512) &&
+           rows * p.K < (int64_t(1) << 31) && p.N * p.K < (int64_t(1) << 31) && rows < (int64_t(1) << 26);
 }
 // Whether one layer call runs as prepare + product.  Below 512 rows from K = 768 on (up to 512 inputs the one-launch kernel
 // is 1 us faster: 7.7 against 9.6 us at 197 x 384 x 384; 12.9 against 11.1 at 2 304 x 768, 43 against 16.5 with a LayerNorm
