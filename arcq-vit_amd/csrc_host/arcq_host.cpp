@@ -63,6 +63,7 @@ PyObject *g_layer_type = nullptr;        // ARCQPackedLinearOnTheFly
 PyObject *g_attention_type = nullptr, *g_mlp_type = nullptr;
 PyObject *g_gelu_type = nullptr, *g_layernorm_type = nullptr;
 PyObject *g_fp8_multiplier = nullptr;    // ops.fp8_weight_multiplier
+PyObject *g_half = nullptr, *g_float = nullptr;      // torch.float16, torch.float32
 
 struct Failure {};      // a Python exception is set
 
@@ -110,7 +111,6 @@ inline const Tensor *as_tensor(PyObject *o) { return o && THPVariable_Check(o) ?
 
 // Inference tensors have no version: a change in place leaves no trace on them, and nothing derived from one is kept.
 inline bool has_version(const Tensor &t) { return t.unsafeGetTensorImpl()->version_counter().enabled(); }
-inline uint32_t version_of(const Tensor &t) { return has_version(t) ? t.unsafeGetTensorImpl()->version_counter().current_version() : 0; }
 inline Tensor empty(at::IntArrayRef sizes, at::ScalarType type, c10::Device device)
 {
     return Tensor(at::detail::empty_cuda(sizes, type, device, std::nullopt));
@@ -137,6 +137,7 @@ inline const uint8_t *bptr(const Tensor &t) { return static_cast<const uint8_t *
 // The memory stays the module's to give back: the storage is held weakly, which is enough for its address to name it.
 struct Slot {
     std::optional<c10::weak_intrusive_ptr<c10::StorageImpl>> storage;
+    const c10::StorageImpl *named = nullptr;
     Tensor copy;              // fp32 / contiguous, where the tensor is not
     bool tracked = true;      // changes in place show in its version
     uint32_t version = 0;
@@ -145,15 +146,18 @@ struct Slot {
     at::DimVector sizes, strides;
     bool same(const Tensor &t) const
     {
-        return storage && storage->_unsafe_get_target() == t.unsafeGetTensorImpl()->unsafe_storage().unsafeGetStorageImpl() &&
-               version == version_of(t) && data == t.const_data_ptr() && type == t.scalar_type() && t.sizes().equals(sizes) &&
-               t.strides().equals(strides) && tracked == has_version(t) && (tracked || !copy.defined());
+        const c10::TensorImpl *impl = t.unsafeGetTensorImpl();
+        const auto &vc = impl->version_counter();
+        return named == impl->unsafe_storage().unsafeGetStorageImpl() && data == t.const_data_ptr() && type == t.scalar_type() &&
+               t.sizes().equals(sizes) && t.strides().equals(strides) &&
+               (tracked ? vc.enabled() && vc.current_version() == version : !vc.enabled() && !copy.defined());
     }
     void set(const Tensor &t, bool as_f32, bool align = false)
     {
         storage.emplace(t.storage().getWeakStorageImpl());
+        named = storage->_unsafe_get_target();
         tracked = has_version(t);
-        version = version_of(t);
+        version = tracked ? t.unsafeGetTensorImpl()->version_counter().current_version() : 0;
         data = t.const_data_ptr();
         type = t.scalar_type();
         sizes = t.sizes();
@@ -396,8 +400,8 @@ bool read_layer(PyObject *module, Refs &refs, Layer &l)
     l.plan = plan_of(module, Kind::OnTheFly, refs, dict);
     if (!l.plan) return false;
     PyObject *od = get(dict, S.out_dtype);
-    if (od == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf))) l.out = at::kHalf;
-    else if (od == reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kFloat))) l.out = at::kFloat;
+    if (od == g_half) l.out = at::kHalf;
+    else if (od == g_float) l.out = at::kFloat;
     PyObject *wo = get(dict, S._weight_buffer);
     l.lends = wo && wo != Py_None;
     PyObject *xo = get(dict, S._x_hat_buffer);
@@ -1136,6 +1140,8 @@ PyObject *py_register_types(PyObject *, PyObject *const *args, Py_ssize_t n)
         Py_XDECREF(*to[i]);
         *to[i] = args[i];
     }
+    g_half = reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf));       // (they live as long as torch)
+    g_float = reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kFloat));
     Py_RETURN_NONE;
 }
 
