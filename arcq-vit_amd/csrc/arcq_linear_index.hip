@@ -304,13 +304,18 @@ linear_index_tile_kernel(const uint8_t *__restrict__ xq, const float *__restrict
 constexpr int kIdxMinWaves = 3, kIdxMaxWaves = 4;
 constexpr int kIdxRegion = 32 * 33 * 8;            // bytes per wave: operands of half a group, then its terms (33-double pitch)
 
-template <int BITS, int R, int C, int MAXW>
-__global__ void __launch_bounds__(64 * MAXW, MAXW > kIdxMaxWaves ? 1 : R == 1 ? 4 : 3)
-linear_index_wide_kernel(const uint8_t *__restrict__ xq, const float *__restrict__ xc, const float *__restrict__ xs,
-                         const float *__restrict__ xcs, const uint8_t *__restrict__ wq,
-                         const float *__restrict__ wc, const float *__restrict__ ws, const float *__restrict__ wcs,
-                         const float *__restrict__ table, const float *__restrict__ a_cb, const float *__restrict__ w_cb,
-                         const float *__restrict__ bias, float *__restrict__ y, int rows, int out_f, int G, int levels)
+struct IndexArgs {
+    const uint8_t *xq;
+    const float *xc, *xs, *xcs;
+    const uint8_t *wq;
+    const float *wc, *ws, *wcs, *table, *a_cb, *w_cb, *bias;
+    float *y;
+    int rows, out_f, G, levels;
+};
+
+// The tile of rows r0 .. and outputs o0 .., by a workgroup of at least MINW waves.
+template <int BITS, int R, int C, int MINW>
+__device__ __forceinline__ void index_wide_tile(const IndexArgs &p, int r0, int o0)
 {
 #pragma clang fp contract(off)
     constexpr bool kPacked = BITS != 0;
@@ -327,7 +332,12 @@ linear_index_wide_kernel(const uint8_t *__restrict__ xq, const float *__restrict
     extern __shared__ __attribute__((aligned(16))) unsigned char idx_smem[];     // [S waves][kIdxRegion]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nthreads = blockDim.x, S = nthreads >> 6;
     const int lx = lane & 7, ly = lane >> 3;
-    const int r0 = blockIdx.y * TR, o0 = blockIdx.x * TC;
+    const int rows = p.rows, out_f = p.out_f, G = p.G, levels = p.levels;
+    const uint8_t *__restrict__ xq = p.xq, *__restrict__ wq = p.wq;
+    const float *__restrict__ xc = p.xc, *__restrict__ xs = p.xs, *__restrict__ xcs = p.xcs, *__restrict__ wc = p.wc, *__restrict__ ws = p.ws;
+    const float *__restrict__ wcs = p.wcs, *__restrict__ table = p.table, *__restrict__ a_cb = p.a_cb, *__restrict__ w_cb = p.w_cb;
+    const float *__restrict__ bias = p.bias;
+    float *__restrict__ y = p.y;
     unsigned char *region = idx_smem + wave * kIdxRegion;
     float *s_x = reinterpret_cast<float *>(region), *s_w = s_x + TR * 32;
 
@@ -365,7 +375,7 @@ linear_index_wide_kernel(const uint8_t *__restrict__ xq, const float *__restrict
     asm volatile("" ::"v"(region) : "memory");
 
     // The outputs this thread sums: TR * TC of them over the workgroup, consecutive in a row.
-    constexpr int kSums = (TR * TC + 64 * kIdxMinWaves - 1) / (64 * kIdxMinWaves);
+    constexpr int kSums = (TR * TC + 64 * MINW - 1) / (64 * MINW);
     acc_t acc[kSums];
 #pragma unroll
     for (int i = 0; i < kSums; ++i) {
@@ -548,14 +558,229 @@ linear_index_wide_kernel(const uint8_t *__restrict__ xq, const float *__restrict
     }
 }
 
-struct IndexArgs {
-    const uint8_t *xq;
-    const float *xc, *xs, *xcs;
-    const uint8_t *wq;
-    const float *wc, *ws, *wcs, *table, *a_cb, *w_cb, *bias;
-    float *y;
-    int rows, out_f, G, levels;
-};
+template <int BITS, int R, int C, int MAXW>
+__global__ void __launch_bounds__(64 * MAXW, MAXW > kIdxMaxWaves ? 1 : R == 1 ? 4 : 3) linear_index_wide_kernel(const IndexArgs p)
+{
+    index_wide_tile<BITS, R, C, kIdxMinWaves>(p, blockIdx.y * 8 * R, blockIdx.x * 8 * C);
+}
+
+// ---- the packed format on the matrix units ---------------------------------------------------------------------------------
+// The table entries are fp32 numbers: over the lowest bit that any of them uses they are integers, and where those have at most 38
+// bits the fp64 sum of 64 of them is exact in every order.  The sum over j is then an integer product: the x codes one-hot (2^bits
+// bytes of 0 and 1 per j) times the signed base-256 digits of the entries T[.][w_j], one product per digit.  A one-hot operand has
+// at most one byte in four, so the products are the 4:2 sparse ones (v_smfmac_i32_32x32x64_i8, twice the dense rate; of the two
+// stored bytes of a four only the first is used).  The five int32 sums together are the sum of the table entries, the same double
+// that the serial loop ends with, and the group's closed form follows in the same operations: the result's bits stay what they
+// are.  Every workgroup looks the table over for its lowest and highest bit; a table that does not qualify (largest entry more
+// than 2^14 times the smallest, subnormals, infinities, NaN) runs the loops above on the same tile.
+//
+// The wide kernel above spends a multiplication, a conversion and an fp64 addition of the vector ALU on every product; here 4 096
+// products take five MFMAs of 32 clocks on a pipe of their own.  A wave owns 32 x 32 outputs for all groups, in order.  The digits
+// come from a 1 280-byte table in LDS by the w code, 16 bytes a read (2^bits different entries: no bank conflicts); the x operand
+// is made in registers, and the fp64 sums lie in LDS between the groups so that three waves fit a SIMD: matrix pipe, vector ALU
+// (the closed form, 13 instructions per output and group) and LDS are each about half busy, and the waves overlap them.
+// Measured, this kernel against the wide one: 1576 x 384 -> 1536 at 4 / 3 / 2 bits 55 / 45 / 32 us against 113 / 103 / 99, 12608
+// rows at 4 bits 307 against 714.  With dense products 82 us; 64 x 32 outputs a wave and the groups dealt over the waves 117.
+constexpr int kDigits = 5, kMaxEntryBits = 38;
+constexpr int kMfmaWaves = 4, kMfmaTile = 32;                      // a wave's tile is 32 x 32, the workgroup's 32 outputs wide
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef int i32x8_t __attribute__((ext_vector_type(8)));
+typedef int i32x16_t __attribute__((ext_vector_type(16)));
+
+template <int BITS>
+__global__ void __launch_bounds__(64 * kMfmaWaves, 3)
+linear_index_mfma_kernel(const IndexArgs p)
+{
+#pragma clang fp contract(off)
+    constexpr int L = 1 << BITS, kEntries = L * L, E = 16 / L;                   // E: j's of 16 bytes
+    constexpr int kSteps = 16 / E;                                               // 4 E j's each
+    __shared__ __attribute__((aligned(16))) signed char s_digits[kDigits * kEntries];        // [digit][w code][x code]
+    __shared__ __attribute__((aligned(16))) double s_meta[kMfmaWaves][3][kMfmaTile];
+    __shared__ int s_low, s_high;
+    extern __shared__ __attribute__((aligned(16))) unsigned char idx_smem[];     // [waves][kIdxRegion]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 31, lh = lane >> 5;
+    constexpr int kThreads = 64 * kMfmaWaves, kEach = (kEntries + kThreads - 1) / kThreads;
+    const int r0 = blockIdx.y * (kMfmaWaves * kMfmaTile), ow = blockIdx.x * kMfmaTile;
+    const int rw = r0 + wave * kMfmaTile;                                        // rows of the wave's tile
+    const int G = p.G;
+
+    // Codes of a group: a lane takes j = 32 lh ... + 31 of row lr, and all 64 of output lr.
+    // (rows and outputs times groups: 32 bits, checked by the launcher)
+    const uint32_t xrow = static_cast<uint32_t>(min(rw + lr, p.rows - 1)) * G, wrow = static_cast<uint32_t>(min(ow + lr, p.out_f - 1)) * G;
+    const float *x_meta = lh ? p.xs : p.xc;                                      // (the halves of the wave share the rows' metadata)
+    uint32_t xn[BITS], wn[2][BITS];
+    float xmn[2], wmn[3];
+    auto fetch = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < BITS; ++d) {
+            xn[d] = reinterpret_cast<const uint32_t *>(p.xq)[(xrow + g) * (2 * BITS) + lh * BITS + d];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) wn[h][d] = reinterpret_cast<const uint32_t *>(p.wq)[(wrow + g) * (2 * BITS) + h * BITS + d];
+        }
+        xmn[0] = x_meta[xrow + g], xmn[1] = p.xcs[xrow + g];
+        wmn[0] = p.wc[wrow + g], wmn[1] = p.ws[wrow + g], wmn[2] = p.wcs[wrow + g];
+    };
+    fetch(0);
+
+    // The table's entries as integers over 2^low.
+    if (tid == 0) s_low = 1 << 20, s_high = -(1 << 20);
+    __syncthreads();
+    uint32_t entry[kEach];                                                       // (a, b) = (x code, w code) = (i / L, i % L)
+    int bad = 0;
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+        const int i = tid + k * kThreads;
+        entry[k] = i < kEntries ? __float_as_uint(p.table[i]) : 0;
+        const int exponent = static_cast<int>((entry[k] >> 23) & 255u);
+        bad |= exponent == 255 || (exponent == 0 && (entry[k] & 0x7fffffu));      // infinity, NaN, subnormal
+        if (exponent != 0) {
+            atomicMin(&s_low, exponent - 150 + (__ffs(static_cast<int>(entry[k] | 0x800000u)) - 1));
+            atomicMax(&s_high, exponent - 126);
+        }
+    }
+    const bool any_bad = __syncthreads_or(bad) != 0;
+    const int low = s_low <= s_high ? s_low : 0;                                 // (else all entries are zero)
+    if (any_bad || s_high - low > kMaxEntryBits) {                               // workgroup-uniform
+        for (int r = r0; r < min(r0 + kMfmaWaves * kMfmaTile, p.rows); r += 16) index_wide_tile<BITS, 2, 4, kMfmaWaves>(p, r, ow);
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+        const int i = tid + k * kThreads, exponent = static_cast<int>((entry[k] >> 23) & 255u);
+        const int shift = exponent - 150 - low;                                  // (negative: by zero bits of the entry)
+        long long v = exponent == 0 ? 0 : static_cast<long long>((entry[k] & 0x7fffffu) | 0x800000u);
+        v = shift >= 0 ? v << min(shift, 40) : v >> min(-shift, 23);
+        if (entry[k] >> 31) v = -v;
+        if (i < kEntries) {
+#pragma unroll
+            for (int d = 0; d < kDigits; ++d) {
+                const signed char digit = static_cast<signed char>(v & 255);
+                s_digits[d * kEntries + (i % L) * L + i / L] = digit;
+                v = (v - digit) >> 8;
+            }
+        }
+    }
+    __syncthreads();
+    const double unit = ldexp(1.0, low), per_unit64 = ldexp(1.0, -low - 6);
+
+    // Bits from..to (of BITS) of code number q, `up` bits to the left.
+    auto code_bits = [](const uint32_t (&w)[BITS], int q, int from, int to, int up) __attribute__((always_inline)) {
+        const int bit = q * BITS, d = bit >> 5, sh = bit & 31;
+        const uint32_t mask = ((1u << to) - (1u << from)) << up;
+        if (sh + BITS > 32) return ((__builtin_amdgcn_alignbit(w[d + 1], w[d], sh)) << up) & mask;
+        return (sh >= up ? w[d] >> (sh - up) : w[d] << (up - sh)) & mask;
+    };
+    // The digits of part k (L bytes) of a 32-byte fragment.
+    auto digit_part = [](i32x8_t &f, int k, const signed char *src) __attribute__((always_inline)) {
+        if constexpr (L == 16) {
+            const int4 v = *reinterpret_cast<const int4 *>(src);
+            f[4 * k] = v.x, f[4 * k + 1] = v.y, f[4 * k + 2] = v.z, f[4 * k + 3] = v.w;
+        } else if constexpr (L == 8) {
+            const int2 v = *reinterpret_cast<const int2 *>(src);
+            f[2 * k] = v.x, f[2 * k + 1] = v.y;
+        } else {
+            f[k] = *reinterpret_cast<const int *>(src);
+        }
+    };
+    // The sums over the groups: lane's outputs v at acc[64 v].
+    double *acc = reinterpret_cast<double *>(idx_smem) + wave * 1024 + lane;
+    {
+        const double b = p.bias && ow + lr < p.out_f ? static_cast<double>(p.bias[ow + lr]) : 0.0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v * 64] = b;
+    }
+    double (&meta)[3][kMfmaTile] = s_meta[wave];
+#pragma unroll 1
+    for (int g = 0; g < G; ++g) {
+        uint32_t xk[BITS], wk[2][BITS];
+#pragma unroll
+        for (int d = 0; d < BITS; ++d) {
+            xk[d] = xn[d];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {      // lanes of the upper half begin E codes further on
+                const uint32_t above = d + 1 < BITS ? wn[h][d + 1] : 0;
+                wk[h][d] = lh ? __builtin_amdgcn_alignbit(above, wn[h][d], E * BITS) : wn[h][d];
+            }
+        }
+        // (Multiplying by powers of two commutes with every rounding below: the sums stay in units of 2^low, the scale takes it in.)
+        const double wcv = wmn[0], wsv = wmn[1] * unit, wcsv = wmn[2] * per_unit64;
+        asm volatile("" ::: "memory");                                           // (the last group's reads of the metadata come first)
+        meta[lh][lr] = lh ? static_cast<double>(xmn[0]) : 64.0 * static_cast<double>(xmn[0]);
+        meta[2][lr] = xmn[1];
+        i32x16_t sum[kDigits];
+#pragma unroll
+        for (int d = 0; d < kDigits; ++d)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sum[d][v] = 0;
+        // The operands of step t + 1 are read under the products of step t.
+        i32x4_t xf[2];
+        uint32_t index[2];
+        i32x8_t wf[2][kDigits];
+        auto operands = [&](int t, i32x4_t &a, uint32_t &ix, i32x8_t (&b)[kDigits]) __attribute__((always_inline)) {
+            const signed char *src[2 * E];
+#pragma unroll
+            for (int k = 0; k < 2 * E; ++k) src[k] = s_digits + code_bits(wk[k / E], 2 * E * t + k % E, 0, BITS, BITS);
+#pragma unroll
+            for (int d = 0; d < kDigits; ++d)
+#pragma unroll
+                for (int k = 0; k < 2 * E; ++k) digit_part(b[d], k, src[k] + d * kEntries);
+            // Stored bytes of the x operand: of the two of a four that the index selects from only the first is used, 1 in the four that
+            // the code is in; the index of all its fours is the code's place in one.
+            ix = 0;
+#pragma unroll
+            for (int k = 0; k < 2 * E; ++k) {
+                const int q = 2 * E * t + k;
+                if constexpr (L == 16) {
+                    const uint64_t v = 1ull << code_bits(xk, q, 2, BITS, 2);
+                    a[2 * k] = static_cast<int>(v), a[2 * k + 1] = static_cast<int>(v >> 32);
+                } else if constexpr (L == 8) {
+                    a[k] = static_cast<int>(1u << code_bits(xk, q, 2, BITS, 2));
+                } else if (k & 1) {
+                    a[k >> 1] = 0x00010001;
+                }
+                ix |= __umul24(code_bits(xk, q, 0, 2, 0), L == 16 ? 0x1111u : L == 8 ? 0x11u : 0x1u) << (k * L);
+            }
+        };
+#pragma unroll
+        for (int t = 0; t < kSteps; ++t) {
+            operands(t, xf[0], index[0], wf[0]);
+#pragma unroll
+            for (int d = 0; d < kDigits; ++d)
+                sum[d] = __builtin_amdgcn_smfmac_i32_32x32x64_i8(xf[0], wf[0][d], sum[d], static_cast<int>(index[0]), 0, 0);
+        }
+        if (g + 1 < G) fetch(g + 1);                                             // (under the closed form; the products need the registers)
+        asm volatile("" ::: "memory");
+        // ---- the group's closed form (EXT/arcq_linear_kernel.cu:65-74) ----
+#pragma unroll
+        for (int v4 = 0; v4 < 4; ++v4) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int v = 4 * v4 + e, row = 8 * v4 + 4 * lh + e;
+                const int lo = sum[0][v] + sum[1][v] * 256 + sum[2][v] * 65536, hi = sum[3][v] + sum[4][v] * 256;      // |digit sums| <= 2^13
+                const double cross = __builtin_fma(static_cast<double>(hi), 16777216.0, static_cast<double>(lo));      // exact
+                const double mu_term = meta[0][row] * wcv;
+                const double residual_term = meta[1][row] * wsv * (cross - meta[2][row] * wcsv);
+                acc[v * 64] += mu_term + residual_term;
+            }
+        }
+    }
+    if (ow + lr < p.out_f) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int r = rw + 8 * (v >> 2) + 4 * lh + (v & 3);
+            if (r < p.rows) p.y[static_cast<int64_t>(r) * p.out_f + ow + lr] = static_cast<float>(acc[v * 64]);
+        }
+    }
+}
+
+template <int BITS>
+void launch_index_mfma(const IndexArgs &a, hipStream_t stream)
+{
+    hipLaunchKernelGGL((linear_index_mfma_kernel<BITS>), dim3((a.out_f + kMfmaTile - 1) / kMfmaTile, (a.rows + kMfmaWaves * kMfmaTile - 1) / (kMfmaWaves * kMfmaTile)),
+                       dim3(64 * kMfmaWaves), kMfmaWaves * kIdxRegion, stream, a);
+}
+
 template <int BITS, int R, int C, int MAXW>
 void launch_index_wide(const IndexArgs &a, hipStream_t stream)
 {
@@ -571,8 +796,7 @@ void launch_index_wide(const IndexArgs &a, hipStream_t stream)
             if ((a.G + s - 1) / s * s < (a.G + S - 1) / S * S) S = s;
     }
     hipLaunchKernelGGL((linear_index_wide_kernel<BITS, R, C, MAXW>), dim3((a.out_f + 8 * C - 1) / (8 * C), (a.rows + 8 * R - 1) / (8 * R)), dim3(64 * S),
-                       S * kIdxRegion, stream, a.xq, a.xc, a.xs, a.xcs, a.wq, a.wc, a.ws, a.wcs, a.table, a.a_cb, a.w_cb, a.bias, a.y, a.rows,
-                       a.out_f, a.G, a.levels);
+                       S * kIdxRegion, stream, a);
 }
 // Four outputs and two rows per lane; one row where that leaves at most 1024 workgroups (four per CU), whose duration is
 // one wave's (197 x 768 -> 768, 600 of them: 30.6 against 34.2 us; 394 x 768 -> 768: 42.4 against 42.9, byte codes 40.6
@@ -581,6 +805,14 @@ template <int BITS>
 void launch_index(const IndexArgs &a, hipStream_t stream)
 {
     const int64_t small_tiles = static_cast<int64_t>((a.rows + 7) / 8) * ((a.out_f + 31) / 32);
+    // The matrix units from 512 wave tiles of 32 x 32 on (two for every compute unit), whatever the number of groups: 788 x 768 -> 768
+    // (600 of them) 46.0 against 54.4 us, 394 x 1536 -> 1536 (624) 83.5 / 106; below, a wave's chain over all groups is what the
+    // launch takes: 394 x 768 -> 768 (312) 45.2 against 34.6 us, 197 x 192 -> 768 (168) 16.1 / 10.1.
+    if constexpr (BITS != 0) {
+        const int64_t tiles = static_cast<int64_t>((a.rows + kMfmaTile - 1) / kMfmaTile) * ((a.out_f + kMfmaTile - 1) / kMfmaTile);
+        if (tiles >= 2 * device_cus() && static_cast<int64_t>(a.rows > a.out_f ? a.rows : a.out_f) * a.G * 2 * BITS < (int64_t(1) << 31))
+            return launch_index_mfma<BITS>(a, stream);
+    }
     // No more workgroups than compute units: up to sixteen waves each, i.e. as few rounds of groups as possible.
     if (small_tiles <= device_cus() && a.G > kIdxMaxWaves) launch_index_wide<BITS, 1, 4, 16>(a, stream);
     else if (small_tiles <= 1024) launch_index_wide<BITS, 1, 4, kIdxMaxWaves>(a, stream);

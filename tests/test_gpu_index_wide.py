@@ -38,3 +38,39 @@ def test_linear_index_bitexact(cuda, oracle, m, n, k, bits, outer):
         a = _lib.LinearIndexArgs(*[v.data_ptr() for v in t], y.data_ptr(), m, n, k, fmt, 64, 1 << bits, 0)
         _lib.check(_lib.load().arcq_linear_index(ctypes.byref(a), torch.cuda.current_stream().cuda_stream))
         assert np.array_equal(y.cpu().numpy(), ref), fmt
+
+
+# From 512 tiles of 32 x 32 on the packed format runs on the matrix units (sums of the table's entries as integers): ragged rows
+# and outputs, one and many groups, and tables that it takes (also with zeros, and all of them zero, and with single-bit entries)
+# and leaves to the fp64 loops (entries too far apart, a subnormal, an infinity, a NaN).
+@pytest.mark.parametrize("m,n,k", [(545, 1000, 128), (4100, 127, 64), (33, 8225, 320)])
+@pytest.mark.parametrize("bits", [4, 3, 2])
+@pytest.mark.parametrize("kind", ["outer", "arbitrary", "zeros", "all_zero", "powers", "far_apart", "subnormal", "infinity", "nan"])
+def test_linear_index_on_the_matrix_units(cuda, oracle, m, n, k, bits, kind):
+    levels = 1 << bits
+    cb = synth.quantile_codebook(bits)
+    table = (1.1 * cb.view(-1, 1) * cb.view(1, -1)).contiguous()
+    if kind == "arbitrary":
+        table = table + 0.25 * torch.arange(table.numel()).view_as(table) / table.numel()
+    elif kind == "zeros":
+        table[1] = 0.0
+        table[:, 2] = -0.0
+    elif kind == "all_zero":
+        table = torch.zeros_like(table)
+    elif kind == "powers":
+        table = torch.sign(table) * 2.0 ** (torch.arange(table.numel()).view_as(table) % 15 - 80)
+    elif kind != "outer":
+        table[1, 1] = {"far_apart": 1.0e-6, "subnormal": 1.0e-40, "infinity": float("inf"), "nan": float("nan")}[kind]
+    rng = np.random.default_rng(7)
+    g = k // 64
+    xq = oracle.pack_codes_np(rng.integers(0, levels, (m, k)).astype(np.uint8), bits)
+    wq = oracle.pack_codes_np(rng.integers(0, levels, (n, k)).astype(np.uint8), bits)
+    meta = [rng.standard_normal((r, g)).astype(np.float32) for r in (m, m, m, n, n, n)]
+    bias = synth.make_bias(n, 5)
+    want = oracle.linear_forward_packed_c(xq, *meta[:3], wq, *meta[3:], table.numpy(), bias.numpy(), bits, 64, k, n)
+    d = lambda t: (torch.from_numpy(t) if isinstance(t, np.ndarray) else t).to(cuda).contiguous()
+    t = [d(v) for v in (xq, *meta[:3], wq, *meta[3:], table, cb, cb, bias)]
+    y = torch.full((m, n), float("nan"), device=cuda)
+    a = _lib.LinearIndexArgs(*[v.data_ptr() for v in t], y.data_ptr(), m, n, k, bits, 64, levels, 0)
+    _lib.check(_lib.load().arcq_linear_index(ctypes.byref(a), torch.cuda.current_stream().cuda_stream))
+    assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
