@@ -156,7 +156,7 @@ __device__ __forceinline__ void pack64(const uint32_t (&c)[64], uint32_t (&w)[2 
 
 // CODES = false drops everything only the code outputs need (the on-the-fly layer asks for x_hat alone).
 template <typename TIN, typename TOUT, int BITS, bool CODES>
-__global__ void __launch_bounds__(64 * kWaves)
+__global__ void __launch_bounds__(64 * kWaves, CODES ? 1 : 2)
 act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const float *__restrict__ cb,
                      uint8_t *__restrict__ packed, uint8_t *__restrict__ codes_u8,
                      float *__restrict__ center, float *__restrict__ scale, float *__restrict__ code_sum,
@@ -165,14 +165,14 @@ act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
     constexpr int L = 1 << BITS;
     constexpr int kStride = (Tile<TIN>::stride > Tile<TOUT>::stride) ? Tile<TIN>::stride : Tile<TOUT>::stride;
     __shared__ uint32_t tiles[kWaves][kTileGroups * kStride];
-    __shared__ float lut[L * 64];          // codebook replicated per lane: lut[c*64 + lane], conflict-free
-    __shared__ Bucket table[kMaxBuckets + 1];
-    __shared__ int slow_slots[kWaves];
+    __shared__ QuantTables tables;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
 
+    QuantParams params{};
+    if (wave == 0) params = load_quant_params<BITS>(thr, cb, lane);
     // The first tile of this wave is requested before anything else: its latency overlaps the setup below.
     const int64_t ntiles = (total_groups + kTileGroups - 1) / kTileGroups;
     const int64_t elem_end = total_groups * 64;
@@ -182,20 +182,13 @@ act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
         fetch_tile<TIN>(x, first * kTileGroups * 64, elem_end, regs, lane);      // zero-fills past the end
     }
 
-    // Thresholds and codebook are requested now and first used after the first tile's statistics: the lookup
-    // tables are built once per workgroup, between the two halves of the first tile, so that their load latency
-    // and the tile's hide behind each other.
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(thr, cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
     // The lookup tables are built once per workgroup, before the first tile's values are unpacked into registers.
     // (Built between the two halves of the first tile, or with both orders in the kernel and a flag to choose, the
     // variants that write codes run 20-40 % slower: registers.)
-    build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, 64 * kWaves);
+    if (wave == 0) build_quant_tables<BITS>(params, tables, lane);
     __syncthreads();
-    bool table_ok = true;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
+    const BucketScale bq = tables.geometry;
+    const bool table_ok = tables.usable != 0;
 
     uint32_t *tile = tiles[wave];
 
@@ -215,7 +208,7 @@ act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
         float mu, var, s, sum_codes;
         uint32_t code[CODES ? 64 : 1];
         group_stats64(xv, eps, mu, var, s);
-        group_codes64<BITS, CODES>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes, code);
+        group_codes64<BITS, CODES>(xv, mu, var, s, tables, bq, table_ok, sum_codes, code);
 
         const int64_t g = group0 + lane;
         if (g < total_groups) {
@@ -285,18 +278,15 @@ act_quant_codes_kernel(const TIN *__restrict__ x, const float *__restrict__ thr,
     constexpr int kLoads = 64 / kVec, kIters = 32 / kVec;              // 16-byte loads per group, per lane and tile
     constexpr int kCodeBits = BYTES ? 8 : BITS;
     __shared__ uint32_t tiles[kWaves][32 * kPitch];
-    __shared__ float lut[L * 64];
-    __shared__ Bucket table[kMaxBuckets + 1];
-    __shared__ int slow_slots[kWaves];
+    __shared__ QuantTables tables;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(thr, cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
     if (BUILDER && wave == kWaves) {
-        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, lane, 64);
+        build_quant_tables<BITS>(load_quant_params<BITS>(thr, cb, lane), tables, lane);
         __syncthreads();
         return;
     }
+    QuantParams params{};
+    if (!BUILDER && wave == 0) params = load_quant_params<BITS>(thr, cb, lane);
     const int64_t ntiles = (total_groups + 31) / 32, step = static_cast<int64_t>(gridDim.x) * kWaves;
     uint32_t *tile = tiles[wave];
     uint4 raw[kIters];
@@ -309,13 +299,13 @@ act_quant_codes_kernel(const TIN *__restrict__ x, const float *__restrict__ thr,
     };
     int64_t t = static_cast<int64_t>(blockIdx.x) * kWaves + wave;
     fetch(t);
+    BucketScale bq{};
     bool table_ok = false, tables_built = false;
     if constexpr (!BUILDER) {
-        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, 64 * kWaves);
+        if (wave == 0) build_quant_tables<BITS>(params, tables, lane);
         __syncthreads();
-        table_ok = true;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
+        bq = tables.geometry;
+        table_ok = tables.usable != 0;
         tables_built = true;
     }
     const int row = lane >> 1, half = lane & 1;
@@ -350,11 +340,12 @@ act_quant_codes_kernel(const TIN *__restrict__ x, const float *__restrict__ thr,
         group_stats32x2(xv, eps, mu, var, s);
         if (BUILDER && !tables_built) {
             __syncthreads();
-            table_ok = slow_slots[0] == 0;
+            bq = tables.geometry;
+            table_ok = tables.usable != 0;
             tables_built = true;
         }
         uint32_t w[kCodeBits];
-        group_codes32x2<BITS, kCodeBits>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes, w);
+        group_codes32x2<BITS, kCodeBits>(xv, mu, var, s, tables, bq, table_ok, sum_codes, w);
         const int64_t g = t * 32 + row;
         if (t < ntiles && g < total_groups) {
             uint8_t *dst = codes + (t * 64 + lane) * (4 * kCodeBits);
@@ -383,25 +374,21 @@ act_quant_small_kernel(const TIN *__restrict__ x, const float *__restrict__ thr,
 {
     constexpr int L = 1 << BITS;
     constexpr int kIn = 32 * sizeof(TIN) / 16, kOut = 32 * sizeof(TOUT) / 16;
-    __shared__ float lut[L * 64];
-    __shared__ Bucket table[kMaxBuckets + 1];
-    __shared__ int slow_slots[kWaves];
+    __shared__ QuantTables tables;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int64_t f = (static_cast<int64_t>(blockIdx.x) * kWaves + (tid >> 6)) * 32 + (lane >> 1);   // this lane's group
     const bool valid = f < total_groups;
     const int64_t e0 = f * 64 + (lane & 1) * 32;                                                    // its first element
 
+    QuantParams params{};
+    if (tid < 64) params = load_quant_params<BITS>(thr, cb, lane);
     uint4 raw[kIn];
 #pragma unroll
     for (int i = 0; i < kIn; ++i)
         raw[i] = valid ? reinterpret_cast<const uint4 *>(x + e0)[i] : make_uint4(0, 0, 0, 0);
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(thr, cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
     // The tables are built while the inputs are still on their way: their latency and the build's overlap (-0.2 us).
-    build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, 64 * kWaves);
-    __syncthreads();
+    if (tid < 64) build_quant_tables<BITS>(params, tables, lane);
 
     float xv[32];
     if constexpr (sizeof(TIN) == 2) {
@@ -423,10 +410,8 @@ act_quant_small_kernel(const TIN *__restrict__ x, const float *__restrict__ thr,
     }
     float mu, var, s, sum_codes;
     group_stats32x2(xv, eps, mu, var, s);
-    bool table_ok = true;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
-    group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
+    __syncthreads();
+    group_codes32x2<BITS>(xv, mu, var, s, tables, tables.geometry, tables.usable != 0, sum_codes);
     const float code_mean = sum_codes * 0.015625f;
 #pragma unroll
     for (int j = 0; j < 32; ++j) xv[j] = fma_f32(s, xv[j] - code_mean, mu);

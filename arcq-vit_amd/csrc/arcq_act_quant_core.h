@@ -5,6 +5,8 @@
 
 #include "arcq_common.h"
 
+#include <type_traits>
+
 namespace arcq {
 
 // ---- FP8 operands (OCP E4M3) ---------------------------------------------------------------------------------------
@@ -49,13 +51,8 @@ constexpr int kMaxBuckets = 512;   // table entries 0 .. nb (nb <= 512); entry n
 constexpr float kBucketBias = 1048576.0f;      // 2^20
 struct BucketScale { float scale, offset; int nb; };      // offset = 8 * scale + 2^20 (exact)
 
-template <int BITS>
-__device__ __forceinline__ BucketScale pick_bucket_scale(const float (&th)[(1 << BITS) - 1])
+__device__ __forceinline__ BucketScale bucket_scale_for(float gap)      // gap: the smallest between neighbouring thresholds
 {
-    constexpr int L = 1 << BITS;
-    float gap = 16.0f;
-#pragma unroll
-    for (int i = 0; i + 1 < L - 1; ++i) gap = fminf(gap, th[i + 1] - th[i]);      // NaN gaps are ignored; checked later
     float scale = 32.0f;
     if (gap * 16.0f > 1.0f) scale = 16.0f;
     if (gap * 8.0f > 1.0f) scale = 8.0f;
@@ -83,61 +80,83 @@ __device__ __forceinline__ uint32_t bucket_offset_of(float t, const BucketScale 
     return __float_as_uint(__fmaf_rn(t, q.scale, q.offset)) & 0x1ff8u;
 }
 
-struct Bucket { float thr; int base; };     // the threshold inside the bucket (+inf if none); thresholds in lower buckets
+struct alignas(8) Bucket { float thr; int base; };     // the threshold inside the bucket (+inf if none); thresholds in lower buckets
 static_assert(sizeof(Bucket) == 8, "bucket_offset_of assumes 8-byte table entries");
 
-template <int BITS>
-__device__ __forceinline__ void load_quant_params(const float *__restrict__ thr, const float *__restrict__ cb,
-                                                  float (&th)[(1 << BITS) - 1], float (&cbv)[1 << BITS])
+// The code: an addition with carry.  (The barrier keeps the compiler from scaling its two operands apart for the lookup that
+// follows: an instruction more per value.)
+__device__ __forceinline__ uint32_t code_in_bucket(const Bucket &bk, bool above)
 {
-    constexpr int L = 1 << BITS;
-#pragma unroll
-    for (int i = 0; i < L - 1; ++i) th[i] = thr[i];
-#pragma unroll
-    for (int c = 0; c < L; ++c) cbv[c] = cb[c];
+    uint32_t c = static_cast<uint32_t>(bk.base) + (above ? 1u : 0u);
+    asm("" : "+v"(c));
+    return c;
 }
 
-// Table construction without barriers, by the `nt` threads numbered t = 0 .. nt-1 (nt a multiple of 64; the calling
-// waves must be complete).  `lut` = codebook replicated per lane (lut[c*64 + lane], conflict-free), `table` = the
-// threshold buckets.  Each participating wave reports through its own slot slow_slots[t / 64] whether the buckets
-// are unusable (two thresholds in one bucket, a threshold outside [-8, 8), unsorted thresholds); the caller
-// synchronizes and ORs the slots.
+// A quantizer's lookup tables in LDS.  `cb` needs no copy per lane: a read of 16 different entries meets no bank twice.
+template <int ENTRIES>
+struct QuantTablesOf {
+    float cb[16], thr[16];
+    BucketScale geometry;
+    int usable;                      // 0: two thresholds in one bucket, one outside [-8, 8), or unsorted ones
+    uint32_t holds[18];              // bit b: bucket b holds a threshold
+    Bucket bucket[ENTRIES];
+};
+using QuantTables = QuantTablesOf<kMaxBuckets + 1>;
+
+// A lane's threshold and codebook value, requested ahead of everything else that the building wave loads (loads complete in the
+// order of their issue: behind a tile's, the tables of a launch of 12 608 x 1 536 values are 0.6 us late).
+struct QuantParams { float thr, cb; };
 template <int BITS>
-__device__ __forceinline__ void build_quant_tables_by(const float (&th)[(1 << BITS) - 1], const float (&cbv)[1 << BITS],
-                                                      const BucketScale &q, float *lut, Bucket *table, int *slow_slots,
-                                                      int t, int nt)
+__device__ __forceinline__ QuantParams load_quant_params(const float *__restrict__ thr, const float *__restrict__ cb, int lane)
 {
     constexpr int L = 1 << BITS;
-    if (t < 64) {
-#pragma unroll
-        for (int c = 0; c < L; ++c) lut[c * 64 + t] = cbv[c];
+    return QuantParams{lane < L - 1 ? thr[lane] : __builtin_huge_valf(), lane < L ? cb[lane] : 0.0f};
+}
+
+// Table construction by ONE complete wave; the caller synchronizes.  Lane i takes threshold i: the smallest gap and the order come
+// from its neighbour's lane, a bit per occupied bucket meets in LDS, and a bucket's number of lower thresholds is the count of
+// lower bits (v_mbcnt).  (Every thread of up to four waves used to go over all thresholds, 15 uniform branches and 95 instructions
+// per 64 buckets with a scalar hazard wait in each: 1.0 us of the 7.8 us that 197 x 384 values with a LayerNorm take.)
+template <int BITS, int ENTRIES>
+__device__ __forceinline__ void build_quant_tables(const QuantParams &p, QuantTablesOf<ENTRIES> &q, int lane)
+{
+    constexpr int L = 1 << BITS;
+    constexpr float inf = __builtin_huge_valf();
+    const float t = p.thr;
+    if (lane < 18) q.holds[lane] = 0;
+    auto dpp = [](float old, float v, auto ctrl) __attribute__((always_inline)) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, false));
+    };
+    const float next = dpp(inf, t, std::integral_constant<int, 0x101>{});        // row_shl:1, lane i + 1's
+    const bool pair = lane < L - 2;
+    bool bad = pair && !(t <= next);
+    float gap = fminf(pair ? next - t : 16.0f, 16.0f);                           // (NaN gaps are ignored: `bad` has them)
+    gap = fminf(gap, dpp(gap, gap, std::integral_constant<int, 0x121>{}));       // row_ror: the minimum of the sixteen lanes
+    gap = fminf(gap, dpp(gap, gap, std::integral_constant<int, 0x122>{}));
+    gap = fminf(gap, dpp(gap, gap, std::integral_constant<int, 0x124>{}));
+    gap = fminf(gap, dpp(gap, gap, std::integral_constant<int, 0x128>{}));
+    const BucketScale g = bucket_scale_for(__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(gap))));
+    const int tb = bucket_of_threshold(t, g);
+    const bool inside = tb >= 0 && tb < g.nb;
+    __builtin_amdgcn_wave_barrier();
+    if (lane < L - 1) {
+        bad = bad || !inside;
+        const uint32_t bit = 1u << (tb & 31);
+        if (inside) bad = bad || (atomicOr(&q.holds[tb >> 5], bit) & bit);
     }
-    int tb[L - 1];
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < L - 1; ++i) {
-        tb[i] = bucket_of_threshold(th[i], q);
-        bad = bad || tb[i] < 0 || tb[i] >= q.nb;
-    }
-#pragma unroll
-    for (int i = 0; i + 1 < L - 1; ++i) bad = bad || !(th[i] <= th[i + 1]);
-    for (int b = t; b <= q.nb; b += nt) {
-        int below = 0, upto = 0;   // thresholds in buckets < b, <= b
-        float inside_thr = __int_as_float(0x7f800000);   // +inf: never exceeded
-#pragma unroll
-        for (int i = 0; i < L - 1; ++i) {
-            below += (tb[i] < b) ? 1 : 0;
-            upto += (tb[i] <= b) ? 1 : 0;
-            inside_thr = (tb[i] == b) ? th[i] : inside_thr;
-        }
-        bad = bad || (upto - below) > 1;
+    if (lane < 16) q.thr[lane] = t, q.cb[lane] = p.cb;
+    const bool usable = !__any(bad);
+    if (lane == 0) q.geometry = g, q.usable = usable;
+    __builtin_amdgcn_wave_barrier();
+    int below = 0;                                                               // thresholds in the buckets before b0
+    for (int b0 = 0; b0 <= g.nb; b0 += 64) {
+        const uint32_t lo = q.holds[b0 >> 5], hi = q.holds[(b0 >> 5) + 1];
         Bucket e;
-        e.base = below;
-        e.thr = inside_thr;
-        table[b] = e;
+        e.base = static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, below)));
+        e.thr = (((lane < 32 ? lo : hi) >> (lane & 31)) & 1u) ? q.thr[min(e.base, 15)] : inf;
+        if (b0 + lane <= g.nb) q.bucket[b0 + lane] = e;
+        below += __popc(lo) + __popc(hi);
     }
-    const bool any_bad = __any(bad);
-    if ((t & 63) == 0) slow_slots[t >> 6] = any_bad ? 1 : 0;
 }
 
 // One group per lane, first half: xv holds the 64 inputs on entry and the residuals d_j = x_j - mu on exit.
@@ -159,15 +178,37 @@ __device__ __forceinline__ void group_stats64(float (&xv)[64], float eps, float 
     s_out = sqrtf(var * 0.015625f + eps);
 }
 
-// Second half: xv holds the residuals on entry and cb[code_j] on exit.  The whole wave must call it (the fast/slow
-// decision is wave-uniform).
-template <int BITS, bool CODES>
-__device__ __forceinline__ void group_codes64(float (&xv)[64], float mu, float var, float s,
-                                              const float (&th)[(1 << BITS) - 1], const BucketScale &bq,
-                                              const Bucket *table, const float *lut, bool table_ok, int lane,
-                                              float &sum_out, uint32_t (&code)[CODES ? 64 : 1])
+// Codes without the buckets: every threshold in turn, while (c < L - 1 && t > thr[c]) ++c; eight values at a time (registers).
+// xv holds the residuals on entry and cb[code_j] on exit; put(j, code).
+template <int BITS, int N, typename Put>
+__device__ __forceinline__ void search_codes(float (&xv)[N], float s, const QuantTables &q, const Put &put)
 {
-    constexpr int L = 1 << BITS;
+#pragma unroll
+    for (int j0 = 0; j0 < N; j0 += 8) {
+        float t[8];
+        uint32_t c[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] = xv[j0 + e] / s, c[e] = 0;
+#pragma unroll 1
+        for (uint32_t i = 0; i + 1 < (1u << BITS); ++i) {
+            const float thr = q.thr[i];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) c[e] += (c[e] == i && t[e] > thr) ? 1u : 0u;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            xv[j0 + e] = q.cb[c[e]];
+            put(j0 + e, c[e]);
+        }
+    }
+}
+
+// Second half: xv holds the residuals on entry and cb[code_j] on exit.  The whole wave must call it (the fast/slow
+// decision is wave-uniform).  `bq`, `table_ok`: q.geometry and q.usable, in registers.
+template <int BITS, bool CODES>
+__device__ __forceinline__ void group_codes64(float (&xv)[64], float mu, float var, float s, const QuantTables &q, const BucketScale &bq,
+                                              bool table_ok, float &sum_out, uint32_t (&code)[CODES ? 64 : 1])
+{
     // Range in which d*y, the residuals and the corrections are exact or harmlessly rounded:
     // s normal and far from the ends, and no non-zero d_j small enough to push a residual
     // into the subnormals (|d_j| >= 2^-90 whenever |mu| >= 2^-66, or all d_j are zero).
@@ -178,38 +219,26 @@ __device__ __forceinline__ void group_codes64(float (&xv)[64], float mu, float v
     if (fast) {
         const float y = 1.0f / s;
         const float ns = -s;
-        const char *lut_lane = reinterpret_cast<const char *>(lut) + lane * 4;      // + 256 c: one shift-add per lookup
 #pragma unroll
         for (int j = 0; j < 64; ++j) {
             const float d = xv[j];
-            float q = d * y;
-            float e = __fmaf_rn(ns, q, d);
-            q = __fmaf_rn(e, y, q);
-            e = __fmaf_rn(ns, q, d);
-            q = __fmaf_rn(e, y, q);        // == RN(d / s)
-            const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(table) + bucket_offset_of(q, bq));
-            const uint32_t c = static_cast<uint32_t>(bk.base) + ((q > bk.thr) ? 1u : 0u);
+            float t = d * y;
+            float e = __fmaf_rn(ns, t, d);
+            t = __fmaf_rn(e, y, t);
+            e = __fmaf_rn(ns, t, d);
+            t = __fmaf_rn(e, y, t);        // == RN(d / s)
+            const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(q.bucket) + bucket_offset_of(t, bq));
+            const uint32_t c = code_in_bucket(bk, t > bk.thr);
             if constexpr (CODES) code[j] = c;
-            const float v = *reinterpret_cast<const float *>(lut_lane + (c << 8));
+            const float v = q.cb[c];
             xv[j] = v;
             sum_codes += v;
         }
     } else {
-#pragma unroll
-        for (int j = 0; j < 64; ++j) {
-            const float t = xv[j] / s;
-            uint32_t c = 0;
-            bool alive = true;
-#pragma unroll
-            for (int i = 0; i < L - 1; ++i) {   // while (c < L-1 && t > thr[c]) ++c
-                alive = alive && (t > th[i]);
-                c += alive ? 1u : 0u;
-            }
+        search_codes<BITS>(xv, s, q, [&](int j, uint32_t c) __attribute__((always_inline)) {
             if constexpr (CODES) code[j] = c;
-            const float v = lut[c * 64 + lane];
-            xv[j] = v;
-            sum_codes += v;
-        }
+            sum_codes += xv[j];
+        });
     }
     sum_out = sum_codes;
 }
@@ -261,12 +290,9 @@ __device__ __forceinline__ void group_stats32x2(float (&xv)[32], float eps, floa
 // whole wave must call it (the fast/slow decision is wave-uniform).  CODE_BITS != 0: the 32 codes too, packed CODE_BITS apart
 // into `words`.
 template <int BITS, int CODE_BITS = 0>
-__device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float var, float s,
-                                                const float (&th)[(1 << BITS) - 1], const BucketScale &bq,
-                                                const Bucket *table, const float *lut, bool table_ok, int lane,
-                                                float &sum_out, uint32_t *words = nullptr)
+__device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float var, float s, const QuantTables &q, const BucketScale &bq,
+                                                bool table_ok, float &sum_out, uint32_t *words = nullptr)
 {
-    constexpr int L = 1 << BITS;
     auto put = [&](int j, uint32_t c) __attribute__((always_inline)) {
         if constexpr (CODE_BITS != 0) {
             const int bit = j * CODE_BITS, d = bit >> 5, sh = bit & 31;
@@ -279,84 +305,21 @@ __device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float
     if (fast) {
         const float y = 1.0f / s;
         const float ns = -s;
-        const char *lut_lane = reinterpret_cast<const char *>(lut) + lane * 4;      // + 256 c: one shift-add per lookup
 #pragma unroll
         for (int j = 0; j < 32; ++j) {
             const float d = xv[j];
-            float q = d * y;
-            float e = __fmaf_rn(ns, q, d);
-            q = __fmaf_rn(e, y, q);
-            e = __fmaf_rn(ns, q, d);
-            q = __fmaf_rn(e, y, q);        // == RN(d / s)
-            const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(table) + bucket_offset_of(q, bq));
-            const uint32_t c = static_cast<uint32_t>(bk.base) + ((q > bk.thr) ? 1u : 0u);
-            xv[j] = *reinterpret_cast<const float *>(lut_lane + (c << 8));
+            float t = d * y;
+            float e = __fmaf_rn(ns, t, d);
+            t = __fmaf_rn(e, y, t);
+            e = __fmaf_rn(ns, t, d);
+            t = __fmaf_rn(e, y, t);        // == RN(d / s)
+            const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(q.bucket) + bucket_offset_of(t, bq));
+            const uint32_t c = code_in_bucket(bk, t > bk.thr);
+            xv[j] = q.cb[c];
             put(j, c);
         }
     } else {
-#pragma unroll
-        for (int j = 0; j < 32; ++j) {
-            const float t = xv[j] / s;
-            uint32_t c = 0;
-            bool alive = true;
-#pragma unroll
-            for (int i = 0; i < L - 1; ++i) {   // while (c < L-1 && t > thr[c]) ++c
-                alive = alive && (t > th[i]);
-                c += alive ? 1u : 0u;
-            }
-            xv[j] = lut[c * 64 + lane];
-            put(j, c);
-        }
-    }
-    sum_out = pair_serial_sum(xv);
-}
-
-// The same with the thresholds of the compare-chain fallback read from LDS in a rolled loop (`th_lds`, L - 1 values)
-// instead of held in registers: for callers that have no registers to keep them in (a GEMM's epilogue).  Same results.
-template <int BITS>
-__device__ __forceinline__ void group_codes32x2_lds(float (&xv)[32], float mu, float var, float s, const float *th_lds,
-                                                    const BucketScale &bq, const Bucket *table, const float *lut,
-                                                    bool table_ok, int lane, float &sum_out)
-{
-    constexpr int L = 1 << BITS;
-    const bool lane_fast = (s >= 0x1p-60f) && (s <= 0x1p60f) && !(fabsf(mu) < 0x1p-66f && var > 0.0f);
-    const bool fast = table_ok && __all(lane_fast);
-    if (fast) {
-        const float y = 1.0f / s;
-        const float ns = -s;
-        const char *lut_lane = reinterpret_cast<const char *>(lut) + lane * 4;
-#pragma unroll
-        for (int j = 0; j < 32; ++j) {
-            const float d = xv[j];
-            float q = d * y;
-            float e = __fmaf_rn(ns, q, d);
-            q = __fmaf_rn(e, y, q);
-            e = __fmaf_rn(ns, q, d);
-            q = __fmaf_rn(e, y, q);        // == RN(d / s)
-            const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(table) + bucket_offset_of(q, bq));
-            const uint32_t c = static_cast<uint32_t>(bk.base) + ((q > bk.thr) ? 1u : 0u);
-            xv[j] = *reinterpret_cast<const float *>(lut_lane + (c << 8));
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 32; ++j) xv[j] = xv[j] / s;
-#pragma unroll 1
-        for (int j = 0; j < 32; ++j) {
-            // (element j of a register array under a rolled loop: select it with a compare chain instead of indexing)
-            float t = 0.0f;
-#pragma unroll
-            for (int q = 0; q < 32; ++q) t = (q == j) ? xv[q] : t;
-            uint32_t c = 0;
-            bool alive = true;
-#pragma unroll 1
-            for (int i = 0; i < L - 1; ++i) {   // while (c < L-1 && t > thr[c]) ++c
-                alive = alive && (t > th_lds[i]);
-                c += alive ? 1u : 0u;
-            }
-            const float v = lut[c * 64 + lane];
-#pragma unroll
-            for (int q = 0; q < 32; ++q) xv[q] = (q == j) ? v : xv[q];
-        }
+        search_codes<BITS>(xv, s, q, put);
     }
     sum_out = pair_serial_sum(xv);
 }
@@ -368,32 +331,15 @@ __device__ __forceinline__ void group_codes32x2_lds(float (&xv)[32], float mu, f
 // have done on the stored tensor (two lanes per group, same arithmetic, same bits), and writes x_hat into the
 // consumer's 32-row block layout.  The consumer's lookup tables live in LDS (built once per workgroup by
 // next_quant_setup).
-// LDS of the consumer's quantizer: [codebook per lane: L x 64 floats][buckets][per-wave flags: 64 bytes]
-// [thresholds: 16 floats][bucket geometry: scale, offset, number of buckets].
-constexpr int next_quant_lds_bytes(int bits) { return (1 << bits) * 64 * 4 + (kMaxBuckets + 64) * 8 + 64 + 64 + 16; }
+// LDS of the consumer's quantizer.
+constexpr int next_quant_lds_bytes() { return (static_cast<int>(sizeof(QuantTables)) + 15) / 16 * 16; }
 
-// All `nthreads` threads of the workgroup call this (before a barrier that precedes the first epilogue): the
-// consumer's lookup tables into `lds` (next_quant_lds_bytes(BITS) bytes, 16-byte aligned).
+// One wave of the workgroup makes the consumer's lookup tables in `lds` (next_quant_lds_bytes() bytes, 16-byte aligned), before a
+// barrier that precedes the first epilogue.
 template <int BITS>
-__device__ __forceinline__ void next_quant_setup(const float *__restrict__ thr, const float *__restrict__ cb,
-                                                 unsigned char *lds, int tid, int nthreads)
+__device__ __forceinline__ void next_quant_setup(const QuantParams &p, unsigned char *lds, int lane)
 {
-    constexpr int L = 1 << BITS;
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(thr, cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
-    float *lut = reinterpret_cast<float *>(lds);
-    Bucket *table = reinterpret_cast<Bucket *>(lut + L * 64);
-    int *slots = reinterpret_cast<int *>(table + kMaxBuckets + 64);
-    build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slots, tid, nthreads);
-    float *th_lds = reinterpret_cast<float *>(slots + 16);
-    if (tid == 0) {
-#pragma unroll
-        for (int i = 0; i < L - 1; ++i) th_lds[i] = th[i];
-        th_lds[16] = bq.scale;
-        th_lds[17] = bq.offset;
-        reinterpret_cast<int *>(th_lds)[18] = bq.nb;
-    }
+    build_quant_tables<BITS>(p, *reinterpret_cast<QuantTables *>(lds), lane);
 }
 
 // One staged chunk (32 rows x 64 fp16 values, the rows `pitch` bytes apart) -> x_hat of the consuming layer.
@@ -402,40 +348,31 @@ __device__ __forceinline__ void next_quant_setup(const float *__restrict__ thr, 
 // the row is stored.  F8: the consumer's operands are FP8 (16 values a piece); `pad`: the chunk is the last of a row whose
 // length is an odd number of groups, and the row's padding to 128 values is written too.  The whole wave calls it.
 template <int BITS, bool F8 = false>
-__device__ __forceinline__ void next_quant_rows(const unsigned char *lds, int nwaves,
-                                                const unsigned char *stage, int pitch, int lane, bool gelu, float eps,
+__device__ __forceinline__ void next_quant_rows(const unsigned char *lds, const unsigned char *stage, int pitch, int lane, bool gelu, float eps,
                                                 void *dst, int rows, bool live, bool pad = false)
 {
     typedef uint32_t u32x4_nq __attribute__((ext_vector_type(4)));
-    constexpr int L = 1 << BITS;
-    const float *lut = reinterpret_cast<const float *>(lds);
-    const Bucket *table = reinterpret_cast<const Bucket *>(lut + L * 64);
-    const int *slots = reinterpret_cast<const int *>(table + kMaxBuckets + 64);
-    const float *th_lds = reinterpret_cast<const float *>(slots + 16);
-    BucketScale bq;
-    bq.scale = th_lds[16];
-    bq.offset = th_lds[17];
-    bq.nb = reinterpret_cast<const int *>(th_lds)[18];
+    const QuantTables &q = *reinterpret_cast<const QuantTables *>(lds);
+    const BucketScale bq = q.geometry;
+    const bool usable = q.usable != 0;
     const int r = lane >> 1, hf = lane & 1;
     float v[32];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const u32x4_nq q = *reinterpret_cast<const u32x4_nq *>(stage + r * pitch + hf * 64 + i * 16);
+        const u32x4_nq w = *reinterpret_cast<const u32x4_nq *>(stage + r * pitch + hf * 64 + i * 16);
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-            v[8 * i + 2 * d] = __half2float(__ushort_as_half(static_cast<unsigned short>(q[d] & 0xffffu)));
-            v[8 * i + 2 * d + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(q[d] >> 16)));
+            v[8 * i + 2 * d] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[d] & 0xffffu)));
+            v[8 * i + 2 * d + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[d] >> 16)));
         }
     }
     if (gelu) {
 #pragma unroll
         for (int j = 0; j < 32; ++j) v[j] = __half2float(__float2half_rn(gelu_f32(v[j])));
     }
-    bool ok = true;
-    for (int w = 0; w < nwaves; ++w) ok = ok && (slots[w] == 0);
     float mu, var, s, sum;
     group_stats32x2(v, eps, mu, var, s);
-    group_codes32x2_lds<BITS>(v, mu, var, s, th_lds, bq, table, lut, ok, lane, sum);
+    group_codes32x2<BITS>(v, mu, var, s, q, bq, usable, sum);
     const float code_mean = sum * 0.015625f;
     char *out = static_cast<char *>(dst);
     if constexpr (F8) {
@@ -464,13 +401,13 @@ __device__ __forceinline__ void next_quant_rows(const unsigned char *lds, int nw
 // The same for a chunk whose 32 rows are block `blk` of the consumer's operand at x_hat (N values a row, M rows): c0 = the
 // chunk's first column.
 template <int BITS, bool F8>
-__device__ __forceinline__ void next_quant_block(const unsigned char *lds, int nwaves, const unsigned char *stage, int pitch,
+__device__ __forceinline__ void next_quant_block(const unsigned char *lds, const unsigned char *stage, int pitch,
                                                  int lane, bool gelu, float eps, void *x_hat, int blk, int M, int N, int c0)
 {
     const int r = lane >> 1, rows = min(32, M - blk * 32);
     const int row_bytes = F8 ? (N + 127) / 128 * 128 : N * 2;
     char *dst = static_cast<char *>(x_hat) + static_cast<int64_t>(blk) * 32 * row_bytes + (static_cast<int64_t>(F8 ? c0 / 16 : c0 / 8) * rows + r) * 16;
-    next_quant_rows<BITS, F8>(lds, nwaves, stage, pitch, lane, gelu, eps, dst, rows, r < rows, F8 && c0 + 64 == N && (N & 64) != 0);
+    next_quant_rows<BITS, F8>(lds, stage, pitch, lane, gelu, eps, dst, rows, r < rows, F8 && c0 + 64 == N && (N & 64) != 0);
 }
 
 }  // namespace arcq

@@ -43,51 +43,77 @@ __device__ __forceinline__ bool in_range(float v) { return (v == 0.0f) | ((fabsf
 // with two thresholds in one bucket one code more than there are.  Both tables have an entry for it.
 template <typename TIN> constexpr int kTableEntries = sizeof(TIN) == 4 ? 0x1ff8 / static_cast<int>(sizeof(Bucket)) + 1 : kMaxBuckets + 1;
 
-// One pixel: its three channels quantized and reconstructed in place.  Returns whether every quotient was in range (FAST).
-template <int BITS, bool FAST, bool HALF>
-__device__ __forceinline__ bool quantize_pixel(float (&x)[kC], float eps, const float (&th)[(1 << BITS) - 1], const float (&cbv)[1 << BITS],
-                                               const BucketScale &bq, const Bucket *table, const char *lut_lane)
+// Eight pixels quantized and reconstructed in place, every operation rounded as IEEE has it.
+template <int BITS, typename Tables>
+__device__ __forceinline__ void quantize_pixels(float (&x)[8][kC], float eps, const Tables &q)
 {
-    constexpr int L = 1 << BITS;
+    constexpr float fgs = static_cast<float>(kC);
+    float mu[8], s[8];
+    uint32_t code[8][kC];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float sum = 0.0f, var = 0.0f;
+#pragma unroll
+        for (int c = 0; c < kC; ++c) sum += x[e][c];
+        mu[e] = sum / fgs;
+#pragma unroll
+        for (int c = 0; c < kC; ++c) {
+            x[e][c] -= mu[e];
+            var += x[e][c] * x[e][c];
+        }
+        s[e] = sqrtf(var / fgs + eps);
+#pragma unroll
+        for (int c = 0; c < kC; ++c) x[e][c] = x[e][c] / s[e], code[e][c] = 0;
+    }
+#pragma unroll 1
+    for (uint32_t i = 0; i + 1 < (1u << BITS); ++i) {      // while (code < L - 1 && t > thr[code]) ++code
+        const float thr = q.thr[i];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int c = 0; c < kC; ++c) code[e][c] += (code[e][c] == i && x[e][c] > thr) ? 1u : 0u;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float sum_codes = 0.0f;
+#pragma unroll
+        for (int c = 0; c < kC; ++c) {
+            x[e][c] = q.cb[code[e][c]];
+            sum_codes += x[e][c];
+        }
+        const float code_mean = sum_codes / fgs;
+#pragma unroll
+        for (int c = 0; c < kC; ++c) x[e][c] = fma_f32(s[e], x[e][c] - code_mean, mu[e]);
+    }
+}
+
+// One pixel on the tables.  Returns whether every quotient was in range.
+template <int BITS, bool HALF, typename Tables>
+__device__ __forceinline__ bool quantize_pixel_fast(float (&x)[kC], float eps, const BucketScale &bq, const Tables &q)
+{
     constexpr float third = 1.0f / 3.0f;
-    const float fgs = static_cast<float>(kC);
-    auto by3 = [&](float v) { return FAST ? quotient(v, fgs, third) : v / fgs; };
     float sum = 0.0f;
 #pragma unroll
     for (int c = 0; c < kC; ++c) sum += x[c];
-    const float mu = by3(sum);
+    const float mu = quotient(sum, 3.0f, third);
     float var = 0.0f;
 #pragma unroll
     for (int c = 0; c < kC; ++c) {
         x[c] -= mu;
         var += x[c] * x[c];
     }
-    const float s = sqrtf(by3(var) + eps);
-    float y = 0.0f, sum_codes = 0.0f;
-    if constexpr (FAST) y = 1.0f / s;
+    const float s = sqrtf(quotient(var, 3.0f, third) + eps);
+    const float y = 1.0f / s;
+    float sum_codes = 0.0f;
 #pragma unroll
     for (int c = 0; c < kC; ++c) {
-        float v;
-        if constexpr (FAST) {
-            const float t = quotient(x[c], s, y);
-            const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(table) + bucket_offset_of(t, bq));
-            const uint32_t code = static_cast<uint32_t>(bk.base) + ((t > bk.thr) ? 1u : 0u);
-            v = *reinterpret_cast<const float *>(lut_lane + (code << 8));
-        } else {
-            // while (code < L - 1 && t > thr[code]) ++code, with the codebook value picked along the way
-            const float t = x[c] / s;
-            v = cbv[0];
-            bool alive = true;
-#pragma unroll
-            for (int q = 0; q < L - 1; ++q) {
-                alive = alive && (t > th[q]);
-                v = alive ? cbv[q + 1] : v;
-            }
-        }
+        const float t = quotient(x[c], s, y);
+        const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(q.bucket) + bucket_offset_of(t, bq));
+        const float v = q.cb[code_in_bucket(bk, t > bk.thr)];
         x[c] = v;
         sum_codes += v;
     }
-    const float code_mean = by3(sum_codes);
+    const float code_mean = quotient(sum_codes, 3.0f, third);
 #pragma unroll
     for (int c = 0; c < kC; ++c) x[c] = fma_f32(s, x[c] - code_mean, mu);
     // d_c is 0 or at least 2^-90 once |mu| >= 2^-66 or all of them are 0 -- and for fp16 inputs (HALF), multiples of 2^-24, always:
@@ -104,10 +130,8 @@ act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ 
 {
     constexpr int L = 1 << BITS;
     constexpr int kIn = 8 * static_cast<int>(sizeof(TIN)) / 16;
-    __shared__ float lut[(L + 1) * 64];
-    __shared__ Bucket table[kTableEntries<TIN>];
-    __shared__ int slow_slots[kPrepWaves];
-    if (prep_weight_workgroup<BITS, false>(weights, PrepWeights{}, lut)) return;
+    __shared__ QuantTablesOf<kTableEntries<TIN>> tables;
+    if (prep_weight_workgroup<BITS, false>(weights, PrepWeights{}, tables.cb)) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int lr = lane & 31, lh = lane >> 5;
     const int pw = W / kP, np = (H / kP) * pw;
@@ -126,18 +150,17 @@ act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ 
 #pragma unroll
             for (int j = 0; j < kIn; ++j) raw[c][j] = reinterpret_cast<const uint4 *>(src + c * plane)[j];
     };
+    QuantParams params{};
+    if (tid < 64) params = load_quant_params<BITS>(thr, cb, lane);
     fetch(item);
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(thr, cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
-    build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, kPrepThreads);
-    if constexpr (sizeof(TIN) == 4)
-        for (int b = bq.nb + 1 + tid; b < kTableEntries<TIN>; b += kPrepThreads) table[b] = Bucket{__int_as_float(0x7f800000), 0};
+    if (tid < 64) {
+        build_quant_tables<BITS>(params, tables, lane);
+        if constexpr (sizeof(TIN) == 4)
+            for (int b = tables.geometry.nb + 1 + lane; b < kTableEntries<TIN>; b += 64) tables.bucket[b] = Bucket{__builtin_huge_valf(), 0};
+    }
     __syncthreads();
-    bool table_ok = true;
-#pragma unroll
-    for (int w = 0; w < kPrepWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
-    const char *lut_lane = reinterpret_cast<const char *>(lut) + lane * 4;
+    const BucketScale bq = tables.geometry;
+    const bool table_ok = tables.usable;
 
     for (; item < items; item += step) {
         float x[8][kC];
@@ -161,11 +184,10 @@ act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ 
         unpack();
         bool ok = table_ok;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ok = ok & quantize_pixel<BITS, true, sizeof(TIN) == 2>(x[e], eps, th, cbv, bq, table, lut_lane);
+        for (int e = 0; e < 8; ++e) ok = ok & quantize_pixel_fast<BITS, sizeof(TIN) == 2>(x[e], eps, bq, tables);
         if (!__all(ok)) {
             unpack();
-#pragma unroll
-            for (int e = 0; e < 8; ++e) quantize_pixel<BITS, false, sizeof(TIN) == 2>(x[e], eps, th, cbv, bq, table, lut_lane);
+            quantize_pixels<BITS>(x, eps, tables);
         }
         const int blk = item >> 4, i = item & 15, m = blk * 32 + lr;
         fetch(item + step);                                    // (the next item's pixels while this one's leave)

@@ -51,7 +51,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
     constexpr int NCH = (NKB + CH - 1) / CH;
     __shared__ __attribute__((aligned(16))) unsigned char ks[kKeys * kKPitch];
     __shared__ __attribute__((aligned(16))) unsigned char vt[kHeadDim * kVPitch];
-    __shared__ __attribute__((aligned(16))) unsigned char nq_lds[NQ ? next_quant_lds_bytes(NQ ? NQ : 2) : 16];
+    __shared__ __attribute__((aligned(16))) unsigned char nq_lds[NQ ? next_quant_lds_bytes() : 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lh = lane >> 5;
     const int h = blockIdx.x, b = blockIdx.y;
@@ -62,6 +62,10 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
     // ---- K row-major and V transposed into LDS (keys past n as zeros).  16 NKB key pairs x 8 pieces of 8 dims =
     //      exactly two items per thread; all eight loads are in flight before the first LDS write ----
     const u32x4_t zero4 = {0u, 0u, 0u, 0u};
+    QuantParams nq_params{};
+    if constexpr (NQ != 0) {                                   // (the last wave has the fewest queries)
+        if (wave == NKB - 1) nq_params = load_quant_params<NQ>(nq_thr, nq_cb, lane);
+    }
     u32x4_t kreg[2][2], vreg[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -74,7 +78,9 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
             vreg[i][j] = key < n ? *reinterpret_cast<const u32x4_t *>(src + C) : zero4;
         }
     }
-    if constexpr (NQ != 0) next_quant_setup<NQ>(nq_thr, nq_cb, nq_lds, tid, 64 * NKB);       // while K and V are on their way
+    if constexpr (NQ != 0) {                                   // while K and V are on their way
+        if (wave == NKB - 1) next_quant_setup<NQ>(nq_params, nq_lds, lane);
+    }
     // ---- this wave's queries: lane (q, half) holds Q[q][16 kk + 8 half ... + 7] for kk = 0..3 ----
     const int q = wave * 32 + lr;
     u32x4_t qf[4];
@@ -205,7 +211,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
         const int nrows = min(32, total_rows - blk * 32);
         const int row_bytes = F8 ? (C + 127) / 128 * 128 : C * 2;
         char *dst = reinterpret_cast<char *>(out) + static_cast<int64_t>(blk) * 32 * row_bytes + (static_cast<int64_t>(h) * (F8 ? 4 : 8) * nrows + (row & 31)) * 16;
-        next_quant_rows<NQ, F8>(nq_lds, NKB, stage, kKPitch, lane, false, 1.0e-6f, dst, nrows, qr < n, F8 && h == H - 1 && (H & 1) != 0);
+        next_quant_rows<NQ, F8>(nq_lds, stage, kKPitch, lane, false, 1.0e-6f, dst, nrows, qr < n, F8 && h == H - 1 && (H & 1) != 0);
         return;
     }
     // ---- normalise, round, store: each lane 4 runs of 4 consecutive dims per 32-dim block ----

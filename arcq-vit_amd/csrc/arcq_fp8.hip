@@ -90,12 +90,10 @@ act_quant_fp8_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
                      uint8_t *__restrict__ x8, float eps, int groups_per_row, int64_t rows, const Fp8Carry carry)
 {
     constexpr int L = 1 << BITS;
-    __shared__ float lut[L * 64];
-    __shared__ Bucket table[kMaxBuckets + 1];
-    __shared__ int slow_slots[kFp8Waves];
+    __shared__ QuantTables tables;
     if constexpr (BLK) {
         if (static_cast<int>(blockIdx.x) < carry.blocks) {      // a weight workgroup (workgroup-uniform)
-            float *s_cb = lut;
+            float *s_cb = tables.cb;
             if (threadIdx.x < L) s_cb[threadIdx.x] = carry.cb[threadIdx.x];
             __syncthreads();
             weight_dequant_fp8_share<BITS>(carry.packed, s_cb, carry.center, carry.scale, carry.code_sum, carry.w8, carry.N,
@@ -108,14 +106,10 @@ act_quant_fp8_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
     const int wg = BLK ? static_cast<int>(blockIdx.x) - carry.blocks : static_cast<int>(blockIdx.x);
     const int n_wg = BLK ? static_cast<int>(gridDim.x) - carry.blocks : static_cast<int>(gridDim.x);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(thr, cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
-    build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, 64 * kFp8Waves);
+    if (wave == 0) build_quant_tables<BITS>(load_quant_params<BITS>(thr, cb, lane), tables, lane);
     __syncthreads();
-    bool table_ok = true;
-#pragma unroll
-    for (int w = 0; w < kFp8Waves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
+    const BucketScale bq = tables.geometry;
+    const bool table_ok = tables.usable != 0;
 
     const int row = lane >> 1, half = lane & 1;
     const int64_t K = static_cast<int64_t>(groups_per_row) * 64;
@@ -149,7 +143,7 @@ act_quant_fp8_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
         }
         float mu, var, s, sum_codes;
         group_stats32x2(xv, eps, mu, var, s);
-        group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
+        group_codes32x2<BITS>(xv, mu, var, s, tables, bq, table_ok, sum_codes);
         const float code_mean = sum_codes * 0.015625f;
         uint32_t out[8];
 #pragma unroll

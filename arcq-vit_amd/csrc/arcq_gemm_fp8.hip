@@ -101,7 +101,9 @@ gemm_fp8_kernel(const uint8_t *__restrict__ xb, const float *__restrict__ bias, 
 
     if (tid < kSlabN) s_bias[tid] = (bias && n_base + tid < N) ? bias[n_base + tid] : 0.0f;
     unsigned char *nq_lds = smem + Fp8Cfg<WAVES, SG, DB>::kSmem;
-    if constexpr (NQ != 0) next_quant_setup<NQ>(nx_thr, nx_cb, nq_lds, tid, 64 * WAVES);      // (the first slab fill's barriers publish it)
+    if constexpr (NQ != 0) {      // (the first slab fill's barriers publish it)
+        if (wave == 0) next_quant_setup<NQ>(load_quant_params<NQ>(nx_thr, nx_cb, lane), nq_lds, lane);
+    }
     // Direct global -> LDS loads: the slab is filled as one flat run of 16-byte pieces (piece p = row * kPieces +
     // column; the hardware writes lane l's piece at the wave-uniform LDS base + 16 l), 64 pieces per instruction
     // whatever the row length; padding pieces and the columns past a short last slice are skipped.  The caller
@@ -298,7 +300,7 @@ gemm_fp8_kernel(const uint8_t *__restrict__ xb, const float *__restrict__ bias, 
                 if constexpr (NQ != 0) {
                     const int c0 = n_base + jb * 32 + ch * kChunkCols;          // the chunk is one group of the consumer's rows
                     if (c0 < N)
-                        next_quant_block<NQ, true>(nq_lds, kWaves, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
+                        next_quant_block<NQ, true>(nq_lds, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
                     __builtin_amdgcn_wave_barrier();
                     continue;
                 }
@@ -490,7 +492,7 @@ gemm_fp8_kernel(const uint8_t *__restrict__ xb, const float *__restrict__ bias, 
 template <typename TOUT, int NQ>
 void launch_fp8_t(const GemmArgs &g, const void *w8, hipStream_t stream)
 {
-    constexpr int kSmem = Fp8Cfg<8, 3, true>::kSmem + (NQ ? next_quant_lds_bytes(NQ) : 0);
+    constexpr int kSmem = Fp8Cfg<8, 3, true>::kSmem + (NQ ? next_quant_lds_bytes() : 0);
     allow_dynamic_lds<gemm_fp8_kernel<TOUT, 8, 3, true, NQ>>(kSmem);
     // Row ranges: one workgroup per compute unit (tiles = slabs x ranges ~ the number of compute units).
     const int n_slabs = (g.N + kSlabN - 1) / kSlabN;

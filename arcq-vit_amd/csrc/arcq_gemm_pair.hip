@@ -105,7 +105,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
     if (tid < kSlabN) s_bias[tid] = (bias && n_base + tid < N) ? bias[n_base + tid] : 0.0f;
     const unsigned char *nq_lds = smem + PairCfg<WAVES, SG, DB>::kSmem;
     if constexpr (NQ != 0)      // (the barriers of the first slab fill publish the tables)
-        next_quant_setup<NQ>(nx_thr, nx_cb, smem + PairCfg<WAVES, SG, DB>::kSmem, tid, 64 * WAVES);
+        if (wave == 0) next_quant_setup<NQ>(load_quant_params<NQ>(nx_thr, nx_cb, lane), smem + PairCfg<WAVES, SG, DB>::kSmem, lane);
     // Direct global -> LDS loads: the slab is filled as one flat run of 16-byte pieces (piece p = row * kPieces +
     // column; the hardware writes lane l's piece at the wave-uniform LDS base + 16 l), 64 pieces per instruction
     // whatever the row length; padding pieces and the columns past a short last slice are skipped.  The caller
@@ -285,7 +285,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
                 if constexpr (NQ != 0) {
                     const int c0 = n_base + jb * 32 + ch * kChunkCols;          // the chunk is one group of the consumer's rows
                     if (c0 < N)
-                        next_quant_block<NQ, false>(nq_lds, kWaves, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
+                        next_quant_block<NQ, false>(nq_lds, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
                     __builtin_amdgcn_wave_barrier();
                     continue;
                 }
@@ -478,7 +478,7 @@ template <typename TOUT, int WAVES, int SG, bool DB, int NQ = 0>
 void launch_pair_t(const GemmArgs &g, hipStream_t stream, const void *w_hat, int ranges, int blocks_per_range)
 {
     auto kernel = gemm_pair_kernel<TOUT, WAVES, SG, DB, NQ>;
-    constexpr int kSmem = PairCfg<WAVES, SG, DB>::kSmem + (NQ ? next_quant_lds_bytes(NQ) : 0);
+    constexpr int kSmem = PairCfg<WAVES, SG, DB>::kSmem + (NQ ? next_quant_lds_bytes() : 0);
     allow_dynamic_lds<gemm_pair_kernel<TOUT, WAVES, SG, DB, NQ>>(kSmem);
     const int n_slabs = (g.N + kSlabN - 1) / kSlabN;
     const int tiles = n_slabs * ranges;

@@ -156,7 +156,7 @@ gemm_slab8_kernel(const __half *__restrict__ xb, const uint8_t *__restrict__ pw,
     if (tid < kSlabN) s_bias[tid] = (bias && n_base + tid < N) ? bias[n_base + tid] : 0.0f;
     const unsigned char *nq_lds = reinterpret_cast<const unsigned char *>(s_bias + kSlabN);
     if constexpr (NQ != 0)      // (the barriers of the first slab fill publish the tables)
-        next_quant_setup<NQ>(nx_thr, nx_cb, reinterpret_cast<unsigned char *>(s_bias + kSlabN), tid, kThreads);
+        if (wave == 0) next_quant_setup<NQ>(load_quant_params<NQ>(nx_thr, nx_cb, lane), reinterpret_cast<unsigned char *>(s_bias + kSlabN), lane);
     // PRE: one direct global -> LDS load per slab row (lanes 0..47 carry the row's 48 16-byte pieces, the hardware
     // writes lane l's piece at the wave-uniform LDS base + 16 l); the caller waits for vmcnt and the barrier.
     auto copy_slice = [&](int g0, int ng) __attribute__((always_inline)) {
@@ -393,7 +393,7 @@ gemm_slab8_kernel(const __half *__restrict__ xb, const uint8_t *__restrict__ pw,
                 if constexpr (NQ != 0) {
                     const int c0 = n_base + jb * 32 + ch * kChunkCols;          // the chunk is one group of the consumer's rows
                     if (c0 < N)
-                        next_quant_block<NQ, false>(nq_lds, kWaves, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
+                        next_quant_block<NQ, false>(nq_lds, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
                     __builtin_amdgcn_wave_barrier();
                     continue;
                 }
@@ -455,7 +455,7 @@ void launch_slab8_w(const GemmArgs &g, hipStream_t stream, const void *w_hat)
 {
     constexpr int L = 1 << BITS;
     const size_t smem = kSlabBytes + WAVES * kStageTile + L * 64 * sizeof(float) + kSlabN * sizeof(float) +
-                        (NQ ? next_quant_lds_bytes(NQ) : 0);
+                        (NQ ? next_quant_lds_bytes() : 0);
     auto kernel = gemm_slab8_kernel<BITS, TOUT, PRE, WAVES, AHEAD, NQ>;
     allow_dynamic_lds<gemm_slab8_kernel<BITS, TOUT, PRE, WAVES, AHEAD, NQ>>(static_cast<int>(smem));
     // One workgroup per CU where possible: split the 32-row blocks into as many ranges as CUs/slabs allow.

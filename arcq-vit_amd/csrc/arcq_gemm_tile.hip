@@ -144,7 +144,9 @@ gemm_tile_kernel(const unsigned char *__restrict__ xb, const unsigned char *__re
         }
     };
     for (int i = tid; i < TN; i += kThreads) s_bias[i] = (bias && n0 + i < N) ? bias[n0 + i] : 0.0f;
-    if constexpr (NQ != 0) next_quant_setup<NQ>(nx_thr, nx_cb, nq_lds, tid, kThreads);
+    if constexpr (NQ != 0) {
+        if (wave == 0) next_quant_setup<NQ>(load_quant_params<NQ>(nx_thr, nx_cb, lane), nq_lds, lane);
+    }
     wait_vm<0>();          // nothing but the operand loads is outstanding from here to the epilogue
 #pragma unroll
     for (int s = 0; s < kStages - 1; ++s)
@@ -218,7 +220,7 @@ gemm_tile_kernel(const unsigned char *__restrict__ xb, const unsigned char *__re
             const int rb = job % RBT, gc = job / RBT;
             const int blk = m0 / 32 + rb, c0 = n0 + gc * 64;
             if (blk < row_blocks && c0 < N)
-                next_quant_block<NQ, F8>(nq_lds, kWaves, smem + rb * 32 * kOutPitch + gc * 128, kOutPitch, lane, gelu != 0, 1.0e-6f, y, blk, M,
+                next_quant_block<NQ, F8>(nq_lds, smem + rb * 32 * kOutPitch + gc * 128, kOutPitch, lane, gelu != 0, 1.0e-6f, y, blk, M,
                                          N, c0);
         }
     } else {
@@ -243,7 +245,7 @@ gemm_tile_kernel(const unsigned char *__restrict__ xb, const unsigned char *__re
 template <int TM, int TN, int WM, int WN, typename TOUT, int NQ, bool F8>
 void launch_tile(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 {
-    constexpr int kSmem = kStages * (TM / 32 + TN / 32) * kGroupBytes + TN * 4 + (NQ ? next_quant_lds_bytes(NQ) : 0);
+    constexpr int kSmem = kStages * (TM / 32 + TN / 32) * kGroupBytes + TN * 4 + (NQ ? next_quant_lds_bytes() : 0);
     allow_dynamic_lds<gemm_tile_kernel<TM, TN, WM, WN, TOUT, NQ, F8>>(kSmem);
     const int mt = (g.M + TM - 1) / TM, nt = (g.N + TN - 1) / TN;
     const int m_fastest = g.M < g.N ? 1 : 0;
@@ -293,11 +295,17 @@ gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char
         }
     };
     Ops o0, o1;
+    QuantParams nq_params{};
+    if constexpr (NQ != 0) {                                          // (the last wave: without operands of its own up to seven groups)
+        if (wave == NW - 1) nq_params = load_quant_params<NQ>(nx_thr, nx_cb, lane);
+    }
     if (wave < G) fetch(wave, o0);
     if (wave + NW < G) fetch(wave + NW, o1);
     // The consumer's lookup tables while the first operands are on their way.
     unsigned char *nq_lds = smem + NW * RT * kPitch;
-    if constexpr (NQ != 0) next_quant_setup<NQ>(nx_thr, nx_cb, nq_lds, tid, 64 * NW);
+    if constexpr (NQ != 0) {
+        if (wave == NW - 1) next_quant_setup<NQ>(nq_params, nq_lds, lane);
+    }
 
     float16_t acc[RB][CB];
 #pragma unroll
@@ -393,7 +401,7 @@ gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char
         if (wave < RB) {
             const int blk = m0 / 32 + wave;
             if (blk < row_blocks && n0 < N)
-                next_quant_block<NQ, false>(nq_lds, NW, smem + wave * 32 * kStageRow, kStageRow, lane, false, 1.0e-6f, y, blk, M, N, n0);
+                next_quant_block<NQ, false>(nq_lds, smem + wave * 32 * kStageRow, kStageRow, lane, false, 1.0e-6f, y, blk, M, N, n0);
         }
     } else if (live) {
         if (residual || gelu) {
@@ -408,7 +416,7 @@ gemm_tile_split_kernel(const unsigned char *__restrict__ xb, const unsigned char
 template <typename TOUT, int RB, int CB, int NQ>
 void launch_split(const GemmArgs &g, const void *w_hat, hipStream_t stream)
 {
-    constexpr int kSmem = 8 * 32 * RB * (32 * CB * 4 + 16) + (NQ ? next_quant_lds_bytes(NQ) : 0);
+    constexpr int kSmem = 8 * 32 * RB * (32 * CB * 4 + 16) + (NQ ? next_quant_lds_bytes() : 0);
     allow_dynamic_lds<gemm_tile_split_kernel<TOUT, RB, CB, NQ>>(kSmem);
     const dim3 grid((g.N + 32 * CB - 1) / (32 * CB), (g.M + 32 * RB - 1) / (32 * RB));
     hipLaunchKernelGGL((gemm_tile_split_kernel<TOUT, RB, CB, NQ>), grid, dim3(512), kSmem, stream,

@@ -126,9 +126,7 @@ otf_rows_kernel(const RowsParams p)
     static_assert(ROUNDS * WV == 2 * G, "waves must divide the 2 G stage-1 tiles");
     constexpr int kStage = rows_stage_bytes(ROUNDS, sizeof(TOUT));  // bytes of a wave's output staging tile
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    __shared__ float lut[L * 64];
-    __shared__ Bucket table[kMaxBuckets + 1];
-    __shared__ int slow_slots[MAXW];
+    __shared__ QuantTables tables;
     __shared__ int s_flag;
 
     constexpr int K = 64 * G, W = WV;
@@ -145,6 +143,9 @@ otf_rows_kernel(const RowsParams p)
     // The wave's stage-1 inputs (wave = (row block rb2, group g): 32 rows x 64 values; a lane pair holds one row's 64,
     // each lane 64 contiguous bytes) are requested first, so that they travel while the weights are rebuilt.
     // (tile t = wave + round * W: row block t / G, group t % G)
+    constexpr int kBuilder = W < 4 ? 0 : 1;
+    QuantParams params{};
+    if (wave == kBuilder) params = load_quant_params<BITS>(p.thr, p.cb_a, lane);
     uint4 raws[ROUNDS][4];
 #pragma unroll
     for (int rnd = 0; rnd < ROUNDS; ++rnd) {
@@ -160,11 +161,8 @@ otf_rows_kernel(const RowsParams p)
     // ---- this workgroup's share of w_hat: the inputs of this thread's first piece are requested here, the piece is
     // finished under stage 1's set-up ----
     // Division of the extra work over the waves (stage 1 is instruction-bound and waves w, w + 4, w + 8 share a SIMD):
-    // waves 1-3 build the activation lookup tables, the others reconstruct the weight pieces -- wave 0 and waves 4..
-    // are piece threads 0..63, 64.. -- so that no SIMD carries more than one builder and one piece wave beside
-    // its plain ones (two piece waves on SIMD 0).
-    constexpr int kBuilders = W < 4 ? 1 : 3;
-    constexpr int kBuilder0 = W < 4 ? 0 : 1;
+    // wave 1 builds the activation lookup tables, wave 0 and waves 4.. reconstruct the weight pieces as threads 0..63,
+    // 64.. -- so that no SIMD carries more than two of them (two piece waves on SIMD 0).
     constexpr int kPieceThreads = W < 4 ? 64 * W : 64 * (W - 3);
     const int ptid = W < 4 ? tid : (wave == 0 ? lane : (wave >= 4 ? (wave - 3) * 64 + lane : -1));
     int64_t share_lo = 0, share_hi = 0;
@@ -200,14 +198,7 @@ otf_rows_kernel(const RowsParams p)
     // ---- stage 1: wave = (row block rb2, group g), two lanes per (row, group) ----
     for (int i = tid; i < p.N; i += nthreads) s_bias[i] = p.bias ? p.bias[i] : 0.0f;
     {
-        float th[L - 1], cbv[L];
-        load_quant_params<BITS>(p.thr, p.cb_a, th, cbv);
-        const BucketScale bq = pick_bucket_scale<BITS>(th);
-        // The lookup tables are built by three waves while the tiles are on their way (every participating thread
-        // pays ~250 instructions of set-up whether or not it owns a table entry: all 2 G waves building cost 17 % of
-        // the phase).
-        if (wave >= kBuilder0 && wave < kBuilder0 + kBuilders)
-            build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid - 64 * kBuilder0, 64 * kBuilders);
+        if (wave == kBuilder) build_quant_tables<BITS>(params, tables, lane);      // while the tiles are on their way
         if (own_share) {
             if (ptid >= 0 && share_lo + ptid < share_hi) finish_piece<BITS>(p, share_lo + ptid, pc);
             for (int64_t idx = share_lo + kPieceThreads + ptid; ptid >= 0 && idx < share_hi; idx += kPieceThreads) {     // (large N*K only)
@@ -279,11 +270,9 @@ otf_rows_kernel(const RowsParams p)
                 }
             }
         }
-        bool table_ok = true;
-        for (int w = 0; w < kBuilders; ++w) table_ok = table_ok && (slow_slots[w] == 0);
         float mu, var, s, sum_codes;
         group_stats32x2(xv, p.eps, mu, var, s);
-        group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
+        group_codes32x2<BITS>(xv, mu, var, s, tables, tables.geometry, tables.usable != 0, sum_codes);
         const float code_mean = sum_codes * 0.015625f;
         unsigned char *dst = xs + (rb2 * 32 + row) * pitch + g * 128 + half * 64;
 #pragma unroll
@@ -512,9 +501,7 @@ otf_rows_phased_kernel(const RowsParams p)
     constexpr int W = 2 * G, GT = G * PHASES, K = 64 * GT, KS = 64 * G;
     static_assert(G % 2 == 0, "the two-slot fragment ring must close on a slice boundary");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    __shared__ float lut[L * 64];
-    __shared__ Bucket table[kMaxBuckets + 1];
-    __shared__ int slow_slots[W];
+    __shared__ QuantTables tables;
     __shared__ int s_flag;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -539,10 +526,12 @@ otf_rows_phased_kernel(const RowsParams p)
         for (int i = 0; i < 4; ++i)
             raw[i] = my_row < p.M ? *reinterpret_cast<const uint4 *>(src + i * 8) : make_uint4(0, 0, 0, 0);
     };
+    constexpr int kBuilder = 1;
+    QuantParams params{};
+    if (wave == kBuilder) params = load_quant_params<BITS>(p.thr, p.cb_a, lane);
     load_slice(0);
 
     // ---- this workgroup's share of w_hat and the lookup tables, as in otf_rows_kernel ----
-    constexpr int kBuilders = 3, kBuilder0 = 1;
     constexpr int kPieceThreads = 64 * (W - 3);
     const int ptid = wave == 0 ? lane : (wave >= 4 ? (wave - 3) * 64 + lane : -1);
     int64_t share_lo = 0, share_hi = 0;
@@ -556,11 +545,7 @@ otf_rows_phased_kernel(const RowsParams p)
         if (ptid >= 0 && share_lo + ptid < share_hi) fetch_piece<BITS, GT>(p, share_lo + ptid, pc);
     }
     for (int i = tid; i < 32 * W * NB; i += nthreads) s_bias[i] = (p.bias && i < p.N) ? p.bias[i] : 0.0f;
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(p.thr, p.cb_a, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
-    if (wave >= kBuilder0 && wave < kBuilder0 + kBuilders)
-        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid - 64 * kBuilder0, 64 * kBuilders);
+    if (wave == kBuilder) build_quant_tables<BITS>(params, tables, lane);
     if (p.counter) {
         if (ptid >= 0 && share_lo + ptid < share_hi) finish_piece<BITS>(p, share_lo + ptid, pc);
         for (int64_t idx = share_lo + kPieceThreads + ptid; ptid >= 0 && idx < share_hi; idx += kPieceThreads) {
@@ -575,8 +560,8 @@ otf_rows_phased_kernel(const RowsParams p)
         const unsigned long long old = __hip_atomic_fetch_add(p.counter, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         target = (old & ~(kEpoch - 1)) + kEpoch;
     }
-    bool table_ok = true;
-    for (int w = 0; w < kBuilders; ++w) table_ok = table_ok && (slow_slots[w] == 0);
+    const BucketScale bq = tables.geometry;
+    const bool table_ok = tables.usable != 0;
 
     // ---- product role: wave = the 32-column blocks wave, wave + W, ... (idle in the product if it has none) ----
     const int lr = lane & 31, lh = lane >> 5;
@@ -616,7 +601,7 @@ otf_rows_phased_kernel(const RowsParams p)
         if (ph + 1 < PHASES) load_slice(ph + 1);
         float mu, var, s, sum_codes;
         group_stats32x2(xv, p.eps, mu, var, s);
-        group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
+        group_codes32x2<BITS>(xv, mu, var, s, tables, bq, table_ok, sum_codes);
         const float code_mean = sum_codes * 0.015625f;
         unsigned char *dst = xs + (ph & 1) * kBuf + (rb2 * 32 + row) * pitch + g * 128 + half * 64;
 #pragma unroll

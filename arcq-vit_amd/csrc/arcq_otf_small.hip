@@ -107,16 +107,14 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
     constexpr int kOsCols = 32 * CB;
     constexpr int kOsRedPitch = os_red_pitch(CB);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    // [x_hat tile | partial tiles] [activation LUT] [weight LUT] [buckets] [per-wave flags]; the partial tiles of
+    // [x_hat tile | partial tiles] [weight codebook] [lookup tables]; the partial tiles of
     // the reduction follow the x_hat tile (partial_off == tile_bytes) or, when K is too long for both, reuse its space
     // (partial_off == 0) after a barrier.
     unsigned char *xt = smem;
     unsigned char *partial = smem + partial_off;
     const int front = max(tile_bytes, partial_off + kOsWaves * RT * kOsRedPitch);
-    float *a_lut = reinterpret_cast<float *>(smem + front);
-    float *w_lut = a_lut + L * 64;
-    Bucket *table = reinterpret_cast<Bucket *>(w_lut + L * 64);
-    int *slow_slots = reinterpret_cast<int *>(table + kMaxBuckets + 64);
+    float *w_lut = reinterpret_cast<float *>(smem + front);
+    QuantTables &tables = *reinterpret_cast<QuantTables *>(w_lut + 16);
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -256,15 +254,8 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
     const int tile_waves = spare_waves ? n_tiles : kOsWaves;
     const bool has_tile = wave < n_tiles;
     if (has_tile) fetch_x(wave);
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(a_thr, a_cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
-    if (spare_waves && !has_tile)
-        build_quant_tables_by<BITS>(th, cbv, bq, a_lut, table, slow_slots, tid - tile_waves * 64, (kOsWaves - tile_waves) * 64);
-    if (wave == kOsWaves - 1) {
-#pragma unroll
-        for (int c = 0; c < L; ++c) w_lut[c * 64 + lane] = w_cb[c];
-    }
+    if (wave == (spare_waves ? tile_waves : 0)) build_quant_tables<BITS>(load_quant_params<BITS>(a_thr, a_cb, lane), tables, lane);
+    if (wave == kOsWaves - 1 && lane < L) w_lut[lane] = w_cb[lane];
     if (has_tile) {
         stats();
         if (wave + kOsWaves < n_tiles) fetch_x(wave + kOsWaves);      // the next tile's inputs, one round ahead
@@ -272,25 +263,15 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
         if constexpr (LPG == 1) group_stats64(xv, eps, mu, var, s);
         else group_stats32x2(xv, eps, mu, var, s);
     }
-    if (!spare_waves) build_quant_tables_by<BITS>(th, cbv, bq, a_lut, table, slow_slots, tid, kOsWaves * 64);
     __syncthreads();
+    const BucketScale bq = tables.geometry;
+    const bool table_ok = tables.usable != 0;
     const bool write_ws = (x_hat_ws != nullptr) && blockIdx.x == 0;
-    bool table_ok = true;
-    for (int w = 0; w < (spare_waves ? kOsWaves - tile_waves : kOsWaves); ++w) table_ok = table_ok && (slow_slots[w] == 0);
     // Quantize-the-output mode (nx_thr != nullptr: y receives stage 1 of the layer that consumes this one's output):
     // that layer's lookup tables are built by the waves without a stage-1 tile while the others run theirs, or, when
     // every wave has a tile, by all of them behind it.
-    float *n_lut = reinterpret_cast<float *>(smem + nx_off);
-    Bucket *n_table = reinterpret_cast<Bucket *>(n_lut + L * 64);
-    int *n_slots = reinterpret_cast<int *>(n_table + kMaxBuckets + 64);
-    const int n_builders = spare_waves ? kOsWaves - tile_waves : kOsWaves;
-    auto build_next_tables = [&]() {
-        float nth[L - 1], ncb[L];
-        load_quant_params<BITS>(nx_thr, nx_cb, nth, ncb);
-        const BucketScale nbq = pick_bucket_scale<BITS>(nth);
-        build_quant_tables_by<BITS>(nth, ncb, nbq, n_lut, n_table, n_slots, tid - (kOsWaves - n_builders) * 64, n_builders * 64);
-    };
-    if (nx_thr && spare_waves && !has_tile) build_next_tables();
+    QuantTables &n_tables = *reinterpret_cast<QuantTables *>(smem + nx_off);
+    if (nx_thr && spare_waves && wave == tile_waves) build_quant_tables<BITS>(load_quant_params<BITS>(nx_thr, nx_cb, lane), n_tables, lane);
     for (int t = wave; t < n_tiles; t += kOsWaves) {
         if (t != wave) {                       // later tiles of this wave: their inputs were requested a round ago
             stats();
@@ -305,9 +286,9 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
         float sum_codes;
         if constexpr (LPG == 1) {
             uint32_t code[1];
-            group_codes64<BITS, false>(xv, mu, var, s, th, bq, table, a_lut, table_ok, lane, sum_codes, code);
+            group_codes64<BITS, false>(xv, mu, var, s, tables, bq, table_ok, sum_codes, code);
         } else {
-            group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, a_lut, table_ok, lane, sum_codes);
+            group_codes32x2<BITS>(xv, mu, var, s, tables, bq, table_ok, sum_codes);
         }
         const float code_mean = sum_codes * 0.015625f;
         u32x4_t out[EL / 8];
@@ -331,7 +312,7 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
             for (int i = 0; i < EL / 8; ++i) dst[i] = out[i];
         }
     }
-    if (nx_thr && !spare_waves) build_next_tables();
+    if (nx_thr && !spare_waves && wave == 0) build_quant_tables<BITS>(load_quant_params<BITS>(nx_thr, nx_cb, lane), n_tables, lane);
     __syncthreads();
 
     // The thread's outputs in the epilogue (E consecutive ones of a row) are known now: their bias and residual values
@@ -377,7 +358,6 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
-    const char *lut_lane = reinterpret_cast<const char *>(w_lut) + lane * 4;
     const unsigned char *a_lane = xt + lr * row_pitch + lh * 64;
     auto compute = [&](int g, const OsWeights<BITS, CB> &o) {
         float mg[CB];
@@ -389,7 +369,7 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
         for (int j = 0; j < CB; ++j)
 #pragma unroll
             for (int q = 0; q < 32; ++q)
-                wv[j][q] = *reinterpret_cast<const float *>(lut_lane + (os_code_at<BITS>(o.codes[j], q) << 8));
+                wv[j][q] = w_lut[os_code_at<BITS>(o.codes[j], q)];
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
             half8_t bf[CB];
@@ -459,11 +439,6 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
             *reinterpret_cast<u32x2_t *>(yt + row * 144 + col * 2) = *reinterpret_cast<const u32x2_t *>(out);
             __syncthreads();
             if (wave == 0) {
-                float nth[L - 1], ncb[L];
-                load_quant_params<BITS>(nx_thr, nx_cb, nth, ncb);
-                const BucketScale nbq = pick_bucket_scale<BITS>(nth);
-                bool n_ok = true;
-                for (int w = 0; w < n_builders; ++w) n_ok = n_ok && (n_slots[w] == 0);
                 const int r2 = lane >> 1, half = lane & 1;
                 float v[32];
 #pragma unroll
@@ -477,7 +452,7 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
                 }
                 float nmu, nvar, ns, nsum;
                 group_stats32x2(v, eps, nmu, nvar, ns);
-                group_codes32x2<BITS>(v, nmu, nvar, ns, nth, nbq, n_table, n_lut, n_ok, lane, nsum);
+                group_codes32x2<BITS>(v, nmu, nvar, ns, n_tables, n_tables.geometry, n_tables.usable != 0, nsum);
                 const float code_mean = nsum * 0.015625f;
                 if (m0 + r2 < M) {
                     u32x4_t *dst = reinterpret_cast<u32x4_t *>(y + static_cast<int64_t>(m0 + r2) * N + n0 + half * 32);
@@ -536,7 +511,6 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
 template <typename TIN, int BITS, typename TOUT, int RB, int LPG, int CB>
 static void launch_os(const OtfSmallArgs &a, hipStream_t stream)
 {
-    constexpr int L = 1 << BITS;
     constexpr int RT = 32 * RB;
     constexpr int kOsCols = 32 * CB;
     constexpr int kOsRedPitch = os_red_pitch(CB);
@@ -544,16 +518,14 @@ static void launch_os(const OtfSmallArgs &a, hipStream_t stream)
     const int xhat_bytes = RT * os_row_pitch(G);
     const int partial_bytes = kOsWaves * RT * kOsRedPitch;
     const int tile_bytes = xhat_bytes;
-    // (lookup tables, per-wave flags, and -- with a LayerNorm in front -- 128 floats per wave for the rows' partial sums)
-    const size_t tables = 2 * L * 64 * sizeof(float) + (kMaxBuckets + 64) * sizeof(Bucket) + 64;
+    // (the weights' codebook, lookup tables, and -- with a LayerNorm in front -- 128 floats per wave for the rows' partial sums)
+    const size_t tables = 64 + next_quant_lds_bytes();
     const size_t ln_bytes = a.ln_weight ? kOsWaves * 128 * sizeof(float) : 0;
     // Both regions side by side while they fit 160 KB of LDS; else the partial tiles reuse the x_hat tile's space.
-    const size_t nx_need = a.next_thr ? L * 64 * sizeof(float) + (kMaxBuckets + 64) * sizeof(Bucket) + 64 : 0;
-    const int partial_off = (tile_bytes + partial_bytes + tables + ln_bytes + nx_need <= 160 * 1024) ? tile_bytes : 0;
+    const size_t nx_bytes = a.next_thr ? next_quant_lds_bytes() : 0;      // (a second set of lookup tables, for the consuming layer's codebook)
+    const int partial_off = (tile_bytes + partial_bytes + tables + ln_bytes + nx_bytes <= 160 * 1024) ? tile_bytes : 0;
     const size_t front = partial_off ? tile_bytes + partial_bytes : (tile_bytes > partial_bytes ? tile_bytes : partial_bytes);
     const int ln_off = static_cast<int>(front + tables);
-    // (quantize-the-output mode: a second set of lookup tables, for the consuming layer's codebook)
-    const size_t nx_bytes = a.next_thr ? L * 64 * sizeof(float) + (kMaxBuckets + 64) * sizeof(Bucket) + 64 : 0;
     const int nx_off = static_cast<int>(front + tables + ln_bytes);
     const size_t smem = front + tables + ln_bytes + nx_bytes;
     auto kernel = otf_small_kernel<TIN, BITS, TOUT, RB, LPG, CB>;

@@ -37,7 +37,6 @@ __global__ void __launch_bounds__(64 * (kPrepWaves + (BUILDER ? 1 : 0)))
 prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const float *__restrict__ cb, char *__restrict__ x_hat, float eps,
                int rows, int G, PrepWeights w0, PrepWeights w1)
 {
-    constexpr int L = 1 << BITS;
     constexpr int kInPitch = PrepTile<TIN>::pitch;
     constexpr int kLoads = 64 / PrepTile<TIN>::vec;        // 16-byte loads per row of the tile (8 fp16 / 16 fp32)
     constexpr int kRowsPerInstr = 64 / kLoads;             // 8 / 4
@@ -45,19 +44,16 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const f
     constexpr int kPieces = F8 ? 4 : 8;                    // 16-byte pieces of a group of x_hat
     constexpr int kOutDwords = kPieces * 4, kOutPitch = kOutDwords + 1;
     __shared__ uint32_t tiles[kPrepWaves][32 * kInPitch];
-    __shared__ float lut[L * 64];
-    __shared__ Bucket table[kMaxBuckets + 1];
-    __shared__ int slow_slots[kPrepWaves];
-    if (prep_weight_workgroup<BITS, F8>(w0, w1, lut)) return;
+    __shared__ QuantTables tables;
+    if (prep_weight_workgroup<BITS, F8>(w0, w1, tables.cb)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(thr, cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
     if (BUILDER && wave == kPrepWaves) {
-        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, lane, 64);
+        build_quant_tables<BITS>(load_quant_params<BITS>(thr, cb, lane), tables, lane);
         __syncthreads();
         return;
     }
+    QuantParams params{};
+    if (!BUILDER && wave == 0) params = load_quant_params<BITS>(thr, cb, lane);
     const int wg = blockIdx.x - (w0.blocks + w1.blocks), wgs = gridDim.x - (w0.blocks + w1.blocks);
     const int tiles_total = ((rows + 31) / 32) * G;
     const int64_t K = static_cast<int64_t>(G) * 64;
@@ -76,14 +72,14 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const f
                                                                       : make_uint4(0, 0, 0, 0);
     };
     fetch(wg * kPrepWaves + wave);
+    BucketScale bq{};
     bool table_ok = false, tables_built = false;
     const int row = lane >> 1, half = lane & 1;
     if constexpr (!BUILDER) {
-        build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, kPrepThreads);
+        if (wave == 0) build_quant_tables<BITS>(params, tables, lane);
         __syncthreads();
-        table_ok = true;
-#pragma unroll
-        for (int w = 0; w < kPrepWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
+        bq = tables.geometry;
+        table_ok = tables.usable != 0;
         tables_built = true;
     }
     for (int tile0 = wg * kPrepWaves; tile0 < tiles_total; tile0 += wgs * kPrepWaves) {
@@ -117,10 +113,11 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const f
         group_stats32x2(xv, eps, mu, var, s);
         if (BUILDER && !tables_built) {                    // once per workgroup: the builder wave's tables are ready
             __syncthreads();
-            table_ok = (slow_slots[0] == 0);
+            bq = tables.geometry;
+            table_ok = tables.usable != 0;
             tables_built = true;
         }
-        group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
+        group_codes32x2<BITS>(xv, mu, var, s, tables, bq, table_ok, sum_codes);
         const float code_mean = sum_codes * 0.015625f;
         {
             uint32_t *dst = tile + row * kOutPitch + half * (kOutDwords / 2);
@@ -166,20 +163,25 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const f
 // of a sum are in flight together, and gamma and beta lie in LDS (pitch 36 per 32 values: conflict-free 16-byte reads).  With
 // one read per loop trip and gamma / beta from L2: see the figures at the launch.
 constexpr int kGammaPitch = 36;
-template <typename TIN, int BITS>
-__global__ void __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(4)))
+// BUILDER: as above; the tables and gamma / beta are first needed behind the first tile's row sums.
+template <typename TIN, int BITS, bool BUILDER>
+__global__ void __launch_bounds__(64 * (kPrepWaves + (BUILDER ? 1 : 0))) __attribute__((amdgpu_waves_per_eu(4)))
 prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta, float ln_eps,
                   const float *__restrict__ thr, const float *__restrict__ cb, char *__restrict__ x_hat, float eps, int rows,
                   int G, int R, int tiles, PrepWeights w0, PrepWeights w1)
 {
-    constexpr int L = 1 << BITS;
     constexpr int kIn = 32 * static_cast<int>(sizeof(TIN)) / 16;       // 16-byte loads per lane (32 values)
     extern __shared__ __attribute__((aligned(16))) unsigned char prep_smem[];
-    __shared__ float lut[L * 64];
-    __shared__ Bucket table[kMaxBuckets + 1];
-    __shared__ int slow_slots[kPrepWaves];
-    if (prep_weight_workgroup<BITS, false>(w0, w1, lut)) return;
+    __shared__ QuantTables tables;
+    if (prep_weight_workgroup<BITS, false>(w0, w1, tables.cb)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (BUILDER && wave == kPrepWaves) {
+        build_quant_tables<BITS>(load_quant_params<BITS>(thr, cb, lane), tables, lane);
+        __syncthreads();
+        return;
+    }
+    QuantParams params{};
+    if (!BUILDER && wave == 0) params = load_quant_params<BITS>(thr, cb, lane);
     const int wg = blockIdx.x - (w0.blocks + w1.blocks), wgs = gridDim.x - (w0.blocks + w1.blocks);
     const int P = 2 * G;                                    // lanes per row
     const int rl = lane / P, pl = lane - rl * P;            // row of the wave, lane of the row
@@ -208,14 +210,9 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
         *reinterpret_cast<float4 *>(s_beta + at) = bv;
     }
     for (int i = lane; i < R * chunks * 8; i += 64) part[i] = 0.0f;
-    float th[L - 1], cbv[L];
-    load_quant_params<BITS>(thr, cb, th, cbv);
-    const BucketScale bq = pick_bucket_scale<BITS>(th);
-    build_quant_tables_by<BITS>(th, cbv, bq, lut, table, slow_slots, tid, kPrepThreads);      // while the first tile is on its way
-    __syncthreads();
-    bool table_ok = true;
-#pragma unroll
-    for (int w = 0; w < kPrepWaves; ++w) table_ok = table_ok && (slow_slots[w] == 0);
+    if (!BUILDER && wave == 0) build_quant_tables<BITS>(params, tables, lane);      // while the first tile is on its way
+    BucketScale bq{};
+    bool table_ok = false, ready = false;
     const float fk = static_cast<float>(K);
     float *my_part = part + (lane_used ? rl : 0) * (chunks * 8);
     const float *my_gamma = s_gamma + (lane_used ? pl : 0) * kGammaPitch, *my_beta = s_beta + (lane_used ? pl : 0) * kGammaPitch;
@@ -281,6 +278,12 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
             q += sq;
         }
         const float rstd = 1.0f / sqrtf(row_total(q) / fk + ln_eps);
+        if (!ready) {                                       // once per workgroup: the tables, gamma and beta are in LDS
+            __syncthreads();
+            bq = tables.geometry;
+            table_ok = tables.usable != 0;
+            ready = true;
+        }
 #pragma unroll
         for (int j4 = 0; j4 < 8; ++j4) {
             const float4 gv = *reinterpret_cast<const float4 *>(my_gamma + 4 * j4), bv = *reinterpret_cast<const float4 *>(my_beta + 4 * j4);
@@ -296,7 +299,7 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
         }
         float mu, var, s, sum_codes;
         group_stats32x2(xv, eps, mu, var, s);
-        group_codes32x2<BITS>(xv, mu, var, s, th, bq, table, lut, table_ok, lane, sum_codes);
+        group_codes32x2<BITS>(xv, mu, var, s, tables, bq, table_ok, sum_codes);
         const float code_mean = sum_codes * 0.015625f;
         // ---- out: piece (k8, row) at LDS slot k8 * RW + row, then 16 bytes per lane, rows fastest ----
         if (lane_used) {
@@ -342,8 +345,12 @@ void launch_prepare_t(const arcq_prepare_args &a, float eps, const PrepWeights &
                                 static_cast<size_t>(2 * G) * kGammaPitch * 8;
             // Beyond four workgroups per CU the waves walk their tiles: the lookup tables are built once per workgroup.
             const int wgs = std::min(tiles, 4 * device_cus());
-            hipLaunchKernelGGL((prepare_ln_kernel<TIN, BITS>), dim3(weights + wgs), dim3(kPrepThreads), smem, stream, x, a.ln_weight,
-                               a.ln_bias, a.ln_eps, a.thresholds, a.codebook, x_hat, eps, rows, G, R, tiles, w0, w1);
+            if (tiles <= 2 * device_cus())
+                hipLaunchKernelGGL((prepare_ln_kernel<TIN, BITS, true>), dim3(weights + wgs), dim3(kPrepThreads + 64), smem, stream, x, a.ln_weight,
+                                   a.ln_bias, a.ln_eps, a.thresholds, a.codebook, x_hat, eps, rows, G, R, tiles, w0, w1);
+            else
+                hipLaunchKernelGGL((prepare_ln_kernel<TIN, BITS, false>), dim3(weights + wgs), dim3(kPrepThreads), smem, stream, x, a.ln_weight,
+                                   a.ln_bias, a.ln_eps, a.thresholds, a.codebook, x_hat, eps, rows, G, R, tiles, w0, w1);
             return;
         }
     }

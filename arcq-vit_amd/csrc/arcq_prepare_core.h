@@ -63,7 +63,7 @@ __device__ __forceinline__ void weights_fp8x16(const float (&v)[32], int j0, flo
     }
 }
 
-// One wave: columns 32 nb ... + 31 of `wave_groups` groups of a layer's weights.  `lut`: the codebook per lane.
+// One wave: columns 32 nb ... + 31 of `wave_groups` groups of a layer's weights.  `lut`: LDS for the codebook.
 template <int BITS, bool F8>
 __device__ __forceinline__ void prep_weights(const PrepWeights &w, unsigned block, float *lut)
 {
@@ -87,12 +87,8 @@ __device__ __forceinline__ void prep_weights(const PrepWeights &w, unsigned bloc
             s[i] = w.scale[mi + i];
             m[i] = w.code_sum[mi + i];
         }
-    if (threadIdx.x < 64) {
-#pragma unroll
-        for (int q = 0; q < L; ++q) lut[q * 64 + lane] = w.cb[q];
-    }
+    if (threadIdx.x < L) lut[threadIdx.x] = w.cb[threadIdx.x];
     __syncthreads();
-    const char *lut_lane = reinterpret_cast<const char *>(lut) + lane * 4;
     const int row_groups = F8 ? (w.G + 1) / 2 * 2 : w.G;
     constexpr int kPieces = F8 ? 4 : 8;            // 16-byte pieces of a group
     char *dst = static_cast<char *>(w.out) + static_cast<int64_t>(nb) * (row_groups * kPieces * 512) + (g0 * kPieces + half * (kPieces / 2)) * 512 +
@@ -103,7 +99,7 @@ __device__ __forceinline__ void prep_weights(const PrepWeights &w, unsigned bloc
         const float mg = m[i] * 0.015625f;          // S/64, exact
         float v[32];
 #pragma unroll
-        for (int e = 0; e < 32; ++e) v[e] = *reinterpret_cast<const float *>(lut_lane + (prep_code_at<BITS>(codes[i], e) << 8));
+        for (int e = 0; e < 32; ++e) v[e] = lut[prep_code_at<BITS>(codes[i], e)];
 #pragma unroll
         for (int p = 0; p < kPieces / 2; ++p) {
             uint32_t o[4];
@@ -143,10 +139,7 @@ __device__ __forceinline__ void prep_weights_rows(const PrepWeights &w, unsigned
     const uint32_t codes = load_codes8<BITS>(src), more = F8 ? load_codes8<BITS>(src + BITS) : 0;
     const int64_t mi = static_cast<int64_t>(n) * w.G + k / kPieces;
     const float c = w.center[mi], s = w.scale[mi], m = w.code_sum[mi] * 0.015625f;
-    if (threadIdx.x < 64) {
-#pragma unroll
-        for (int q = 0; q < L; ++q) lut[q * 64 + lane] = w.cb[q];
-    }
+    if (threadIdx.x < L) lut[threadIdx.x] = w.cb[threadIdx.x];
     __syncthreads();
     if (!mine) return;
     uint32_t o[4] = {0, 0, 0, 0};
@@ -154,7 +147,7 @@ __device__ __forceinline__ void prep_weights_rows(const PrepWeights &w, unsigned
         if (!padding) {
             float v[32];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) v[e] = lut[(((e < 8 ? codes : more) >> (BITS * (e & 7))) & (L - 1)) * 64 + lane];
+            for (int e = 0; e < 16; ++e) v[e] = lut[((e < 8 ? codes : more) >> (BITS * (e & 7))) & (L - 1)];
             weights_fp8x16(v, 0, m, s, c, w.mult, o);
         }
         store_writethrough16(static_cast<char *>(w.out) + static_cast<int64_t>(idx) * 16, o[0], o[1], o[2], o[3]);
@@ -164,7 +157,7 @@ __device__ __forceinline__ void prep_weights_rows(const PrepWeights &w, unsigned
     for (int d = 0; d < 4; ++d) {
         float v[2];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) v[e] = fma_f32(lut[((codes >> (BITS * (2 * d + e))) & (L - 1)) * 64 + lane] - m, s, c);
+        for (int e = 0; e < 2; ++e) v[e] = fma_f32(lut[(codes >> (BITS * (2 * d + e))) & (L - 1)] - m, s, c);
         const __half2 h = __floats2half2_rn(v[0], v[1]);
         o[d] = *reinterpret_cast<const uint32_t *>(&h);
     }

@@ -1,0 +1,60 @@
+"""A quantizer's lookup tables as each kernel builds them: thresholds that share a bucket, repeat, lie outside the table or are out of
+order (the search goes over all of them then: it stops at the first threshold that is not below the value), at every bucket width."""
+import numpy as np
+import pytest
+import torch
+
+from arcq_vit_amd import _lib, ops, synth
+from test_gpu_patch_conv import _blocked
+from test_gpu_prepared import _linear, _prepare, _stream
+
+pytestmark = pytest.mark.gpu
+INF = float("inf")
+
+
+def _tables(bits):
+    """name -> thresholds"""
+    n = (1 << bits) - 1
+    spread = lambda gap: (torch.arange(n) - (n - 1) / 2) * gap
+    plain = synth.midpoint_thresholds(synth.quantile_codebook(bits))
+    t = {f"gap {g}": spread(g) for g in (0.4, 0.2, 0.1, 0.05, 0.02)}      # 64, 128, 256 and 512 buckets; two in a bucket
+    t["at the ends"] = torch.cat([torch.tensor([-8.0]), plain[1:-1], torch.tensor([7.99])]) if n > 1 else plain
+    t["repeated"], t["out of order"], t["outside"], t["infinite"] = (plain.clone() for _ in range(4))
+    t["repeated"][1] = t["repeated"][0]
+    t["out of order"][[0, 2]] = t["out of order"][[2, 0]]
+    t["outside"][-1] = 8.0
+    t["infinite"][0], t["infinite"][-1] = -INF, INF
+    return {k: v.float().contiguous() for k, v in t.items()}
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+def test_tables(cuda, oracle, bits):
+    cb = synth.quantile_codebook(bits)
+    stage1 = lambda x, thr: oracle.act_quant_c(x.float().numpy(), thr, cb, bits, 64)["x_hat"].astype(np.float16)
+    f32 = synth.make_activation(70, 192, 3)
+    f16 = {m: synth.make_activation(m, k, 5).half() for m, k in ((197, 384), (20000, 64))}     # a wave that builds; more tiles than that
+    bias = synth.make_activation(1, 64, 7).half()
+    qkv = synth.make_activation(2 * 33, 3 * 2 * 64, 9).half()
+    att = ops.attention_fwd(qkv.to(cuda).view(2, 33, -1), 2).reshape(66, 128).cpu()
+    img = synth.make_activation(2 * 3 * 32, 32, 11).view(2, 3, 32, 32)
+    pix = img.permute(0, 2, 3, 1).reshape(-1, 3).contiguous()
+    zeros = torch.zeros(700 * 64, dtype=torch.float16, device=cuda)
+    for name, thr in _tables(bits).items():
+        t, c = thr.to(cuda), cb.to(cuda)
+
+        def same(got, want, what):
+            assert np.array_equal(got.reshape(-1).cpu().numpy().view(np.uint16), want.reshape(-1).view(np.uint16)), (name, what)
+
+        same(ops.quantize_activation_dequant(f32.to(cuda), t, c, bits, 64).half(), stage1(f32, thr), "row-major")
+        for m, x in f16.items():
+            same(_prepare(x.to(cuda), t, c, bits)[0], _blocked(stage1(x, thr)), m)
+        for m in (33, 700):                                                                  # behind a product: split and tile kernel
+            got = _linear(zeros, zeros, bias.to(cuda).float().reshape(-1), m, 64, 64, nq=(t, c), bits=bits)
+            same(got, _blocked(stage1(bias.expand(m, 64).contiguous(), thr)), ("product", m))
+        got = torch.empty(66 * 128, dtype=torch.float16, device=cuda)
+        _lib.check(_lib.load().arcq_attention_quant_fwd(qkv.to(cuda).data_ptr(), t.data_ptr(), c.data_ptr(), bits, got.data_ptr(), 2, 33, 2,
+                                                        64, 0.125, _stream()))
+        same(got, _blocked(stage1(att, thr)), "attention")
+        rows = oracle.act_quant_c(pix.numpy(), thr, cb, bits, 3)["x_hat"].astype(np.float16)
+        rows = rows.reshape(2, 2, 16, 2, 16, 3).transpose(0, 1, 3, 5, 2, 4).reshape(8, 768)
+        same(ops.quantize_patches(img.to(cuda), t, c, bits), rows, "patches")
