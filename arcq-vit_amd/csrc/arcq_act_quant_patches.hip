@@ -13,8 +13,10 @@
 //
 // Bound by the vector ALUs.  With plain divisions (six of them a pixel, about ten instructions each) and the compare chain (45
 // instructions a value at four bits) a pixel took 230 instructions and 64 images 28 us, 19 MB in and 19 MB out (8 us at the copy
-// rate).  The quotients are therefore reciprocal products with two fused corrections and the codes bucket lookups, as in
-// arcq_act_quant_core.h (about 110 instructions); waves walk their items so that a workgroup builds its tables once.
+// rate).  The quotients are therefore reciprocal products with fused corrections and the codes bucket lookups, as in
+// arcq_act_quant_core.h, and root and reciprocal come from one hardware reciprocal root: about 100 instructions a pixel, 64 images
+// 13.5 us, 256 35.7 (with IEEE's square root and division expanded by the compiler and every wave building the tables 16.7 and
+// 42.4).  Waves walk their items so that a workgroup builds its tables once.
 #include "arcq_prepare_core.h"
 #include "arcq_gemm.h"
 
@@ -27,6 +29,30 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kP = 16, kC = 3, kKP = kC * kP * kP;      // patch side, channels, 768 values per patch row
 
+// v / 3 rounded to nearest: the product with RN(1/3), which is within a unit in the last place, and one fused correction.  Exact
+// while the residual stays in the normal range (every mantissa checked on the CPU; |v| >= 2^-100 or v = 0).
+__device__ __forceinline__ float third_of(float v)
+{
+    const float q = v * (1.0f / 3.0f);
+    return __fmaf_rn(__fmaf_rn(-3.0f, q, v), 1.0f / 3.0f, q);
+}
+// The square root rounded to nearest and the reciprocal of that, rounded to nearest: from the hardware's reciprocal root by one
+// coupled iteration (Goldschmidt), a fused correction for the root and two for its reciprocal.  Equal to sqrtf for every float of
+// [2^-100, 2^100) and to the division but for roots whose mantissa is all ones (their reciprocal lies next to a midpoint), at a
+// third of their instructions.
+__device__ __forceinline__ float sqrt_and_reciprocal(float a, float &y)
+{
+    const float r = __builtin_amdgcn_rsqf(a);
+    float g = a * r, h = 0.5f * r;
+    const float e = __fmaf_rn(-h, g, 0.5f);
+    g = __fmaf_rn(g, e, g);
+    h = __fmaf_rn(h, e, h);
+    const float s = __fmaf_rn(__fmaf_rn(-g, g, a), h, g);
+    y = h + h;
+    y = __fmaf_rn(__fmaf_rn(-s, y, 1.0f), y, y);
+    y = __fmaf_rn(__fmaf_rn(-s, y, 1.0f), y, y);
+    return s;
+}
 // RN(d / s) from y = RN(1 / s): exact where neither the operands nor the residuals leave the normal range.
 __device__ __forceinline__ float quotient(float d, float s, float y)
 {
@@ -87,23 +113,26 @@ __device__ __forceinline__ void quantize_pixels(float (&x)[8][kC], float eps, co
     }
 }
 
-// One pixel on the tables.  Returns whether every quotient was in range.
-template <int BITS, bool HALF, typename Tables>
+// One pixel on the tables.  Returns whether every intermediate was in the range where the result is the above's.  SIMPLE (fp16
+// input, eps >= 2^-30, codebook values 0 or within 2^+-60): the sums are multiples of 2^-24 or of 2^-83 and cannot be too small,
+// a variance below 2^-60 vanishes beside eps, d_c is 0 or a multiple of 2^-49, and whatever is not finite shows in s.
+// (Searching with d y alone, exact only where a quotient comes close to a threshold, is 15 instructions less a pixel and slower:
+// one item in five hundred is close, and the wave that has one is what the launch waits for.)
+template <int BITS, bool SIMPLE, typename Tables>
 __device__ __forceinline__ bool quantize_pixel_fast(float (&x)[kC], float eps, const BucketScale &bq, const Tables &q)
 {
-    constexpr float third = 1.0f / 3.0f;
     float sum = 0.0f;
 #pragma unroll
     for (int c = 0; c < kC; ++c) sum += x[c];
-    const float mu = quotient(sum, 3.0f, third);
+    const float mu = third_of(sum);
     float var = 0.0f;
 #pragma unroll
     for (int c = 0; c < kC; ++c) {
         x[c] -= mu;
         var += x[c] * x[c];
     }
-    const float s = sqrtf(quotient(var, 3.0f, third) + eps);
-    const float y = 1.0f / s;
+    float y;
+    const float s = sqrt_and_reciprocal(third_of(var) + eps, y);
     float sum_codes = 0.0f;
 #pragma unroll
     for (int c = 0; c < kC; ++c) {
@@ -113,14 +142,15 @@ __device__ __forceinline__ bool quantize_pixel_fast(float (&x)[kC], float eps, c
         x[c] = v;
         sum_codes += v;
     }
-    const float code_mean = quotient(sum_codes, 3.0f, third);
+    const float code_mean = third_of(sum_codes);
 #pragma unroll
     for (int c = 0; c < kC; ++c) x[c] = fma_f32(s, x[c] - code_mean, mu);
-    // d_c is 0 or at least 2^-90 once |mu| >= 2^-66 or all of them are 0 -- and for fp16 inputs (HALF), multiples of 2^-24, always:
-    // their mean is 0 or at least 2^-26, and a mean of exactly 0 (one pixel in a thousand) leaves d_c = x_c.
+    const bool root_ok = (s >= 0x1p-60f) & (s <= 0x1p60f) & ((__float_as_uint(s) & 0x7fffffu) != 0x7fffffu);
+    if constexpr (SIMPLE) return root_ok;
+    // d_c is 0 or at least 2^-90 once |mu| >= 2^-66 or all of them are 0.
     // (No short circuits: a branch per pixel would keep the eight pixels of a lane from overlapping.)
-    const bool means_ok = HALF | !((fabsf(mu) < 0x1p-66f) & (var > 0.0f));
-    return in_range(sum) & in_range(var) & in_range(sum_codes) & (s >= 0x1p-60f) & (s <= 0x1p60f) & means_ok;
+    const bool means_ok = !((fabsf(mu) < 0x1p-66f) & (var > 0.0f));
+    return in_range(sum) & in_range(var) & in_range(sum_codes) & root_ok & means_ok;
 }
 
 template <typename TIN, int BITS>
@@ -159,8 +189,9 @@ act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ 
             for (int b = tables.geometry.nb + 1 + lane; b < kTableEntries<TIN>; b += 64) tables.bucket[b] = Bucket{__builtin_huge_valf(), 0};
     }
     __syncthreads();
+    constexpr bool kSimple = sizeof(TIN) == 2;
     const BucketScale bq = tables.geometry;
-    const bool table_ok = tables.usable;
+    const bool table_ok = tables.usable && (!kSimple || (eps >= 0x1p-30f && __all(in_range(tables.cb[lane & (L - 1)]))));
 
     for (; item < items; item += step) {
         float x[8][kC];
@@ -184,7 +215,7 @@ act_quant_patches_kernel(const TIN *__restrict__ img, const float *__restrict__ 
         unpack();
         bool ok = table_ok;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ok = ok & quantize_pixel_fast<BITS, sizeof(TIN) == 2>(x[e], eps, bq, tables);
+        for (int e = 0; e < 8; ++e) ok = ok & quantize_pixel_fast<BITS, kSimple>(x[e], eps, bq, tables);
         if (!__all(ok)) {
             unpack();
             quantize_pixels<BITS>(x, eps, tables);
@@ -217,7 +248,8 @@ void launch_patches(const void *img, const float *thr, const float *cb, void *x_
 {
     const int64_t M = static_cast<int64_t>(B) * (H / kP) * (W / kP);
     const int items = static_cast<int>((M + 31) / 32 * 16);
-    const int wgs = std::min((items + kPrepWaves - 1) / kPrepWaves, 4 * device_cus());
+    // (what the chip holds at once: 256 images 35.7 us against 38.3 with four workgroups per CU and 39.3 with six)
+    const int wgs = std::min((items + kPrepWaves - 1) / kPrepWaves, 5 * device_cus());
     hipLaunchKernelGGL((act_quant_patches_kernel<TIN, BITS>), dim3(weights.blocks + wgs), dim3(kPrepThreads), 0, stream,
                        static_cast<const TIN *>(img), thr, cb, static_cast<__half *>(x_hat), B, H, W, eps, blocked, items, weights);
 }
