@@ -368,7 +368,9 @@ __device__ __forceinline__ void next_quant_rows(const unsigned char *lds, const 
     }
     if (gelu) {
 #pragma unroll
-        for (int j = 0; j < 32; ++j) v[j] = __half2float(__float2half_rn(gelu_f32(v[j])));
+        for (int i = 0; i < 4; ++i) gelu_of_halves(v + 8 * i);
+#pragma unroll
+        for (int j = 0; j < 32; ++j) v[j] = __half2float(__float2half_rn(v[j]));
     }
     float mu, var, s, sum;
     group_stats32x2(v, eps, mu, var, s);

@@ -145,3 +145,21 @@ def test_prepared_argument_errors(cuda):
     assert lib.arcq_prepare(ctypes.byref(a), None) == -2
     b.M, b.N, b.K = 4, 33, 64
     assert lib.arcq_linear_prepared(ctypes.byref(b), None) == -4
+
+
+# one output a thread, and eight behind the tile kernel and the one of large launches; neighbouring columns hold neighbouring values
+# (a wave of small values takes a form of its own) or values far apart
+@pytest.mark.parametrize("m", [32, 512, 6400])
+@pytest.mark.parametrize("apart", [False, True])
+def test_gelu_of_every_fp16_value(cuda, m, apart):
+    every = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    if apart:
+        every = every.view(256, 256).t().reshape(-1)
+    n, k = 16384, 64
+    x_hat = torch.zeros(m * k, dtype=torch.float16, device=cuda)
+    w_hat = torch.zeros(n * k, dtype=torch.float16, device=cuda)
+    for part in every.to(cuda).split(n):
+        y = _linear(x_hat, w_hat, part.float(), m, n, k, gelu=True)               # zero operands: the output is the bias
+        want = torch.nn.functional.gelu(part)
+        wrong = ~((y == want) | (y.isnan() & want.isnan())).all(0)
+        assert not bool(wrong.any()), part[wrong][:8]
