@@ -47,9 +47,12 @@ constexpr int kMaxBuckets = 512;   // table entries 0 .. nb (nb <= 512); entry n
 // pair of thresholds (scale * smallest gap > 1), so the usual codebooks need a 65- or 129-entry table instead of 513.
 // f is formed as 2^20 + f in one fma: in that binade a float's unit in the last place is 1/8, so the low mantissa bits
 // of the result ARE 8 * f -- the byte offset of an 8-byte table entry once the three fraction bits are masked off.
-// The map t -> bucket is monotone (fma and the mask are), which is all the code search needs.
+// The map t -> bucket is monotone (fma and the mask are).  t = d/s itself is not formed: f comes from d and an approximate 1/s, which
+// puts a value into its bucket or, within 2^-15 of an edge, into the one beside it; no threshold lies as close to an edge, so both
+// give the same code.
 constexpr float kBucketBias = 1048576.0f;      // 2^20
-struct BucketScale { float scale, offset; int nb; };      // offset = 8 * scale + 2^20 (exact)
+constexpr float kEdgeMargin = 0x1p-12f;        // between a threshold and the edges of its bucket, in buckets
+struct BucketScale { float scale, offset; int nb; };      // offset = 8 * scale + 2^20, or 1/4 more (exact)
 
 __device__ __forceinline__ BucketScale bucket_scale_for(float gap)      // gap: the smallest between neighbouring thresholds
 {
@@ -73,23 +76,42 @@ __device__ __forceinline__ int bucket_of_threshold(float t, const BucketScale &q
     return __float2int_rz(f - kBucketBias);     // exact difference
 }
 
-// Byte offset into the table of the bucket of t = d/s on the fast path: |t| <= 8, so f lies in [0, nb] <= 512 and the
-// offset is bits 3..12 of the biased sum.
-__device__ __forceinline__ uint32_t bucket_offset_of(float t, const BucketScale &q)
+// Whether a threshold lies next to an edge (f rounds to a multiple of 1/8: the edges are at b - 1/16).
+__device__ __forceinline__ bool near_an_edge(float t, const BucketScale &q)
 {
-    return __float_as_uint(__fmaf_rn(t, q.scale, q.offset)) & 0x1ff8u;
+    const float f = __fmaf_rn(t, q.scale, (q.offset - kBucketBias) - 8.0f * q.scale + 0.0625f);
+    return !(fabsf(f - rintf(f)) >= kEdgeMargin);
 }
 
-struct alignas(8) Bucket { float thr; int base; };     // the threshold inside the bucket (+inf if none); thresholds in lower buckets
-static_assert(sizeof(Bucket) == 8, "bucket_offset_of assumes 8-byte table entries");
+// `u`: the threshold inside the bucket (+inf if none), or for a negative one the next float above it; `base`: 4 times the number of
+// thresholds in lower buckets.
+struct alignas(8) Bucket { float u; int base; };
 
-// The code: an addition with carry.  (The barrier keeps the compiler from scaling its two operands apart for the lookup that
-// follows: an instruction more per value.)
-__device__ __forceinline__ uint32_t code_in_bucket(const Bucket &bk, bool above)
+// RN(d / s) > T, the quotient rounded to nearest, without a division: it holds exactly where d / s lies beyond T + h, h half the
+// distance from T to the next float above (a quotient is never halfway between two floats), that is where s u - d + s e 2^-24 < 0
+// with u = T, e = 2^k in T's binade for T >= 0, and u the next float, e = -2^k for T < 0: in both cases e is u without its mantissa.
+// The first difference is a remainder, exact where it is small enough to matter, so the sign of the second is right: with
+// 2^-60 <= s <= 2^58, T = 0 or |T| >= 2^-60, d = 0 or |d| >= 2^-90.  (A quotient rounded to nearest takes a product and four fused
+// corrections where this takes two and a mask: 10 instructions a value with the lookup, now 7.  Stage 1 with a LayerNorm
+// 12 608 x 768 16.1 -> 15.3 us, 50 432 x 1 024 58.0 -> 55.5; behind a product with GELU, 50 432 x 1 024 -> 4 096 616 -> 596 us.)
+struct CodeScale { float s, s24, to_bucket; };
+__device__ __forceinline__ CodeScale code_scale_of(float s, float about_1_over_s, const BucketScale &q)
 {
-    uint32_t c = static_cast<uint32_t>(bk.base) + (above ? 1u : 0u);
-    asm("" : "+v"(c));
-    return c;
+    return CodeScale{s, s * 0x1p-24f, about_1_over_s * q.scale};
+}
+// 4 times the code of d.  In range |d / s| <= 8, f lies in [0, nb] <= 512.25 and the bucket's offset is bits 3..12 of the biased sum.
+__device__ __forceinline__ uint32_t code_offset_of(float d, const CodeScale &c, const BucketScale &q, const Bucket *table)
+{
+    static_assert(sizeof(Bucket) == 8, "the offset assumes 8-byte table entries");
+    const uint32_t at = __float_as_uint(__fmaf_rn(d, c.to_bucket, q.offset)) & 0x1ff8u;
+    const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(table) + at);
+    const float e = __uint_as_float(__float_as_uint(bk.u) & 0xff800000u);
+    const float r = __fmaf_rn(c.s24, e, __fmaf_rn(c.s, bk.u, -d));
+    return ((__float_as_uint(r) >> 31) << 2) + static_cast<uint32_t>(bk.base);
+}
+__device__ __forceinline__ float code_value(const float *cb, uint32_t offset)
+{
+    return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(cb) + offset);
 }
 
 // A quantizer's lookup tables in LDS.  `cb` needs no copy per lane: a read of 16 different entries meets no bank twice.
@@ -97,7 +119,7 @@ template <int ENTRIES>
 struct QuantTablesOf {
     float cb[16], thr[16];
     BucketScale geometry;
-    int usable;                      // 0: two thresholds in one bucket, one outside [-8, 8), or unsorted ones
+    int usable;                      // 0: two thresholds in one bucket, one outside [-8, 8) or at an edge or tiny, or unsorted ones
     uint32_t holds[18];              // bit b: bucket b holds a threshold
     Bucket bucket[ENTRIES];
 };
@@ -135,12 +157,13 @@ __device__ __forceinline__ void build_quant_tables(const QuantParams &p, QuantTa
     gap = fminf(gap, dpp(gap, gap, std::integral_constant<int, 0x122>{}));
     gap = fminf(gap, dpp(gap, gap, std::integral_constant<int, 0x124>{}));
     gap = fminf(gap, dpp(gap, gap, std::integral_constant<int, 0x128>{}));
-    const BucketScale g = bucket_scale_for(__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(gap))));
+    BucketScale g = bucket_scale_for(__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(gap))));
+    if (__any(lane < L - 1 && near_an_edge(t, g))) g.offset += 0.25f;
     const int tb = bucket_of_threshold(t, g);
     const bool inside = tb >= 0 && tb < g.nb;
     __builtin_amdgcn_wave_barrier();
     if (lane < L - 1) {
-        bad = bad || !inside;
+        bad = bad || !inside || near_an_edge(t, g) || (t != 0.0f && fabsf(t) < 0x1p-60f);
         const uint32_t bit = 1u << (tb & 31);
         if (inside) bad = bad || (atomicOr(&q.holds[tb >> 5], bit) & bit);
     }
@@ -151,9 +174,11 @@ __device__ __forceinline__ void build_quant_tables(const QuantParams &p, QuantTa
     int below = 0;                                                               // thresholds in the buckets before b0
     for (int b0 = 0; b0 <= g.nb; b0 += 64) {
         const uint32_t lo = q.holds[b0 >> 5], hi = q.holds[(b0 >> 5) + 1];
+        const int base = static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, below)));
+        const float thr = (((lane < 32 ? lo : hi) >> (lane & 31)) & 1u) ? q.thr[min(base, 15)] : inf;
         Bucket e;
-        e.base = static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, below)));
-        e.thr = (((lane < 32 ? lo : hi) >> (lane & 31)) & 1u) ? q.thr[min(e.base, 15)] : inf;
+        e.u = thr < 0.0f ? __int_as_float(__float_as_int(thr) - 1) : thr + 0.0f;      // (-0 as 0)
+        e.base = 4 * base;
         if (b0 + lane <= g.nb) q.bucket[b0 + lane] = e;
         below += __popc(lo) + __popc(hi);
     }
@@ -209,28 +234,18 @@ template <int BITS, bool CODES>
 __device__ __forceinline__ void group_codes64(float (&xv)[64], float mu, float var, float s, const QuantTables &q, const BucketScale &bq,
                                               bool table_ok, float &sum_out, uint32_t (&code)[CODES ? 64 : 1])
 {
-    // Range in which d*y, the residuals and the corrections are exact or harmlessly rounded:
-    // s normal and far from the ends, and no non-zero d_j small enough to push a residual
-    // into the subnormals (|d_j| >= 2^-90 whenever |mu| >= 2^-66, or all d_j are zero).
-    const bool lane_fast = (s >= 0x1p-60f) && (s <= 0x1p60f) && !(fabsf(mu) < 0x1p-66f && var > 0.0f);
+    // The range that code_offset_of asks for: |d_j| >= 2^-90 whenever |mu| >= 2^-66, or all d_j are zero.
+    const bool lane_fast = (s >= 0x1p-60f) && (s <= 0x1p58f) && !(fabsf(mu) < 0x1p-66f && var > 0.0f);
     const bool fast = table_ok && __all(lane_fast);
 
     float sum_codes = 0.0f;
     if (fast) {
-        const float y = 1.0f / s;
-        const float ns = -s;
+        const CodeScale cs = code_scale_of(s, __builtin_amdgcn_rcpf(s), bq);
 #pragma unroll
         for (int j = 0; j < 64; ++j) {
-            const float d = xv[j];
-            float t = d * y;
-            float e = __fmaf_rn(ns, t, d);
-            t = __fmaf_rn(e, y, t);
-            e = __fmaf_rn(ns, t, d);
-            t = __fmaf_rn(e, y, t);        // == RN(d / s)
-            const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(q.bucket) + bucket_offset_of(t, bq));
-            const uint32_t c = code_in_bucket(bk, t > bk.thr);
-            if constexpr (CODES) code[j] = c;
-            const float v = q.cb[c];
+            const uint32_t c = code_offset_of(xv[j], cs, bq, q.bucket);
+            if constexpr (CODES) code[j] = c >> 2;
+            const float v = code_value(q.cb, c);
             xv[j] = v;
             sum_codes += v;
         }
@@ -300,23 +315,15 @@ __device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float
             if (sh + CODE_BITS > 32) words[d + 1] = c >> (32 - sh);
         }
     };
-    const bool lane_fast = (s >= 0x1p-60f) && (s <= 0x1p60f) && !(fabsf(mu) < 0x1p-66f && var > 0.0f);
+    const bool lane_fast = (s >= 0x1p-60f) && (s <= 0x1p58f) && !(fabsf(mu) < 0x1p-66f && var > 0.0f);      // (as above)
     const bool fast = table_ok && __all(lane_fast);
     if (fast) {
-        const float y = 1.0f / s;
-        const float ns = -s;
+        const CodeScale cs = code_scale_of(s, __builtin_amdgcn_rcpf(s), bq);
 #pragma unroll
         for (int j = 0; j < 32; ++j) {
-            const float d = xv[j];
-            float t = d * y;
-            float e = __fmaf_rn(ns, t, d);
-            t = __fmaf_rn(e, y, t);
-            e = __fmaf_rn(ns, t, d);
-            t = __fmaf_rn(e, y, t);        // == RN(d / s)
-            const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(q.bucket) + bucket_offset_of(t, bq));
-            const uint32_t c = code_in_bucket(bk, t > bk.thr);
-            xv[j] = q.cb[c];
-            put(j, c);
+            const uint32_t c = code_offset_of(xv[j], cs, bq, q.bucket);
+            xv[j] = code_value(q.cb, c);
+            put(j, c >> 2);
         }
     } else {
         search_codes<BITS>(xv, s, q, put);

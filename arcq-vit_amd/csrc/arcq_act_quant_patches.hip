@@ -13,10 +13,10 @@
 //
 // Bound by the vector ALUs.  With plain divisions (six of them a pixel, about ten instructions each) and the compare chain (45
 // instructions a value at four bits) a pixel took 230 instructions and 64 images 28 us, 19 MB in and 19 MB out (8 us at the copy
-// rate).  The quotients are therefore reciprocal products with fused corrections and the codes bucket lookups, as in
-// arcq_act_quant_core.h, and root and reciprocal come from one hardware reciprocal root: about 100 instructions a pixel, 64 images
-// 13.5 us, 256 35.7 (with IEEE's square root and division expanded by the compiler and every wave building the tables 16.7 and
-// 42.4).  Waves walk their items so that a workgroup builds its tables once.
+// rate).  The means are therefore products with fused corrections, the codes bucket lookups without a quotient as in
+// arcq_act_quant_core.h, and root and reciprocal come from one hardware reciprocal root: about 85 instructions a pixel, 128 images
+// 16.1 us and 256 32.2 (IEEE's square root and division expanded by the compiler, quotients by fused corrections and every wave
+// building the tables: 256 42.4).  Waves walk their items so that a workgroup builds its tables once.
 #include "arcq_prepare_core.h"
 #include "arcq_gemm.h"
 
@@ -36,10 +36,8 @@ __device__ __forceinline__ float third_of(float v)
     const float q = v * (1.0f / 3.0f);
     return __fmaf_rn(__fmaf_rn(-3.0f, q, v), 1.0f / 3.0f, q);
 }
-// The square root rounded to nearest and the reciprocal of that, rounded to nearest: from the hardware's reciprocal root by one
-// coupled iteration (Goldschmidt), a fused correction for the root and two for its reciprocal.  Equal to sqrtf for every float of
-// [2^-100, 2^100) and to the division but for roots whose mantissa is all ones (their reciprocal lies next to a midpoint), at a
-// third of their instructions.
+// The square root rounded to nearest, from the hardware's reciprocal root by one coupled iteration (Goldschmidt) and a fused
+// correction: equal to sqrtf for every float of [2^-100, 2^100), at a third of its instructions.  y: the reciprocal, within 2^-22.
 __device__ __forceinline__ float sqrt_and_reciprocal(float a, float &y)
 {
     const float r = __builtin_amdgcn_rsqf(a);
@@ -47,25 +45,13 @@ __device__ __forceinline__ float sqrt_and_reciprocal(float a, float &y)
     const float e = __fmaf_rn(-h, g, 0.5f);
     g = __fmaf_rn(g, e, g);
     h = __fmaf_rn(h, e, h);
-    const float s = __fmaf_rn(__fmaf_rn(-g, g, a), h, g);
     y = h + h;
-    y = __fmaf_rn(__fmaf_rn(-s, y, 1.0f), y, y);
-    y = __fmaf_rn(__fmaf_rn(-s, y, 1.0f), y, y);
-    return s;
-}
-// RN(d / s) from y = RN(1 / s): exact where neither the operands nor the residuals leave the normal range.
-__device__ __forceinline__ float quotient(float d, float s, float y)
-{
-    float q = d * y;
-    float e = __fmaf_rn(-s, q, d);
-    q = __fmaf_rn(e, y, q);
-    e = __fmaf_rn(-s, q, d);
-    return __fmaf_rn(e, y, q);
+    return __fmaf_rn(__fmaf_rn(-g, g, a), h, g);
 }
 __device__ __forceinline__ bool in_range(float v) { return (v == 0.0f) | ((fabsf(v) >= 0x1p-60f) & (fabsf(v) <= 0x1p60f)); }
 
-// The fast form looks every quotient up before it is known to be in range (what it finds otherwise is not used): the payload of an
-// fp32 NaN may name any of the offsets that bucket_offset_of can give (that of an fp16 one, widened, has no bits there), and a table
+// The fast form looks every value up before it is known to be in range (what it finds otherwise is not used): the payload of an
+// fp32 NaN may name any of the offsets that code_offset_of can form (that of an fp16 one, widened, has no bits there), and a table
 // with two thresholds in one bucket one code more than there are.  Both tables have an entry for it.
 template <typename TIN> constexpr int kTableEntries = sizeof(TIN) == 4 ? 0x1ff8 / static_cast<int>(sizeof(Bucket)) + 1 : kMaxBuckets + 1;
 
@@ -116,8 +102,6 @@ __device__ __forceinline__ void quantize_pixels(float (&x)[8][kC], float eps, co
 // One pixel on the tables.  Returns whether every intermediate was in the range where the result is the above's.  SIMPLE (fp16
 // input, eps >= 2^-30, codebook values 0 or within 2^+-60): the sums are multiples of 2^-24 or of 2^-83 and cannot be too small,
 // a variance below 2^-60 vanishes beside eps, d_c is 0 or a multiple of 2^-49, and whatever is not finite shows in s.
-// (Searching with d y alone, exact only where a quotient comes close to a threshold, is 15 instructions less a pixel and slower:
-// one item in five hundred is close, and the wave that has one is what the launch waits for.)
 template <int BITS, bool SIMPLE, typename Tables>
 __device__ __forceinline__ bool quantize_pixel_fast(float (&x)[kC], float eps, const BucketScale &bq, const Tables &q)
 {
@@ -133,19 +117,18 @@ __device__ __forceinline__ bool quantize_pixel_fast(float (&x)[kC], float eps, c
     }
     float y;
     const float s = sqrt_and_reciprocal(third_of(var) + eps, y);
+    const CodeScale cs = code_scale_of(s, y, bq);
     float sum_codes = 0.0f;
 #pragma unroll
     for (int c = 0; c < kC; ++c) {
-        const float t = quotient(x[c], s, y);
-        const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(q.bucket) + bucket_offset_of(t, bq));
-        const float v = q.cb[code_in_bucket(bk, t > bk.thr)];
+        const float v = code_value(q.cb, code_offset_of(x[c], cs, bq, q.bucket));
         x[c] = v;
         sum_codes += v;
     }
     const float code_mean = third_of(sum_codes);
 #pragma unroll
     for (int c = 0; c < kC; ++c) x[c] = fma_f32(s, x[c] - code_mean, mu);
-    const bool root_ok = (s >= 0x1p-60f) & (s <= 0x1p60f) & ((__float_as_uint(s) & 0x7fffffu) != 0x7fffffu);
+    const bool root_ok = (s >= 0x1p-50f) & (s < 0x1p50f);
     if constexpr (SIMPLE) return root_ok;
     // d_c is 0 or at least 2^-90 once |mu| >= 2^-66 or all of them are 0.
     // (No short circuits: a branch per pixel would keep the eight pixels of a lane from overlapping.)
@@ -248,7 +231,8 @@ void launch_patches(const void *img, const float *thr, const float *cb, void *x_
 {
     const int64_t M = static_cast<int64_t>(B) * (H / kP) * (W / kP);
     const int items = static_cast<int>((M + 31) / 32 * 16);
-    // (what the chip holds at once: 256 images 35.7 us against 38.3 with four workgroups per CU and 39.3 with six)
+    // (what the chip holds at once: 256 images 35.7 us against 38.3 with four workgroups per CU and 39.3 with six, all before the
+    // codes were found without a quotient)
     const int wgs = std::min((items + kPrepWaves - 1) / kPrepWaves, 5 * device_cus());
     hipLaunchKernelGGL((act_quant_patches_kernel<TIN, BITS>), dim3(weights.blocks + wgs), dim3(kPrepThreads), 0, stream,
                        static_cast<const TIN *>(img), thr, cb, static_cast<__half *>(x_hat), B, H, W, eps, blocked, items, weights);
