@@ -236,7 +236,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
     // The NB blocks from b0 (32 x 32 NJ values each, columns from tile jb) leave in chunks of 128 bytes per row through
     // the wave's private staging tile (LDS operations of one wave execute in order: no wait is needed between them).
     auto write_out = [&](auto nbc, auto njc, const float16_t (&acc)[decltype(nbc)::value][decltype(njc)::value],
-                         const int b0, const int jb) __attribute__((always_inline)) {
+                         const int b0, const int jb, auto lane_per_group) __attribute__((always_inline)) {
         constexpr int NB = decltype(nbc)::value;
         constexpr int NJ = decltype(njc)::value;
         constexpr int kChunkCols = 128 / static_cast<int>(sizeof(TOUT));     // 64 (fp16) / 32 (fp32)
@@ -248,6 +248,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const int pblk = b0 + nb;
+            [[maybe_unused]] StagedGroup staged;
 #pragma unroll
             for (int ch = 0; ch < kChunks; ++ch) {
                 // Bias values first: the compiler cannot tell the bias reads from the staging writes (both LDS) and
@@ -282,10 +283,16 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
                     }
                 }
                 __builtin_amdgcn_wave_barrier();
-                if constexpr (NQ != 0) {
-                    const int c0 = n_base + jb * 32 + ch * kChunkCols;          // the chunk is one group of the consumer's rows
-                    if (c0 < N)
-                        next_quant_block<NQ, false>(nq_lds, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
+                if constexpr (NQ != 0) {          // the chunk is one group of the consumer's rows
+                    // (while the next pass's fragments are in flight two row blocks leave no room for a group in one lane:
+                    // 50 432 x 1 024 -> 4 096 then takes 633 us instead of 581)
+                    if constexpr (kChunks == 2 && decltype(lane_per_group)::value) {
+                        take_staged_group(staged, stage, kStageRow, lane, ch);
+                        if (ch == 1) next_quant_groups<NQ, false>(nq_lds, staged, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, n_base);
+                    } else {
+                        const int c0 = n_base + jb * 32 + ch * kChunkCols;
+                        if (c0 < N) next_quant_block<NQ, false>(nq_lds, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
+                    }
                     __builtin_amdgcn_wave_barrier();
                     continue;
                 }
@@ -346,7 +353,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
                           u32x4_t (&xs)[4][decltype(nbc)::value], const char *const (&xbase)[decltype(nbc)::value],
                           const int (&kstep)[decltype(nbc)::value], const char *const (&xnext)[decltype(nbc)::value],
                           const int (&knext)[decltype(nbc)::value], const int b0, const int jb, const bool live,
-                          const bool then_first) __attribute__((always_inline)) {
+                          const bool then_first, auto last_one) __attribute__((always_inline)) {
         constexpr int NB = decltype(nbc)::value;
         for (int sl = 0; sl < slices; ++sl) {
             const int g0 = sl * kSliceGroups;
@@ -366,7 +373,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
             }
         }
         if constexpr (DB) {
-            if (live) write_out(nbc, njc, acc, b0, jb);
+            if (live) write_out(nbc, njc, acc, b0, jb, last_one);
             if (then_first) {
                 if (live) wait_vmcnt<4 * NB>(); else wait_vmcnt<0>();      // (stores are younger still: some of them are waited for too)
                 __syncthreads();
@@ -378,7 +385,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
                 __syncthreads();      // every wave is done reading the last slice
                 copy_slice_unseen(slab, 0, min(kSliceGroups, G));
             }
-            if (live) write_out(nbc, njc, acc, b0, jb);
+            if (live) write_out(nbc, njc, acc, b0, jb, last_one);
             if (refill) {
                 wait_vmcnt<0>();
                 __syncthreads();
@@ -418,7 +425,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) acc[nb][j][v] = 0.0f;
-            run_slices(I2{}, I4{}, acc, xs, xcur, kcur, xnxt, knxt, b0, 0, true, more || rest > 0);
+            run_slices(I2{}, I4{}, acc, xs, xcur, kcur, xnxt, knxt, b0, 0, true, more || rest > 0, std::false_type{});
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
                 xcur[nb] = xnxt[nb];
@@ -447,7 +454,7 @@ gemm_pair_kernel(const __half *__restrict__ xb, const float *__restrict__ bias, 
         u32x4_t xs[4][NB];
         if (live) first_fragments(nbc, xs, xbase, kstep);
         if (full_passes == 0) fill_slice(0, min(kSliceGroups, G));      // (else the last full pass left slice 0 resident)
-        run_slices(nbc, njc, acc, xs, xbase, kstep, xlast, kstep, b0, jb, live, false);
+        run_slices(nbc, njc, acc, xs, xbase, kstep, xlast, kstep, b0, jb, live, false, std::true_type{});
     };
     if (rest > 0) {
         const int base = blk0 + full_passes * 2 * kWaves;

@@ -351,6 +351,7 @@ gemm_slab8_kernel(const __half *__restrict__ xb, const uint8_t *__restrict__ pw,
         if (live) {
             // Whole 16-byte pieces everywhere in this slab (wave-uniform): the common case takes no per-piece branch.
             const bool whole = (N % kVec) == 0 && n_base + kSlabN <= N;
+            [[maybe_unused]] StagedGroup staged;
 #pragma unroll
             for (int ch = 0; ch < kChunks; ++ch) {
                 // Bias values first, a batch at a time (the whole chunk with eight waves; one 32-column block with
@@ -390,10 +391,14 @@ gemm_slab8_kernel(const __half *__restrict__ xb, const uint8_t *__restrict__ pw,
                     }
                 }
                 __builtin_amdgcn_wave_barrier();
-                if constexpr (NQ != 0) {
-                    const int c0 = n_base + jb * 32 + ch * kChunkCols;          // the chunk is one group of the consumer's rows
-                    if (c0 < N)
-                        next_quant_block<NQ, false>(nq_lds, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
+                if constexpr (NQ != 0) {          // the chunk is one group of the consumer's rows
+                    if constexpr (kChunks == 2) {
+                        take_staged_group(staged, stage, kStageRow, lane, ch);
+                        if (ch == 1) next_quant_groups<NQ, false>(nq_lds, staged, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, n_base);
+                    } else {
+                        const int c0 = n_base + jb * 32;
+                        if (c0 < N) next_quant_block<NQ, false>(nq_lds, stage, kStageRow, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, c0);
+                    }
                     __builtin_amdgcn_wave_barrier();
                     continue;
                 }

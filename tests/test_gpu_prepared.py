@@ -163,3 +163,11 @@ def test_gelu_of_every_fp16_value(cuda, m, apart):
         want = torch.nn.functional.gelu(part)
         wrong = ~((y == want) | (y.isnan() & want.isnan())).all(0)
         assert not bool(wrong.any()), part[wrong][:8]
+
+
+# the weight-stationary kernels with a lane per group: every way of dealing the last blocks, ragged rows, a half slab past the last
+# column
+@pytest.mark.parametrize("m,n,k,bits", [(12608, 1536, 384, 4), (6301, 1600, 320, 3), (9000, 448, 64, 2), (3152, 3072, 768, 4),
+                                        (4001, 832, 448, 4), (12577, 3136, 768, 3)])
+def test_linear_prepared_quantizes_many_rows(cuda, oracle, m, n, k, bits):
+    test_linear_prepared_quantizes_for_the_next_layer(cuda, oracle, m, n, k, bits)
