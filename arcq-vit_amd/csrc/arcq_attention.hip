@@ -9,7 +9,8 @@
 // whole-block fusion around the packed linears: at batch 1 the library attention plus the two copies that reshape
 // its operands take as long as two packed layers.
 //
-// One workgroup per (batch, head); wave w owns the 32 queries 32 w ... (n <= 256 tokens: at most eight waves).  K of
+// One workgroup per (batch, head), or where these are few one per part of a head: wave w owns the 32 queries of tile w, or of tile
+// parts * w + part, and the waves without a tile only load (n <= 256 tokens: at most eight waves).  K of
 // the head sits in LDS row-major, V transposed, both zero-padded to whole 32-key blocks.  Scores: S^T = K Q^T on
 // v_mfma_f32_32x32x16_f16 with K as the first operand, so that a lane (query q = lane % 32, half h = lane / 32) ends
 // up holding, of every 32-key block, the 16 keys 8 t + 4 h + c (t, c = 0..3) of its own query: the row maximum and sum
@@ -19,6 +20,9 @@
 // matching eight values of V^T are two 8-byte LDS reads.  fp32 scores, softmax and accumulation; P rounded to fp16;
 // normalisation by the row sum at the end.  Beyond 128 keys the keys go in two chunks with a running maximum and sum.
 #include "arcq_act_quant_core.h"
+#include "arcq_gemm.h"
+
+#include <algorithm>
 
 namespace arcq {
 namespace {
@@ -38,8 +42,9 @@ constexpr int kKPitch = kHeadDim * 2 + 16;          // bytes per key row of K in
 // the output.  A wave's 32 x 64 outputs go through its own 32 rows of K in LDS (all waves are done with it) into the
 // lane-pair routine of the GEMM epilogues.
 // F8: that operand as FP8 (rows padded to 128 values).
-template <int NKB, int NQ, bool F8>
-__global__ void __launch_bounds__(64 * NKB) __attribute__((amdgpu_waves_per_eu(4)))     // two workgroups of up to 8 waves on a CU
+// SPLIT: a head has gridDim.z workgroups.  (A template: the two registers that it takes cost 5 % at 256 images of 16 heads.)
+template <int NKB, int NQ, bool F8, bool SPLIT>
+__global__ void __launch_bounds__(64 * NKB) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 : 4)))     // two workgroups of up to 8 waves on a CU, or one
 attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n, int H, float scale,
                  const float *__restrict__ nq_thr, const float *__restrict__ nq_cb, int total_rows)
 {
@@ -82,7 +87,9 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
         if (wave == NKB - 1) next_quant_setup<NQ>(nq_params, nq_lds, lane);
     }
     // ---- this wave's queries: lane (q, half) holds Q[q][16 kk + 8 half ... + 7] for kk = 0..3 ----
-    const int q = wave * 32 + lr;
+    const int tile = SPLIT ? wave * gridDim.z + blockIdx.z : wave;      // (parts of a head take its query tiles in turn)
+    const bool busy = !SPLIT || tile < NKB;
+    const int q = tile * 32 + lr;
     u32x4_t qf[4];
     {
         const __half *src = base + (row0 + min(q, n - 1)) * 3 * C + 8 * lh;
@@ -104,6 +111,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
     }
     __syncthreads();
 
+    if (NQ == 0 && !busy) return;
     // Keys in chunks of CH blocks with a running maximum and sum (the scores of one chunk are live at a time, which
     // keeps the wave at half the registers and two workgroups on a CU); one chunk is the plain two-pass softmax.
     const float ninf = -__builtin_inff();
@@ -116,6 +124,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
         for (int v = 0; v < 16; ++v) oacc[jb][v] = 0.0f;
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch) {
+        if (NQ != 0 && !busy) break;                            // (the wave has a barrier left)
         constexpr int kLast = NKB - CH * (NCH - 1);
         const int nb = ch == NCH - 1 ? kLast : CH;          // constant after unrolling
         if (ch > 0) __builtin_amdgcn_sched_barrier(0);      // keep the next chunk's scores out of this one's live range
@@ -190,6 +199,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
     l += __shfl_xor(l, 32);
     if constexpr (NQ != 0) {
         __syncthreads();                                     // everyone is done with K
+        if (!busy) return;
         unsigned char *stage = ks + wave * 32 * kKPitch;
         const float inv = 1.0f / l;
 #pragma unroll
@@ -205,7 +215,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
             }
         __builtin_amdgcn_wave_barrier();
         // This lane's row of the chunk (rows past the image's last query: zero scores of zero queries, not stored).
-        const int qr = wave * 32 + (lane >> 1);
+        const int qr = tile * 32 + (lane >> 1);
         const int64_t row = row0 + qr;
         const int blk = static_cast<int>(row >> 5);
         const int nrows = min(32, total_rows - blk * 32);
@@ -235,7 +245,13 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
 template <int NKB, int NQ, bool F8>
 void launch_attention(const void *qkv, void *out, int B, int n, int H, float scale, const float *thr, const float *cb, hipStream_t stream)
 {
-    hipLaunchKernelGGL((attention_kernel<NKB, NQ, F8>), dim3(H, B), dim3(64 * NKB), 0, stream, static_cast<const __half *>(qkv),
+    // Parts of a head: as many as the compute units take, so that the waves that share a SIMD in a workgroup of a whole head have one
+    // each.  197 tokens of 6 heads (with the consumer's stage 1): 9.9 us in one part, 8.0 in two, 7.7 in seven; 16 images 10.2 / 8.5
+    // in two parts, 10.7 in three (288 workgroups).
+    const int64_t heads = static_cast<int64_t>(B) * H;
+    const int parts = static_cast<int>(std::min<int64_t>(NKB, std::max<int64_t>(1, device_cus() / heads)));
+    auto kernel = NKB > 1 && parts > 1 ? attention_kernel<NKB, NQ, F8, (NKB > 1)> : attention_kernel<NKB, NQ, F8, false>;
+    hipLaunchKernelGGL(kernel, dim3(H, B, parts), dim3(64 * NKB), 0, stream, static_cast<const __half *>(qkv),
                        static_cast<__half *>(out), n, H, scale, thr, cb, B * n);
 }
 

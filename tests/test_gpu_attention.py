@@ -102,3 +102,11 @@ def test_vit_with_own_attention(cuda, model, batch):
     assert bool(torch.isfinite(a).all())
     cos = torch.nn.functional.cosine_similarity(a.float().flatten(), b.float().flatten(), dim=0).item()
     assert cos > 0.99, cos
+
+
+@pytest.mark.parametrize("b,n,h", [(1, 33, 1), (1, 197, 6), (2, 256, 12), (3, 65, 20), (5, 129, 16), (11, 197, 11), (8, 97, 16)])
+def test_parts_of_a_head(cuda, b, n, h):
+    """Few heads are dealt in parts (every number of parts from two to a tile each): the same bits as in a batch of whole heads."""
+    many = -(-260 // h) + b
+    qkv = torch.randn(many, n, 3 * h * 64, generator=torch.Generator().manual_seed(n)).half().to(cuda)
+    assert torch.equal(ops.attention_fwd(qkv[:b].contiguous(), h), ops.attention_fwd(qkv, h)[:b])
