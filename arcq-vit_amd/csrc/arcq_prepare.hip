@@ -162,15 +162,17 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const f
 // a row go through wave-private LDS padded with zeros to a multiple of eight (x + 0 leaves the sum as it is), so that all reads
 // of a sum are in flight together, and gamma and beta lie in LDS (pitch 36 per 32 values: conflict-free 16-byte reads).  With
 // one read per loop trip and gamma / beta from L2: see the figures at the launch.
-constexpr int kGammaPitch = 36;
+// LANES lanes a group: two, or four or eight in launches of a few rows, which are one chain of instructions long.
+constexpr int gamma_pitch(int lanes) { return 64 / lanes + 4; }
 // BUILDER: as above; the tables and gamma / beta are first needed behind the first tile's row sums.
-template <typename TIN, int BITS, bool BUILDER>
+template <typename TIN, int BITS, int LANES, bool BUILDER>
 __global__ void __launch_bounds__(64 * (kPrepWaves + (BUILDER ? 1 : 0))) __attribute__((amdgpu_waves_per_eu(4)))
 prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta, float ln_eps,
                   const float *__restrict__ thr, const float *__restrict__ cb, char *__restrict__ x_hat, float eps, int rows,
                   int G, int R, uint32_t rw_inverse, int tiles, PrepWeights w0, PrepWeights w1)
 {
-    constexpr int kIn = 32 * static_cast<int>(sizeof(TIN)) / 16;       // 16-byte loads per lane (32 values)
+    constexpr int V = 64 / LANES, kGammaPitch = gamma_pitch(LANES);    // values per lane
+    constexpr int kIn = V * static_cast<int>(sizeof(TIN)) / 16;        // 16-byte loads per lane
     extern __shared__ __attribute__((aligned(16))) unsigned char prep_smem[];
     __shared__ QuantTables tables;
     if (prep_weight_workgroup<BITS, false>(w0, w1, tables.cb)) return;
@@ -183,12 +185,12 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
     QuantParams params{};
     if (!BUILDER && wave == 0) params = load_quant_params<BITS>(thr, cb, lane);
     const int wg = blockIdx.x - (w0.blocks + w1.blocks), wgs = gridDim.x - (w0.blocks + w1.blocks);
-    const int P = 2 * G;                                    // lanes per row
+    const int P = LANES * G;                                // lanes per row
     const int rl = lane / P, pl = lane - rl * P;            // row of the wave, lane of the row
     const int K = G * 64;
     const bool lane_used = rl < R;
     const int RW = kPrepWaves * R;                          // rows of a tile
-    const int chunks = (P + 7) / 8;                         // of eight partial sums
+    const int chunks = (2 * G + 7) / 8;                     // of eight partial sums (32 values each)
     unsigned char *tile = prep_smem;                        // RW * G * 128 bytes
     float *part = reinterpret_cast<float *>(prep_smem + RW * G * 128) + wave * (R * chunks * 8);
     float *s_gamma = reinterpret_cast<float *>(prep_smem + RW * G * 128) + kPrepWaves * (R * chunks * 8);
@@ -198,14 +200,14 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
     auto fetch = [&](int t) {
         const int row = t * RW + wave * R + rl;
         const bool valid = lane_used && t < tiles && row < rows;
-        const uint4 *p = reinterpret_cast<const uint4 *>(x + static_cast<int64_t>(valid ? row : 0) * K + (valid ? pl * 32 : 0));
+        const uint4 *p = reinterpret_cast<const uint4 *>(x + static_cast<int64_t>(valid ? row : 0) * K + (valid ? pl * V : 0));
 #pragma unroll
         for (int i = 0; i < kIn; ++i) raw[i] = valid ? p[i] : make_uint4(0, 0, 0, 0);
     };
     fetch(wg);
     for (int i = tid; i < K / 4; i += kPrepThreads) {
         const float4 gv = reinterpret_cast<const float4 *>(gamma)[i], bv = reinterpret_cast<const float4 *>(beta)[i];
-        const int at = (i >> 3) * kGammaPitch + (i & 7) * 4;
+        const int at = i / (V / 4) * kGammaPitch + i % (V / 4) * 4;
         *reinterpret_cast<float4 *>(s_gamma + at) = gv;
         *reinterpret_cast<float4 *>(s_beta + at) = bv;
     }
@@ -218,7 +220,7 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
     const float *my_gamma = s_gamma + (lane_used ? pl : 0) * kGammaPitch, *my_beta = s_beta + (lane_used ? pl : 0) * kGammaPitch;
 
     for (int t = wg; t < tiles; t += wgs) {
-        float xv[32];
+        float xv[V];
         if constexpr (sizeof(TIN) == 2) {
 #pragma unroll
             for (int i = 0; i < kIn; ++i) {
@@ -237,10 +239,11 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
             }
         }
         if (t + wgs < tiles) fetch(t + wgs);                // the next tile loads under this one's arithmetic
-        // Row sums: every lane folds its 32 values serially, the row's 2 G partial sums are added in order (group by group,
-        // lower half first) by every lane of the row.
+        // Row sums: every 32 values are folded serially, the row's 2 G partial sums are added in order (group by group, lower half
+        // first) by every lane of the row.
+        constexpr int kPer = LANES / 2;                     // lanes per partial sum (the last one has it)
         auto row_total = [&](float mine) {
-            if (lane_used) my_part[pl] = mine;
+            if (lane_used && pl % kPer == kPer - 1) my_part[pl / kPer] = mine;
             __builtin_amdgcn_wave_barrier();
             float acc = 0.0f;
             for (int c0 = 0; c0 < chunks; c0 += 4) {        // (one trip up to K = 1 024)
@@ -266,18 +269,14 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
             __builtin_amdgcn_wave_barrier();
             return acc;
         };
-        float a = 0.0f;
+        const float mean = row_total(lanes_serial_sum<kPer>(xv)) / fk;
+        float sq[V];
 #pragma unroll
-        for (int j = 0; j < 32; ++j) a += xv[j];
-        const float mean = row_total(a) / fk;
-        float q = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 32; ++j) {
+        for (int j = 0; j < V; ++j) {
             xv[j] -= mean;
-            const float sq = xv[j] * xv[j];
-            q += sq;
+            sq[j] = xv[j] * xv[j];
         }
-        const float rstd = 1.0f / sqrtf(row_total(q) / fk + ln_eps);
+        const float rstd = 1.0f / sqrtf(row_total(lanes_serial_sum<kPer>(sq)) / fk + ln_eps);
         if (!ready) {                                       // once per workgroup: the tables, gamma and beta are in LDS
             __syncthreads();
             bq = tables.geometry;
@@ -285,7 +284,7 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
             ready = true;
         }
 #pragma unroll
-        for (int j4 = 0; j4 < 8; ++j4) {
+        for (int j4 = 0; j4 < V / 4; ++j4) {
             const float4 gv = *reinterpret_cast<const float4 *>(my_gamma + 4 * j4), bv = *reinterpret_cast<const float4 *>(my_beta + 4 * j4);
             const float g4[4] = {gv.x, gv.y, gv.z, gv.w}, b4[4] = {bv.x, bv.y, bv.z, bv.w};
 #pragma unroll
@@ -298,13 +297,18 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
             }
         }
         float mu, var, s, sum_codes;
-        group_stats32x2(xv, eps, mu, var, s);
-        group_codes32x2<BITS>(xv, mu, var, s, tables, bq, table_ok, sum_codes);
+        if constexpr (LANES == 2) {
+            group_stats32x2(xv, eps, mu, var, s);
+            group_codes32x2<BITS>(xv, mu, var, s, tables, bq, table_ok, sum_codes);
+        } else {
+            group_stats_lanes<LANES>(xv, eps, lane, mu, var, s);
+            group_codes_lanes<BITS, LANES>(xv, mu, var, s, tables, bq, table_ok, lane, sum_codes);
+        }
         const float code_mean = sum_codes * 0.015625f;
         // ---- out: piece (k8, row) at LDS slot k8 * RW + row, then 16 bytes per lane, rows fastest ----
         if (lane_used) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < V / 8; ++i) {
                 uint32_t w[4];
 #pragma unroll
                 for (int d = 0; d < 4; ++d) {
@@ -312,7 +316,7 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
                     const __half2 h = __floats2half2_rn(fma_f32(s, xv[j] - code_mean, mu), fma_f32(s, xv[j + 1] - code_mean, mu));
                     w[d] = *reinterpret_cast<const uint32_t *>(&h);
                 }
-                *reinterpret_cast<uint4 *>(tile + ((pl * 4 + i) * RW + wave * R + rl) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+                *reinterpret_cast<uint4 *>(tile + ((pl * (V / 8) + i) * RW + wave * R + rl) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
             }
         }
         __syncthreads();
@@ -340,20 +344,32 @@ void launch_prepare_t(const arcq_prepare_args &a, float eps, const PrepWeights &
     char *x_hat = static_cast<char *>(a.x_hat);
     if constexpr (!F8) {
         if (a.ln_weight && rows > 0) {
-            const int R = 64 / (2 * G), tiles = (rows + kPrepWaves * R - 1) / (kPrepWaves * R);
-            // (2^20 / RW rounded up: exact for all 1 024 pieces or fewer of a tile, whatever the number of groups.  The division cost
-            // 20 instructions a piece: 12 608 x 1 024 16.9 -> 16.1 us)
-            const uint32_t inverse = ((1u << 20) + kPrepWaves * R - 1) / (kPrepWaves * R);
-            const size_t smem = static_cast<size_t>(kPrepWaves) * R * G * 128 + kPrepWaves * (R * ((2 * G + 7) / 8) * 8) * 4 +
-                                static_cast<size_t>(2 * G) * kGammaPitch * 8;
-            // Beyond four workgroups per CU the waves walk their tiles: the lookup tables are built once per workgroup.
-            const int wgs = std::min(tiles, 4 * device_cus());
-            if (tiles <= 2 * device_cus())
-                hipLaunchKernelGGL((prepare_ln_kernel<TIN, BITS, true>), dim3(weights + wgs), dim3(kPrepThreads + 64), smem, stream, x, a.ln_weight,
-                                   a.ln_bias, a.ln_eps, a.thresholds, a.codebook, x_hat, eps, rows, G, R, inverse, tiles, w0, w1);
-            else
-                hipLaunchKernelGGL((prepare_ln_kernel<TIN, BITS, false>), dim3(weights + wgs), dim3(kPrepThreads), smem, stream, x, a.ln_weight,
-                                   a.ln_bias, a.ln_eps, a.thresholds, a.codebook, x_hat, eps, rows, G, R, inverse, tiles, w0, w1);
+            auto run = [&](auto lanes, auto builder) {
+                constexpr int LANES = decltype(lanes)::value;
+                constexpr bool BUILDER = decltype(builder)::value;
+                const int R = 64 / (LANES * G), RW = kPrepWaves * R, tiles = (rows + RW - 1) / RW;      // rows per wave and tile
+                const size_t smem = static_cast<size_t>(RW) * G * 128 + kPrepWaves * (R * ((2 * G + 7) / 8) * 8) * 4 +
+                                    static_cast<size_t>(LANES * G) * gamma_pitch(LANES) * 8;
+                // Beyond four workgroups per CU the waves walk their tiles: the lookup tables are built once per workgroup.
+                // (2^20 / RW rounded up: exact for all 1 024 pieces or fewer of a tile, whatever the number of groups.  The division
+                // cost 20 instructions a piece: 12 608 x 1 024 16.9 -> 16.1 us)
+                hipLaunchKernelGGL((prepare_ln_kernel<TIN, BITS, LANES, BUILDER>), dim3(weights + std::min(tiles, 4 * device_cus())),
+                                   dim3(kPrepThreads + (BUILDER ? 64 : 0)), smem, stream, x, a.ln_weight, a.ln_bias, a.ln_eps, a.thresholds,
+                                   a.codebook, x_hat, eps, rows, G, R, static_cast<uint32_t>(((1 << 20) + RW - 1) / RW), tiles, w0, w1);
+            };
+            using I2 = std::integral_constant<int, 2>;
+            using I4 = std::integral_constant<int, 4>;
+            using I8 = std::integral_constant<int, 8>;
+            auto tiles_of = [&](int lanes) {
+                const int RW = kPrepWaves * (64 / (lanes * G));
+                return (rows + RW - 1) / RW;
+            };
+            // With more lanes a group while that is at most two tiles per CU: 197 x 384 6.3 -> 4.3 us with eight lanes, 2 048 x 384
+            // 6.6 -> 4.7, 1 576 x 768 6.6 -> 5.4 with four; beyond, 6 304 x 384 (1 576 tiles of eight lanes) 7.4 -> 8.4.
+            if (G <= 8 && tiles_of(8) <= 2 * device_cus()) run(I8{}, std::true_type{});
+            else if (G <= 16 && tiles_of(4) <= 2 * device_cus()) run(I4{}, std::true_type{});
+            else if (tiles_of(2) <= 2 * device_cus()) run(I2{}, std::true_type{});
+            else run(I2{}, std::false_type{});
             return;
         }
     }

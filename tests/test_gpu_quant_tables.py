@@ -58,3 +58,19 @@ def test_tables(cuda, oracle, bits):
         rows = oracle.act_quant_c(pix.numpy(), thr, cb, bits, 3)["x_hat"].astype(np.float16)
         rows = rows.reshape(2, 2, 16, 2, 16, 3).transpose(0, 1, 3, 5, 2, 4).reshape(8, 768)
         same(ops.quantize_patches(img.to(cuda), t, c, bits), rows, "patches")
+
+
+# eight, four and two lanes a group: the fewest and the most groups of each, ragged tiles, both sides of two tiles per compute unit
+@pytest.mark.parametrize("m,k", [(1, 64), (5, 512), (197, 384), (2049, 192), (2057, 320), (3, 576), (33, 1024), (1700, 640), (5, 1088),
+                                 (21, 2048), (16390, 64), (6304, 384)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_lanes_per_group_behind_a_layernorm(cuda, oracle, m, k, dtype):
+    cb = synth.quantile_codebook(4)
+    thr = synth.midpoint_thresholds(cb)
+    x = (synth.make_activation(m, k, 21) * 1.7 + 0.3).to(dtype)
+    g, b = torch.linspace(0.5, 1.5, k), torch.linspace(-0.2, 0.2, k)
+    ln = oracle.layernorm_rows_np(x.float().numpy(), g.numpy(), b.numpy(), 1e-6, out_f16=dtype == torch.float16)
+    for t in (thr, thr[torch.randperm(15, generator=torch.Generator().manual_seed(m))].contiguous()):      # buckets; every threshold in turn
+        want = oracle.act_quant_c(ln, t, cb, 4, 64)["x_hat"].astype(np.float16)
+        got = _prepare(x.to(cuda), t.to(cuda), cb.to(cuda), 4, (g.to(cuda), b.to(cuda), 1e-6))[0]
+        assert np.array_equal(got.cpu().numpy().view(np.uint16), _blocked(want).view(np.uint16))
