@@ -203,25 +203,26 @@ __device__ __forceinline__ void group_stats64(float (&xv)[64], float eps, float 
     s_out = sqrtf(var * 0.015625f + eps);
 }
 
-// Codes without the buckets: every threshold in turn, while (c < L - 1 && t > thr[c]) ++c; eight values at a time (registers).
+// Codes without the buckets: every threshold in turn, while (c < L - 1 && t > thr[c]) ++c; up to eight values at a time (registers).
 // xv holds the residuals on entry and cb[code_j] on exit; put(j, code).
 template <int BITS, int N, typename Put>
 __device__ __forceinline__ void search_codes(float (&xv)[N], float s, const QuantTables &q, const Put &put)
 {
+    constexpr int B = N < 8 ? N : 8;
 #pragma unroll
-    for (int j0 = 0; j0 < N; j0 += 8) {
-        float t[8];
-        uint32_t c[8];
+    for (int j0 = 0; j0 < N; j0 += B) {
+        float t[B];
+        uint32_t c[B];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) t[e] = xv[j0 + e] / s, c[e] = 0;
+        for (int e = 0; e < B; ++e) t[e] = xv[j0 + e] / s, c[e] = 0;
 #pragma unroll 1
         for (uint32_t i = 0; i + 1 < (1u << BITS); ++i) {
             const float thr = q.thr[i];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) c[e] += (c[e] == i && t[e] > thr) ? 1u : 0u;
+            for (int e = 0; e < B; ++e) c[e] += (c[e] == i && t[e] > thr) ? 1u : 0u;
         }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < B; ++e) {
             xv[j0 + e] = q.cb[c[e]];
             put(j0 + e, c[e]);
         }
@@ -333,7 +334,7 @@ __device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float
     sum_out = pair_serial_sum(xv);
 }
 
-// ---- four or eight lanes per group -------------------------------------------------------------------------------
+// ---- four, eight or sixteen lanes per group -------------------------------------------------------------------------------
 // Where a launch leaves most of the chip idle: the serial sums stay as long (in LANES phases, a lane's partial sum handed to its
 // neighbour after each; what a lane adds in a phase that is not its own is discarded), everything else of a value is spread.
 // 197 x 384 values with a LayerNorm in front: 6.3 us with two lanes a group, 4.3 with eight.
@@ -357,8 +358,9 @@ __device__ __forceinline__ float lanes_serial_sum(const float (&v)[V])
 template <int LANES>
 __device__ __forceinline__ float from_last_lane(float v, int lane)
 {
-    static_assert(LANES == 2 || LANES == 4 || LANES == 8, "lanes per group");
+    static_assert(LANES == 2 || LANES == 4 || LANES == 8 || LANES == 16, "lanes per group");
     if constexpr (LANES == 2) return from_odd_lane(v);
+    if constexpr (LANES == 16) return lane_moved<0x15F>(v);    // row_newbcast:15
     const float quad = lane_moved<0xFF>(v);                    // quad_perm [3,3,3,3]
     if constexpr (LANES == 4) return quad;
     const float other = lane_moved<0x141>(quad);               // row_half_mirror (not inside the choice: every lane has to take part)
@@ -412,6 +414,21 @@ template <int BITS>
 __device__ __forceinline__ void next_quant_setup(const QuantParams &p, unsigned char *lds, int lane)
 {
     build_quant_tables<BITS>(p, *reinterpret_cast<QuantTables *>(lds), lane);
+}
+
+// The consumer's stage 1 of a group that 64 / V neighbouring lanes (aligned) hold in registers, V fp16-rounded values each: v is
+// replaced by the reconstruction.
+template <int BITS, int V>
+__device__ __forceinline__ void next_quant_lanes(const unsigned char *lds, float (&v)[V], int lane, float eps)
+{
+    constexpr int LANES = 64 / V;
+    const QuantTables &q = *reinterpret_cast<const QuantTables *>(lds);
+    float mu, var, s, sum;
+    group_stats_lanes<LANES>(v, eps, lane, mu, var, s);
+    group_codes_lanes<BITS, LANES>(v, mu, var, s, q, q.geometry, q.usable != 0, lane, sum);
+    const float code_mean = sum * 0.015625f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) v[j] = fma_f32(s, v[j] - code_mean, mu);
 }
 
 // One staged chunk (32 rows x 64 fp16 values, the rows `pitch` bytes apart) -> x_hat of the consuming layer.

@@ -83,7 +83,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
             vreg[i][j] = key < n ? *reinterpret_cast<const u32x4_t *>(src + C) : zero4;
         }
     }
-    if constexpr (NQ != 0) {                                   // while K and V are on their way
+    if constexpr (NQ != 0 && !SPLIT) {                         // while K and V are on their way
         if (wave == NKB - 1) next_quant_setup<NQ>(nq_params, nq_lds, lane);
     }
     // ---- this wave's queries: lane (q, half) holds Q[q][16 kk + 8 half ... + 7] for kk = 0..3 ----
@@ -112,6 +112,9 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
     __syncthreads();
 
     if (NQ == 0 && !busy) return;
+    if constexpr (NQ != 0 && SPLIT) {                          // (under the others' product: that wave has no tile in a part)
+        if (wave == NKB - 1) next_quant_setup<NQ>(nq_params, nq_lds, lane);
+    }
     // Keys in chunks of CH blocks with a running maximum and sum (the scores of one chunk are live at a time, which
     // keeps the wave at half the registers and two workgroups on a CU); one chunk is the plain two-pass softmax.
     const float ninf = -__builtin_inff();
@@ -199,13 +202,13 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
     l += __shfl_xor(l, 32);
     if constexpr (NQ != 0) {
         __syncthreads();                                     // everyone is done with K
-        if (!busy) return;
         unsigned char *stage = ks + wave * 32 * kKPitch;
         const float inv = 1.0f / l;
 #pragma unroll
         for (int jb = 0; jb < 2; ++jb)
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
+                if (!busy) break;
                 const __half2 a = __floats2half2_rn(oacc[jb][4 * t] * inv, oacc[jb][4 * t + 1] * inv);
                 const __half2 c = __floats2half2_rn(oacc[jb][4 * t + 2] * inv, oacc[jb][4 * t + 3] * inv);
                 u32x2_t pk;
@@ -213,6 +216,53 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
                 pk[1] = *reinterpret_cast<const uint32_t *>(&c);
                 *reinterpret_cast<u32x2_t *>(stage + lr * kKPitch + (jb * 32 + 8 * t + 4 * lh) * 2) = pk;
             }
+        const int parts = SPLIT ? gridDim.z : 1;
+        if (SPLIT && 4 * ((NKB + parts - 1) / parts) <= NKB) {
+            // Few waves have a tile, but all of them quantize: eight lanes a row (FP8: four), one 16-byte piece a lane.
+            constexpr int V = F8 ? 16 : 8, LANES = 64 / V, ROWS = 64 / LANES;
+            __syncthreads();
+            const int part = blockIdx.z, tiles = (NKB - part + parts - 1) / parts;
+            for (int job = wave; job < tiles * (32 / ROWS); job += NKB) {
+                const int at = job * ROWS + lane / LANES, piece = lane % LANES;       // row of the part, piece of the row
+                float v[V];
+#pragma unroll
+                for (int i = 0; i < V / 8; ++i) {
+                    const u32x4_t w = *reinterpret_cast<const u32x4_t *>(ks + at * kKPitch + (piece * (V / 8) + i) * 16);
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        v[8 * i + 2 * d] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[d] & 0xffffu)));
+                        v[8 * i + 2 * d + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[d] >> 16)));
+                    }
+                }
+                next_quant_lanes<NQ>(nq_lds, v, lane, 1.0e-6f);
+                const int qr = ((at >> 5) * parts + part) * 32 + (at & 31);
+                if (qr < n) {
+                    const int64_t row = row0 + qr;
+                    const int blk = static_cast<int>(row >> 5), nrows = min(32, total_rows - blk * 32);
+                    const int row_bytes = F8 ? (C + 127) / 128 * 128 : C * 2;
+                    char *dst = reinterpret_cast<char *>(out) + static_cast<int64_t>(blk) * 32 * row_bytes +
+                                (static_cast<int64_t>(h * LANES + piece) * nrows + (row & 31)) * 16;
+                    uint32_t o[4];
+                    if constexpr (F8) {
+                        float lo[8], hi[8];
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) lo[e] = v[e], hi[e] = v[V - 8 + e];
+                        to_fp8x8(lo, o[0], o[1]);
+                        to_fp8x8(hi, o[2], o[3]);
+                    } else {
+#pragma unroll
+                        for (int d = 0; d < 4; ++d) {
+                            const __half2 pr = __floats2half2_rn(v[2 * d], v[2 * d + 1]);
+                            o[d] = *reinterpret_cast<const uint32_t *>(&pr);
+                        }
+                    }
+                    store_writethrough16(dst, o[0], o[1], o[2], o[3]);
+                    if (F8 && h == H - 1 && (H & 1) != 0) store_writethrough16(dst + LANES * nrows * 16, 0, 0, 0, 0);
+                }
+            }
+            return;
+        }
+        if (!busy) return;
         __builtin_amdgcn_wave_barrier();
         // This lane's row of the chunk (rows past the image's last query: zero scores of zero queries, not stored).
         const int qr = tile * 32 + (lane >> 1);
@@ -246,8 +296,8 @@ template <int NKB, int NQ, bool F8>
 void launch_attention(const void *qkv, void *out, int B, int n, int H, float scale, const float *thr, const float *cb, hipStream_t stream)
 {
     // Parts of a head: as many as the compute units take, so that the waves that share a SIMD in a workgroup of a whole head have one
-    // each.  197 tokens of 6 heads (with the consumer's stage 1): 9.9 us in one part, 8.0 in two, 7.7 in seven; 16 images 10.2 / 8.5
-    // in two parts, 10.7 in three (288 workgroups).
+    // each, the tables are built under the product and (one tile a part) all waves share the consumer's stage 1.  197 tokens of 6
+    // heads with that stage 1: 9.5 us in one part, 6.5 in seven; 16 images 9.9 and 7.7 in two parts.
     const int64_t heads = static_cast<int64_t>(B) * H;
     const int parts = static_cast<int>(std::min<int64_t>(NKB, std::max<int64_t>(1, device_cus() / heads)));
     auto kernel = NKB > 1 && parts > 1 ? attention_kernel<NKB, NQ, F8, (NKB > 1)> : attention_kernel<NKB, NQ, F8, false>;
