@@ -157,6 +157,68 @@ prepare_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const f
     }
 }
 
+// The same for launches of a few rows, which are one chain of instructions long: eight lanes a group (FP8: four), each with the
+// values of one 16-byte piece of x_hat, eight (sixteen) rows a wave, no LDS but the tables.
+template <typename TIN, int BITS, bool F8>
+__global__ void __launch_bounds__(64 * (kPrepWaves + 1))
+prepare_few_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const float *__restrict__ cb, char *__restrict__ x_hat, float eps,
+                   int rows, int G, PrepWeights w0, PrepWeights w1)
+{
+    constexpr int LANES = F8 ? 4 : 8, V = 64 / LANES, ROWS = 64 / LANES;
+    constexpr int kIn = V * static_cast<int>(sizeof(TIN)) / 16;
+    __shared__ QuantTables tables;
+    if (prep_weight_workgroup<BITS, F8>(w0, w1, tables.cb)) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (wave == kPrepWaves) {
+        build_quant_tables<BITS>(load_quant_params<BITS>(thr, cb, lane), tables, lane);
+        __syncthreads();
+        return;
+    }
+    const int t = static_cast<int>(blockIdx.x - (w0.blocks + w1.blocks)) * kPrepWaves + wave;
+    const int rb = t / G, g = t - rb * G;
+    const int r = rb * ROWS + lane / LANES, piece = lane % LANES;
+    const bool live = r < rows;
+    const int64_t K = static_cast<int64_t>(G) * 64;
+    const uint4 *src = reinterpret_cast<const uint4 *>(x + min(r, rows - 1) * K + g * 64 + piece * V);
+    uint4 raw[kIn];
+#pragma unroll
+    for (int i = 0; i < kIn; ++i) raw[i] = src[i];
+    float v[V];
+#pragma unroll
+    for (int i = 0; i < kIn; ++i) {
+        const uint32_t w[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            if constexpr (sizeof(TIN) == 2) {
+                v[8 * i + 2 * d] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[d] & 0xffffu)));
+                v[8 * i + 2 * d + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[d] >> 16)));
+            } else {
+                v[4 * i + d] = __uint_as_float(w[d]);
+            }
+        }
+    }
+    float mu, var, s, sum_codes;
+    group_stats_lanes<LANES>(v, eps, lane, mu, var, s);
+    __syncthreads();
+    group_codes_lanes<BITS, LANES>(v, mu, var, s, tables, tables.geometry, tables.usable != 0, lane, sum_codes);
+    if (!live) return;
+    const float code_mean = sum_codes * 0.015625f;
+    uint32_t o[4];
+    if constexpr (F8) {
+        xhat_fp8x16(v, 0, s, code_mean, mu, o);
+    } else {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const __half2 h = __floats2half2_rn(fma_f32(s, v[2 * d] - code_mean, mu), fma_f32(s, v[2 * d + 1] - code_mean, mu));
+            o[d] = *reinterpret_cast<const uint32_t *>(&h);
+        }
+    }
+    const int blk = r >> 5, nrows = min(32, rows - blk * 32), row_groups = F8 ? (G + 1) / 2 * 2 : G;
+    char *dst = x_hat + (static_cast<int64_t>(blk) * 32 * row_groups * LANES + (g * LANES + piece) * nrows + (r & 31)) * 16;
+    store_writethrough16(dst, o[0], o[1], o[2], o[3]);
+    if (F8 && row_groups > G && g == G - 1) store_writethrough16(dst + LANES * nrows * 16, 0, 0, 0, 0);
+}
+
 // LayerNorm over the rows first.  Wave w of a workgroup's tile takes rows R w ... R w + R - 1, 2 G lanes per row, so that the
 // row sums stay inside the wave.  Vector-ALU-bound from a few thousand rows on, one dependent chain below.  The partial sums of
 // a row go through wave-private LDS padded with zeros to a multiple of eight (x + 0 leaves the sum as it is), so that all reads
@@ -373,19 +435,29 @@ void launch_prepare_t(const arcq_prepare_args &a, float eps, const PrepWeights &
             return;
         }
     }
-    // Up to 2 048 tiles (two workgroups per CU) the launch is latency-bound: every wave takes one tile and a fifth wave builds the
-    // tables meanwhile (6 304 x 384: 6.7 us against 7.6 without it).  Beyond that the grid is what the chip holds at once (fp32: three
-    // workgroups per CU; 12 608 x 1 536 25.4 -> 21.7 us against four), the
-    // tables are built once per workgroup and the waves walk their tiles with the next one's loads in flight (12 608 x 1 536:
-    // 18-19 us; a workgroup per four tiles 27-30).
+    // Few rows: 197 x 384 4.7 -> 3.8 us, 3 349 x 384 5.0 -> 4.6; fp32 and FP8 move other amounts and win longer (6 304 x 384 fp32
+    // 7.1 -> 5.3, 6 304 x 768 FP8 8.0 -> 6.9, both 1 182 workgroups, where fp16 takes 5.5 against 5.1).
+    const int few = ((rows + (F8 ? 15 : 7)) / (F8 ? 16 : 8) * G + kPrepWaves - 1) / kPrepWaves;
+    if (weights + few == 0) return;
+    if (few <= (F8 || sizeof(TIN) == 4 ? 6 : 4) * device_cus()) {
+        hipLaunchKernelGGL((prepare_few_kernel<TIN, BITS, F8>), dim3(weights + few), dim3(kPrepThreads + 64), 0, stream, x, a.thresholds,
+                           a.codebook, x_hat, eps, rows, G, w0, w1);
+        return;
+    }
+    // Up to 2 048 tiles (two workgroups per CU) every wave takes one tile and a fifth wave builds the tables meanwhile (6 304 x 384:
+    // 5.1 us).  Beyond that the grid is what the chip holds at once (fp32: three workgroups per CU; 12 608 x 1 536 25.4 -> 21.7 us
+    // against four), the tables are built once per workgroup and the waves walk their tiles with the next one's loads in flight
+    // (12 608 x 1 536: 18-19 us; a workgroup per four tiles 27-30).
     const int tiles = ((rows + 31) / 32) * G, wgs = std::min((tiles + kPrepWaves - 1) / kPrepWaves, (sizeof(TIN) == 4 ? 3 : 4) * device_cus());
-    if (weights + wgs == 0) return;
-    if (tiles <= 2048)
-        hipLaunchKernelGGL((prepare_kernel<TIN, BITS, F8, true>), dim3(weights + wgs), dim3(kPrepThreads + 64), 0, stream, x, a.thresholds,
-                           a.codebook, x_hat, eps, rows, G, w0, w1);
-    else
-        hipLaunchKernelGGL((prepare_kernel<TIN, BITS, F8, false>), dim3(weights + wgs), dim3(kPrepThreads), 0, stream, x, a.thresholds,
-                           a.codebook, x_hat, eps, rows, G, w0, w1);
+    if constexpr (!F8) {
+        if (tiles <= 2048) {
+            hipLaunchKernelGGL((prepare_kernel<TIN, BITS, F8, true>), dim3(weights + wgs), dim3(kPrepThreads + 64), 0, stream, x, a.thresholds,
+                               a.codebook, x_hat, eps, rows, G, w0, w1);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((prepare_kernel<TIN, BITS, F8, false>), dim3(weights + wgs), dim3(kPrepThreads), 0, stream, x, a.thresholds,
+                       a.codebook, x_hat, eps, rows, G, w0, w1);
 }
 
 template <typename TIN, bool F8>

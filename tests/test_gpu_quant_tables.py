@@ -74,3 +74,21 @@ def test_lanes_per_group_behind_a_layernorm(cuda, oracle, m, k, dtype):
         want = oracle.act_quant_c(ln, t, cb, 4, 64)["x_hat"].astype(np.float16)
         got = _prepare(x.to(cuda), t.to(cuda), cb.to(cuda), 4, (g.to(cuda), b.to(cuda), 1e-6))[0]
         assert np.array_equal(got.cpu().numpy().view(np.uint16), _blocked(want).view(np.uint16))
+
+
+# stage 1 alone: a piece per lane, a tile per wave, walking waves; ragged row tiles, infinities and NaN
+@pytest.mark.parametrize("m,k", [(1, 64), (7, 192), (197, 384), (2049, 960), (4097, 512), (6304, 384), (6309, 768), (20011, 384)])
+@pytest.mark.parametrize("bits,dtype", [(4, torch.float16), (3, torch.float32), (2, torch.float16)])
+def test_stage_1_alone(cuda, oracle, m, k, bits, dtype):
+    cb = synth.quantile_codebook(bits)
+    thr = synth.midpoint_thresholds(cb)
+    x = synth.make_activation(m, k, 23).to(dtype)
+    x[m - 1, :4] = torch.tensor([1.0, INF, -INF, float("nan")], dtype=dtype)
+    x[m // 2, k - 64:] = 0.25
+    x[m // 3] *= 6e-5 if dtype == torch.float16 else 1e-30
+    for t in (thr, torch.cat([thr[1:], thr[:1]])):
+        with np.errstate(all="ignore"):
+            want = _blocked(oracle.act_quant_c(x.float().numpy(), t, cb, bits, 64)["x_hat"].astype(np.float16))
+        got = _prepare(x.to(cuda), t.contiguous().to(cuda), cb.to(cuda), bits)[0].cpu().numpy()
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got), nan) and np.array_equal(got.view(np.uint16)[~nan], want.view(np.uint16)[~nan])
