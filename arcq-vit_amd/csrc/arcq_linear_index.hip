@@ -10,6 +10,7 @@
 #include "arcq_gemm.h"
 
 #include <type_traits>
+#include <cstdlib>
 
 namespace arcq {
 
@@ -311,15 +312,30 @@ struct IndexArgs {
     const float *wc, *ws, *wcs, *table, *a_cb, *w_cb, *bias;
     float *y;
     int rows, out_f, G, levels;
+    int workers;                     // linear_index_mfma_kernel: the workgroups that share the tiles where the table does not qualify
 };
 
-// The tile of rows r0 .. and outputs o0 .., by a workgroup of at least MINW waves.
-template <int BITS, int R, int C, int MINW>
-__device__ __forceinline__ void index_wide_tile(const IndexArgs &p, int r0, int o0)
+// The product table and the codebooks in LDS.
+template <int LEVELS>
+struct IndexTables {
+    float table[LEVELS * LEVELS], a_cb[LEVELS], w_cb[LEVELS];
+};
+// Stores entry i; whether it is the product of its two codebook values.
+template <int LEVELS>
+__device__ __forceinline__ int index_table_entry(const IndexArgs &p, IndexTables<LEVELS> &t, int i, float value)
+{
+    t.table[i] = value;
+    if (i < p.levels) t.a_cb[i] = p.a_cb[i], t.w_cb[i] = p.w_cb[i];
+    return static_cast<int>(__float_as_uint(value) == __float_as_uint(p.a_cb[i / p.levels] * p.w_cb[i % p.levels]));
+}
+
+// The tile of rows r0 .. and outputs o0 .., by a workgroup of at least MINW waves.  FILL: the tables are loaded here; otherwise they
+// are complete, and `outer` says whether the product table is one of the codebooks.
+template <int BITS, int R, int C, int MINW, bool FILL>
+__device__ __forceinline__ void index_wide_tile(const IndexArgs &p, int r0, int o0, IndexTables<BITS ? 1 << BITS : 16> &tables, int outer)
 {
 #pragma clang fp contract(off)
     constexpr bool kPacked = BITS != 0;
-    constexpr int kLevels = kPacked ? 1 << BITS : 16;
     constexpr int TR = 8 * R, TC = 8 * C;
     constexpr int kRowBytes = kPacked ? 8 * BITS : 64;
     constexpr int kPieceBytes = kRowBytes / 8;                        // eight codes
@@ -328,15 +344,14 @@ __device__ __forceinline__ void index_wide_tile(const IndexArgs &p, int r0, int 
     constexpr int kPitch = TC + 1;                                     // terms per row of the tile
     using acc_t = typename std::conditional<kPacked, double, float>::type;
     static_assert((TR + TC) * 32 * 4 <= kIdxRegion && TR * kPitch * static_cast<int>(sizeof(acc_t)) <= kIdxRegion, "LDS region");
-    __shared__ float s_table[kLevels * kLevels], s_acb[kLevels], s_wcb[kLevels];
+    const float *s_table = tables.table, *s_acb = tables.a_cb, *s_wcb = tables.w_cb;
     extern __shared__ __attribute__((aligned(16))) unsigned char idx_smem[];     // [S waves][kIdxRegion]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nthreads = blockDim.x, S = nthreads >> 6;
     const int lx = lane & 7, ly = lane >> 3;
     const int rows = p.rows, out_f = p.out_f, G = p.G, levels = p.levels;
     const uint8_t *__restrict__ xq = p.xq, *__restrict__ wq = p.wq;
     const float *__restrict__ xc = p.xc, *__restrict__ xs = p.xs, *__restrict__ xcs = p.xcs, *__restrict__ wc = p.wc, *__restrict__ ws = p.ws;
-    const float *__restrict__ wcs = p.wcs, *__restrict__ table = p.table, *__restrict__ a_cb = p.a_cb, *__restrict__ w_cb = p.w_cb;
-    const float *__restrict__ bias = p.bias;
+    const float *__restrict__ wcs = p.wcs, *__restrict__ bias = p.bias;
     float *__restrict__ y = p.y;
     unsigned char *region = idx_smem + wave * kIdxRegion;
     float *s_x = reinterpret_cast<float *>(region), *s_w = s_x + TR * 32;
@@ -362,14 +377,11 @@ __device__ __forceinline__ void index_wide_tile(const IndexArgs &p, int r0, int 
         for (int i = 0; i < kWJobs; ++i) load_piece(w_src + static_cast<int64_t>(g) * kRowBytes + i * (64 / TC) * kPieceBytes, wn[i]);
     };
     if (wave < G) fetch(wave);
-    int same = 1;
-    for (int i = tid; i < levels * levels; i += nthreads) {
-        const float t = table[i];
-        s_table[i] = t;
-        same &= static_cast<int>(__float_as_uint(t) == __float_as_uint(a_cb[i / levels] * w_cb[i % levels]));
+    if constexpr (FILL) {
+        int same = 1;
+        for (int i = tid; i < levels * levels; i += nthreads) same &= index_table_entry(p, tables, i, p.table[i]);
+        outer = __syncthreads_and(same);
     }
-    if (tid < levels) s_acb[tid] = a_cb[tid], s_wcb[tid] = w_cb[tid];
-    const bool outer = __syncthreads_and(same) != 0;
     // With its address seen by an asm statement the region is memory the statements in the loops below may touch, so its
     // reads stay where they are written.  (The compiler otherwise moves all reads of a group to its top: 500 registers.)
     asm volatile("" ::"v"(region) : "memory");
@@ -548,7 +560,7 @@ __device__ __forceinline__ void index_wide_tile(const IndexArgs &p, int r0, int 
             __syncthreads();
         }
     };
-    if (outer) body(std::true_type{});
+    if (outer != 0) body(std::true_type{});
     else body(std::false_type{});
 #pragma unroll
     for (int i = 0; i < kSums; ++i) {
@@ -561,7 +573,8 @@ __device__ __forceinline__ void index_wide_tile(const IndexArgs &p, int r0, int 
 template <int BITS, int R, int C, int MAXW>
 __global__ void __launch_bounds__(64 * MAXW, MAXW > kIdxMaxWaves ? 1 : R == 1 ? 4 : 3) linear_index_wide_kernel(const IndexArgs p)
 {
-    index_wide_tile<BITS, R, C, kIdxMinWaves>(p, blockIdx.y * 8 * R, blockIdx.x * 8 * C);
+    __shared__ IndexTables<BITS ? 1 << BITS : 16> tables;
+    index_wide_tile<BITS, R, C, kIdxMinWaves, true>(p, blockIdx.y * 8 * R, blockIdx.x * 8 * C, tables, 0);
 }
 
 // ---- the packed format on the matrix units ---------------------------------------------------------------------------------
@@ -571,37 +584,53 @@ __global__ void __launch_bounds__(64 * MAXW, MAXW > kIdxMaxWaves ? 1 : R == 1 ? 
 // at most one byte in four, so the products are the 4:2 sparse ones (v_smfmac_i32_32x32x64_i8, twice the dense rate; of the two
 // stored bytes of a four only the first is used).  The five int32 sums together are the sum of the table entries, the same double
 // that the serial loop ends with, and the group's closed form follows in the same operations: the result's bits stay what they
-// are.  Every workgroup looks the table over for its lowest and highest bit; a table that does not qualify (largest entry more
-// than 2^14 times the smallest, subnormals, infinities, NaN) runs the loops above on the same tile.
+// are.  Every workgroup looks the table over for its lowest and highest bit.  A table that does not qualify (largest entry more
+// than 2^14 times the smallest, subnormals, infinities, NaN: fitted codebooks with a level near zero are like that) runs the loops
+// above, 16 rows a tile.
 //
 // The wide kernel above spends a multiplication, a conversion and an fp64 addition of the vector ALU on every product; here 4 096
 // products take five MFMAs of 32 clocks on a pipe of their own.  A wave owns 32 x 32 outputs for all groups, in order.  The digits
-// come from a 1 280-byte table in LDS by the w code, 16 bytes a read (2^bits different entries: no bank conflicts); the x operand
-// is made in registers, and the fp64 sums lie in LDS between the groups so that three waves fit a SIMD: matrix pipe, vector ALU
-// (the closed form, 13 instructions per output and group) and LDS are each about half busy, and the waves overlap them.
-// Measured, this kernel against the wide one: 1576 x 384 -> 1536 at 4 / 3 / 2 bits 55 / 45 / 32 us against 113 / 103 / 99, 12608
-// rows at 4 bits 307 against 714.  With dense products 82 us; 64 x 32 outputs a wave and the groups dealt over the waves 117.
+// come from a 1 280-byte table in LDS by the w code, 16 bytes a read (2^bits different entries: no bank conflicts, measured); the
+// x operand is made in registers, and the fp64 sums lie in LDS between the groups so that three waves fit a SIMD.  What bounds it
+// is the LDS: 184 reads of 16 bytes a lane for a wave's group, 160 of them digits; of a launch of 12608 x 1536 -> 384 at 4 bits it
+// is busy 64 %, the matrix pipes and the vector ALU (the closed form, 13 instructions per output and group) 47 % each.
+// Measured, this kernel against the wide one: 1576 x 384 -> 1536 at 4 / 3 / 2 bits 51 / 44 / 33 us against 103 / 108 / 104, 12608
+// rows at 4 bits 309 against 725.  With dense products 82 us; 64 x 32 outputs a wave and the groups dealt over the waves 117.
 constexpr int kDigits = 5, kMaxEntryBits = 38;
-constexpr int kMfmaWaves = 4, kMfmaTile = 32;                      // a wave's tile is 32 x 32, the workgroup's 32 outputs wide
+constexpr int kMfmaTile = 32;                      // a wave's tile is 32 x 32, the workgroup's 32 outputs wide
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
 typedef int i32x16_t __attribute__((ext_vector_type(16)));
 
+// The smallest of the lanes' numbers, in a scalar register.
+__device__ __forceinline__ int wave_min(int v)
+{
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x121, 0xf, 0xf, false));       // row_ror: the minimum of the sixteen lanes
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x122, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x124, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false));
+    return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
 template <int BITS>
-__global__ void __launch_bounds__(64 * kMfmaWaves, 3)
+__global__ void __launch_bounds__(64 * kIdxMaxWaves, 3)
 linear_index_mfma_kernel(const IndexArgs p)
 {
 #pragma clang fp contract(off)
     constexpr int L = 1 << BITS, kEntries = L * L, E = 16 / L;                   // E: j's of 16 bytes
     constexpr int kSteps = 16 / E;                                               // 4 E j's each
     __shared__ __attribute__((aligned(16))) signed char s_digits[kDigits * kEntries];        // [digit][w code][x code]
-    __shared__ __attribute__((aligned(16))) double s_meta[kMfmaWaves][3][kMfmaTile];
-    __shared__ int s_low, s_high;
+    __shared__ __attribute__((aligned(16))) double s_meta[kIdxMaxWaves][3][kMfmaTile];
+    __shared__ IndexTables<L> tables;
+    __shared__ int s_low[kIdxMaxWaves], s_high[kIdxMaxWaves];
     extern __shared__ __attribute__((aligned(16))) unsigned char idx_smem[];     // [waves][kIdxRegion]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lh = lane >> 5;
-    constexpr int kThreads = 64 * kMfmaWaves, kEach = (kEntries + kThreads - 1) / kThreads;
-    const int r0 = blockIdx.y * (kMfmaWaves * kMfmaTile), ow = blockIdx.x * kMfmaTile;
+    const int nthreads = blockDim.x, S = nthreads >> 6;
+    constexpr int kEach = (kEntries + 64 * kIdxMinWaves - 1) / (64 * kIdxMinWaves);
+    const int across = (p.out_f + kMfmaTile - 1) / kMfmaTile;                    // workgroups side by side
+    const int r0 = blockIdx.x / across * (S * kMfmaTile), ow = blockIdx.x % across * kMfmaTile;
     const int rw = r0 + wave * kMfmaTile;                                        // rows of the wave's tile
     const int G = p.G;
 
@@ -621,33 +650,34 @@ linear_index_mfma_kernel(const IndexArgs p)
         xmn[0] = x_meta[xrow + g], xmn[1] = p.xcs[xrow + g];
         wmn[0] = p.wc[wrow + g], wmn[1] = p.ws[wrow + g], wmn[2] = p.wcs[wrow + g];
     };
-    fetch(0);
-
     // The table's entries as integers over 2^low.
-    if (tid == 0) s_low = 1 << 20, s_high = -(1 << 20);
-    __syncthreads();
     uint32_t entry[kEach];                                                       // (a, b) = (x code, w code) = (i / L, i % L)
-    int bad = 0;
+    int same = 1, lo = 1 << 20, hi = -(1 << 20);                                           // the bits that any of this thread's use
 #pragma unroll
     for (int k = 0; k < kEach; ++k) {
-        const int i = tid + k * kThreads;
+        const int i = tid + k * nthreads;
         entry[k] = i < kEntries ? __float_as_uint(p.table[i]) : 0;
+        if (i < kEntries) same &= index_table_entry(p, tables, i, __uint_as_float(entry[k]));
         const int exponent = static_cast<int>((entry[k] >> 23) & 255u);
-        bad |= exponent == 255 || (exponent == 0 && (entry[k] & 0x7fffffu));      // infinity, NaN, subnormal
-        if (exponent != 0) {
-            atomicMin(&s_low, exponent - 150 + (__ffs(static_cast<int>(entry[k] | 0x800000u)) - 1));
-            atomicMax(&s_high, exponent - 126);
-        }
+        if (exponent != 0) lo = min(lo, exponent - 150 + (__ffs(static_cast<int>(entry[k] | 0x800000u)) - 1)), hi = max(hi, exponent - 126);
+        if (exponent == 255 || (exponent == 0 && (entry[k] & 0x7fffffu))) hi = 1 << 21;      // infinity, NaN, subnormal: too wide
     }
-    const bool any_bad = __syncthreads_or(bad) != 0;
-    const int low = s_low <= s_high ? s_low : 0;                                 // (else all entries are zero)
-    if (any_bad || s_high - low > kMaxEntryBits) {                               // workgroup-uniform
-        for (int r = r0; r < min(r0 + kMfmaWaves * kMfmaTile, p.rows); r += 16) index_wide_tile<BITS, 2, 4, kMfmaWaves>(p, r, ow);
+    lo = wave_min(lo), hi = -wave_min(-hi);
+    if (lane == 0) s_low[wave] = lo, s_high[wave] = hi;
+    same = __syncthreads_and(same);
+    for (int w = 0; w < S; ++w) lo = min(lo, s_low[w]), hi = max(hi, s_high[w]);
+    const int low = lo <= hi ? lo : 0;                                           // (else all entries are zero)
+    if (hi - low > kMaxEntryBits) {                                              // workgroup-uniform
+        const int tiles = across * ((p.rows + 15) / 16);
+        for (int t = blockIdx.x; t < tiles && static_cast<int>(blockIdx.x) < p.workers; t += p.workers)
+            index_wide_tile<BITS, 2, 4, kIdxMinWaves, false>(p, t / across * 16, t % across * 32, tables, same);
         return;
     }
+    if (r0 >= p.rows) return;                                                    // (a workgroup that is here for the loops above only)
+    fetch(0);
 #pragma unroll
     for (int k = 0; k < kEach; ++k) {
-        const int i = tid + k * kThreads, exponent = static_cast<int>((entry[k] >> 23) & 255u);
+        const int i = tid + k * nthreads, exponent = static_cast<int>((entry[k] >> 23) & 255u);
         const int shift = exponent - 150 - low;                                  // (negative: by zero bits of the entry)
         long long v = exponent == 0 ? 0 : static_cast<long long>((entry[k] & 0x7fffffu) | 0x800000u);
         v = shift >= 0 ? v << min(shift, 40) : v >> min(-shift, 23);
@@ -662,7 +692,8 @@ linear_index_mfma_kernel(const IndexArgs p)
         }
     }
     __syncthreads();
-    const double unit = ldexp(1.0, low), per_unit64 = ldexp(1.0, -low - 6);
+    const int low_s = __builtin_amdgcn_readfirstlane(low);                       // 2^low and 2^(-low - 6), in scalar registers
+    const double unit = __longlong_as_double((1023LL + low_s) << 52), per_unit64 = __longlong_as_double((1017LL - low_s) << 52);
 
     // Bits from..to (of BITS) of code number q, `up` bits to the left.
     auto code_bits = [](const uint32_t (&w)[BITS], int q, int from, int to, int up) __attribute__((always_inline)) {
@@ -709,14 +740,16 @@ linear_index_mfma_kernel(const IndexArgs p)
         meta[lh][lr] = lh ? static_cast<double>(xmn[0]) : 64.0 * static_cast<double>(xmn[0]);
         meta[2][lr] = xmn[1];
         i32x16_t sum[kDigits];
+        int zero = 0;
+        asm volatile("" : "+s"(zero));                                           // (of the constant the compiler keeps sixteen in scratch)
 #pragma unroll
         for (int d = 0; d < kDigits; ++d)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) sum[d][v] = 0;
-        // The operands of step t + 1 are read under the products of step t.
-        i32x4_t xf[2];
-        uint32_t index[2];
-        i32x8_t wf[2][kDigits];
+            for (int v = 0; v < 16; ++v) sum[d][v] = zero;
+        // (The reads of a step's digits run under the products before it as far as the registers go: three fragments of eight.)
+        i32x4_t xf;
+        uint32_t index;
+        i32x8_t wf[kDigits];
         auto operands = [&](int t, i32x4_t &a, uint32_t &ix, i32x8_t (&b)[kDigits]) __attribute__((always_inline)) {
             const signed char *src[2 * E];
 #pragma unroll
@@ -744,10 +777,10 @@ linear_index_mfma_kernel(const IndexArgs p)
         };
 #pragma unroll
         for (int t = 0; t < kSteps; ++t) {
-            operands(t, xf[0], index[0], wf[0]);
+            operands(t, xf, index, wf);
 #pragma unroll
             for (int d = 0; d < kDigits; ++d)
-                sum[d] = __builtin_amdgcn_smfmac_i32_32x32x64_i8(xf[0], wf[0][d], sum[d], static_cast<int>(index[0]), 0, 0);
+                sum[d] = __builtin_amdgcn_smfmac_i32_32x32x64_i8(xf, wf[d], sum[d], static_cast<int>(index), 0, 0);
         }
         if (g + 1 < G) fetch(g + 1);                                             // (under the closed form; the products need the registers)
         asm volatile("" ::: "memory");
@@ -774,26 +807,44 @@ linear_index_mfma_kernel(const IndexArgs p)
     }
 }
 
+// Waves per workgroup: the count that leaves the fewest of them without a group in the last round, the larger one of equals
+// (384 -> 1536, six groups, 12608 rows, wide kernel: three waves 744, four waves 832 us).
+inline int index_waves(int G)
+{
+    int S = kIdxMaxWaves;
+    for (int s = kIdxMaxWaves - 1; s >= kIdxMinWaves; --s)
+        if ((G + s - 1) / s * s < (G + S - 1) / S * S) S = s;
+    return S;
+}
+
+// The host does not see the table, so the launch serves both cases.  Waves per workgroup as above: the matrix-unit tiles are a
+// wave's own and do not mind (1576 x 384 -> 1536 51.0 us with three, 51.7 with four).  Where their workgroups would leave compute
+// units idle, more are launched for the 16-row tiles of the loops, as many as are resident at once; a table that qualifies sends
+// them home after the look at it (512 x 384 -> 1024 26 us with and without them).  From one resident set on the tiles are dealt to
+// as many workgroups as are resident (of three-wave ones not quite four fit a compute unit), from three on to all of them, and the
+// dispatch evens out the last round.  Tables that do not qualify, against the wide kernel alone: 512 x 384 -> 1024 29 / 28 us with
+// computed and 48 / 48 with gathered entries, 1576 x 384 -> 1536 111 / 103 and 208 / 216, 12608 x 384 -> 1536 763 / 725 and
+// 1570 / 1562, 12608 x 1536 -> 384 755 / 690 and 1479 / 1562; at worst, where two rounds are not full, 5000 x 576 -> 768 275 / 228.
+// (Eight tiles in turn per 128-row workgroup: 100, 164, 936 and 811 us with computed entries.)
 template <int BITS>
 void launch_index_mfma(const IndexArgs &a, hipStream_t stream)
 {
-    hipLaunchKernelGGL((linear_index_mfma_kernel<BITS>), dim3((a.out_f + kMfmaTile - 1) / kMfmaTile, (a.rows + kMfmaWaves * kMfmaTile - 1) / (kMfmaWaves * kMfmaTile)),
-                       dim3(64 * kMfmaWaves), kMfmaWaves * kIdxRegion, stream, a);
+    const int across = (a.out_f + kMfmaTile - 1) / kMfmaTile, S = index_waves(a.G), resident = 4 * kIdxMinWaves / S * device_cus();
+    const int own = across * ((a.rows + S * kMfmaTile - 1) / (S * kMfmaTile)), grid = max(own, min(resident, across * ((a.rows + 15) / 16)));
+    IndexArgs b = a;
+    b.workers = own <= resident || own >= 3 * resident ? grid : S == kIdxMaxWaves ? resident : resident - resident / 16;
+    hipLaunchKernelGGL((linear_index_mfma_kernel<BITS>), dim3(grid), dim3(64 * S), S * kIdxRegion, stream, b);
 }
 
 template <int BITS, int R, int C, int MAXW>
 void launch_index_wide(const IndexArgs &a, hipStream_t stream)
 {
-    // Waves per workgroup: the count that leaves the fewest of them without a group in the last round, the larger one of
-    // equals (384 -> 1536, six groups, 12608 rows: three waves 744, four waves 832 us); of sixteen, the fewest for the fewest rounds.
-    int S = MAXW;
+    // Of up to sixteen waves the fewest for the fewest rounds.
+    int S = index_waves(a.G);
     if constexpr (MAXW > kIdxMaxWaves) {
         const int rounds = (a.G + MAXW - 1) / MAXW;
         S = (a.G + rounds - 1) / rounds;
         allow_dynamic_lds<linear_index_wide_kernel<BITS, R, C, MAXW>>(MAXW * kIdxRegion);
-    } else {
-        for (int s = kIdxMaxWaves - 1; s >= kIdxMinWaves; --s)
-            if ((a.G + s - 1) / s * s < (a.G + S - 1) / S * S) S = s;
     }
     hipLaunchKernelGGL((linear_index_wide_kernel<BITS, R, C, MAXW>), dim3((a.out_f + 8 * C - 1) / (8 * C), (a.rows + 8 * R - 1) / (8 * R)), dim3(64 * S),
                        S * kIdxRegion, stream, a);
@@ -810,7 +861,7 @@ void launch_index(const IndexArgs &a, hipStream_t stream)
     // launch takes: 394 x 768 -> 768 (312) 45.2 against 34.6 us, 197 x 192 -> 768 (168) 16.1 / 10.1.
     if constexpr (BITS != 0) {
         const int64_t tiles = static_cast<int64_t>((a.rows + kMfmaTile - 1) / kMfmaTile) * ((a.out_f + kMfmaTile - 1) / kMfmaTile);
-        if (tiles >= 2 * device_cus() && static_cast<int64_t>(a.rows > a.out_f ? a.rows : a.out_f) * a.G * 2 * BITS < (int64_t(1) << 31))
+        if (tiles >= 2 * device_cus() && tiles < (int64_t(1) << 24) && static_cast<int64_t>(a.rows > a.out_f ? a.rows : a.out_f) * a.G * 2 * BITS < (int64_t(1) << 31))
             return launch_index_mfma<BITS>(a, stream);
     }
     // No more workgroups than compute units: up to sixteen waves each, i.e. as few rounds of groups as possible.
@@ -945,7 +996,7 @@ ARCQ_API int arcq_linear_index(const arcq_linear_index_args *a, void *stream)
     }
     const IndexArgs g{a->x_codes, a->x_center, a->x_scale, a->x_code_sum, a->w_codes, a->w_center, a->w_scale, a->w_code_sum, a->product_table,
                       a->a_codebook, a->w_codebook, a->bias, a->y, static_cast<int>(a->rows), static_cast<int>(a->out_features),
-                      static_cast<int>(a->in_features / 64), a->levels};
+                      static_cast<int>(a->in_features / 64), a->levels, 0};
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (a->bits == 4) launch_index<4>(g, st);
     else if (a->bits == 3) launch_index<3>(g, st);

@@ -45,7 +45,7 @@ def test_linear_index_bitexact(cuda, oracle, m, n, k, bits, outer):
 # and leaves to the fp64 loops (entries too far apart, a subnormal, an infinity, a NaN).
 @pytest.mark.parametrize("m,n,k", [(545, 1000, 128), (4100, 127, 64), (33, 8225, 320)])
 @pytest.mark.parametrize("bits", [4, 3, 2])
-@pytest.mark.parametrize("kind", ["outer", "arbitrary", "zeros", "all_zero", "powers", "far_apart", "subnormal", "infinity", "nan"])
+@pytest.mark.parametrize("kind", ["outer", "arbitrary", "zeros", "all_zero", "powers", "far_apart", "subnormal", "all_subnormal", "infinity", "nan"])
 def test_linear_index_on_the_matrix_units(cuda, oracle, m, n, k, bits, kind):
     levels = 1 << bits
     cb = synth.quantile_codebook(bits)
@@ -59,6 +59,8 @@ def test_linear_index_on_the_matrix_units(cuda, oracle, m, n, k, bits, kind):
         table = torch.zeros_like(table)
     elif kind == "powers":
         table = torch.sign(table) * 2.0 ** (torch.arange(table.numel()).view_as(table) % 15 - 80)
+    elif kind == "all_subnormal":
+        table = table * 1.0e-40
     elif kind != "outer":
         table[1, 1] = {"far_apart": 1.0e-6, "subnormal": 1.0e-40, "infinity": float("inf"), "nan": float("nan")}[kind]
     rng = np.random.default_rng(7)
@@ -74,3 +76,61 @@ def test_linear_index_on_the_matrix_units(cuda, oracle, m, n, k, bits, kind):
     a = _lib.LinearIndexArgs(*[v.data_ptr() for v in t], y.data_ptr(), m, n, k, bits, 64, levels, 0)
     _lib.check(_lib.load().arcq_linear_index(ctypes.byref(a), torch.cuda.current_stream().cuda_stream))
     assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
+
+
+def _microseconds(calls, stream):
+    """The shortest of ten runs of ``calls``, five times over each."""
+    best = float("inf")
+    for _ in range(10):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        for _ in range(5):
+            for a in calls:
+                _lib.check(_lib.load().arcq_linear_index(ctypes.byref(a), stream))
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, begin.elapsed_time(end) * 200.0)
+    return best
+
+
+def _call(cuda, m, n, k, bits, table, a_cb, w_cb):
+    g = k // 64
+    t = [torch.randint(0, 256, (m, k * bits // 8), dtype=torch.uint8, device=cuda), *(torch.randn(m, g, device=cuda) for _ in range(3)),
+         torch.randint(0, 256, (n, k * bits // 8), dtype=torch.uint8, device=cuda), *(torch.randn(n, g, device=cuda) for _ in range(3)),
+         table.to(cuda), a_cb.to(cuda), w_cb.to(cuda), torch.randn(n, device=cuda), torch.empty(m, n, device=cuda)]
+    return _lib.LinearIndexArgs(*[v.data_ptr() for v in t], m, n, k, bits, 64, 1 << bits, 0), t
+
+
+def _codebook_with_a_level_near_zero(bits):
+    cb = synth.quantile_codebook(bits).clone()
+    cb[(1 << bits) // 2] = 0.001234567
+    return cb, (cb.view(-1, 1) * cb.view(1, -1)).contiguous()
+
+
+# Such a table runs on the loops, with as many workgroups as are resident at once or, of larger launches, with all (256 compute
+# units; three and four waves): the same bits as the entry point without codebooks gives.
+@pytest.mark.parametrize("m,n,k", [(1000, 550, 192), (4100, 775, 192), (4100, 2400, 192), (4100, 775, 256), (4100, 2331, 256)])
+@pytest.mark.parametrize("outer", [True, False])
+def test_tables_that_do_not_qualify_in_larger_launches(cuda, m, n, k, outer):
+    cb, table = _codebook_with_a_level_near_zero(4)
+    if not outer:
+        table[1, 1] = 1.0e-6
+    a, t = _call(cuda, m, n, k, 4, table, cb, cb)
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.check(_lib.load().arcq_linear_index(ctypes.byref(a), stream))
+    y = torch.full_like(t[-1], float("nan"))
+    xq, xc, xs, xcs, wq, wc, ws, wcs, table, _, _, bias, _ = (v.data_ptr() for v in t)
+    _lib.check(_lib.load().arcq_linear_forward_packed(xq, xc, xs, xcs, wq, wc, ws, wcs, table, bias, y.data_ptr(), m, n, k, 4, 64, 16, stream))
+    assert torch.equal(t[-1], y)
+
+
+# A fitted codebook with a level near zero (43 bits between the table's entries) is computed with the fp64 loops whatever the size
+# of the call: 512 rows cost no more than twice what two calls of 256 rows do, which are too small for the matrix units (29 us,
+# 37 both; in the shape of the matrix-unit launch the loops took 100).
+@pytest.mark.parametrize("bits", [4, 3, 2])
+def test_tables_that_do_not_qualify_fill_the_chip(cuda, bits):
+    cb, table = _codebook_with_a_level_near_zero(bits)
+    stream = torch.cuda.current_stream().cuda_stream
+    whole, kept = _call(cuda, 512, 1024, 384, bits, table, cb, cb)
+    halves = [_call(cuda, 256, 1024, 384, bits, table, cb, cb) for _ in range(2)]
+    assert _microseconds([whole], stream) < 2 * _microseconds([h for h, _ in halves], stream)
