@@ -693,6 +693,7 @@ linear_index_mfma_kernel(const IndexArgs p)
     }
     __syncthreads();
     const int low_s = __builtin_amdgcn_readfirstlane(low);                       // 2^low and 2^(-low - 6), in scalar registers
+    if (rw >= p.rows) return;                                                    // (a wave past the last row; there is no barrier below)
     const double unit = __longlong_as_double((1023LL + low_s) << 52), per_unit64 = __longlong_as_double((1017LL - low_s) << 52);
 
     // Bits from..to (of BITS) of code number q, `up` bits to the left.
@@ -856,12 +857,14 @@ template <int BITS>
 void launch_index(const IndexArgs &a, hipStream_t stream)
 {
     const int64_t small_tiles = static_cast<int64_t>((a.rows + 7) / 8) * ((a.out_f + 31) / 32);
-    // The matrix units from 512 wave tiles of 32 x 32 on (two for every compute unit), whatever the number of groups: 788 x 768 -> 768
-    // (600 of them) 46.0 against 54.4 us, 394 x 1536 -> 1536 (624) 83.5 / 106; below, a wave's chain over all groups is what the
-    // launch takes: 394 x 768 -> 768 (312) 45.2 against 34.6 us, 197 x 192 -> 768 (168) 16.1 / 10.1.
+    // The matrix units from 1024 half tiles of 16 x 32 on (two wave tiles of 32 x 32 for every compute unit), whatever the number of
+    // groups: 788 x 768 -> 768 (1200 of them) 45 against 57 us, 394 x 1536 -> 1536 (1200) 83.5 / 106; below, a wave's chain over all
+    // groups is what the launch takes: 394 x 768 -> 768 (600) 45.2 against 34.6 us, 197 x 192 -> 768 (312) 16.1 / 10.1.  Half tiles,
+    // because padding counts: 16 x 384 -> 16416 (513) 24.6 / 24.7, 8 rows 25 / 16, 48 x 384 -> 8225 (774) 29 / 26.5, 24 x 384 -> 16416
+    // (1026) 25 / 35, 64 x 384 -> 8225 (1032) 29.5 / 34.6, 16416 x 384 -> 8 (1026) 24 / 32.6.
     if constexpr (BITS != 0) {
-        const int64_t tiles = static_cast<int64_t>((a.rows + kMfmaTile - 1) / kMfmaTile) * ((a.out_f + kMfmaTile - 1) / kMfmaTile);
-        if (tiles >= 2 * device_cus() && tiles < (int64_t(1) << 24) && static_cast<int64_t>(a.rows > a.out_f ? a.rows : a.out_f) * a.G * 2 * BITS < (int64_t(1) << 31))
+        const int64_t halves = static_cast<int64_t>((a.rows + 15) / 16) * ((a.out_f + kMfmaTile - 1) / kMfmaTile);
+        if (halves >= 4 * device_cus() && halves < (int64_t(1) << 24) && static_cast<int64_t>(a.rows > a.out_f ? a.rows : a.out_f) * a.G * 2 * BITS < (int64_t(1) << 31))
             return launch_index_mfma<BITS>(a, stream);
     }
     // No more workgroups than compute units: up to sixteen waves each, i.e. as few rounds of groups as possible.

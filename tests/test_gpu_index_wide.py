@@ -78,6 +78,28 @@ def test_linear_index_on_the_matrix_units(cuda, oracle, m, n, k, bits, kind):
     assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
 
 
+# Few rows of very many outputs, on both sides of the rule that leaves tiles which are mostly padding to the wide kernel: waves of the
+# matrix-unit launch past the last row leave early.
+@pytest.mark.parametrize("m,n,k", [(1, 16416, 64), (16, 16416, 128), (17, 16416, 64), (33, 16390, 128), (64, 8225, 192)])
+@pytest.mark.parametrize("bits", [4, 2])
+def test_few_rows_of_many_outputs(cuda, m, n, k, bits):
+    cb = synth.quantile_codebook(bits)
+    a, t = _call(cuda, m, n, k, bits, (cb.view(-1, 1) * cb.view(1, -1)).contiguous(), cb, cb)
+    assert torch.equal(*_both_entry_points(cuda, a, t, m, n, k, bits))
+
+
+# 8 x 768 -> 16416 against its two halves of outputs, which are too small for the matrix units: 28 us against 35 to 40, on the matrix
+# units it took 80 to 90.
+@pytest.mark.parametrize("bits", [4, 3])
+def test_few_rows_of_many_outputs_cost_what_their_halves_do(cuda, bits):
+    cb = synth.quantile_codebook(bits)
+    table = (cb.view(-1, 1) * cb.view(1, -1)).contiguous()
+    stream = torch.cuda.current_stream().cuda_stream
+    whole, kept = _call(cuda, 8, 16416, 768, bits, table, cb, cb)
+    halves = [_call(cuda, 8, 8208, 768, bits, table, cb, cb) for _ in range(2)]
+    assert _microseconds([whole], stream) < 1.5 * _microseconds([h for h, _ in halves], stream)
+
+
 def _microseconds(calls, stream):
     """The shortest of ten runs of ``calls``, five times over each."""
     best = float("inf")
@@ -101,6 +123,16 @@ def _call(cuda, m, n, k, bits, table, a_cb, w_cb):
     return _lib.LinearIndexArgs(*[v.data_ptr() for v in t], m, n, k, bits, 64, 1 << bits, 0), t
 
 
+def _both_entry_points(cuda, a, t, m, n, k, bits):
+    """The outputs with the codebooks at hand, and of the entry point that has only the table."""
+    stream = torch.cuda.current_stream().cuda_stream
+    y = torch.full_like(t[-1], float("nan"))
+    xq, xc, xs, xcs, wq, wc, ws, wcs, table, _, _, bias, _ = (v.data_ptr() for v in t)
+    _lib.check(_lib.load().arcq_linear_index(ctypes.byref(a), stream))
+    _lib.check(_lib.load().arcq_linear_forward_packed(xq, xc, xs, xcs, wq, wc, ws, wcs, table, bias, y.data_ptr(), m, n, k, bits, 64, 1 << bits, stream))
+    return t[-1], y
+
+
 def _codebook_with_a_level_near_zero(bits):
     cb = synth.quantile_codebook(bits).clone()
     cb[(1 << bits) // 2] = 0.001234567
@@ -116,12 +148,7 @@ def test_tables_that_do_not_qualify_in_larger_launches(cuda, m, n, k, outer):
     if not outer:
         table[1, 1] = 1.0e-6
     a, t = _call(cuda, m, n, k, 4, table, cb, cb)
-    stream = torch.cuda.current_stream().cuda_stream
-    _lib.check(_lib.load().arcq_linear_index(ctypes.byref(a), stream))
-    y = torch.full_like(t[-1], float("nan"))
-    xq, xc, xs, xcs, wq, wc, ws, wcs, table, _, _, bias, _ = (v.data_ptr() for v in t)
-    _lib.check(_lib.load().arcq_linear_forward_packed(xq, xc, xs, xcs, wq, wc, ws, wcs, table, bias, y.data_ptr(), m, n, k, 4, 64, 16, stream))
-    assert torch.equal(t[-1], y)
+    assert torch.equal(*_both_entry_points(cuda, a, t, m, n, k, 4))
 
 
 # A fitted codebook with a level near zero (43 bits between the table's entries) is computed with the fp64 loops whatever the size
