@@ -330,13 +330,10 @@ ORACLE_API void oracle_linear_forward_u8(
 }
 
 /* ------------------------------------------------------------------------- */
-/* Checker for the GPU stage-1 kernel's divide: t = d/s evaluated as          */
-/*   y = 1/s;  q = d*y;  e = fma(-s,q,d);  q = fma(e,y,q);  (twice)           */
-/* must equal the IEEE quotient d/s for every input its guard admits          */
-/* (2^-60 <= s <= 2^60, |d| <= 8s, and d == 0 or |d| >= 2^-90).  Draws n      */
-/* pseudo-random (d, s) pairs in that range, mantissa extremes included, and  */
-/* returns how many disagree (0 expected).  Not part of the reference; it     */
-/* exists so that the equivalence is tested on the CPU as well as on the GPU. */
+/* Checkers of arithmetic that the GPU kernels use in the place of IEEE        */
+/* operations, restated here.  Not part of the reference: they exist so that   */
+/* each equivalence is tested on the CPU over its whole range, or densely      */
+/* where it is decided.  Every one returns how many cases disagree.            */
 /* ------------------------------------------------------------------------- */
 static inline float u32_as_float(uint32_t b)
 {
@@ -344,39 +341,88 @@ static inline float u32_as_float(uint32_t b)
     memcpy(&f, &b, 4);
     return f;
 }
-
-ORACLE_API float oracle_div_sequence(float d, float s)
+static inline uint32_t float_as_u32(float f)
 {
-    const float y = 1.0f / s;
-    float q = d * y;
-    float e = fmaf(-s, q, d);
-    q = fmaf(e, y, q);
-    e = fmaf(-s, q, d);
-    return fmaf(e, y, q);
+    uint32_t b;
+    memcpy(&b, &f, 4);
+    return b;
+}
+static inline uint64_t next_random(uint64_t *rng)
+{
+    *rng ^= *rng << 13; *rng ^= *rng >> 7; *rng ^= *rng << 17;
+    return *rng;
 }
 
-ORACLE_API int64_t oracle_check_div_sequence(int64_t n, uint64_t seed)
+/* RN(d / s) > T without a division: the sign of s u - d + s e 2^-24 with u = T (the next float above it for T < 0; -0 as 0) and e =
+ * u without its mantissa (arcq_act_quant_core.h, code_offset_of). */
+ORACLE_API int oracle_quotient_above(float d, float s, float threshold)
+{
+    const float u = threshold < 0.0f ? u32_as_float(float_as_u32(threshold) - 1) : threshold + 0.0f;
+    const float e = u32_as_float(float_as_u32(u) & 0xff800000u);
+    return (int)(float_as_u32(fmaf(s * 0x1p-24f, e, fmaf(s, u, -d))) >> 31);
+}
+
+/* Against the division: n draws of T in (-8, 8) (any, +-2^k and its neighbours, 0; |T| >= 2^-60), s in [2^-60, 2^58] (both ends and
+ * the ends of its binades among them) and d, four times out of five within eight floats of s T, else any; d = 0 or |d| >= 2^-90,
+ * |d| <= 8 s: the range that the kernels' guard admits. */
+ORACLE_API int64_t oracle_check_quotient_above(int64_t n, uint64_t seed)
 {
     uint64_t rng = seed ? seed : 88172645463325252ull;
     int64_t bad = 0;
     for (int64_t i = 0; i < n; ++i) {
-        rng ^= rng << 13; rng ^= rng >> 7; rng ^= rng << 17;
-        const uint64_t a = rng;
-        rng ^= rng << 13; rng ^= rng >> 7; rng ^= rng << 17;
-        const uint64_t b = rng;
-        const int es = (int)(a % 121) - 60;
-        uint32_t ms = (uint32_t)(a >> 20) & 0x7fffffu;
-        if ((i & 15) == 0) ms = (i & 16) ? 0x7fffffu : 0u;
-        float s = u32_as_float(((uint32_t)(es + 127) << 23) | ms);
-        if (s > 0x1p60f) s = 0x1p60f;
-        int er = es + 3 - (int)((b >> 8) % 44);
-        if (er < -90) er = -90;
-        uint32_t mr = (uint32_t)(b >> 24) & 0x7fffffu;
-        if ((i & 31) == 1) mr = 0u;
-        float d = u32_as_float(((uint32_t)(b & 1u) << 31) | ((uint32_t)(er + 127) << 23) | mr);
-        if (fabsf(d) > 8.0f * s) d = ((b & 1u) ? -7.9f : 7.9f) * s;
-        const float want = d / s, got = oracle_div_sequence(d, s);
-        if (memcmp(&want, &got, 4) != 0) ++bad;
+        const uint64_t a = next_random(&rng), b = next_random(&rng), c = next_random(&rng);
+        const int wide = (int)((a >> 3) & 1);
+        uint32_t mt = (uint32_t)(a >> 8) & 0x7fffffu;
+        if ((a & 7) >= 6) mt = (uint32_t)((a >> 8) % 5 - 2) & 0x7fffffu;
+        float t = u32_as_float(((uint32_t)(a >> 63) << 31) | ((uint32_t)(127 + 2 - (int)((a >> 32) % (wide ? 63 : 16))) << 23) | mt);
+        if ((a & 7) == 0 && (a & 0x70) == 0) t = (a >> 63) ? -0.0f : 0.0f;
+        if (!(fabsf(t) < 8.0f) || (t != 0.0f && fabsf(t) < 0x1p-60f)) continue;
+        uint32_t ms = (uint32_t)(b >> 8) & 0x7fffffu;
+        if ((b & 7) >= 6) ms = (uint32_t)((b >> 8) % 9 - 4) & 0x7fffffu;
+        float s = u32_as_float(((uint32_t)(127 + ((b >> 3) & 1 ? (int)((b >> 32) % 119) - 60 : (int)((b >> 32) % 12) - 6)) << 23) | ms);
+        if ((b & 0xff0) == 0) s = (b >> 63) ? 0x1p-60f : 0x1p58f;
+        if (s < 0x1p-60f || s > 0x1p58f) continue;
+        float d;
+        if (c % 5) {
+            d = u32_as_float(float_as_u32(s * t) + (uint32_t)((int)((c >> 8) % 17) - 8));
+        } else {
+            d = (float)((double)s * ((double)(c >> 11) * 0x1p-49 - 8.0));
+        }
+        if (!(fabsf(d) <= 8.0f * s)) continue;
+        if (d != 0.0f && fabsf(d) < 0x1p-90f) d = (c >> 40) & 1 ? 0.0f : copysignf(0x1p-90f, d);
+        if (oracle_quotient_above(d, s, t) != (d / s > t)) ++bad;
+    }
+    return bad;
+}
+
+/* v / 3 as a product with RN(1/3) and one fused correction (arcq_act_quant_patches.hip, third_of): every mantissa of one binade. */
+ORACLE_API int64_t oracle_check_third(int exponent)
+{
+    int64_t bad = 0;
+    for (uint32_t m = 0; m < (1u << 23); ++m) {
+        const float v = u32_as_float(((uint32_t)(exponent + 127) << 23) | m);
+        const float q = v * (1.0f / 3.0f);
+        if (fmaf(fmaf(-3.0f, q, v), 1.0f / 3.0f, q) != v / 3.0f) ++bad;
+    }
+    return bad;
+}
+
+/* The square root from an approximate reciprocal root by one coupled iteration and a fused correction (sqrt_and_reciprocal there):
+ * every mantissa of one binade, the reciprocal root `ulps` floats from the one rounded to nearest; and whether the reciprocal that
+ * comes with it is within 2^-22. */
+ORACLE_API int64_t oracle_check_root(int exponent, int ulps)
+{
+    int64_t bad = 0;
+    for (uint32_t m = 0; m < (1u << 23); ++m) {
+        const float a = u32_as_float(((uint32_t)(exponent + 127) << 23) | m);
+        const double exact = 1.0 / sqrt((double)a);
+        const float r = u32_as_float(float_as_u32((float)exact) + (uint32_t)ulps);
+        float g = a * r, h = 0.5f * r;
+        const float e = fmaf(-h, g, 0.5f);
+        g = fmaf(g, e, g);
+        h = fmaf(h, e, h);
+        const float root = fmaf(fmaf(-g, g, a), h, g);
+        if (root != sqrtf(a) || fabs((double)(h + h) / exact - 1.0) > 0x1p-22) ++bad;
     }
     return bad;
 }

@@ -52,11 +52,26 @@ def _c():
     return _lib
 
 
-def check_div_sequence(n: int, seed: int = 1) -> int:
-    """Mismatches between the GPU kernel's fma-based divide and IEEE division on ``n`` random inputs."""
+def check_quotient_above(n: int, seed: int = 1) -> int:
+    """Cases of ``n`` random ones in which the GPU kernels' test for RN(d / s) > T disagrees with the division."""
     lib = _c()
-    lib.oracle_check_div_sequence.restype = ctypes.c_int64
-    return int(lib.oracle_check_div_sequence(ctypes.c_int64(n), ctypes.c_uint64(seed)))
+    lib.oracle_check_quotient_above.restype = ctypes.c_int64
+    return int(lib.oracle_check_quotient_above(ctypes.c_int64(n), ctypes.c_uint64(seed)))
+
+
+def check_third(exponent: int) -> int:
+    """Mantissas of the binade 2^exponent for which the patch quantizer's v / 3 is not IEEE's."""
+    lib = _c()
+    lib.oracle_check_third.restype = ctypes.c_int64
+    return int(lib.oracle_check_third(ctypes.c_int(exponent)))
+
+
+def check_root(exponent: int, ulps: int) -> int:
+    """Mantissas of the binade 2^exponent for which the patch quantizer's square root is not IEEE's, or its reciprocal not
+    within 2^-22, when it starts ``ulps`` floats from the correctly rounded reciprocal root."""
+    lib = _c()
+    lib.oracle_check_root.restype = ctypes.c_int64
+    return int(lib.oracle_check_root(ctypes.c_int(exponent), ctypes.c_int(ulps)))
 
 
 def _p(a: Optional[np.ndarray]):

@@ -323,11 +323,32 @@ def test_linear_f64_and_error_scale(oracle):
     assert np.allclose(y2, ref - b, rtol=1e-13, atol=1e-13)
 
 
-def test_fma_division_sequence_is_ieee_division(oracle):
-    """The stage-1 kernel computes t = d/s as d*RN(1/s) plus two fused residual corrections; within its
-    guard range that is the correctly rounded quotient.  20 million random pairs incl. mantissa extremes."""
+def test_code_remainder_decides_like_the_division(oracle):
+    """The stage-1 kernels decide RN(d / s) > T by the sign of s u - d + s e 2^-24, without the quotient.  20 million random cases
+    of the range that their guard admits, most of them within eight floats of s T."""
     for seed in (1, 2, 3, 4):
-        assert oracle.check_div_sequence(5_000_000, seed) == 0
+        assert oracle.check_quotient_above(5_000_000, seed) == 0
+
+
+def test_third_is_ieee_division_by_three(oracle):
+    """The patch quantizer's means: every mantissa, at the ends of the range that it admits and in the middle."""
+    assert [oracle.check_third(e) for e in (-100, -60, 0, 1, 60)] == [0] * 5
+
+
+def test_root_from_a_reciprocal_root_is_ieee_square_root(oracle):
+    """The patch quantizer's root for every mantissa of an even and an odd binade and at the ends of its range, from any reciprocal
+    root within one unit in the last place (what the hardware's instruction gives); from a coarse one the check fails."""
+    assert [oracle.check_root(e, u) for e in (0, 1) for u in (-1, 0, 1)] == [0] * 6
+    assert [oracle.check_root(e, 1) for e in (-100, 99)] == [0] * 2
+    assert oracle.check_root(0, 4096) > 0
+
+
+def test_layernorm_pieces_by_a_product(oracle):
+    """The LayerNorm form of stage 1 finds a piece's column as p * ceil(2^20 / RW) >> 20: equal to p / RW for the 1024 pieces and
+    256 rows that a tile can have."""
+    p = np.arange(1024, dtype=np.uint32)
+    for rw in range(1, 257):
+        assert np.array_equal((p * np.uint32(((1 << 20) + rw - 1) // rw)) >> np.uint32(20), p // np.uint32(rw)), rw
 
 
 def test_layernorm_restatement_is_layernorm(oracle):
