@@ -218,7 +218,10 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
             }
         const int parts = SPLIT ? gridDim.z : 1;
         if (SPLIT && 4 * ((NKB + parts - 1) / parts) <= NKB) {
-            // Few waves have a tile, but all of them quantize: eight lanes a row (FP8: four), one 16-byte piece a lane.
+            // Few waves have a tile, but all of them quantize: eight lanes a row (FP8: four), one 16-byte piece a lane.  With one
+            // tile to four or more waves that beats two lanes a row on the waves that have one at every size measured (4 to 8 waves,
+            // one tile: 0.86 .. 0.95 of its time; 8 waves, two tiles: 0.88); with fewer it does not (2 and 3 waves: 1.05 .. 1.09;
+            // two tiles to 3 .. 7 waves: 1.00 .. 1.24; three or four tiles: 0.97 .. 1.15), but for FP8 with two tiles to 7 waves (0.93).
             constexpr int V = F8 ? 16 : 8, LANES = 64 / V, ROWS = 64 / LANES;
             __syncthreads();
             const int part = blockIdx.z, tiles = (NKB - part + parts - 1) / parts;

@@ -162,7 +162,9 @@ otf_rows_kernel(const RowsParams p)
     // finished under stage 1's set-up ----
     // Division of the extra work over the waves (stage 1 is instruction-bound and waves w, w + 4, w + 8 share a SIMD):
     // wave 1 builds the activation lookup tables, wave 0 and waves 4.. reconstruct the weight pieces as threads 0..63,
-    // 64.. -- so that no SIMD carries more than two of them (two piece waves on SIMD 0).
+    // 64.. -- so that no SIMD carries more than two of them (two piece waves on SIMD 0).  Waves 2 and 3 get none: with them
+    // 12 608 x 384 -> 1 152 takes 27.0 us against 27.0, 12 608 x 768 -> 2 304 70.6 / 70.8, 12 608 x 3 072 -> 768 108.0 / 107.9
+    // (the next piece's inputs requested ahead of the last one's arithmetic as well: 26.9, 70.7, 105.9).
     constexpr int kPieceThreads = W < 4 ? 64 * W : 64 * (W - 3);
     const int ptid = W < 4 ? tid : (wave == 0 ? lane : (wave >= 4 ? (wave - 3) * 64 + lane : -1));
     int64_t share_lo = 0, share_hi = 0;

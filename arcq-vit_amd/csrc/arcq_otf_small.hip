@@ -246,9 +246,9 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
             }
         }
     };
-    // Wave w owns the tiles w, w + 8, ... of the row tile.  With fewer than eight tiles the waves without one build
-    // the lookup tables while the others take their statistics, and one barrier joins the two halves; otherwise all
-    // eight waves build the tables between the two halves of their first tile.
+    // Wave w owns the tiles w, w + 8, ... of the row tile.  One wave builds the lookup tables: with fewer than eight tiles the
+    // first without one, while the others take their statistics, otherwise wave 0 ahead of its first tile's.  One barrier joins
+    // statistics and tables.
     const int n_tiles = (groups + gpt - 1) / gpt;
     const bool spare_waves = n_tiles < kOsWaves;
     const int tile_waves = spare_waves ? n_tiles : kOsWaves;
@@ -268,8 +268,8 @@ otf_small_kernel(const TIN *__restrict__ x, const float *__restrict__ a_thr, con
     const bool table_ok = tables.usable != 0;
     const bool write_ws = (x_hat_ws != nullptr) && blockIdx.x == 0;
     // Quantize-the-output mode (nx_thr != nullptr: y receives stage 1 of the layer that consumes this one's output):
-    // that layer's lookup tables are built by the waves without a stage-1 tile while the others run theirs, or, when
-    // every wave has a tile, by all of them behind it.
+    // that layer's lookup tables are built by the first wave without a stage-1 tile while the others run theirs, or, when
+    // every wave has a tile, by wave 0 behind its last one.
     QuantTables &n_tables = *reinterpret_cast<QuantTables *>(smem + nx_off);
     if (nx_thr && spare_waves && wave == tile_waves) build_quant_tables<BITS>(load_quant_params<BITS>(nx_thr, nx_cb, lane), n_tables, lane);
     for (int t = wave; t < n_tiles; t += kOsWaves) {
