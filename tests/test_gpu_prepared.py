@@ -124,7 +124,10 @@ def test_linear_prepared_quantizes_for_the_next_layer(cuda, oracle, m, n, k, bit
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), gelu
 
 
-@pytest.mark.parametrize("b,n,h,bits", [(1, 197, 6, 4), (3, 197, 12, 3), (2, 33, 3, 2), (5, 1, 1, 4), (7, 101, 2, 4), (2, 256, 16, 3)])
+# (from the seventh: parts of a head with several query tiles, whose idle waves leave early, or, at (4, 256, 15) and (3, 225, 13) with
+# two tiles in a part, quantize with the others)
+@pytest.mark.parametrize("b,n,h,bits", [(1, 197, 6, 4), (3, 197, 12, 3), (2, 33, 3, 2), (5, 1, 1, 4), (7, 101, 2, 4), (2, 256, 16, 3),
+                                        (16, 197, 6, 4), (11, 197, 11, 3), (2, 197, 24, 4), (5, 129, 16, 2), (4, 256, 15, 4), (3, 225, 13, 3)])
 def test_attention_quantizes_for_the_proj_layer(cuda, oracle, b, n, h, bits):
     cb, thr, _, _ = _layer(oracle, cuda, 32, 64, bits, 29)
     qkv = synth.make_activation(b * n, 3 * h * 64, 31).to(cuda, torch.float16).reshape(b, n, 3 * h * 64).contiguous()

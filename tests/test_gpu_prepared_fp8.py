@@ -95,7 +95,10 @@ def test_linear_prepared_fp8(cuda, oracle, m, n, k, bits):
                 assert torch.equal(_linear(x8, w8, bias, m, n, k, mult, row_major, gelu=gelu, nq=(thr, cb), bits=bits), want), (row_major, gelu)
 
 
-@pytest.mark.parametrize("b,n,h,bits", [(1, 197, 6, 4), (2, 33, 3, 2), (7, 101, 5, 3)])
+# (from the fourth: parts of a head with several query tiles, with odd and even numbers of heads; two tiles in a part and all waves
+# quantizing from the seventh)
+@pytest.mark.parametrize("b,n,h,bits", [(1, 197, 6, 4), (2, 33, 3, 2), (7, 101, 5, 3), (16, 197, 6, 4), (11, 197, 11, 3), (5, 129, 16, 2),
+                                        (4, 256, 15, 4), (3, 225, 13, 3), (3, 225, 14, 4)])
 def test_attention_quant_fp8(cuda, oracle, b, n, h, bits):
     cb, thr, _, _ = _layer(oracle, cuda, 32, 64, bits, 29)
     qkv = synth.make_activation(b * n, 3 * h * 64, 31).to(cuda, torch.float16).reshape(b, n, 3 * h * 64).contiguous()
