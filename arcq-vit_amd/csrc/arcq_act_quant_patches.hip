@@ -37,7 +37,9 @@ __device__ __forceinline__ float third_of(float v)
     return __fmaf_rn(__fmaf_rn(-3.0f, q, v), 1.0f / 3.0f, q);
 }
 // The square root rounded to nearest, from the hardware's reciprocal root by one coupled iteration (Goldschmidt) and a fused
-// correction: equal to sqrtf for every float of [2^-100, 2^100), at a third of its instructions.  y: the reciprocal, within 2^-22.
+// correction: equal to sqrtf for every float of [2^-100, 2^100) from any reciprocal root within one unit in the last place, which is the
+// instruction's accuracy (every mantissa of an even and an odd binade checked on the CPU), at a third of sqrtf's instructions.  y: the
+// reciprocal, within 2^-22.
 __device__ __forceinline__ float sqrt_and_reciprocal(float a, float &y)
 {
     const float r = __builtin_amdgcn_rsqf(a);
@@ -51,8 +53,8 @@ __device__ __forceinline__ float sqrt_and_reciprocal(float a, float &y)
 __device__ __forceinline__ bool in_range(float v) { return (v == 0.0f) | ((fabsf(v) >= 0x1p-60f) & (fabsf(v) <= 0x1p60f)); }
 
 // The fast form looks every value up before it is known to be in range (what it finds otherwise is not used): the payload of an
-// fp32 NaN may name any of the offsets that code_offset_of can form (that of an fp16 one, widened, has no bits there), and a table
-// with two thresholds in one bucket one code more than there are.  Both tables have an entry for it.
+// fp32 NaN may name any of the offsets that code_offset_of can form (that of an fp16 one, widened, has no bits there): its table has
+// all those entries.  And the sign of a NaN remainder may make one code more than there are, which reads the member behind `cb`.
 template <typename TIN> constexpr int kTableEntries = sizeof(TIN) == 4 ? 0x1ff8 / static_cast<int>(sizeof(Bucket)) + 1 : kMaxBuckets + 1;
 
 // Eight pixels quantized and reconstructed in place, every operation rounded as IEEE has it.

@@ -300,7 +300,7 @@ gemm_fp8_kernel(const uint8_t *__restrict__ xb, const float *__restrict__ bias, 
                 __builtin_amdgcn_wave_barrier();
                 if constexpr (NQ != 0) {          // the chunk is one group of the consumer's rows
                     // (while the next pass's fragments are in flight two row blocks leave no room for a group in one lane:
-                    // 50 432 x 1 024 -> 4 096 then takes 633 us instead of 581)
+                    // 6 304 x 768 -> 3 072 with GELU then takes 50.7 us instead of 45.5, 50 432 x 1 024 -> 4 096 447 instead of 406)
                     if constexpr (kChunks == 2 && decltype(lane_per_group)::value) {
                         take_staged_group(staged, stage, kStageRow, lane, ch);
                         if (ch == 1) next_quant_groups<NQ, true>(nq_lds, staged, lane, gelu != 0, 1.0e-6f, y, pblk, M, N, n_base);

@@ -10,7 +10,6 @@
 #include "arcq_gemm.h"
 
 #include <type_traits>
-#include <cstdlib>
 
 namespace arcq {
 

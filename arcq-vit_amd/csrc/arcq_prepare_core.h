@@ -126,7 +126,6 @@ template <int BITS, bool F8>
 __device__ __forceinline__ void prep_weights_rows(const PrepWeights &w, unsigned block, float *lut)
 {
     constexpr int L = 1 << BITS;
-    const int lane = threadIdx.x & 63;
     constexpr uint32_t kPieces = F8 ? 4 : 8;       // of a group
     const uint32_t live = static_cast<uint32_t>(w.G) * kPieces;
     const uint32_t per_row = F8 ? (live + 7) / 8 * 8 : live;
