@@ -829,8 +829,12 @@ inline int index_waves(int G)
 template <int BITS>
 void launch_index_mfma(const IndexArgs &a, hipStream_t stream)
 {
-    const int across = (a.out_f + kMfmaTile - 1) / kMfmaTile, S = index_waves(a.G), resident = 4 * kIdxMinWaves / S * device_cus();
-    const int own = across * ((a.rows + S * kMfmaTile - 1) / (S * kMfmaTile)), grid = max(own, min(resident, across * ((a.rows + 15) / 16)));
+    const int across = (a.out_f + kMfmaTile - 1) / kMfmaTile;
+    auto workgroups = [&](int waves) { return across * ((a.rows + waves * kMfmaTile - 1) / (waves * kMfmaTile)); };
+    auto busiest_simd = [&](int waves) { return ((workgroups(waves) + device_cus() - 1) / device_cus() * waves + 3) / 4; };
+    int S = index_waves(a.G);
+    if (busiest_simd(S) > busiest_simd(kIdxMaxWaves)) S = kIdxMaxWaves;
+    const int resident = 4 * kIdxMinWaves / S * device_cus(), own = workgroups(S), grid = max(own, min(resident, across * ((a.rows + 15) / 16)));
     IndexArgs b = a;
     b.workers = own <= resident || own >= 3 * resident ? grid : S == kIdxMaxWaves ? resident : resident - resident / 16;
     hipLaunchKernelGGL((linear_index_mfma_kernel<BITS>), dim3(grid), dim3(64 * S), S * kIdxRegion, stream, b);

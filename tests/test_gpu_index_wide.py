@@ -141,7 +141,8 @@ def _codebook_with_a_level_near_zero(bits):
 
 # Such a table runs on the loops, with as many workgroups as are resident at once or, of larger launches, with all (256 compute
 # units; three and four waves): the same bits as the entry point without codebooks gives.
-@pytest.mark.parametrize("m,n,k", [(1000, 550, 192), (4100, 775, 192), (4100, 2400, 192), (4100, 775, 256), (4100, 2331, 256)])
+@pytest.mark.parametrize("m,n,k", [(1000, 550, 192), (4100, 775, 192), (4100, 2400, 192), (4100, 775, 256), (4100, 2331, 256),
+                                   (5721, 330, 192)])
 @pytest.mark.parametrize("outer", [True, False])
 def test_tables_that_do_not_qualify_in_larger_launches(cuda, m, n, k, outer):
     cb, table = _codebook_with_a_level_near_zero(4)
@@ -149,6 +150,17 @@ def test_tables_that_do_not_qualify_in_larger_launches(cuda, m, n, k, outer):
         table[1, 1] = 1.0e-6
     a, t = _call(cuda, m, n, k, 4, table, cb, cb)
     assert torch.equal(*_both_entry_points(cuda, a, t, m, n, k, 4))
+
+
+# 21 groups would be three waves' work in the loops of other tables; on the matrix units three-wave workgroups put more waves on the
+# busiest SIMD than four-wave ones here (81 us against 63), and the time is to be 21 / 20 of that of 20 groups.
+@pytest.mark.parametrize("bits", [4, 2])
+def test_number_of_groups_does_not_unbalance_the_matrix_units(cuda, bits):
+    cb = synth.quantile_codebook(bits)
+    table = (cb.view(-1, 1) * cb.view(1, -1)).contiguous()
+    stream = torch.cuda.current_stream().cuda_stream
+    (a, kept), (b, also_kept) = (_call(cuda, 5721, 352, 64 * g, bits, table, cb, cb) for g in (21, 20))
+    assert _microseconds([a], stream) < 1.15 * _microseconds([b], stream)
 
 
 # A fitted codebook with a level near zero (43 bits between the table's entries) is computed with the fp64 loops whatever the size
