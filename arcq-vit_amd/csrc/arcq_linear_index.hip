@@ -311,7 +311,9 @@ struct IndexArgs {
     const float *wc, *ws, *wcs, *table, *a_cb, *w_cb, *bias;
     float *y;
     int rows, out_f, G, levels;
-    int workers;                     // linear_index_mfma_kernel: the workgroups that share the tiles where the table does not qualify
+    // linear_index_mfma_kernel, where the table does not qualify: the workgroups that share the tiles, and how many behind them take
+    // one of the last tiles each
+    int workers, singles;
 };
 
 // The product table and the codebooks in LDS.
@@ -667,8 +669,9 @@ linear_index_mfma_kernel(const IndexArgs p)
     for (int w = 0; w < S; ++w) lo = min(lo, s_low[w]), hi = max(hi, s_high[w]);
     const int low = lo <= hi ? lo : 0;                                           // (else all entries are zero)
     if (hi - low > kMaxEntryBits) {                                              // workgroup-uniform
-        const int tiles = across * ((p.rows + 15) / 16);
-        for (int t = blockIdx.x; t < tiles && static_cast<int>(blockIdx.x) < p.workers; t += p.workers)
+        const int tiles = across * ((p.rows + 15) / 16), wg = blockIdx.x, shared = tiles - p.singles;
+        const int first = wg < p.workers ? wg : shared + wg - p.workers, end = wg < p.workers ? shared : min(first + 1, tiles);
+        for (int t = first; t < end; t += p.workers)
             index_wide_tile<BITS, 2, 4, kIdxMinWaves, false>(p, t / across * 16, t % across * 32, tables, same);
         return;
     }
@@ -817,15 +820,21 @@ inline int index_waves(int G)
     return S;
 }
 
-// The host does not see the table, so the launch serves both cases.  Waves per workgroup as above: the matrix-unit tiles are a
-// wave's own and do not mind (1576 x 384 -> 1536 51.0 us with three, 51.7 with four).  Where their workgroups would leave compute
-// units idle, more are launched for the 16-row tiles of the loops, as many as are resident at once; a table that qualifies sends
-// them home after the look at it (512 x 384 -> 1024 26 us with and without them).  From one resident set on the tiles are dealt to
-// as many workgroups as are resident (of three-wave ones not quite four fit a compute unit), from three on to all of them, and the
-// dispatch evens out the last round.  Tables that do not qualify, against the wide kernel alone: 512 x 384 -> 1024 29 / 28 us with
-// computed and 48 / 48 with gathered entries, 1576 x 384 -> 1536 111 / 103 and 208 / 216, 12608 x 384 -> 1536 763 / 725 and
-// 1570 / 1562, 12608 x 1536 -> 384 755 / 690 and 1479 / 1562; at worst, where two rounds are not full, 5000 x 576 -> 768 275 / 228.
-// (Eight tiles in turn per 128-row workgroup: 100, 164, 936 and 811 us with computed entries.)
+// The host does not see the table, so the launch serves both cases.  Waves per workgroup as above (1576 x 384 -> 1536 51.0 us with
+// three, 51.7 with four: the matrix-unit tiles are a wave's own), but four where three would put more wave tiles on the busiest SIMD
+// (workgroups are dealt whole: 5721 x 1344 -> 352 at 2 bits 81 us with three, 66 with four; 9303 x 1088 -> 224 94 and 78).
+//
+// Tables that do not qualify: where the workgroups above would leave compute units idle, more are launched for the 16-row tiles of the
+// loops, as many as are resident at once; a table that qualifies sends them home after the look at it (512 x 384 -> 1024 24.5 us with
+// and without them).  Four waves: from one resident set on that set shares the tiles and every workgroup behind it takes one of the
+// last ones, which evens out the end; from four tiles for each on there are a third more for that (2343 x 448 -> 960 124 -> 113 us,
+// 3192 x 1408 -> 736 358 -> 324; 6170 x 1472 -> 1408, dealt to all 2156 workgroups alike, 1326 -> 1210).  Three waves, of which not
+// quite four workgroups fit a compute unit: the tiles are dealt to fifteen sixteenths of a resident set, from three sets on to all
+// (12608 x 384 -> 1536: to all 761 us, the four waves' rule 894; 5000 x 576 -> 768 273 and 285).
+// Against the wide kernel alone, at 44 sizes of 512 .. 12608 rows and 2 .. 24 groups: with computed entries 0.97 of its speed in the
+// mean (512 x 384 -> 1024 27.4 / 26.8 us, 1576 x 384 -> 1536 111 / 105, 12608 x 384 -> 1536 758 / 710; at worst, where two rounds are
+// not full, 5000 x 576 -> 768 273 / 218), with gathered ones 1.00 (at worst, nine groups on four waves, 10800 x 576 -> 1056
+// 1620 / 1350).  (Eight tiles in turn per 128-row workgroup: 512 rows 100 us, 1576 164, 12608 936.)
 template <int BITS>
 void launch_index_mfma(const IndexArgs &a, hipStream_t stream)
 {
@@ -834,9 +843,11 @@ void launch_index_mfma(const IndexArgs &a, hipStream_t stream)
     auto busiest_simd = [&](int waves) { return ((workgroups(waves) + device_cus() - 1) / device_cus() * waves + 3) / 4; };
     int S = index_waves(a.G);
     if (busiest_simd(S) > busiest_simd(kIdxMaxWaves)) S = kIdxMaxWaves;
-    const int resident = 4 * kIdxMinWaves / S * device_cus(), own = workgroups(S), grid = max(own, min(resident, across * ((a.rows + 15) / 16)));
+    const int resident = 4 * kIdxMinWaves / S * device_cus(), tiles = across * ((a.rows + 15) / 16), own = workgroups(S);
+    const int grid = max(own, min(tiles, S == kIdxMaxWaves && tiles >= 4 * resident ? resident + resident / 3 : resident));
     IndexArgs b = a;
-    b.workers = own <= resident || own >= 3 * resident ? grid : S == kIdxMaxWaves ? resident : resident - resident / 16;
+    b.workers = S == kIdxMaxWaves ? min(grid, resident) : own <= resident || own >= 3 * resident ? grid : resident - resident / 16;
+    b.singles = S == kIdxMaxWaves ? grid - b.workers : 0;
     hipLaunchKernelGGL((linear_index_mfma_kernel<BITS>), dim3(grid), dim3(64 * S), S * kIdxRegion, stream, b);
 }
 
@@ -1002,7 +1013,7 @@ ARCQ_API int arcq_linear_index(const arcq_linear_index_args *a, void *stream)
     }
     const IndexArgs g{a->x_codes, a->x_center, a->x_scale, a->x_code_sum, a->w_codes, a->w_center, a->w_scale, a->w_code_sum, a->product_table,
                       a->a_codebook, a->w_codebook, a->bias, a->y, static_cast<int>(a->rows), static_cast<int>(a->out_features),
-                      static_cast<int>(a->in_features / 64), a->levels, 0};
+                      static_cast<int>(a->in_features / 64), a->levels, 0, 0};
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (a->bits == 4) launch_index<4>(g, st);
     else if (a->bits == 3) launch_index<3>(g, st);

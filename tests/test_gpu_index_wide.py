@@ -139,8 +139,9 @@ def _codebook_with_a_level_near_zero(bits):
     return cb, (cb.view(-1, 1) * cb.view(1, -1)).contiguous()
 
 
-# Such a table runs on the loops, with as many workgroups as are resident at once or, of larger launches, with all (256 compute
-# units; three and four waves): the same bits as the entry point without codebooks gives.
+# Such a table runs on the loops, dealt to the workgroups that are resident at once and, of four waves, to those behind them a tile
+# each (256 compute units; three and four waves; (5721, 330, 192) has four because of the matrix units): the same bits as the entry
+# point without codebooks gives.
 @pytest.mark.parametrize("m,n,k", [(1000, 550, 192), (4100, 775, 192), (4100, 2400, 192), (4100, 775, 256), (4100, 2331, 256),
                                    (5721, 330, 192)])
 @pytest.mark.parametrize("outer", [True, False])
