@@ -63,7 +63,7 @@ __device__ __forceinline__ void quantize_pixels(float (&x)[8][kC], float eps, co
 {
     constexpr float fgs = static_cast<float>(kC);
     float mu[8], s[8];
-    uint32_t code[8][kC];
+    uint32_t at[8][kC];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         float sum = 0.0f, var = 0.0f;
@@ -77,22 +77,16 @@ __device__ __forceinline__ void quantize_pixels(float (&x)[8][kC], float eps, co
         }
         s[e] = sqrtf(var / fgs + eps);
 #pragma unroll
-        for (int c = 0; c < kC; ++c) x[e][c] = x[e][c] / s[e], code[e][c] = 0;
+        for (int c = 0; c < kC; ++c) x[e][c] = x[e][c] / s[e];
     }
-#pragma unroll 1
-    for (uint32_t i = 0; i + 1 < (1u << BITS); ++i) {      // while (code < L - 1 && t > thr[code]) ++code
-        const float thr = q.thr[i];
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-#pragma unroll
-            for (int c = 0; c < kC; ++c) code[e][c] += (code[e][c] == i && x[e][c] > thr) ? 1u : 0u;
-    }
+    for (int e = 0; e < 8; ++e) bisect_codes<BITS>(x[e], q.thr, at[e]);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         float sum_codes = 0.0f;
 #pragma unroll
         for (int c = 0; c < kC; ++c) {
-            x[e][c] = q.cb[code[e][c]];
+            x[e][c] = code_value(q.cb, at[e][c]);
             sum_codes += x[e][c];
         }
         const float code_mean = sum_codes / fgs;

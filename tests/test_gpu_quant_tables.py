@@ -92,3 +92,52 @@ def test_stage_1_alone(cuda, oracle, m, k, bits, dtype):
         got = _prepare(x.to(cuda), t.contiguous().to(cuda), cb.to(cuda), bits)[0].cpu().numpy()
         nan = np.isnan(want)
         assert np.array_equal(np.isnan(got), nan) and np.array_equal(got.view(np.uint16)[~nan], want.view(np.uint16)[~nan])
+
+
+# thresholds in any order with NaN and infinities among them: the search stops at the first one that is not below the value
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_codes_of_thresholds_in_any_order(cuda, oracle, bits, dtype):
+    rng = np.random.default_rng(bits)
+    cb = synth.quantile_codebook(bits)
+    x = synth.make_activation(301, 192, 41).to(dtype)
+    x[7], x[8, :3] = 0.0, torch.tensor([float("nan"), INF, -INF], dtype=dtype)
+    for case in range(24):
+        thr = np.sort(rng.normal(size=(1 << bits) - 1)).astype(np.float32)
+        if case % 3:
+            thr = rng.permutation(thr)
+        if case % 2:
+            thr[rng.integers(thr.size)] = rng.choice(np.float32([np.nan, np.inf, -np.inf, -0.0, 1e-42]))
+        thr[rng.integers(thr.size)] = thr[0]
+        t = torch.from_numpy(thr)
+        with np.errstate(all="ignore"):
+            want = oracle.act_quant_c(x.float().numpy(), t, cb, bits, 64)
+        packed, _, center, _, total = ops._act_quant(x.to(cuda), t.to(cuda), cb.to(cuda), bits, 64, want_packed=True, want_meta=True, strict_f32=False)
+        codes = ops._act_quant(x.to(cuda), t.to(cuda), cb.to(cuda), bits, 64, want_u8=True, strict_f32=False)[1]
+        assert np.array_equal(packed.cpu().numpy(), want["packed"]), (case, thr)
+        assert np.array_equal(codes.cpu().numpy(), want["codes"]), (case, thr)
+        assert np.array_equal(total.cpu().numpy(), want["code_sum"]) and np.array_equal(center.cpu().numpy(), want["center"], equal_nan=True)
+
+
+# A fitted codebook may repeat a level.  That takes 1.4 times as long as one whose thresholds the buckets hold (every threshold in turn:
+# 3 times).
+def test_repeated_thresholds_cost_little(cuda):
+    cb = synth.quantile_codebook(4)
+    thr = synth.midpoint_thresholds(cb)
+    x, cb = torch.randn(50432, 1024, device=cuda), cb.to(cuda)
+
+    def microseconds(t):
+        best = INF
+        for _ in range(8):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(5):
+                ops.quantize_activation(x, t, cb, 4, 64)
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, begin.elapsed_time(end) * 200.0)
+        return best
+
+    repeated = thr.clone()
+    repeated[1] = repeated[0]
+    assert microseconds(repeated.to(cuda)) < 2 * microseconds(thr.to(cuda))
