@@ -118,40 +118,45 @@ __device__ __forceinline__ void write_row(uint32_t *__restrict__ row, const floa
     }
 }
 
-// Appends the 64 codes (one per array slot) to packed dwords, LSB first.
+// The 64 codes, a byte each, as packed dwords, LSB first.
 template <int BITS>
-__device__ __forceinline__ void pack64(const uint32_t (&c)[64], uint32_t (&w)[2 * BITS])
+__device__ __forceinline__ void pack64(const uint32_t (&c)[16], uint32_t (&w)[2 * BITS])
 {
+    uint32_t four[16];      // 4 BITS bits each
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        constexpr uint32_t mask = (1u << BITS) - 1;
+        four[k] = c[k] & mask;
+#pragma unroll
+        for (int q = 1; q < 4; ++q) four[k] |= (c[k] >> (q * (8 - BITS))) & (mask << (q * BITS));
+    }
     if constexpr (BITS == 4 || BITS == 2) {
-        constexpr int per = 32 / BITS;
+        constexpr int per = 8 / BITS;
 #pragma unroll
         for (int d = 0; d < 2 * BITS; ++d) {
-            uint32_t v = 0;
+            uint32_t v = four[d * per];
 #pragma unroll
-            for (int q = 0; q < per; ++q) v |= c[d * per + q] << (BITS * q);
+            for (int q = 1; q < per; ++q) v |= four[d * per + q] << (4 * BITS * q);
             w[d] = v;
         }
     } else {
-        uint32_t ch[8];   // 8 codes -> one 24-bit chunk; 4 chunks -> 3 dwords
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            uint32_t v = 0;
+        for (int h = 0; h < 2; ++h) {      // 8 codes -> one 24-bit chunk; 4 chunks -> 3 dwords
+            uint32_t ch[4];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) v |= c[k * 8 + q] << (3 * q);
-            ch[k] = v;
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            w[3 * h + 0] = ch[4 * h + 0] | (ch[4 * h + 1] << 24);
-            w[3 * h + 1] = (ch[4 * h + 1] >> 8) | (ch[4 * h + 2] << 16);
-            w[3 * h + 2] = (ch[4 * h + 2] >> 16) | (ch[4 * h + 3] << 8);
+            for (int k = 0; k < 4; ++k) ch[k] = four[8 * h + 2 * k] | four[8 * h + 2 * k + 1] << 12;
+            w[3 * h + 0] = ch[0] | (ch[1] << 24);
+            w[3 * h + 1] = (ch[1] >> 8) | (ch[2] << 16);
+            w[3 * h + 2] = (ch[2] >> 16) | (ch[3] << 8);
         }
     }
 }
 
-// CODES = false drops everything only the code outputs need (the on-the-fly layer asks for x_hat alone).
+// CODES = false drops everything only the code outputs need (the on-the-fly layer asks for x_hat alone).  The codes of a group stay a
+// byte each in sixteen registers, so that two waves share a SIMD in every form (a register for each code: 300 of them and one wave;
+// packed codes and x_hat of 12 608 x 1 536 fp32 42.6 us, 49.5 with all lookups in flight, 30.6 now).
 template <typename TIN, typename TOUT, int BITS, bool CODES>
-__global__ void __launch_bounds__(64 * kWaves, CODES ? 1 : 2)
+__global__ void __launch_bounds__(64 * kWaves, 2)
 act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, const float *__restrict__ cb,
                      uint8_t *__restrict__ packed, uint8_t *__restrict__ codes_u8,
                      float *__restrict__ center, float *__restrict__ scale, float *__restrict__ code_sum,
@@ -201,7 +206,7 @@ act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
         fetch_tile<TIN>(x, (group0 + tile_step * kTileGroups) * 64, elem_end, regs, lane);
 
         float mu, var, s, sum_codes;
-        uint32_t code[CODES ? 64 : 1];
+        uint32_t code[CODES ? 16 : 1];
         group_stats64(xv, eps, mu, var, s);
         // (eight lookups in flight: with all 64 the compiler delays the sums, x_hat of 12 608 x 1 536 fp32 32.9 us against 28.3)
         group_codes64<BITS, CODES, 8>(xv, mu, var, s, tables, bq, table_ok, sum_codes, code);
@@ -230,15 +235,7 @@ act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
                 if (codes_u8) {
                     uint4 *dst = reinterpret_cast<uint4 *>(codes_u8 + g * 64);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        uint32_t d[4];
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            const int b = q * 16 + k * 4;
-                            d[k] = code[b] | (code[b + 1] << 8) | (code[b + 2] << 16) | (code[b + 3] << 24);
-                        }
-                        dst[q] = make_uint4(d[0], d[1], d[2], d[3]);
-                    }
+                    for (int q = 0; q < 4; ++q) dst[q] = make_uint4(code[4 * q], code[4 * q + 1], code[4 * q + 2], code[4 * q + 3]);
                 }
             }
         }
@@ -261,7 +258,7 @@ act_quant_g64_kernel(const TIN *__restrict__ x, const float *__restrict__ thr, c
 // contiguous in the row-major tensor; two lanes share a group (arcq_act_quant_core.h), the inputs are loaded coalesced and
 // change places in a wave-private LDS tile, and lane l's 32 codes lie at l times their size behind the tile's first: every
 // store of the wave is one contiguous run.  The waves walk their tiles with the next one's loads in flight.  (A lane per group,
-// act_quant_g64_kernel: 297 registers, one or two waves per SIMD; 12 608 x 1 536 fp32 at four bits 31.7 us against 19.1; 18.4 at the copy rate.)
+// act_quant_g64_kernel, when it took 297 registers: 12 608 x 1 536 fp32 at four bits 31.7 us against 19.1; 18.4 at the copy rate.)
 // BUILDER as in prepare_kernel: a fifth wave builds the lookup tables of a workgroup whose waves have one tile each.
 template <typename TIN, int BITS, bool BYTES, bool BUILDER>
 __global__ void __launch_bounds__(64 * (kWaves + (BUILDER ? 1 : 0)))

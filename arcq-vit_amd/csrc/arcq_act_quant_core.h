@@ -255,14 +255,15 @@ __device__ __forceinline__ void search_codes(float (&xv)[N], float s, const Quan
 
 // Second half: xv holds the residuals on entry and cb[code_j] on exit.  The whole wave must call it (the fast/slow
 // decision is wave-uniform).  `bq`, `table_ok`: q.geometry and q.usable, in registers.  BATCH: how many lookups may be in flight
-// (all of them take registers that a product's accumulators leave no room for).
+// (all of them take registers that a product's accumulators leave no room for).  `code`: the codes, a byte each.
 template <int BITS, bool CODES, int BATCH = 64>
 __device__ __forceinline__ void group_codes64(float (&xv)[64], float mu, float var, float s, const QuantTables &q, const BucketScale &bq,
-                                              bool table_ok, float &sum_out, uint32_t (&code)[CODES ? 64 : 1])
+                                              bool table_ok, float &sum_out, uint32_t (&code)[CODES ? 16 : 1])
 {
     // The range that code_offset_of asks for: |d_j| >= 2^-90 whenever |mu| >= 2^-66, or all d_j are zero.
     const bool lane_fast = (s >= 0x1p-60f) && (s <= 0x1p58f) && !(fabsf(mu) < 0x1p-66f && var > 0.0f);
     const bool fast = table_ok && __all(lane_fast);
+    auto put = [&](int j, uint32_t c) __attribute__((always_inline)) { code[j / 4] = j % 4 == 0 ? c : code[j / 4] | c << (8 * (j % 4)); };
 
     float sum_codes = 0.0f;
     if (fast) {
@@ -270,7 +271,7 @@ __device__ __forceinline__ void group_codes64(float (&xv)[64], float mu, float v
 #pragma unroll
         for (int j = 0; j < 64; ++j) {
             const uint32_t c = code_offset_of(xv[j], cs, bq, q.bucket);
-            if constexpr (CODES) code[j] = c >> 2;
+            if constexpr (CODES) put(j, c >> 2);
             const float v = code_value(q.cb, c);
             xv[j] = v;
             sum_codes += v;
@@ -278,7 +279,7 @@ __device__ __forceinline__ void group_codes64(float (&xv)[64], float mu, float v
         }
     } else {
         search_codes<BITS>(xv, s, q, [&](int j, uint32_t c) __attribute__((always_inline)) {
-            if constexpr (CODES) code[j] = c;
+            if constexpr (CODES) put(j, c);
             sum_codes += xv[j];
         });
     }
