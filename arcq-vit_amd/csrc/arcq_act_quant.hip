@@ -19,13 +19,13 @@
 //
 // Two things keep the per-element VALU work low without changing a single result bit:
 //  * t = d/s is not formed.  Whether RN(d/s) lies above a threshold is the sign of a remainder, two fused operations; groups
-//    whose s or mu fall outside the range where that is exact take the plain division and every threshold in turn.
+//    whose s or mu fall outside the range where that is exact take the plain division and a bisection over the thresholds.
 //  * the threshold search is one table lookup and one such sign: d times an approximate 1/s names one of up to 513 buckets over
 //    [-8, 8] (|t| <= 8 always, since s^2 >= d_j^2/64; the bucket width adapts to the smallest gap between thresholds); a bucket
 //    stores how many thresholds lie in lower buckets and the single threshold inside it.  Thresholds keep a margin from the
 //    buckets' edges, so the neighbouring bucket that the approximate quotient may name gives the same code.  The codebook
 //    lies in LDS once: a read of sixteen different entries meets no bank twice.  If two thresholds share a bucket, one lies
-//    outside [-8, 8) or at an edge both ways, or they are not sorted, every threshold is gone over in turn.
+//    outside [-8, 8) or at an edge both ways, or they are not sorted, that is how all codes are found.
 // The arithmetic itself lives in arcq_act_quant_core.h (shared with the fused small-M layer kernel).
 #include "arcq_act_quant_core.h"
 #include "arcq_gemm.h"

@@ -831,9 +831,9 @@ inline int index_waves(int G)
 // 3192 x 1408 -> 736 358 -> 324; 6170 x 1472 -> 1408, dealt to all 2156 workgroups alike, 1326 -> 1210).  Three waves, of which not
 // quite four workgroups fit a compute unit: the tiles are dealt to fifteen sixteenths of a resident set, from three sets on to all
 // (12608 x 384 -> 1536: to all 761 us, the four waves' rule 894; 5000 x 576 -> 768 273 and 285).
-// Against the wide kernel alone, at 44 sizes of 512 .. 12608 rows and 2 .. 24 groups: with computed entries 0.97 of its speed in the
+// Against the wide kernel alone, at 44 sizes of 512 .. 12608 rows and 2 .. 24 groups: with computed entries 0.96 of its speed in the
 // mean (512 x 384 -> 1024 27.4 / 26.8 us, 1576 x 384 -> 1536 111 / 105, 12608 x 384 -> 1536 758 / 710; at worst, where two rounds are
-// not full, 5000 x 576 -> 768 273 / 218), with gathered ones 1.00 (at worst, nine groups on four waves, 10800 x 576 -> 1056
+// not full, 5000 x 576 -> 768 273 / 218), with gathered ones 0.99 (at worst, nine groups on four waves, 10800 x 576 -> 1056
 // 1620 / 1350).  (Eight tiles in turn per 128-row workgroup: 512 rows 100 us, 1576 164, 12608 936.)
 template <int BITS>
 void launch_index_mfma(const IndexArgs &a, hipStream_t stream)

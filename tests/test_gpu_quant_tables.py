@@ -1,5 +1,5 @@
 """A quantizer's lookup tables as each kernel builds them: thresholds that share a bucket, repeat, lie outside the table or are out of
-order (the search goes over all of them then: it stops at the first threshold that is not below the value), at every bucket width."""
+order (a search over all of them finds the code then: the first threshold that is not below the value), at every bucket width."""
 import numpy as np
 import pytest
 import torch
@@ -70,7 +70,7 @@ def test_lanes_per_group_behind_a_layernorm(cuda, oracle, m, k, dtype):
     x = (synth.make_activation(m, k, 21) * 1.7 + 0.3).to(dtype)
     g, b = torch.linspace(0.5, 1.5, k), torch.linspace(-0.2, 0.2, k)
     ln = oracle.layernorm_rows_np(x.float().numpy(), g.numpy(), b.numpy(), 1e-6, out_f16=dtype == torch.float16)
-    for t in (thr, thr[torch.randperm(15, generator=torch.Generator().manual_seed(m))].contiguous()):      # buckets; every threshold in turn
+    for t in (thr, thr[torch.randperm(15, generator=torch.Generator().manual_seed(m))].contiguous()):      # buckets; a search over the thresholds
         want = oracle.act_quant_c(ln, t, cb, 4, 64)["x_hat"].astype(np.float16)
         got = _prepare(x.to(cuda), t.to(cuda), cb.to(cuda), 4, (g.to(cuda), b.to(cuda), 1e-6))[0]
         assert np.array_equal(got.cpu().numpy().view(np.uint16), _blocked(want).view(np.uint16))
