@@ -232,11 +232,11 @@ __device__ __forceinline__ void bisect_codes(const float (&t)[N], const float *m
         for (int e = 0; e < N; ++e) at[e] += t[e] > m[e] ? step : 0u;
     }
 }
-// xv holds the residuals on entry and cb[code_j] on exit; put(j, code).  Eight values at a time (registers).
-template <int BITS, int N, typename Put>
+// xv holds the residuals on entry and cb[code_j] on exit; put(j, code).  BATCH values at a time (registers).
+template <int BITS, int BATCH = 8, int N, typename Put>
 __device__ __forceinline__ void search_codes(float (&xv)[N], float s, const QuantTables &q, const Put &put)
 {
-    constexpr int B = N < 8 ? N : 8;
+    constexpr int B = N < BATCH ? N : BATCH;
 #pragma unroll
     for (int j0 = 0; j0 < N; j0 += B) {
         float t[B];
@@ -332,7 +332,7 @@ __device__ __forceinline__ void group_stats32x2(float (&xv)[32], float eps, floa
 // xv: residuals on entry, cb[code_j] on exit; sum_out = the serial sum of all 64 cb[code_j], in both lanes.  The
 // whole wave must call it (the fast/slow decision is wave-uniform).  CODE_BITS != 0: the 32 codes too, packed CODE_BITS apart
 // into `words`.
-template <int BITS, int CODE_BITS = 0>
+template <int BITS, int CODE_BITS = 0, int BATCH = 8>
 __device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float var, float s, const QuantTables &q, const BucketScale &bq,
                                                 bool table_ok, float &sum_out, uint32_t *words = nullptr)
 {
@@ -354,7 +354,7 @@ __device__ __forceinline__ void group_codes32x2(float (&xv)[32], float mu, float
             put(j, c >> 2);
         }
     } else {
-        search_codes<BITS>(xv, s, q, put);
+        search_codes<BITS, BATCH>(xv, s, q, put);
     }
     sum_out = pair_serial_sum(xv);
 }

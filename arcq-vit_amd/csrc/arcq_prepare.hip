@@ -361,7 +361,7 @@ prepare_ln_kernel(const TIN *__restrict__ x, const float *__restrict__ gamma, co
         float mu, var, s, sum_codes;
         if constexpr (LANES == 2) {
             group_stats32x2(xv, eps, mu, var, s);
-            group_codes32x2<BITS>(xv, mu, var, s, tables, bq, table_ok, sum_codes);
+            group_codes32x2<BITS, 0, sizeof(TIN) == 4 ? 4 : 8>(xv, mu, var, s, tables, bq, table_ok, sum_codes);      // (fp32: eight at a time spill)
         } else {
             group_stats_lanes<LANES>(xv, eps, lane, mu, var, s);
             group_codes_lanes<BITS, LANES>(xv, mu, var, s, tables, bq, table_ok, lane, sum_codes);
