@@ -68,6 +68,19 @@ class LinearIndexArgs(ctypes.Structure):
         (n, ctypes.c_int32) for n in ("bits", "group_size", "levels", "reserved")]
 
 
+class MlpLayer(ctypes.Structure):
+    """``arcq_mlp_layer``."""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("a_thresholds", "a_codebook", "packed_w", "w_codebook", "w_center", "w_scale",
+                                               "w_code_sum", "bias", "w_hat_ws")]
+
+
+class MlpArgs(ctypes.Structure):
+    """``arcq_mlp_args``."""
+    _fields_ = [("bits", ctypes.c_int32), ("eps", ctypes.c_float), ("ln_eps", ctypes.c_float)] + [
+        (n, ctypes.c_int64) for n in ("M", "K", "H")] + [(n, ctypes.c_void_p) for n in ("x", "ln_weight", "ln_bias")] + [
+        ("fc1", MlpLayer), ("fc2", MlpLayer), ("y", ctypes.c_void_p)]
+
+
 ARCQ_PRODUCER_NONE, ARCQ_PRODUCER_LAYERNORM, ARCQ_PRODUCER_XHAT = 0, 1, 2
 ARCQ_ACT_NONE, ARCQ_ACT_GELU = 0, 1
 
@@ -97,6 +110,9 @@ _SIGNATURES = {
                              ctypes.POINTER(PrepareWeights), _c_ptr],
     "arcq_prepare": [ctypes.POINTER(PrepareArgs), _c_ptr],
     "arcq_linear_prepared": [ctypes.POINTER(LinearPreparedArgs), _c_ptr],
+    "arcq_mlp_otf": [ctypes.POINTER(MlpArgs), _c_ptr],
+    "arcq_mlp_otf_supported": [_c_i64, _c_i64, _c_i64],
+    "arcq_mlp_otf_pays": [_c_i64, _c_i64, _c_i64],
     "arcq_act_quant_blocked_ln": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_f32, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_int,
                                   _c_f32, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr],
     "arcq_act_quant_blocked": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_int, _c_f32, _c_ptr],

@@ -40,6 +40,17 @@ __device__ __forceinline__ void xhat_fp8x16(const float (&v)[N], int j0, float s
     }
 }
 
+// Values rounded to fp16 and widened again, two to a conversion.
+template <int N>
+__device__ __forceinline__ void round_to_half(float (&v)[N])
+{
+#pragma unroll
+    for (int j = 0; j < N; j += 2) {
+        const __half2 h = __floats2half2_rn(v[j], v[j + 1]);
+        v[j] = __low2float(h), v[j + 1] = __high2float(h);
+    }
+}
+
 constexpr int kMaxBuckets = 512;   // table entries 0 .. nb (nb <= 512); entry nb is reached by t == 8 only
 
 // Bucket geometry: t in [-8, 8] maps to floor(f), f = t * scale + 8 * scale rounded to a multiple of 1/8; nb = 16 * scale
@@ -99,15 +110,25 @@ __device__ __forceinline__ CodeScale code_scale_of(float s, float about_1_over_s
 {
     return CodeScale{s, s * 0x1p-24f, about_1_over_s * q.scale};
 }
-// 4 times the code of d.  In range |d / s| <= 8, f lies in [0, nb] <= 512.25 and the bucket's offset is bits 3..12 of the biased sum.
-__device__ __forceinline__ uint32_t code_offset_of(float d, const CodeScale &c, const BucketScale &q, const Bucket *table)
+// The bucket of d.  In range |d / s| <= 8, f lies in [0, nb] <= 512.25 and the bucket's offset is bits 3..12 of the biased sum.
+__device__ __forceinline__ Bucket bucket_of(float d, const CodeScale &c, const BucketScale &q, const Bucket *table)
 {
     static_assert(sizeof(Bucket) == 8, "the offset assumes 8-byte table entries");
     const uint32_t at = __float_as_uint(__fmaf_rn(d, c.to_bucket, q.offset)) & 0x1ff8u;
-    const Bucket bk = *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(table) + at);
+    return *reinterpret_cast<const Bucket *>(reinterpret_cast<const char *>(table) + at);
+}
+// 4 times the code of d, whose bucket is bk.
+__device__ __forceinline__ uint32_t code_offset_in(const Bucket &bk, float d, const CodeScale &c)
+{
     const float e = __uint_as_float(__float_as_uint(bk.u) & 0xff800000u);
     const float r = __fmaf_rn(c.s24, e, __fmaf_rn(c.s, bk.u, -d));
-    return ((__float_as_uint(r) >> 31) << 2) + static_cast<uint32_t>(bk.base);
+    uint32_t below = __float_as_uint(r) >> 31;
+    asm("" : "+v"(below));      // (a shift and one v_lshl_add; left alone the two shifts become one shift, a mask and an addition)
+    return (below << 2) + static_cast<uint32_t>(bk.base);
+}
+__device__ __forceinline__ uint32_t code_offset_of(float d, const CodeScale &c, const BucketScale &q, const Bucket *table)
+{
+    return code_offset_in(bucket_of(d, c, q, table), d, c);
 }
 __device__ __forceinline__ float code_value(const float *cb, uint32_t offset)
 {
@@ -253,9 +274,40 @@ __device__ __forceinline__ void search_codes(float (&xv)[N], float s, const Quan
     }
 }
 
+// The lookups of 64 values for a wave that has its SIMD for itself (or shares it with one that multiplies): the first read of eight
+// values, the second read of the eight before and the sum of the eight before those are under way at a time, so that no read is waited
+// for.  xv as in group_codes64; returns the sum.  A wave's 64 x 64 values beside another one's product: 9 300 -> 8 700 clocks.
+__device__ __forceinline__ float codes64_in_turns(float (&xv)[64], const CodeScale &cs, const QuantTables &q, const BucketScale &bq)
+{
+    float sum = 0.0f;
+    Bucket bk[2][8];
+#pragma unroll
+    for (int b = 0; b < 10; ++b) {
+        if (b < 8) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) bk[b & 1][e] = bucket_of(xv[8 * b + e], cs, bq, q.bucket);
+        }
+        if (b >= 2) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum += xv[8 * (b - 2) + e];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (b >= 1 && b < 9) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float &v = xv[8 * (b - 1) + e];
+                v = code_value(q.cb, code_offset_in(bk[(b - 1) & 1][e], v, cs));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    return sum;
+}
+
 // Second half: xv holds the residuals on entry and cb[code_j] on exit.  The whole wave must call it (the fast/slow
 // decision is wave-uniform).  `bq`, `table_ok`: q.geometry and q.usable, in registers.  BATCH: how many lookups may be in flight
 // (all of them take registers that a product's accumulators leave no room for).  `code`: the codes, a byte each.
+// BATCH = 0: codes64_in_turns.
 template <int BITS, bool CODES, int BATCH = 64>
 __device__ __forceinline__ void group_codes64(float (&xv)[64], float mu, float var, float s, const QuantTables &q, const BucketScale &bq,
                                               bool table_ok, float &sum_out, uint32_t (&code)[CODES ? 16 : 1])
@@ -268,14 +320,19 @@ __device__ __forceinline__ void group_codes64(float (&xv)[64], float mu, float v
     float sum_codes = 0.0f;
     if (fast) {
         const CodeScale cs = code_scale_of(s, __builtin_amdgcn_rcpf(s), bq);
+        if constexpr (BATCH == 0) {
+            static_assert(!CODES, "codes64_in_turns keeps none");
+            sum_codes = codes64_in_turns(xv, cs, q, bq);
+        } else {
 #pragma unroll
-        for (int j = 0; j < 64; ++j) {
-            const uint32_t c = code_offset_of(xv[j], cs, bq, q.bucket);
-            if constexpr (CODES) put(j, c >> 2);
-            const float v = code_value(q.cb, c);
-            xv[j] = v;
-            sum_codes += v;
-            if (BATCH < 64 && j % BATCH == BATCH - 1) __builtin_amdgcn_sched_barrier(0);
+            for (int j = 0; j < 64; ++j) {
+                const uint32_t c = code_offset_of(xv[j], cs, bq, q.bucket);
+                if constexpr (CODES) put(j, c >> 2);
+                const float v = code_value(q.cb, c);
+                xv[j] = v;
+                sum_codes += v;
+                if (BATCH < 64 && j % BATCH == BATCH - 1) __builtin_amdgcn_sched_barrier(0);
+            }
         }
     } else {
         search_codes<BITS>(xv, s, q, [&](int j, uint32_t c) __attribute__((always_inline)) {
@@ -483,8 +540,7 @@ __device__ __forceinline__ void next_quant_rows(const unsigned char *lds, const 
     if (gelu) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) gelu_of_halves(v + 8 * i);
-#pragma unroll
-        for (int j = 0; j < 32; ++j) v[j] = __half2float(__float2half_rn(v[j]));
+        round_to_half(v);
     }
     float mu, var, s, sum;
     group_stats32x2(v, eps, mu, var, s);
@@ -561,8 +617,7 @@ __device__ __forceinline__ void next_quant_groups(const unsigned char *lds, cons
     if (gelu) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) gelu_of_halves(v + 8 * i);
-#pragma unroll
-        for (int j = 0; j < 64; ++j) v[j] = __half2float(__float2half_rn(v[j]));
+        round_to_half(v);
     }
     float mu, var, s, sum;
     uint32_t none[1];

@@ -177,38 +177,51 @@ __device__ __forceinline__ float gelu_f32(float x)
 // coefficient is negative, so 2^q runs to 0 for every larger input and infinities and NaN come out as above.
 // 12 608 x 384 -> 1 536 with GELU 30.0 -> 25.9 us (17.5 without), 50 432 x 1 024 -> 4 096 with GELU and the next layer's quantizer
 // 639 -> 564 us.
+// Eight values a lane, coefficient by coefficient: a wave that has its SIMD's vector ALU for itself would wait for every step of one
+// value's chain (a quantizing epilogue of 64 values a lane beside another wave's products: DeiT-B's MLP, see arcq_otf_mlp.hip).
+template <int N>
+__device__ __forceinline__ void gelu_of_halves_wide(float *v)
+{
+    constexpr float c[9] = {0x1.4db25cp-20f, -0x1.d74ab4p-17f, 0x1.775b7ep-14f, -0x1.461452p-12f, 0x1.64986cp-15f,
+                            0x1.c5462ap-8f,  -0x1.ad857p-5f,   -0x1.d63e1ap-2f, -0x1.26aec8p+0f};
+    float p[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = -0x1.a0d3f2p-25f;
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+#pragma unroll
+        for (int i = 0; i < N; ++i) p[i] = __fmaf_rn(fabsf(v[i]), p[i], c[k]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = 1.0f - __builtin_amdgcn_exp2f(fabsf(v[i]) * p[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float h = 0.5f * v[i];
+        v[i] = fma_f32(fabsf(h), p[i], h);
+    }
+}
 __device__ __forceinline__ float gelu_of_half(float x)
 {
-    const float a = fabsf(x);
-    float p = -0x1.a0d3f2p-25f;
-    p = __fmaf_rn(a, p, 0x1.4db25cp-20f);
-    p = __fmaf_rn(a, p, -0x1.d74ab4p-17f);
-    p = __fmaf_rn(a, p, 0x1.775b7ep-14f);
-    p = __fmaf_rn(a, p, -0x1.461452p-12f);
-    p = __fmaf_rn(a, p, 0x1.64986cp-15f);
-    p = __fmaf_rn(a, p, 0x1.c5462ap-8f);
-    p = __fmaf_rn(a, p, -0x1.ad857p-5f);
-    p = __fmaf_rn(a, p, -0x1.d63e1ap-2f);
-    p = __fmaf_rn(a, p, -0x1.26aec8p+0f);
-    const float h = 0.5f * x;
-    return fma_f32(fabsf(h), 1.0f - __builtin_amdgcn_exp2f(a * p), h);
+    gelu_of_halves_wide<1>(&x);
+    return x;
 }
 // The same where |x| < 2.5: erf(x / sqrt(2)) = x Q(x^2), Q of degree 8; 12 slots, the same bits again.
 constexpr float kGeluNarrow = 2.5f;
-__device__ __forceinline__ float gelu_of_half_narrow(float x)
+__device__ __forceinline__ void gelu_of_halves_narrow(float *v)
 {
-    const float u = x * x;
-    float p = 0x1.190f2p-30f;
-    p = __fmaf_rn(u, p, -0x1.98875cp-25f);
-    p = __fmaf_rn(u, p, 0x1.2ad372p-20f);
-    p = __fmaf_rn(u, p, -0x1.2e3f06p-16f);
-    p = __fmaf_rn(u, p, 0x1.df8c04p-13f);
-    p = __fmaf_rn(u, p, -0x1.36cf0ep-9f);
-    p = __fmaf_rn(u, p, 0x1.46c424p-6f);
-    p = __fmaf_rn(u, p, -0x1.10579ap-3f);
-    p = __fmaf_rn(u, p, 0x1.98844ep-1f);
-    const float h = 0.5f * x;
-    return fma_f32(h, x * p, h);
+    constexpr float c[8] = {-0x1.98875cp-25f, 0x1.2ad372p-20f, -0x1.2e3f06p-16f, 0x1.df8c04p-13f,
+                            -0x1.36cf0ep-9f,  0x1.46c424p-6f,  -0x1.10579ap-3f,  0x1.98844ep-1f};
+    float u[8], p[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) u[i] = v[i] * v[i], p[i] = 0x1.190f2p-30f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) p[i] = __fmaf_rn(u[i], p[i], c[k]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float h = 0.5f * v[i];
+        v[i] = fma_f32(h, v[i] * p[i], h);
+    }
 }
 // Eight values a lane: the narrow form where none of the wave's is beyond it.
 __device__ __forceinline__ void gelu_of_halves(float *v)
@@ -217,11 +230,9 @@ __device__ __forceinline__ void gelu_of_halves(float *v)
 #pragma unroll
     for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(v[i]));      // (a NaN is one in both forms)
     if (__any(m >= kGeluNarrow)) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = gelu_of_half(v[i]);
+        gelu_of_halves_wide<8>(v);
     } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = gelu_of_half_narrow(v[i]);
+        gelu_of_halves_narrow(v);
     }
 }
 

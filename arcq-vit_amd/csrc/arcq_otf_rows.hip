@@ -33,9 +33,7 @@
 #include "arcq_common.h"
 #include "arcq_gemm.h"
 #include "arcq_act_quant_core.h"
-
-#include <mutex>
-#include <vector>
+#include "arcq_rows_share.h"
 
 namespace arcq {
 namespace {
@@ -49,7 +47,6 @@ constexpr int kWaveLds = 4608;               // bytes of LDS per wave: the outpu
 // otf_rows_kernel's staging tile: kWaveLds, or, where a wave quantizes two tiles (K = 768: LDS is short), just the
 // 32 rows of 32 outputs + 16 bytes that the epilogue uses.
 constexpr int rows_stage_bytes(int rounds, size_t out_size) { return rounds == 1 ? kWaveLds : 32 * (32 * static_cast<int>(out_size) + 16); }
-constexpr unsigned long long kEpoch = 1ull << 20;     // what one launch adds to its counter, whatever its grid
 
 constexpr int gcd_of(int a, int b) { return b == 0 ? a : gcd_of(b, a % b); }
 
@@ -59,10 +56,8 @@ struct RowsParams {
     float eps;
     const float *gamma, *beta;       // LayerNorm weight / bias (fp32), gamma == nullptr: no LayerNorm
     float ln_eps;
-    const uint8_t *pw;               // packed weight codes [N, K*bits/8]
-    const float *cb_w, *wc, *ws, *wcs;
-    __half *w_blk;                   // weight workspace, block layout
-    unsigned long long *counter;     // nullptr: w_blk is complete already
+    WeightShare w;
+    unsigned long long *counter;     // nullptr: w.out is complete already
     long long wait_ticks;            // bound of the wait for the other workgroups' shares, ticks of the 100 MHz clock
     unsigned long long *timeouts;    // counts the workgroups whose wait ran out (a diagnostic: arcq_rows_wait_timeouts)
     const float *bias;               // [N] or nullptr
@@ -71,45 +66,6 @@ struct RowsParams {
     int gelu;
     int M, N, G;
 };
-
-// Piece idx of the block-layout w_hat, idx = ((n / 32) * (K / 8) + k / 8) * 32 + n % 32, holds w_hat[n][k .. k + 8):
-// value (cb[code] - code_sum/64) * scale + center with one fma (FQ/arcq_packed_triton.py:59-74), stored at
-// out + 8 idx, written through to memory.  In two steps so that the loads of the first can travel under other work.
-struct Piece {
-    uint32_t w;
-    float c, s, m;
-};
-template <int BITS, int G>
-__device__ __forceinline__ void fetch_piece(const RowsParams &p, int64_t idx, Piece &pc)
-{
-    constexpr int K = 64 * G, P = K / 8, pcols = K * BITS / 8;     // compile-time: the divisions below are multiplications
-    const uint32_t i = static_cast<uint32_t>(idx);                 // N * K / 8 < 2^31 (N <= 16384, K <= 384)
-    const uint32_t r = i & 31u;
-    const uint32_t t = i >> 5;
-    const uint32_t nb = t / P;
-    const uint32_t pp = t - nb * P;
-    const uint32_t n = nb * 32u + r;
-    pc.w = load_codes8<BITS>(p.pw + n * pcols + pp * BITS);
-    const uint32_t mi = n * G + (pp >> 3);
-    pc.c = p.wc[mi];
-    pc.s = p.ws[mi];
-    pc.m = p.wcs[mi] * 0.015625f;      // code_sum / 64, exact
-}
-template <int BITS>
-__device__ __forceinline__ void finish_piece(const RowsParams &p, int64_t idx, const Piece &pc)
-{
-    constexpr int L = 1 << BITS;
-    float cbv[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) cbv[q] = p.cb_w[(pc.w >> (BITS * q)) & (L - 1)];      // 64 bytes, cached
-    uint32_t out[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const __half2 h = __floats2half2_rn(fma_f32(cbv[2 * q] - pc.m, pc.s, pc.c), fma_f32(cbv[2 * q + 1] - pc.m, pc.s, pc.c));
-        out[q] = *reinterpret_cast<const uint32_t *>(&h);
-    }
-    store_writethrough16(p.w_blk + idx * 8, out[0], out[1], out[2], out[3]);
-}
 
 // G = K / 64 groups per row (the workgroup has 2 G waves); RING = groups of w_hat fragments a wave holds (the one
 // being multiplied and RING - 1 on their way from L2); AHEAD = k-steps by which the LDS reads of the x_hat fragments
@@ -180,8 +136,8 @@ otf_rows_kernel(const RowsParams p)
         const int64_t lo = (static_cast<int>(blockIdx.x) - row_wgs) * per;
         const int64_t hi = lo + per < pieces ? lo + per : pieces;
         for (int64_t idx = lo + tid; idx < hi; idx += nthreads) {
-            fetch_piece<BITS, G>(p, idx, pc);
-            finish_piece<BITS>(p, idx, pc);
+            fetch_piece<BITS, G>(p.w, idx, pc);
+            finish_piece<BITS>(p.w, idx, pc);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
@@ -194,7 +150,7 @@ otf_rows_kernel(const RowsParams p)
         per = (per + 7) & ~int64_t(7);                          // whole 128-byte lines per workgroup
         share_lo = blockIdx.x * per;
         share_hi = share_lo + per < pieces ? share_lo + per : pieces;
-        if (ptid >= 0 && share_lo + ptid < share_hi) fetch_piece<BITS, G>(p, share_lo + ptid, pc);
+        if (ptid >= 0 && share_lo + ptid < share_hi) fetch_piece<BITS, G>(p.w, share_lo + ptid, pc);
     }
 
     // ---- stage 1: wave = (row block rb2, group g), two lanes per (row, group) ----
@@ -202,10 +158,10 @@ otf_rows_kernel(const RowsParams p)
     {
         if (wave == kBuilder) build_quant_tables<BITS>(params, tables, lane);      // while the tiles are on their way
         if (own_share) {
-            if (ptid >= 0 && share_lo + ptid < share_hi) finish_piece<BITS>(p, share_lo + ptid, pc);
+            if (ptid >= 0 && share_lo + ptid < share_hi) finish_piece<BITS>(p.w, share_lo + ptid, pc);
             for (int64_t idx = share_lo + kPieceThreads + ptid; ptid >= 0 && idx < share_hi; idx += kPieceThreads) {     // (large N*K only)
-                fetch_piece<BITS, G>(p, idx, pc);
-                finish_piece<BITS>(p, idx, pc);
+                fetch_piece<BITS, G>(p.w, idx, pc);
+                finish_piece<BITS>(p.w, idx, pc);
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the written-through pieces have reached memory
         }
@@ -312,8 +268,8 @@ otf_rows_kernel(const RowsParams p)
     if (p.counter) {
         if (!s_flag) {                            // workgroup-uniform
             for (int64_t idx = tid; idx < pieces; idx += nthreads) {
-                fetch_piece<BITS, G>(p, idx, pc);
-                finish_piece<BITS>(p, idx, pc);
+                fetch_piece<BITS, G>(p.w, idx, pc);
+                finish_piece<BITS>(p.w, idx, pc);
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
@@ -324,7 +280,7 @@ otf_rows_kernel(const RowsParams p)
     const int lr = lane & 31, lh = lane >> 5;
     const int ncb = p.N / 32;
     const unsigned char *xs_lane = xs + lr * pitch + lh * 64;
-    const char *w_lane = reinterpret_cast<const char *>(p.w_blk) + lh * 2048 + lr * 16;
+    const char *w_lane = reinterpret_cast<const char *>(p.w.out) + lh * 2048 + lr * 16;
     const int64_t cb_bytes = static_cast<int64_t>(K) * 64;     // bytes per 32-column block
     // The wave's blocks are a run of adjacent ones: a row's 64-byte segments of two neighbouring blocks share a
     // 128-byte line, and written by one wave shortly after each other they are more often merged on their way to
@@ -544,15 +500,15 @@ otf_rows_phased_kernel(const RowsParams p)
         per = (per + 7) & ~int64_t(7);
         share_lo = blockIdx.x * per;
         share_hi = share_lo + per < pieces ? share_lo + per : pieces;
-        if (ptid >= 0 && share_lo + ptid < share_hi) fetch_piece<BITS, GT>(p, share_lo + ptid, pc);
+        if (ptid >= 0 && share_lo + ptid < share_hi) fetch_piece<BITS, GT>(p.w, share_lo + ptid, pc);
     }
     for (int i = tid; i < 32 * W * NB; i += nthreads) s_bias[i] = (p.bias && i < p.N) ? p.bias[i] : 0.0f;
     if (wave == kBuilder) build_quant_tables<BITS>(params, tables, lane);
     if (p.counter) {
-        if (ptid >= 0 && share_lo + ptid < share_hi) finish_piece<BITS>(p, share_lo + ptid, pc);
+        if (ptid >= 0 && share_lo + ptid < share_hi) finish_piece<BITS>(p.w, share_lo + ptid, pc);
         for (int64_t idx = share_lo + kPieceThreads + ptid; ptid >= 0 && idx < share_hi; idx += kPieceThreads) {
-            fetch_piece<BITS, GT>(p, idx, pc);
-            finish_piece<BITS>(p, idx, pc);
+            fetch_piece<BITS, GT>(p.w, idx, pc);
+            finish_piece<BITS>(p.w, idx, pc);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // the written-through pieces have reached memory
     }
@@ -570,7 +526,7 @@ otf_rows_phased_kernel(const RowsParams p)
     const int ncb = p.N / 32;
     const int nv = wave < ncb ? min(NB, (ncb - wave + W - 1) / W) : 0;      // this wave's blocks: nb < nv
     const bool has_block = nv > 0;
-    const char *w_col = reinterpret_cast<const char *>(p.w_blk) + lh * 2048 + lr * 16 +
+    const char *w_col = reinterpret_cast<const char *>(p.w.out) + lh * 2048 + lr * 16 +
                         static_cast<int64_t>(has_block ? wave : 0) * (static_cast<int64_t>(K) * 64);
     constexpr int64_t kBlockStride = static_cast<int64_t>(W) * K * 64;      // bytes from a wave's block to its next one
     // The fragment groups are consumed slice by slice, within a slice block by block, within a block group by group;
@@ -690,8 +646,8 @@ otf_rows_phased_kernel(const RowsParams p)
         if (ph == -1) {
             if (p.counter && !s_flag) {          // workgroup-uniform: the others are not resident; rebuild everything
                 for (int64_t idx = tid; idx < pieces; idx += nthreads) {
-                    fetch_piece<BITS, GT>(p, idx, pc);
-                    finish_piece<BITS>(p, idx, pc);
+                    fetch_piece<BITS, GT>(p.w, idx, pc);
+                    finish_piece<BITS>(p.w, idx, pc);
                 }
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __syncthreads();
@@ -764,7 +720,7 @@ otf_rows_phased_kernel(const RowsParams p)
 // two-launch path (a model shares one workspace between its layers; the table is sized for processes that allocate
 // and free workspaces all the time, such as a test suite).
 constexpr int kCounterSlots = 4096;
-__device__ unsigned long long g_rows_counters[kCounterSlots];
+__device__ unsigned long long g_rows_counters[2 * kCounterSlots];       // (a launch may rebuild the weights of two layers)
 __device__ unsigned long long g_rows_timeouts;          // workgroups whose bounded wait ran out, ever
 
 constexpr int kMaxDevices = 64;
@@ -796,10 +752,8 @@ int rows_counter_slot(const void **table, int slots, const void *key)
     return -1;
 }
 
-namespace {
-
-// Device address of the counter that belongs to weight workspace `key` on the current device; nullptr if none is left.
-unsigned long long *counter_for(const void *key, unsigned long long **timeouts)
+// Device address of the counters that belong to weight workspace `key` on the current device; nullptr if none are left.
+unsigned long long *rows_counters_for(const void *key, unsigned long long **timeouts)
 {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
@@ -815,33 +769,8 @@ unsigned long long *counter_for(const void *key, unsigned long long **timeouts)
     const int slot = rows_counter_slot(g_slot_key[dev].data(), kCounterSlots, key);
     if (slot < 0) return nullptr;            // more workspaces than counters: the caller falls back
     *timeouts = g_timeouts_ptr[dev];
-    return g_counters_ptr[dev] + slot;
+    return g_counters_ptr[dev] + 2 * slot;
 }
-
-// Workgroups of `Kernel` (threads, dynamic LDS bytes) the current device holds at once.  A launch must not be larger:
-// every workgroup waits for the weight shares of all the others, and those that are not resident write theirs only
-// after a resident one has given up waiting (correct, but milliseconds late).  Asked once per device, kernel and LDS
-// size; 0 if the runtime cannot tell.
-template <auto Kernel>
-int resident_workgroups(int threads, size_t smem)
-{
-    struct Entry { int dev; size_t smem; int blocks; };
-    static std::mutex mutex;
-    static std::vector<Entry> known;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    std::lock_guard<std::mutex> lock(mutex);
-    for (const Entry &e : known)
-        if (e.dev == dev && e.smem == smem) return e.blocks;
-    int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(Kernel), threads, smem) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        per_cu = cus = 0;
-    known.push_back({dev, smem, per_cu * cus});
-    return per_cu * cus;
-}
-
-}  // namespace
 
 // Compute units of the current device (256 when there is none to ask: the host-side predicates also run without a GPU).
 int device_cus()
@@ -981,9 +910,8 @@ int launch_otf_rows(const OtfRowsArgs &a, hipStream_t stream)
     p.x = static_cast<const __half *>(a.x);
     p.thr = a.a_thr, p.cb_a = a.a_cb, p.eps = a.eps;
     p.gamma = a.ln_weight, p.beta = a.ln_bias, p.ln_eps = a.ln_eps;
-    p.pw = a.pw, p.cb_w = a.w_cb, p.wc = a.wc, p.ws = a.ws, p.wcs = a.wcs;
-    p.w_blk = static_cast<__half *>(a.w_hat_ws);
-    p.counter = counter_for(a.w_hat_ws, &p.timeouts);
+    p.w = WeightShare{a.pw, a.w_cb, a.wc, a.ws, a.wcs, static_cast<__half *>(a.w_hat_ws)};
+    p.counter = rows_counters_for(a.w_hat_ws, &p.timeouts);
     if (!p.counter) return kNotLaunched;     // more workspaces than counters: the caller takes the two-launch path
     p.wait_ticks = tuning().rows_wait_ticks;
     p.bias = a.bias, p.y = a.y, p.residual = a.residual, p.gelu = a.gelu ? 1 : 0;

@@ -687,9 +687,12 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
     if ((fuse_ln && C > 2048) || pf1.N % 64 != 0 || !aligned16(x)) return std::nullopt;      // (x is also proj's residual)
     for (const Plan *p : {&pq, &pp, &pf1, &pf2})
         if (!can_prepare(*p, rows) || p->bits != pq.bits) return std::nullopt;
-    // Not where the one-launch layer kernels are at their best (one 64-row tile on most compute units, short rows).  With the
-    // LayerNorms inside: DeiT-S at 12 608 rows 1 625 us a forward against 1 939, DeiT-B 3 969 against 4 373; at 9 456 rows 4 %
-    // either way, below and above that range the seven launches win (6 304 rows: 1 353 -> 1 262 us; 25 216 rows: 3 341 -> 3 286).
+    // Not where the one-launch kernels are at their best (one 64-row tile on most compute units, short rows).  With the LayerNorms
+    // inside, hidden rows of four times the width and lent weight buffers, the block is four launches there, the last of them the
+    // whole MLP: a block of DeiT-S at 11 032 rows 111 us against 124, at 16 351 127 / 141, DeiT-B 260 / 287 and 316 / 372, DeiT-Tiny at
+    // 12 608 rows 69 / 79; at 9 456 rows 110 / 106, 250 / 242 and 66 / 64, below that the seven launches win by more, and with more row
+    // tiles than compute units they win too (DeiT-Tiny at 19 700 rows 99 against 112).  Without the one-launch MLP 9 000 rows: DeiT-S at
+    // 12 608 rows 1 625 us a forward against 1 939 (five launches a block), at 6 304 rows 1 353 -> 1 262.
     // With torch's LayerNorms and GELU those kernels run only on lent weight buffers, and win later and only beside torch's
     // attention: 10 638 rows DeiT-S 2 311 us against 2 264 here, DeiT-B 4 498 / 4 406, 11 032 rows 2 318 / 2 439 and 4 607 / 4 879,
     // 12 608 rows 2 399 / 2 564 and 4 892 / 5 147; without lent buffers (two launches a layer) 2 667 / 2 590 and 5 207 / 5 178, with
@@ -697,7 +700,8 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
     // compute unit (DeiT-Tiny, 17 730 rows) 2 287 / 2 201.
     if (!fp8 && strncmp(arcq_linear_otf_ws_kernel(rows, pq.N, C, 1), "otf_rows", 8) == 0) {
         const bool lends = k.qkv.lends && k.proj.lends && k.fc1.lends && k.fc2.lends;
-        if (fuse_ln ? rows > 9000 : lends && !own_attention && rows > 10800 && rows <= 16384) return std::nullopt;
+        const bool alone = lends && (pf1.N == 4 * C ? arcq_mlp_otf_pays(rows, C, pf1.N) != 0 : rows > 9000);
+        if (fuse_ln ? alone : lends && !own_attention && rows > 10800 && rows <= 16384) return std::nullopt;
     }
     Tensor t = fuse_ln ? x : k.norm1(x);
     void *stream = stream_of(x);
@@ -734,6 +738,41 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
     return y;
 }
 
+// The block's second half, x + fc2(GELU(fc1(LayerNorm(x)))), in one launch; nullopt before it where that does not serve or pay.
+std::optional<Tensor> run_mlp(const Layer &fc1, const Layer &fc2, const FusedLayerNorm &ln, const Tensor &x)
+{
+    const Plan &p1 = *fc1.plan, &p2 = *fc2.plan;
+    const int64_t rows = x.numel() / p1.K;
+    if (!arcq_mlp_otf_pays(rows, p1.K, p1.N) || !fc1.lends || !fc2.lends || !lent(fc1.weight_buffer, p1.N * p1.K, x)) return std::nullopt;
+    if (p1.bits != p2.bits || p1.gs != 64 || p2.gs != 64 || fc1.fp8 || fc2.fp8 || fc1.out != at::kHalf || fc2.out != at::kHalf) return std::nullopt;
+    if (!takes(fc1, x) || !f16(x) || p2.K != p1.N || p2.N != p1.K || p2.device != p1.device || !aligned16(x) || !aligned16(ln.weight) ||
+        !aligned16(ln.bias))
+        return std::nullopt;
+    const Tensor w2 = empty({p2.N * p2.K}, at::kHalf, x.device());
+    void *const ws[2] = {fc1.weight_buffer->mutable_data_ptr(), w2.mutable_data_ptr()};
+    arcq_mlp_args a = {};
+    a.bits = static_cast<int32_t>(p1.bits);
+    a.eps = 1.0e-6f, a.ln_eps = ln.eps;
+    a.M = rows, a.K = p1.K, a.H = p1.N;
+    a.x = x.const_data_ptr();
+    a.ln_weight = ln.weight, a.ln_bias = ln.bias;
+    arcq_mlp_layer *const l[2] = {&a.fc1, &a.fc2};
+    const Plan *const plans[2] = {&p1, &p2};
+    for (int i = 0; i < 2; ++i) {
+        const auto *p = plans[i]->p;
+        auto fp = [&](int j) { return static_cast<const float *>(p[j]); };
+        if (reinterpret_cast<uintptr_t>(p[W_PACKED]) % 4 != 0 || reinterpret_cast<uintptr_t>(ws[i]) % 128 != 0) return std::nullopt;
+        *l[i] = arcq_mlp_layer{fp(A_THR), fp(A_CB), static_cast<const uint8_t *>(p[W_PACKED]), fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM),
+                               fp(W_BIAS), ws[i]};
+    }
+    Tensor y = empty(x.sizes(), at::kHalf, x.device());
+    a.y = y.mutable_data_ptr();
+    const int rc = arcq_mlp_otf(&a, stream_of(x));
+    if (rc == ARCQ_ERR_UNSUPPORTED) return std::nullopt;      // (nothing launched: no counter left, or a device that holds fewer workgroups)
+    check(rc);
+    return y;
+}
+
 // One transformer block (vit.Block.forward), both of its forms.  No Python object is touched.
 std::optional<Tensor> run_block(const BlockParts &k, const Tensor &x, bool chain)
 {
@@ -753,6 +792,10 @@ std::optional<Tensor> run_block(const BlockParts &k, const Tensor &x, bool chain
         o2.residual = &x;
         auto x1 = run_layer(k.proj, a, o2);
         if (!x1) return std::nullopt;
+        if (chain) {
+            auto y = run_mlp(k.fc1, k.fc2, k.fused2, *x1);
+            if (y) return y;
+        }
         Options o3, o4;
         o3.layernorm = &k.fused2;
         o3.gelu = true;

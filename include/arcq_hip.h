@@ -320,6 +320,30 @@ int arcq_linear_prepared(const arcq_linear_prepared_args *args, void *stream);
  * (the weight-stationary kernels, which want many row blocks; fp16 operands: M >= 512). */
 int arcq_prepared_row_major(int64_t M, int64_t N, int64_t K);
 
+/* The MLP half of a transformer block in one launch: y = x + fc2(GELU(fc1(LayerNorm(x)))), both layers packed on-the-fly layers of
+ * group size 64 with `bits`-bit codes, x and y [M,K] fp16, fc1 [H,K], fc2 [K,H].  y has the bits of the two layer calls with the fused
+ * options (arcq_linear_otf_ex).  Each layer brings a workspace of H*K fp16 values; calls that share fc1's must not overlap. */
+typedef struct arcq_mlp_layer {
+    const float *a_thresholds, *a_codebook;
+    const uint8_t *packed_w;
+    const float *w_codebook, *w_center, *w_scale, *w_code_sum, *bias;     /* bias may be NULL */
+    void *w_hat_ws;
+} arcq_mlp_layer;
+typedef struct arcq_mlp_args {
+    int32_t bits;
+    float eps, ln_eps;
+    int64_t M, K, H;
+    const void *x;
+    const float *ln_weight, *ln_bias;
+    arcq_mlp_layer fc1, fc2;
+    void *y;
+} arcq_mlp_args;
+int arcq_mlp_otf(const arcq_mlp_args *args, void *stream);
+/* Whether it serves these sizes (ARCQ_ERR_UNSUPPORTED otherwise): K = 192, 256, 384 or 768, H = 4 K, 512 rows up to 64 per compute unit. */
+int arcq_mlp_otf_supported(int64_t M, int64_t K, int64_t H);
+/* Whether it is the faster way there. */
+int arcq_mlp_otf_pays(int64_t M, int64_t K, int64_t H);
+
 /* arcq_linear_otf_ws for callers that cannot allocate device memory or lend workspaces (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The two
  * scratch buffers come from a static device array of ARCQ_STATIC_SCRATCH_BYTES inside the library, of which every GPU
