@@ -106,6 +106,7 @@ _SIGNATURES = {
     "arcq_linear_otf_ex": [ctypes.POINTER(LinearExArgs), _c_ptr],
     "arcq_xhat_layout": [_c_i64],
     "arcq_prepared_row_major": [_c_i64, _c_i64, _c_i64],
+    "arcq_prepared_quant_row_major": [_c_i64, _c_i64, _c_i64, _c_int],
     "arcq_prepare_patches": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_f32,
                              ctypes.POINTER(PrepareWeights), _c_ptr],
     "arcq_prepare": [ctypes.POINTER(PrepareArgs), _c_ptr],

@@ -653,4 +653,95 @@ __device__ __forceinline__ void next_quant_groups(const unsigned char *lds, cons
     }
 }
 
+// ---- a row per lane, straight from a wave's 64 x 64 tile of a product ----
+// A 2 x 2 tile of 32 x 32 MFMA blocks (acc[column block][row block], operand roles swapped: lane (l % 32, l / 32) holds row l % 32 of a
+// row block at columns 8 t + 4 (l / 32) + c) is one quantization group of 64 rows.  One v_permlane32_swap per pair of values gives lane
+// l all of row l: no trip through LDS, and the quantizer's serial sums run once.
+typedef float mfma_block_t __attribute__((ext_vector_type(16)));
+// SCALED: products are multiplied by `scale` first.  bias: of the tile's first column.  row: fp16 pairs.
+template <bool SCALED>
+__device__ __forceinline__ void tile_to_rows(const mfma_block_t (&acc)[2][2], float scale, const float *bias, int lane, uint32_t (&row)[32])
+{
+    const int lh = lane >> 5;
+    uint32_t w[2][2][8];                     // [row block, later the half][column block][pair of columns]
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float4 b = *reinterpret_cast<const float4 *>(bias + cb * 32 + 8 * t + 4 * lh);
+            const float b4[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {
+                    const float lo = acc[cb][rb][4 * t + 2 * d], hi = acc[cb][rb][4 * t + 2 * d + 1];
+                    const __half2 h = SCALED ? __floats2half2_rn(lo * scale + b4[2 * d], hi * scale + b4[2 * d + 1])
+                                             : __floats2half2_rn(lo + b4[2 * d], hi + b4[2 * d + 1]);
+                    w[rb][cb][2 * t + d] = *reinterpret_cast<const uint32_t *>(&h);
+                }
+        }
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            // The lower lanes keep row block 0 and take its other columns, the upper ones row block 1.
+            const auto r = __builtin_amdgcn_permlane32_swap(w[0][cb][i], w[1][cb][i], false, false);
+            const int pair = cb * 16 + 4 * (i >> 1) + (i & 1);
+            row[pair] = r[0], row[pair + 2] = r[1];
+        }
+}
+__device__ __forceinline__ void widen(const uint32_t *pairs, float *v, int n)
+{
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+        v[2 * i] = __half2float(__ushort_as_half(static_cast<unsigned short>(pairs[i] & 0xffffu)));
+        v[2 * i + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(pairs[i] >> 16)));
+    }
+}
+__device__ __forceinline__ uint32_t half_pair(float a, float b)
+{
+    const __half2 h = __floats2half2_rn(a, b);
+    return *reinterpret_cast<const uint32_t *>(&h);
+}
+// GELU of the row's values 8 FROM .. 8 TO.
+template <int FROM, int TO>
+__device__ __forceinline__ void gelu_pairs(uint32_t (&row)[32])
+{
+#pragma unroll
+    for (int o = FROM; o < TO; ++o) {
+        float v[8];
+        widen(row + 4 * o, v, 4);
+        gelu_of_halves(v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) row[4 * o + i] = half_pair(v[2 * i], v[2 * i + 1]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+// Stage 1 of the row's group: x_hat as fp16 pairs, or (F8) as FP8.  The whole wave calls it.
+template <int BITS, bool F8>
+__device__ __forceinline__ void quantize_row(const uint32_t (&row)[32], const QuantTables &q, float eps, uint32_t (&out)[F8 ? 16 : 32])
+{
+    float v[64];
+    widen(row, v, 32);
+    float mu, var, s, sum;
+    uint32_t none[1];
+    const BucketScale geometry = q.geometry;
+    const bool usable = q.usable != 0;
+    group_stats64(v, eps, mu, var, s);
+    group_codes64<BITS, false, 0>(v, mu, var, s, q, geometry, usable, sum, none);
+    const float code_mean = sum * 0.015625f;
+    if constexpr (F8) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t o[4];
+            xhat_fp8x16(v, 16 * i, s, code_mean, mu, o);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[4 * i + e] = o[e];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) out[i] = half_pair(fma_f32(s, v[2 * i] - code_mean, mu), fma_f32(s, v[2 * i + 1] - code_mean, mu));
+    }
+}
+
 }  // namespace arcq

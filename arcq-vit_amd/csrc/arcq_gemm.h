@@ -67,6 +67,9 @@ int device_cus();
 // Prepared operands (arcq_prepare): g.x_hat in the 32-row block layout, w_hat in the 32-column block layout; N a multiple
 // of 32, K of 64.
 void launch_gemm_tile(const GemmArgs &g, const void *w_hat, hipStream_t stream);
+// The same with the consumer's quantizer (g.next_thr) for many rows, weights resident in LDS; column blocks, fp16 or FP8.
+void launch_gemm_quant(const GemmArgs &g, const void *w_hat, hipStream_t stream);
+bool gemm_quant_pays(int64_t M, int64_t N, int64_t K, bool fp8);
 // FP8 operands, w_hat row-major [N][K rounded up to 128].
 void launch_gemm_fp8(const GemmArgs &g, const void *w_hat, hipStream_t stream);
 

@@ -499,6 +499,11 @@ ARCQ_API int arcq_prepared_row_major(int64_t M, int64_t N, int64_t K)
     return (blocks + ranges - 1) / ranges >= 5 ? 1 : 0;
 }
 
+ARCQ_API int arcq_prepared_quant_row_major(int64_t M, int64_t N, int64_t K, int fp8)
+{
+    return gemm_quant_pays(M, N, K, fp8 != 0) ? 0 : arcq_prepared_row_major(M, N, K);
+}
+
 ARCQ_API int arcq_linear_prepared(const arcq_linear_prepared_args *a, void *stream)
 {
     if (!a) return fail(ARCQ_ERR_NULL, "arcq_linear_prepared: args must not be NULL");
@@ -528,6 +533,12 @@ ARCQ_API int arcq_linear_prepared(const arcq_linear_prepared_args *a, void *stre
     if (g.fp8) {
         if (!(a->w_mult > 0.0f)) return fail(ARCQ_ERR_UNSUPPORTED, "arcq_linear_prepared: w_mult must be positive");
         g.fp8_inv = 1.0f / a->w_mult;
+    }
+    if (g.next_thr && !a->w_row_major && gemm_quant_pays(a->M, a->N, a->K, g.fp8)) {
+        launch_gemm_quant(g, a->w_hat, static_cast<hipStream_t>(stream));
+        return launch_status("arcq_linear_prepared");
+    }
+    if (g.fp8) {
         if (a->w_row_major) launch_gemm_fp8(g, a->w_hat, static_cast<hipStream_t>(stream));
         else launch_gemm_tile(g, a->w_hat, static_cast<hipStream_t>(stream));
         return launch_status("arcq_linear_prepared");

@@ -136,79 +136,6 @@ struct TileProduct {
     }
 };
 
-// fc1's tile of a wave (64 rows x 64 columns) -> GELU's input, lane l holding row l in fp16 pairs: bias, rounding.  `bias`: of the
-// tile's first column.
-__device__ __forceinline__ void tile_to_rows(const float16_t (&acc)[2][2], const float *bias, int lane, uint32_t (&out)[32])
-{
-    const int lh = lane >> 5;
-    uint32_t w[2][2][8];                     // [row block, later the half][column block][pair of columns]
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const float4 b = *reinterpret_cast<const float4 *>(bias + cb * 32 + 8 * t + 4 * lh);
-#pragma unroll
-            for (int rb = 0; rb < 2; ++rb) {
-                const __half2 lo = __floats2half2_rn(acc[cb][rb][4 * t] + b.x, acc[cb][rb][4 * t + 1] + b.y);
-                const __half2 hi = __floats2half2_rn(acc[cb][rb][4 * t + 2] + b.z, acc[cb][rb][4 * t + 3] + b.w);
-                w[rb][cb][2 * t] = *reinterpret_cast<const uint32_t *>(&lo);
-                w[rb][cb][2 * t + 1] = *reinterpret_cast<const uint32_t *>(&hi);
-            }
-        }
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            // The lower lanes keep row block 0 and take its other columns, the upper ones row block 1.
-            const auto r = __builtin_amdgcn_permlane32_swap(w[0][cb][i], w[1][cb][i], false, false);
-            const int pair = cb * 16 + 4 * (i >> 1) + (i & 1);
-            out[pair] = r[0], out[pair + 2] = r[1];
-        }
-}
-__device__ __forceinline__ void widen(const uint32_t *pairs, float *v, int n)
-{
-#pragma unroll
-    for (int i = 0; i < n; ++i) {
-        v[2 * i] = __half2float(__ushort_as_half(static_cast<unsigned short>(pairs[i] & 0xffffu)));
-        v[2 * i + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(pairs[i] >> 16)));
-    }
-}
-__device__ __forceinline__ uint32_t half_pair(float a, float b)
-{
-    const __half2 h = __floats2half2_rn(a, b);
-    return *reinterpret_cast<const uint32_t *>(&h);
-}
-// GELU of the values 8 FROM .. 8 TO of a row.
-template <int FROM, int TO>
-__device__ __forceinline__ void gelu_pairs(uint32_t (&row)[32])
-{
-#pragma unroll
-    for (int o = FROM; o < TO; ++o) {
-        float v[8];
-        widen(row + 4 * o, v, 4);
-        gelu_of_halves(v);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) row[4 * o + i] = half_pair(v[2 * i], v[2 * i + 1]);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-// The consumer's stage 1 of a row's group.
-template <int BITS>
-__device__ __forceinline__ void quantize_row(uint32_t (&row)[32], const QuantTables &q, float eps)
-{
-    float v[64];
-    widen(row, v, 32);
-    float mu, var, s, sum;
-    uint32_t none[1];
-    const BucketScale geometry = q.geometry;
-    const bool usable = q.usable != 0;
-    group_stats64(v, eps, mu, var, s);
-    group_codes64<BITS, false, 0>(v, mu, var, s, q, geometry, usable, sum, none);
-    const float code_mean = sum * 0.015625f;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) row[i] = half_pair(fma_f32(s, v[2 * i] - code_mean, mu), fma_f32(s, v[2 * i + 1] - code_mean, mu));
-}
-
 // Waits (a bounded time) until the counter shows that all workgroups have written their shares; one thread.
 __device__ __forceinline__ bool shares_written(const MlpParams &p, const unsigned long long *counter, unsigned long long target)
 {
@@ -448,7 +375,7 @@ otf_mlp_kernel(const MlpParams p)
         const bool mine = t >= 0 && t < CHUNKS && set == (t & 1);
         if (mine) {
             gelu_pairs<kEarly, 8>(pairs);
-            quantize_row<BITS>(pairs, q2, p.eps);
+            quantize_row<BITS, false>(pairs, q2, p.eps, pairs);
             fc2.start(t >= 1 ? w2 + (t - 1) * (kChunk / 64 * 4096) : w1, at, last2);      // (at t = 0 nothing: unused, but never what is not yet written)
         }
         if (t >= 1) add_chunk(t - 1);
@@ -465,7 +392,7 @@ otf_mlp_kernel(const MlpParams p)
             const char *w = w1 + static_cast<int64_t>(t + 1) * (kChunk / 32) * stride1;
             fc1.start(w, at, stride1);
             fc1.template run<2>(x_lane, w, at, stride1, tile);
-            tile_to_rows(tile, s_bias1 + (t + 1) * kChunk + (wave % kSet) * 64, lane, pairs);
+            tile_to_rows<false>(tile, 1.0f, s_bias1 + (t + 1) * kChunk + (wave % kSet) * 64, lane, pairs);
             gelu_pairs<0, kEarly>(pairs);
         } else if (t == -1) {
             rebuild_pieces<BITS, HG, 3>(p.w2, share_lo + (wave % kSet) * 64 + lane, share_hi, 64 * kSet);

@@ -720,7 +720,7 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
     Tensor qkv = empty({b, n, pq.N}, at::kHalf, x.device());
     Tensor x1 = empty(x.sizes(), at::kHalf, x.device()), y = empty(x.sizes(), at::kHalf, x.device());
     const Weights hq{at_byte(w_attn, 0), layout(pq), fp8, k.qkv.fp8_mult}, hp{at_byte(w_attn, wq), layout(pp), fp8, k.proj.fp8_mult},
-                  h1{at_byte(w_fc1, 0), layout(pf1), fp8, k.fc1.fp8_mult}, h2{at_byte(w_fc2, 0), layout(pf2), fp8, k.fc2.fp8_mult};
+                  h1{at_byte(w_fc1, 0), arcq_prepared_quant_row_major(rows, pf1.N, pf1.K, fp8 ? 1 : 0) != 0, fp8, k.fc1.fp8_mult}, h2{at_byte(w_fc2, 0), layout(pf2), fp8, k.fc2.fp8_mult};
     run_prepare(t, rows, pq, fuse_ln ? &k.fused1 : nullptr, xh.mutable_data_ptr(), hq, &pp, &hp, stream);
     run_product(pq, rows, xh.const_data_ptr(), hq, nullptr, false, nullptr, qkv.mutable_data_ptr(), ARCQ_F16, stream);
     if (own_attention) {

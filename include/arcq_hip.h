@@ -319,6 +319,8 @@ int arcq_linear_prepared(const arcq_linear_prepared_args *args, void *stream);
 /* Layout of w_hat that arcq_linear_prepared runs fastest on for these sizes: 0 = column blocks (any M), 1 = row-major
  * (the weight-stationary kernels, which want many row blocks; fp16 operands: M >= 512). */
 int arcq_prepared_row_major(int64_t M, int64_t N, int64_t K);
+/* The same where the call quantizes its output for the next layer (next_thresholds). */
+int arcq_prepared_quant_row_major(int64_t M, int64_t N, int64_t K, int fp8);
 
 /* The MLP half of a transformer block in one launch: y = x + fc2(GELU(fc1(LayerNorm(x)))), both layers packed on-the-fly layers of
  * group size 64 with `bits`-bit codes, x and y [M,K] fp16, fc1 [H,K], fc2 [K,H].  y has the bits of the two layer calls with the fused
