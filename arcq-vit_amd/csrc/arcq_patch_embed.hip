@@ -14,9 +14,11 @@
 //
 // A k-step of 16 covers half of one 16-pixel image row of a patch: the eight values a lane needs of it are 16
 // contiguous bytes of the image, so the fragments are plain 16-byte loads from the image (and from w, whose row is the
-// patch in the same order).  Two kernels: patch_embed_kernel (workgroup = 256 patches x 32 channels, weight rows in LDS)
+// patch in the same order).  Three kernels: patch_embed_kernel (workgroup = 256 patches x 32 channels, weight rows in LDS),
+// patch_embed_rows_kernel (many patches, at most 384 channels: workgroup = 64 patches x all channels, patches in LDS)
 // and, up to 256 tiles of 32 x 32, patch_embed_small_kernel (a workgroup per tile, the k-steps split over its waves).
 #include "arcq_common.h"
+#include "arcq_gemm.h"
 
 namespace arcq {
 namespace {
@@ -143,6 +145,139 @@ patch_embed_kernel(const __half *__restrict__ img, const __half *__restrict__ w,
     }
 }
 
+// The same for many patches and at most 384 channels: a workgroup owns 64 patches and all channels.  Above, every 32-channel tile reads
+// the image again, and 64 images cost 173 MB of traffic for the 29 that they are; here the patches lie in LDS (64 x 768 values, read
+// once, in runs of a row's patches), and the weights stream through it 32 values at a time, one barrier a chunk: the next chunk is
+// written to the other buffer while later ones are on their way from L2.  Wave = 64 patches x 32 channels (32 x 32 where there are no
+// more than six such tiles).  What bounds it is the LDS: 3 KB of reads and 1 of writes for two MFMAs, 15 us for 384 channels however
+// few the workgroups; a second pass for more channels loses (768 of 64 images 41 us against 40, of 256 162 / 144).
+// 64 images, 384 channels 31.0 -> 21.7 us, 192 channels 24.7 -> 15.8; 256 images 101 -> 90 and 69 -> 63.
+constexpr int kRowsWaves = 12, kChunkK = 32, kChunks = kK / kChunkK;      // 24
+constexpr int kAPitch = kK * 2 + 16, kBPitch = kChunkK * 2 + 16;          // bytes; odd numbers of 16-byte pieces
+constexpr int kRowsN = 32 * kRowsWaves;                                   // the most channels
+constexpr int kBBytes = kRowsN * kBPitch;
+constexpr int kAheadB = 4;                                                // chunks on their way from L2 or in a buffer
+constexpr int kRowsLds = 64 * kAPitch + 2 * kBBytes;
+
+__global__ void __launch_bounds__(64 * kRowsWaves)
+patch_embed_rows_kernel(const __half *__restrict__ img, const __half *__restrict__ w, const __half *__restrict__ bias,
+                        const __half *__restrict__ cls, const __half *__restrict__ pos, __half *__restrict__ out, int B, int H,
+                        int W, int N, int row_tiles)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    unsigned char *as = smem, *bs = smem + 64 * kAPitch;
+    constexpr int kThreads = 64 * kRowsWaves;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 31, lh = lane >> 5;
+    const int pw = W / kPatch, np = (H / kPatch) * pw;
+    const int M = B * np;
+    if (static_cast<int>(blockIdx.x) >= row_tiles) {        // the class-token rows: element e = b * N + n
+        const int64_t e0 = (static_cast<int64_t>(blockIdx.x - row_tiles) * kThreads + tid) * 8;
+        if (e0 < static_cast<int64_t>(B) * N) {
+            const int b = static_cast<int>(e0 / N), n = static_cast<int>(e0 - static_cast<int64_t>(b) * N);
+            __half *dst = out + static_cast<int64_t>(b) * (np + 1) * N + n;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) dst[i] = __float2half_rn(__half2float(cls[n + i]) + __half2float(pos[n + i]));
+        }
+        return;
+    }
+    const int m0 = blockIdx.x * 64;
+    // ---- the weights' first two chunks and the patches: 48 image rows x 64 patches x 2 pieces, eight a thread, all in flight.
+    // Neighbouring threads take neighbouring patches of one image row. ----
+    u32x4_t bt[kAheadB][2];
+    auto fetch_b = [&](int c, u32x4_t (&t)[2]) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int p = tid + kThreads * j, row = p >> 2, piece = p & 3;
+            t[j] = *reinterpret_cast<const u32x4_t *>(w + static_cast<int64_t>(min(row, N - 1)) * kK + c * kChunkK + piece * 8);
+        }
+    };
+    auto store_b = [&](int buf, const u32x4_t (&t)[2]) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int p = tid + kThreads * j;
+            *reinterpret_cast<u32x4_t *>(bs + buf * kBBytes + (p >> 2) * kBPitch + (p & 3) * 16) = t[j];
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < kAheadB; ++c) fetch_b(c, bt[c]);
+    {
+        const int pl = (tid >> 1) & 63, h = tid & 1;
+        const int mc = min(m0 + pl, M - 1), b = mc / np, p = mc - b * np, py = p / pw, px = p - py * pw;
+        const __half *src = img + (static_cast<int64_t>(b) * kChannels * H + py * kPatch) * W + px * kPatch + h * 8;
+        u32x4_t at[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int ci = (tid >> 7) + 6 * j, c = ci >> 4, i = ci & 15;      // 768 threads: six image rows a round
+            at[j] = *reinterpret_cast<const u32x4_t *>(src + (static_cast<int64_t>(c) * H + i) * W);
+        }
+        store_b(0, bt[0]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) *reinterpret_cast<u32x4_t *>(as + pl * kAPitch + ((tid >> 7) + 6 * j) * 32 + h * 16) = at[j];
+    }
+    int64_t out_row[2];
+    int pos_row[2];
+    bool valid[2];
+#pragma unroll
+    for (int tm = 0; tm < 2; ++tm) {
+        const int m = m0 + tm * 32 + lr, mc = min(m, M - 1), b = mc / np, p = mc - b * np;
+        out_row[tm] = static_cast<int64_t>(b) * (np + 1) + 1 + p;
+        pos_row[tm] = 1 + p;
+        valid[tm] = m < M;
+    }
+    const unsigned char *a_lane = as + lr * kAPitch + lh * 16;
+    const int tiles = N / 32;
+    const bool halves = tiles <= kRowsWaves / 2;             // two waves a tile, a row block each
+    const int ct = halves ? wave % (kRowsWaves / 2) : wave, tm0 = halves ? wave / (kRowsWaves / 2) : 0;
+    float16_t acc[2];
+#pragma unroll
+    for (int tm = 0; tm < 2; ++tm)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[tm][v] = 0.0f;
+    const unsigned char *b_lane = bs + (ct * 32 + lr) * kBPitch + lh * 16;
+#pragma unroll 4
+    for (int c = 0; c < kChunks; ++c) {
+        __syncthreads();                                     // chunk c is in buffer c & 1, chunk c - 1 has been read
+        store_b((c + 1) & 1, bt[(c + 1) % kAheadB]);
+        fetch_b(min(c + kAheadB, kChunks - 1), bt[c % kAheadB]);
+#pragma unroll
+        for (int s = 0; s < kChunkK / 16; ++s) {
+            const half8_t wb = *reinterpret_cast<const half8_t *>(b_lane + (c & 1) * kBBytes + s * 32);
+            const half8_t x0 = *reinterpret_cast<const half8_t *>(a_lane + tm0 * 32 * kAPitch + (c * 2 + s) * 32);
+            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wb, x0, acc[0], 0, 0, 0);
+            if (!halves) {
+                const half8_t x1 = *reinterpret_cast<const half8_t *>(a_lane + 32 * kAPitch + (c * 2 + s) * 32);
+                acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wb, x1, acc[1], 0, 0, 0);
+            }
+        }
+    }
+    // acc[tm][v]: patch lr of row block tm, channel 8 (v / 4) + 4 lh + v % 4 of the tile
+    if (ct >= tiles) return;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if (i == 1 && halves) break;
+        const int tm = halves ? tm0 : i;
+        if (!(tm ? valid[1] : valid[0])) continue;
+        __half *dst = out + (tm ? out_row[1] : out_row[0]) * N;
+        const __half *ps = pos + static_cast<int64_t>(tm ? pos_row[1] : pos_row[0]) * N;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int n = ct * 32 + 8 * q + 4 * lh;
+            const u32x2_t pv = *reinterpret_cast<const u32x2_t *>(ps + n);
+            u32x2_t bv = {0u, 0u};
+            if (bias) bv = *reinterpret_cast<const u32x2_t *>(bias + n);
+            const __half *ph = reinterpret_cast<const __half *>(&pv), *bh = reinterpret_cast<const __half *>(&bv);
+            __half o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const __half y = __float2half_rn(acc[i][4 * q + e] + __half2float(bh[e]));
+                o[e] = __float2half_rn(__half2float(y) + __half2float(ph[e]));
+            }
+            *reinterpret_cast<u32x2_t *>(dst + n) = *reinterpret_cast<const u32x2_t *>(o);
+        }
+    }
+}
+
 // The same for few patches (batch 1-2): one 32 x 32 tile per workgroup, its 48 k-steps dealt to the four waves (twelve
 // each, all 24 fragment loads of a wave in flight at once: the launch is one memory latency, twelve MFMAs and a
 // reduction of the four partial tiles through LDS, in wave order).
@@ -252,6 +387,13 @@ ARCQ_API int arcq_patch_embed_fwd(const void *img, const void *w, const void *bi
         const int row_tiles = static_cast<int>((M + 31) / 32);
         hipLaunchKernelGGL(patch_embed_small_kernel, dim3(row_tiles * col_tiles + cls_wgs), dim3(256), 0, st, pi, pwt, pb, pc, pp, po,
                            b, h, wd, n, row_tiles, col_tiles);
+    } else if (n <= kRowsN && (M + 63) / 64 * 8 >= device_cus() * 5) {
+        // Its workgroups take as long however few they are: from five eighths of the compute units on (98 of them, 32 images: 20.1 us
+        // against 20.4 at 384 channels, 15.4 / 12.7 at 192; 332: 43 / 44 and 31 / 33).
+        allow_dynamic_lds<patch_embed_rows_kernel>(kRowsLds);
+        const int row_tiles = static_cast<int>((M + 63) / 64);
+        hipLaunchKernelGGL(patch_embed_rows_kernel, dim3(row_tiles + (cls_wgs + 2) / 3), dim3(64 * kRowsWaves), kRowsLds, st, pi, pwt, pb, pc, pp, po,
+                           b, h, wd, n, row_tiles);
     } else {
         const int row_groups = static_cast<int>((M + 128 * kTM - 1) / (128 * kTM));      // four waves of 32 kTM patches
         hipLaunchKernelGGL(patch_embed_kernel, dim3(row_groups * col_tiles + cls_wgs), dim3(256), 0, st, pi, pwt, pb, pc, pp, po, b, h, wd,

@@ -98,3 +98,10 @@ def test_vit_with_own_patch_embed(cuda, model, batch):
     assert float((seen[0].float() - seen[1].float()).abs().max()) <= 2.0 ** -8
     cos = torch.nn.functional.cosine_similarity(a.float().flatten(), b.float().flatten(), dim=0).item()
     assert cos > 0.99, cos
+
+
+@pytest.mark.parametrize("b,h,w,n,with_bias", [(53, 224, 224, 192, True), (161, 128, 128, 32, False), (54, 208, 240, 224, True),
+                                               (215, 112, 112, 384, False)])
+def test_patch_embed_of_many_patches(cuda, b, h, w, n, with_bias):
+    """The kernel that keeps 64 patches in LDS: ragged last tiles, one tile of channels to all twelve, up to six and more than six."""
+    test_patch_embed_matches_float64(cuda, b, h, w, n, with_bias)
