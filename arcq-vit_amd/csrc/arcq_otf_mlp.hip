@@ -355,7 +355,8 @@ otf_mlp_kernel(const MlpParams p)
     const unsigned char *h_lane = hs + lr * kHiddenPitch + lh * 64;
     const uint32_t at = lh * 2048 + lr * 16;
     const char *w1 = reinterpret_cast<const char *>(p.w1.out) + (wave % kSet) * 2 * stride1;
-    const char *w2 = reinterpret_cast<const char *>(p.w2.out) + static_cast<int64_t>(wave) * (H * 64);
+    // (K = 192: six blocks.  The last two waves use none, but request one with the others.)
+    const char *w2 = reinterpret_cast<const char *>(p.w2.out) + static_cast<int64_t>(BLOCKS < kWaves ? min(wave, BLOCKS - 1) : wave) * (H * 64);
     const int blocks = (BLOCKS - wave + kWaves - 1) / kWaves;                // of fc2's columns: wave, wave + 8, ...
     float16_t acc[NB][2];
 #pragma unroll
