@@ -43,7 +43,11 @@ constexpr int kKPitch = kHeadDim * 2 + 16;          // bytes per key row of K in
 // lane-pair routine of the GEMM epilogues.
 // F8: that operand as FP8 (rows padded to 128 values).
 // SPLIT: a head has gridDim.z workgroups.  (A template: the two registers that it takes cost 5 % at 256 images of 16 heads.)
-template <int NKB, int NQ, bool F8, bool SPLIT>
+// FEW: the last key block holds at most eight keys (197 or 101 tokens: five).  The other 24 would get scores of minus infinity and
+// probabilities of zero: no maximum, no exponentials, no second half of the product.  197 tokens (the vector instructions bound it, a
+// tenth of them are gone): 64 images of 6 heads 17.8 -> 16.9 us, of 12 28.7 -> 27.9, 256 of 16 with proj's stage 1 137 -> 133, one of 6
+// 7.1 -> 6.9.  A template: as a branch on the number of keys it spills 13 to 69 registers.
+template <int NKB, int NQ, bool F8, bool SPLIT, bool FEW>
 __global__ void __launch_bounds__(64 * NKB) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 : 4)))     // two workgroups of up to 8 waves on a CU, or one
 attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n, int H, float scale,
                  const float *__restrict__ nq_thr, const float *__restrict__ nq_cb, int total_rows)
@@ -151,6 +155,7 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
             // only the last key block can hold keys past n)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
+                if (FEW && kb == NKB - 1 && v >= 4) break;
                 if (kb == NKB - 1) {
                     const int key = kb * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
                     acc[i][v] = key < n ? acc[i][v] : ninf;
@@ -177,12 +182,17 @@ attention_kernel(const __half *__restrict__ qkv, __half *__restrict__ out, int n
             const int kb = ch * CH + i;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
+                if (FEW && kb == NKB - 1 && v >= 4) {
+                    acc[i][v] = 0.0f;
+                    continue;
+                }
                 const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[i][v], c2, mc));      // exp(scale (s - m))
                 acc[i][v] = p;
                 l += p;
             }
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
+                if (FEW && kb == NKB - 1 && s == 1) break;
                 half8_t pf;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) pf[e] = static_cast<_Float16>(acc[i][8 * s + e]);
@@ -303,7 +313,9 @@ void launch_attention(const void *qkv, void *out, int B, int n, int H, float sca
     // heads with that stage 1: 9.5 us in one part, 6.5 in seven; 16 images 9.9 and 7.7 in two parts.
     const int64_t heads = static_cast<int64_t>(B) * H;
     const int parts = static_cast<int>(std::min<int64_t>(NKB, std::max<int64_t>(1, device_cus() / heads)));
-    auto kernel = NKB > 1 && parts > 1 ? attention_kernel<NKB, NQ, F8, (NKB > 1)> : attention_kernel<NKB, NQ, F8, false>;
+    const bool few = n - 32 * (NKB - 1) <= 8;
+    auto kernel = NKB > 1 && parts > 1 ? (few ? attention_kernel<NKB, NQ, F8, (NKB > 1), true> : attention_kernel<NKB, NQ, F8, (NKB > 1), false>)
+                                       : (few ? attention_kernel<NKB, NQ, F8, false, true> : attention_kernel<NKB, NQ, F8, false, false>);
     hipLaunchKernelGGL(kernel, dim3(H, B, parts), dim3(64 * NKB), 0, stream, static_cast<const __half *>(qkv),
                        static_cast<__half *>(out), n, H, scale, thr, cb, B * n);
 }

@@ -110,3 +110,16 @@ def test_parts_of_a_head(cuda, b, n, h):
     many = -(-260 // h) + b
     qkv = torch.randn(many, n, 3 * h * 64, generator=torch.Generator().manual_seed(n)).half().to(cuda)
     assert torch.equal(ops.attention_fwd(qkv[:b].contiguous(), h), ops.attention_fwd(qkv, h)[:b])
+
+
+@pytest.mark.parametrize("n", [5, 8, 9, 33, 40, 41, 101, 104, 105, 197, 200, 201, 232, 233])
+def test_last_key_block_of_few_keys(cuda, n):
+    """At most eight keys in the last block have kernels of their own: both sides of that line, keys that dominate in it and negative
+    scores throughout (a zero score, which padding has, would win)."""
+    heads = 2
+    qkv = torch.randn(3, n, 3, heads, 64, generator=torch.Generator().manual_seed(n))
+    qkv[0, -1, 1] *= 5.0
+    qkv[1, :, 0] = qkv[1, :, 0].abs()
+    qkv[1, :, 1] = -qkv[1, :, 1].abs()
+    qkv = qkv.reshape(3, n, 3 * heads * 64).half().to(cuda)
+    _check(qkv, heads)
