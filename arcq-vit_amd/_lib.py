@@ -78,7 +78,7 @@ class MlpArgs(ctypes.Structure):
     """``arcq_mlp_args``."""
     _fields_ = [("bits", ctypes.c_int32), ("eps", ctypes.c_float), ("ln_eps", ctypes.c_float)] + [
         (n, ctypes.c_int64) for n in ("M", "K", "H")] + [(n, ctypes.c_void_p) for n in ("x", "ln_weight", "ln_bias")] + [
-        ("fc1", MlpLayer), ("fc2", MlpLayer), ("y", ctypes.c_void_p)]
+        ("fc1", MlpLayer), ("fc2", MlpLayer), ("y", ctypes.c_void_p), ("attn", ctypes.c_void_p), ("proj", MlpLayer)]
 
 
 ARCQ_PRODUCER_NONE, ARCQ_PRODUCER_LAYERNORM, ARCQ_PRODUCER_XHAT = 0, 1, 2

@@ -688,11 +688,12 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
     for (const Plan *p : {&pq, &pp, &pf1, &pf2})
         if (!can_prepare(*p, rows) || p->bits != pq.bits) return std::nullopt;
     // Not where the one-launch kernels are at their best (one 64-row tile on most compute units, short rows).  With the LayerNorms
-    // inside, hidden rows of four times the width and lent weight buffers, the block is four launches there, the last of them the
-    // whole MLP: a block of DeiT-S at 11 032 rows 111 us against 124, at 16 351 127 / 141, DeiT-B 260 / 287 and 316 / 372, DeiT-Tiny at
-    // 12 608 rows 69 / 79; at 9 456 rows 110 / 106, 250 / 242 and 66 / 64, below that the seven launches win by more, and with more row
-    // tiles than compute units they win too (DeiT-Tiny at 19 700 rows 99 against 112).  Without the one-launch MLP 9 000 rows: DeiT-S at
-    // 12 608 rows 1 625 us a forward against 1 939 (five launches a block), at 6 304 rows 1 353 -> 1 262.
+    // inside, hidden rows of four times the width and lent weight buffers, the block is three launches there, the last of them proj and
+    // the whole MLP.  Forwards against the seven launches: DeiT-S 10 047 rows 1 336 us against 1 271, 10 638 1 346 / 1 344, 11 032 1 344 /
+    // 1 529 (a round of 128-row tiles more), 12 608 1 381; DeiT-B 10 638 3 117 / 3 038, 11 032 3 160 / 3 342; DeiT-Tiny 6 304 718 / 685,
+    // 7 092 726 / 748, 9 259 763 / 783; with more row tiles than compute units the seven win (a block of DeiT-Tiny at 19 700 rows 99
+    // against 112).  Without the one-launch MLP 9 000 rows: DeiT-S at 12 608 rows 1 625 us a forward against 1 939 (five launches a
+    // block), at 6 304 rows 1 353 -> 1 262.
     // With torch's LayerNorms and GELU those kernels run only on lent weight buffers, and win later and only beside torch's
     // attention: 10 638 rows DeiT-S 2 311 us against 2 264 here, DeiT-B 4 498 / 4 406, 11 032 rows 2 318 / 2 439 and 4 607 / 4 879,
     // 12 608 rows 2 399 / 2 564 and 4 892 / 5 147; without lent buffers (two launches a layer) 2 667 / 2 590 and 5 207 / 5 178, with
@@ -739,27 +740,37 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
 }
 
 // The block's second half, x + fc2(GELU(fc1(LayerNorm(x)))), in one launch; nullopt before it where that does not serve or pay.
-std::optional<Tensor> run_mlp(const Layer &fc1, const Layer &fc2, const FusedLayerNorm &ln, const Tensor &x)
+// With `attn`, attention's output, x + proj(attn) takes the place of x, in the same launch.
+std::optional<Tensor> run_mlp(const Layer &fc1, const Layer &fc2, const FusedLayerNorm &ln, const Tensor &x, const Layer *proj = nullptr,
+                              const Tensor *attn = nullptr)
 {
     const Plan &p1 = *fc1.plan, &p2 = *fc2.plan;
     const int64_t rows = x.numel() / p1.K;
-    if (!arcq_mlp_otf_pays(rows, p1.K, p1.N) || !fc1.lends || !fc2.lends || !lent(fc1.weight_buffer, p1.N * p1.K, x)) return std::nullopt;
-    if (p1.bits != p2.bits || p1.gs != 64 || p2.gs != 64 || fc1.fp8 || fc2.fp8 || fc1.out != at::kHalf || fc2.out != at::kHalf) return std::nullopt;
-    if (!takes(fc1, x) || !f16(x) || p2.K != p1.N || p2.N != p1.K || p2.device != p1.device || !aligned16(x) || !aligned16(ln.weight) ||
-        !aligned16(ln.bias))
+    if (!arcq_mlp_otf_pays(rows, p1.K, p1.N) || !lent(fc1.weight_buffer, p1.N * p1.K, x)) return std::nullopt;
+    if (!takes(fc1, x) || !f16(x) || p2.K != p1.N || p2.N != p1.K || !aligned16(x) || !aligned16(ln.weight) || !aligned16(ln.bias))
         return std::nullopt;
-    const Tensor w2 = empty({p2.N * p2.K}, at::kHalf, x.device());
-    void *const ws[2] = {fc1.weight_buffer->mutable_data_ptr(), w2.mutable_data_ptr()};
+    if (attn && (!takes(*proj, *attn) || !f16(*attn) || attn->numel() != x.numel() || proj->plan->K != p1.K || proj->plan->N != p1.K ||
+                 !aligned16(*attn)))
+        return std::nullopt;
+    const Layer *const layers[3] = {&fc1, &fc2, proj};
+    const int count = attn ? 3 : 2;
+    for (int i = 0; i < count; ++i) {
+        const Layer &l = *layers[i];
+        if (!l.lends || l.fp8 || l.out != at::kHalf || l.plan->gs != 64 || l.plan->bits != p1.bits || l.plan->device != p1.device) return std::nullopt;
+    }
+    const Tensor others = empty({p2.N * p2.K + (attn ? p1.K * p1.K : 0)}, at::kHalf, x.device());      // (layers may share the buffer they lend)
+    char *const w2 = static_cast<char *>(others.mutable_data_ptr());
+    void *const ws[3] = {fc1.weight_buffer->mutable_data_ptr(), w2, w2 + 2 * p2.N * p2.K};
     arcq_mlp_args a = {};
     a.bits = static_cast<int32_t>(p1.bits);
     a.eps = 1.0e-6f, a.ln_eps = ln.eps;
     a.M = rows, a.K = p1.K, a.H = p1.N;
     a.x = x.const_data_ptr();
+    a.attn = attn ? attn->const_data_ptr() : nullptr;
     a.ln_weight = ln.weight, a.ln_bias = ln.bias;
-    arcq_mlp_layer *const l[2] = {&a.fc1, &a.fc2};
-    const Plan *const plans[2] = {&p1, &p2};
-    for (int i = 0; i < 2; ++i) {
-        const auto *p = plans[i]->p;
+    arcq_mlp_layer *const l[3] = {&a.fc1, &a.fc2, &a.proj};
+    for (int i = 0; i < count; ++i) {
+        const auto *p = layers[i]->plan->p;
         auto fp = [&](int j) { return static_cast<const float *>(p[j]); };
         if (reinterpret_cast<uintptr_t>(p[W_PACKED]) % 4 != 0 || reinterpret_cast<uintptr_t>(ws[i]) % 128 != 0) return std::nullopt;
         *l[i] = arcq_mlp_layer{fp(A_THR), fp(A_CB), static_cast<const uint8_t *>(p[W_PACKED]), fp(W_CB), fp(W_CENTER), fp(W_SCALE), fp(W_SUM),
@@ -788,6 +799,10 @@ std::optional<Tensor> run_block(const BlockParts &k, const Tensor &x, bool chain
         auto t = run_layer(k.qkv, x, o1);
         if (!t) return std::nullopt;
         const Tensor a = as_operand(mix(*t, k.heads, k.own));
+        if (chain) {
+            auto y = run_mlp(k.fc1, k.fc2, k.fused2, x, &k.proj, &a);
+            if (y) return y;
+        }
         Options o2;
         o2.residual = &x;
         auto x1 = run_layer(k.proj, a, o2);

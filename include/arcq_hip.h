@@ -324,7 +324,8 @@ int arcq_prepared_quant_row_major(int64_t M, int64_t N, int64_t K, int fp8);
 
 /* The MLP half of a transformer block in one launch: y = x + fc2(GELU(fc1(LayerNorm(x)))), both layers packed on-the-fly layers of
  * group size 64 with `bits`-bit codes, x and y [M,K] fp16, fc1 [H,K], fc2 [K,H].  y has the bits of the two layer calls with the fused
- * options (arcq_linear_otf_ex).  Each layer brings a workspace of H*K fp16 values; calls that share fc1's must not overlap. */
+ * options (arcq_linear_otf_ex).  Each layer brings a workspace
+ * for its weights in fp16; calls that share fc1's must not overlap.  y is no other tensor of the call. */
 typedef struct arcq_mlp_layer {
     const float *a_thresholds, *a_codebook;
     const uint8_t *packed_w;
@@ -339,6 +340,8 @@ typedef struct arcq_mlp_args {
     const float *ln_weight, *ln_bias;
     arcq_mlp_layer fc1, fc2;
     void *y;
+    const void *attn;             /* NULL, or [M,K] fp16: x + proj(attn) takes the place of x (proj [K,K], a layer like the others) */
+    arcq_mlp_layer proj;
 } arcq_mlp_args;
 int arcq_mlp_otf(const arcq_mlp_args *args, void *stream);
 /* Whether it serves these sizes (ARCQ_ERR_UNSUPPORTED otherwise): K = 192, 256, 384 or 768, H = 4 K, 512 rows up to 64 per compute unit. */

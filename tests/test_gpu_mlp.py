@@ -28,9 +28,9 @@ def _layer(cuda, n, k, bits, gen, bias=True, thresholds=None):
     return layer
 
 
-def _one_launch(x, norm, fc1, fc2):
+def _one_launch(x, norm, fc1, fc2, proj=None, attn=None):
     k, h = x.shape[1], fc1.out_features
-    ws = [torch.empty(h * k, dtype=torch.float16, device=x.device) for _ in range(2)]
+    ws = [torch.empty(n * k, dtype=torch.float16, device=x.device) for n in (h, h, k)]
     y = torch.empty_like(x)
     keep = []
 
@@ -43,7 +43,8 @@ def _one_launch(x, norm, fc1, fc2):
 
     g, b = norm.weight.float().contiguous(), norm.bias.float().contiguous()
     a = _lib.MlpArgs(fc1.bits, 1.0e-6, norm.eps, x.shape[0], k, h, x.data_ptr(), g.data_ptr(), b.data_ptr(), part(fc1, ws[0]),
-                     part(fc2, ws[1]), y.data_ptr())
+                     part(fc2, ws[1]), y.data_ptr(), None if attn is None else attn.data_ptr(),
+                     part(proj, ws[2]) if proj is not None else _lib.MlpLayer())
     lib = _lib.load()
     rc = lib.arcq_mlp_otf(ctypes.byref(a), torch.cuda.current_stream().cuda_stream)
     assert rc == 0, lib.arcq_last_error()
@@ -93,6 +94,40 @@ def test_one_launch_mlp_has_the_bits_of_the_two_layers(cuda, monkeypatch, m, k, 
         h = fc1(x, layernorm=norm, activation="gelu")
         want = fc2(h, residual=x)
     # (a NaN's payload is nobody's contract)
+    same = (y.view(torch.int16) == want.view(torch.int16)) | (torch.isnan(y) & torch.isnan(want))
+    assert bool(same.all()), int((~same).sum())
+    if case != "inf":
+        assert bool(torch.isfinite(y).all())
+
+
+@pytest.mark.parametrize("m,k,bits,case", [(512, 192, 4, ""), (705, 192, 2, "no wait"), (1001, 256, 3, "no bias"), (12608, 384, 4, ""),
+                                           (767, 384, 3, "thresholds"), (1000, 384, 2, "inf"), (513, 768, 4, ""), (12608, 768, 4, ""),
+                                           (2047, 768, 3, "zeros"), (700, 768, 2, "no wait")])
+def test_one_launch_with_proj_has_the_bits_of_the_three_layers(cuda, monkeypatch, m, k, bits, case):
+    """The same with proj and the first skip connection in front: attention's output in, its own quantizer tables, the rows that the
+    LayerNorm reads come from the product before it."""
+    gen = torch.Generator().manual_seed(11 * m + k)
+    thr = None
+    if case == "thresholds":
+        thr = synth.midpoint_thresholds(synth.quantile_codebook(bits)).clone()
+        thr[3] = thr[4]
+    proj = _layer(cuda, k, k, bits, gen, case != "no bias", thr)
+    fc1, fc2 = _layer(cuda, 4 * k, k, bits, gen), _layer(cuda, k, 4 * k, bits, gen)
+    norm = _norm(cuda, k, gen)
+    x = torch.randn(m, k, generator=gen) * (1.0 + 3.0 * torch.rand(m, 1, generator=gen))
+    attn = torch.randn(m, k, generator=gen)
+    if case == "zeros":
+        attn[5:70] = 0.0
+    if case == "inf":
+        attn[3, 7] = float("inf")
+        x[65, 2] = float("-inf")
+    x, attn = x.half().to(cuda), attn.half().to(cuda)
+    if case == "no wait":
+        monkeypatch.setenv("ARCQ_ROWS_WAIT_TICKS", "0")
+    y = _one_launch(x, norm, fc1, fc2, proj, attn)
+    with torch.no_grad():
+        x1 = proj(attn, residual=x)
+        want = fc2(fc1(x1, layernorm=norm, activation="gelu"), residual=x1)
     same = (y.view(torch.int16) == want.view(torch.int16)) | (torch.isnan(y) & torch.isnan(want))
     assert bool(same.all()), int((~same).sum())
     if case != "inf":
