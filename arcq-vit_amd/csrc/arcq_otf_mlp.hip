@@ -26,7 +26,7 @@
 // 3 364 us); K = 384 29 + 39 -> 68 (1 559 -> 1 470); K = 192 -> 34 (a block 79 -> 69).  Clocks of a workgroup at K = 768, 320 000 in
 // all: set-up 19 000 (x from memory, shares of weights), LayerNorm and stage 1 33 000 (vector ALU, on two waves a SIMD), thirteen steps
 // of 17 000 each, output 12 000.  In a step the quantizing wave takes 3 300 for the rest of GELU, 8 800 for the quantizer and 3 800 for
-// fc2's 96 MFMAs (3 072 at full rate), its partner 3 500 for those, 7 600 for fc1's 192 (6 144) and 4 000 for the first half of GELU: a
+// fc2's 96 MFMAs (3 072 at full rate), its partner 3 500 for those, 7 600 for fc1's 192 (6 144) and 4 000 for the first half of GELU (now three eighths): a
 // wave alone issues a vector instruction every five clocks or so, and the other's MFMAs take about eight of them each.
 //
 // Weights: rebuilt by the launch's workgroups between them, as in arcq_otf_rows.hip (proj's and fc1's together); fc2's under
@@ -471,7 +471,9 @@ otf_mlp_kernel(const MlpParams p)
     // ---- the chunks.  Step t: one set quantizes chunk t of the hidden row, then adds chunk t - 1 to fc2's sums; the other one adds
     // chunk t - 1, multiplies chunk t + 1 of fc1 and takes the first kEarly eighths of its GELU, so that both are done at about the
     // same time and the matrix units and vector ALUs of every SIMD have work side by side.  Then they change places. ----
-    constexpr int kEarly = G >= 12 ? 4 : 8;
+    // (Beside 4 and 8, from before the quantizer's lookups had constant addresses: base model at 64 images 3 389 -> 3 369 us, 3 442 with
+    // five eighths; small model 1 400 -> 1 394.)
+    constexpr int kEarly = G >= 12 ? 3 : 5;
     constexpr int64_t stride1 = static_cast<int64_t>(K) * 64, stride2 = static_cast<int64_t>(kWaves) * H * 64;
     const unsigned char *h_lane = hs + lr * kHiddenPitch + lh * 64;
     const char *w1 = reinterpret_cast<const char *>(p.w1.out) + (wave % kSet) * 2 * stride1;
