@@ -15,7 +15,7 @@
 // A k-step of 16 covers half of one 16-pixel image row of a patch: the eight values a lane needs of it are 16
 // contiguous bytes of the image, so the fragments are plain 16-byte loads from the image (and from w, whose row is the
 // patch in the same order).  Three kernels: patch_embed_kernel (workgroup = 256 patches x 32 channels, weight rows in LDS),
-// patch_embed_rows_kernel (many patches, at most 384 channels: workgroup = 64 patches x all channels, patches in LDS)
+// patch_embed_rows_kernel (many patches, 128 to 384 channels: workgroup = 64 patches x all channels, patches in LDS; patch_rows_pay)
 // and, up to 256 tiles of 32 x 32, patch_embed_small_kernel (a workgroup per tile, the k-steps split over its waves).
 #include "arcq_common.h"
 #include "arcq_gemm.h"
@@ -145,7 +145,7 @@ patch_embed_kernel(const __half *__restrict__ img, const __half *__restrict__ w,
     }
 }
 
-// The same for many patches and at most 384 channels: a workgroup owns 64 patches and all channels.  Above, every 32-channel tile reads
+// The same for many patches and 128 to 384 channels: a workgroup owns 64 patches and all channels.  Above, every 32-channel tile reads
 // the image again, and 64 images cost 173 MB of traffic for the 29 that they are; here the patches lie in LDS (64 x 768 values, read
 // once, in runs of a row's patches), and the weights stream through it 32 values at a time, one barrier a chunk: the next chunk is
 // written to the other buffer while later ones are on their way from L2.  Wave = 64 patches x 32 channels (32 x 32 where there are no
@@ -182,7 +182,7 @@ patch_embed_rows_kernel(const __half *__restrict__ img, const __half *__restrict
         return;
     }
     const int m0 = blockIdx.x * 64;
-    // ---- the weights' first two chunks and the patches: 48 image rows x 64 patches x 2 pieces, eight a thread, all in flight.
+    // ---- the weights' first four chunks and the patches: 48 image rows x 64 patches x 2 pieces, eight a thread, all in flight.
     // Neighbouring threads take neighbouring patches of one image row. ----
     u32x4_t bt[kAheadB][2];
     auto fetch_b = [&](int c, u32x4_t (&t)[2]) {
@@ -356,6 +356,25 @@ patch_embed_small_kernel(const __half *__restrict__ img, const __half *__restric
     }
 }
 
+// Where patch_embed_rows_kernel is the faster one.  Its workgroups have a compute unit each, so it takes whole rounds of them, about
+// 2 N / 32 + 3 parts a round (the channels, the patches); the other kernel's (256 patches x 32 channels) are a sixth to a fifth of a
+// round and several share a compute unit.  Measured at 160 to 1 500 tiles of 64 patches, 224 x 224 and 128 x 128 images, us here / there:
+//   one round      384 channels, 160 tiles 20.4 / 23.5, 224 22.7 / 32.2; 192: 14.9 / 17.6, 15.7 / 25.7; 128: 13.6 / 13.6, 14.5 / 16.8;
+//                  96: 12.9 / 11.2, 13.6 / 13.6; fewer tiles: 384 channels, 98 tiles 20.1 / 20.4, 192 15.4 / 12.7
+//   a second begun 257 tiles: 384 channels 39.1 / 37.2, 320 36.8 / 34.3, 256 33.8 / 35.8, 224 31.6 / 28.4, 192 28.1 / 25.9, 160 26.4 / 24.2;
+//                  304: 42.1 / 42.1, 38.6 / 39.0, 35.4 / 40.0, 32.9 / 38.5, 29.9 / 29.3, 27.9 / 26.2; 350: 42.8 / 50.7, 39.2 / 47.0,
+//                  35.8 / 42.6, 33.3 / 40.0, 30.4 / 38.9, 28.6 / 28.3; 512: 52.5 / 65.1, 192 channels 36.7 / 46.3
+//   more           513: 63.7 / 66.0, 192 channels 45.7 / 49.4, 160 42.6 / 39.6; 784: 90.5 / 101, 63.2 / 69.3, 59.0 / 58.4
+bool patch_rows_pay(int64_t M, int64_t n)
+{
+    const int64_t cus = device_cus(), tiles = (M + 63) / 64;
+    if (n < 128 || n > kRowsN || tiles * 8 < cus * 5) return false;
+    const int64_t rounds = (tiles + cus - 1) / cus;
+    if (rounds == 1) return true;
+    const int64_t groups = (M + 128 * kTM - 1) / (128 * kTM), others = (groups * (n / 32) + cus - 1) / cus;      // the other kernel's on a compute unit
+    return n >= 160 && 5 * rounds * (2 * (n / 32) + 3) <= 64 * others;
+}
+
 }  // namespace
 }  // namespace arcq
 
@@ -387,9 +406,7 @@ ARCQ_API int arcq_patch_embed_fwd(const void *img, const void *w, const void *bi
         const int row_tiles = static_cast<int>((M + 31) / 32);
         hipLaunchKernelGGL(patch_embed_small_kernel, dim3(row_tiles * col_tiles + cls_wgs), dim3(256), 0, st, pi, pwt, pb, pc, pp, po,
                            b, h, wd, n, row_tiles, col_tiles);
-    } else if (n <= kRowsN && (M + 63) / 64 * 8 >= device_cus() * 5) {
-        // Its workgroups take as long however few they are: from five eighths of the compute units on (98 of them, 32 images: 20.1 us
-        // against 20.4 at 384 channels, 15.4 / 12.7 at 192; 332: 43 / 44 and 31 / 33).
+    } else if (patch_rows_pay(M, n)) {
         allow_dynamic_lds<patch_embed_rows_kernel>(kRowsLds);
         const int row_tiles = static_cast<int>((M + 63) / 64);
         hipLaunchKernelGGL(patch_embed_rows_kernel, dim3(row_tiles + (cls_wgs + 2) / 3), dim3(64 * kRowsWaves), kRowsLds, st, pi, pwt, pb, pc, pp, po,

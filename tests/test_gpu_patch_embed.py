@@ -101,7 +101,29 @@ def test_vit_with_own_patch_embed(cuda, model, batch):
 
 
 @pytest.mark.parametrize("b,h,w,n,with_bias", [(53, 224, 224, 192, True), (161, 128, 128, 32, False), (54, 208, 240, 224, True),
-                                               (215, 112, 112, 384, False)])
+                                               (215, 112, 112, 384, False), (53, 224, 224, 128, False)])
 def test_patch_embed_of_many_patches(cuda, b, h, w, n, with_bias):
-    """The kernel that keeps 64 patches in LDS: ragged last tiles, one tile of channels to all twelve, up to six and more than six."""
+    """The kernel that keeps 64 patches in LDS: ragged last tiles, four tiles of channels to all twelve, up to six and more than six
+    (and as many patches of so few channels that the other kernel takes them)."""
     test_patch_embed_matches_float64(cuda, b, h, w, n, with_bias)
+
+
+# Tiles of 64 patches on 256 compute units: where the round of workgroups is at most a quarter used the kernel of 256 patches is the
+# faster one (39 us against 37 at 257 tiles of 384 channels, 28 against 26 at 192), and at every size below 128 channels.
+@pytest.mark.parametrize("tiles,n,rows", [(159, 384, False), (160, 384, True), (256, 192, True), (257, 192, False), (257, 384, False),
+                                          (273, 384, False), (257, 256, True), (304, 320, False), (305, 320, True), (350, 384, True),
+                                          (513, 384, True), (513, 160, False), (200, 96, False), (200, 128, True), (300, 128, False),
+                                          (1000, 32, False)])
+def test_choice_of_the_kernel_of_many_patches(cuda, tiles, n, rows):
+    if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
+        pytest.skip("the sizes stand for 256 compute units")
+    from test_gpu_host_extension import _kernels
+    g = torch.Generator(device=cuda).manual_seed(tiles + n)
+    img = torch.randn(tiles, 3, 128, 128, generator=g, device=cuda).half()
+    w = (torch.randn(n, 3, 16, 16, generator=g, device=cuda) * 0.05).half()
+    cls, pos = (torch.randn(1, t, n, generator=g, device=cuda).half() for t in (1, 65))
+    out = []
+    names = _kernels(lambda: out.append(ops.patch_embed_fwd(img, w, None, cls, pos)))
+    assert ("patch_embed_rows_kernel" in names) == rows and ("patch_embed_kernel" in names) == (not rows)
+    # (a batch of 150 takes the other kernel; the sums run in the same order in both)
+    assert torch.equal(out[0][:150], ops.patch_embed_fwd(img[:150].contiguous(), w, None, cls, pos))
