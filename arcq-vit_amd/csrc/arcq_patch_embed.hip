@@ -359,7 +359,7 @@ patch_embed_small_kernel(const __half *__restrict__ img, const __half *__restric
 // Where patch_embed_rows_kernel is the faster one.  Its workgroups have a compute unit each, so it takes whole rounds of them, about
 // 2 N / 32 + 3 parts a round (the channels, the patches); the other kernel's (256 patches x 32 channels) are a sixth to a fifth of a
 // round and several share a compute unit.  Measured at 160 to 1 500 tiles of 64 patches, 224 x 224 and 128 x 128 images, us here / there:
-//   one round      384 channels, 160 tiles 20.4 / 23.5, 224 22.7 / 32.2; 192: 14.9 / 17.6, 15.7 / 25.7; 128: 13.6 / 13.6, 14.5 / 16.8;
+//   one round      384 channels, 160 tiles 20.4 / 23.5, 224 22.7 / 32.2; 192: 14.9 / 17.6, 15.7 / 25.7; 128: 13.6 / 13.1, 14.5 / 16.8;
 //                  96: 12.9 / 11.2, 13.6 / 13.6; fewer tiles: 384 channels, 98 tiles 20.1 / 20.4, 192 15.4 / 12.7
 //   a second begun 257 tiles: 384 channels 39.1 / 37.2, 320 36.8 / 34.3, 256 33.8 / 35.8, 224 31.6 / 28.4, 192 28.1 / 25.9, 160 26.4 / 24.2;
 //                  304: 42.1 / 42.1, 38.6 / 39.0, 35.4 / 40.0, 32.9 / 38.5, 29.9 / 29.3, 27.9 / 26.2; 350: 42.8 / 50.7, 39.2 / 47.0,
@@ -368,7 +368,7 @@ patch_embed_small_kernel(const __half *__restrict__ img, const __half *__restric
 bool patch_rows_pay(int64_t M, int64_t n)
 {
     const int64_t cus = device_cus(), tiles = (M + 63) / 64;
-    if (n < 128 || n > kRowsN || tiles * 8 < cus * 5) return false;
+    if (n < 128 || n > kRowsN || tiles * 16 < cus * (n < 160 ? 11 : 10)) return false;
     const int64_t rounds = (tiles + cus - 1) / cus;
     if (rounds == 1) return true;
     const int64_t groups = (M + 128 * kTM - 1) / (128 * kTM), others = (groups * (n / 32) + cus - 1) / cus;      // the other kernel's on a compute unit

@@ -112,7 +112,7 @@ def test_patch_embed_of_many_patches(cuda, b, h, w, n, with_bias):
 # faster one (39 us against 37 at 257 tiles of 384 channels, 28 against 26 at 192), and at every size below 128 channels.
 @pytest.mark.parametrize("tiles,n,rows", [(159, 384, False), (160, 384, True), (256, 192, True), (257, 192, False), (257, 384, False),
                                           (273, 384, False), (257, 256, True), (304, 320, False), (305, 320, True), (350, 384, True),
-                                          (513, 384, True), (513, 160, False), (200, 96, False), (200, 128, True), (300, 128, False),
+                                          (513, 384, True), (513, 160, False), (200, 96, False), (175, 128, False), (176, 128, True), (300, 128, False),
                                           (1000, 32, False)])
 def test_choice_of_the_kernel_of_many_patches(cuda, tiles, n, rows):
     if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
