@@ -225,16 +225,45 @@ void launch_quant(const QuantArgs &a, hipStream_t stream)
 
 }  // namespace
 
-// Measured beside the kernels that end the same way (a whole block, us, at these rows): at least 4.5 tiles of 64 x 64 a compute unit
-// (1 576 rows: 1 024 -> 4 096 116 -> 109, 768 -> 3 072 86 -> 80, FP8 93 -> 88 and 75 -> 72; 985 rows, four tiles: 83 -> 86 and 69 -> 72).
-// Six units of fp16 (K = 384) are too little work a tile to hide the epilogue under: 3 349 .. 9 456 rows 64 -> 62.6 .. 107 -> 106,
-// 25 216 rows 207 -> 209; below that it never pays.
+namespace {
+// Row ranges of 64-row tiles, one workgroup each for every 64 columns: as many as the compute units hold at once.
+struct Ranges {
+    int64_t count, tiles;      // tiles per range
+};
+Ranges ranges_of(int64_t tiles, int64_t slabs)
+{
+    const int64_t count = std::min(std::max(device_cus() / slabs, int64_t(1)), tiles);
+    return {count, (tiles + count - 1) / count};
+}
+}  // namespace
+
+// Measured beside the kernels that end the same way, in blocks (us a block at these rows; one after the other from a graph, with everything
+// in the caches, the quotients are up to 5 % lower):
+//   - At least 4.5 tiles of 64 x 64 a compute unit (1 576 rows: 1 024 -> 4 096 116 -> 109, 768 -> 3 072 86 -> 80, FP8 93 -> 88 and
+//     75 -> 72; 985 rows, four tiles: 83 -> 86 and 69 -> 72).
+//   - Six units of fp16 (K = 384) are too little work a tile to hide the epilogue under: 3 152 .. 9 456 rows 65.6 -> 64.0 .. 107 -> 106,
+//     25 216 rows 207 -> 209; below 4.5 tiles it never pays.
+//   - A range's ninth to twelfth tile is a third turn for its SIMDs, four tiles a turn.  The other kernels' workgroups (128 columns, more
+//     often all of the chip) have eight blocks of 32 rows there or nine: eight are fewer.  5 122 rows: 384 -> 1 536 83.3 -> 80.6,
+//     512 -> 1 536 108 -> 104, 768 -> 1 536 FP8 127 -> 121; 2 167 rows: 768 -> 3 328 114 -> 112, FP8 93.8 -> 92.0; three ranges, 1 576
+//     rows: 768 -> 4 160 FP8 87.4 -> 85.5, fp16 102.8 / 102.8, 512 -> 4 160 83.3 / 87.2.  With fewer ranges the weights' way into LDS
+//     counts for more, and this kernel's are half (1 182 rows: 768 -> 5 504 101.5 / 102, -> 10 240 at 788 rows 123 / 130).
+//   - 129 slabs and a few more leave half of the chip idle (the others: 195 workgroups).  Long ranges: 768 -> 8 256 at 5 910 rows
+//     380 -> 367, FP8 at 4 531 219 -> 210; short ones 123 / 128 at 1 182 rows; 160 slabs 230 / 250 at 2 758, FP8 1 024 -> 10 240
+//     198 / 210 at 3 152; 257 slabs are two rounds in both.
 bool gemm_quant_pays(int64_t M, int64_t N, int64_t K, bool fp8)
 {
     const int units = operand_units(static_cast<int>(K), fp8);
     if (N % 64 != 0 || M < 512 || units < 6 || units % kAhead != 0 || quant_lds_bytes(units) > kMaxLds) return false;
-    const int64_t tiles = (M + 63) / 64 * (N / 64), cus = device_cus();
-    return 2 * tiles >= 9 * cus && (fp8 || units >= 8 || tiles <= 16 * cus);
+    const int64_t rows = (M + 63) / 64, slabs = N / 64, tiles = rows * slabs, cus = device_cus();
+    if (2 * tiles < 9 * cus || (!fp8 && units < 8 && tiles > 16 * cus)) return false;
+    const Ranges r = ranges_of(rows, slabs);
+    if (r.tiles > 64 && slabs <= cus && 16 * slabs * r.count < 9 * cus) return false;
+    if (r.count >= (fp8 ? 3 : 4) && r.tiles > 8 && r.tiles <= 12) {
+        const int64_t blocks = (M + 31) / 32, others = std::max(cus / ((N + 127) / 128), int64_t(1));
+        if ((blocks + others - 1) / others <= 8) return false;
+    }
+    return true;
 }
 
 void launch_gemm_quant(const GemmArgs &g, const void *w_hat, hipStream_t stream)
@@ -249,9 +278,8 @@ void launch_gemm_quant(const GemmArgs &g, const void *w_hat, hipStream_t stream)
     // 1 653 -> 1 636 us, of 768 (310 MB) 1 070 -> 1 057; 25 216 rows of 768 (155 MB) 551 -> 557.
     a.streaming = static_cast<int64_t>(g.M) * g.N * (g.fp8 ? 1 : 2) > int64_t(200) << 20;
     a.slabs = g.N / 64;
-    const int tiles = (g.M + 63) / 64;
-    a.ranges = std::min(std::max(device_cus() / a.slabs, 1), tiles);
-    a.tiles_per_range = (tiles + a.ranges - 1) / a.ranges;
+    const Ranges r = ranges_of((g.M + 63) / 64, a.slabs);
+    a.ranges = static_cast<int>(r.count), a.tiles_per_range = static_cast<int>(r.tiles);
     if (g.fp8) {
         if (g.bits == 4) launch_quant<4, true>(a, stream);
         else if (g.bits == 3) launch_quant<3, true>(a, stream);

@@ -334,6 +334,27 @@ def test_synth():
     assert [s[1:] for s in synth.block_linear_shapes("deit_small")] == [(384, 1152), (384, 384), (384, 1536), (1536, 384)]
 
 
+@pytest.mark.parametrize("m,n,k,fp8,pays", [
+    (1576, 4096, 1024, 0, True), (1576, 3072, 768, 0, True), (1576, 3072, 768, 1, True), (985, 4096, 1024, 0, False),
+    (3152, 1536, 384, 0, True), (9456, 1536, 384, 0, True), (12608, 1536, 384, 0, False), (50432, 4096, 1024, 0, True),
+    # nine tiles a range: the other kernels' eight blocks of rows, or nine
+    (5120, 1536, 384, 0, True), (5122, 1536, 384, 0, False), (5319, 1536, 768, 1, False), (5376, 1536, 384, 0, False),
+    (5377, 1536, 384, 0, True), (2167, 3328, 768, 0, False), (1576, 4160, 768, 1, False), (1576, 4160, 768, 0, True),
+    (1182, 5504, 768, 1, True), (788, 10240, 768, 0, True), (2849, 2752, 768, 0, True),
+    # half of the chip for long, and two rounds of workgroups
+    (5910, 8256, 768, 0, False), (4531, 8256, 768, 1, False), (1182, 8256, 768, 0, True), (2758, 10240, 768, 0, True),
+    (5910, 16448, 768, 0, True),
+    # eighteen units of 128 bytes are the most that LDS holds
+    (1601, 3072, 1152, 0, True), (1601, 3072, 1280, 0, False), (1601, 3072, 2304, 1, True), (1601, 3072, 2560, 1, False)])
+def test_where_the_quantizing_product_keeps_its_weights_in_lds(m, n, k, fp8, pays):
+    """Sizes on both sides of the lines that arcq_gemm_quant.hip draws (256 compute units, also without a GPU): row-major weights
+    select the other kernels."""
+    lib = A._lib.load()
+    assert lib.arcq_prepared_quant_row_major(m, n, k, fp8) == (0 if pays else lib.arcq_prepared_row_major(m, n, k))
+    if not pays and m != 985:
+        assert lib.arcq_prepared_row_major(m, n, k) == 1
+
+
 def test_fused_kernel_choice_is_reported_without_a_gpu(monkeypatch):
     """arcq_linear_fused_kernel is a pure function of the shape (and of the ARCQ_GEMM_KERNEL override)."""
     lib = A._lib.load()
