@@ -598,7 +598,8 @@ ARCQ_API int arcq_mlp_otf_pays(int64_t M, int64_t K, int64_t H)
 {
     if (!arcq_mlp_otf_supported(M, K, H) || tuning().gemm_kernel) return 0;
     if (const char *e = tuning().rows) return e[0] != '0';
-    return M > (K == 192 ? 7000 : 10700);      // (the launch takes as long however few its workgroups are; figures beside the block's launches, arcq_host.cpp)
+    // (the launch takes as long however few its workgroups are; figures beside the block's launches, arcq_host.cpp)
+    return M > (K == 192 ? 6600 : K == 256 ? 7200 : K == 384 ? 8700 : 10240);
 }
 
 ARCQ_API int arcq_mlp_otf(const arcq_mlp_args *a, void *stream)

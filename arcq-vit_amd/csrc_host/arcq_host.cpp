@@ -689,11 +689,13 @@ std::optional<Tensor> block_prepared(const BlockParts &k, const Tensor &x, int64
         if (!can_prepare(*p, rows) || p->bits != pq.bits) return std::nullopt;
     // Not where the one-launch kernels are at their best (one 64-row tile on most compute units, short rows).  With the LayerNorms
     // inside, hidden rows of four times the width and lent weight buffers, the block is three launches there, the last of them proj and
-    // the whole MLP.  Forwards against the seven launches: DeiT-S 10 047 rows 1 336 us against 1 271, 10 638 1 346 / 1 344, 11 032 1 344 /
-    // 1 529 (a round of 128-row tiles more), 12 608 1 381; DeiT-B 10 638 3 117 / 3 038, 11 032 3 160 / 3 342; DeiT-Tiny 6 304 718 / 685,
-    // 7 092 726 / 748, 9 259 763 / 783; with more row tiles than compute units the seven win (a block of DeiT-Tiny at 19 700 rows 99
-    // against 112).  Without the one-launch MLP 9 000 rows: DeiT-S at 12 608 rows 1 625 us a forward against 1 939 (five launches a
-    // block), at 6 304 rows 1 353 -> 1 262.
+    // the whole MLP.  Forwards of twelve blocks against the seven launches, us: K = 192 6 501 rows 709 / 693, 6 698 706 / 716, 7 092
+    // 714 / 739; K = 256 6 698 837 / 827, 7 092 837 / 836, 7 486 846 / 854, 8 668 857 / 1 019; K = 384 8 668 1 299 / 1 300, 8 865
+    // 1 306 / 1 317, 10 244 1 341 / 1 429; K = 768 10 047 3 168 / 3 096, 10 244 3 179 / 3 181, 10 638 3 198 / 3 255, 10 835 3 205 / 3 569;
+    // with more row tiles than compute units the seven win (a block of DeiT-Tiny at 19 700 rows 99 against 112).  Hidden rows of another
+    // width, five launches: 9 000 rows (DeiT-S as five launches at 12 608 rows 1 625 us a forward against 1 939, at 6 304 1 353 -> 1 262).
+    // Without lent buffers every layer call would be two launches; the seven are faster at every width (12 608 rows, six blocks: K = 192
+    // 498 us against 577, 256 600 / 682, 384 889 / 970, 768 1 974 / 2 298).
     // With torch's LayerNorms and GELU those kernels run only on lent weight buffers, and win later and only beside torch's
     // attention: 10 638 rows DeiT-S 2 311 us against 2 264 here, DeiT-B 4 498 / 4 406, 11 032 rows 2 318 / 2 439 and 4 607 / 4 879,
     // 12 608 rows 2 399 / 2 564 and 4 892 / 5 147; without lent buffers (two launches a layer) 2 667 / 2 590 and 5 207 / 5 178, with

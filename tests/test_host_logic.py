@@ -355,6 +355,16 @@ def test_where_the_quantizing_product_keeps_its_weights_in_lds(m, n, k, fp8, pay
         assert lib.arcq_prepared_row_major(m, n, k) == 1
 
 
+@pytest.mark.parametrize("k,least,window", [(192, 6698, (6501, 16548)), (256, 7486, (6698, 16548)), (384, 8865, (8471, 16548)),
+                                            (768, 10441, (10047, 16548))])
+def test_where_the_one_launch_mlp_pays(k, least, window):
+    """Row counts at which both forms of a block were timed, on both sides of the lines for each width (64 rows on at most 256 compute units)."""
+    lib = A._lib.load()
+    assert lib.arcq_mlp_otf_pays(least, k, 4 * k) == 1 and lib.arcq_mlp_otf_pays(16384, k, 4 * k) == 1
+    assert lib.arcq_mlp_otf_pays(window[0], k, 4 * k) == 0 and lib.arcq_mlp_otf_pays(window[1], k, 4 * k) == 0
+    assert lib.arcq_mlp_otf_pays(12608, k, 3 * k) == 0
+
+
 def test_fused_kernel_choice_is_reported_without_a_gpu(monkeypatch):
     """arcq_linear_fused_kernel is a pure function of the shape (and of the ARCQ_GEMM_KERNEL override)."""
     lib = A._lib.load()
