@@ -87,9 +87,11 @@ def test_one_launch_mlp_has_the_bits_of_the_two_layers(cuda, monkeypatch, m, k, 
         x[3, 7] = float("inf")
     x = x.half().to(cuda)
     assert _lib.load().arcq_mlp_otf_supported(m, k, 4 * k)
+    before = _lib.load().arcq_rows_wait_timeouts()
     if case == "no wait":
         monkeypatch.setenv("ARCQ_ROWS_WAIT_TICKS", "0")
     y = _one_launch(x, norm, fc1, fc2)
+    assert case != "no wait" or _lib.load().arcq_rows_wait_timeouts() > before
     with torch.no_grad():
         h = fc1(x, layernorm=norm, activation="gelu")
         want = fc2(h, residual=x)
@@ -122,9 +124,11 @@ def test_one_launch_with_proj_has_the_bits_of_the_three_layers(cuda, monkeypatch
         attn[3, 7] = float("inf")
         x[65, 2] = float("-inf")
     x, attn = x.half().to(cuda), attn.half().to(cuda)
+    before = _lib.load().arcq_rows_wait_timeouts()
     if case == "no wait":
         monkeypatch.setenv("ARCQ_ROWS_WAIT_TICKS", "0")
     y = _one_launch(x, norm, fc1, fc2, proj, attn)
+    assert case != "no wait" or _lib.load().arcq_rows_wait_timeouts() > before
     with torch.no_grad():
         x1 = proj(attn, residual=x)
         want = fc2(fc1(x1, layernorm=norm, activation="gelu"), residual=x1)
@@ -144,27 +148,58 @@ def test_sizes_that_it_does_not_serve_are_refused_before_a_launch(cuda):
         assert lib.arcq_mlp_otf(ctypes.byref(a), None) < 0
 
 
-def test_blocks_with_lent_buffers_take_it(cuda):
-    """A fused block at a size where it pays: the bits of the block that runs fc1 and fc2 as two launches, also replayed as a graph."""
+@pytest.mark.parametrize("model,k", [("deit_tiny", 192), ("deit_small", 384), ("deit_base", 768)])
+def test_blocks_with_lent_buffers_take_it(cuda, model, k):
+    """A fused block at a size where it pays: three launches, proj in the last one; the bits of the block that runs proj, fc1 and fc2
+    as three, also replayed as a graph."""
+    from test_gpu_host_extension import _kernels
     from arcq_vit_amd.vit import build_packed_vit
-    net = build_packed_vit("deit_tiny", 4, device=str(cuda), depth=1, shared_buffers=True, max_rows=64 * 197, fuse_elementwise=True,
+    net = build_packed_vit(model, 4, device=str(cuda), depth=1, shared_buffers=True, max_rows=64 * 197, fuse_elementwise=True,
                            own_attention=True, own_patch_embed=True)
     block = net.blocks[0]
-    x = torch.randn(64, 197, 192, generator=torch.Generator().manual_seed(5)).half().to(cuda)
-    assert _lib.load().arcq_mlp_otf_pays(64 * 197, 192, 768) == 1
+    x = torch.randn(64, 197, k, generator=torch.Generator().manual_seed(5)).half().to(cuda)
+    assert _lib.load().arcq_mlp_otf_pays(64 * 197, k, 4 * k) == 1
     with torch.no_grad():
         block.chain_mlp = False
         want = block(x)
+        assert "otf_mlp_kernel" not in _kernels(lambda: block(x))
         block.chain_mlp = True
         assert torch.equal(block(x), want)
+        names = _kernels(lambda: block(x))
+        assert [names.count(n) for n in ("otf_rows_kernel", "attention_kernel", "otf_mlp_kernel")] == [1, 1, 1], names
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             y = block(x)
         for i in range(4):
-            x.copy_(torch.randn(64, 197, 192, generator=torch.Generator().manual_seed(10 + i)).half())
+            x.copy_(torch.randn(64, 197, k, generator=torch.Generator().manual_seed(10 + i)).half())
             block.chain_mlp = i % 2 == 0
             eager = block(x)
             torch.cuda.synchronize()
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, eager), i
+
+
+@pytest.mark.parametrize("case", ["proj of three bits", "fc2 of three bits"])
+def test_blocks_that_it_serves_in_part_or_not(cuda, case):
+    """A proj of other code bits is a layer call and the launch starts at the LayerNorm; with other bits in fc2 there is no such launch."""
+    from test_gpu_host_extension import _kernels
+    from arcq_vit_amd.packed_convert import share_buffers
+    from arcq_vit_amd.vit import build_packed_vit
+    gen = torch.Generator().manual_seed(9)
+    net = build_packed_vit("deit_small", 4, device=str(cuda), depth=1, shared_buffers=True, max_rows=64 * 197, fuse_elementwise=True,
+                           own_attention=True, own_patch_embed=True)
+    block = net.blocks[0]
+    x = torch.randn(64, 197, 384, generator=gen).half().to(cuda)
+    if case == "proj of three bits":
+        block.attn.proj = _layer(cuda, 384, 384, 3, gen)
+    else:
+        block.mlp.fc2 = _layer(cuda, 384, 1536, 3, gen)
+    share_buffers(net, 64 * 197)
+    with torch.no_grad():
+        block.chain_mlp = False
+        want = block(x)
+        block.chain_mlp = True
+        assert torch.equal(block(x), want)
+        names = _kernels(lambda: block(x))
+    assert names.count("otf_mlp_kernel") == (0 if case == "fc2 of three bits" else 1), names
