@@ -10,9 +10,10 @@ from arcq_vit_amd import _lib, ops, synth
 pytestmark = pytest.mark.gpu
 
 # One row past a pair of row blocks, past a block, whole pairs; slabs that do not divide the compute units, more slabs than compute
-# units; odd numbers of output groups; six units to the most that LDS holds; outputs beyond 200 MB.
+# units; odd numbers of output groups; six units to the eighteen that LDS holds; outputs beyond 200 MB.
 SHAPES = [(1153, 4096, 1024, 4, ""), (1249, 4160, 768, 3, ""), (2048, 2304, 1024, 2, ""), (3360, 1536, 384, 4, ""), (513, 17408, 512, 4, ""),
-          (1216, 4096, 768, 4, "thresholds"), (1153, 4096, 1024, 3, "large"), (26017, 4160, 512, 4, "")]
+          (1216, 4096, 768, 4, "thresholds"), (1153, 4096, 1024, 3, "large"), (26017, 4160, 512, 4, ""),
+          (1601, 3072, 1152, 4, "")]
 
 
 @pytest.mark.parametrize("m,n,k,bits,case", SHAPES)
@@ -31,7 +32,8 @@ def test_fp16(cuda, oracle, m, n, k, bits, case):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), gelu
 
 
-@pytest.mark.parametrize("m,n,k,bits", [(1153, 4096, 1024, 4), (1249, 4160, 768, 3), (2048, 4096, 1536, 2), (513, 17408, 1024, 4), (6304, 3072, 704, 4)])
+@pytest.mark.parametrize("m,n,k,bits", [(1153, 4096, 1024, 4), (1249, 4160, 768, 3), (2048, 4096, 1536, 2), (513, 17408, 1024, 4), (6304, 3072, 704, 4),
+                                        (1601, 3072, 2304, 4)])
 def test_fp8(cuda, oracle, m, n, k, bits):
     """Also the padding of a row to 128 values, of the operands (704 values) and of the output (4 160)."""
     cb, thr, w, bias = f16._layer(oracle, cuda, n, k, bits, 3)
