@@ -23,11 +23,14 @@
 // The arithmetic, the order of every sum and the roundings are those of the two layers run one after the other: y has their bits.
 //
 // Measured: 12 608 rows, K = 768, fc1 and fc2 as two launches 110 + 120 us, this one 160 (the base model's forward at 64 images 3 809 ->
-// 3 364 us); K = 384 29 + 39 -> 68 (1 559 -> 1 470); K = 192 -> 34 (a block 79 -> 69).  Clocks of a workgroup at K = 768, 320 000 in
-// all: set-up 19 000 (x from memory, shares of weights), LayerNorm and stage 1 33 000 (vector ALU, on two waves a SIMD), thirteen steps
-// of 17 000 each, output 12 000.  In a step the quantizing wave takes 3 300 for the rest of GELU, 8 800 for the quantizer and 3 800 for
-// fc2's 96 MFMAs (3 072 at full rate), its partner 3 500 for those, 7 600 for fc1's 192 (6 144) and 4 000 for the first half of GELU (now three eighths): a
-// wave alone issues a vector instruction every five clocks or so, and the other's MFMAs take about eight of them each.
+// 3 364 us); K = 384 29 + 39 -> 68 (1 559 -> 1 470); K = 192 -> 34 (a block 79 -> 69).  Clocks of a workgroup with proj in front, K =
+// 768: 358 000 in all: set-up 20 000 (inputs from memory, shares of weights), proj's stage 1 and the wait 16 000, proj with its epilogue
+// 31 700, LayerNorm and stage 1 29 500 (vector ALU, on two waves a SIMD), the first chunk of fc1 21 000, twelve steps of 16 800 to
+// 20 200 (18 500 on average), the last product and output 17 500.  In a step the quantizing wave takes 3 700 for the rest of GELU,
+// 7 500 to 8 900 for the quantizer and 4 400 to 5 100 for fc2's 96 MFMAs (3 072 at full rate), its partner 3 450 for those, 7 700 for
+// fc1's 192 (6 144) and 3 000 for the first three eighths of GELU: a wave alone issues a vector instruction every five clocks or so, and
+// the other's MFMAs take about eight of them each.  K = 384: 156 000, of them six steps of 12 600 to 14 800.
+// Registers: all 256.  K = 768 keeps 19 to 22 more in scratch, a dozen of its loads and stores a step; K = 384 with proj two.
 //
 // Weights: rebuilt by the launch's workgroups between them, as in arcq_otf_rows.hip (proj's and fc1's together); fc2's under
 // the first fc1 chunk, by the set that has nothing to multiply yet.
@@ -471,8 +474,7 @@ otf_mlp_kernel(const MlpParams p)
     // ---- the chunks.  Step t: one set quantizes chunk t of the hidden row, then adds chunk t - 1 to fc2's sums; the other one adds
     // chunk t - 1, multiplies chunk t + 1 of fc1 and takes the first kEarly eighths of its GELU, so that both are done at about the
     // same time and the matrix units and vector ALUs of every SIMD have work side by side.  Then they change places. ----
-    // (Beside 4 and 8, from before the quantizer's lookups had constant addresses: base model at 64 images 3 389 -> 3 369 us, 3 442 with
-    // five eighths; small model 1 400 -> 1 394.)
+    // (Base model at 64 images 3 369 us; half of GELU instead 3 389, five eighths 3 442.  Small model 1 394; all of it 1 400.)
     constexpr int kEarly = G >= 12 ? 3 : 5;
     constexpr int64_t stride1 = static_cast<int64_t>(K) * 64, stride2 = static_cast<int64_t>(kWaves) * H * 64;
     const unsigned char *h_lane = hs + lr * kHiddenPitch + lh * 64;

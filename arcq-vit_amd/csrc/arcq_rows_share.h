@@ -29,7 +29,7 @@ template <int BITS, int G>
 __device__ __forceinline__ void fetch_piece(const WeightShare &p, int64_t idx, Piece &pc)
 {
     constexpr int K = 64 * G, P = K / 8, pcols = K * BITS / 8;     // compile-time: the divisions below are multiplications
-    const uint32_t i = static_cast<uint32_t>(idx);                 // N * K / 8 < 2^31 (N <= 16384, K <= 384)
+    const uint32_t i = static_cast<uint32_t>(idx);                 // N * K / 8 < 2^23 (N <= 16384, K <= 3072)
     const uint32_t r = i & 31u;
     const uint32_t t = i >> 5;
     const uint32_t nb = t / P;
@@ -56,7 +56,6 @@ __device__ __forceinline__ void finish_piece(const WeightShare &p, int64_t idx, 
     }
     store_writethrough16(p.out + idx * 8, out[0], out[1], out[2], out[3]);
 }
-
 
 // Two counter words (zero when the code object is loaded) that belong to weight workspace `key` on the current device, nullptr if none
 // is left, and the device's count of workgroups whose wait ran out.
